@@ -1927,7 +1927,10 @@ int norm_linear_launch(const char* name, const void* x, int64_t ldx, const void*
   const int num_tiles = static_cast<int>(tiles64);  // upper bound: with a row index the kernel derives its own
   const int cus = compute_units();
   if (cus <= 0) return set_error(TAAC_ERR_LAUNCH, "%s: cannot query the device", name);
-  int grid = num_tiles < cus ? num_tiles : cus;
+  // Fewer token tiles than compute units: the kernel splits the tiles of a partial round by output chunks over the workgroups
+  // it has, so the grid is not held to one workgroup per tile (one request of 512 tokens ran on one compute unit: q | k | v
+  // projection 44 -> 12.6 us, 45 900 positions of the narrow network 31 -> 18 us).
+  int grid = static_cast<int64_t>(num_tiles) * (N / kNC) < cus ? num_tiles * (N / kNC) : cus;
   // taac_test_hooks: cap the number of persistent workgroups so that small inputs exercise the multi-tile path.
   if (const int limit = test_max_workgroups(); limit > 0 && limit < grid) grid = limit;
 #define TAAC_LIN_LAUNCH(KK, TT, RR, QQ)                                                                           \
