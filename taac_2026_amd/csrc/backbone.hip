@@ -664,17 +664,21 @@ extern "C" int taac_backbone_fwd(const void* emb, const int32_t* key_lengths, co
         if ((rc = check_launch(name)) != TAAC_OK) return rc;
         q_col_scale = prod;
       }
-      if (weights_in_epilogue) {
+      const void* q_weight = weights_in_epilogue ? w.query_norm_weight : nullptr;
+      const void* k_weight = weights_in_epilogue ? w.key_norm_weight : nullptr;
+      if (weights_in_epilogue && (!planes || !aligned16(q_weight) || !aligned16(k_weight))) {
         if (hipMemcpyAsync(qk_weight, w.query_norm_weight, static_cast<size_t>(D) * 2, hipMemcpyDeviceToDevice,
                            as_stream(stream)) != hipSuccess ||
             hipMemcpyAsync(qk_weight + D, w.key_norm_weight, static_cast<size_t>(D) * 2, hipMemcpyDeviceToDevice,
                            as_stream(stream)) != hipSuccess)
           return set_error(TAAC_ERR_LAUNCH, "%s: copy of the query / key norm weights failed", name);
+        q_weight = qk_weight;
+        k_weight = qk_weight + D;
       }
       if (planes)
-        rc = norm_linear_qk_heads(cur, D, w.attn_norm_weight, eps, w.qkv_bias, pk_qkv, qkv, M, D, heads, T,
-                                  weights_in_epilogue ? qk_weight : nullptr, rope_cos_sin, qk_norm ? qk_sumsq : nullptr,
-                                  rows, n_rows, w.attn_norm_weight != nullptr, stream);
+        rc = norm_linear_qk_heads(cur, D, w.attn_norm_weight, eps, w.qkv_bias, pk_qkv, qkv, M, D, heads, T, q_weight,
+                                  k_weight, rope_cos_sin, qk_norm ? qk_sumsq : nullptr, qk_norm ? qk_rstd : nullptr, rows,
+                                  n_rows, w.attn_norm_weight != nullptr, stream);
       else
         rc = taac_norm_linear_qk_fwd(cur, D, w.attn_norm_weight, eps, nullptr, w.qkv_bias, pk_qkv, qkv, 3 * D, M, D, heads,
                                      T, weights_in_epilogue ? qk_weight : nullptr, rope_cos_sin,
@@ -682,7 +686,9 @@ extern "C" int taac_backbone_fwd(const void* emb, const int32_t* key_lengths, co
                                      stream);
       if (rc != TAAC_OK) return rc;
       if (qk_norm) {
-        if ((rc = taac_row_rstd(qk_sumsq, M, D, eps, qk_rstd, rows, n_rows, stream)) != TAAC_OK) return rc;
+        if (!(planes && dense_few_rows(M, D)) &&
+            (rc = taac_row_rstd(qk_sumsq, M, D, eps, qk_rstd, rows, n_rows, stream)) != TAAC_OK)
+          return rc;
         q_scale = qk_rstd;
         k_scale = qk_rstd + M;
       }

@@ -24,71 +24,10 @@
 // of roundings of the reference's bf16 evaluation (linear output rounded, then the residual add rounded).
 #include "common.h"
 #include "ts_common.h"
+#include "ts_dense.h"
 
 namespace taac {
 namespace {
-
-constexpr int kFrag = 1024;  // bytes of one 32 x 16 bf16 MFMA operand fragment
-constexpr int kNC = 64;      // output features per chunk of the plain linear kernel
-constexpr int kHU = 16;      // hidden units per FFN chunk
-constexpr int kCPB = 2;      // FFN chunks per barrier step
-constexpr int kStageRow = kNC * 2 + 16;       // bytes per token row of the epilogue tile (64 features + pad)
-constexpr int kStageWave = 32 * kStageRow;    // epilogue tile of one wavefront: 32 tokens x 64 features
-
-struct TsParams {
-  const bf16_t* x;          // [M, D] row stride ldx
-  const bf16_t* norm_w;     // [D] or null (no normalisation)
-  const bf16_t* w1;         // FFN: w_up [2F, D] or the packed blob; linear: w [N, D] or the packed blob
-  const bf16_t* b1;         // FFN: b_up [2F] or null; linear: bias [N] or null
-  const bf16_t* w2;         // FFN: w_down [D, F] (unused when packed)
-  const bf16_t* b2;         // FFN: b_down [D] or null
-  const bf16_t* residual;   // [M, D or N] row stride ldr, or null
-  bf16_t* out;              // [M, D or N] row stride ldo
-  int64_t M, ldx, ldr, ldo;
-  int32_t F;                // FFN hidden size
-  int32_t N;                // linear output features
-  float eps;
-  int32_t gate_first;
-  int32_t packed;           // weights are in fragment order
-  const int32_t* rows;      // optional row index: token i lives in row rows[i] of x / residual / out
-  const int32_t* n_rows;    // with rows: device pointer to the number of tokens (at most M)
-  const int32_t* x_rows;    // optional, with rows: token i's row of x when it differs from rows[i] (x and residual / out
-                            // laid out differently: samples with their valid tokens moved to the front on one side)
-  int32_t units;            // FFN: compute units the last, partial round of workgroups is spread over
-  // Query / key mode of the linear kernel (the packed q | k | v projection of an attention layer):
-  const bf16_t* qk_w;       // [qk_chunks * 64] norm weights of the query and key features (q | k), or null (ones)
-  const bf16_t* cos_sin;    // rotary table [tokens_per_sample][head_dim] of (cos, sin) pairs, or null
-  float* qk_sumsq;          // [qk_chunks][M] sum of squares of a token's 64 features of one chunk
-  int32_t qk_chunks;        // leading 64-feature chunks that belong to the query and key projections
-  int32_t head_dim, tokens_per_sample;
-  // Attention output projection in front of the FFN (x is then the attention output, residual the block input):
-  const bf16_t* w0;         // packed [D, D] projection (linear blob)
-  const bf16_t* b0;         // its bias [D] or null
-  int32_t norm_folded;      // linear kernel: norm_w is already part of the packed weights (taac_linear_pack_weights_norm):
-                            // the rows enter the products as they are and only the factor rsqrt(mean + eps) is applied, to the
-                            // accumulators
-  const bf16_t* gate;       // GATE: [M, D] pre-activation of the update's gate (rows like residual), row stride ldg
-  int64_t ldg;
-  // Feature planes (the backbone's private q | k | v and attention-output buffers): with a shift s > 0 the tensor is a
-  // stack of planes of 2^s features, [cols / 2^s][M][2^s] - element (row, col) at ((col >> s) * M + row) * 2^s + col % 2^s -
-  // instead of [M][cols] rows; a head's rows are then contiguous for the attention kernel.
-  int32_t x_plane_shift;    // layout of x (0: rows of ldx elements)
-  int32_t out_plane_shift;  // layout of out (linear kernel without residual or query / key epilogue; 0: rows of ldo elements)
-  // Readout riding on the feed-forward epilogue: token_dots[row] = sum over the features of out[row] * head_w (fp32, from
-  // the rounded output), so that a mean-pooling linear head behind the layer need not read the rows again.
-  const bf16_t* head_w;     // [D] or null
-  float* token_dots;        // [M] (rows like out), written for the tokens the kernel stores
-};
-
-__device__ __forceinline__ float silu_f(float v) {
-  return v * __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(-1.4426950408889634f * v));
-}
-
-// Hidden unit (0..15) loaded into row slot m16 of the gate (or value) half of an up fragment: chosen so that
-// accumulator register j < 8 of lane half hh holds hidden unit 8*hh + j, the k order of a W_down fragment.
-__host__ __device__ __forceinline__ int up_unit_of_slot(int m16) {
-  return 8 * ((m16 >> 2) & 1) + 4 * (m16 >> 3) + (m16 & 3);
-}
 
 // ---- fragment-order packing ------------------------------------------------------------------------------------------
 // FFN blob: step s (32 hidden units) holds, for chunk q = 0, 1: KS up fragments (k-step r) then MB down fragments
@@ -98,7 +37,6 @@ __host__ __device__ __forceinline__ int up_unit_of_slot(int m16) {
 // fold_act: the constants of the gate's activation join the same rounding - the gated half is multiplied by -log2(e), the
 // other half by -ln 2, so that silu(g) * u = g' * u' / (1 + 2^g') with g' and u' as they leave the matrix unit (the
 // kernel's FOLD form: one multiplication less per hidden unit and token; the first-layer bias is scaled when it is staged).
-constexpr float kFoldGate = -1.4426950408889634f, kFoldValue = -0.6931471805599453f;
 __device__ __forceinline__ void ffn_pack_piece(const bf16_t* __restrict__ w_up, const bf16_t* __restrict__ w_down,
                                                bf16x8* __restrict__ packed, int D, int F, int gate_first, int64_t gid,
                                                const bf16_t* __restrict__ col_scale = nullptr, bool fold_act = false) {
@@ -212,238 +150,6 @@ __global__ void pack_blocks_kernel(const PackBatch batch, int D, int F, bool fol
   gid -= n_out;
   if (gid < n_ffn)
     ffn_pack_piece(batch.up[blk], batch.down[blk], batch.packed_ffn[blk], D, F, 1, gid, batch.ffn_norm[blk], fold_act);
-}
-
-// ---- shared pieces ---------------------------------------------------------------------------------------------------
-
-// Number of tokens to process: M, or *n_rows (clamped to M) when a row index is given.
-__device__ __forceinline__ int64_t token_count(const TsParams& p) {
-  if (p.rows == nullptr) return p.M;
-  const int64_t n = *p.n_rows;
-  return n < p.M ? n : p.M;
-}
-
-// Row of x / residual / out that holds token `tok`. Tokens at or beyond the count are mapped to the last token: they
-// compute bit-identical values, so loading and storing them again is benign and every wavefront issues the same
-// number of memory operations.
-__device__ __forceinline__ int64_t token_row(const TsParams& p, int64_t count, int64_t tok) {
-  tok = tok < count ? tok : count - 1;
-  return p.rows != nullptr ? static_cast<int64_t>(p.rows[tok]) : tok;
-}
-
-// Row of x that holds token `tok`: its own index when one is given, the common one otherwise.
-__device__ __forceinline__ int64_t input_row(const TsParams& p, int64_t count, int64_t tok) {
-  if (p.x_rows == nullptr) return token_row(p, count, tok);
-  tok = tok < count ? tok : count - 1;
-  return static_cast<int64_t>(p.x_rows[tok]);
-}
-
-// Rows of N tokens at once (token i = tok_of(i)), in two phases: request() issues the N index loads inside ONE test of
-// the index pointer and touches none of the loaded values, row() turns entry i into a row number. Whatever the caller
-// requests between the two is in flight together with the index (token_row() per token puts every load behind its own
-// test of the pointer and a wait behind every load).
-template <int N>
-struct TokenRows {
-  int64_t tok[N];
-  int32_t loaded[N];
-  bool indexed;
-  template <typename F>
-  __device__ __forceinline__ void request(const int32_t* index, int64_t count, F tok_of) {
-#pragma unroll
-    for (int i = 0; i < N; ++i) {
-      const int64_t t = tok_of(i);
-      tok[i] = t < count ? t : count - 1;
-      loaded[i] = 0;
-    }
-    indexed = index != nullptr;
-    if (indexed) {
-#pragma unroll
-      for (int i = 0; i < N; ++i) loaded[i] = index[tok[i]];
-    }
-  }
-  // Marks the point up to which the loaded entries stay untouched (the compiler would otherwise widen them right behind
-  // their loads, with a wait in front).
-  __device__ __forceinline__ void arrive() {
-#pragma unroll
-    for (int i = 0; i < N; ++i) asm volatile("" : "+v"(loaded[i]));
-  }
-  __device__ __forceinline__ int64_t row(int i) const { return indexed ? static_cast<int64_t>(loaded[i]) : tok[i]; }
-};
-template <int N, typename F>
-__device__ __forceinline__ void token_rows_batch(const int32_t* index, int64_t count, F tok_of, int64_t (&row)[N]) {
-  TokenRows<N> rows;
-  rows.request(index, count, tok_of);
-  // the entries are awaited here, on this path: left pending, the compiler protects their registers with waits for ALL
-  // vector-memory operations wherever the paths of the caller meet again (in front of the MFMAs of every step)
-  rows.arrive();
-#pragma unroll
-  for (int i = 0; i < N; ++i) row[i] = rows.row(i);
-}
-
-// Loads the wavefront's token rows as B-operand fragments: lane (l32, hh) holds features 16*ks + 8*hh .. +7 of token
-// l32 of each 32-token tile.
-// The same from row numbers the caller already holds (r[t]: memory row of token l32 of tile t).
-template <int D, int TT>
-__device__ __forceinline__ void load_token_rows_at(const TsParams& p, const int64_t (&r)[TT], int hh, bf16x8 (&xf)[TT][D / 16]) {
-  constexpr int KS = D / 16;
-  if (p.x_plane_shift > 0) {  // feature planes: k-step ks lies in plane (16 * ks) >> shift
-    const int sh = p.x_plane_shift;
-    const int64_t plane_elems = p.M << sh;
-#pragma unroll
-    for (int t = 0; t < TT; ++t) {
-      const bf16_t* row = p.x + (r[t] << sh) + hh * 8;
-#pragma unroll
-      for (int ks = 0; ks < KS; ++ks)
-        xf[t][ks] = *reinterpret_cast<const bf16x8*>(row + ((ks * 16) >> sh) * plane_elems + ((ks * 16) & ((1 << sh) - 1)));
-    }
-    return;
-  }
-#pragma unroll
-  for (int t = 0; t < TT; ++t) {
-    const bf16_t* row = p.x + r[t] * p.ldx + hh * 8;
-#pragma unroll
-    for (int ks = 0; ks < KS; ++ks) xf[t][ks] = *reinterpret_cast<const bf16x8*>(row + ks * 16);
-  }
-}
-
-template <int D, int TT>
-__device__ __forceinline__ void load_token_rows(const TsParams& p, int64_t count, int64_t tok0, int l32, int hh,
-                                                bf16x8 (&xf)[TT][D / 16]) {
-  // the row numbers of all tiles first: one memory latency in front of the row loads, not one per tile
-  int64_t r[TT];
-  token_rows_batch<TT>(p.x_rows != nullptr ? p.x_rows : p.rows, count, [&](int t) { return tok0 + t * 32 + l32; }, r);
-  load_token_rows_at<D, TT>(p, r, hh, xf);
-}
-
-// RMS-normalises the loaded rows in place: y = bf16( x * rsqrt(mean(x^2) + eps) * w ), w read from its LDS copy.
-// folded: the norm's weight is part of the layer that consumes the rows; only the per-token factor is applied.
-template <int D, int TT>
-__device__ __forceinline__ void normalize_tokens(float eps, const bf16_t* norm_w_lds, int hh, bf16x8 (&xf)[TT][D / 16],
-                                                 bool folded = false) {
-  constexpr int KS = D / 16;
-  float scale[TT];
-#pragma unroll
-  for (int t = 0; t < TT; ++t) {
-    float ss = 0.f;
-#pragma unroll
-    for (int ks = 0; ks < KS; ++ks)
-#pragma unroll
-      for (int e = 0; e < 8; ++e) {
-        const float v = static_cast<float>(xf[t][ks][e]);
-        ss += v * v;
-      }
-    ss += __shfl_xor(ss, 32, kWave);
-    scale[t] = rsqrtf(ss * (1.0f / D) + eps);
-  }
-  // Make the packed rows opaque here: otherwise the compiler keeps all D fp32 copies from the first sweep alive for
-  // the second one, which does not fit the register file next to the accumulators.
-#pragma unroll
-  for (int t = 0; t < TT; ++t)
-#pragma unroll
-    for (int ks = 0; ks < KS; ++ks) asm volatile("" : "+v"(xf[t][ks]));
-  if (folded) {
-#pragma unroll
-    for (int ks = 0; ks < KS; ++ks)
-#pragma unroll
-      for (int t = 0; t < TT; ++t) {
-#pragma unroll
-        for (int e = 0; e < 8; ++e) xf[t][ks][e] = static_cast<bf16_t>(static_cast<float>(xf[t][ks][e]) * scale[t]);
-        asm volatile("" : "+v"(xf[t][ks]));
-      }
-    return;
-  }
-#pragma unroll
-  for (int ks = 0; ks < KS; ++ks) {
-    const bf16x8 wv = *reinterpret_cast<const bf16x8*>(norm_w_lds + ks * 16 + hh * 8);
-#pragma unroll
-    for (int t = 0; t < TT; ++t) {
-#pragma unroll
-      for (int e = 0; e < 8; ++e)
-        xf[t][ks][e] = static_cast<bf16_t>(static_cast<float>(xf[t][ks][e]) * scale[t] * static_cast<float>(wv[e]));
-      asm volatile("" : "+v"(xf[t][ks]));
-    }
-  }
-}
-
-// rsqrt(mean(x^2) + eps) of the loaded rows, per lane for its token of each tile; the rows themselves stay as they are
-// (the norm's weight is part of the packed layer, the factor goes to the accumulators). The squares are summed two
-// elements per instruction (v_dot2_f32_bf16).
-template <int D, int TT>
-__device__ __forceinline__ void token_rstd(float eps, const bf16x8 (&xf)[TT][D / 16], float (&rstd)[TT]) {
-  typedef __attribute__((__vector_size__(2 * sizeof(__bf16)))) __bf16 bf16x2;
-#pragma unroll
-  for (int t = 0; t < TT; ++t) {
-    float ss = 0.f;
-#pragma unroll
-    for (int ks = 0; ks < D / 16; ++ks)
-#pragma unroll
-      for (int e = 0; e < 8; e += 2) {
-        const bf16x2 pair = {xf[t][ks][e], xf[t][ks][e + 1]};
-        ss = __builtin_amdgcn_fdot2_f32_bf16(pair, pair, ss, false);
-      }
-    ss += __shfl_xor(ss, 32, kWave);
-    rstd[t] = rsqrtf(ss * (1.0f / D) + eps);
-  }
-}
-
-// Bias values of a 64-feature chunk in accumulator order: piece rb*4 + jq holds features rb*32 + jq*8 + hh*4 .. +3.
-__device__ __forceinline__ void read_chunk_bias(const bf16_t* bias_lds, int hh, bf16x4 (&bv)[8]) {
-#pragma unroll
-  for (int q = 0; q < 8; ++q) bv[q] = *reinterpret_cast<const bf16x4*>(bias_lds + (q / 4) * 32 + (q % 4) * 8 + hh * 4);
-}
-
-// The same from a float32 copy of the bias (no widening per value in the epilogue).
-__device__ __forceinline__ void read_chunk_bias(const float* bias_lds, int hh, f32x4 (&bv)[8]) {
-#pragma unroll
-  for (int q = 0; q < 8; ++q) bv[q] = *reinterpret_cast<const f32x4*>(bias_lds + (q / 4) * 32 + (q % 4) * 8 + hh * 4);
-}
-
-// Writes two 32-feature accumulator blocks (64 features) of one 32-token tile into the wavefront's epilogue tile,
-// adding the bias and rounding to bf16. Accumulator register jq*4 + e of lane (l32, hh) is feature jq*8 + hh*4 + e.
-template <typename BiasVec>  // bf16x4 or f32x4 pieces
-__device__ __forceinline__ void tile_to_lds(uint8_t* tile, const f32x16& a0, const f32x16& a1, const BiasVec (&bv)[8],
-                                            int l32, int hh, float scale = 1.0f) {
-#pragma unroll
-  for (int rb = 0; rb < 2; ++rb) {
-#pragma unroll
-    for (int jq = 0; jq < 4; ++jq) {
-      const int col = rb * 32 + jq * 8 + hh * 4;
-      bf16x4 ov;
-#pragma unroll
-      for (int e = 0; e < 4; ++e)
-        ov[e] = static_cast<bf16_t>(fmaf(rb == 0 ? a0[jq * 4 + e] : a1[jq * 4 + e], scale, static_cast<float>(bv[rb * 4 + jq][e])));
-      *reinterpret_cast<bf16x4*>(tile + l32 * kStageRow + col * 2) = ov;
-    }
-  }
-}
-
-// tile_to_lds that also returns the sum of squares of the lane's 32 rounded values (half of its token's 64 features).
-__device__ __forceinline__ float tile_to_lds_sumsq(uint8_t* tile, const f32x16& a0, const f32x16& a1,
-                                                   const bf16x4 (&bv)[8], int l32, int hh, float scale = 1.0f) {
-  float ss = 0.f;
-#pragma unroll
-  for (int rb = 0; rb < 2; ++rb) {
-#pragma unroll
-    for (int jq = 0; jq < 4; ++jq) {
-      const int col = rb * 32 + jq * 8 + hh * 4;
-      bf16x4 ov;
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        ov[e] = static_cast<bf16_t>(fmaf(rb == 0 ? a0[jq * 4 + e] : a1[jq * 4 + e], scale, static_cast<float>(bv[rb * 4 + jq][e])));
-        const float r = static_cast<float>(ov[e]);
-        ss = fmaf(r, r, ss);
-      }
-      *reinterpret_cast<bf16x4*>(tile + l32 * kStageRow + col * 2) = ov;
-    }
-  }
-  return ss;
-}
-
-// Sum of a value and the one held by lane ^ 32.
-__device__ __forceinline__ float half_wave_pair_sum(float v) {
-  const uint32_t u = __builtin_bit_cast(uint32_t, v);
-  const auto r = __builtin_amdgcn_permlane32_swap(u, u, false, false);
-  return __builtin_bit_cast(float, static_cast<uint32_t>(r[0])) + __builtin_bit_cast(float, static_cast<uint32_t>(r[1]));
 }
 
 // Reads the epilogue tile back row-wise (lane -> token 8*i + lane/8, features 8*(lane%8) .. +7), adds the residual
@@ -1405,7 +1111,8 @@ __global__ __launch_bounds__(8 * kWave, 2) void norm_linear_kernel(const TsParam
       if (XF) {
 #pragma unroll
         for (int e = 0; e < 8; ++e) wn[e] = static_cast<bf16_t>(1.0f);
-        if (qk_chunk && p.qk_w != nullptr) wn = *reinterpret_cast<const bf16x8*>(p.qk_w + col8);
+        if (qk_chunk && p.qk_w != nullptr)
+          wn = *reinterpret_cast<const bf16x8*>(2 * chunk < p.qk_chunks ? p.qk_w + col8 : p.qk_wk + (col8 - D));
       }
       const int d0 = rotate ? col8 % p.head_dim : 0;
 #pragma unroll
@@ -1851,9 +1558,12 @@ namespace {
 
 // Query / key extras of the linear kernel; all null / zero for a plain layer.
 struct QkExtras {
-  const void* qk_weight = nullptr;
+  const void* q_weight = nullptr;
+  const void* k_weight = nullptr;
   const void* cos_sin = nullptr;
   float* qk_sumsq = nullptr;
+  float* qk_rstd = nullptr;  // with qk_sumsq: written by the few-token form instead
+  float qk_eps = 0.f;
   int32_t qk_chunks = 0, head_dim = 0, tokens_per_sample = 0;
   bool enabled = false;
 };
@@ -1884,7 +1594,7 @@ int norm_linear_launch(const char* name, const void* x, int64_t ldx, const void*
   if (M * (ldo / 8) + 8 > 0xffffffffLL)
     return set_error(TAAC_ERR_UNSUPPORTED, "%s: the output spans more than 2^32 16-byte pieces", name);
   if (!ptr_ok(x, 15) || !ptr_ok(w, 15) || !ptr_ok(out, 15) || !ptr_ok(residual, 15) || !ptr_ok(norm_weight, 15) ||
-      !ptr_ok(bias, 15) || !ptr_ok(packed_weights, 15) || !ptr_ok(qk.qk_weight, 15) || !ptr_ok(qk.cos_sin, 15) ||
+      !ptr_ok(bias, 15) || !ptr_ok(packed_weights, 15) || !ptr_ok(qk.q_weight, 15) || !ptr_ok(qk.k_weight, 15) || !ptr_ok(qk.cos_sin, 15) ||
       !ptr_ok(qk.qk_sumsq, 3))
     return set_error(TAAC_ERR_UNSUPPORTED, "%s: tensor base pointers must be 16-byte aligned", name);
   // behind the 16-bit bias and norm weight: the query / key epilogue's row table, or the float32 copy of the bias
@@ -1912,13 +1622,20 @@ int norm_linear_launch(const char* name, const void* x, int64_t ldx, const void*
   p.n_rows = n_rows;
   p.x_rows = x_rows;
   p.out_plane_shift = out_plane == 32 ? 5 : (out_plane == 64 ? 6 : 0);
-  p.qk_w = static_cast<const bf16_t*>(qk.qk_weight);
+  p.qk_w = static_cast<const bf16_t*>(qk.q_weight);
+  p.qk_wk = static_cast<const bf16_t*>(qk.k_weight);
+  p.qk_rstd = qk.qk_rstd;
+  p.qk_eps = qk.qk_eps;
   p.cos_sin = static_cast<const bf16_t*>(qk.cos_sin);
   p.qk_sumsq = qk.qk_sumsq;
   p.qk_chunks = qk.qk_chunks;
   p.head_dim = qk.head_dim;
   p.tokens_per_sample = qk.tokens_per_sample;
   hipStream_t s = as_stream(stream);
+  const bool qk_transform = qk.enabled && (qk.q_weight != nullptr || qk.cos_sin != nullptr);
+  if (dense_few_rows(M, K) && packed_weights && (norm_weight == nullptr || norm_folded))
+    return norm_linear_small(p, K, qk_transform ? 2 : (qk.enabled ? 1 : 0), s, name);
+  p.qk_rstd = nullptr;
   // Without a residual two token tiles per wavefront fit the register file: every weight fragment read from LDS then
   // feeds two MFMAs, which halves the LDS reads (and their share of the power budget) per token.
   const int tt = residual ? 1 : 2;
@@ -1941,7 +1658,6 @@ int norm_linear_launch(const char* name, const void* x, int64_t ldx, const void*
     hipLaunchKernelGGL((norm_linear_kernel<KK, TT, RR, QQ>), dim3(grid), dim3(8 * kWave), lds_bytes, s, p);       \
     return check_launch(name);                                                                                    \
   } while (0)
-  const bool qk_transform = qk.enabled && (qk.qk_weight != nullptr || qk.cos_sin != nullptr);
   if (K == 256) {
     if (qk_transform) TAAC_LIN_LAUNCH(256, 2, false, 2);
     if (qk.enabled) TAAC_LIN_LAUNCH(256, 2, false, 1);
@@ -2006,13 +1722,16 @@ namespace taac {
 // taac_norm_linear_qk_fwd (packed weights) writing q | k | v as per-head planes like taac_norm_linear_heads_fwd.
 int norm_linear_qk_heads(const void* x, int64_t ldx, const void* norm_weight, float eps, const void* bias,
                          const void* packed_weights, void* out, int64_t M, int32_t d_model, int32_t num_heads,
-                         int32_t tokens_per_sample, const void* qk_weight, const void* cos_sin, float* qk_sumsq,
-                         const int32_t* rows, const int32_t* n_rows, int norm_folded, void* stream) {
+                         int32_t tokens_per_sample, const void* q_weight, const void* k_weight, const void* cos_sin,
+                         float* qk_sumsq, float* qk_rstd, const int32_t* rows, const int32_t* n_rows, int norm_folded, void* stream) {
   QkExtras qk;
   qk.enabled = true;
-  qk.qk_weight = qk_weight;
+  qk.q_weight = q_weight;
+  qk.k_weight = k_weight;
   qk.cos_sin = cos_sin;
   qk.qk_sumsq = qk_sumsq;
+  qk.qk_rstd = qk_rstd;
+  qk.qk_eps = eps;
   qk.qk_chunks = 2 * d_model / kNC;
   qk.head_dim = d_model / num_heads;
   qk.tokens_per_sample = tokens_per_sample;
@@ -2031,6 +1750,14 @@ int attn_out_ffn_readout(const void* attn, int64_t ld_attn, int attn_plane, cons
   return ffn_entry("taac_backbone_fwd", attn, ld_attn, out_bias, packed_out_weights, norm_weight, eps, nullptr, b_up, nullptr,
                    b_down, packed_ffn_weights, residual, ldr, out, ldo, M, D, F, 1, rows, n_rows, nullptr, norm_folded,
                    stream, nullptr, 0, true, attn_plane, head_w, token_dots);
+}
+
+// Whether a projection over at most M rows of D features runs as the few-token kernel. Measured for q | k | v (launches
+// back to back, few-token / persistent kernel, us): D = 256 - 512 rows 6.0 / 13.6, 4096 9.9 / 14.1, 8192 14.4 / 15.6,
+// 16384 24.5 / 21.4; D = 128 - 512 rows 3.8 / 8.7, 8192 6.3 / 9.2, 16384 9.6 / 10.4, 24576 12.6 / 12.4. Below the line a tile's
+// latency chain decides, above it the weights, which every 32-token workgroup fetches from L2 for itself.
+bool dense_few_rows(int64_t M, int32_t D) {
+  return test_max_workgroups() == 0 && M * D <= 10240 * 256;  // taac_test_hooks: a capped grid keeps the persistent kernels
 }
 
 // Whether the kernels take the activation's constants from the packed weights at this shape: the gated form with the
@@ -2067,7 +1794,8 @@ extern "C" int taac_norm_linear_qk_fwd(const void* x, int64_t ldx, const void* n
     return set_error(TAAC_ERR_INVALID_VALUE, "%s: nothing to do for the query and key features", name);
   QkExtras qk;
   qk.enabled = true;
-  qk.qk_weight = qk_weight;
+  qk.q_weight = qk_weight;
+  qk.k_weight = qk_weight ? static_cast<const bf16_t*>(qk_weight) + d_model : nullptr;
   qk.cos_sin = cos_sin;
   qk.qk_sumsq = qk_sumsq;
   qk.qk_chunks = 2 * d_model / kNC;
