@@ -39,6 +39,7 @@ HIPCC_FLAGS = (
 EXTRA_FLAGS = {
     "attention.hip": ("-mllvm", "-amdgpu-mfma-vgpr-form=1"),
     "attention_bwd.hip": ("-mllvm", "-amdgpu-mfma-vgpr-form=1"),
+    "ffn_small.hip": ("-mllvm", "-amdgpu-mfma-vgpr-form=1"),
 }
 
 

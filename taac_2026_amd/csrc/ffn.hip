@@ -1354,6 +1354,13 @@ extern "C" int taac_linear_pack_weights_norm(const void* w, const void* norm_wei
 namespace taac {
 namespace {
 
+// Whether the gated feed-forward over at most M rows of D features runs as the few-token kernel: as long as its 32-token
+// workgroups fit the chip in one round. Measured with the out projection in front, launches back to back, few-token /
+// persistent kernel, us: D = 256, F = 1024 - 512 rows 21.5 / 49.9, 8192 27.8 / 55.6, 16384 53.8 / 57.7, 24576 72.5 / 58.2;
+// F = 512 - 8192 18.8 / 34.7, 16384 34.4 / 36.4; D = 128 (two workgroups per compute unit), F = 512 - 512 rows 9.2 / 19.5,
+// 16384 16.8 / 21.9, 24576 23.0 / 22.2.
+bool ffn_few_rows(int64_t M, int32_t D) { return test_max_workgroups() == 0 && M * D <= 8192 * 256; }
+
 // Shared body of taac_swiglu_ffn_fwd and taac_attn_out_ffn_fwd (out_packed != null: the attention output projection
 // runs in front; x is then the attention output and residual the block input).
 int ffn_entry(const char* name, const void* x, int64_t ldx, const void* out_bias, const void* out_packed,
@@ -1440,6 +1447,10 @@ int ffn_entry(const char* name, const void* x, int64_t ldx, const void* out_bias
   if (p.units <= 0) return set_error(TAAC_ERR_LAUNCH, "%s: cannot query the device", name);
   if (const int limit = test_max_workgroups(); limit > 0 && limit < p.units) p.units = limit;  // taac_test_hooks
   hipStream_t s = as_stream(stream);
+  if (ffn_few_rows(M, D) && glu && update_gate == nullptr && packed_weights && (norm_weight == nullptr || norm_folded)) {
+    const int rc = swiglu_ffn_small(p, D, with_proj, act_folded, s, name);
+    if (rc != 1) return rc;
+  }
 #define TAAC_FFN_LAUNCH(DD, TT, NW, CPB, DEFER, ...)                                                         \
   return launch_ts(swiglu_ffn_kernel<DD, TT, NW, CPB, DEFER, __VA_ARGS__>, p, NW * kWave, NW * 32 * TT,      \
                    static_cast<size_t>((DEFER ? 3 : 2) * CPB * (KS + MB)) * kFrag + bias_bytes, s, name)

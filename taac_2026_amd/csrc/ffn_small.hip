@@ -159,6 +159,243 @@ __global__ __launch_bounds__(D, 2) void norm_linear_small_kernel(const TsParams 
   }
 }
 
+// ------------------------------------------------------------------------------------------------------------------
+// The feed-forward half for few tokens: [out projection + residual ->] RMSNorm -> up -> SiLU-gate -> down -> + residual of
+// 32 tokens per workgroup (the products, blobs and roundings of swiglu_ffn_kernel). Four wavefronts share the tokens and divide
+// the HIDDEN units: wavefront w takes the 16-unit chunks w, w + 4, ...; each holds a [D, 32] partial of the down projection
+// in its accumulators, and the four partials meet once, in LDS, where every wavefront adds up its share of the features in a
+// fixed order. The projection in front is divided by output features; its result reaches the other wavefronts through LDS.
+// A wavefront is alone on its SIMD and reads its fragments from L2 through a ring as deep as a chunk (24 KB in flight at
+// D = 256, 96 KB per compute unit).
+// Bound: the 1.6 MB of weights a compute unit pulls from L2 for its 32 tokens (0.7 us per chunk and wavefront, 64 bytes per
+// clock of the compute unit: 11 us) behind and in front of which lie 9.5 us of latency chains; the persistent kernel has one
+// or two of its eight wavefronts at work there and takes 50 us whatever the number of tokens (512 tokens, D = 256, F = 1024:
+// 49.9 -> 21.5 us; 8192 tokens: 55.6 -> 27.8; its line is at ffn_few_rows).
+// LDS: [4 partials of 32 x D floats][x1 (32 padded rows of D bf16)][first-layer bias 2F][4 x 32 row sums]
+// ------------------------------------------------------------------------------------------------------------------
+template <int D, bool OUTP, bool FOLD>
+__global__ __launch_bounds__(4 * kWave, 1) void swiglu_ffn_small_kernel(const TsParams p) {
+  constexpr int NW = 4;
+  constexpr int KS = D / 16, MB = D / 32;
+  constexpr int CFRAG = KS + MB;
+  constexpr int MBW = MB / NW;              // 32-feature blocks a wavefront projects in front and adds up behind
+  constexpr int kRow = D * 2 + 16;          // bytes per row of the x1 tile
+  constexpr int kPart = MB * 4 * kWave * 16;  // bytes of one partial
+  extern __shared__ __attribute__((aligned(1024))) uint8_t smem[];
+  uint8_t* x1_lds = smem + NW * kPart;
+  bf16_t* bias_lds = reinterpret_cast<bf16_t*>(x1_lds + 32 * kRow);
+  float* sums = reinterpret_cast<float*>(bias_lds + 2 * p.F);  // [NW][32]
+
+  const int tid = threadIdx.x;
+  const int wave = __builtin_amdgcn_readfirstlane(tid / kWave);
+  const int lane = tid % kWave;
+  const int l32 = lane % 32, hh = lane / 32;
+  const int F = p.F;
+  const int nchunks = F / kHU;
+
+  // weights of the projection first: they depend on nothing
+  [[maybe_unused]] bf16x8 w0[OUTP ? MBW * KS : 1];
+  if constexpr (OUTP) {
+    const char* src = reinterpret_cast<const char*>(p.w0) + static_cast<int64_t>(wave * MBW * KS) * kFrag;
+#pragma unroll
+    for (int i = 0; i < MBW * KS; ++i) w0[i] = *reinterpret_cast<const bf16x8*>(src + i * kFrag + lane * 16);
+    __builtin_amdgcn_sched_barrier(0);
+  }
+  const int64_t count = token_count(p);
+  const int64_t tok0 = static_cast<int64_t>(blockIdx.x) * 32;
+  if (tok0 >= count) return;  // whole workgroup
+  TokenRows<1> xr, orow;
+  xr.request(p.x_rows != nullptr ? p.x_rows : p.rows, count, [&](int) { return tok0 + l32; });
+  orow.request(p.rows, count, [&](int) { return tok0 + l32; });
+  // first-layer bias, gated half first; FOLD: with the constants the packed layer carries
+  for (int i = tid * 8; i < 2 * F; i += NW * kWave * 8) {
+    const bool gated = i < F;  // F is a multiple of 32: a piece lies in one half
+    bf16x8 v;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) v[e] = static_cast<bf16_t>(0.f);
+    if (p.b1 != nullptr) v = *reinterpret_cast<const bf16x8*>(p.b1 + (gated == (p.gate_first != 0) ? i % F : F + i % F));
+    if constexpr (FOLD) {
+#pragma unroll
+      for (int e = 0; e < 8; ++e) v[e] = static_cast<bf16_t>(static_cast<float>(v[e]) * (gated ? kFoldGate : kFoldValue));
+    }
+    *reinterpret_cast<bf16x8*>(bias_lds + i) = v;
+  }
+  xr.arrive();
+  orow.arrive();
+  const int64_t xrow[1] = {xr.row(0)};
+  const int64_t row = orow.row(0);  // of token l32 in residual / out
+  bf16x8 xf[1][KS];
+  load_token_rows_at<D, 1>(p, xrow, hh, xf);
+  const char* ffn_blob = reinterpret_cast<const char*>(p.w1) + lane * 16;
+  bf16x8 ring[CFRAG];
+  auto load_chunk_frag = [&](int chunk, int i) {
+    return *reinterpret_cast<const bf16x8*>(ffn_blob + (static_cast<int64_t>(chunk) * CFRAG + i) * kFrag);
+  };
+  const int first = wave < nchunks ? wave : nchunks - 1;
+
+  if constexpr (OUTP) {
+    bf16x4 hv[MBW][4], b0v[MBW][4];  // block input and projection bias of the lane's features, in accumulator order
+#pragma unroll
+    for (int m = 0; m < MBW; ++m)
+#pragma unroll
+      for (int jq = 0; jq < 4; ++jq) {
+        const int col = (wave * MBW + m) * 32 + jq * 8 + hh * 4;
+        hv[m][jq] = *reinterpret_cast<const bf16x4*>(p.residual + row * p.ldr + col);
+        if (p.b0 != nullptr) {
+          b0v[m][jq] = *reinterpret_cast<const bf16x4*>(p.b0 + col);
+        } else {
+#pragma unroll
+          for (int e = 0; e < 4; ++e) b0v[m][jq][e] = static_cast<bf16_t>(0.f);
+        }
+      }
+    float ss = 0.f;
+#pragma unroll
+    for (int m = 0; m < MBW; ++m) {
+      f32x16 acc;
+#pragma unroll
+      for (int j = 0; j < 16; ++j) acc[j] = 0.f;
+#pragma unroll
+      for (int ks = 0; ks < KS; ++ks) acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(w0[m * KS + ks], xf[0][ks], acc, 0, 0, 0);
+#pragma unroll
+      for (int jq = 0; jq < 4; ++jq) {
+        bf16x4 x1;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const float lin = static_cast<float>(static_cast<bf16_t>(acc[jq * 4 + e] + static_cast<float>(b0v[m][jq][e])));
+          x1[e] = static_cast<bf16_t>(lin + static_cast<float>(hv[m][jq][e]));
+          const float r = static_cast<float>(x1[e]);
+          ss = fmaf(r, r, ss);
+        }
+        *reinterpret_cast<bf16x4*>(x1_lds + l32 * kRow + ((wave * MBW + m) * 32 + jq * 8 + hh * 4) * 2) = x1;
+      }
+    }
+    ss = half_wave_pair_sum(ss);
+    if (hh == 0) sums[wave * 32 + l32] = ss;
+  }
+#pragma unroll
+  for (int i = 0; i < CFRAG; ++i) ring[i] = load_chunk_frag(first, i);
+  __builtin_amdgcn_sched_barrier(0);
+  __syncthreads();
+  if constexpr (OUTP) {
+    float total = 0.f;
+#pragma unroll
+    for (int w = 0; w < NW; ++w) total += sums[w * 32 + l32];
+    const float scale = p.norm_w != nullptr ? rsqrtf(total * (1.0f / D) + p.eps) : 1.0f;
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks) {
+      xf[0][ks] = *reinterpret_cast<const bf16x8*>(x1_lds + l32 * kRow + (ks * 16 + hh * 8) * 2);
+#pragma unroll
+      for (int e = 0; e < 8; ++e) xf[0][ks][e] = static_cast<bf16_t>(static_cast<float>(xf[0][ks][e]) * scale);
+    }
+  } else if (p.norm_w != nullptr) {
+    float rstd[1];
+    token_rstd<D, 1>(p.eps, xf, rstd);
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks)
+#pragma unroll
+      for (int e = 0; e < 8; ++e) xf[0][ks][e] = static_cast<bf16_t>(static_cast<float>(xf[0][ks][e]) * rstd[0]);
+  }
+
+  f32x16 oacc[MB];
+#pragma unroll
+  for (int mb = 0; mb < MB; ++mb)
+#pragma unroll
+    for (int j = 0; j < 16; ++j) oacc[mb][j] = 0.f;
+  for (int chunk = wave; chunk < nchunks; chunk += NW) {
+    const int next = chunk + NW < nchunks ? chunk + NW : chunk;  // the last chunk is requested once more, and not used
+    const bf16x8 bg = *reinterpret_cast<const bf16x8*>(bias_lds + chunk * kHU + hh * 8);
+    const bf16x8 bu = *reinterpret_cast<const bf16x8*>(bias_lds + F + chunk * kHU + hh * 8);
+    f32x16 gu;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      gu[e] = static_cast<float>(bg[e]);
+      gu[8 + e] = static_cast<float>(bu[e]);
+    }
+    static_for<KS>([&](auto ic) {
+      constexpr int i = decltype(ic)::value;
+      gu = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ring[i], xf[0][i], gu, 0, 0, 0);
+      ring[i] = load_chunk_frag(next, i);
+      __builtin_amdgcn_sched_barrier(0);
+    });
+    bf16x8 hb;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      if constexpr (FOLD)
+        hb[e] = static_cast<bf16_t>(gu[e] * gu[8 + e] * __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(gu[e])));
+      else
+        hb[e] = static_cast<bf16_t>(silu_f(gu[e]) * gu[8 + e]);
+    }
+    static_for<MB>([&](auto ic) {
+      constexpr int i = decltype(ic)::value;
+      oacc[i] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ring[KS + i], hb, oacc[i], 0, 0, 0);
+      ring[KS + i] = load_chunk_frag(next, KS + i);
+      __builtin_amdgcn_sched_barrier(0);
+    });
+  }
+
+  // ---- the four partials: [wavefront][feature block][register quad][lane] -------------------------------------------------
+#pragma unroll
+  for (int mb = 0; mb < MB; ++mb)
+#pragma unroll
+    for (int jq = 0; jq < 4; ++jq) {
+      const f32x4 v = {oacc[mb][jq * 4], oacc[mb][jq * 4 + 1], oacc[mb][jq * 4 + 2], oacc[mb][jq * 4 + 3]};
+      *reinterpret_cast<f32x4*>(smem + wave * kPart + ((mb * 4 + jq) * kWave + lane) * 16) = v;
+    }
+  __syncthreads();
+  const bool live = tok0 + l32 < count;
+  float hdot = 0.f;
+#pragma unroll
+  for (int m = 0; m < MBW; ++m)
+#pragma unroll
+    for (int jq = 0; jq < 4; ++jq) {
+      const int mb = wave * MBW + m;
+      const int col = mb * 32 + jq * 8 + hh * 4;
+      f32x4 s = *reinterpret_cast<const f32x4*>(smem + ((mb * 4 + jq) * kWave + lane) * 16);
+#pragma unroll
+      for (int w = 1; w < NW; ++w) {
+        const f32x4 v = *reinterpret_cast<const f32x4*>(smem + w * kPart + ((mb * 4 + jq) * kWave + lane) * 16);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) s[e] += v[e];
+      }
+      if (p.b2 != nullptr) {
+        const bf16x4 b = *reinterpret_cast<const bf16x4*>(p.b2 + col);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) s[e] += static_cast<float>(b[e]);
+      }
+      bf16x4 o;
+      if constexpr (OUTP) {  // x1 + down, rounded once
+        const bf16x4 x1 = *reinterpret_cast<const bf16x4*>(x1_lds + l32 * kRow + col * 2);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) o[e] = static_cast<bf16_t>(s[e] + static_cast<float>(x1[e]));
+      } else {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) o[e] = static_cast<bf16_t>(s[e]);
+        if (p.residual != nullptr) {
+          const bf16x4 r = *reinterpret_cast<const bf16x4*>(p.residual + row * p.ldr + col);
+#pragma unroll
+          for (int e = 0; e < 4; ++e) o[e] = static_cast<bf16_t>(static_cast<float>(o[e]) + static_cast<float>(r[e]));
+        }
+      }
+      if (live) *reinterpret_cast<bf16x4*>(p.out + row * p.ldo + col) = o;
+      if (p.head_w != nullptr) {
+        const bf16x4 hw = *reinterpret_cast<const bf16x4*>(p.head_w + col);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) hdot = fmaf(static_cast<float>(o[e]), static_cast<float>(hw[e]), hdot);
+      }
+    }
+  if (p.head_w != nullptr) {
+    hdot = half_wave_pair_sum(hdot);
+    if (hh == 0) sums[wave * 32 + l32] = hdot;
+    __syncthreads();
+    if (wave == 0 && hh == 0 && live) {
+      float d = 0.f;
+#pragma unroll
+      for (int w = 0; w < NW; ++w) d += sums[w * 32 + l32];
+      p.token_dots[row] = d;
+    }
+  }
+}
+
 }  // namespace
 
 int norm_linear_small(const TsParams& p, int32_t K, int qk_mode, hipStream_t s, const char* name) {
@@ -178,6 +415,31 @@ int norm_linear_small(const TsParams& p, int32_t K, int qk_mode, hipStream_t s, 
   if (qk_mode == 1) TAAC_SMALL(128, false, 1);
   if (p.residual != nullptr) TAAC_SMALL(128, true, 0);
   TAAC_SMALL(128, false, 0);
+#undef TAAC_SMALL
+}
+
+int swiglu_ffn_small(const TsParams& p, int32_t D, bool with_proj, bool act_folded, hipStream_t s, const char* name) {
+  const size_t lds_bytes = static_cast<size_t>(4) * 32 * D * 4 + 32 * (D * 2 + 16) + static_cast<size_t>(2) * p.F * 2 + 4 * 32 * 4;
+  if (lds_bytes > 160 * 1024) return 1;
+  const dim3 grid(static_cast<uint32_t>((p.M + 31) / 32));
+#define TAAC_SMALL(DD, OO, FF)                                                                                        \
+  do {                                                                                                                \
+    if (hipFuncSetAttribute(reinterpret_cast<const void*>(swiglu_ffn_small_kernel<DD, OO, FF>),                       \
+                            hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds_bytes)) != hipSuccess)   \
+      return set_error(TAAC_ERR_LAUNCH, "%s: cannot reserve %zu bytes of LDS", name, lds_bytes);                      \
+    hipLaunchKernelGGL((swiglu_ffn_small_kernel<DD, OO, FF>), grid, dim3(4 * kWave), lds_bytes, s, p);                \
+    return check_launch(name);                                                                                        \
+  } while (0)
+#define TAAC_SMALL_D(DD)                        \
+  do {                                          \
+    if (with_proj && act_folded) TAAC_SMALL(DD, true, true);   \
+    if (with_proj) TAAC_SMALL(DD, true, false);                \
+    if (act_folded) TAAC_SMALL(DD, false, true);               \
+    TAAC_SMALL(DD, false, false);                              \
+  } while (0)
+  if (D == 256) TAAC_SMALL_D(256);
+  TAAC_SMALL_D(128);
+#undef TAAC_SMALL_D
 #undef TAAC_SMALL
 }
 

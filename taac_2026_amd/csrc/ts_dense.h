@@ -67,6 +67,9 @@ struct TsParams {
 
 // The few-token form of the projection (ffn_small.hip): packed weights, the norm in front folded into them or absent.
 int norm_linear_small(const TsParams& p, int32_t K, int qk_mode, hipStream_t s, const char* name);
+// The few-token form of the gated feed-forward (with_proj: the out projection in front), same conditions; 1 when the shape does
+// not fit its LDS.
+int swiglu_ffn_small(const TsParams& p, int32_t D, bool with_proj, bool act_folded, hipStream_t s, const char* name);
 
 namespace {
 

@@ -6,7 +6,8 @@ from __future__ import annotations
 import pytest
 import torch
 
-from taac_2026_amd.api import norm_linear, norm_linear_heads, qkv_projection, valid_rows
+from taac_2026_amd.api import (attention_out_ffn, attention_out_ffn_heads, norm_linear, norm_linear_heads, qkv_projection,
+                               swiglu_ffn, valid_rows)
 
 pytestmark = pytest.mark.gpu
 
@@ -64,3 +65,34 @@ def test_query_key_epilogue_equals_the_persistent_kernel(device, test_hooks, d_m
                 small, large = _both(test_hooks, lambda: norm_linear_heads(x, w, b, head_dim=d_model // heads, norm_weight=nw,
                                                                            token_rows=index))
                 assert torch.equal(small, large)
+
+
+@pytest.mark.parametrize("m,d,f", [(1, 256, 32), (33, 128, 32), (31, 256, 96), (64, 128, 512), (100, 256, 1024), (8192, 256, 64)])
+@pytest.mark.parametrize("gate_first", [True, False])
+def test_feed_forward_matches_the_persistent_kernel(device, test_hooks, m, d, f, gate_first):
+    """The hidden units are added up in another order (four partial sums instead of one). Bound: the reordering moves a sum by
+    about 2**-20 of its terms, which flips roundings to bf16: of the layer output before the residual joins (magnitude
+    below 4 here, one step = 2**-6 at most, whole when the residual cancels the value) and of the result (one step, 2**-7
+    relative); a flipped step of a single normalised input or hidden unit is worth less than 2**-9 in a sum."""
+    g = torch.Generator().manual_seed(m + f)
+    x, res, nw = _bf16(g, m, d).to(device), _bf16(g, m, d).to(device), (1 + _bf16(g, d, scale=0.1)).to(device)
+    wo, bo = _bf16(g, d, d, scale=d ** -0.5).to(device), _bf16(g, d, scale=0.1).to(device)
+    wu, bu = _bf16(g, 2 * f, d, scale=d ** -0.5).to(device), _bf16(g, 2 * f, scale=0.1).to(device)
+    wd, bd = _bf16(g, d, f, scale=f ** -0.5).to(device), _bf16(g, d, scale=0.1).to(device)
+
+    def check(call):
+        small, large = _both(test_hooks, call)
+        torch.testing.assert_close(small.float(), large.float(), rtol=2 ** -7, atol=2 ** -6)
+
+    with torch.no_grad():
+        for fold in (True, False):
+            check(lambda: swiglu_ffn(x, wu, bu, wd, bd, residual=res, gate_first=gate_first, norm_weight=nw, fold_activation=fold))
+            check(lambda: swiglu_ffn(x, wu, None, wd, None, gate_first=gate_first, fold_activation=fold))
+            if gate_first:
+                check(lambda: attention_out_ffn(x, wo, bo, res, wu, bu, wd, bd, norm_weight=nw, fold_activation=fold))
+                planes = x.view(m, -1, 32).permute(1, 0, 2).contiguous()
+                assert torch.equal(attention_out_ffn_heads(planes, wo, bo, res, wu, bu, wd, bd, norm_weight=nw, fold_activation=fold),
+                                   attention_out_ffn(x, wo, bo, res, wu, bu, wd, bd, norm_weight=nw, fold_activation=fold))
+        held = res.clone()
+        attention_out_ffn(x, wo, bo, held, wu, bu, wd, bd, norm_weight=nw, out=held)
+        assert torch.equal(held, attention_out_ffn(x, wo, bo, res, wu, bu, wd, bd, norm_weight=nw))
