@@ -4,6 +4,7 @@
 #include <vector>
 
 #include "common.h"
+#include "row_index.h"
 
 namespace taac {
 namespace {
@@ -83,25 +84,8 @@ __global__ __launch_bounds__(kBlock) void token_dots_head_kernel(const float* __
   }
 }
 
-// Number of valid tokens of sample b: its clamped length, or the set bits among the first T of its bit row.
-__device__ __forceinline__ int32_t valid_count(const int32_t* __restrict__ lengths, const uint32_t* __restrict__ bits,
-                                               int b, int T) {
-  if (lengths != nullptr) {
-    const int32_t len = lengths[b];
-    return len < 0 ? 0 : (len > T ? T : len);
-  }
-  const int wpr = (T + 31) / 32;
-  int32_t n = 0;
-  for (int w = 0; w < wpr; ++w) {
-    uint32_t word = bits[static_cast<int64_t>(b) * wpr + w];
-    if (w == wpr - 1 && T % 32 != 0) word &= (1u << (T % 32)) - 1u;
-    n += __popc(word);
-  }
-  return n;
-}
-
-// Exclusive prefix sums of the per-sample valid counts (one workgroup; B is walked in slabs of kBlock with a running
-// carry).
+// Batches of more than kMaxScanBatch samples: exclusive prefix sums of the per-sample valid counts (one workgroup; B is walked
+// in slabs of kBlock with a running carry), then the rows (valid_rows_kernel / valid_rows_bits_kernel).
 __global__ __launch_bounds__(kBlock) void length_offsets_kernel(const int32_t* __restrict__ lengths,
                                                                 const uint32_t* __restrict__ bits, int B, int T,
                                                                 int32_t* __restrict__ offsets,
@@ -110,7 +94,7 @@ __global__ __launch_bounds__(kBlock) void length_offsets_kernel(const int32_t* _
   int32_t carry = 0;
   for (int base = 0; base < B; base += kBlock) {
     const int b = base + threadIdx.x;
-    const int32_t len = b < B ? valid_count(lengths, bits, b, T) : 0;
+    const int32_t len = b >= B ? 0 : (lengths != nullptr ? clamped_length(lengths, b, T) : valid_bit_count(bits, b, T));
     s_scan[threadIdx.x] = len;
     __syncthreads();
     for (int step = 1; step < kBlock; step <<= 1) {  // inclusive scan, Hillis-Steele
@@ -153,6 +137,17 @@ __global__ __launch_bounds__(kBlock) void valid_rows_bits_kernel(const uint32_t*
   int32_t rank = __popc(word & ((1u << (t % 32)) - 1u));
   for (int w = 0; w < t / 32; ++w) rank += __popc(row[w]);
   rows[offsets[b] + rank] = b * T + t;
+}
+
+// The index in one launch (see row_index.h).
+__global__ __launch_bounds__(kRowThreads) void valid_rows_scan_kernel(const int32_t* __restrict__ lengths, int B, int T,
+                                                                      int32_t* __restrict__ rows, int32_t* __restrict__ n_rows) {
+  write_valid_rows(lengths, B, T, blockIdx.x, rows, n_rows);
+}
+__global__ __launch_bounds__(kRowThreads) void valid_rows_bits_scan_kernel(const uint32_t* __restrict__ bits, int B, int T,
+                                                                           int32_t* __restrict__ rows,
+                                                                           int32_t* __restrict__ n_rows) {
+  write_valid_rows_bits(bits, B, T, blockIdx.x, rows, n_rows);
 }
 
 // front_rows[i] = b * T + (i - offsets[b]) for token i of sample b = rows[i] / T; lengths[b] = offsets[b + 1] - offsets[b].
@@ -214,31 +209,6 @@ __global__ __launch_bounds__(kBlock) void mask_front_bits_kernel(const uint32_t*
       if (lane < 2 && j0 / 32 + lane < wpr) dst[j0 / 32 + lane] = static_cast<uint32_t>(bits >> (32 * lane));
     }
   }
-}
-
-// prod[d] = wq[d] * wk[d] in fp32: the weights of a query and a key norm act on an attention score only through their
-// product, which the attention kernel applies to the query features.
-__global__ __launch_bounds__(kBlock) void weight_product_kernel(const bf16_t* __restrict__ wq,
-                                                                const bf16_t* __restrict__ wk,
-                                                                float* __restrict__ prod, int D) {
-  const int d = blockIdx.x * kBlock + threadIdx.x;
-  if (d < D) prod[d] = static_cast<float>(wq[d]) * static_cast<float>(wk[d]);
-}
-
-// Zero-fills the rows of the padded positions of x [B, T, D] (16 bytes per thread).
-__global__ __launch_bounds__(kBlock) void zero_padded_rows_kernel(bf16_t* __restrict__ x,
-                                                                  const int32_t* __restrict__ lengths, int T, int D) {
-  const int b = blockIdx.y;
-  int32_t len = lengths[b];
-  len = len < 0 ? 0 : (len > T ? T : len);
-  const int c8n = D / 8;
-  const int64_t idx = static_cast<int64_t>(blockIdx.x) * kBlock + threadIdx.x;
-  const int64_t t = len + idx / c8n;
-  if (t >= T) return;
-  bf16x8 z;
-#pragma unroll
-  for (int e = 0; e < 8; ++e) z[e] = static_cast<bf16_t>(0.f);
-  *reinterpret_cast<bf16x8*>(x + (static_cast<int64_t>(b) * T + t) * D + (idx % c8n) * 8) = z;
 }
 
 }  // namespace
@@ -393,6 +363,11 @@ extern "C" int taac_valid_rows(const int32_t* key_lengths, int32_t B, int32_t T,
     return set_error(TAAC_ERR_UNSUPPORTED, "%s: B * T must fit 32-bit row numbers", name);
   if (!rows || !n_rows || (B > 0 && !key_lengths)) return set_error(TAAC_ERR_INVALID_VALUE, "%s: null pointer", name);
   if (B > 65535) return set_error(TAAC_ERR_UNSUPPORTED, "%s: at most 65535 samples", name);
+  if (B > 0 && T > 0 && B <= kMaxScanBatch) {
+    const uint32_t units = static_cast<uint32_t>(B) * ((T + kRowThreads - 1) / kRowThreads);
+    hipLaunchKernelGGL(valid_rows_scan_kernel, dim3(units), dim3(kRowThreads), 0, as_stream(stream), key_lengths, B, T, rows, n_rows);
+    return check_launch(name);
+  }
   int32_t* offsets = rows + static_cast<int64_t>(B) * T;
   hipLaunchKernelGGL(length_offsets_kernel, dim3(1), dim3(kBlock), 0, as_stream(stream), key_lengths,
                      static_cast<const uint32_t*>(nullptr), B, T, offsets, n_rows);
@@ -411,6 +386,11 @@ extern "C" int taac_valid_rows_from_bits(const uint32_t* valid_bits, int32_t B, 
     return set_error(TAAC_ERR_UNSUPPORTED, "%s: B * T must fit 32-bit row numbers", name);
   if (!rows || !n_rows || (B > 0 && T > 0 && !valid_bits)) return set_error(TAAC_ERR_INVALID_VALUE, "%s: null pointer", name);
   if (B > 65535) return set_error(TAAC_ERR_UNSUPPORTED, "%s: at most 65535 samples", name);
+  if (B > 0 && T > 0 && B <= kMaxScanBatch) {
+    const uint32_t units = static_cast<uint32_t>(B) * ((T + kRowThreads - 1) / kRowThreads);
+    hipLaunchKernelGGL(valid_rows_bits_scan_kernel, dim3(units), dim3(kRowThreads), 0, as_stream(stream), valid_bits, B, T, rows, n_rows);
+    return check_launch(name);
+  }
   int32_t* offsets = rows + static_cast<int64_t>(B) * T;
   hipLaunchKernelGGL(length_offsets_kernel, dim3(1), dim3(kBlock), 0, as_stream(stream),
                      static_cast<const int32_t*>(nullptr), valid_bits, B, T, offsets, n_rows);
@@ -448,10 +428,10 @@ inline int64_t packed_block_bytes(int32_t D, int32_t F) {
   return align256(static_cast<int64_t>(3) * D * D * 2) + align256(static_cast<int64_t>(D) * D * 2) +
          align256(static_cast<int64_t>(3) * D * F * 2);
 }
-// Query / key norm scratch of the fused path: per-chunk sums of squares [2D / 64, M], factors [2, M], the
-// concatenated query | key norm weights [2D].
-inline int64_t qk_norm_bytes(int64_t M, int32_t D) {
-  return align256((2 * D / 64) * M * 4) + align256(2 * M * 4) + align256(static_cast<int64_t>(D) * 4);
+// Query / key norm scratch of the fused path: per-chunk sums of squares [2D / 64, M], factors [2, M], per block the product
+// of the query and key norm weights (fp32 [D]) or, with a rotary table, the two weights side by side (bf16 [2D]).
+inline int64_t qk_norm_bytes(int64_t M, int32_t D, int32_t n_blocks) {
+  return align256((2 * D / 64) * M * 4) + align256(2 * M * 4) + align256(static_cast<int64_t>(D) * 4 * n_blocks);
 }
 // FP8 mode (TAAC_BACKBONE_FP8; D = 256, F a multiple of 64): per block the e4m3 qkv / out weights, the packed feed-forward
 // blob and 8 scales (weights: qkv, out, up, down; activations: block input, attention output, feed-forward input, gated
@@ -474,7 +454,7 @@ extern "C" int64_t taac_backbone_workspace_bytes(int32_t B, int32_t T, int32_t D
   // x, h (shared with the attention output), qkv, then either the packed weights + the valid-row index (fused path)
   // or the gated hidden state
   const int64_t acts = align256(M * D * 2) * 2 + align256(M * 3 * D * 2);
-  return acts + (fused_shape(D, F) ? n_blocks * packed_block_bytes(D, F) + row_index_bytes(B, T) + qk_norm_bytes(M, D) +
+  return acts + (fused_shape(D, F) ? n_blocks * packed_block_bytes(D, F) + row_index_bytes(B, T) + qk_norm_bytes(M, D, n_blocks) +
                                          fp8_bytes(D, F, n_blocks)
                                    : align256(M * F * 2));
 }
@@ -536,11 +516,12 @@ extern "C" int taac_backbone_fwd(const void* emb, const int32_t* key_lengths, co
   bf16_t* qk_weight = reinterpret_cast<bf16_t*>(reinterpret_cast<char*>(qk_rstd) + align256(2 * M * 4));
   if (rope_cos_sin != nullptr && !aligned16(rope_cos_sin))
     return set_error(TAAC_ERR_UNSUPPORTED, "%s: the rotary table must be 16-byte aligned", name);
-  if (fused && n_blocks > 0 && !(flags & TAAC_BACKBONE_DENSE_TOKENS)) {
+  const bool sparse = fused && n_blocks > 0 && !(flags & TAAC_BACKBONE_DENSE_TOKENS);
+  if (sparse) {
+    if (M > 0x7fffffffLL - B - 1 || B > 65535)
+      return set_error(TAAC_ERR_UNSUPPORTED, "%s: the row index covers at most 65535 samples and 2^31 rows", name);
     rows = reinterpret_cast<int32_t*>(after_packed);
     n_rows = rows + M + B + 1;
-    const int rc_rows = taac_valid_rows(key_lengths, B, T, rows, n_rows, stream);
-    if (rc_rows != TAAC_OK) return rc_rows;
   }
 
   const int dh = D / heads;
@@ -551,24 +532,31 @@ extern "C" int taac_backbone_fwd(const void* emb, const int32_t* key_lengths, co
   int rc;
   // TAAC_BACKBONE_SPLIT_OUT_FFN: the out projection and the feed-forward half as two kernels (comparison route).
   const bool split_out_ffn = (flags & TAAC_BACKBONE_SPLIT_OUT_FFN) != 0;
-  if (fused && !fp8 && n_blocks > 0) {
-    // One launch re-lays the weights of all blocks into fragment order.
+  float* norm_product = reinterpret_cast<float*>(qk_weight);  // [n_blocks, D]
+  if (fused && n_blocks > 0) {
+    // One launch: the weights of all blocks in fragment order (the FP8 mode packs its own), the row index, the products of the
+    // query and key norm weights, zeros in the padded rows of the returned hidden state.
     std::vector<void*> pk(3 * static_cast<size_t>(n_blocks));
+    bool qk_norms = false;
     for (int i = 0; i < n_blocks; ++i) {
       const taac_block_weights& w = blocks[i];
       if (!w.qkv_weight || !w.out_weight || !w.up_weight || !w.down_weight)
         return set_error(TAAC_ERR_INVALID_VALUE, "%s: block %d has a null weight", name, i);
+      if ((w.query_norm_weight == nullptr) != (w.key_norm_weight == nullptr))
+        return set_error(TAAC_ERR_INVALID_VALUE, "%s: block %d: query and key norm weights come together", name, i);
+      qk_norms = qk_norms || w.query_norm_weight != nullptr;
       char* base = packed + static_cast<int64_t>(i) * packed_block_bytes(D, F);
       pk[i] = base;
       pk[n_blocks + i] = base + align256(static_cast<int64_t>(3) * D * D * 2);
       pk[2 * n_blocks + i] = base + align256(static_cast<int64_t>(3) * D * D * 2) + align256(static_cast<int64_t>(D) * D * 2);
     }
-    if ((rc = pack_backbone_blocks(blocks, n_blocks, D, F, pk.data(), pk.data() + n_blocks, pk.data() + 2 * n_blocks,
-                                   fold_act, as_stream(stream), name)) != TAAC_OK)
+    if ((rc = backbone_setup(blocks, n_blocks, D, F, fp8 ? nullptr : pk.data(), pk.data() + n_blocks, pk.data() + 2 * n_blocks,
+                             fold_act, qk_norms && rope_cos_sin == nullptr ? norm_product : nullptr, key_lengths, B, T, rows,
+                             n_rows, sparse ? hidden_out : nullptr, as_stream(stream), name)) != TAAC_OK)
       return rc;
   }
   // FP8 mode: scales and e4m3 weights of all blocks (three launches), then the scale of the first block's input
-  char* fp8_base = reinterpret_cast<char*>(qk_weight) + align256(static_cast<int64_t>(D) * 4);
+  char* fp8_base = reinterpret_cast<char*>(qk_weight) + align256(static_cast<int64_t>(D) * 4 * n_blocks);
   float* fp8_scales = reinterpret_cast<float*>(fp8_base + static_cast<int64_t>(n_blocks) * (fp8 ? fp8_block_bytes(D, F) : 0));
   auto fp8_qkv = [&](int i) { return fp8_base + static_cast<int64_t>(i) * fp8_block_bytes(D, F); };
   auto fp8_out = [&](int i) { return fp8_qkv(i) + align256(static_cast<int64_t>(3) * D * D); };
@@ -656,14 +644,7 @@ extern "C" int taac_backbone_fwd(const void* emb, const int32_t* key_lengths, co
       // product on the query features; with one, the epilogue applies weight and rotation. Either way there is no
       // pass of its own over q and k.
       const bool weights_in_epilogue = qk_norm && rope_cos_sin != nullptr;
-      if (qk_norm && !weights_in_epilogue) {
-        float* prod = reinterpret_cast<float*>(qk_weight);
-        hipLaunchKernelGGL(weight_product_kernel, dim3((D + kBlock - 1) / kBlock), dim3(kBlock), 0, as_stream(stream),
-                           static_cast<const bf16_t*>(w.query_norm_weight),
-                           static_cast<const bf16_t*>(w.key_norm_weight), prod, D);
-        if ((rc = check_launch(name)) != TAAC_OK) return rc;
-        q_col_scale = prod;
-      }
+      if (qk_norm && !weights_in_epilogue) q_col_scale = norm_product + static_cast<int64_t>(i) * D;
       const void* q_weight = weights_in_epilogue ? w.query_norm_weight : nullptr;
       const void* k_weight = weights_in_epilogue ? w.key_norm_weight : nullptr;
       if (weights_in_epilogue && (!planes || !aligned16(q_weight) || !aligned16(k_weight))) {
@@ -758,13 +739,6 @@ extern "C" int taac_backbone_fwd(const void* emb, const int32_t* key_lengths, co
         return rc;
     }
     cur = x_out;
-  }
-  if (rows != nullptr && hidden_out != nullptr) {
-    // The padded positions of the returned hidden state were never written: define them as zeros.
-    const int64_t pieces = static_cast<int64_t>(T) * (D / 8);
-    hipLaunchKernelGGL(zero_padded_rows_kernel, dim3(static_cast<uint32_t>((pieces + kBlock - 1) / kBlock), B),
-                       dim3(kBlock), 0, as_stream(stream), static_cast<bf16_t*>(hidden_out), key_lengths, T, D);
-    if ((rc = check_launch(name)) != TAAC_OK) return rc;
   }
   if (n_blocks == 0 && hidden_out != nullptr) {
     if (hipMemcpyAsync(hidden_out, emb, static_cast<size_t>(M) * D * 2, hipMemcpyDeviceToDevice, as_stream(stream)) !=

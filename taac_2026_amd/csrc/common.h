@@ -33,11 +33,15 @@ int compute_units();
 // is routed to its tiled kernel.
 int test_max_workgroups();
 bool test_fp8_tiled();
-// Packs the qkv / out / feed-forward weights (gate first) of n backbone blocks into fragment order (ffn.hip).
+// What a backbone forward prepares in front of its blocks (ffn.hip), each part optional: the qkv / out / feed-forward weights
+// (gate first) of n blocks in fragment order (packed_qkv null: none); norm_product [n, D] = query times key norm weight of the
+// blocks that have them; the valid-row index of `lengths` (rows null: none); zeros in the padded rows of zero_rows [B, T, D].
 // fold_act: the up projection also takes the constants of the gate's activation (the kernels are then called with
 // TAAC_FOLDED_ACTIVATION; allowed where ffn_act_fold_supported says so).
-int pack_backbone_blocks(const taac_block_weights* blocks, int n, int32_t D, int32_t F, void* const* packed_qkv,
-                         void* const* packed_out, void* const* packed_ffn, bool fold_act, hipStream_t s, const char* name);
+int backbone_setup(const taac_block_weights* blocks, int n, int32_t D, int32_t F, void* const* packed_qkv,
+                   void* const* packed_out, void* const* packed_ffn, bool fold_act, float* norm_product,
+                   const int32_t* lengths, int32_t B, int32_t T, int32_t* rows, int32_t* n_rows, void* zero_rows,
+                   hipStream_t s, const char* name);
 bool ffn_act_fold_supported(int32_t D, int32_t F);
 // RMSNorm + q | k | v projection with the query / key epilogue (ffn.hip; the arguments of taac_norm_linear_qk_fwd with
 // packed weights, the two norm weights apart) whose output is a stack of per-head planes [3 * num_heads][M][head_dim],

@@ -24,6 +24,7 @@
 // of roundings of the reference's bf16 evaluation (linear output rounded, then the residual add rounded).
 #include "common.h"
 #include "ts_common.h"
+#include "row_index.h"
 #include "ts_dense.h"
 
 namespace taac {
@@ -125,8 +126,7 @@ __global__ void linear_pack_kernel(const bf16_t* __restrict__ w, bf16x8* __restr
   if (gid < total) linear_pack_piece(w, packed, K, gid, col_scale);
 }
 
-// All weights of up to kPackBatch backbone blocks in one launch: blockIdx.y = block, blockIdx.x walks the 16-byte
-// pieces of its qkv, out and feed-forward blobs in that order.
+// Weights of up to kPackBatch backbone blocks: the 16-byte pieces of a block's qkv, out and feed-forward blobs in that order.
 constexpr int kPackBatch = 16;
 struct PackBatch {
   const bf16_t* qkv[kPackBatch];
@@ -139,17 +139,62 @@ struct PackBatch {
   bf16x8* packed_out[kPackBatch];
   bf16x8* packed_ffn[kPackBatch];
 };
-__global__ void pack_blocks_kernel(const PackBatch batch, int D, int F, bool fold_act) {
-  const int blk = blockIdx.y;
-  const int64_t n_qkv = static_cast<int64_t>(3) * D * D / 8, n_out = static_cast<int64_t>(D) * D / 8;
-  const int64_t n_ffn = static_cast<int64_t>(3) * D * F / 8;
-  int64_t gid = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (gid < n_qkv) return linear_pack_piece(batch.qkv[blk], batch.packed_qkv[blk], D, gid, batch.qkv_norm[blk]);
-  gid -= n_qkv;
-  if (gid < n_out) return linear_pack_piece(batch.out[blk], batch.packed_out[blk], D, gid);
-  gid -= n_out;
-  if (gid < n_ffn)
-    ffn_pack_piece(batch.up[blk], batch.down[blk], batch.packed_ffn[blk], D, F, 1, gid, batch.ffn_norm[blk], fold_act);
+// What a backbone forward prepares in front of its first block, in one launch: the weights of up to kPackBatch blocks in
+// fragment order, the valid-row index, the products of the query and key norm weights, the padded rows of the returned
+// hidden state (zeros; the blocks write valid rows only). None depends on another; every workgroup has one of the roles.
+// (As launches of their own - two for the index - they cost a small batch 4 to 5 us each.)
+struct SetupParams {
+  PackBatch pack;
+  const bf16_t* query_norm[kPackBatch];  // with norm_product: prod[blk][d] = query_norm[d] * key_norm[d] in fp32 - the two weights
+  const bf16_t* key_norm[kPackBatch];    // act on a score only through it - or null
+  float* norm_product;
+  const int32_t* lengths;
+  int32_t* rows;                         // null: no index
+  int32_t* n_rows;
+  bf16_t* zero_rows;                     // [B, T, D] or null
+  int32_t B, T, D, F;
+  int32_t first_block;                   // index of pack entry 0 in the product table
+  bool fold_act;
+  uint32_t pack_units, row_units, product_units;  // workgroups of the roles, in this order; the zero rows take the rest
+  uint32_t pack_units_per_block;
+};
+__global__ __launch_bounds__(kRowThreads) void backbone_setup_kernel(const SetupParams p) {
+  uint32_t unit = blockIdx.x;
+  const int D = p.D;
+  if (unit < p.pack_units) {
+    const int blk = static_cast<int>(unit / p.pack_units_per_block);
+    const int64_t n_qkv = static_cast<int64_t>(3) * D * D / 8, n_out = static_cast<int64_t>(D) * D / 8;
+    const int64_t n_ffn = static_cast<int64_t>(3) * D * p.F / 8;
+    int64_t gid = static_cast<int64_t>(unit % p.pack_units_per_block) * kRowThreads + threadIdx.x;
+    if (gid < n_qkv) return linear_pack_piece(p.pack.qkv[blk], p.pack.packed_qkv[blk], D, gid, p.pack.qkv_norm[blk]);
+    gid -= n_qkv;
+    if (gid < n_out) return linear_pack_piece(p.pack.out[blk], p.pack.packed_out[blk], D, gid);
+    gid -= n_out;
+    if (gid < n_ffn)
+      ffn_pack_piece(p.pack.up[blk], p.pack.down[blk], p.pack.packed_ffn[blk], D, p.F, 1, gid, p.pack.ffn_norm[blk], p.fold_act);
+    return;
+  }
+  unit -= p.pack_units;
+  if (unit < p.row_units) return write_valid_rows(p.lengths, p.B, p.T, static_cast<int>(unit), p.rows, p.n_rows);
+  unit -= p.row_units;
+  if (unit < p.product_units) {
+    const bf16_t* wq = p.query_norm[unit];
+    if (wq == nullptr) return;
+    float* prod = p.norm_product + static_cast<int64_t>(p.first_block + unit) * D;
+    for (int d = threadIdx.x; d < D; d += kRowThreads) prod[d] = static_cast<float>(wq[d]) * static_cast<float>(p.key_norm[unit][d]);
+    return;
+  }
+  unit -= p.product_units;
+  const int c8n = D / 8;
+  const uint32_t per = (static_cast<uint32_t>(p.T) * c8n + kRowThreads - 1) / kRowThreads;
+  const int b = static_cast<int>(unit / per);
+  const int idx = static_cast<int>(unit % per) * kRowThreads + static_cast<int>(threadIdx.x);
+  const int t = clamped_length(p.lengths, b, p.T) + idx / c8n;
+  if (t >= p.T) return;
+  bf16x8 z;
+#pragma unroll
+  for (int e = 0; e < 8; ++e) z[e] = static_cast<bf16_t>(0.f);
+  *reinterpret_cast<bf16x8*>(p.zero_rows + (static_cast<int64_t>(b) * p.T + t) * D + (idx % c8n) * 8) = z;
 }
 
 // Reads the epilogue tile back row-wise (lane -> token 8*i + lane/8, features 8*(lane%8) .. +7), adds the residual
@@ -1233,30 +1278,64 @@ constexpr int kMaxLdsBytes = 160 * 1024;
 }  // namespace taac
 
 namespace taac {
-// Packs the qkv / out / feed-forward weights (gate first) of n backbone blocks with as few launches as possible.
-int pack_backbone_blocks(const taac_block_weights* blocks, int n, int32_t D, int32_t F, void* const* packed_qkv,
-                         void* const* packed_out, void* const* packed_ffn, bool fold_act, hipStream_t s, const char* name) {
-  for (int base = 0; base < n; base += kPackBatch) {
-    PackBatch batch{};
+// See common.h. One launch (more only for more than kPackBatch blocks).
+int backbone_setup(const taac_block_weights* blocks, int n, int32_t D, int32_t F, void* const* packed_qkv,
+                   void* const* packed_out, void* const* packed_ffn, bool fold_act, float* norm_product,
+                   const int32_t* lengths, int32_t B, int32_t T, int32_t* rows, int32_t* n_rows, void* zero_rows,
+                   hipStream_t s, const char* name) {
+  for (int base = 0; base == 0 || base < n; base += kPackBatch) {
+    SetupParams p{};
     const int m = n - base < kPackBatch ? n - base : kPackBatch;
-    for (int i = 0; i < m; ++i) {
-      const taac_block_weights& w = blocks[base + i];
-      if (!ptr_ok(w.qkv_weight, 15) || !ptr_ok(w.out_weight, 15) || !ptr_ok(w.up_weight, 15) ||
-          !ptr_ok(w.down_weight, 15) || !ptr_ok(w.attn_norm_weight, 15) || !ptr_ok(w.ffn_norm_weight, 15))
-        return set_error(TAAC_ERR_UNSUPPORTED, "%s: weights must be 16-byte aligned", name);
-      batch.qkv[i] = static_cast<const bf16_t*>(w.qkv_weight);
-      batch.qkv_norm[i] = static_cast<const bf16_t*>(w.attn_norm_weight);
-      batch.out[i] = static_cast<const bf16_t*>(w.out_weight);
-      batch.up[i] = static_cast<const bf16_t*>(w.up_weight);
-      batch.ffn_norm[i] = static_cast<const bf16_t*>(w.ffn_norm_weight);
-      batch.down[i] = static_cast<const bf16_t*>(w.down_weight);
-      batch.packed_qkv[i] = static_cast<bf16x8*>(packed_qkv[base + i]);
-      batch.packed_out[i] = static_cast<bf16x8*>(packed_out[base + i]);
-      batch.packed_ffn[i] = static_cast<bf16x8*>(packed_ffn[base + i]);
+    if (packed_qkv != nullptr) {
+      for (int i = 0; i < m; ++i) {
+        const taac_block_weights& w = blocks[base + i];
+        if (!ptr_ok(w.qkv_weight, 15) || !ptr_ok(w.out_weight, 15) || !ptr_ok(w.up_weight, 15) ||
+            !ptr_ok(w.down_weight, 15) || !ptr_ok(w.attn_norm_weight, 15) || !ptr_ok(w.ffn_norm_weight, 15))
+          return set_error(TAAC_ERR_UNSUPPORTED, "%s: weights must be 16-byte aligned", name);
+        p.pack.qkv[i] = static_cast<const bf16_t*>(w.qkv_weight);
+        p.pack.qkv_norm[i] = static_cast<const bf16_t*>(w.attn_norm_weight);
+        p.pack.out[i] = static_cast<const bf16_t*>(w.out_weight);
+        p.pack.up[i] = static_cast<const bf16_t*>(w.up_weight);
+        p.pack.ffn_norm[i] = static_cast<const bf16_t*>(w.ffn_norm_weight);
+        p.pack.down[i] = static_cast<const bf16_t*>(w.down_weight);
+        p.pack.packed_qkv[i] = static_cast<bf16x8*>(packed_qkv[base + i]);
+        p.pack.packed_out[i] = static_cast<bf16x8*>(packed_out[base + i]);
+        p.pack.packed_ffn[i] = static_cast<bf16x8*>(packed_ffn[base + i]);
+        p.query_norm[i] = static_cast<const bf16_t*>(w.query_norm_weight);
+        p.key_norm[i] = static_cast<const bf16_t*>(w.key_norm_weight);
+      }
+      const int64_t pieces = (static_cast<int64_t>(4) * D * D + static_cast<int64_t>(3) * D * F) / 8;
+      p.pack_units_per_block = static_cast<uint32_t>((pieces + kRowThreads - 1) / kRowThreads);
+      p.pack_units = p.pack_units_per_block * m;
+      p.product_units = norm_product != nullptr ? m : 0;
     }
-    const int64_t pieces = (static_cast<int64_t>(4) * D * D + static_cast<int64_t>(3) * D * F) / 8;
-    hipLaunchKernelGGL(pack_blocks_kernel, dim3(static_cast<uint32_t>((pieces + 255) / 256), m), dim3(256), 0, s, batch,
-                       D, F, fold_act);
+    p.norm_product = norm_product;
+    p.first_block = base;
+    p.fold_act = fold_act;
+    p.lengths = lengths;
+    p.B = B;
+    p.T = T;
+    p.D = D;
+    p.F = F;
+    int64_t units = static_cast<int64_t>(p.pack_units) + p.product_units;
+    if (base == 0) {
+      if (rows != nullptr && B <= kMaxScanBatch) {
+        p.rows = rows;
+        p.n_rows = n_rows;
+        p.row_units = static_cast<uint32_t>(B) * (T > kRowThreads ? (T + kRowThreads - 1) / kRowThreads : 1);
+        units += p.row_units;
+      } else if (rows != nullptr) {
+        const int rc = taac_valid_rows(lengths, B, T, rows, n_rows, s);
+        if (rc != TAAC_OK) return rc;
+      }
+      if (zero_rows != nullptr) {
+        p.zero_rows = static_cast<bf16_t*>(zero_rows);
+        units += static_cast<int64_t>(B) * ((static_cast<int64_t>(T) * (D / 8) + kRowThreads - 1) / kRowThreads);
+      }
+    }
+    if (units == 0) continue;
+    if (units > 0x7fffffffLL) return set_error(TAAC_ERR_UNSUPPORTED, "%s: too many workgroups", name);
+    hipLaunchKernelGGL(backbone_setup_kernel, dim3(static_cast<uint32_t>(units)), dim3(kRowThreads), 0, s, p);
     const int rc = check_launch(name);
     if (rc != TAAC_OK) return rc;
   }
