@@ -455,7 +455,7 @@ extern "C" int64_t taac_backbone_workspace_bytes(int32_t B, int32_t T, int32_t D
   // or the gated hidden state
   const int64_t acts = align256(M * D * 2) * 2 + align256(M * 3 * D * 2);
   return acts + (fused_shape(D, F) ? n_blocks * packed_block_bytes(D, F) + row_index_bytes(B, T) + qk_norm_bytes(M, D, n_blocks) +
-                                         fp8_bytes(D, F, n_blocks)
+                                         align256(ffn_split_bytes(M, D, F)) + fp8_bytes(D, F, n_blocks)
                                    : align256(M * F * 2));
 }
 
@@ -533,6 +533,12 @@ extern "C" int taac_backbone_fwd(const void* emb, const int32_t* key_lengths, co
   // TAAC_BACKBONE_SPLIT_OUT_FFN: the out projection and the feed-forward half as two kernels (comparison route).
   const bool split_out_ffn = (flags & TAAC_BACKBONE_SPLIT_OUT_FFN) != 0;
   float* norm_product = reinterpret_cast<float*>(qk_weight);  // [n_blocks, D]
+  // partials and counters of a feed-forward whose token tiles are shared by several workgroups (small batches)
+  const int ffn_split = fused ? ffn_splits(M, D, F) : 1;
+  char* split_scratch = ffn_split > 1 ? reinterpret_cast<char*>(norm_product) + align256(static_cast<int64_t>(D) * 4 * n_blocks) : nullptr;
+  const int64_t tiles = (M + 31) / 32;
+  uint32_t* split_counters =
+      split_scratch != nullptr ? reinterpret_cast<uint32_t*>(split_scratch + tiles * ffn_split * 32 * D * 4) : nullptr;
   if (fused && n_blocks > 0) {
     // One launch: the weights of all blocks in fragment order (the FP8 mode packs its own), the row index, the products of the
     // query and key norm weights, zeros in the padded rows of the returned hidden state.
@@ -552,11 +558,13 @@ extern "C" int taac_backbone_fwd(const void* emb, const int32_t* key_lengths, co
     }
     if ((rc = backbone_setup(blocks, n_blocks, D, F, fp8 ? nullptr : pk.data(), pk.data() + n_blocks, pk.data() + 2 * n_blocks,
                              fold_act, qk_norms && rope_cos_sin == nullptr ? norm_product : nullptr, key_lengths, B, T, rows,
-                             n_rows, sparse ? hidden_out : nullptr, as_stream(stream), name)) != TAAC_OK)
+                             n_rows, sparse ? hidden_out : nullptr, split_counters,
+                             ffn_split > 1 ? static_cast<int32_t>(tiles) : 0, as_stream(stream), name)) != TAAC_OK)
       return rc;
   }
   // FP8 mode: scales and e4m3 weights of all blocks (three launches), then the scale of the first block's input
-  char* fp8_base = reinterpret_cast<char*>(qk_weight) + align256(static_cast<int64_t>(D) * 4 * n_blocks);
+  char* fp8_base = reinterpret_cast<char*>(qk_weight) + align256(static_cast<int64_t>(D) * 4 * n_blocks) +
+                   align256(ffn_split_bytes(M, D, F));
   float* fp8_scales = reinterpret_cast<float*>(fp8_base + static_cast<int64_t>(n_blocks) * (fp8 ? fp8_block_bytes(D, F) : 0));
   auto fp8_qkv = [&](int i) { return fp8_base + static_cast<int64_t>(i) * fp8_block_bytes(D, F); };
   auto fp8_out = [&](int i) { return fp8_qkv(i) + align256(static_cast<int64_t>(3) * D * D); };
@@ -701,7 +709,7 @@ extern "C" int taac_backbone_fwd(const void* emb, const int32_t* key_lengths, co
         return rc;
       if ((rc = attn_out_ffn_readout(h, D, dh, w.out_bias, pk_out, cur, D, w.ffn_norm_weight, eps, w.up_bias, w.down_bias,
                                      pk_ffn, x_out, D, M, D, F, rows, n_rows, ffn_folded,
-                                     ride ? w_head : nullptr, ride ? token_dots : nullptr, stream)) != TAAC_OK)
+                                     ride ? w_head : nullptr, ride ? token_dots : nullptr, split_scratch, stream)) != TAAC_OK)
         return rc;
       dots_ready = ride;
       cur = x_out;
@@ -715,7 +723,7 @@ extern "C" int taac_backbone_fwd(const void* emb, const int32_t* key_lengths, co
       // out projection + residual and the whole feed-forward half in one kernel; the stream between them stays on chip
       if ((rc = attn_out_ffn_readout(h, D, 0, w.out_bias, pk_out, cur, D, w.ffn_norm_weight, eps, w.up_bias, w.down_bias,
                                      pk_ffn, x_out, D, M, D, F, rows, n_rows, ffn_folded,
-                                     ride ? w_head : nullptr, ride ? token_dots : nullptr, stream)) != TAAC_OK)
+                                     ride ? w_head : nullptr, ride ? token_dots : nullptr, split_scratch, stream)) != TAAC_OK)
         return rc;
       dots_ready = ride;
     } else if (fused) {

@@ -35,14 +35,21 @@ int test_max_workgroups();
 bool test_fp8_tiled();
 // What a backbone forward prepares in front of its blocks (ffn.hip), each part optional: the qkv / out / feed-forward weights
 // (gate first) of n blocks in fragment order (packed_qkv null: none); norm_product [n, D] = query times key norm weight of the
-// blocks that have them; the valid-row index of `lengths` (rows null: none); zeros in the padded rows of zero_rows [B, T, D].
+// blocks that have them; the valid-row index of `lengths` (rows null: none); zeros in the padded rows of zero_rows [B, T, D] and
+// in n_counters counters.
 // fold_act: the up projection also takes the constants of the gate's activation (the kernels are then called with
 // TAAC_FOLDED_ACTIVATION; allowed where ffn_act_fold_supported says so).
 int backbone_setup(const taac_block_weights* blocks, int n, int32_t D, int32_t F, void* const* packed_qkv,
                    void* const* packed_out, void* const* packed_ffn, bool fold_act, float* norm_product,
                    const int32_t* lengths, int32_t B, int32_t T, int32_t* rows, int32_t* n_rows, void* zero_rows,
-                   hipStream_t s, const char* name);
+                   uint32_t* counters, int32_t n_counters, hipStream_t s, const char* name);
 bool ffn_act_fold_supported(int32_t D, int32_t F);
+bool ffn_few_rows(int64_t M, int32_t D);
+// Workgroups that share the hidden units of a token tile when the gated feed-forward over at most M rows runs as the few-token
+// kernel and is given the scratch memory for it (ffn_split_bytes; the counters behind the partials zeroed once): a power of
+// two as long as the tiles leave that many compute units idle. 1 otherwise.
+int ffn_splits(int64_t M, int32_t D, int32_t F);
+int64_t ffn_split_bytes(int64_t M, int32_t D, int32_t F);
 // RMSNorm + q | k | v projection with the query / key epilogue (ffn.hip; the arguments of taac_norm_linear_qk_fwd with
 // packed weights, the two norm weights apart) whose output is a stack of per-head planes [3 * num_heads][M][head_dim],
 // head_dim 32 or 64; qk_rstd [2, M] (with qk_sumsq): the factors of taac_row_rstd, written when dense_few_rows(M, d_model).
@@ -55,12 +62,13 @@ int norm_linear_qk_heads(const void* x, int64_t ldx, const void* norm_weight, fl
 // projection itself and no taac_row_rstd is needed).
 bool dense_few_rows(int64_t M, int32_t D);
 // Out projection + feed-forward half of a block (ffn.hip; attn_plane: 0 = rows of ld_attn elements, 32 / 64 = per-head
-// planes) that also writes the dot product of every stored output row with head_w to token_dots[row].
+// planes) that also writes the dot product of every stored output row with head_w to token_dots[row]; split_scratch:
+// ffn_split_bytes(M, D, F) bytes, or null.
 int attn_out_ffn_readout(const void* attn, int64_t ld_attn, int attn_plane, const void* out_bias,
                          const void* packed_out_weights, const void* residual, int64_t ldr, const void* norm_weight,
                          float eps, const void* b_up, const void* b_down, const void* packed_ffn_weights, void* out,
                          int64_t ldo, int64_t M, int32_t D, int32_t F, const int32_t* rows, const int32_t* n_rows,
-                         int norm_folded, const void* head_w, float* token_dots, void* stream);
+                         int norm_folded, const void* head_w, float* token_dots, void* split_scratch, void* stream);
 // Token-stationary e4m3 dense layer (fp8_ts.hip): TAAC_OK after a launch, a negative status on an error, 1 when the shape
 // is not covered and the caller must use the tiled kernel.
 int launch_linear_fp8_ts(const void* a, int a_is_fp8, int64_t lda, const void* w, const float* amax_a,

@@ -157,10 +157,14 @@ struct SetupParams {
   bool fold_act;
   uint32_t pack_units, row_units, product_units;  // workgroups of the roles, in this order; the zero rows take the rest
   uint32_t pack_units_per_block;
+  uint32_t* counters;                    // cleared by workgroup 0 besides its role
+  int32_t n_counters;
 };
 __global__ __launch_bounds__(kRowThreads) void backbone_setup_kernel(const SetupParams p) {
   uint32_t unit = blockIdx.x;
   const int D = p.D;
+  if (unit == 0)
+    for (int i = threadIdx.x; i < p.n_counters; i += kRowThreads) p.counters[i] = 0u;
   if (unit < p.pack_units) {
     const int blk = static_cast<int>(unit / p.pack_units_per_block);
     const int64_t n_qkv = static_cast<int64_t>(3) * D * D / 8, n_out = static_cast<int64_t>(D) * D / 8;
@@ -1282,7 +1286,7 @@ namespace taac {
 int backbone_setup(const taac_block_weights* blocks, int n, int32_t D, int32_t F, void* const* packed_qkv,
                    void* const* packed_out, void* const* packed_ffn, bool fold_act, float* norm_product,
                    const int32_t* lengths, int32_t B, int32_t T, int32_t* rows, int32_t* n_rows, void* zero_rows,
-                   hipStream_t s, const char* name) {
+                   uint32_t* counters, int32_t n_counters, hipStream_t s, const char* name) {
   for (int base = 0; base == 0 || base < n; base += kPackBatch) {
     SetupParams p{};
     const int m = n - base < kPackBatch ? n - base : kPackBatch;
@@ -1319,6 +1323,8 @@ int backbone_setup(const taac_block_weights* blocks, int n, int32_t D, int32_t F
     p.F = F;
     int64_t units = static_cast<int64_t>(p.pack_units) + p.product_units;
     if (base == 0) {
+      p.counters = counters;
+      p.n_counters = n_counters;
       if (rows != nullptr && B <= kMaxScanBatch) {
         p.rows = rows;
         p.n_rows = n_rows;
@@ -1433,13 +1439,6 @@ extern "C" int taac_linear_pack_weights_norm(const void* w, const void* norm_wei
 namespace taac {
 namespace {
 
-// Whether the gated feed-forward over at most M rows of D features runs as the few-token kernel: as long as its 32-token
-// workgroups fit the chip in one round. Measured with the out projection in front, launches back to back, few-token /
-// persistent kernel, us: D = 256, F = 1024 - 512 rows 21.5 / 49.9, 8192 27.8 / 55.6, 16384 53.8 / 57.7, 24576 72.5 / 58.2;
-// F = 512 - 8192 18.8 / 34.7, 16384 34.4 / 36.4; D = 128 (two workgroups per compute unit), F = 512 - 512 rows 9.2 / 19.5,
-// 16384 16.8 / 21.9, 24576 23.0 / 22.2.
-bool ffn_few_rows(int64_t M, int32_t D) { return test_max_workgroups() == 0 && M * D <= 8192 * 256; }
-
 // Shared body of taac_swiglu_ffn_fwd and taac_attn_out_ffn_fwd (out_packed != null: the attention output projection
 // runs in front; x is then the attention output and residual the block input).
 int ffn_entry(const char* name, const void* x, int64_t ldx, const void* out_bias, const void* out_packed,
@@ -1447,7 +1446,8 @@ int ffn_entry(const char* name, const void* x, int64_t ldx, const void* out_bias
               const void* b_down, const void* packed_weights, const void* residual, int64_t ldr, void* out, int64_t ldo,
               int64_t M, int32_t D, int32_t F, int gate_first, const int32_t* rows, const int32_t* n_rows,
               const int32_t* x_rows, int norm_folded, void* stream, const void* update_gate = nullptr, int64_t ldg = 0,
-              bool glu = true, int x_plane = 0, const void* head_w = nullptr, float* token_dots = nullptr) {
+              bool glu = true, int x_plane = 0, const void* head_w = nullptr, float* token_dots = nullptr,
+              void* split_scratch = nullptr) {
   const bool with_proj = out_packed != nullptr;
   if (norm_folded < 0 || norm_folded > (TAAC_FOLDED_NORM | TAAC_FOLDED_ACTIVATION))
     return set_error(TAAC_ERR_INVALID_VALUE, "%s: norm_folded holds TAAC_FOLDED_NORM and / or TAAC_FOLDED_ACTIVATION", name);
@@ -1527,6 +1527,10 @@ int ffn_entry(const char* name, const void* x, int64_t ldx, const void* out_bias
   if (const int limit = test_max_workgroups(); limit > 0 && limit < p.units) p.units = limit;  // taac_test_hooks
   hipStream_t s = as_stream(stream);
   if (ffn_few_rows(M, D) && glu && update_gate == nullptr && packed_weights && (norm_weight == nullptr || norm_folded)) {
+    if (split_scratch != nullptr && (p.splits = ffn_splits(M, D, F)) > 1) {
+      p.split_partials = static_cast<float*>(split_scratch);
+      p.split_counters = reinterpret_cast<uint32_t*>(p.split_partials + (M + 31) / 32 * p.splits * 32 * D);
+    }
     const int rc = swiglu_ffn_small(p, D, with_proj, act_folded, s, name);
     if (rc != 1) return rc;
   }
@@ -1836,11 +1840,18 @@ int attn_out_ffn_readout(const void* attn, int64_t ld_attn, int attn_plane, cons
                          const void* packed_out_weights, const void* residual, int64_t ldr, const void* norm_weight,
                          float eps, const void* b_up, const void* b_down, const void* packed_ffn_weights, void* out,
                          int64_t ldo, int64_t M, int32_t D, int32_t F, const int32_t* rows, const int32_t* n_rows,
-                         int norm_folded, const void* head_w, float* token_dots, void* stream) {
+                         int norm_folded, const void* head_w, float* token_dots, void* split_scratch, void* stream) {
   return ffn_entry("taac_backbone_fwd", attn, ld_attn, out_bias, packed_out_weights, norm_weight, eps, nullptr, b_up, nullptr,
                    b_down, packed_ffn_weights, residual, ldr, out, ldo, M, D, F, 1, rows, n_rows, nullptr, norm_folded,
-                   stream, nullptr, 0, true, attn_plane, head_w, token_dots);
+                   stream, nullptr, 0, true, attn_plane, head_w, token_dots, split_scratch);
 }
+
+// Whether the gated feed-forward over at most M rows of D features runs as the few-token kernel: as long as its 32-token
+// workgroups fit the chip in one round. Measured with the out projection in front, launches back to back, few-token /
+// persistent kernel, us: D = 256, F = 1024 - 512 rows 21.5 / 49.9, 8192 27.8 / 55.6, 16384 53.8 / 57.7, 24576 72.5 / 58.2;
+// F = 512 - 8192 18.8 / 34.7, 16384 34.4 / 36.4; D = 128 (two workgroups per compute unit), F = 512 - 512 rows 9.2 / 19.5,
+// 16384 16.8 / 21.9, 24576 23.0 / 22.2.
+bool ffn_few_rows(int64_t M, int32_t D) { return test_max_workgroups() == 0 && M * D <= 8192 * 256; }
 
 // Whether a projection over at most M rows of D features runs as the few-token kernel. Measured for q | k | v (launches
 // back to back, few-token / persistent kernel, us): D = 256 - 512 rows 6.0 / 13.6, 4096 9.9 / 14.1, 8192 14.4 / 15.6,

@@ -14,6 +14,35 @@
 namespace taac {
 namespace {
 
+// Memory rows of N tokens. The index entries are requested before the number of tokens is known (the index holds M entries; what
+// lies beyond the count is not used), so that the two latencies run side by side. A token at or beyond the count reads row 0:
+// its values stay in its own column of every product, and it is not stored.
+template <int N>
+struct SmallRows {
+  int64_t tok[N];
+  int32_t loaded[N];
+  bool indexed;
+  template <typename F>
+  __device__ __forceinline__ void request(const TsParams& p, const int32_t* index, F tok_of) {
+    indexed = index != nullptr;
+#pragma unroll
+    for (int i = 0; i < N; ++i) {
+      tok[i] = tok_of(i);
+      loaded[i] = 0;
+    }
+    if (indexed) {
+#pragma unroll
+      for (int i = 0; i < N; ++i) loaded[i] = index[tok[i] < p.M ? tok[i] : p.M - 1];
+    }
+  }
+  __device__ __forceinline__ void resolve(int64_t count, int64_t (&row)[N]) {
+#pragma unroll
+    for (int i = 0; i < N; ++i) asm volatile("" : "+v"(loaded[i]));  // untouched up to here
+#pragma unroll
+    for (int i = 0; i < N; ++i) row[i] = tok[i] >= count ? 0 : (indexed ? static_cast<int64_t>(loaded[i]) : tok[i]);
+  }
+};
+
 // [RMSNorm (weight folded) ->] linear [-> + residual], K = D, weights in fragment order. A workgroup takes 32 tokens
 // (blockIdx.x) and D output features (blockIdx.y), 64 per wavefront. QK as in norm_linear_kernel: the features of the query
 // (blockIdx.y = 0) and of the key (1) leave their sum of squares behind - as the norm's factor per token in qk_rstd when that
@@ -43,19 +72,16 @@ __global__ __launch_bounds__(D, 2) void norm_linear_small_kernel(const TsParams 
 #pragma unroll
   for (int i = 0; i < NFRAG; ++i) w[i] = *reinterpret_cast<const bf16x8*>(wsrc + i * kFrag + lane * 16);
   __builtin_amdgcn_sched_barrier(0);
-  const int64_t count = token_count(p);
   const int64_t tok0 = static_cast<int64_t>(blockIdx.x) * 32;
+  SmallRows<1> xr;  // memory rows: of x for token l32; of out / residual for token 8 * i + lane / 8
+  SmallRows<4> pr;
+  xr.request(p, p.x_rows != nullptr ? p.x_rows : p.rows, [&](int) { return tok0 + l32; });
+  pr.request(p, p.rows, [&](int i) { return tok0 + i * 8 + lane / 8; });
+  const int64_t count = token_count(p);
   if (tok0 >= count) return;  // whole workgroup
-  int64_t xrow[1], prow[4];   // memory rows: of x for token l32; of out / residual for token 8 * i + lane / 8
-  TokenRows<1> xr;
-  TokenRows<4> pr;
-  xr.request(p.x_rows != nullptr ? p.x_rows : p.rows, count, [&](int) { return tok0 + l32; });
-  pr.request(p.rows, count, [&](int i) { return tok0 + i * 8 + lane / 8; });
-  xr.arrive();
-  pr.arrive();
-  xrow[0] = xr.row(0);
-#pragma unroll
-  for (int i = 0; i < 4; ++i) prow[i] = pr.row(i);
+  int64_t xrow[1], prow[4];
+  xr.resolve(count, xrow);
+  pr.resolve(count, prow);
   bf16x8 xf[1][KS];
   load_token_rows_at<D, 1>(p, xrow, hh, xf);
   const bf16_t* bias = p.b1 != nullptr ? p.b1 + chunk * kNC : nullptr;
@@ -101,7 +127,7 @@ __global__ __launch_bounds__(D, 2) void norm_linear_small_kernel(const TsParams 
         }
       } else {
         const int64_t row = token_row(p, count, tok0 + l32);
-        if (hh == 0) p.qk_sumsq[static_cast<int64_t>(chunk) * p.M + row] = ss;
+        if (hh == 0 && tok0 + l32 < count) p.qk_sumsq[static_cast<int64_t>(chunk) * p.M + row] = ss;
       }
     } else {
       tile_to_lds(tile, acc0, acc1, bv, l32, hh, rstd[0]);
@@ -159,6 +185,23 @@ __global__ __launch_bounds__(D, 2) void norm_linear_small_kernel(const TsParams 
   }
 }
 
+// Data that other workgroups of the same launch read: accesses at the scope of the whole chip, which go through the L2 of the die
+// to the memory all dies share. (Ordinary stores with a fence behind them write back and drop everything the die's L2 holds:
+// 8 us per launch.)
+__device__ __forceinline__ void store_through(f32x4* dst, const f32x4& v) {
+  const u32x4 bits = __builtin_bit_cast(u32x4, v);
+  uint64_t* d = reinterpret_cast<uint64_t*>(dst);
+  __hip_atomic_store(d, static_cast<uint64_t>(bits[0]) | static_cast<uint64_t>(bits[1]) << 32, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  __hip_atomic_store(d + 1, static_cast<uint64_t>(bits[2]) | static_cast<uint64_t>(bits[3]) << 32, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ f32x4 load_through(const f32x4* src) {
+  const uint64_t* s = reinterpret_cast<const uint64_t*>(src);
+  const uint64_t lo = __hip_atomic_load(s, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  const uint64_t hi = __hip_atomic_load(s + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  const u32x4 bits = {static_cast<uint32_t>(lo), static_cast<uint32_t>(lo >> 32), static_cast<uint32_t>(hi), static_cast<uint32_t>(hi >> 32)};
+  return __builtin_bit_cast(f32x4, bits);
+}
+
 // ------------------------------------------------------------------------------------------------------------------
 // The feed-forward half for few tokens: [out projection + residual ->] RMSNorm -> up -> SiLU-gate -> down -> + residual of
 // 32 tokens per workgroup (the products, blobs and roundings of swiglu_ffn_kernel). Four wavefronts share the tokens and divide
@@ -171,6 +214,9 @@ __global__ __launch_bounds__(D, 2) void norm_linear_small_kernel(const TsParams 
 // clock of the compute unit: 11 us) behind and in front of which lie 9.5 us of latency chains; the persistent kernel has one
 // or two of its eight wavefronts at work there and takes 50 us whatever the number of tokens (512 tokens, D = 256, F = 1024:
 // 49.9 -> 21.5 us; 8192 tokens: 55.6 -> 27.8; its line is at ffn_few_rows).
+// splits > 1 (see TsParams): for batches that leave most of the chip idle even so, the hidden units of a tile are also divided over
+// workgroups, eight at most (one request of 512 positions, eight splits, with the requests below ordered by need: the whole
+// 4-block call 164 -> 140 us; fences instead of the write-through accesses: 156).
 // LDS: [4 partials of 32 x D floats][x1 (32 padded rows of D bf16)][first-layer bias 2F][4 x 32 row sums]
 // ------------------------------------------------------------------------------------------------------------------
 template <int D, bool OUTP, bool FOLD>
@@ -193,7 +239,14 @@ __global__ __launch_bounds__(4 * kWave, 1) void swiglu_ffn_small_kernel(const Ts
   const int F = p.F;
   const int nchunks = F / kHU;
 
-  // weights of the projection first: they depend on nothing
+  // Requests in the order in which their values are needed (they arrive in that order): row index and count, the projection's
+  // weights behind them, then - one latency later - the token rows, and last what is used after the projection.
+  const int64_t tok0 = static_cast<int64_t>(blockIdx.x) * 32;
+  SmallRows<1> xr, orow;
+  xr.request(p, p.x_rows != nullptr ? p.x_rows : p.rows, [&](int) { return tok0 + l32; });
+  orow.request(p, p.rows, [&](int) { return tok0 + l32; });
+  const int64_t count = token_count(p);
+  __builtin_amdgcn_sched_barrier(0);
   [[maybe_unused]] bf16x8 w0[OUTP ? MBW * KS : 1];
   if constexpr (OUTP) {
     const char* src = reinterpret_cast<const char*>(p.w0) + static_cast<int64_t>(wave * MBW * KS) * kFrag;
@@ -201,53 +254,58 @@ __global__ __launch_bounds__(4 * kWave, 1) void swiglu_ffn_small_kernel(const Ts
     for (int i = 0; i < MBW * KS; ++i) w0[i] = *reinterpret_cast<const bf16x8*>(src + i * kFrag + lane * 16);
     __builtin_amdgcn_sched_barrier(0);
   }
-  const int64_t count = token_count(p);
-  const int64_t tok0 = static_cast<int64_t>(blockIdx.x) * 32;
   if (tok0 >= count) return;  // whole workgroup
-  TokenRows<1> xr, orow;
-  xr.request(p.x_rows != nullptr ? p.x_rows : p.rows, count, [&](int) { return tok0 + l32; });
-  orow.request(p.rows, count, [&](int) { return tok0 + l32; });
-  // first-layer bias, gated half first; FOLD: with the constants the packed layer carries
-  for (int i = tid * 8; i < 2 * F; i += NW * kWave * 8) {
-    const bool gated = i < F;  // F is a multiple of 32: a piece lies in one half
-    bf16x8 v;
-#pragma unroll
-    for (int e = 0; e < 8; ++e) v[e] = static_cast<bf16_t>(0.f);
-    if (p.b1 != nullptr) v = *reinterpret_cast<const bf16x8*>(p.b1 + (gated == (p.gate_first != 0) ? i % F : F + i % F));
-    if constexpr (FOLD) {
-#pragma unroll
-      for (int e = 0; e < 8; ++e) v[e] = static_cast<bf16_t>(static_cast<float>(v[e]) * (gated ? kFoldGate : kFoldValue));
-    }
-    *reinterpret_cast<bf16x8*>(bias_lds + i) = v;
-  }
-  xr.arrive();
-  orow.arrive();
-  const int64_t xrow[1] = {xr.row(0)};
-  const int64_t row = orow.row(0);  // of token l32 in residual / out
+  int64_t xrow[1], orows[1];
+  xr.resolve(count, xrow);
+  orow.resolve(count, orows);
+  const int64_t row = orows[0];  // of token l32 in residual / out
   bf16x8 xf[1][KS];
   load_token_rows_at<D, 1>(p, xrow, hh, xf);
+  // Four features per register quad of the lane's blocks, in accumulator order. A vector that is absent is read from the weights
+  // instead (finite, in bounds for D values) and cleared where it is used: no branch between the loads.
+  auto feature_vectors = [&](const bf16_t* v, bf16x4 (&dst)[MBW][4]) {
+    const bf16_t* src = v != nullptr ? v : p.w1;
+#pragma unroll
+    for (int m = 0; m < MBW; ++m)
+#pragma unroll
+      for (int jq = 0; jq < 4; ++jq)
+        dst[m][jq] = *reinterpret_cast<const bf16x4*>(src + (wave * MBW + m) * 32 + jq * 8 + hh * 4);
+  };
+  [[maybe_unused]] bf16x4 hv[MBW][4], b0v[MBW][4];  // block input, projection bias
+  if constexpr (OUTP) {
+    feature_vectors(p.residual + row * p.ldr, hv);
+    feature_vectors(p.b0, b0v);
+  }
+  __builtin_amdgcn_sched_barrier(0);
+  const int splits = p.splits > 1 ? p.splits : 1;
+  const int first_chunk = static_cast<int>(blockIdx.y) * NW + wave, stride = NW * splits;
+  const int first = first_chunk < nchunks ? first_chunk : nchunks - 1;
   const char* ffn_blob = reinterpret_cast<const char*>(p.w1) + lane * 16;
   bf16x8 ring[CFRAG];
   auto load_chunk_frag = [&](int chunk, int i) {
     return *reinterpret_cast<const bf16x8*>(ffn_blob + (static_cast<int64_t>(chunk) * CFRAG + i) * kFrag);
   };
-  const int first = wave < nchunks ? wave : nchunks - 1;
+#pragma unroll
+  for (int i = 0; i < CFRAG; ++i) ring[i] = load_chunk_frag(first, i);
+  // first-layer bias, gated half first; FOLD: with the constants the packed layer carries. 8 entries per thread and round.
+  auto bias_piece = [&](int i) {
+    const bool gated = i < F;  // F is a multiple of 32: a piece lies in one half
+    return *reinterpret_cast<const bf16x8*>(p.b1 != nullptr ? p.b1 + (gated == (p.gate_first != 0) ? i % F : F + i % F) : p.w1);
+  };
+  auto store_bias = [&](int i, bf16x8 v) {
+    const float c = p.b1 == nullptr ? 0.f : (!FOLD ? 1.f : (i < F ? kFoldGate : kFoldValue));
+#pragma unroll
+    for (int e = 0; e < 8; ++e) v[e] = static_cast<bf16_t>(static_cast<float>(v[e]) * c);
+    if (i < 2 * F) *reinterpret_cast<bf16x8*>(bias_lds + i) = v;
+  };
+  const bf16x8 bias_regs = bias_piece(tid * 8 < 2 * F ? tid * 8 : 0);
+  bf16x4 b2v[MBW][4], hwv[MBW][4];  // for the end of the kernel: down-projection bias, readout weight
+  feature_vectors(p.b2, b2v);
+  feature_vectors(p.head_w, hwv);
+  __builtin_amdgcn_sched_barrier(0);
 
   if constexpr (OUTP) {
-    bf16x4 hv[MBW][4], b0v[MBW][4];  // block input and projection bias of the lane's features, in accumulator order
-#pragma unroll
-    for (int m = 0; m < MBW; ++m)
-#pragma unroll
-      for (int jq = 0; jq < 4; ++jq) {
-        const int col = (wave * MBW + m) * 32 + jq * 8 + hh * 4;
-        hv[m][jq] = *reinterpret_cast<const bf16x4*>(p.residual + row * p.ldr + col);
-        if (p.b0 != nullptr) {
-          b0v[m][jq] = *reinterpret_cast<const bf16x4*>(p.b0 + col);
-        } else {
-#pragma unroll
-          for (int e = 0; e < 4; ++e) b0v[m][jq][e] = static_cast<bf16_t>(0.f);
-        }
-      }
+    const float b0_on = p.b0 != nullptr ? 1.f : 0.f;
     float ss = 0.f;
 #pragma unroll
     for (int m = 0; m < MBW; ++m) {
@@ -261,7 +319,7 @@ __global__ __launch_bounds__(4 * kWave, 1) void swiglu_ffn_small_kernel(const Ts
         bf16x4 x1;
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
-          const float lin = static_cast<float>(static_cast<bf16_t>(acc[jq * 4 + e] + static_cast<float>(b0v[m][jq][e])));
+          const float lin = static_cast<float>(static_cast<bf16_t>(fmaf(static_cast<float>(b0v[m][jq][e]), b0_on, acc[jq * 4 + e])));
           x1[e] = static_cast<bf16_t>(lin + static_cast<float>(hv[m][jq][e]));
           const float r = static_cast<float>(x1[e]);
           ss = fmaf(r, r, ss);
@@ -272,9 +330,8 @@ __global__ __launch_bounds__(4 * kWave, 1) void swiglu_ffn_small_kernel(const Ts
     ss = half_wave_pair_sum(ss);
     if (hh == 0) sums[wave * 32 + l32] = ss;
   }
-#pragma unroll
-  for (int i = 0; i < CFRAG; ++i) ring[i] = load_chunk_frag(first, i);
-  __builtin_amdgcn_sched_barrier(0);
+  store_bias(tid * 8, bias_regs);
+  for (int i = (NW * kWave + tid) * 8; i < 2 * F; i += NW * kWave * 8) store_bias(i, bias_piece(i));
   __syncthreads();
   if constexpr (OUTP) {
     float total = 0.f;
@@ -301,8 +358,8 @@ __global__ __launch_bounds__(4 * kWave, 1) void swiglu_ffn_small_kernel(const Ts
   for (int mb = 0; mb < MB; ++mb)
 #pragma unroll
     for (int j = 0; j < 16; ++j) oacc[mb][j] = 0.f;
-  for (int chunk = wave; chunk < nchunks; chunk += NW) {
-    const int next = chunk + NW < nchunks ? chunk + NW : chunk;  // the last chunk is requested once more, and not used
+  for (int chunk = first_chunk; chunk < nchunks; chunk += stride) {
+    const int next = chunk + stride < nchunks ? chunk + stride : chunk;  // the last chunk is requested once more, and not used
     const bf16x8 bg = *reinterpret_cast<const bf16x8*>(bias_lds + chunk * kHU + hh * 8);
     const bf16x8 bu = *reinterpret_cast<const bf16x8*>(bias_lds + F + chunk * kHU + hh * 8);
     f32x16 gu;
@@ -342,26 +399,68 @@ __global__ __launch_bounds__(4 * kWave, 1) void swiglu_ffn_small_kernel(const Ts
       *reinterpret_cast<f32x4*>(smem + wave * kPart + ((mb * 4 + jq) * kWave + lane) * 16) = v;
     }
   __syncthreads();
+  f32x4 total[MBW][4];
+#pragma unroll
+  for (int m = 0; m < MBW; ++m)
+#pragma unroll
+    for (int jq = 0; jq < 4; ++jq) {
+      const int piece = ((wave * MBW + m) * 4 + jq) * kWave + lane;
+      total[m][jq] = *reinterpret_cast<const f32x4*>(smem + piece * 16);
+#pragma unroll
+      for (int w = 1; w < NW; ++w) {
+        const f32x4 v = *reinterpret_cast<const f32x4*>(smem + w * kPart + piece * 16);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) total[m][jq][e] += v[e];
+      }
+    }
+  if (splits > 1) {
+    // The partial of this workgroup becomes visible to the chip, then the workgroup counts itself: whoever counts last finds all
+    // partials of the tile (nobody waits for anybody). They are added in the order of the splits: the same result every run.
+    f32x4* parts = reinterpret_cast<f32x4*>(p.split_partials) + static_cast<int64_t>(blockIdx.x) * splits * (kPart / 16);
+    f32x4* mine = parts + static_cast<int64_t>(blockIdx.y) * (kPart / 16);
+#pragma unroll
+    for (int m = 0; m < MBW; ++m)
+#pragma unroll
+      for (int jq = 0; jq < 4; ++jq) store_through(mine + ((wave * MBW + m) * 4 + jq) * kWave + lane, total[m][jq]);
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // this wavefront's partials have reached the chip's common memory
+    __syncthreads();
+    uint32_t* arrived = reinterpret_cast<uint32_t*>(sums);
+    if (tid == 0)
+      *arrived = __hip_atomic_fetch_add(p.split_counters + blockIdx.x, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    __syncthreads();
+    const bool last = *arrived == static_cast<uint32_t>(splits - 1);
+    __syncthreads();  // (the row sums of the readout reuse the word)
+    if (!last) return;
+    if (tid == 0) p.split_counters[blockIdx.x] = 0u;
+#pragma unroll
+    for (int m = 0; m < MBW; ++m)
+#pragma unroll
+      for (int jq = 0; jq < 4; ++jq)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) total[m][jq][e] = 0.f;
+    for (int w = 0; w < splits; ++w) {
+      const f32x4* other = parts + static_cast<int64_t>(w) * (kPart / 16);
+#pragma unroll
+      for (int m = 0; m < MBW; ++m)
+#pragma unroll
+        for (int jq = 0; jq < 4; ++jq) {
+          const f32x4 v = load_through(other + ((wave * MBW + m) * 4 + jq) * kWave + lane);
+#pragma unroll
+          for (int e = 0; e < 4; ++e) total[m][jq][e] += v[e];
+        }
+    }
+  }
   const bool live = tok0 + l32 < count;
+  const float b2_on = p.b2 != nullptr ? 1.f : 0.f;
   float hdot = 0.f;
 #pragma unroll
   for (int m = 0; m < MBW; ++m)
 #pragma unroll
     for (int jq = 0; jq < 4; ++jq) {
-      const int mb = wave * MBW + m;
-      const int col = mb * 32 + jq * 8 + hh * 4;
-      f32x4 s = *reinterpret_cast<const f32x4*>(smem + ((mb * 4 + jq) * kWave + lane) * 16);
+      const int col = (wave * MBW + m) * 32 + jq * 8 + hh * 4;
+      f32x4 s = total[m][jq];
 #pragma unroll
-      for (int w = 1; w < NW; ++w) {
-        const f32x4 v = *reinterpret_cast<const f32x4*>(smem + w * kPart + ((mb * 4 + jq) * kWave + lane) * 16);
-#pragma unroll
-        for (int e = 0; e < 4; ++e) s[e] += v[e];
-      }
-      if (p.b2 != nullptr) {
-        const bf16x4 b = *reinterpret_cast<const bf16x4*>(p.b2 + col);
-#pragma unroll
-        for (int e = 0; e < 4; ++e) s[e] += static_cast<float>(b[e]);
-      }
+      for (int e = 0; e < 4; ++e) s[e] = fmaf(static_cast<float>(b2v[m][jq][e]), b2_on, s[e]);
       bf16x4 o;
       if constexpr (OUTP) {  // x1 + down, rounded once
         const bf16x4 x1 = *reinterpret_cast<const bf16x4*>(x1_lds + l32 * kRow + col * 2);
@@ -377,11 +476,8 @@ __global__ __launch_bounds__(4 * kWave, 1) void swiglu_ffn_small_kernel(const Ts
         }
       }
       if (live) *reinterpret_cast<bf16x4*>(p.out + row * p.ldo + col) = o;
-      if (p.head_w != nullptr) {
-        const bf16x4 hw = *reinterpret_cast<const bf16x4*>(p.head_w + col);
 #pragma unroll
-        for (int e = 0; e < 4; ++e) hdot = fmaf(static_cast<float>(o[e]), static_cast<float>(hw[e]), hdot);
-      }
+      for (int e = 0; e < 4; ++e) hdot = fmaf(static_cast<float>(o[e]), static_cast<float>(hwv[m][jq][e]), hdot);
     }
   if (p.head_w != nullptr) {
     hdot = half_wave_pair_sum(hdot);
@@ -397,6 +493,22 @@ __global__ __launch_bounds__(4 * kWave, 1) void swiglu_ffn_small_kernel(const Ts
 }
 
 }  // namespace
+
+int ffn_splits(int64_t M, int32_t D, int32_t F) {
+  const int64_t tiles = (M + 31) / 32;
+  const int cus = compute_units();
+  int splits = 1;
+  if (ffn_few_rows(M, D))
+    while (splits < 8 && 2 * splits * tiles <= cus && 2 * splits * 4 * kHU <= F) splits *= 2;
+  return splits;
+}
+
+int64_t ffn_split_bytes(int64_t M, int32_t D, int32_t F) {
+  const int splits = ffn_splits(M, D, F);
+  if (splits == 1) return 0;
+  const int64_t tiles = (M + 31) / 32;
+  return tiles * splits * 32 * D * 4 + (tiles * 4 + 255) / 256 * 256;
+}
 
 int norm_linear_small(const TsParams& p, int32_t K, int qk_mode, hipStream_t s, const char* name) {
   const dim3 grid(static_cast<uint32_t>((p.M + 31) / 32), static_cast<uint32_t>((p.N + K - 1) / K));
@@ -421,7 +533,7 @@ int norm_linear_small(const TsParams& p, int32_t K, int qk_mode, hipStream_t s, 
 int swiglu_ffn_small(const TsParams& p, int32_t D, bool with_proj, bool act_folded, hipStream_t s, const char* name) {
   const size_t lds_bytes = static_cast<size_t>(4) * 32 * D * 4 + 32 * (D * 2 + 16) + static_cast<size_t>(2) * p.F * 2 + 4 * 32 * 4;
   if (lds_bytes > 160 * 1024) return 1;
-  const dim3 grid(static_cast<uint32_t>((p.M + 31) / 32));
+  const dim3 grid(static_cast<uint32_t>((p.M + 31) / 32), p.splits > 1 ? p.splits : 1);
 #define TAAC_SMALL(DD, OO, FF)                                                                                        \
   do {                                                                                                                \
     if (hipFuncSetAttribute(reinterpret_cast<const void*>(swiglu_ffn_small_kernel<DD, OO, FF>),                       \

@@ -63,6 +63,12 @@ struct TsParams {
   // the rounded output), so that a mean-pooling linear head behind the layer need not read the rows again.
   const bf16_t* head_w;     // [D] or null
   float* token_dots;        // [M] (rows like out), written for the tokens the kernel stores
+  // Few-token feed-forward with the hidden units of a 32-token tile divided over `splits` workgroups (0: one): every workgroup
+  // leaves its fp32 partial in split_partials [tile][splits][32 x D] and counts itself in split_counters [tile] (zero before
+  // the launch); the last one to arrive adds the partials up in order, finishes the tile and sets the counter back to zero.
+  int32_t splits;
+  float* split_partials;
+  uint32_t* split_counters;
 };
 
 // The few-token form of the projection (ffn_small.hip): packed weights, the norm in front folded into them or absent.

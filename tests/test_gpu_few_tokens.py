@@ -6,7 +6,8 @@ from __future__ import annotations
 import pytest
 import torch
 
-from taac_2026_amd.api import (attention_out_ffn, attention_out_ffn_heads, norm_linear, norm_linear_heads, qkv_projection,
+from taac_2026_amd import workloads
+from taac_2026_amd.api import (PCVRBackbone, attention_out_ffn, attention_out_ffn_heads, norm_linear, norm_linear_heads, qkv_projection,
                                swiglu_ffn, valid_rows)
 
 pytestmark = pytest.mark.gpu
@@ -96,3 +97,24 @@ def test_feed_forward_matches_the_persistent_kernel(device, test_hooks, m, d, f,
         held = res.clone()
         attention_out_ffn(x, wo, bo, held, wu, bu, wd, bd, norm_weight=nw, out=held)
         assert torch.equal(held, attention_out_ffn(x, wo, bo, res, wu, bu, wd, bd, norm_weight=nw))
+
+
+@pytest.mark.parametrize("batch,sequence,d_model,heads,d_ff", [(1, 20, 256, 8, 1024), (1, 480, 256, 8, 1024), (5, 90, 256, 4, 64),
+                                                               (16, 120, 256, 8, 512), (3, 61, 128, 4, 256)])
+def test_backbone_with_hidden_units_divided_over_workgroups(device, test_hooks, batch, sequence, d_model, heads, d_ff):
+    """Batches small enough for 2 to 8 workgroups per token tile, against the persistent kernels and from run to run (the
+    partial sums are added in a fixed order, whoever arrives last). Bound of the hidden state: roundings of the blocks'
+    outputs flip by one bf16 step (2**-8 relative) and travel through the following blocks."""
+    inputs = workloads.backbone_inputs(batch=batch, n_feature_tokens=8, n_sequence_tokens=sequence, d_model=d_model,
+                                       num_heads=heads, d_ff=d_ff, n_blocks=2, min_sequence_len=1, seed=batch)
+    model = PCVRBackbone(d_model=d_model, num_heads=heads, d_ff=d_ff, n_blocks=2)
+    workloads.load_backbone_state(model, inputs)
+    model = model.to(device=device, dtype=torch.bfloat16).eval()
+    emb, lengths = 50 * inputs.emb.to(device), inputs.key_lengths.to(device)
+    with torch.no_grad():
+        (p, h), (p_large, h_large) = _both(test_hooks, lambda: model(emb, lengths, return_hidden=True))
+        torch.testing.assert_close(p, p_large, rtol=0, atol=2e-3)
+        torch.testing.assert_close(h.float(), h_large.float(), rtol=2 ** -5, atol=2 ** -4)
+        for _ in range(3):
+            again, h_again = model(emb, lengths, return_hidden=True)
+            assert torch.equal(again, p) and torch.equal(h_again, h)
