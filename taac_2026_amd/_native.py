@@ -347,7 +347,10 @@ def ptr(tensor: torch.Tensor | None) -> int | None:
 
 
 def current_stream(device: torch.device) -> int:
-    return torch.cuda.current_stream(device).cuda_stream
+    """The raw stream of the calling thread on ``device`` (without a ``torch.cuda.Stream`` object around it: 0.2 instead of 2.5
+    us per operator call)."""
+    index = device.index
+    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device() if index is None else index)
 
 
 __all__ = [

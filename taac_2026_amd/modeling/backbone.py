@@ -536,25 +536,29 @@ class PCVRBackbone(nn.Module):
 
         keep_alive: list[torch.Tensor] = []
 
-        def dev(parameter: torch.Tensor | None) -> int | None:
-            tensor = _bf16(parameter)
-            if tensor is None:
+        def dev(module: nn.Module | None, name: str) -> int | None:
+            # (the registries directly: attribute lookups on modules and no-op conversions of 42 parameters are most of what
+            # the host does in this call)
+            parameter = None if module is None else module._parameters[name]
+            if parameter is None:
                 return None
-            tensor = tensor.detach().contiguous()
+            if parameter.dtype is torch.bfloat16 and parameter.is_contiguous():
+                return parameter.data_ptr()
+            tensor = _bf16(parameter).detach().contiguous()
             keep_alive.append(tensor)
             return tensor.data_ptr()
 
         packed = (_native.BlockWeights * len(self.blocks))()
         for slot, block in zip(packed, self.blocks):
-            slot.attn_norm_weight = dev(block.attn_norm.weight)
-            slot.qkv_weight, slot.qkv_bias = dev(block.qkv.weight), dev(block.qkv.bias)
-            slot.out_weight, slot.out_bias = dev(block.out.weight), dev(block.out.bias)
-            slot.ffn_norm_weight = dev(block.ffn_norm.weight)
-            slot.up_weight, slot.up_bias = dev(block.up.weight), dev(block.up.bias)
-            slot.down_weight, slot.down_bias = dev(block.down.weight), dev(block.down.bias)
-            if block.query_norm is not None:
-                slot.query_norm_weight = dev(block.query_norm.weight)
-                slot.key_norm_weight = dev(block.key_norm.weight)
+            parts = block._modules
+            slot.attn_norm_weight = dev(parts["attn_norm"], "weight")
+            slot.qkv_weight, slot.qkv_bias = dev(parts["qkv"], "weight"), dev(parts["qkv"], "bias")
+            slot.out_weight, slot.out_bias = dev(parts["out"], "weight"), dev(parts["out"], "bias")
+            slot.ffn_norm_weight = dev(parts["ffn_norm"], "weight")
+            slot.up_weight, slot.up_bias = dev(parts["up"], "weight"), dev(parts["up"], "bias")
+            slot.down_weight, slot.down_bias = dev(parts["down"], "weight"), dev(parts["down"], "bias")
+            slot.query_norm_weight = dev(parts.get("query_norm"), "weight")
+            slot.key_norm_weight = dev(parts.get("key_norm"), "weight")
         table = None
         if self.rope_base is not None:
             table = rope_table(tokens, self.d_model // self.num_heads, self.rope_base, torch.bfloat16, emb.device)
@@ -566,8 +570,8 @@ class PCVRBackbone(nn.Module):
                  | (_native.BACKBONE_FP8 if fp8 else 0) | (_native.BACKBONE_ROW_MAJOR_QKV if row_major_qkv else 0))
         probabilities = torch.empty(batch, dtype=torch.float32, device=emb.device)
         status = library.taac_backbone_fwd(
-            emb.data_ptr(), key_lengths.data_ptr(), packed, len(self.blocks), dev(self.head.weight.reshape(-1)),
-            dev(self.head.bias), batch, tokens, self.d_model, self.num_heads, self.d_ff, ctypes.c_float(self.eps),
+            emb.data_ptr(), key_lengths.data_ptr(), packed, len(self.blocks), dev(self.head, "weight"),
+            dev(self.head, "bias"), batch, tokens, self.d_model, self.num_heads, self.d_ff, ctypes.c_float(self.eps),
             _native.ptr(table), flags, workspace.data_ptr(), workspace.numel(), _native.ptr(hidden),
             probabilities.data_ptr(),
             _native.current_stream(emb.device),
