@@ -901,6 +901,46 @@ int taac_backbone_fwd(const void* emb, const int32_t* key_lengths, const taac_bl
                       float eps, const void* rope_cos_sin, int flags, void* workspace, int64_t workspace_bytes,
                       void* hidden_out, float* p, void* stream);
 
+/*
+ * Training of a stack of n_blocks interaction blocks (experiments/symbiosis/backbone.py:51-68; no rotary embedding, no dropout)
+ * and, optionally, of the pCVR readout behind it, over the valid tokens only (padded tokens pass through the stack, as the
+ * reference's `update * ~padding_mask` makes them): the forward keeps what the backward needs in `saved`, both use `scratch`
+ * while they run. Replaces the autograd graph of the reference's blocks under torch. No host synchronisation.
+ *
+ * taac_stack_train_bytes: bytes of `saved` (what = 0), of the forward's scratch (1), of the backward's scratch (2); -1 when the
+ * shape is not covered (D = 128 / 256, D / H = 32 / 64, F a multiple of 32 within taac_swiglu_ffn_bwd_packed_bytes). Both buffers
+ * 256-byte aligned.
+ *
+ * tokens: bf16 [B, T, D]. Valid tokens: t < key_lengths[b] (rows_given NULL), or any pattern: rows_given / count_given as written
+ * by taac_valid_rows_from_bits, valid_bits the words it was built from, key_lengths the samples' numbers of valid tokens;
+ * struct_bits (with rows_given; NULL: all pairs of valid tokens) the visibility among a sample's valid tokens in their order
+ * ([T, ceil(T / 32)] words per sample, struct_sample_stride words apart: taac_mask_front_bits).
+ * blocks: weights of dtype param_dtype (TAAC_BF16, or TAAC_F32 masters, which are rounded to bf16); query / key norm weights in
+ * all blocks or in none. head_w [D], head_b [1] (may be NULL), p float [B]: pCVR readout of the masked mean, all three NULL for
+ * none. out: bf16 [B, T, D] or NULL; its padded rows repeat the tokens, or are zeros with zero_padded_rows. attn_tokens_out: the
+ * tokens between the halves of the LAST block, or NULL.
+ *
+ * Backward: grad_out / grad_attn_tokens (bf16 [B, T, D]) and grad_p (float [B]) may be NULL (at least one is given;
+ * grad_attn_tokens only for a stack of one block). grads: where every block's gradients go, of dtype param_dtype; a NULL bias
+ * gradient is not computed. When neither grad_out nor grad_p is given no gradient reaches the feed-forward half and its
+ * gradients are left untouched. grad_tokens: bf16 [B, T, D] or NULL; padded rows receive grad_out + grad_attn_tokens, or zeros
+ * with zero_padded_rows.
+ */
+int64_t taac_stack_train_bytes(int32_t B, int32_t T, int32_t D, int32_t H, int32_t F, int32_t n_blocks, int qk_norm, int what);
+int taac_stack_train_fwd(const void* tokens, const int32_t* key_lengths, const int32_t* rows_given, const int32_t* count_given,
+                         const uint32_t* valid_bits, const uint32_t* struct_bits, int64_t struct_sample_stride,
+                         const taac_block_weights* blocks, int32_t n_blocks, int param_dtype, int32_t B, int32_t T, int32_t D,
+                         int32_t H, int32_t F, float attn_eps, float ffn_eps, float qk_eps, int gate_first, const void* head_w,
+                         const void* head_b, void* saved, void* scratch, void* out, int zero_padded_rows, void* attn_tokens_out,
+                         float* p, void* stream);
+int taac_stack_train_bwd(const void* grad_out, const void* grad_attn_tokens, const float* grad_p, const float* p,
+                         const int32_t* key_lengths, const int32_t* rows_given, const int32_t* count_given,
+                         const uint32_t* valid_bits, const uint32_t* struct_bits, int64_t struct_sample_stride,
+                         const taac_block_weights* blocks, const taac_block_weights* grads, int32_t n_blocks, int param_dtype,
+                         int32_t B, int32_t T, int32_t D, int32_t H, int32_t F, float qk_eps, int gate_first, void* grad_head_w,
+                         void* grad_head_b, int zero_padded_rows, const void* saved, void* scratch, void* grad_tokens,
+                         void* stream);
+
 #ifdef __cplusplus
 }
 #endif

@@ -65,6 +65,8 @@ struct AttnParams {
   int64_t qs[4], ks[4], vs[4], os[4];
   float scale_log2;  // log2(e) / sqrt(d)
   int32_t zero_pad;
+  const int32_t* row_offsets;  // direct-transfer kernel: sample b's rows start at row row_offsets[b] of q, k, v and o (a compact
+                               // tensor of the batch's valid tokens) instead of at b times the batch strides; or null
   uint32_t nqc;    // query chunks per (batch, head)
   uint32_t total;  // workgroups
   uint32_t nqc_magic, h_magic;  // floor(2^32 / nqc), floor(2^32 / H) (0 for a divisor of 1): divisions without a divide
@@ -636,10 +638,13 @@ __global__ __launch_bounds__(kThreads) void flash_attn_fwd_dma_kernel(const Attn
   const int qc_a = static_cast<int>(qg_u);
   const int qc_b = p.pair_blocks ? static_cast<int>(p.nqc) - 1 - qc_a : qc_a;
 
-  const T* qb = static_cast<const T*>(p.q) + b * p.qs[0] + h * p.qs[1];
-  const T* kb = static_cast<const T*>(p.k) + b * p.ks[0] + h * p.ks[1];
-  const T* vb = static_cast<const T*>(p.v) + b * p.vs[0] + h * p.vs[1];
-  T* ob = static_cast<T*>(p.o) + b * p.os[0] + h * p.os[1];
+  // first row of the sample: one scalar load in the compact layout, a product otherwise
+  const bool compact = p.row_offsets != nullptr;
+  const int64_t row0 = compact ? p.row_offsets[b] : b;
+  const T* qb = static_cast<const T*>(p.q) + row0 * (compact ? p.qs[2] : p.qs[0]) + h * p.qs[1];
+  const T* kb = static_cast<const T*>(p.k) + row0 * (compact ? p.ks[2] : p.ks[0]) + h * p.ks[1];
+  const T* vb = static_cast<const T*>(p.v) + row0 * (compact ? p.vs[2] : p.vs[0]) + h * p.vs[1];
+  T* ob = static_cast<T*>(p.o) + row0 * (compact ? p.os[2] : p.os[0]) + h * p.os[1];
 
   int len = p.Tk;
   if (p.key_lengths != nullptr) {
@@ -1469,7 +1474,7 @@ int attention_entry(const char* name, const void* q, const void* k, const void* 
                     float* lse, float* amax_out, void* o, int32_t B, int32_t H, int32_t Tq, int32_t Tk, int32_t d, const int64_t q_strides[4],
                     const int64_t k_strides[4], const int64_t v_strides[4], const int64_t o_strides[4], int mask_flags,
                     int zero_padded_queries, int dtype, void* stream, const uint8_t* drop_mask = nullptr,
-                    float drop_scale = 1.f) {
+                    float drop_scale = 1.f, const int32_t* row_offsets = nullptr) {
   if (drop_mask != nullptr && (mask.self_bits != nullptr || mask.compact_keys != nullptr || q_row_scale != nullptr ||
                                k_row_scale != nullptr || q_col_scale != nullptr))
     return set_error(TAAC_ERR_UNSUPPORTED, "%s: dropout does not come with self-only query rows or row factors", name);
@@ -1523,6 +1528,7 @@ int attention_entry(const char* name, const void* q, const void* k, const void* 
   p.drop_mask = drop_mask;
   p.drop_scale = drop_scale;
   p.lse = lse;
+  p.row_offsets = row_offsets;
   p.struct_bits = mask.struct_bits;
   p.struct_stride = mask.struct_stride;
   p.valid_bits = mask.valid_bits;
@@ -1571,6 +1577,22 @@ int attention_entry(const char* name, const void* q, const void* k, const void* 
 }
 
 }  // namespace
+}  // namespace taac
+
+namespace taac {
+int attention_compact_fwd(const char* name, const void* qk, const void* v, int64_t ld_qk, int64_t ld_v, const int32_t* lengths,
+                          const int32_t* row_offsets, const uint32_t* struct_bits, int64_t struct_stride, void* o, int64_t ld_o,
+                          float* lse, int32_t B, int32_t H, int32_t T, int32_t dh, hipStream_t s) {
+  if (dh != 32 && dh != 64) return set_error(TAAC_ERR_UNSUPPORTED, "%s: head dims 32 and 64", name);
+  MaskArgs mask;
+  mask.struct_bits = struct_bits;
+  mask.struct_stride = struct_stride;
+  const int64_t width = static_cast<int64_t>(H) * dh;
+  const int64_t qs[4] = {0, dh, ld_qk, 1}, vs[4] = {0, dh, ld_v, 1}, os[4] = {0, dh, ld_o, 1};
+  const bf16_t* q = static_cast<const bf16_t*>(qk);
+  return attention_entry(name, q, q + width, v, lengths, mask, nullptr, nullptr, nullptr, lse, nullptr, o, B, H, T, T, dh, qs, qs,
+                         vs, os, 0, 2, TAAC_BF16, s, nullptr, 1.f, row_offsets);
+}
 }  // namespace taac
 
 extern "C" int taac_flash_attn_fwd(const void* q, const void* k, const void* v, const int32_t* key_lengths, void* o,

@@ -47,12 +47,21 @@ struct AttnBwdParams {
   float drop_scale;          // 1 / (1 - p)
   int32_t B, H, Tq, Tk, d;
   int64_t qs[4], ks[4], vs[4], os[4], dos[4], dqs[4], dks[4], dvs[4];
+  const int32_t* row_offsets;  // sample b's rows start at row row_offsets[b] of every tensor (a compact tensor of the batch's valid
+                               // tokens: rows at or beyond the length belong to the next sample and are not written), or null
   float scale;            // 1 / sqrt(d)
   int32_t zero_pad;       // query rows at or beyond key_lengths[b] carry no gradient
   int32_t causal;
   uint32_t nblk;          // owned-row blocks per (batch, head)
   uint32_t total;
 };
+
+// First row of (sample b, head h).
+template <typename T>
+__device__ __forceinline__ T* head_rows(T* base, const int64_t (&strides)[4], const AttnBwdParams& p, int b, int h) {
+  const int64_t row0 = p.row_offsets != nullptr ? p.row_offsets[b] * strides[2] : b * strides[0];
+  return base + row0 + h * strides[1];
+}
 
 template <typename T>
 struct Mfma32;
@@ -300,12 +309,12 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(DP == 
   const int bh = static_cast<int>(logical / p.nblk);
   const int h = bh % p.H, b = bh / p.H;
   const int tid = threadIdx.x, wave = tid / kWave, lane = tid % kWave, l32 = lane % 32, hh = lane / 32;
-  const T* qb = static_cast<const T*>(p.q) + b * p.qs[0] + h * p.qs[1];
-  const T* kb = static_cast<const T*>(p.k) + b * p.ks[0] + h * p.ks[1];
-  const T* vb = static_cast<const T*>(p.v) + b * p.vs[0] + h * p.vs[1];
-  const T* ob = static_cast<const T*>(p.o) + b * p.os[0] + h * p.os[1];
-  const T* dob = static_cast<const T*>(p.dout) + b * p.dos[0] + h * p.dos[1];
-  T* dqb = static_cast<T*>(p.dq) + b * p.dqs[0] + h * p.dqs[1];
+  const T* qb = head_rows(static_cast<const T*>(p.q), p.qs, p, b, h);
+  const T* kb = head_rows(static_cast<const T*>(p.k), p.ks, p, b, h);
+  const T* vb = head_rows(static_cast<const T*>(p.v), p.vs, p, b, h);
+  const T* ob = head_rows(static_cast<const T*>(p.o), p.os, p, b, h);
+  const T* dob = head_rows(static_cast<const T*>(p.dout), p.dos, p, b, h);
+  T* dqb = head_rows(static_cast<T*>(p.dq), p.dqs, p, b, h);
 
   int len = p.Tk;
   if (p.key_lengths != nullptr) {
@@ -479,7 +488,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(DP == 
     }
   }
   __syncthreads();  // the staging buffers now hold the output tiles
-  store_owned<T, DP>(dqacc, smem + wave * (32 * OROW), dqb, p.dqs[2], q_begin + wave * 32, p.Tq, p.d, lane);
+  store_owned<T, DP>(dqacc, smem + wave * (32 * OROW), dqb, p.dqs[2], q_begin + wave * 32, p.row_offsets != nullptr ? len : p.Tq, p.d, lane);
 }
 
 template <typename T, int DP, bool DMA, int MODE = kMaskNone>
@@ -504,12 +513,12 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu((DP ==
   const int bh = static_cast<int>(logical / p.nblk);
   const int h = bh % p.H, b = bh / p.H;
   const int tid = threadIdx.x, wave = tid / kWave, lane = tid % kWave, l32 = lane % 32, hh = lane / 32;
-  const T* qb = static_cast<const T*>(p.q) + b * p.qs[0] + h * p.qs[1];
-  const T* kb = static_cast<const T*>(p.k) + b * p.ks[0] + h * p.ks[1];
-  const T* vb = static_cast<const T*>(p.v) + b * p.vs[0] + h * p.vs[1];
-  const T* dob = static_cast<const T*>(p.dout) + b * p.dos[0] + h * p.dos[1];
-  T* dkb = static_cast<T*>(p.dk) + b * p.dks[0] + h * p.dks[1];
-  T* dvb = static_cast<T*>(p.dv) + b * p.dvs[0] + h * p.dvs[1];
+  const T* qb = head_rows(static_cast<const T*>(p.q), p.qs, p, b, h);
+  const T* kb = head_rows(static_cast<const T*>(p.k), p.ks, p, b, h);
+  const T* vb = head_rows(static_cast<const T*>(p.v), p.vs, p, b, h);
+  const T* dob = head_rows(static_cast<const T*>(p.dout), p.dos, p, b, h);
+  T* dkb = head_rows(static_cast<T*>(p.dk), p.dks, p, b, h);
+  T* dvb = head_rows(static_cast<T*>(p.dv), p.dvs, p, b, h);
 
   int len = p.Tk;
   if (p.key_lengths != nullptr) {
@@ -679,9 +688,10 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu((DP ==
   }
   __syncthreads();
   uint8_t* tile = smem + wave * (32 * OROW);
-  store_owned<T, DP>(dkacc, tile, dkb, p.dks[2], k_begin + wave * 32, p.Tk, p.d, lane);
+  const int k_store_end = p.row_offsets != nullptr ? len : p.Tk;
+  store_owned<T, DP>(dkacc, tile, dkb, p.dks[2], k_begin + wave * 32, k_store_end, p.d, lane);
   asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-  store_owned<T, DP>(dvacc, tile, dvb, p.dvs[2], k_begin + wave * 32, p.Tk, p.d, lane);
+  store_owned<T, DP>(dvacc, tile, dvb, p.dvs[2], k_begin + wave * 32, k_store_end, p.d, lane);
 }
 
 bool strides_ok(const int64_t* st) {
@@ -748,7 +758,8 @@ int attention_bwd_entry(const char* name, const void* q, const void* k, const vo
                         const int64_t o_strides[4], const int64_t do_strides[4], const int64_t dq_strides[4],
                         const int64_t dk_strides[4], const int64_t dv_strides[4], int is_causal, int zero_padded_queries,
                         int dtype, void* stream, int mask_mode = -1, int64_t mask_bs = 0, int64_t mask_hs = 0,
-                        const uint8_t* key_valid = nullptr, const uint32_t* bit_words = nullptr, int64_t bits_bs = 0) {
+                        const uint8_t* key_valid = nullptr, const uint32_t* bit_words = nullptr, int64_t bits_bs = 0,
+                        const int32_t* row_offsets = nullptr) {
   // mask_mode -1: dropout when a mask is given (its matrices follow the (B, H) order), nothing otherwise
   if (mask_mode < 0 || mask_mode == kMaskBitsDropout) {
     if (mask_mode < 0) mask_mode = drop_mask != nullptr ? kMaskDropout : kMaskNone;
@@ -802,6 +813,7 @@ int attention_bwd_entry(const char* name, const void* q, const void* k, const vo
   p.key_valid = key_valid;
   p.bit_words = bit_words;
   p.bits_bs = bits_bs;
+  p.row_offsets = row_offsets;
   p.drop_scale = drop_scale;
   p.B = B;
   p.H = H;
@@ -829,6 +841,22 @@ int attention_bwd_entry(const char* name, const void* q, const void* k, const vo
   return check_launch(name);
 }
 }  // namespace
+}  // namespace taac
+
+namespace taac {
+int attention_compact_bwd(const char* name, const void* qk, const void* v, int64_t ld_qk, int64_t ld_v, const void* o, int64_t ld_o,
+                          const void* dout, int64_t ld_do, const float* lse, const int32_t* lengths, const int32_t* row_offsets,
+                          const uint32_t* struct_bits, int64_t struct_stride, void* dqkv, int64_t ld_dqkv, float* delta, int32_t B,
+                          int32_t H, int32_t T, int32_t dh, hipStream_t s) {
+  const int64_t width = static_cast<int64_t>(H) * dh;
+  const int64_t qs[4] = {0, dh, ld_qk, 1}, vs[4] = {0, dh, ld_v, 1}, os[4] = {0, dh, ld_o, 1}, dos[4] = {0, dh, ld_do, 1},
+                gs[4] = {0, dh, ld_dqkv, 1};
+  const bf16_t* q = static_cast<const bf16_t*>(qk);
+  bf16_t* g = static_cast<bf16_t*>(dqkv);
+  return attention_bwd_entry(name, q, q + width, v, o, dout, lse, lengths, nullptr, 1.f, g, g + width, g + 2 * width, delta, B, H,
+                             T, T, dh, qs, qs, vs, os, dos, gs, gs, gs, 0, 1, TAAC_BF16, s,
+                             struct_bits != nullptr ? kMaskBits : -1, 0, 0, nullptr, struct_bits, struct_stride, row_offsets);
+}
 }  // namespace taac
 
 extern "C" int taac_flash_attn_bwd(const void* q, const void* k, const void* v, const void* o, const void* dout,

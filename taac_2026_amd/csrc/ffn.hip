@@ -24,50 +24,12 @@
 // of roundings of the reference's bf16 evaluation (linear output rounded, then the residual add rounded).
 #include "common.h"
 #include "ts_common.h"
+#include "pack.h"
 #include "row_index.h"
 #include "ts_dense.h"
 
 namespace taac {
 namespace {
-
-// ---- fragment-order packing ------------------------------------------------------------------------------------------
-// FFN blob: step s (32 hidden units) holds, for chunk q = 0, 1: KS up fragments (k-step r) then MB down fragments
-// (row block r - KS); exactly the image one barrier step needs in LDS. A fragment is 64 lanes x 16 bytes.
-// col_scale (optional, [D]): weight of the RMSNorm in front of the up projection, folded into its fragments (see
-// linear_pack_piece).
-// fold_act: the constants of the gate's activation join the same rounding - the gated half is multiplied by -log2(e), the
-// other half by -ln 2, so that silu(g) * u = g' * u' / (1 + 2^g') with g' and u' as they leave the matrix unit (the
-// kernel's FOLD form: one multiplication less per hidden unit and token; the first-layer bias is scaled when it is staged).
-__device__ __forceinline__ void ffn_pack_piece(const bf16_t* __restrict__ w_up, const bf16_t* __restrict__ w_down,
-                                               bf16x8* __restrict__ packed, int D, int F, int gate_first, int64_t gid,
-                                               const bf16_t* __restrict__ col_scale = nullptr, bool fold_act = false) {
-  const int KS = D / 16, MB = D / 32, CFRAG = KS + MB, NFRAG = kCPB * CFRAG;
-  const int lane = static_cast<int>(gid % 64);
-  const int f = static_cast<int>((gid / 64) % NFRAG);
-  const int64_t step = gid / 64 / NFRAG;
-  const int q = f / CFRAG, r = f % CFRAG;
-  const int64_t unit0 = (step * kCPB + q) * kHU;
-  const int l32 = lane % 32, hh = lane / 32;
-  const bf16_t* src;
-  if (r < KS)
-    src = w_up + (((l32 < 16) == (gate_first != 0) ? 0 : F) + unit0 + up_unit_of_slot(l32 & 15)) * D + r * 16 + hh * 8;
-  else
-    src = w_down + static_cast<int64_t>((r - KS) * 32 + l32) * F + unit0 + hh * 8;
-  bf16x8 v = *reinterpret_cast<const bf16x8*>(src);
-  if ((col_scale != nullptr || fold_act) && r < KS) {
-    bf16x8 g;
-    if (col_scale != nullptr) {
-      g = *reinterpret_cast<const bf16x8*>(col_scale + r * 16 + hh * 8);
-    } else {
-#pragma unroll
-      for (int e = 0; e < 8; ++e) g[e] = static_cast<bf16_t>(1.0f);
-    }
-    const float c = fold_act ? (l32 < 16 ? kFoldGate : kFoldValue) : 1.0f;
-#pragma unroll
-    for (int e = 0; e < 8; ++e) v[e] = static_cast<bf16_t>(static_cast<float>(v[e]) * static_cast<float>(g[e]) * c);
-  }
-  packed[gid] = v;
-}
 
 __global__ void ffn_pack_kernel(const bf16_t* __restrict__ w_up, const bf16_t* __restrict__ w_down,
                                 bf16x8* __restrict__ packed, int D, int F, int gate_first,
@@ -96,27 +58,6 @@ __global__ void mlp_pack_kernel(const bf16_t* __restrict__ w1, const bf16_t* __r
   else
     src = w2 + static_cast<int64_t>(((r - KS) % MB) * 32 + l32) * F + unit0 + ((r - KS) / MB) * 16 + hh * 8;
   packed[gid] = *reinterpret_cast<const bf16x8*>(src);
-}
-
-// Linear blob: chunk c (64 output features) holds fragments (row block rb, k-step ks) at index rb * KS + ks.
-// col_scale (optional, [K]): every weight is multiplied by the factor of its input feature and rounded once - the weight
-// of an RMSNorm in front of the layer, folded into the layer (linear(x * r * g) = r * linear_g(x) with linear_g's weights
-// w[n, k] * g[k]; the kernel then applies the per-token factor r to its accumulators).
-__device__ __forceinline__ void linear_pack_piece(const bf16_t* __restrict__ w, bf16x8* __restrict__ packed, int K,
-                                                  int64_t gid, const bf16_t* __restrict__ col_scale = nullptr) {
-  const int KS = K / 16, NFRAG = 2 * KS;
-  const int lane = static_cast<int>(gid % 64);
-  const int f = static_cast<int>((gid / 64) % NFRAG);
-  const int64_t chunk = gid / 64 / NFRAG;
-  const int l32 = lane % 32, hh = lane / 32;
-  const int col = (f % KS) * 16 + hh * 8;
-  bf16x8 v = *reinterpret_cast<const bf16x8*>(w + (chunk * kNC + (f / KS) * 32 + l32) * K + col);
-  if (col_scale != nullptr) {
-    const bf16x8 g = *reinterpret_cast<const bf16x8*>(col_scale + col);
-#pragma unroll
-    for (int e = 0; e < 8; ++e) v[e] = static_cast<bf16_t>(static_cast<float>(v[e]) * static_cast<float>(g[e]));
-  }
-  packed[gid] = v;
 }
 
 __global__ void linear_pack_kernel(const bf16_t* __restrict__ w, bf16x8* __restrict__ packed, int N, int K,
@@ -268,8 +209,11 @@ __device__ __forceinline__ void load_residual(const bf16_t* residual, int64_t ld
 // the gate layer reads the normalised block input, which only the projection kernel in front of attention holds, so
 // it arrives as a tensor). Its pieces of a chunk are requested behind the chunk's MFMAs, into the registers the weight
 // fragments have left, so the variant takes no registers of its own.
+//
+// KEEP (with OUTP): the training forward; x1 and the norm's factor are stored for the backward (p.x1_out, p.rstd_out). A variant
+// of its own: with a run-time test the serving kernel takes 532 instead of 475 us per block of 285 k tokens (D = 256, F = 1024).
 // ------------------------------------------------------------------------------------------------------------------
-template <int D, int TT, int NWAVES, int CPB, bool DEFER, bool OUTP, bool GATE = false, bool GLU = true, bool FOLD = false>
+template <int D, int TT, int NWAVES, int CPB, bool DEFER, bool OUTP, bool GATE = false, bool GLU = true, bool FOLD = false, bool KEEP = false>
 __global__ __launch_bounds__(NWAVES * kWave, TT == 1 ? 2 : 1) void swiglu_ffn_kernel(const TsParams p) {
   static_assert(!GATE || OUTP, "the gate belongs to the projection in front");
   static_assert(!FOLD || GLU, "the folded constants belong to the gated form");
@@ -674,6 +618,27 @@ __global__ __launch_bounds__(NWAVES * kWave, TT == 1 ? 2 : 1) void swiglu_ffn_ke
                               static_cast<uint32_t>(r1[1])};
           xf[t][ks] = __builtin_bit_cast(bf16x8, frag);
         });
+        if constexpr (KEEP) {
+          if (hh == 0) p.rstd_out[hrow_index[t]] = scale;
+          // x1 itself in the same fragment form: 16-byte stores, two lanes per 32-byte run of a row
+          bf16_t* x1row = p.x1_out + hrow_index[t] * D + hh * 8;
+          static_for<KS>([&](auto kc) {
+            constexpr int ks = decltype(kc)::value;
+            constexpr int mb = ks / 2, jq = 2 * (ks % 2);
+            bf16x4 lo, hi;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+              lo[e] = static_cast<bf16_t>(oacc[t][mb][jq * 4 + e]);
+              hi[e] = static_cast<bf16_t>(oacc[t][mb][(jq + 1) * 4 + e]);
+            }
+            const u32x2 ul = __builtin_bit_cast(u32x2, lo), uh = __builtin_bit_cast(u32x2, hi);
+            const auto r0 = __builtin_amdgcn_permlane32_swap(ul[0], uh[0], false, false);
+            const auto r1 = __builtin_amdgcn_permlane32_swap(ul[1], uh[1], false, false);
+            const u32x4 frag = {static_cast<uint32_t>(r0[0]), static_cast<uint32_t>(r1[0]), static_cast<uint32_t>(r0[1]),
+                                static_cast<uint32_t>(r1[1])};
+            *reinterpret_cast<bf16x8*>(x1row + ks * 16) = __builtin_bit_cast(bf16x8, frag);
+          });
+        }
       }
     }
   }
@@ -1051,10 +1016,16 @@ __global__ __launch_bounds__(8 * kWave, 2) void norm_linear_kernel(const TsParam
   for (int t = 0; t < TT; ++t) rstd[t] = 1.0f;
   auto apply_norm = [&]() {
     if (p.norm_w == nullptr) return;
-    if (p.norm_folded)
+    if (p.norm_folded) {
       token_rstd<D, TT>(p.eps, xf, rstd);
-    else
+      if (p.rstd_out != nullptr) {  // (the workgroups that share a tile write the same values)
+#pragma unroll
+        for (int t = 0; t < TT; ++t)
+          if (hh == 0) p.rstd_out[token_row(p, count, tok_wave + t * 32 + l32)] = rstd[t];
+      }
+    } else {
       normalize_tokens<D, TT>(p.eps, bias_lds + p.N, hh, xf);
+    }
   };
   apply_norm();
 
@@ -1447,7 +1418,8 @@ int ffn_entry(const char* name, const void* x, int64_t ldx, const void* out_bias
               int64_t M, int32_t D, int32_t F, int gate_first, const int32_t* rows, const int32_t* n_rows,
               const int32_t* x_rows, int norm_folded, void* stream, const void* update_gate = nullptr, int64_t ldg = 0,
               bool glu = true, int x_plane = 0, const void* head_w = nullptr, float* token_dots = nullptr,
-              void* split_scratch = nullptr) {
+              void* split_scratch = nullptr, const int32_t* count = nullptr, void* x1_out = nullptr,
+              float* rstd_out = nullptr) {
   const bool with_proj = out_packed != nullptr;
   if (norm_folded < 0 || norm_folded > (TAAC_FOLDED_NORM | TAAC_FOLDED_ACTIVATION))
     return set_error(TAAC_ERR_INVALID_VALUE, "%s: norm_folded holds TAAC_FOLDED_NORM and / or TAAC_FOLDED_ACTIVATION", name);
@@ -1522,6 +1494,9 @@ int ffn_entry(const char* name, const void* x, int64_t ldx, const void* out_bias
   p.x_plane_shift = x_plane == 32 ? 5 : (x_plane == 64 ? 6 : 0);
   p.head_w = static_cast<const bf16_t*>(head_w);
   p.token_dots = token_dots;
+  if (count != nullptr) p.n_rows = count;
+  p.x1_out = static_cast<bf16_t*>(x1_out);
+  p.rstd_out = rstd_out;
   p.units = compute_units();
   if (p.units <= 0) return set_error(TAAC_ERR_LAUNCH, "%s: cannot query the device", name);
   if (const int limit = test_max_workgroups(); limit > 0 && limit < p.units) p.units = limit;  // taac_test_hooks
@@ -1548,6 +1523,14 @@ int ffn_entry(const char* name, const void* x, int64_t ldx, const void* out_bias
   if (with_proj && update_gate) {
     if (D == 256) TAAC_FFN_LAUNCH(256, 1, 8, 2, true, true, true);
     TAAC_FFN_LAUNCH(128, 1, 8, 2, true, true, true);
+  }
+  if (with_proj && x1_out != nullptr) {  // the training forward: x1 and the norm's factor are stored on the way
+    if (act_folded) {
+      if (D == 256) TAAC_FFN_LAUNCH(256, 1, 8, 2, true, true, false, true, true, true);
+      TAAC_FFN_LAUNCH(128, 1, 8, 2, true, true, false, true, true, true);
+    }
+    if (D == 256) TAAC_FFN_LAUNCH(256, 1, 8, 2, true, true, false, true, false, true);
+    TAAC_FFN_LAUNCH(128, 1, 8, 2, true, true, false, true, false, true);
   }
   if (with_proj && act_folded) {
     if (D == 256) TAAC_FFN_LAUNCH(256, 1, 8, 2, true, true, false, true, true);
@@ -1665,7 +1648,8 @@ struct QkExtras {
 int norm_linear_launch(const char* name, const void* x, int64_t ldx, const void* norm_weight, float eps, const void* w,
                        const void* bias, const void* packed_weights, const void* residual, int64_t ldr, void* out,
                        int64_t ldo, int64_t M, int32_t N, int32_t K, const int32_t* rows, const int32_t* n_rows,
-                       const int32_t* x_rows, const QkExtras& qk, int norm_folded, void* stream, int out_plane = 0) {
+                       const int32_t* x_rows, const QkExtras& qk, int norm_folded, void* stream, int out_plane = 0,
+                       const int32_t* count = nullptr, float* rstd_out = nullptr) {
   if (out_plane != 0 && (residual || (out_plane != 32 && out_plane != 64) || static_cast<int64_t>(8) * M + 8 > 0xffffffffLL ||
                          (qk.enabled && qk.head_dim != out_plane)))
     return set_error(TAAC_ERR_UNSUPPORTED, "%s: output planes are 32 or 64 features wide (the head width under a query / key epilogue), without residual", name);
@@ -1714,6 +1698,8 @@ int norm_linear_launch(const char* name, const void* x, int64_t ldx, const void*
   p.norm_folded = norm_folded ? 1 : 0;
   p.rows = rows;
   p.n_rows = n_rows;
+  if (count != nullptr) p.n_rows = count;
+  p.rstd_out = rstd_out;
   p.x_rows = x_rows;
   p.out_plane_shift = out_plane == 32 ? 5 : (out_plane == 64 ? 6 : 0);
   p.qk_w = static_cast<const bf16_t*>(qk.q_weight);
@@ -1844,6 +1830,22 @@ int attn_out_ffn_readout(const void* attn, int64_t ld_attn, int attn_plane, cons
   return ffn_entry("taac_backbone_fwd", attn, ld_attn, out_bias, packed_out_weights, norm_weight, eps, nullptr, b_up, nullptr,
                    b_down, packed_ffn_weights, residual, ldr, out, ldo, M, D, F, 1, rows, n_rows, nullptr, norm_folded,
                    stream, nullptr, 0, true, attn_plane, head_w, token_dots, split_scratch);
+}
+
+int norm_linear_count(const char* name, const void* x, const void* norm_weight, float eps, const void* bias, const void* packed,
+                      void* out, int64_t M, int32_t N, int32_t K, const int32_t* count, float* rstd_out, hipStream_t s) {
+  return norm_linear_launch(name, x, K, norm_weight, eps, nullptr, bias, packed, nullptr, 0, out, N, M, N, K, nullptr, nullptr,
+                            nullptr, QkExtras{}, norm_weight != nullptr ? TAAC_FOLDED_NORM : 0, s, 0, count, rstd_out);
+}
+
+int attn_out_ffn_count(const char* name, const void* attn, const void* out_bias, const void* packed_out, const void* residual,
+                       const void* norm_weight, float eps, const void* b_up, const void* b_down, const void* packed_ffn,
+                       void* out, void* x1_out, float* rstd_out, int64_t M, int32_t D, int32_t F, bool gate_first, bool act_folded,
+                       const int32_t* count, const void* head_w, float* token_dots, void* split_scratch, hipStream_t s) {
+  return ffn_entry(name, attn, D, out_bias, packed_out, norm_weight, eps, nullptr, b_up, nullptr, b_down, packed_ffn, residual, D,
+                   out, D, M, D, F, gate_first ? 1 : 0, nullptr, nullptr, nullptr,
+                   TAAC_FOLDED_NORM | (act_folded ? TAAC_FOLDED_ACTIVATION : 0), s, nullptr, 0, true, 0, head_w, token_dots,
+                   split_scratch, count, x1_out, rstd_out);
 }
 
 // Whether the gated feed-forward over at most M rows of D features runs as the few-token kernel: as long as its 32-token

@@ -19,16 +19,16 @@
 // eight k-steps of the three blocks: half a step at D = 256, a whole one at D = 128; with two whole-step buffers, one
 // step ahead, the wait for the weights was exposed in every step: 1.54 ms against the time below at 524 288 tokens);
 // results leave through a wavefront-private LDS tile as 16-byte stores that cover 64-byte runs of a row.
+#include "pack.h"
 #include "ts_common.h"
 
 namespace taac {
 namespace {
 
-constexpr int kFrag = 1024;                     // bytes of one 32 x 16 bf16 MFMA operand fragment
 constexpr int kWaves = 8;
 constexpr int kTokPerWg = kWaves * 32;
-constexpr int kUnits = 32;                      // hidden units per step
-constexpr int kSubK = 8;                        // k-steps (of 16 features) per sub-step
+constexpr int kUnits = kBwdUnits;               // hidden units per step
+constexpr int kSubK = kBwdSubK;                 // k-steps (of 16 features) per sub-step
 constexpr int kRing = 4;                        // weight buffers
 constexpr int kTileRow = 3 * kUnits * 2 + 16;   // epilogue tile row: hidden | grad first half | grad second half | pad
 constexpr int kTileWave = 32 * kTileRow;
@@ -42,33 +42,16 @@ struct FfnBwdParams {
   bf16_t* grad_pre;       // [M, 2F] row stride ldgp
   int64_t M, ldh, lddy, ldhid, ldgp;
   int32_t F;
+  const int32_t* count;   // number of tokens on the device (at most M), or null: M
+  const float* rstd;      // [M]: h holds rows x in front of a norm whose weight is part of the packed up projection; the rows
+                          // enter as bf16(x * rstd), as in the forward kernel. Null: h as it is
 };
 
-// Blob: step s (32 hidden units), sub-step u (k-steps 8 u .. 8 u + 7) holds fragments (block b, k-step 8 u + j) at index
-// b * 8 + j; block 0 = rows 32 s .. of the first half of w_up, block 1 = the same rows of its second half, block 2 =
-// columns 32 s .. of w_down (rows of its transpose). Lane (l32, hh) of a fragment holds k = 16 ks + 8 hh .. + 7 of row l32.
 __global__ void ffn_bwd_pack_kernel(const bf16_t* __restrict__ w_up, const bf16_t* __restrict__ w_down,
                                     bf16x8* __restrict__ packed, int D, int F) {
   const int64_t total = static_cast<int64_t>(3) * D * F / 8;
   const int64_t gid = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (gid >= total) return;
-  const int NSUB = D / 16 / kSubK, NFRAG = 3 * kSubK;
-  const int lane = static_cast<int>(gid % 64);
-  const int f = static_cast<int>((gid / 64) % NFRAG);
-  const int64_t sub = gid / 64 / NFRAG;  // step * NSUB + u
-  const int64_t step = sub / NSUB;
-  const int b = f / kSubK, ks = static_cast<int>(sub % NSUB) * kSubK + f % kSubK;
-  const int l32 = lane % 32, hh = lane / 32;
-  const int64_t unit = step * kUnits + l32;
-  const int k0 = ks * 16 + hh * 8;
-  bf16x8 v;
-  if (b < 2) {
-    v = *reinterpret_cast<const bf16x8*>(w_up + (b * static_cast<int64_t>(F) + unit) * D + k0);
-  } else {
-#pragma unroll
-    for (int e = 0; e < 8; ++e) v[e] = w_down[static_cast<int64_t>(k0 + e) * F + unit];
-  }
-  packed[gid] = v;
+  if (gid < total) ffn_bwd_pack_piece(w_up, w_down, packed, D, F, gid);
 }
 
 template <int N>
@@ -98,9 +81,15 @@ __global__ __launch_bounds__(kWaves * kWave, 2) void swiglu_ffn_bwd_hidden_kerne
   const int nsteps = p.F / kUnits;
   const int nsub = nsteps * NSUB;
   const int64_t tok0 = static_cast<int64_t>(blockIdx.x) * kTokPerWg + wave * 32;
+  int64_t M = p.M;
+  if (p.count != nullptr) {
+    const int64_t n = *p.count;
+    M = n < M ? n : M;
+    if (static_cast<int64_t>(blockIdx.x) * kTokPerWg >= M) return;  // whole workgroup
+  }
   // Tokens at or beyond M are mapped to the last token: they compute the same values, so the duplicate stores are
   // benign and every wavefront issues the same number of memory operations (the hand-counted waits rely on that).
-  auto row_of = [&](int64_t tok) -> int64_t { return tok < p.M ? tok : p.M - 1; };
+  auto row_of = [&](int64_t tok) -> int64_t { return tok < M ? tok : M - 1; };
 
   const char* w_bytes = reinterpret_cast<const char*>(p.packed);
   auto stage = [&](int q) {  // sub-step q -> ring slot q % kRing
@@ -131,6 +120,15 @@ __global__ __launch_bounds__(kWaves * kWave, 2) void swiglu_ffn_bwd_hidden_kerne
     // consumed here, so that the compiler's wait for the rows sits in front of the loop and not inside it
 #pragma unroll
     for (int ks = 0; ks < KS; ++ks) asm volatile("" : "+v"(hf[ks]), "+v"(df[ks]));
+    if (p.rstd != nullptr) {
+      const float r = p.rstd[row];
+#pragma unroll
+      for (int ks = 0; ks < KS; ++ks) {
+#pragma unroll
+        for (int e = 0; e < 8; ++e) hf[ks][e] = static_cast<bf16_t>(static_cast<float>(hf[ks][e]) * r);
+        asm volatile("" : "+v"(hf[ks]));
+      }
+    }
   }
   // memory rows of the epilogue stores: piece i = token 16 * i + lane / 4
   int64_t prow[2];
@@ -268,6 +266,28 @@ int launch_bwd_hidden(const FfnBwdParams& p, bool gate_first, hipStream_t s, con
 }  // namespace
 }  // namespace taac
 
+namespace taac {
+int ffn_bwd_hidden_count(const char* name, const void* x, const float* rstd, const void* dy, const void* packed, const void* b_up,
+                         void* hidden, void* grad_pre, int64_t M, int32_t D, int32_t F, bool gate_first, const int32_t* count,
+                         hipStream_t s) {
+  FfnBwdParams p{};
+  p.h = static_cast<const bf16_t*>(x);
+  p.dy = static_cast<const bf16_t*>(dy);
+  p.packed = static_cast<const bf16_t*>(packed);
+  p.b_up = static_cast<const bf16_t*>(b_up);
+  p.hidden = static_cast<bf16_t*>(hidden);
+  p.grad_pre = static_cast<bf16_t*>(grad_pre);
+  p.M = M;
+  p.ldh = p.lddy = D;
+  p.ldhid = F;
+  p.ldgp = 2 * F;
+  p.F = F;
+  p.count = count;
+  p.rstd = rstd;
+  return D == 256 ? launch_bwd_hidden<256>(p, gate_first, s, name) : launch_bwd_hidden<128>(p, gate_first, s, name);
+}
+}  // namespace taac
+
 extern "C" int64_t taac_swiglu_ffn_bwd_packed_bytes(int32_t D, int32_t F) {
   if (!taac::bwd_shape_ok(D, F)) return -1;
   return static_cast<int64_t>(3) * D * F * 2;
@@ -303,7 +323,7 @@ extern "C" int taac_swiglu_ffn_bwd_hidden(const void* h, int64_t ldh, const void
   if (!aligned16(h) || !aligned16(dy) || !aligned16(packed) || !aligned16(hidden) || !aligned16(grad_pre) ||
       (b_up && !aligned16(b_up)))
     return set_error(TAAC_ERR_UNSUPPORTED, "%s: tensor base pointers must be 16-byte aligned", name);
-  FfnBwdParams p;
+  FfnBwdParams p{};
   p.h = static_cast<const bf16_t*>(h);
   p.dy = static_cast<const bf16_t*>(dy);
   p.packed = static_cast<const bf16_t*>(packed);

@@ -108,6 +108,8 @@ __global__ __launch_bounds__(D, 2) void norm_linear_small_kernel(const TsParams 
   }
   float rstd[1] = {1.0f};
   if (p.norm_w != nullptr) token_rstd<D, 1>(p.eps, xf, rstd);  // the norm's weight is part of the packed layer
+  if (p.rstd_out != nullptr && part == 0 && wave == 0 && hh == 0 && tok0 + l32 < count)
+    p.rstd_out[token_row(p, count, tok0 + l32)] = rstd[0];
 
   uint8_t* tile = tiles + wave * kStageWave;
   [[maybe_unused]] const bool qk_part = QK != 0 && chunk < p.qk_chunks;  // the same for all wavefronts of a part
@@ -338,6 +340,7 @@ __global__ __launch_bounds__(4 * kWave, 1) void swiglu_ffn_small_kernel(const Ts
 #pragma unroll
     for (int w = 0; w < NW; ++w) total += sums[w * 32 + l32];
     const float scale = p.norm_w != nullptr ? rsqrtf(total * (1.0f / D) + p.eps) : 1.0f;
+    if (p.rstd_out != nullptr && wave == 0 && hh == 0 && tok0 + l32 < count) p.rstd_out[row] = scale;
 #pragma unroll
     for (int ks = 0; ks < KS; ++ks) {
       xf[0][ks] = *reinterpret_cast<const bf16x8*>(x1_lds + l32 * kRow + (ks * 16 + hh * 8) * 2);
@@ -451,6 +454,14 @@ __global__ __launch_bounds__(4 * kWave, 1) void swiglu_ffn_small_kernel(const Ts
     }
   }
   const bool live = tok0 + l32 < count;
+  if (OUTP && p.x1_out != nullptr) {
+    for (int idx = tid; idx < 32 * (D / 8); idx += NW * kWave) {
+      const int t = idx / (D / 8), c = idx % (D / 8) * 8;
+      if (tok0 + t >= count) continue;
+      const int64_t r = p.rows != nullptr ? static_cast<int64_t>(p.rows[tok0 + t]) : tok0 + t;
+      *reinterpret_cast<bf16x8*>(p.x1_out + r * D + c) = *reinterpret_cast<const bf16x8*>(x1_lds + t * kRow + c * 2);
+    }
+  }
   const float b2_on = p.b2 != nullptr ? 1.f : 0.f;
   float hdot = 0.f;
 #pragma unroll

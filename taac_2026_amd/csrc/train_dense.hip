@@ -1,0 +1,622 @@
+// Dense backward kernels of the training stack (see train_ops.h): the input gradient of a normalised layer with the norm's
+// backward and the residual gradient in its epilogue, and the weight gradients of a block's four layers in one launch.
+#include "train_ops.h"
+#include "ts_common.h"
+
+namespace taac {
+namespace {
+
+// ------------------------------------------------------------------------------------------------------------------
+// dx = dres + rstd * (g - x_hat * mean(g * x_hat)),  g = (dy W) * norm_w,  x_hat = x * rstd.
+//
+// The product is the narrow output of a long contraction (K = 2F or 3D, D features): a workgroup takes 64 * TG tokens x all
+// features, so dy is read once and complete rows meet in the workgroup; 2 * TG wavefronts, TG token groups of 64 x 2 feature
+// halves. K is walked in slabs of 32: both operands' slabs go from global memory straight into LDS (16 rows x 64 bytes per
+// transfer) into a ring of four stages, three slabs ahead; the four 16-byte pieces of a row are XOR-swizzled by (row / 4) % 4, so
+// that the 16 lanes of a fragment read hit distinct banks. Rows beyond the count repeat the last row and are not stored.
+// The epilogue replaces a store of dh = dy W, the norm's backward over x and dh, and the residual add: 3 of the 8 passes over
+// [M, D] that the layer-by-layer backward makes here. The gradient of the norm's weight is left to the weight-gradient kernels,
+// which hold sum_m dy[m, n] x_hat[m, k] anyway (d norm_w[k] = sum_n w[n, k] of it).
+// Bound: HBM (dy, K * 2 bytes per token); 64-token workgroups (TG = 1) where 256-token ones would leave compute units idle.
+// ------------------------------------------------------------------------------------------------------------------
+constexpr int kSlab = 32;
+constexpr int kRing = 4;
+
+struct DgradParams {
+  const bf16_t* dy;
+  const bf16_t* w_t;
+  const bf16_t* x;
+  const float* rstd;
+  const bf16_t* norm_w;
+  const bf16_t* dres;
+  bf16_t* dx;
+  const int32_t* count;
+  int64_t M;
+  int32_t K;
+};
+
+template <int D, int TG>
+__global__ __launch_bounds__(TG * 2 * kWave, 2) void dgrad_norm_kernel(const DgradParams p) {
+  constexpr int NWAVES = 2 * TG;
+  constexpr int TOK = 64 * TG;
+  constexpr int NI = D / 64;                    // 32-feature blocks per wavefront
+  constexpr int kTokBytes = TOK * kSlab * 2, kStage = kTokBytes + D * kSlab * 2;
+  constexpr int WT = D / 16 / NWAVES;           // weight transfers per wavefront and slab
+  constexpr int PW = 2 + WT;                    // all transfers: TOK / 16 = 2 * NWAVES token rows' worth
+  static_assert(D % (16 * NWAVES) == 0, "every wavefront stages the same number of pieces");
+  extern __shared__ __attribute__((aligned(1024))) uint8_t smem[];
+
+  int64_t rows = p.M;
+  {
+    const int64_t n = *p.count;
+    rows = n < rows ? n : rows;
+  }
+  const int64_t m0 = static_cast<int64_t>(blockIdx.x) * TOK;
+  if (m0 >= rows) return;  // whole workgroup
+  const int tid = threadIdx.x;
+  const int wave = __builtin_amdgcn_readfirstlane(tid / kWave);
+  const int lane = tid % kWave;
+  const int l32 = lane % 32, hh = lane / 32;
+  const int wt = wave % TG, wn = wave / TG;
+  const int nslabs = p.K / kSlab;
+
+  const bf16_t* a_src[2];
+  const bf16_t* w_src[WT];
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    const int row = 16 * (2 * wave + i) + lane / 4;
+    const int64_t arow = m0 + row < rows ? m0 + row : rows - 1;
+    a_src[i] = p.dy + arow * p.K + ((lane % 4) ^ ((row >> 2) & 3)) * 8;
+  }
+#pragma unroll
+  for (int i = 0; i < WT; ++i) {
+    const int row = 16 * (WT * wave + i) + lane / 4;
+    w_src[i] = p.w_t + static_cast<int64_t>(row) * p.K + ((lane % 4) ^ ((row >> 2) & 3)) * 8;
+  }
+  // every workgroup starts its walk over K at a different slab: with all of them on the same columns of a matrix whose row pitch
+  // is a power of two their requests crowd the same memory channels
+  const int rot = static_cast<int>((blockIdx.x * 5u) % static_cast<uint32_t>(nslabs));
+  auto stage = [&](int slab) {
+    uint8_t* base = smem + (slab % kRing) * kStage;
+    const int turned = slab + rot;
+    const int k0 = (turned >= nslabs ? turned - nslabs : turned) * kSlab;
+#pragma unroll
+    for (int i = 0; i < 2; ++i) lds_dma16(a_src[i] + k0, base + (2 * wave + i) * 1024);
+#pragma unroll
+    for (int i = 0; i < WT; ++i) lds_dma16(w_src[i] + k0, base + kTokBytes + (WT * wave + i) * 1024);
+  };
+  const int swz = (l32 >> 2) & 3;
+  int piece_off[2];
+#pragma unroll
+  for (int ks = 0; ks < 2; ++ks) piece_off[ks] = ((2 * ks + hh) ^ swz) * 16;
+  const int a_row_off = (wt * 64 + l32) * (kSlab * 2);
+  const int w_row_off = kTokBytes + (wn * (D / 2) + l32) * (kSlab * 2);
+
+  f32x16 acc[NI][2];
+#pragma unroll
+  for (int ni = 0; ni < NI; ++ni)
+#pragma unroll
+    for (int mi = 0; mi < 2; ++mi)
+#pragma unroll
+      for (int j = 0; j < 16; ++j) acc[ni][mi][j] = 0.f;
+
+#pragma unroll
+  for (int q = 0; q < kRing - 1; ++q)
+    if (q < nslabs) stage(q);
+  if (nslabs > 2) vm_wait<2 * PW>();
+  else if (nslabs > 1) vm_wait<PW>();
+  else vm_wait<0>();
+  __syncthreads();
+  for (int s = 0; s < nslabs; ++s) {
+    if (s + kRing - 1 < nslabs) stage(s + kRing - 1);  // the slot last read in slab s - 1, which every wavefront has left
+    const uint8_t* st = smem + (s % kRing) * kStage;
+#pragma unroll
+    for (int ks = 0; ks < kSlab / 16; ++ks) {
+      bf16x8 wf[NI], af[2];
+#pragma unroll
+      for (int mi = 0; mi < 2; ++mi) af[mi] = *reinterpret_cast<const bf16x8*>(st + a_row_off + mi * 32 * (kSlab * 2) + piece_off[ks]);
+#pragma unroll
+      for (int ni = 0; ni < NI; ++ni) wf[ni] = *reinterpret_cast<const bf16x8*>(st + w_row_off + ni * 32 * (kSlab * 2) + piece_off[ks]);
+#pragma unroll
+      for (int ni = 0; ni < NI; ++ni)
+#pragma unroll
+        for (int mi = 0; mi < 2; ++mi) acc[ni][mi] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(wf[ni], af[mi], acc[ni][mi], 0, 0, 0);
+    }
+    if (s + 1 < nslabs) {
+      // the transfers of slab s + 1 were issued three slabs ago; behind them are those of slabs s + 2 and s + 3
+      if (s + 3 < nslabs) vm_wait<2 * PW>();
+      else if (s + 2 < nslabs) vm_wait<PW>();
+      else vm_wait<0>();
+    }
+    __syncthreads();
+  }
+
+  // acc[ni][mi][jq * 4 + e]: feature wn * D / 2 + ni * 32 + jq * 8 + hh * 4 + e of token wt * 64 + mi * 32 + l32
+  float* red = reinterpret_cast<float*>(smem);  // [2 feature halves][TOK] sums of g * x_hat
+  // (the rows of x are read twice, the second time from the caches: held between the passes they do not fit the registers)
+  float scale[2], part[2];
+#pragma unroll
+  for (int mi = 0; mi < 2; ++mi) {
+    const int64_t m = m0 + wt * 64 + mi * 32 + l32;
+    const int64_t row = m < rows ? m : rows - 1;
+    scale[mi] = p.rstd[row];
+    part[mi] = 0.f;
+    const bf16_t* xrow = p.x + row * D + wn * (D / 2) + hh * 4;
+#pragma unroll
+    for (int ni = 0; ni < NI; ++ni) {
+      bf16x4 xv[4], wv[4];
+#pragma unroll
+      for (int jq = 0; jq < 4; ++jq) {
+        xv[jq] = *reinterpret_cast<const bf16x4*>(xrow + ni * 32 + jq * 8);
+        wv[jq] = *reinterpret_cast<const bf16x4*>(p.norm_w + wn * (D / 2) + ni * 32 + jq * 8 + hh * 4);
+      }
+#pragma unroll
+      for (int jq = 0; jq < 4; ++jq)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const float g = acc[ni][mi][jq * 4 + e] * static_cast<float>(wv[jq][e]);
+          acc[ni][mi][jq * 4 + e] = g;
+          part[mi] = fmaf(g, static_cast<float>(xv[jq][e]), part[mi]);  // times rstd: x_hat
+        }
+    }
+  }
+#pragma unroll
+  for (int mi = 0; mi < 2; ++mi) {
+    const uint32_t u = __builtin_bit_cast(uint32_t, part[mi]);
+    const auto r = __builtin_amdgcn_permlane32_swap(u, u, false, false);
+    const float both = __builtin_bit_cast(float, static_cast<uint32_t>(r[0])) + __builtin_bit_cast(float, static_cast<uint32_t>(r[1]));
+    if (hh == 0) red[wn * TOK + wt * 64 + mi * 32 + l32] = both;
+  }
+  __syncthreads();
+#pragma unroll
+  for (int mi = 0; mi < 2; ++mi) {
+    const int64_t m = m0 + wt * 64 + mi * 32 + l32;
+    if (m >= rows) continue;
+    const int t = wt * 64 + mi * 32 + l32;
+    // mean(g * x_hat) * x_hat = (sum of g * x) / D * rstd^2 * x
+    const float proj = (red[t] + red[TOK + t]) * (1.0f / D) * scale[mi] * scale[mi];
+#pragma unroll
+    for (int ni = 0; ni < NI; ++ni) {
+      const int64_t at = m * D + wn * (D / 2) + ni * 32 + hh * 4;
+      bf16x4 xv[4], rv[4];
+#pragma unroll
+      for (int jq = 0; jq < 4; ++jq) {
+        xv[jq] = *reinterpret_cast<const bf16x4*>(p.x + at + jq * 8);
+        rv[jq] = *reinterpret_cast<const bf16x4*>(p.dres + at + jq * 8);
+      }
+#pragma unroll
+      for (int jq = 0; jq < 4; ++jq) {
+        bf16x4 ov;
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+          ov[e] = static_cast<bf16_t>(static_cast<float>(rv[jq][e]) +
+                                      scale[mi] * (acc[ni][mi][jq * 4 + e] - static_cast<float>(xv[jq][e]) * proj));
+        *reinterpret_cast<bf16x4*>(p.dx + at + jq * 8) = ov;
+      }
+    }
+  }
+}
+
+template <int D, int TG>
+int launch_dgrad(const DgradParams& p, hipStream_t s, const char* name) {
+  constexpr size_t lds = static_cast<size_t>(kRing) * (64 * TG + D) * kSlab * 2;
+  if (hipFuncSetAttribute(reinterpret_cast<const void*>(dgrad_norm_kernel<D, TG>), hipFuncAttributeMaxDynamicSharedMemorySize,
+                          static_cast<int>(lds)) != hipSuccess)
+    return set_error(TAAC_ERR_LAUNCH, "%s: cannot reserve %zu bytes of LDS", name, lds);
+  const int64_t grid = (p.M + 64 * TG - 1) / (64 * TG);
+  if (grid > 0x7fffffffLL) return set_error(TAAC_ERR_UNSUPPORTED, "%s: too many workgroups", name);
+  hipLaunchKernelGGL((dgrad_norm_kernel<D, TG>), dim3(static_cast<uint32_t>(grid)), dim3(TG * 2 * kWave), lds, s, p);
+  return check_launch(name);
+}
+
+// ------------------------------------------------------------------------------------------------------------------
+// Weight gradients. Both operands are [tokens, features] row-major and the MFMA needs eight consecutive tokens of one feature
+// per lane from each, so 64-token chunks of both slabs pass through registers into one of two LDS buffers (rows padded by 32
+// bytes: the four rows and pieces a 16-lane group of a transposed read touches fall on distinct banks) while the chunk before is
+// multiplied, and both fragments are read with ds_read_b64_tr_b16. A workgroup owns a TN x TK tile of one layer's gradient over its
+// share of the tokens; all tiles of all layers form one launch of about one workgroup per compute unit (a workgroup fills one with
+// its LDS), so a block's partial sums are one chip's worth of tiles (64 MB at D = 256) instead of one per layer.
+// Bound: HBM - the operands are read once per 256 features of the other side.
+// ------------------------------------------------------------------------------------------------------------------
+constexpr int kChunk = 64;
+
+struct WgradParams {
+  WgradItem item[kWgradItems];
+  int32_t first_tile[kWgradItems + 1];
+  float* partial;          // per item [splits][N][K], items one behind the other
+  float* bias_partial;     // per item [splits][N]
+  int64_t partial_at[kWgradItems], bias_at[kWgradItems];
+  const int32_t* count;
+  int64_t M;
+  int32_t splits, n_items;
+};
+
+template <int TN, int TK, int WN, int WK>
+__global__ __launch_bounds__(WN * WK * kWave, 2) void wgrad_block_kernel(const WgradParams p) {
+  constexpr int THREADS = WN * WK * kWave;
+  constexpr int BN = TN / WN / 32, BK = TK / WK / 32;   // 32 x 32 blocks of a wavefront
+  constexpr int ROWN = TN * 2 + 32, ROWK = TK * 2 + 32;  // LDS row bytes
+  constexpr int SLABN = kChunk * ROWN, SLABK = kChunk * ROWK;
+  constexpr int PN = kChunk * (TN / 8) / THREADS, PK = kChunk * (TK / 8) / THREADS;  // 16-byte pieces per thread and chunk
+  constexpr int RN = THREADS / (TN / 8), RK = THREADS / (TK / 8);                    // rows between a thread's pieces
+  extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
+
+  const int tile = static_cast<int>(blockIdx.x), split = static_cast<int>(blockIdx.y);
+  int which = 0;
+#pragma unroll
+  for (int i = 1; i < kWgradItems; ++i)
+    if (i < p.n_items && tile >= p.first_tile[i]) which = i;
+  const WgradItem& it = p.item[which];
+  const int N = it.N, K = it.K;
+  const int tiles_k = (K + TK - 1) / TK;
+  const int local = tile - p.first_tile[which];
+  const int n0 = (local / tiles_k) * TN, k0 = (local % tiles_k) * TK;
+  int64_t rows = p.M;
+  {
+    const int64_t n = *p.count;
+    rows = n < rows ? n : rows;
+  }
+  const int64_t per = ((rows + p.splits - 1) / p.splits + kChunk - 1) / kChunk * kChunk;
+  const int64_t m_begin = split * per;
+  const int64_t m_end = m_begin + per < rows ? m_begin + per : rows;
+  const int tid = threadIdx.x, wave = tid / kWave, lane = tid % kWave;
+  const int wn = wave / WK, wk = wave % WK;
+  const int g = lane / 16, r = lane % 16;
+  const uint32_t a_lane = static_cast<uint32_t>((8 * (g / 2) + r / 4) * ROWN + (16 * (g % 2) + 4 * (r % 4)) * 2 + wn * (TN / WN) * 2);
+  const uint32_t b_lane = static_cast<uint32_t>(SLABN + (8 * (g / 2) + r / 4) * ROWK + (16 * (g % 2) + 4 * (r % 4)) * 2 + wk * (TK / WK) * 2);
+
+  f32x16 acc[BN][BK];
+#pragma unroll
+  for (int i = 0; i < BN; ++i)
+#pragma unroll
+    for (int j = 0; j < BK; ++j)
+#pragma unroll
+      for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.f;
+
+  // a thread's pieces: always the same eight columns, rows tid / (T / 8) + R * i
+  const int rn = tid / (TN / 8), cn = n0 + tid % (TN / 8) * 8;
+  const int rk = tid / (TK / 8), ck = k0 + tid % (TK / 8) * 8;
+  const bool n_ok = cn < N, k_ok = ck < K;
+  const bf16_t* dy_col = it.dy + (n_ok ? cn : 0);
+  const bf16_t* a_col = it.a + (k_ok ? ck : 0);
+  const float* rscale = it.scale;
+  u32x4 va[PN], vb[PK];
+  float sb[PK];
+  const u32x4 zero = {0u, 0u, 0u, 0u};
+  auto fetch = [&](int64_t m0) {
+#pragma unroll
+    for (int i = 0; i < PN; ++i) {
+      const int64_t m = m0 + rn + RN * i;
+      va[i] = (m < m_end && n_ok) ? *reinterpret_cast<const u32x4*>(dy_col + m * N) : zero;
+    }
+#pragma unroll
+    for (int i = 0; i < PK; ++i) {
+      const int64_t m = m0 + rk + RK * i;
+      const bool ok = m < m_end && k_ok;
+      vb[i] = ok ? *reinterpret_cast<const u32x4*>(a_col + m * K) : zero;
+      sb[i] = (ok && rscale != nullptr) ? rscale[m] : 1.f;
+    }
+  };
+  if (m_begin < m_end) fetch(m_begin);
+  const bool with_bias = it.db != nullptr && k0 == 0;
+  float csum[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+  int buf = 0;
+  for (int64_t m0 = m_begin; m0 < m_end; m0 += kChunk) {
+    // the buffer written now was last read two chunks ago; the barrier of the chunk in between lies behind those reads
+    uint8_t* stage = smem + buf * (SLABN + SLABK);
+    if (with_bias) {
+#pragma unroll
+      for (int i = 0; i < PN; ++i)
+#pragma unroll
+        for (int w = 0; w < 4; ++w) {
+          csum[2 * w] += __uint_as_float(va[i][w] << 16);
+          csum[2 * w + 1] += __uint_as_float(va[i][w] & 0xffff0000u);
+        }
+    }
+#pragma unroll
+    for (int i = 0; i < PN; ++i) *reinterpret_cast<u32x4*>(stage + (rn + RN * i) * ROWN + (cn - n0) * 2) = va[i];
+#pragma unroll
+    for (int i = 0; i < PK; ++i) {
+      if (rscale != nullptr) {
+        bf16x8 v = __builtin_bit_cast(bf16x8, vb[i]);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) v[e] = static_cast<bf16_t>(static_cast<float>(v[e]) * sb[i]);
+        vb[i] = __builtin_bit_cast(u32x4, v);
+      }
+      *reinterpret_cast<u32x4*>(stage + SLABN + (rk + RK * i) * ROWK + (ck - k0) * 2) = vb[i];
+    }
+    if (m0 + kChunk < m_end) fetch(m0 + kChunk);
+    __syncthreads();
+    const uint32_t base = lds_offset(stage);
+    static_for<kChunk / 16>([&](auto ks_tag) {
+      constexpr int ks = decltype(ks_tag)::value;
+      u32x2 fa[BN][2], fb[BK][2];
+      static_for<BN>([&](auto t_tag) {
+        constexpr int t = decltype(t_tag)::value;
+        lds_read_tr16<(ks * 16) * ROWN + t * 64>(fa[t][0], base + a_lane);
+        lds_read_tr16<(ks * 16 + 4) * ROWN + t * 64>(fa[t][1], base + a_lane);
+      });
+      static_for<BK>([&](auto t_tag) {
+        constexpr int t = decltype(t_tag)::value;
+        lds_read_tr16<(ks * 16) * ROWK + t * 64>(fb[t][0], base + b_lane);
+        lds_read_tr16<(ks * 16 + 4) * ROWK + t * 64>(fb[t][1], base + b_lane);
+      });
+      asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(fa[0][0]), "+v"(fa[0][1]) : : "memory");
+#pragma unroll
+      for (int t = 0; t < BN; ++t) asm volatile("" : "+v"(fa[t][0]), "+v"(fa[t][1]));
+#pragma unroll
+      for (int t = 0; t < BK; ++t) asm volatile("" : "+v"(fb[t][0]), "+v"(fb[t][1]));
+#pragma unroll
+      for (int i = 0; i < BN; ++i)
+#pragma unroll
+        for (int j = 0; j < BK; ++j) {
+          const u32x4 abits = {fa[i][0][0], fa[i][0][1], fa[i][1][0], fa[i][1][1]};
+          const u32x4 bbits = {fb[j][0][0], fb[j][0][1], fb[j][1][0], fb[j][1][1]};
+          acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, abits), __builtin_bit_cast(bf16x8, bbits),
+                                                              acc[i][j], 0, 0, 0);
+        }
+    });
+    buf ^= 1;
+  }
+  float* out = p.partial + p.partial_at[which] + static_cast<int64_t>(split) * N * K;
+  const int l32 = lane % 32, hh = lane / 32;
+#pragma unroll
+  for (int i = 0; i < BN; ++i)
+#pragma unroll
+    for (int j = 0; j < BK; ++j) {
+      const int col = k0 + wk * (TK / WK) + j * 32 + l32;
+#pragma unroll
+      for (int e = 0; e < 16; ++e) {
+        const int row = n0 + wn * (TN / WN) + i * 32 + (e / 4) * 8 + hh * 4 + (e % 4);
+        if (row < N && col < K) out[static_cast<int64_t>(row) * K + col] = acc[i][j][e];
+      }
+    }
+  if (with_bias) {
+    __syncthreads();  // every wavefront is done with the chunk buffers
+    float* red = reinterpret_cast<float*>(smem);  // [RN row groups][TN columns]
+#pragma unroll
+    for (int e = 0; e < 8; ++e) red[rn * TN + (cn - n0) + e] = csum[e];
+    __syncthreads();
+    for (int c = tid; c < TN; c += THREADS) {
+      if (n0 + c >= N) continue;
+      float sum = 0.f;
+#pragma unroll
+      for (int rg = 0; rg < RN; ++rg) sum += red[rg * TN + c];
+      p.bias_partial[p.bias_at[which] + static_cast<int64_t>(split) * N + n0 + c] = sum;
+    }
+  }
+}
+
+// dw = sum of the splits, in order, times the norm's weight per column; per workgroup of kReduceRows rows the column sums of
+// w * G (the gradient of the norm's weight) are left in norm_partial [row blocks][K].
+constexpr int kReduceThreads = 256;
+constexpr int kReduceRows = 16;
+struct ReduceParams {
+  WgradItem item[kWgradItems];
+  int32_t first_unit[kWgradItems + 1];   // workgroups: row blocks x column blocks of an item
+  const float* partial;
+  int64_t partial_at[kWgradItems];
+  float* norm_partial;
+  int64_t norm_at[kWgradItems];
+  int32_t splits, n_items;
+};
+template <typename T>
+__global__ __launch_bounds__(kReduceThreads) void wgrad_reduce_kernel(const ReduceParams p) {
+  __shared__ f32x4 red[4][kWave];
+  int which = 0;
+#pragma unroll
+  for (int i = 1; i < kWgradItems; ++i)
+    if (i < p.n_items && static_cast<int>(blockIdx.x) >= p.first_unit[i]) which = i;
+  const WgradItem& it = p.item[which];
+  const int N = it.N, K = it.K;
+  const int col_blocks = (K + 255) / 256;
+  const int local = static_cast<int>(blockIdx.x) - p.first_unit[which];
+  const int row0 = local / col_blocks * kReduceRows;
+  const int col = local % col_blocks * 256 + static_cast<int>(threadIdx.x % kWave) * 4;  // K is a multiple of 8
+  const int rg = threadIdx.x / kWave;
+  const int64_t nk = static_cast<int64_t>(N) * K;
+  const float* src = p.partial + p.partial_at[which];
+  f32x4 nw = {1.f, 1.f, 1.f, 1.f}, nsum = {0.f, 0.f, 0.f, 0.f};
+  const bool ok = col < K;
+  if (ok && it.norm_w != nullptr)
+#pragma unroll
+    for (int e = 0; e < 4; ++e) nw[e] = static_cast<float>(static_cast<const T*>(it.norm_w)[col + e]);
+#pragma unroll
+  for (int i = 0; i < kReduceRows / 4; ++i) {
+    const int row = row0 + rg + 4 * i;
+    if (!ok || row >= N) continue;
+    const int64_t at = static_cast<int64_t>(row) * K + col;
+    f32x4 s = {0.f, 0.f, 0.f, 0.f};
+    for (int k = 0; k < p.splits; ++k) {
+      const f32x4 v = *reinterpret_cast<const f32x4*>(src + k * nk + at);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) s[e] += v[e];
+    }
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      if (it.dnorm != nullptr) nsum[e] = fmaf(s[e], static_cast<float>(static_cast<const T*>(it.w)[at + e]), nsum[e]);
+      static_cast<T*>(it.dw)[at + e] = static_cast<T>(s[e] * nw[e]);
+    }
+  }
+  if (it.dnorm == nullptr) return;  // the same for the whole workgroup
+  red[rg][threadIdx.x % kWave] = nsum;
+  __syncthreads();
+  if (rg == 0 && ok) {
+#pragma unroll
+    for (int w = 1; w < 4; ++w)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) nsum[e] += red[w][threadIdx.x][e];
+    *reinterpret_cast<f32x4*>(p.norm_partial + p.norm_at[which] + static_cast<int64_t>(row0 / kReduceRows) * K + col) = nsum;
+  }
+}
+
+constexpr int kVectorItems = 64;
+struct VectorParams {
+  VectorItem item[kVectorItems];
+  int32_t first_unit[kVectorItems + 1];
+  int32_t n;
+};
+// 16 columns per workgroup, 16 slices of the partial rows: slice sums in row order, added in slice order.
+template <typename T>
+__global__ __launch_bounds__(256) void sum_vectors_kernel(const VectorParams p) {
+  __shared__ float red[16][16];
+  int which = 0;
+  for (int lo = 0, hi = p.n; lo < hi;) {  // last item whose first unit is not above this one
+    const int mid = (lo + hi) / 2;
+    if (p.first_unit[mid] <= static_cast<int>(blockIdx.x)) {
+      which = mid;
+      lo = mid + 1;
+    } else {
+      hi = mid;
+    }
+  }
+  const VectorItem& it = p.item[which];
+  const int c = (static_cast<int>(blockIdx.x) - p.first_unit[which]) * 16 + static_cast<int>(threadIdx.x % 16);
+  const int slice = threadIdx.x / 16;
+  float sum = 0.f;
+  if (c < it.cols)
+    for (int i = slice; i < it.parts; i += 16) sum += it.src[static_cast<int64_t>(i) * it.stride + c];
+  red[slice][threadIdx.x % 16] = sum;
+  __syncthreads();
+  if (slice == 0 && c < it.cols) {
+    float total = 0.f;
+#pragma unroll
+    for (int sl = 0; sl < 16; ++sl) total += red[sl][threadIdx.x];
+    static_cast<T*>(it.dst)[c] = static_cast<T>(total);
+  }
+}
+
+// 256 x 256 tiles where the layers are that wide, 128 x 128 tiles of four wavefronts for the narrow model.
+struct WgradPlan {
+  int tn, tk, tiles, splits;
+};
+WgradPlan plan_of(int64_t M, const int32_t (*shapes)[2], int items) {
+  WgradPlan pl{};
+  int min_side = 1 << 30;
+  for (int i = 0; i < items; ++i) min_side = shapes[i][0] < min_side ? shapes[i][0] : (shapes[i][1] < min_side ? shapes[i][1] : min_side);
+  pl.tn = pl.tk = min_side >= 256 ? 256 : 128;
+  for (int i = 0; i < items; ++i) pl.tiles += ((shapes[i][0] + pl.tn - 1) / pl.tn) * ((shapes[i][1] + pl.tk - 1) / pl.tk);
+  // about one workgroup per compute unit (two of the small ones), but no split of fewer than 1 024 tokens: a split costs a pass
+  // over its partial tile
+  const int cus = compute_units();
+  const int want = (pl.tn == 256 ? 1 : 2) * (cus > 0 ? cus : 1) / pl.tiles;
+  const int64_t most = (M + 1023) / 1024;
+  pl.splits = want < 1 ? 1 : want;
+  if (pl.splits > most) pl.splits = most < 1 ? 1 : static_cast<int>(most);
+  return pl;
+}
+
+}  // namespace
+
+int dgrad_norm(const char* name, const void* dy, int32_t K, const void* w_t, const void* x, const float* rstd, const void* norm_w,
+               const void* dres, void* dx, int64_t M, int32_t D, const int32_t* count, hipStream_t s) {
+  DgradParams p{};
+  p.dy = static_cast<const bf16_t*>(dy);
+  p.w_t = static_cast<const bf16_t*>(w_t);
+  p.x = static_cast<const bf16_t*>(x);
+  p.rstd = rstd;
+  p.norm_w = static_cast<const bf16_t*>(norm_w);
+  p.dres = static_cast<const bf16_t*>(dres);
+  p.dx = static_cast<bf16_t*>(dx);
+  p.count = count;
+  p.M = M;
+  p.K = K;
+  const int cus = compute_units();
+  const bool small = M < 128 * static_cast<int64_t>(cus);
+  if (D == 256) return small ? launch_dgrad<256, 1>(p, s, name) : launch_dgrad<256, 4>(p, s, name);
+  return small ? launch_dgrad<128, 1>(p, s, name) : launch_dgrad<128, 4>(p, s, name);
+}
+
+int64_t wgrad_scratch_floats(int64_t M, const int32_t (*shapes)[2], int items) {
+  const WgradPlan pl = plan_of(M, shapes, items);
+  int64_t n = 0;
+  for (int i = 0; i < items; ++i) n += static_cast<int64_t>(pl.splits) * shapes[i][0] * shapes[i][1];
+  return n;
+}
+
+int64_t wgrad_vector_floats(int64_t M, const int32_t (*shapes)[2], int items) {
+  const WgradPlan pl = plan_of(M, shapes, items);
+  int64_t n = 0;
+  for (int i = 0; i < items; ++i)
+    n += static_cast<int64_t>(pl.splits) * shapes[i][0] + static_cast<int64_t>((shapes[i][0] + kReduceRows - 1) / kReduceRows) * shapes[i][1];
+  return n;
+}
+
+int wgrad_block(const char* name, const WgradItem* items, int n_items, int64_t M, const int32_t* count, float* scratch,
+                float* vectors, int dtype, VectorItem* out_vectors, int* n_vectors, hipStream_t s) {
+  int32_t shapes[kWgradItems][2];
+  for (int i = 0; i < n_items; ++i) {
+    shapes[i][0] = items[i].N;
+    shapes[i][1] = items[i].K;
+  }
+  const WgradPlan pl = plan_of(M, shapes, n_items);
+  WgradParams p{};
+  ReduceParams q{};
+  int tiles = 0, units = 0;
+  int64_t at = 0, vec = 0;
+  for (int i = 0; i < n_items; ++i) {
+    const WgradItem& it = items[i];
+    p.item[i] = q.item[i] = it;
+    p.first_tile[i] = tiles;
+    tiles += ((it.N + pl.tn - 1) / pl.tn) * ((it.K + pl.tk - 1) / pl.tk);
+    p.partial_at[i] = q.partial_at[i] = at;
+    at += static_cast<int64_t>(pl.splits) * it.N * it.K;
+    p.bias_at[i] = vec;
+    if (it.db != nullptr) out_vectors[(*n_vectors)++] = VectorItem{vectors + vec, it.db, pl.splits, it.N, it.N};
+    vec += static_cast<int64_t>(pl.splits) * it.N;
+    const int row_blocks = (it.N + kReduceRows - 1) / kReduceRows;
+    q.first_unit[i] = units;
+    units += row_blocks * ((it.K + 255) / 256);
+    q.norm_at[i] = vec;
+    if (it.dnorm != nullptr) out_vectors[(*n_vectors)++] = VectorItem{vectors + vec, it.dnorm, row_blocks, it.K, it.K};
+    vec += static_cast<int64_t>(row_blocks) * it.K;
+  }
+  p.first_tile[n_items] = tiles;
+  q.first_unit[n_items] = units;
+  p.partial = scratch;
+  p.bias_partial = vectors;
+  p.count = count;
+  p.M = M;
+  p.splits = q.splits = pl.splits;
+  p.n_items = q.n_items = n_items;
+  q.partial = scratch;
+  q.norm_partial = vectors;
+  const dim3 grid(tiles, pl.splits);
+  auto go = [&](auto kernel, int threads, size_t lds) -> int {
+    if (hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds)) !=
+        hipSuccess)
+      return set_error(TAAC_ERR_LAUNCH, "%s: cannot reserve %zu bytes of LDS", name, lds);
+    hipLaunchKernelGGL(kernel, grid, dim3(threads), lds, s, p);
+    return check_launch(name);
+  };
+  const size_t lds = 2 * 2 * static_cast<size_t>(kChunk) * (pl.tn * 2 + 32);
+  const int rc = pl.tn == 256 ? go(wgrad_block_kernel<256, 256, 2, 4>, 512, lds) : go(wgrad_block_kernel<128, 128, 2, 2>, 256, lds);
+  if (rc != TAAC_OK) return rc;
+  if (dtype == TAAC_F32)
+    hipLaunchKernelGGL(wgrad_reduce_kernel<float>, dim3(units), dim3(kReduceThreads), 0, s, q);
+  else
+    hipLaunchKernelGGL(wgrad_reduce_kernel<bf16_t>, dim3(units), dim3(kReduceThreads), 0, s, q);
+  return check_launch(name);
+}
+
+int sum_vectors(const char* name, const VectorItem* items, int n, int dtype, hipStream_t s) {
+  for (int base = 0; base < n; base += kVectorItems) {
+    VectorParams p{};
+    p.n = n - base < kVectorItems ? n - base : kVectorItems;
+    int units = 0;
+    for (int i = 0; i < p.n; ++i) {
+      p.item[i] = items[base + i];
+      p.first_unit[i] = units;
+      units += (items[base + i].cols + 15) / 16;
+    }
+    if (dtype == TAAC_F32)
+      hipLaunchKernelGGL(sum_vectors_kernel<float>, dim3(units), dim3(256), 0, s, p);
+    else
+      hipLaunchKernelGGL(sum_vectors_kernel<bf16_t>, dim3(units), dim3(256), 0, s, p);
+    const int rc = check_launch(name);
+    if (rc != TAAC_OK) return rc;
+  }
+  return TAAC_OK;
+}
+
+}  // namespace taac

@@ -33,7 +33,8 @@ struct TsParams {
   int32_t gate_first;
   int32_t packed;           // weights are in fragment order
   const int32_t* rows;      // optional row index: token i lives in row rows[i] of x / residual / out
-  const int32_t* n_rows;    // with rows: device pointer to the number of tokens (at most M)
+  const int32_t* n_rows;    // device pointer to the number of tokens (at most M), or null: M. Without rows the tokens are the
+                            // first *n_rows rows (a compact tensor whose length the host does not know)
   const int32_t* x_rows;    // optional, with rows: token i's row of x when it differs from rows[i] (x and residual / out
                             // laid out differently: samples with their valid tokens moved to the front on one side)
   int32_t units;            // FFN: compute units the last, partial round of workgroups is spread over
@@ -66,6 +67,8 @@ struct TsParams {
   // Few-token feed-forward with the hidden units of a 32-token tile divided over `splits` workgroups (0: one): every workgroup
   // leaves its fp32 partial in split_partials [tile][splits][32 x D] and counts itself in split_counters [tile] (zero before
   // the launch); the last one to arrive adds the partials up in order, finishes the tile and sets the counter back to zero.
+  float* rstd_out;          // [M]: the per-token factor of the norm in front (of the up projection; of the linear layer), or null
+  bf16_t* x1_out;           // OUTP: the tokens between the two halves of the block, [M, D] rows like out; or null
   int32_t splits;
   float* split_partials;
   uint32_t* split_counters;
@@ -94,9 +97,9 @@ constexpr float kFoldGate = -1.4426950408889634f, kFoldValue = -0.69314718055994
 
 // ---- shared pieces ---------------------------------------------------------------------------------------------------
 
-// Number of tokens to process: M, or *n_rows (clamped to M) when a row index is given.
+// Number of tokens to process: M, or *n_rows (clamped to M) when a count is given.
 __device__ __forceinline__ int64_t token_count(const TsParams& p) {
-  if (p.rows == nullptr) return p.M;
+  if (p.n_rows == nullptr) return p.M;
   const int64_t n = *p.n_rows;
   return n < p.M ? n : p.M;
 }

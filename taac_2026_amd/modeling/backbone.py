@@ -24,7 +24,8 @@ from taac_2026_amd.accelerators.attention import StructuredAttentionMask, front_
 from taac_2026_amd.accelerators.linear import (attention_out_ffn, front_rows, norm_linear, qkv_projection, silu_mlp,
                                                swiglu_ffn, swiglu_ffn_backward_supported, swiglu_ffn_dropout, valid_rows)
 from taac_2026_amd.accelerators.tensor_validation import require_cuda_tensors, require_inference
-from taac_2026_amd.modeling.block_training import run_training_block, training_route_applies
+from taac_2026_amd.modeling.block_training import (InteractionStackFunction, run_training_block, run_training_stack,
+                                                   training_route_applies, uniform_parameters)
 from taac_2026_amd.modeling.normalization import RMSNorm
 from taac_2026_amd.modeling.sequence import scaled_dot_product_attention
 
@@ -449,8 +450,16 @@ def run_interaction_blocks(blocks, tokens: torch.Tensor, padding_mask: torch.Ten
     ``final_norm``, which the readout head applies): every block receives the same padding mask and attention mask and
     only its output stream is kept. The stream is copied once and the blocks then update it in place; with a mask from
     ``MetadataAttentionMask`` the row indices and the mask gathered per sample are built by the first block and shared
-    by the others. The padding mask must not be modified while the loop runs."""
+    by the others. The padding mask must not be modified while the loop runs. With tensors that take a gradient the blocks
+    run as one function where ``UnifiedInteractionBlock`` would take its training route."""
     stream = tokens
+    if (len(blocks) > 0 and torch.is_grad_enabled() and isinstance(attention_mask, StructuredAttentionMask)
+            and attention_mask.query_self is None
+            and all(type(block).forward is UnifiedInteractionBlock.forward and not block._fused_route(tokens)
+                    and training_route_applies(block, tokens, attention_mask, None, padding_mask) for block in blocks)):
+        output = run_training_stack(blocks, tokens, attention_mask, padding_mask)
+        if output is not None:
+            return output
     for position, block in enumerate(blocks):
         stream, _ = block(stream, padding_mask, attention_mask, return_attention_tokens=False, inplace=position > 0)
     return stream
@@ -586,13 +595,14 @@ class PCVRBackbone(nn.Module):
             return probabilities, hidden
         return probabilities
 
-    def _forward_training(self, emb: torch.Tensor, key_lengths: torch.Tensor, return_hidden: bool):
-        """The same network under autograd: every block as one function over the valid rows
-        (:class:`InteractionBlockFunction`), then the masked mean over the valid tokens, the head and the sigmoid as
-        differentiable tensor operations (``masked_mean``, modeling/sequence.py:54-60). One host synchronisation per
-        ``key_lengths`` tensor (the number of valid rows sizes the backward's tensors)."""
-        from taac_2026_amd.modeling.block_training import InteractionBlockFunction
+    # parameters of a block in the order of taac_block_weights
+    _TRAINED = (("attn_norm", "weight"), ("qkv", "weight"), ("qkv", "bias"), ("out", "weight"), ("out", "bias"),
+                ("ffn_norm", "weight"), ("up", "weight"), ("up", "bias"), ("down", "weight"), ("down", "bias"),
+                ("query_norm", "weight"), ("key_norm", "weight"))
 
+    def _forward_training(self, emb: torch.Tensor, key_lengths: torch.Tensor, return_hidden: bool):
+        """The same network under autograd: blocks and readout as one function over the valid tokens
+        (:class:`InteractionStackFunction`), without a host synchronisation."""
         name = "hip PCVRBackbone"
         if emb.ndim != 3 or emb.shape[-1] != self.d_model or emb.dtype != torch.bfloat16:
             raise ValueError(f"{name} expects bfloat16 embeddings of shape (batch, tokens, {self.d_model})")
@@ -607,23 +617,22 @@ class PCVRBackbone(nn.Module):
                                "(taac_swiglu_ffn_bwd_packed_bytes) and no rotary embedding")
         if key_lengths.dtype != torch.int32 or not key_lengths.is_contiguous():
             key_lengths = key_lengths.to(torch.int32).contiguous()
-        stream = emb
+        if emb.numel() == 0 or len(self.blocks) == 0:  # nothing in front of the readout
+            valid = (torch.arange(emb.shape[1], device=emb.device)[None, :] < key_lengths[:, None]).to(emb.dtype).unsqueeze(-1)
+            pooled = (emb * valid).sum(dim=1) / valid.sum(dim=1).clamp_min(1.0)
+            logits = torch.nn.functional.linear(pooled, _bf16(self.head.weight), _bf16(self.head.bias)).squeeze(-1)
+            return (torch.sigmoid(logits.float()), emb * valid) if return_hidden else torch.sigmoid(logits.float())
+        params: list[torch.Tensor | None] = []
         for block in self.blocks:
-            qk = block.query_norm is not None
-            stream, _ = InteractionBlockFunction.apply(
-                stream, key_lengths, None, None, False, self.num_heads, self.eps, self.eps, True, self.eps,
-                _bf16(block.attn_norm.weight), _bf16(block.qkv.weight), _bf16(block.qkv.bias), _bf16(block.out.weight),
-                _bf16(block.out.bias), _bf16(block.ffn_norm.weight), _bf16(block.up.weight), _bf16(block.up.bias),
-                _bf16(block.down.weight), _bf16(block.down.bias), _bf16(block.query_norm.weight) if qk else None,
-                _bf16(block.key_norm.weight) if qk else None)
-        tokens = emb.shape[1]
-        valid = (torch.arange(tokens, device=emb.device)[None, :] < key_lengths[:, None]).to(stream.dtype).unsqueeze(-1)
-        pooled = (stream * valid).sum(dim=1) / valid.sum(dim=1).clamp_min(1.0)
-        logits = torch.nn.functional.linear(pooled, _bf16(self.head.weight), _bf16(self.head.bias)).squeeze(-1)
-        probabilities = torch.sigmoid(logits.float())
-        if return_hidden:
-            return probabilities, stream * valid      # rows at or beyond key_lengths[b] are zeros, as in the forward-only route
-        return probabilities
+            parts = block._modules                    # (the registries directly, as in forward)
+            for part, parameter in self._TRAINED:
+                module = parts.get(part)
+                params.append(None if module is None else module._parameters[parameter])
+        params += [self.head.weight, self.head.bias]
+        hidden, _, probabilities = InteractionStackFunction.apply(
+            emb, key_lengths, None,
+            (self.num_heads, self.eps, self.eps, self.eps, True, bool(return_hidden), True, False, True), *uniform_parameters(params))
+        return (probabilities, hidden) if return_hidden else probabilities
 
     FP8_MAXIMA = ("qkv.weight", "out.weight", "up.weight", "down.weight", "attn_norm", "attention", "ffn_norm", "hidden")
 

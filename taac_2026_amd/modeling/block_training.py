@@ -1,25 +1,24 @@
-"""Training route of ``UnifiedInteractionBlock`` (experiments/symbiosis/backbone.py:51-68) under prefix padding (key
-lengths) or under a structured mask built from the padding mask (scattered padding, e.g. the role mask of
-experiments/symbiosis/attention.py:21-60): one autograd function for the whole block whose forward and backward run over
-the VALID tokens only.
+"""Training route of ``UnifiedInteractionBlock`` (experiments/symbiosis/backbone.py:51-68), of a stack of them and of
+``PCVRBackbone``, under prefix padding (key lengths) or under a structured mask built from the padding mask (scattered
+padding, e.g. the role mask of experiments/symbiosis/attention.py:21-60): one autograd function for the whole stack whose
+forward and backward run over the VALID tokens only.
 
 The reference multiplies both residual updates by ``~padding_mask``, so a padded position passes its input through and
-contributes nothing to any weight gradient. The function therefore gathers the valid rows of the token stream once
-into a compact ``[valid, D]`` tensor and runs every dense layer, norm and weight gradient on compact tensors; only the
-attention kernels see the padded ``[B, T, .]`` layout, which the projections on either side of them write and read
-through the row index of :func:`valid_rows` (no copy). At the benchmark's lengths (54 % of the positions valid) the dense
-forward and backward kernels do 54 % of the work of the layer-by-layer route, the packed q | k | v gradient is written
-in place (no concatenation) and the mask multiplications and residual adds of autograd disappear.
+contributes nothing to any weight gradient. ``InteractionStackFunction`` therefore gathers the valid rows of the token
+stream once into a compact tensor, runs every kernel of every block on compact tensors (the attention kernels address a
+sample by its row offset) and scatters the result once. Forward and backward are one library call each
+(``taac_stack_train_fwd`` / ``taac_stack_train_bwd``), which sequence the kernels natively: the number of valid rows stays
+on the device (no host synchronisation), parameters are taken as they are (bf16, or float32 masters, which the set-up
+kernel rounds as it packs them) and their gradients are written in the same dtype.
 
-The number of valid rows sizes the compact tensors, so it is read back from the device once per ``key_lengths`` tensor
-or mask object (one host synchronisation, shared by the blocks of a stack).
+``InteractionBlockFunction`` keeps the positions' layout for the one case that the compact layout does not cover: a mask
+with self-only queries.
 """
 
 from __future__ import annotations
 
 import ctypes
 import importlib
-import weakref
 
 import torch
 
@@ -31,17 +30,23 @@ from taac_2026_amd.accelerators.normalization import hip_rms_norm_backward_kerne
 
 
 class _RowIndex:
-    """Valid-row index of a ``key_lengths`` tensor: ``rows`` (int32, :func:`valid_rows`) and ``count`` (device scalar) at
-    once; ``compact()`` adds what the backward needs and what costs the host synchronisation: ``valid`` (the count on the
-    host) and ``identity`` (int32 ``0..valid-1``: the row numbers of a compact tensor). The index of the last tensor seen
-    is kept, so the blocks of a stack share it."""
+    """Valid-row index of a padding mask (any pattern): ``rows`` (int32, :func:`valid_rows`), ``count`` (device scalar) and
+    ``bits`` (the validity as packed words), and, when the mask has no self-only queries, ``lengths`` (valid tokens per sample)
+    and ``front_mask`` (the mask's structure gathered per sample over its valid tokens). ``compact()`` adds ``valid``
+    (the count on the host: one synchronisation) and ``identity`` (int32 ``0..valid-1``)."""
 
-    _last: tuple | None = None
+    def __init__(self, mask, padding_mask: torch.Tensor, tokens: int) -> None:
+        from taac_2026_amd.accelerators.attention import _pack_bits, front_structured_mask
 
-    def __init__(self, key_lengths: torch.Tensor, tokens: int) -> None:
-        self.rows, self.count = _linear.valid_rows(key_lengths, tokens)
+        self.rows, self.count = _linear.valid_rows(None, tokens, padding_mask=padding_mask)
+        self.bits = _pack_bits((~padding_mask).contiguous())
         self.valid: int | None = None
         self.identity = None
+        self.lengths = self.front_mask = None
+        if mask.query_self is None:
+            batch = padding_mask.shape[0]
+            self.lengths = _linear.front_rows((self.rows, self.count), batch, tokens)[1]
+            self.front_mask = front_structured_mask(mask, (self.rows, self.count), batch)
 
     def compact(self) -> "_RowIndex":
         if self.valid is None:
@@ -51,43 +56,11 @@ class _RowIndex:
 
     @classmethod
     def for_mask(cls, mask, padding_mask: torch.Tensor, tokens: int) -> "_RowIndex":
-        """Index of the positions ``~padding_mask`` (any pattern), kept on the mask object the blocks of a stack share;
-        ``bits``: the same validity as packed words, for ``taac_rows_merge_bits``."""
+        """The index of ``~padding_mask``, kept on the mask object the blocks of a stack share."""
         entry = mask.cache.get("training_rows")
         if entry is None or entry[0] != padding_mask._version:
-            from taac_2026_amd.accelerators.attention import _pack_bits
-
-            from taac_2026_amd.accelerators.attention import front_structured_mask
-
-            index = cls.__new__(cls)
-            index.rows, index.count = _linear.valid_rows(None, tokens, padding_mask=padding_mask)
-            index.bits = _pack_bits((~padding_mask).contiguous())
-            # valid tokens in the 32-token words before each word: the rank of a position without a walk over the words
-            words = index.bits.shape[1]
-            per_word = torch.nn.functional.pad(~padding_mask, (0, words * 32 - tokens)).view(-1, words, 32).sum(-1)
-            index.word_prefix = (per_word.cumsum(1) - per_word).to(torch.int32).contiguous()
-            index.valid = None
-            index.identity = None
-            # Without self-only queries the attention side runs in the layout that has every sample's valid tokens at the
-            # front of its rows (prefix padding: its cost follows the valid tokens), under the structure gathered per sample.
-            index.front = index.lengths = index.front_mask = None
-            if mask.query_self is None:
-                batch = padding_mask.shape[0]
-                index.front, index.lengths = _linear.front_rows((index.rows, index.count), batch, tokens)
-                index.front_mask = front_structured_mask(mask, (index.rows, index.count), batch)
-            entry = mask.cache["training_rows"] = (padding_mask._version, index)
+            entry = mask.cache["training_rows"] = (padding_mask._version, cls(mask, padding_mask, tokens))
         return entry[1]
-
-    @classmethod
-    def get(cls, key_lengths: torch.Tensor, tokens: int) -> "_RowIndex":
-        stamp = cls._last
-        if stamp is not None:
-            ref, version, pointer, width, entry = stamp
-            if ref() is key_lengths and version == key_lengths._version and pointer == key_lengths.data_ptr() and width == tokens:
-                return entry
-        entry = cls(key_lengths, tokens)
-        cls._last = (weakref.ref(key_lengths), key_lengths._version, key_lengths.data_ptr(), tokens, entry)
-        return entry
 
 
 def _indexed_linear(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | None, out: torch.Tensor, *, tokens: int,
@@ -107,12 +80,10 @@ def _indexed_linear(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | 
     _native.check(status, "interaction block (training): projection")
 
 
-def _gather_rows(src: torch.Tensor, index: "_RowIndex", rows: torch.Tensor | None = None) -> torch.Tensor:
-    """The valid rows of a padded ``[B * T, W]`` tensor as a compact ``[valid, W]`` one (``taac_rows_gather``); ``rows``:
-    where the valid tokens lie when that is not their position (the front layout of the attention side)."""
+def _gather_rows(src: torch.Tensor, index: "_RowIndex") -> torch.Tensor:
+    """The valid rows of a padded ``[B * T, W]`` tensor as a compact ``[valid, W]`` one (``taac_rows_gather``)."""
     out = torch.empty(index.valid, src.shape[1], dtype=src.dtype, device=src.device)
-    rows = index.rows if rows is None else rows
-    status = _native.load_library().taac_rows_gather(src.data_ptr(), src.stride(0), rows.data_ptr(), index.valid,
+    status = _native.load_library().taac_rows_gather(src.data_ptr(), src.stride(0), index.rows.data_ptr(), index.valid,
                                                      out.data_ptr(), src.shape[1], _native.current_stream(src.device))
     _native.check(status, "interaction block (training): gather")
     return out
@@ -125,36 +96,28 @@ def _attention_strides(width: int, heads: int, row_stride: int, tokens: int):
 
 class InteractionBlockFunction(torch.autograd.Function):
     """``UnifiedInteractionBlock.forward`` (with or without the query / key norms) without rotary embedding or dropout,
-    under key lengths (``mask`` None) or under a structured mask whose key validity comes from ``padding_mask`` (``key_lengths``
-    None). Inputs: tokens ``[B, T, D]`` bf16, ``key_lengths`` int32 ``[B]`` or None, the mask and its padding mask or None,
-    then the block's parameters. Returns ``(output, attn_tokens)`` like the module (``attn_tokens`` is None unless asked for)."""
+    under a structured mask with self-only queries whose key validity comes from ``padding_mask``: the dense layers over the
+    valid rows, the attention side in the layout of the positions. Inputs: tokens ``[B, T, D]`` bf16, the mask and its padding
+    mask, then the block's parameters. Returns ``(output, attn_tokens)`` like the module (``attn_tokens`` is None unless
+    asked for)."""
 
     @staticmethod
-    def forward(ctx, tokens, key_lengths, mask, padding_mask, want_attn_tokens, num_heads, attn_eps, ffn_eps, gate_first,
+    def forward(ctx, tokens, mask, padding_mask, want_attn_tokens, num_heads, attn_eps, ffn_eps, gate_first,
                 qk_eps, attn_norm_w, w_qkv, b_qkv, w_out, b_out, ffn_norm_w, w_up, b_up, w_down, b_down, query_norm_w,
                 key_norm_w):
         batch, token_count, width = tokens.shape
         total = batch * token_count
-        index = _RowIndex.get(key_lengths, token_count) if mask is None else _RowIndex.for_mask(mask, padding_mask, token_count)
+        index = _RowIndex.for_mask(mask, padding_mask, token_count)
         rows, count = index.rows, index.count
         flat = tokens.detach().reshape(total, width)
         if not flat.is_contiguous():
             flat = flat.contiguous()
         library = _native.load_library()
-        # Layout of the attention side (q | k | v, the attention output and their gradients): the positions (key lengths,
-        # or a mask with self-only queries), or the samples' valid tokens in front (any other mask), where the mask's
-        # structure is the one gathered per sample and the samples' numbers of valid tokens are the key lengths.
-        front = getattr(index, "front", None) if mask is not None else None
-        arows = rows if front is None else front
-        if front is not None:
-            mask, key_lengths = index.front_mask, index.lengths
-        # q | k | v of the valid rows. Under key lengths the attention kernels never read a row beyond a sample's length;
-        # under a mask over the positions they do (an invisible pair is a zero factor, not a skipped one), so the padded
-        # rows hold zeros there.
-        in_positions = mask is not None and front is None
-        qkv = (torch.zeros if in_positions else torch.empty)(total, 3 * width, dtype=flat.dtype, device=flat.device)
-        _indexed_linear(flat, w_qkv, b_qkv, qkv, tokens=total, out_rows=arows, count=count,
-                        x_rows=None if front is None else rows, norm_weight=attn_norm_w, eps=attn_eps)
+        # q | k | v of the valid rows. The attention kernels read the padded rows too (an invisible pair is a zero factor,
+        # not a skipped one), so those hold zeros.
+        qkv = torch.zeros(total, 3 * width, dtype=flat.dtype, device=flat.device)
+        _indexed_linear(flat, w_qkv, b_qkv, qkv, tokens=total, out_rows=rows, count=count, x_rows=None,
+                        norm_weight=attn_norm_w, eps=attn_eps)
         element = qkv.element_size()
         if query_norm_w is not None:
             # RMSNorm(d_model) of the query and of the key, in place on the valid rows of the packed projection; the
@@ -162,34 +125,26 @@ class InteractionBlockFunction(torch.autograd.Function):
             status = library.taac_qk_norm_rope_fwd(
                 qkv.data_ptr(), qkv.data_ptr() + width * element, 3 * width, qkv.data_ptr(), qkv.data_ptr() + width * element,
                 3 * width, total, token_count, width, int(num_heads), query_norm_w.data_ptr(), key_norm_w.data_ptr(),
-                float(qk_eps), None, arows.data_ptr(), count.data_ptr(), _native.dtype_code(flat.dtype),
+                float(qk_eps), None, rows.data_ptr(), count.data_ptr(), _native.dtype_code(flat.dtype),
                 _native.current_stream(tokens.device))
             _native.check(status, "interaction block (training): query / key norm")
         attended = torch.empty(total, width, dtype=flat.dtype, device=flat.device)
         lse = torch.empty(batch, num_heads, token_count, dtype=torch.float32, device=flat.device)
         qkv_strides = _attention_strides(width, num_heads, 3 * width, token_count)
         out_strides = _attention_strides(width, num_heads, width, token_count)
-        if mask is None:
-            status = library.taac_flash_attn_train_fwd(
-                qkv.data_ptr(), qkv.data_ptr() + width * element, qkv.data_ptr() + 2 * width * element, key_lengths.data_ptr(),
-                attended.data_ptr(), lse.data_ptr(), batch, num_heads, token_count, token_count, width // num_heads,
-                qkv_strides, qkv_strides, qkv_strides, out_strides, 0, 1, _native.dtype_code(flat.dtype),
-                _native.current_stream(tokens.device))
-        else:
-            status = library.taac_flash_attn_masked_train_fwd(
-                qkv.data_ptr(), qkv.data_ptr() + width * element, qkv.data_ptr() + 2 * width * element,
-                _native.ptr(key_lengths), mask.struct_bits.data_ptr(), int(mask.sample_stride), _native.ptr(mask.block_any),
-                _native.ptr(mask.valid_bits), _native.ptr(mask.self_bits), None, ctypes.c_float(1.0), attended.data_ptr(),
-                lse.data_ptr(), batch, num_heads, token_count, token_count, width // num_heads, qkv_strides, qkv_strides,
-                qkv_strides, out_strides, 0 if front is None else 1, _native.dtype_code(flat.dtype),
-                _native.current_stream(tokens.device))
+        status = library.taac_flash_attn_masked_train_fwd(
+            qkv.data_ptr(), qkv.data_ptr() + width * element, qkv.data_ptr() + 2 * width * element, None,
+            mask.struct_bits.data_ptr(), int(mask.sample_stride), _native.ptr(mask.block_any), _native.ptr(mask.valid_bits),
+            _native.ptr(mask.self_bits), None, ctypes.c_float(1.0), attended.data_ptr(), lse.data_ptr(), batch, num_heads,
+            token_count, token_count, width // num_heads, qkv_strides, qkv_strides, qkv_strides, out_strides, 0,
+            _native.dtype_code(flat.dtype), _native.current_stream(tokens.device))
         _native.check(status, "interaction block (training): attention")
         # Second half on the valid rows of copies of the stream (padded rows pass through): one kernel when the caller
         # does not want the tokens between the halves, two otherwise.
         attn_tokens = None
         if want_attn_tokens or not gate_first:
             attn_tokens = flat.clone()
-            _indexed_linear(attended, w_out, b_out, attn_tokens, tokens=total, out_rows=rows, count=count, x_rows=front,
+            _indexed_linear(attended, w_out, b_out, attn_tokens, tokens=total, out_rows=rows, count=count, x_rows=None,
                             residual=flat)
             output = attn_tokens.clone()
             _linear.swiglu_ffn(attn_tokens, w_up, b_up, w_down, b_down, residual=attn_tokens, gate_first=gate_first,
@@ -197,11 +152,9 @@ class InteractionBlockFunction(torch.autograd.Function):
         else:
             output = flat.clone()
             _linear.attention_out_ffn(attended, w_out, b_out, flat, w_up, b_up, w_down, b_down, norm_weight=ffn_norm_w,
-                                      eps=ffn_eps, token_rows=(rows, count), input_rows=front, out=output)
-        ctx.mask, ctx.front = mask, front
-        # (a mask over the positions has no key lengths: the slot keeps a tensor it never reads)
-        ctx.save_for_backward(flat, qkv, attended, lse, key_lengths if key_lengths is not None else lse, attn_norm_w, w_qkv,
-                              w_out, ffn_norm_w, w_up, w_down,
+                                      eps=ffn_eps, token_rows=(rows, count), out=output)
+        ctx.mask = mask
+        ctx.save_for_backward(flat, qkv, attended, lse, attn_norm_w, w_qkv, w_out, ffn_norm_w, w_up, w_down,
                               *(t for t in (b_out, b_up, attn_tokens, b_qkv if query_norm_w is not None else None,
                                             query_norm_w, key_norm_w) if t is not None))
         ctx.index = index
@@ -215,7 +168,7 @@ class InteractionBlockFunction(torch.autograd.Function):
 
     @staticmethod
     def backward(ctx, grad_output, grad_attn_tokens):
-        (flat, qkv, attended, lse, key_lengths, attn_norm_w, w_qkv, w_out, ffn_norm_w, w_up, w_down, *rest) = ctx.saved_tensors
+        (flat, qkv, attended, lse, attn_norm_w, w_qkv, w_out, ffn_norm_w, w_up, w_down, *rest) = ctx.saved_tensors
         (batch, token_count, width, num_heads, attn_eps, ffn_eps, gate_first, has_b_qkv, has_b_out, has_b_up, has_b_down,
          has_attn_tokens, has_qk_norm, qk_eps) = ctx.config
         rest = list(rest)
@@ -226,13 +179,12 @@ class InteractionBlockFunction(torch.autograd.Function):
         query_norm_w, key_norm_w = (rest.pop(0), rest.pop(0)) if has_qk_norm else (None, None)
         index = ctx.index.compact()
         rows, count, valid, identity = index.rows, index.count, index.valid, index.identity
-        mask, front = ctx.mask, ctx.front
-        arows = rows if front is None else front       # where the attention side keeps the valid tokens
+        mask = ctx.mask
         total = batch * token_count
         dtype, device = flat.dtype, flat.device
         if valid == 0:                              # no valid token: the block is the identity
             grads = [g for g in (grad_output, grad_attn_tokens) if g is not None]
-            return (sum(grads[1:], grads[0]) if grads else None,) + (None,) * 21
+            return (sum(grads[1:], grads[0]) if grads else None,) + (None,) * 20
         # the compact rows of the stream and of the tokens between the halves (gathered, or recomputed from the attention
         # output when the forward ran the one-kernel second half)
         xc = _gather_rows(flat, index)
@@ -240,7 +192,7 @@ class InteractionBlockFunction(torch.autograd.Function):
             x1c = _gather_rows(attn_tokens_saved, index)
         else:
             x1c = torch.empty(valid, width, dtype=dtype, device=device)
-            _indexed_linear(attended, w_out, b_out, x1c, tokens=valid, out_rows=identity, count=count, x_rows=arows, residual=xc)
+            _indexed_linear(attended, w_out, b_out, x1c, tokens=valid, out_rows=identity, count=count, x_rows=rows, residual=xc)
 
         def flat_grad(g):
             g = g.reshape(total, width)
@@ -267,43 +219,27 @@ class InteractionBlockFunction(torch.autograd.Function):
             grad_x1_norm, weight_grads["ffn_norm"] = hip_rms_norm_backward_kernel(x1c, ffn_norm_w, grad_h2, ffn_eps)
             grad_x1c = gc.add_(grad_x1_norm) if grad_x1c is None else grad_x1c.add_(gc).add_(grad_x1_norm)
         if grad_x1c is None:
-            return (None,) * 22
+            return (None,) * 21
         # ---- out projection: weight gradient on compact rows, input gradient written into the padded layout ------------
-        attended_c = _gather_rows(attended, index, arows)
+        attended_c = _gather_rows(attended, index)
         grad_w_out, grad_b_out = _linear.linear_wgrad(grad_x1c, attended_c, with_bias=has_b_out)
         del attended_c
         grad_attended = torch.zeros(total, width, dtype=dtype, device=device)
-        _indexed_linear(grad_x1c, w_out.t().contiguous(), None, grad_attended, tokens=valid, out_rows=arows, count=count,
+        _indexed_linear(grad_x1c, w_out.t().contiguous(), None, grad_attended, tokens=valid, out_rows=rows, count=count,
                         x_rows=identity, cache_weight=False)
         # ---- attention: the gradient of the packed q | k | v projection in place ---------------------------------------------
         grad_qkv = torch.empty(total, 3 * width, dtype=dtype, device=device)
         delta = torch.empty_like(lse)
-        library = _native.load_library()
-        qkv_strides = _attention_strides(width, num_heads, 3 * width, token_count)
-        out_strides = _attention_strides(width, num_heads, width, token_count)
-        element = qkv.element_size()
-        q_ptr, g_ptr = qkv.data_ptr(), grad_qkv.data_ptr()
-        if mask is None:
-            status = library.taac_flash_attn_bwd(
-                q_ptr, q_ptr + width * element, q_ptr + 2 * width * element, attended.data_ptr(), grad_attended.data_ptr(),
-                lse.data_ptr(), key_lengths.data_ptr(), g_ptr, g_ptr + width * element, g_ptr + 2 * width * element,
-                delta.data_ptr(), batch, num_heads, token_count, token_count, width // num_heads, qkv_strides, qkv_strides,
-                qkv_strides, out_strides, out_strides, qkv_strides, qkv_strides, qkv_strides, 0, 1, _native.dtype_code(dtype),
-                _native.current_stream(device))
-            _native.check(status, "interaction block (training): attention backward")
-        else:
-            from taac_2026_amd.accelerators.attention import masked_attention_backward
+        from taac_2026_amd.accelerators.attention import masked_attention_backward
 
-            head_dim = width // num_heads
-            heads_of = lambda t, parts: t.view(batch, token_count, parts, num_heads, head_dim).permute(2, 0, 3, 1, 4)  # noqa: E731
-            q4, k4, v4 = heads_of(qkv, 3)
-            dq4, dk4, dv4 = heads_of(grad_qkv, 3)
-            (o4,), (do4,) = heads_of(attended, 1), heads_of(grad_attended, 1)
-            # positions: the padded rows of q | k | v are zeros and receive finite values that nobody reads; front layout:
-            # the rows beyond a sample's number of valid tokens are never touched
-            masked_attention_backward(q4, k4, v4, o4, do4, lse, None if front is None else key_lengths, mask, dq4, dk4, dv4,
-                                      zero_padded_queries=front is not None)
-        grad_qkv_c = _gather_rows(grad_qkv, index, arows)                             # [valid, 3D]
+        head_dim = width // num_heads
+        heads_of = lambda t, parts: t.view(batch, token_count, parts, num_heads, head_dim).permute(2, 0, 3, 1, 4)  # noqa: E731
+        q4, k4, v4 = heads_of(qkv, 3)
+        dq4, dk4, dv4 = heads_of(grad_qkv, 3)
+        (o4,), (do4,) = heads_of(attended, 1), heads_of(grad_attended, 1)
+        # (the padded rows of q | k | v are zeros and receive finite values that nobody reads)
+        masked_attention_backward(q4, k4, v4, o4, do4, lse, None, mask, dq4, dk4, dv4, zero_padded_queries=False)
+        grad_qkv_c = _gather_rows(grad_qkv, index)                                   # [valid, 3D]
         del grad_qkv, grad_attended
         grad_query_norm = grad_key_norm = None
         if has_qk_norm:
@@ -329,25 +265,153 @@ class InteractionBlockFunction(torch.autograd.Function):
         grad_xc_norm, grad_attn_norm = hip_rms_norm_backward_kernel(xc, attn_norm_w, grad_h1, attn_eps)
         # valid rows: the gradient of the tokens between the halves + that of the norm's input; padded rows: what arrived
         grad_tokens = torch.empty(total, width, dtype=dtype, device=device)
-        if not hasattr(index, "bits"):
-            status = library.taac_rows_merge(grad_padded.data_ptr(), grad_x1c.data_ptr(), grad_xc_norm.data_ptr(),
-                                             key_lengths.data_ptr(), rows.data_ptr() + 4 * total, grad_tokens.data_ptr(),
-                                             batch, token_count, width, _native.current_stream(device))
-        else:
-            status = library.taac_rows_merge_bits(grad_padded.data_ptr(), grad_x1c.data_ptr(), grad_xc_norm.data_ptr(),
-                                                  ctx.index.bits.data_ptr(), ctx.index.word_prefix.data_ptr(),
-                                                  rows.data_ptr() + 4 * total,
-                                                  grad_tokens.data_ptr(), batch, token_count, width,
-                                                  _native.current_stream(device))
+        status = _native.load_library().taac_rows_merge_bits(
+            grad_padded.data_ptr(), grad_x1c.data_ptr(), grad_xc_norm.data_ptr(), index.bits.data_ptr(), None,
+            rows.data_ptr() + 4 * total, grad_tokens.data_ptr(), batch, token_count, width, _native.current_stream(device))
         _native.check(status, "interaction block (training): gradient merge")
-        return (grad_tokens.view(batch, token_count, width), None, None, None, None, None, None, None, None, None,
-                grad_attn_norm,
+        return (grad_tokens.view(batch, token_count, width), None, None, None, None, None, None, None, None, grad_attn_norm,
                 grad_w_qkv, grad_b_qkv, grad_w_out, grad_b_out, weight_grads["ffn_norm"], weight_grads["up"],
                 weight_grads["b_up"], weight_grads["down"], weight_grads["b_down"], grad_query_norm, grad_key_norm)
 
 
+_SLOTS = 12  # parameters per block, in the order of taac_block_weights
+
+
+def _addresses(tensors: list, keep: list):
+    """Array of device addresses (null for None) of contiguous 16-byte aligned tensors; others are copied (into ``keep``)."""
+    table = (ctypes.c_void_p * len(tensors))()
+    for i, tensor in enumerate(tensors):
+        if tensor is None:
+            continue
+        address = tensor.data_ptr()
+        if address & 15 or not tensor.is_contiguous():
+            tensor = tensor.detach().clone(memory_format=torch.contiguous_format)
+            keep.append(tensor)
+            address = tensor.data_ptr()
+        table[i] = address
+    return table
+
+
+def _plain(tensor: torch.Tensor | None, dtype: torch.dtype) -> torch.Tensor | None:
+    """``tensor`` contiguous, 16-byte aligned and of ``dtype``."""
+    if tensor is None:
+        return None
+    tensor = tensor.to(dtype).contiguous()
+    return tensor.clone() if tensor.data_ptr() & 15 else tensor
+
+
+class InteractionStackFunction(torch.autograd.Function):
+    """A stack of interaction blocks, optionally followed by the pCVR readout (masked mean, linear, sigmoid), over the valid
+    tokens. Inputs: tokens ``[B, T, D]`` bf16; int32 ``lengths`` ``[B]`` (valid tokens per sample); ``index``: the
+    :class:`_RowIndex` of a scattered padding or None (prefix padding); ``config`` = (heads, attn_eps, ffn_eps, qk_eps,
+    gate_first, want_out, zero_padded_rows, want_attn_tokens, has_head); then 12 parameters per block in the order of
+    ``taac_block_weights`` (None where a block has none) and the head's weight and bias. All parameters are of one dtype
+    (bf16 or float32). Returns ``(output, attn_tokens, probabilities)``, None where not asked for."""
+
+    @staticmethod
+    def forward(ctx, tokens, lengths, index, config, *params):
+        heads, attn_eps, ffn_eps, qk_eps, gate_first, want_out, zero_padded_rows, want_attn_tokens, has_head = config
+        batch, token_count, width = tokens.shape
+        n_blocks = (len(params) - 2) // _SLOTS if has_head else len(params) // _SLOTS
+        hidden = params[8].shape[1]
+        qk_norm = int(params[10] is not None)
+        device = tokens.device
+        library = _native.load_library()
+        saved_bytes = library.taac_stack_train_bytes(batch, token_count, width, heads, hidden, n_blocks, qk_norm, 0)
+        scratch_bytes = library.taac_stack_train_bytes(batch, token_count, width, heads, hidden, n_blocks, qk_norm, 1)
+        if saved_bytes < 0 or scratch_bytes < 0:
+            raise RuntimeError(f"interaction blocks (training): shape ({batch}, {token_count}, {width}) is not covered")
+        source = _plain(tokens.detach(), torch.bfloat16)
+        saved = torch.empty(saved_bytes, dtype=torch.uint8, device=device)
+        scratch = torch.empty(scratch_bytes, dtype=torch.uint8, device=device)
+        output = torch.empty_like(source) if want_out else None
+        attn_tokens = torch.empty_like(source) if want_attn_tokens else None
+        probabilities = torch.empty(batch, dtype=torch.float32, device=device) if has_head else None
+        keep: list[torch.Tensor] = []
+        table = _addresses(params, keep)
+        head = len(params) - 2
+        rows = count = bits = struct = None
+        stride = 0
+        if index is not None:
+            rows, count, bits = index.rows.data_ptr(), index.count.data_ptr(), index.bits.data_ptr()
+            struct, stride = index.front_mask.struct_bits.data_ptr(), int(index.front_mask.sample_stride)
+        status = library.taac_stack_train_fwd(
+            source.data_ptr(), lengths.data_ptr(), rows, count, bits, struct, stride, table, n_blocks,
+            _native.dtype_code(params[0].dtype), batch, token_count, width, heads, hidden, attn_eps, ffn_eps, qk_eps,
+            int(gate_first), table[head] if has_head else None, table[head + 1] if has_head else None, saved.data_ptr(),
+            scratch.data_ptr(), _native.ptr(output), int(zero_padded_rows), _native.ptr(attn_tokens),
+            _native.ptr(probabilities), _native.current_stream(device))
+        _native.check(status, "interaction blocks (training): forward")
+        ctx.save_for_backward(saved, lengths, probabilities, *params)
+        ctx.index = index
+        ctx.config = (batch, token_count, width, heads, hidden, n_blocks, qk_norm, qk_eps, gate_first, zero_padded_rows, has_head)
+        ctx.set_materialize_grads(False)
+        return output, attn_tokens, probabilities
+
+    @staticmethod
+    def backward(ctx, grad_output, grad_attn_tokens, grad_p):
+        saved, lengths, probabilities, *params = ctx.saved_tensors
+        batch, token_count, width, heads, hidden, n_blocks, qk_norm, qk_eps, gate_first, zero_padded_rows, has_head = ctx.config
+        if grad_output is None and grad_attn_tokens is None and grad_p is None:
+            return (None,) * (4 + len(params))
+        device = saved.device
+        library = _native.load_library()
+        scratch = torch.empty(library.taac_stack_train_bytes(batch, token_count, width, heads, hidden, n_blocks, qk_norm, 2),
+                              dtype=torch.uint8, device=device)
+        grad_output, grad_attn_tokens = _plain(grad_output, torch.bfloat16), _plain(grad_attn_tokens, torch.bfloat16)
+        grad_p = None if grad_p is None else grad_p.to(torch.float32).contiguous()
+        grads = [None if p is None else torch.empty(p.shape, dtype=p.dtype, device=device) for p in params]
+        if grad_output is None and grad_p is None:  # nothing reaches the feed-forward half
+            for slot in range(5, 10):
+                grads[slot] = None
+        head = len(params) - 2
+        if has_head and grad_p is None:
+            grads[head] = grads[head + 1] = None
+        grad_tokens = None
+        if ctx.needs_input_grad[0]:
+            grad_tokens = torch.empty(batch, token_count, width, dtype=torch.bfloat16, device=device)
+        keep: list[torch.Tensor] = []
+        table, grad_table = _addresses(params, keep), (ctypes.c_void_p * len(grads))(*map(_native.ptr, grads))
+        rows = count = bits = struct = None
+        stride = 0
+        index = ctx.index
+        if index is not None:
+            rows, count, bits = index.rows.data_ptr(), index.count.data_ptr(), index.bits.data_ptr()
+            struct, stride = index.front_mask.struct_bits.data_ptr(), int(index.front_mask.sample_stride)
+        status = library.taac_stack_train_bwd(
+            _native.ptr(grad_output), _native.ptr(grad_attn_tokens), _native.ptr(grad_p), _native.ptr(probabilities),
+            lengths.data_ptr(), rows, count, bits, struct, stride, table, grad_table, n_blocks,
+            _native.dtype_code(params[0].dtype), batch, token_count, width, heads, hidden, qk_eps, int(gate_first),
+            grad_table[head] if has_head else None, grad_table[head + 1] if has_head else None, int(zero_padded_rows),
+            saved.data_ptr(), scratch.data_ptr(), _native.ptr(grad_tokens), _native.current_stream(device))
+        _native.check(status, "interaction blocks (training): backward")
+        return (grad_tokens, None, None, None, *grads)
+
+
+def uniform_parameters(params: list) -> list:
+    """``params`` as they are when all are bf16 or all float32; else rounded to bf16 (autograd carries the gradients back)."""
+    dtypes = {p.dtype for p in params if p is not None}
+    if len(dtypes) == 1:
+        return params
+    return [p if p is None or p.dtype == torch.bfloat16 else p.to(torch.bfloat16) for p in params]
+
+
+def _block_parameters(block) -> list:
+    attention, ffn = block.attention, block.ffn
+    qk_norm = attention.query_norm is not None
+    return [block.attn_norm.weight, attention.qkv.weight, attention.qkv.bias, attention.out.weight, attention.out.bias,
+            block.ffn_norm.weight, ffn.up.weight, ffn.up.bias, ffn.down.weight, ffn.down.bias,
+            attention.query_norm.weight if qk_norm else None, attention.key_norm.weight if qk_norm else None]
+
+
+def _block_config(block) -> tuple:
+    attention = block.attention
+    return (attention.num_heads, float(block.attn_norm.eps), float(block.ffn_norm.eps),
+            1e-6 if attention.query_norm is None else float(attention.query_norm.eps), bool(block.ffn.gate_first))
+
+
 def training_route_applies(block, tokens: torch.Tensor, attention_mask, key_lengths, padding_mask=None) -> bool:
-    """Whether :class:`InteractionBlockFunction` covers this call of ``block`` (a ``UnifiedInteractionBlock``): key lengths
+    """Whether :func:`run_training_block` covers this call of ``block`` (a ``UnifiedInteractionBlock``): key lengths
     and no mask, or a structured mask (same for every sample apart from key validity) that was built from
     ``padding_mask``, so that no query can see a padded key."""
     from taac_2026_amd.accelerators.attention import StructuredAttentionMask
@@ -365,6 +429,8 @@ def training_route_applies(block, tokens: torch.Tensor, attention_mask, key_leng
         return False
     if not (tokens.is_cuda and tokens.dtype == torch.bfloat16 and tokens.ndim == 3 and tokens.shape[-1] in (128, 256)):
         return False
+    if tokens.numel() == 0:
+        return False
     attention, ffn = block.attention, block.ffn
     width = tokens.shape[-1]
     head_dim = width // attention.num_heads
@@ -379,23 +445,41 @@ def training_route_applies(block, tokens: torch.Tensor, attention_mask, key_leng
     if key_lengths is not None and (key_lengths.dtype != torch.int32 or not key_lengths.is_cuda
                                     or not key_lengths.is_contiguous()):
         return False
-    # float32 parameters (master weights of mixed-precision training) are cast to bf16 on the way in, as every route of the
-    # module does; autograd carries the gradient back through the cast
+    # (float32 parameters - master weights of mixed-precision training - are rounded to bf16 on the way in, as every route of
+    # the module does)
     return all(p.dtype in (torch.bfloat16, torch.float32) and p.is_cuda for p in block.parameters())
 
 
 def run_training_block(block, tokens: torch.Tensor, key_lengths: torch.Tensor | None, return_attention_tokens: bool,
                        mask=None, padding_mask: torch.Tensor | None = None):
-    """The block through :class:`InteractionBlockFunction`."""
+    """One block through :class:`InteractionStackFunction` (:class:`InteractionBlockFunction` under self-only queries)."""
     attention, ffn = block.attention, block.ffn
-    qk_norm = attention.query_norm is not None
+    if mask is not None and mask.query_self is not None:
+        def bf16(parameter):
+            return parameter if parameter is None or parameter.dtype == torch.bfloat16 else parameter.to(torch.bfloat16)
 
-    def bf16(parameter):
-        return parameter if parameter is None or parameter.dtype == torch.bfloat16 else parameter.to(torch.bfloat16)
+        return InteractionBlockFunction.apply(
+            tokens, mask, padding_mask, bool(return_attention_tokens), attention.num_heads, block.attn_norm.eps,
+            block.ffn_norm.eps, ffn.gate_first, 1e-6 if attention.query_norm is None else attention.query_norm.eps,
+            *map(bf16, _block_parameters(block)))
+    index = None if mask is None else _RowIndex.for_mask(mask, padding_mask, tokens.shape[1])
+    output, attn_tokens, _ = InteractionStackFunction.apply(
+        tokens, key_lengths if index is None else index.lengths, index,
+        (*_block_config(block), True, False, bool(return_attention_tokens), False), *uniform_parameters(_block_parameters(block)))
+    return output, attn_tokens
 
-    return InteractionBlockFunction.apply(
-        tokens, key_lengths, mask, padding_mask, bool(return_attention_tokens), attention.num_heads, block.attn_norm.eps,
-        block.ffn_norm.eps, ffn.gate_first, attention.query_norm.eps if qk_norm else 1e-6, bf16(block.attn_norm.weight),
-        bf16(attention.qkv.weight), bf16(attention.qkv.bias), bf16(attention.out.weight), bf16(attention.out.bias),
-        bf16(block.ffn_norm.weight), bf16(ffn.up.weight), bf16(ffn.up.bias), bf16(ffn.down.weight), bf16(ffn.down.bias),
-        bf16(attention.query_norm.weight) if qk_norm else None, bf16(attention.key_norm.weight) if qk_norm else None)
+
+def run_training_stack(blocks, tokens: torch.Tensor, mask, padding_mask: torch.Tensor) -> torch.Tensor | None:
+    """All ``blocks`` as one function, or None when they do not form one (different settings, hooks, self-only queries)."""
+    config = _block_config(blocks[0])
+    params: list = []
+    for block in blocks:
+        if (block._forward_hooks or block._forward_pre_hooks or block._backward_hooks or block._backward_pre_hooks
+                or _block_config(block) != config):
+            return None
+        params += _block_parameters(block)
+        if params[-_SLOTS + 8].shape != params[8].shape or (params[-1] is None) != (params[11] is None):
+            return None
+    index = _RowIndex.for_mask(mask, padding_mask, tokens.shape[1])
+    return InteractionStackFunction.apply(tokens, index.lengths, index, (*config, True, False, False, False),
+                                          *uniform_parameters(params))[0]

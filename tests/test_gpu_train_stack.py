@@ -1,0 +1,102 @@
+"""GPU parity: the training stack (``taac_stack_train_fwd`` / ``_bwd``: blocks and readout over the compact valid tokens) at the
+edges of its kernels' tiles, against float64 autograd of the CPU oracle. Tolerance: every stored intermediate is rounded to bf16
+once (2^-9 relative); a block stores eight in front of its output (normalised rows, q | k | v, probabilities, attention, x1, hidden
+state, output; weights) and as many gradients behind it, so the error of a result in the 2-norm stays below 16 * 2^-9 = 2^-5 of its
+norm per block it passes."""
+
+from __future__ import annotations
+
+import pytest
+import torch
+import torch.nn.functional as F
+
+from oracle import reference as oracle
+from taac_2026_amd.api import MetadataAttentionMask, PCVRBackbone, UnifiedInteractionBlock, run_interaction_blocks
+
+pytestmark = pytest.mark.gpu
+
+
+def _near(name: str, got: torch.Tensor, want: torch.Tensor, blocks: int) -> None:
+    got, want = got.detach().cpu().double(), want.double()
+    assert (got - want).norm() <= 2.0 ** -5 * blocks * want.norm() + 1e-9, (name, (got - want).norm() / want.norm())
+
+
+@pytest.mark.parametrize("d_model,heads,d_ff,n_blocks,lengths,tokens,qk_norm,dtype", [
+    (256, 8, 1024, 1, [1], 1, False, torch.bfloat16),                     # one token
+    (256, 4, 96, 2, [0, 65, 64, 1], 65, True, torch.float32),             # around a 64-token tile; F not a multiple of a gradient tile
+    (128, 4, 160, 2, [31, 33, 0], 33, False, torch.float32),
+    (128, 2, 256, 1, [257, 3], 257, True, torch.bfloat16),                # rows of a sample over two workgroups of the index
+    (256, 8, 512, 1, [(7 * i) % 33 for i in range(1100)], 32, False, torch.bfloat16),   # 256-token workgroups, some past the count
+    (128, 4, 128, 1, [(5 * i) % 41 for i in range(900)], 40, False, torch.float32),
+])
+def test_training_stack_at_the_edges_of_its_tiles(device, d_model, heads, d_ff, n_blocks, lengths, tokens, qk_norm, dtype):
+    batch = len(lengths)
+    g = torch.Generator().manual_seed(d_model + tokens)
+    model = PCVRBackbone(d_model=d_model, num_heads=heads, d_ff=d_ff, n_blocks=n_blocks, qk_norm=qk_norm)
+    with torch.no_grad():
+        for parameter in model.parameters():
+            if parameter.ndim == 1:
+                parameter.copy_((1.0 if parameter.mean() > 0.5 else 0.0) + 0.1 * torch.randn(parameter.shape, generator=g))
+            else:
+                parameter.copy_(torch.randn(parameter.shape, generator=g) * parameter.shape[1] ** -0.5)
+            parameter.copy_(parameter.to(torch.bfloat16))                 # float32 masters hold bf16 values: the same network
+    reference = {name: value.detach().double().requires_grad_(True) for name, value in model.named_parameters()}
+    model = model.to(dtype).to(device).train()
+    emb = torch.randn(batch, tokens, d_model, generator=g).to(torch.bfloat16)
+    grad_hidden = torch.randn(batch, tokens, d_model, generator=g).to(torch.bfloat16)
+    grad_p = torch.randn(batch, generator=g)
+    lengths = torch.tensor(lengths, dtype=torch.int32)
+
+    emb_d = emb.to(device).requires_grad_(True)
+    p, hidden = model(emb_d, lengths.to(device), return_hidden=True)
+    torch.autograd.backward([p, hidden], [grad_p.to(device), grad_hidden.to(device)])
+
+    emb_r = emb.double().requires_grad_(True)
+    padding = torch.arange(tokens)[None, :] >= lengths[:, None]
+    mask = (~padding)[:, None, None, :].expand(batch, 1, tokens, tokens)
+    x = emb_r
+    for i in range(n_blocks):
+        block = {name.split(".", 2)[2]: value for name, value in reference.items() if name.startswith(f"blocks.{i}.")}
+        x, _ = oracle.interaction_block(x, padding, mask, block, num_heads=heads)
+    keep = (~padding).double().unsqueeze(-1)
+    pooled = (x * keep).sum(1) / keep.sum(1).clamp_min(1.0)
+    want_p = torch.sigmoid(F.linear(pooled, reference["head.weight"], reference["head.bias"]).squeeze(-1))
+    torch.autograd.backward([want_p, x * keep], [grad_p.double(), grad_hidden.double()])
+    _near("p", p, want_p.detach(), n_blocks)
+    _near("hidden", hidden, (x * keep).detach(), n_blocks)
+    _near("tokens", emb_d.grad, emb_r.grad, n_blocks)
+    for name, parameter in model.named_parameters():
+        assert parameter.grad.dtype == dtype
+        _near(name, parameter.grad, reference[name].grad, n_blocks)
+
+
+def test_a_stack_is_its_blocks_one_after_the_other(device):
+    """``run_interaction_blocks`` under autograd (17 blocks: more than one set-up launch) = the blocks called one by one, bit for
+    bit: every kernel is the same, and gathering and scattering the valid rows in between changes no value."""
+    g = torch.Generator().manual_seed(3)
+    roles = torch.tensor([0, 1] + [2] * 5 + [3] * 3 + [6] * 30 + [7] * 2).to(device)
+    batch, tokens, n_blocks = 3, roles.numel(), 17
+    blocks = [UnifiedInteractionBlock(128, 4, 1).to(torch.bfloat16).to(device).train() for _ in range(n_blocks)]
+    x = torch.randn(batch, tokens, 128, generator=g).to(torch.bfloat16).to(device)
+    padding = torch.rand(batch, tokens, generator=g) < 0.4
+    padding[:, :2] = False
+    padding[1] = True
+    padding = padding.to(device)
+    grad = torch.randn(batch, tokens, 128, generator=g).to(torch.bfloat16).to(device)
+
+    def run(one_by_one: bool):
+        mask = MetadataAttentionMask(enabled=True)(padding, roles)
+        xd = x.clone().requires_grad_(True)
+        for block in blocks:
+            block.zero_grad(set_to_none=True)
+        out = xd
+        if one_by_one:
+            for block in blocks:
+                out, _ = block(out, padding, mask, return_attention_tokens=False)
+        else:
+            out = run_interaction_blocks(blocks, xd, padding, mask)
+        out.backward(grad)
+        return [out.detach(), xd.grad] + [p.grad for block in blocks for p in block.parameters()]
+
+    for got, want in zip(run(False), run(True)):
+        assert torch.equal(got, want)
