@@ -18,8 +18,10 @@
 // and stream L2 -> LDS by direct transfers through a ring of four 24 KB buffers, three sub-steps ahead (a sub-step is
 // eight k-steps of the three blocks: half a step at D = 256, a whole one at D = 128; with two whole-step buffers, one
 // step ahead, the wait for the weights was exposed in every step: 1.54 ms against the time below at 524 288 tokens);
-// results leave through a wavefront-private LDS tile as 16-byte stores that cover 64-byte runs of a row.
+// results leave through a wavefront-private LDS tile as 16-byte stores that cover 64-byte runs of a row, or, in panel order
+// (train_ops.h, the training stack), 1 KB in one run: 294 912 tokens, D = 256, F = 1024: 749 -> 600 us.
 #include "pack.h"
+#include "train_ops.h"
 #include "ts_common.h"
 
 namespace taac {
@@ -28,6 +30,7 @@ namespace {
 constexpr int kWaves = 8;
 constexpr int kTokPerWg = kWaves * 32;
 constexpr int kUnits = kBwdUnits;               // hidden units per step
+static_assert(kUnits == kPanelCols && kTokPerWg == kPanelRows, "a workgroup's step is one panel of each result");
 constexpr int kSubK = kBwdSubK;                 // k-steps (of 16 features) per sub-step
 constexpr int kRing = 4;                        // weight buffers
 constexpr int kTileRow = 3 * kUnits * 2 + 16;   // epilogue tile row: hidden | grad first half | grad second half | pad
@@ -42,6 +45,8 @@ struct FfnBwdParams {
   bf16_t* grad_pre;       // [M, 2F] row stride ldgp
   int64_t M, ldh, lddy, ldhid, ldgp;
   int32_t F;
+  bool panels;            // hidden and grad_pre are written in panel order (train_ops.h): every store of a step is a contiguous
+                          // 1 KB run, against 64 bytes per row and 4 KB pitch
   const int32_t* count;   // number of tokens on the device (at most M), or null: M
   const float* rstd;      // [M]: h holds rows x in front of a norm whose weight is part of the packed up projection; the rows
                           // enter as bf16(x * rstd), as in the forward kernel. Null: h as it is
@@ -131,9 +136,16 @@ __global__ __launch_bounds__(kWaves * kWave, 2) void swiglu_ffn_bwd_hidden_kerne
     }
   }
   // memory rows of the epilogue stores: piece i = token 16 * i + lane / 4
-  int64_t prow[2];
+  bf16_t* hid_row[2];
+  bf16_t* gp_row[2];
 #pragma unroll
-  for (int i = 0; i < 2; ++i) prow[i] = row_of(tok0 + i * 16 + lane / 4);
+  for (int i = 0; i < 2; ++i) {
+    const int64_t row = row_of(tok0 + i * 16 + lane / 4);
+    hid_row[i] = p.hidden + (p.panels ? panel_row(row, p.F) : row * p.ldhid) + (lane % 4) * 8;
+    gp_row[i] = p.grad_pre + (p.panels ? panel_row(row, 2 * p.F) : row * p.ldgp) + (lane % 4) * 8;
+  }
+  const int64_t step_stride = p.panels ? kPanel : kUnits;                             // from 32 columns to the next
+  const int64_t half_stride = p.panels ? static_cast<int64_t>(p.F) * kPanelRows : p.F;  // from column 0 to column F
   vm_wait<0>();
   __syncthreads();
 
@@ -211,7 +223,7 @@ __global__ __launch_bounds__(kWaves * kWave, 2) void swiglu_ffn_bwd_hidden_kerne
         }
         asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
         // ---- row-wise out of the tile: lane -> token 16 * i + lane / 4, 16-byte piece lane % 4 of each 64-byte run --------
-        const int unit0 = s * kUnits + (lane % 4) * 8;
+        const int64_t unit0 = s * step_stride;
 #pragma unroll
         for (int i = 0; i < 2; ++i) {
           const uint8_t* src = tile + (i * 16 + lane / 4) * kTileRow + (lane % 4) * 16;
@@ -219,9 +231,9 @@ __global__ __launch_bounds__(kWaves * kWave, 2) void swiglu_ffn_bwd_hidden_kerne
           const bf16x8 ga = *reinterpret_cast<const bf16x8*>(src + kUnits * 2);
           const bf16x8 gb = *reinterpret_cast<const bf16x8*>(src + 2 * kUnits * 2);
           // streaming stores: 6 KB per token leave the kernel and nothing of it is read again here (1.50 -> 1.34 ms)
-          __builtin_nontemporal_store(hv, reinterpret_cast<bf16x8*>(p.hidden + prow[i] * p.ldhid + unit0));
-          __builtin_nontemporal_store(ga, reinterpret_cast<bf16x8*>(p.grad_pre + prow[i] * p.ldgp + unit0));
-          __builtin_nontemporal_store(gb, reinterpret_cast<bf16x8*>(p.grad_pre + prow[i] * p.ldgp + p.F + unit0));
+          __builtin_nontemporal_store(hv, reinterpret_cast<bf16x8*>(hid_row[i] + unit0));
+          __builtin_nontemporal_store(ga, reinterpret_cast<bf16x8*>(gp_row[i] + unit0));
+          __builtin_nontemporal_store(gb, reinterpret_cast<bf16x8*>(gp_row[i] + half_stride + unit0));
         }
         asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
       }
@@ -282,6 +294,7 @@ int ffn_bwd_hidden_count(const char* name, const void* x, const float* rstd, con
   p.ldhid = F;
   p.ldgp = 2 * F;
   p.F = F;
+  p.panels = true;
   p.count = count;
   p.rstd = rstd;
   return D == 256 ? launch_bwd_hidden<256>(p, gate_first, s, name) : launch_bwd_hidden<128>(p, gate_first, s, name);

@@ -489,8 +489,8 @@ Scratch scratch_layout(const Sizes& z, char* base, bool backward) {
     const int64_t row = z.M * z.D * 2;
     s.dy = reinterpret_cast<bf16_t*>(take(row));
     s.dx1 = reinterpret_cast<bf16_t*>(take(row));
-    s.hidden = reinterpret_cast<bf16_t*>(take(z.M * z.F * 2));
-    s.grad_pre = reinterpret_cast<bf16_t*>(take(z.M * z.F * 4));
+    s.hidden = reinterpret_cast<bf16_t*>(take(panel_rows(z.M) * z.F * 2));  // panel order
+    s.grad_pre = reinterpret_cast<bf16_t*>(take(panel_rows(z.M) * z.F * 4));
     s.datt = reinterpret_cast<bf16_t*>(take(row));
     s.dqkv = reinterpret_cast<bf16_t*>(take(3 * row));
     s.delta = reinterpret_cast<float*>(take(static_cast<int64_t>(z.B) * z.H * z.T * 4));
@@ -733,7 +733,7 @@ extern "C" int taac_stack_train_bwd(const void* grad_out, const void* grad_attn_
       if ((rc = ffn_bwd_hidden_count(name, b.x1, b.rstd_ffn, dy, pk + sv.pb.ffn_bwd, v.up_bias, sc.hidden, sc.grad_pre, M, D, F,
                                      gate_first != 0, count, s)) != TAAC_OK)
         return rc;
-      if ((rc = dgrad_norm(name, sc.grad_pre, 2 * F, pk + sv.pb.up_t, b.x1, b.rstd_ffn, v.ffn_norm, dy, dx1, M, D, count, s)) != TAAC_OK)
+      if ((rc = dgrad_norm(name, sc.grad_pre, true, 2 * F, pk + sv.pb.up_t, b.x1, b.rstd_ffn, v.ffn_norm, dy, dx1, M, D, count, s)) != TAAC_OK)
         return rc;
     }
     // (a gradient of the tokens between the halves belongs to a stack of one block)
@@ -760,18 +760,18 @@ extern "C" int taac_stack_train_bwd(const void* grad_out, const void* grad_attn_
       vectors[n_vectors++] = VectorItem{part + D, const_cast<void*>(g.key_norm_weight), static_cast<int32_t>(nb), 2 * D, D};
     }
     WgradItem items[kWgradItems] = {
-        {sc.dqkv, b.x, b.rstd_attn, 3 * D, D, w.qkv_weight, w.attn_norm_weight, const_cast<void*>(g.qkv_weight),
+        {sc.dqkv, b.x, b.rstd_attn, 3 * D, D, false, false, w.qkv_weight, w.attn_norm_weight, const_cast<void*>(g.qkv_weight),
          const_cast<void*>(g.qkv_bias), const_cast<void*>(g.attn_norm_weight)},
-        {dx1, b.att, nullptr, D, D, nullptr, nullptr, const_cast<void*>(g.out_weight), const_cast<void*>(g.out_bias), nullptr},
-        {sc.grad_pre, b.x1, b.rstd_ffn, 2 * F, D, w.up_weight, w.ffn_norm_weight, const_cast<void*>(g.up_weight),
+        {dx1, b.att, nullptr, D, D, false, false, nullptr, nullptr, const_cast<void*>(g.out_weight), const_cast<void*>(g.out_bias), nullptr},
+        {sc.grad_pre, b.x1, b.rstd_ffn, 2 * F, D, true, false, w.up_weight, w.ffn_norm_weight, const_cast<void*>(g.up_weight),
          const_cast<void*>(g.up_bias), const_cast<void*>(g.ffn_norm_weight)},
-        {dy, sc.hidden, nullptr, D, F, nullptr, nullptr, const_cast<void*>(g.down_weight), const_cast<void*>(g.down_bias), nullptr}};
+        {dy, sc.hidden, nullptr, D, F, false, true, nullptr, nullptr, const_cast<void*>(g.down_weight), const_cast<void*>(g.down_bias), nullptr}};
     if ((rc = wgrad_block(name, items, have_dy ? 4 : 2, M, count, sc.wgrad, sc.vectors + i * sc.vector_stride, param_dtype,
                           vectors.data(), &n_vectors, s)) != TAAC_OK)
       return rc;
     // the block's input gradient takes the place of dy, which nothing reads any more
     if ((i > 0 || grad_tokens != nullptr) &&
-        (rc = dgrad_norm(name, sc.dqkv, 3 * D, pk + sv.pb.qkv_t, b.x, b.rstd_attn, v.attn_norm, dx1, dy, M, D, count, s)) != TAAC_OK)
+        (rc = dgrad_norm(name, sc.dqkv, false, 3 * D, pk + sv.pb.qkv_t, b.x, b.rstd_attn, v.attn_norm, dx1, dy, M, D, count, s)) != TAAC_OK)
       return rc;
     have_dy = true;
   }

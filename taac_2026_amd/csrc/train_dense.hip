@@ -33,6 +33,7 @@ struct DgradParams {
   const int32_t* count;
   int64_t M;
   int32_t K;
+  bool panels;           // dy in panel order
 };
 
 template <int D, int TG>
@@ -66,7 +67,7 @@ __global__ __launch_bounds__(TG * 2 * kWave, 2) void dgrad_norm_kernel(const Dgr
   for (int i = 0; i < 2; ++i) {
     const int row = 16 * (2 * wave + i) + lane / 4;
     const int64_t arow = m0 + row < rows ? m0 + row : rows - 1;
-    a_src[i] = p.dy + arow * p.K + ((lane % 4) ^ ((row >> 2) & 3)) * 8;
+    a_src[i] = p.dy + (p.panels ? panel_row(arow, p.K) : arow * p.K) + ((lane % 4) ^ ((row >> 2) & 3)) * 8;
   }
 #pragma unroll
   for (int i = 0; i < WT; ++i) {
@@ -76,12 +77,16 @@ __global__ __launch_bounds__(TG * 2 * kWave, 2) void dgrad_norm_kernel(const Dgr
   // every workgroup starts its walk over K at a different slab: with all of them on the same columns of a matrix whose row pitch
   // is a power of two their requests crowd the same memory channels
   const int rot = static_cast<int>((blockIdx.x * 5u) % static_cast<uint32_t>(nslabs));
+  static_assert(kSlab == kPanelCols && kPanelRows % TOK == 0, "a slab of a workgroup lies in one panel");
+  const int64_t slab_stride = p.panels ? kPanel : kSlab;
   auto stage = [&](int slab) {
     uint8_t* base = smem + (slab % kRing) * kStage;
     const int turned = slab + rot;
-    const int k0 = (turned >= nslabs ? turned - nslabs : turned) * kSlab;
+    const int at = turned >= nslabs ? turned - nslabs : turned;
+    const int64_t a0 = at * slab_stride;
+    const int k0 = at * kSlab;
 #pragma unroll
-    for (int i = 0; i < 2; ++i) lds_dma16(a_src[i] + k0, base + (2 * wave + i) * 1024);
+    for (int i = 0; i < 2; ++i) lds_dma16(a_src[i] + a0, base + (2 * wave + i) * 1024);
 #pragma unroll
     for (int i = 0; i < WT; ++i) lds_dma16(w_src[i] + k0, base + kTokBytes + (WT * wave + i) * 1024);
   };
@@ -277,23 +282,29 @@ __global__ __launch_bounds__(WN * WK * kWave, 2) void wgrad_block_kernel(const W
   const int rn = tid / (TN / 8), cn = n0 + tid % (TN / 8) * 8;
   const int rk = tid / (TK / 8), ck = k0 + tid % (TK / 8) * 8;
   const bool n_ok = cn < N, k_ok = ck < K;
-  const bf16_t* dy_col = it.dy + (n_ok ? cn : 0);
-  const bf16_t* a_col = it.a + (k_ok ? ck : 0);
+  // (a chunk of kChunk tokens lies in one row block of the panel order, a piece of eight columns in one panel)
+  static_assert(kPanelRows % kChunk == 0 && kPanelCols % 8 == 0, "chunks and pieces do not straddle panels");
+  auto column = [](int c, bool panels) -> int64_t { return panels ? c / kPanelCols * kPanel + c % kPanelCols : c; };
+  const bf16_t* dy_col = it.dy + column(n_ok ? cn : 0, it.dy_panels);
+  const bf16_t* a_col = it.a + column(k_ok ? ck : 0, it.a_panels);
+  const int64_t dy_ld = it.dy_panels ? kPanelCols : N, a_ld = it.a_panels ? kPanelCols : K;
   const float* rscale = it.scale;
   u32x4 va[PN], vb[PK];
   float sb[PK];
   const u32x4 zero = {0u, 0u, 0u, 0u};
   auto fetch = [&](int64_t m0) {
+    const bf16_t* dy_chunk = dy_col + (it.dy_panels ? panel_row(m0, N) : m0 * N);
+    const bf16_t* a_chunk = a_col + (it.a_panels ? panel_row(m0, K) : m0 * K);
 #pragma unroll
     for (int i = 0; i < PN; ++i) {
       const int64_t m = m0 + rn + RN * i;
-      va[i] = (m < m_end && n_ok) ? *reinterpret_cast<const u32x4*>(dy_col + m * N) : zero;
+      va[i] = (m < m_end && n_ok) ? *reinterpret_cast<const u32x4*>(dy_chunk + (rn + RN * i) * dy_ld) : zero;
     }
 #pragma unroll
     for (int i = 0; i < PK; ++i) {
       const int64_t m = m0 + rk + RK * i;
       const bool ok = m < m_end && k_ok;
-      vb[i] = ok ? *reinterpret_cast<const u32x4*>(a_col + m * K) : zero;
+      vb[i] = ok ? *reinterpret_cast<const u32x4*>(a_chunk + (rk + RK * i) * a_ld) : zero;
       sb[i] = (ok && rscale != nullptr) ? rscale[m] : 1.f;
     }
   };
@@ -508,7 +519,7 @@ WgradPlan plan_of(int64_t M, const int32_t (*shapes)[2], int items) {
 
 }  // namespace
 
-int dgrad_norm(const char* name, const void* dy, int32_t K, const void* w_t, const void* x, const float* rstd, const void* norm_w,
+int dgrad_norm(const char* name, const void* dy, bool dy_panels, int32_t K, const void* w_t, const void* x, const float* rstd, const void* norm_w,
                const void* dres, void* dx, int64_t M, int32_t D, const int32_t* count, hipStream_t s) {
   DgradParams p{};
   p.dy = static_cast<const bf16_t*>(dy);
@@ -521,6 +532,7 @@ int dgrad_norm(const char* name, const void* dy, int32_t K, const void* w_t, con
   p.count = count;
   p.M = M;
   p.K = K;
+  p.panels = dy_panels;
   const int cus = compute_units();
   const bool small = M < 128 * static_cast<int64_t>(cus);
   if (D == 256) return small ? launch_dgrad<256, 1>(p, s, name) : launch_dgrad<256, 4>(p, s, name);

@@ -8,6 +8,17 @@
 
 namespace taac {
 
+// Panel order of a tall [M, N] matrix that one kernel writes and the next ones read in column slabs: panels of 256 rows x 32
+// columns, each contiguous, the panels of a row block one behind the other (N and the row capacity are multiples of 32 and 256).
+// A 32-column slab of 256 rows is 16 KB in one run; in row-major order it is 64-byte runs a power of two apart, which take half a
+// cache line each and crowd the same memory channels.
+constexpr int kPanelRows = 256, kPanelCols = 32;
+constexpr int64_t kPanel = kPanelRows * kPanelCols;
+inline int64_t panel_rows(int64_t M) { return (M + kPanelRows - 1) / kPanelRows * kPanelRows; }
+__device__ __forceinline__ int64_t panel_row(int64_t m, int64_t N) {  // element offset of column 0 of row m
+  return (m / kPanelRows) * kPanelRows * N + (m % kPanelRows) * kPanelCols;
+}
+
 // out = linear([rmsnorm](x)), K = D in {128, 256}; the norm's weight is folded into `packed` (norm_weight only says that there is
 // one); rstd_out [M]: the norm's factor per row, or null.
 int norm_linear_count(const char* name, const void* x, const void* norm_weight, float eps, const void* bias, const void* packed,
@@ -30,14 +41,14 @@ int attention_compact_bwd(const char* name, const void* qk, const void* v, int64
                           const uint32_t* struct_bits, int64_t struct_stride, void* dqkv, int64_t ld_dqkv, float* delta, int32_t B,
                           int32_t H, int32_t T, int32_t dh, hipStream_t s);
 // hidden [M, F] and the gradient of the up projection [M, 2F] from x (in front of the norm; rstd its factor) and the gradient dy
-// of the feed-forward output.
+// of the feed-forward output. Both results are in panel order.
 int ffn_bwd_hidden_count(const char* name, const void* x, const float* rstd, const void* dy, const void* packed, const void* b_up,
                          void* hidden, void* grad_pre, int64_t M, int32_t D, int32_t F, bool gate_first, const int32_t* count,
                          hipStream_t s);
 
 // dx = dres + d rmsnorm(x) applied to dy W (train_dense.hip): dy [M, K], w_t [D, K] (the layer's weight transposed), x [M, D] the
-// rows in front of the norm, rstd its factor, norm_w [D] its weight. dx may be dres.
-int dgrad_norm(const char* name, const void* dy, int32_t K, const void* w_t, const void* x, const float* rstd, const void* norm_w,
+// rows in front of the norm, rstd its factor, norm_w [D] its weight. dx may be dres. dy_panels: dy is in panel order.
+int dgrad_norm(const char* name, const void* dy, bool dy_panels, int32_t K, const void* w_t, const void* x, const float* rstd, const void* norm_w,
                const void* dres, void* dx, int64_t M, int32_t D, const int32_t* count, hipStream_t s);
 
 // Weight gradients of the four dense layers of a block in one launch (train_dense.hip): G[n, k] = sum over the rows of dy[m, n] *
@@ -48,6 +59,7 @@ struct WgradItem {
   const bf16_t* a;
   const float* scale;       // [M] or null
   int32_t N, K;             // dy [M, N], a [M, K]
+  bool dy_panels, a_panels; // ... in panel order
   // reduction: dw [N, K] = G * norm_w (per column) when norm_w is given; dnorm[k] = sum over n of w[n, k] * G[n, k]
   const void* w;            // [N, K] the layer's weight (with norm_w)
   const void* norm_w;       // [K] or null
