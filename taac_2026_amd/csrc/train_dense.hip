@@ -17,6 +17,8 @@ namespace {
 // The epilogue replaces a store of dh = dy W, the norm's backward over x and dh, and the residual add: 3 of the 8 passes over
 // [M, D] that the layer-by-layer backward makes here. The gradient of the norm's weight is left to the weight-gradient kernels,
 // which hold sum_m dy[m, n] x_hat[m, k] anyway (d norm_w[k] = sum_n w[n, k] of it).
+// The epilogue's rows pass through LDS: read and written as a lane's own eight bytes of 32 rows at once, they cost 46 us per
+// 256-token workgroup whatever K (294 912 tokens, D = 256: K = 768 337 -> 220 us, K = 2048 515 -> 400 us).
 // Bound: HBM (dy, K * 2 bytes per token); 64-token workgroups (TG = 1) where 256-token ones would leave compute units idle.
 // ------------------------------------------------------------------------------------------------------------------
 constexpr int kSlab = 32;
@@ -136,75 +138,85 @@ __global__ __launch_bounds__(TG * 2 * kWave, 2) void dgrad_norm_kernel(const Dgr
     __syncthreads();
   }
 
-  // acc[ni][mi][jq * 4 + e]: feature wn * D / 2 + ni * 32 + jq * 8 + hh * 4 + e of token wt * 64 + mi * 32 + l32
-  float* red = reinterpret_cast<float*>(smem);  // [2 feature halves][TOK] sums of g * x_hat
-  // (the rows of x are read twice, the second time from the caches: held between the passes they do not fit the registers)
-  float scale[2], part[2];
+  // acc[ni][mi][jq * 4 + e]: feature wn * D / 2 + ni * 32 + jq * 8 + hh * 4 + e of token wt * 64 + mi * 32 + l32.
+  // A lane holds eight bytes out of each 32 features of one row, so x, dres and dx pass through LDS, 32 * TG tokens (one mi) at a
+  // time over the ring's memory: whole rows in and out of memory, the 16-byte pieces of a tile row XOR-swizzled by row % 16.
+  constexpr int TILE_ROWS = 32 * TG, kRowBytes = D * 2, kTile = TILE_ROWS * kRowBytes;
+  constexpr int RPT = 1024 / kRowBytes;           // rows per transfer
+  constexpr int NT = TILE_ROWS / NWAVES / RPT;    // transfers per wavefront and tile
+  constexpr int PIECES = D / 8;
+  uint8_t* x_tile = smem;
+  uint8_t* res_tile = smem + kTile;
+  float* red = reinterpret_cast<float*>(smem + 2 * kTile);  // [2 feature halves][TILE_ROWS] sums of g * x
+  const int trow = wt * 32 + l32;
+  auto token_of = [&](int tile_row, int mi) { return m0 + tile_row / 32 * 64 + mi * 32 + tile_row % 32; };
+  auto lane_piece = [&](int ni, int jq) { return trow * kRowBytes + (((wn * (D / 16) + ni * 4 + jq) ^ (trow & 15)) * 16) + hh * 8; };
 #pragma unroll
   for (int mi = 0; mi < 2; ++mi) {
-    const int64_t m = m0 + wt * 64 + mi * 32 + l32;
-    const int64_t row = m < rows ? m : rows - 1;
-    scale[mi] = p.rstd[row];
-    part[mi] = 0.f;
-    const bf16_t* xrow = p.x + row * D + wn * (D / 2) + hh * 4;
+    if (mi > 0) __syncthreads();  // the tiles have been stored
 #pragma unroll
-    for (int ni = 0; ni < NI; ++ni) {
-      bf16x4 xv[4], wv[4];
+    for (int i = 0; i < NT; ++i) {
+      const int tr = (wave * NT + i) * RPT + lane / PIECES;
+      const int64_t m = token_of(tr, mi);
+      const int64_t at = (m < rows ? m : rows - 1) * D + ((lane % PIECES) ^ (tr & 15)) * 8;
+      lds_dma16(p.x + at, x_tile + (wave * NT + i) * 1024);
+      lds_dma16(p.dres + at, res_tile + (wave * NT + i) * 1024);
+    }
+    const int64_t m = token_of(trow, mi);
+    const float scale = p.rstd[m < rows ? m : rows - 1];
+    vm_wait<0>();
+    __syncthreads();
+    float part = 0.f;
+#pragma unroll
+    for (int ni = 0; ni < NI; ++ni)
 #pragma unroll
       for (int jq = 0; jq < 4; ++jq) {
-        xv[jq] = *reinterpret_cast<const bf16x4*>(xrow + ni * 32 + jq * 8);
-        wv[jq] = *reinterpret_cast<const bf16x4*>(p.norm_w + wn * (D / 2) + ni * 32 + jq * 8 + hh * 4);
-      }
-#pragma unroll
-      for (int jq = 0; jq < 4; ++jq)
+        const bf16x4 xv = *reinterpret_cast<const bf16x4*>(x_tile + lane_piece(ni, jq));
+        const bf16x4 wv = *reinterpret_cast<const bf16x4*>(p.norm_w + wn * (D / 2) + ni * 32 + jq * 8 + hh * 4);
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
-          const float g = acc[ni][mi][jq * 4 + e] * static_cast<float>(wv[jq][e]);
+          const float g = acc[ni][mi][jq * 4 + e] * static_cast<float>(wv[e]);
           acc[ni][mi][jq * 4 + e] = g;
-          part[mi] = fmaf(g, static_cast<float>(xv[jq][e]), part[mi]);  // times rstd: x_hat
+          part = fmaf(g, static_cast<float>(xv[e]), part);  // times rstd: x_hat
         }
-    }
-  }
-#pragma unroll
-  for (int mi = 0; mi < 2; ++mi) {
-    const uint32_t u = __builtin_bit_cast(uint32_t, part[mi]);
+      }
+    const uint32_t u = __builtin_bit_cast(uint32_t, part);
     const auto r = __builtin_amdgcn_permlane32_swap(u, u, false, false);
     const float both = __builtin_bit_cast(float, static_cast<uint32_t>(r[0])) + __builtin_bit_cast(float, static_cast<uint32_t>(r[1]));
-    if (hh == 0) red[wn * TOK + wt * 64 + mi * 32 + l32] = both;
-  }
-  __syncthreads();
-#pragma unroll
-  for (int mi = 0; mi < 2; ++mi) {
-    const int64_t m = m0 + wt * 64 + mi * 32 + l32;
-    if (m >= rows) continue;
-    const int t = wt * 64 + mi * 32 + l32;
+    if (hh == 0) red[wn * TILE_ROWS + trow] = both;
+    __syncthreads();
     // mean(g * x_hat) * x_hat = (sum of g * x) / D * rstd^2 * x
-    const float proj = (red[t] + red[TOK + t]) * (1.0f / D) * scale[mi] * scale[mi];
+    const float proj = (red[trow] + red[TILE_ROWS + trow]) * (1.0f / D) * scale * scale;
 #pragma unroll
-    for (int ni = 0; ni < NI; ++ni) {
-      const int64_t at = m * D + wn * (D / 2) + ni * 32 + hh * 4;
-      bf16x4 xv[4], rv[4];
+    for (int ni = 0; ni < NI; ++ni)
 #pragma unroll
       for (int jq = 0; jq < 4; ++jq) {
-        xv[jq] = *reinterpret_cast<const bf16x4*>(p.x + at + jq * 8);
-        rv[jq] = *reinterpret_cast<const bf16x4*>(p.dres + at + jq * 8);
-      }
-#pragma unroll
-      for (int jq = 0; jq < 4; ++jq) {
+        bf16x4* xp = reinterpret_cast<bf16x4*>(x_tile + lane_piece(ni, jq));
+        const bf16x4 xv = *xp;
+        const bf16x4 rv = *reinterpret_cast<const bf16x4*>(res_tile + lane_piece(ni, jq));
         bf16x4 ov;
 #pragma unroll
         for (int e = 0; e < 4; ++e)
-          ov[e] = static_cast<bf16_t>(static_cast<float>(rv[jq][e]) +
-                                      scale[mi] * (acc[ni][mi][jq * 4 + e] - static_cast<float>(xv[jq][e]) * proj));
-        *reinterpret_cast<bf16x4*>(p.dx + at + jq * 8) = ov;
+          ov[e] = static_cast<bf16_t>(static_cast<float>(rv[e]) +
+                                      scale * (acc[ni][mi][jq * 4 + e] - static_cast<float>(xv[e]) * proj));
+        *xp = ov;
       }
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < NT; ++i) {
+      const int tr = (wave * NT + i) * RPT + lane / PIECES;
+      const int64_t mo = token_of(tr, mi);
+      const bf16x8 ov = *reinterpret_cast<const bf16x8*>(x_tile + tr * kRowBytes + ((lane % PIECES) ^ (tr & 15)) * 16);
+      if (mo < rows) *reinterpret_cast<bf16x8*>(p.dx + mo * D + lane % PIECES * 8) = ov;
     }
   }
 }
 
 template <int D, int TG>
 int launch_dgrad(const DgradParams& p, hipStream_t s, const char* name) {
-  constexpr size_t lds = static_cast<size_t>(kRing) * (64 * TG + D) * kSlab * 2;
+  constexpr size_t ring = static_cast<size_t>(kRing) * (64 * TG + D) * kSlab * 2;
+  constexpr size_t tiles = 2 * static_cast<size_t>(32 * TG) * (D * 2 + sizeof(float));
+  constexpr size_t lds = ring > tiles ? ring : tiles;
   if (hipFuncSetAttribute(reinterpret_cast<const void*>(dgrad_norm_kernel<D, TG>), hipFuncAttributeMaxDynamicSharedMemorySize,
                           static_cast<int>(lds)) != hipSuccess)
     return set_error(TAAC_ERR_LAUNCH, "%s: cannot reserve %zu bytes of LDS", name, lds);
