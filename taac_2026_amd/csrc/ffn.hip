@@ -1849,11 +1849,12 @@ int attn_out_ffn_count(const char* name, const void* attn, const void* out_bias,
 }
 
 // Whether the gated feed-forward over at most M rows of D features runs as the few-token kernel: as long as its 32-token
-// workgroups fit the chip in one round. Measured with the out projection in front, launches back to back, few-token /
+// workgroups are at most two rounds of the chip. M counts padded rows; with half of them valid (9 648 rows, 6 100 tokens,
+// training) 26.9 / 64.8 us. Measured with the out projection in front, launches back to back, few-token /
 // persistent kernel, us: D = 256, F = 1024 - 512 rows 21.5 / 49.9, 8192 27.8 / 55.6, 16384 53.8 / 57.7, 24576 72.5 / 58.2;
 // F = 512 - 8192 18.8 / 34.7, 16384 34.4 / 36.4; D = 128 (two workgroups per compute unit), F = 512 - 512 rows 9.2 / 19.5,
 // 16384 16.8 / 21.9, 24576 23.0 / 22.2.
-bool ffn_few_rows(int64_t M, int32_t D) { return test_max_workgroups() == 0 && M * D <= 8192 * 256; }
+bool ffn_few_rows(int64_t M, int32_t D) { return test_max_workgroups() == 0 && M * D <= 16384 * 256; }
 
 // Whether a projection over at most M rows of D features runs as the few-token kernel. Measured for q | k | v (launches
 // back to back, few-token / persistent kernel, us): D = 256 - 512 rows 6.0 / 13.6, 4096 9.9 / 14.1, 8192 14.4 / 15.6,

@@ -83,7 +83,9 @@ __global__ __launch_bounds__(kWaves * kWave, 2) void swiglu_ffn_bwd_hidden_kerne
   const int lane = tid % kWave;
   const int l32 = lane % 32;
   const int hh = lane / 32;
-  const int nsteps = p.F / kUnits;
+  const int total_steps = p.F / kUnits;
+  const int step0 = total_steps * static_cast<int>(blockIdx.y) / static_cast<int>(gridDim.y);  // this workgroup's steps
+  const int nsteps = total_steps * (static_cast<int>(blockIdx.y) + 1) / static_cast<int>(gridDim.y) - step0;
   const int nsub = nsteps * NSUB;
   const int64_t tok0 = static_cast<int64_t>(blockIdx.x) * kTokPerWg + wave * 32;
   int64_t M = p.M;
@@ -96,7 +98,7 @@ __global__ __launch_bounds__(kWaves * kWave, 2) void swiglu_ffn_bwd_hidden_kerne
   // benign and every wavefront issues the same number of memory operations (the hand-counted waits rely on that).
   auto row_of = [&](int64_t tok) -> int64_t { return tok < M ? tok : M - 1; };
 
-  const char* w_bytes = reinterpret_cast<const char*>(p.packed);
+  const char* w_bytes = reinterpret_cast<const char*>(p.packed) + static_cast<int64_t>(step0) * NSUB * kBuf;
   auto stage = [&](int q) {  // sub-step q -> ring slot q % kRing
     int ln = lane;
     asm volatile("" : "+v"(ln));
@@ -155,7 +157,7 @@ __global__ __launch_bounds__(kWaves * kWave, 2) void swiglu_ffn_bwd_hidden_kerne
     // hidden unit 32 s + jq * 8 + hh * 4 + e of token l32)
     f32x16 acc_a, acc_b, acc_d;
     {
-      const bf16_t* bias = bias_lds + s * kUnits + hh * 4;
+      const bf16_t* bias = bias_lds + (step0 + s) * kUnits + hh * 4;
 #pragma unroll
       for (int jq = 0; jq < 4; ++jq) {
         const bf16x4 ba = *reinterpret_cast<const bf16x4*>(bias + jq * 8);
@@ -223,7 +225,7 @@ __global__ __launch_bounds__(kWaves * kWave, 2) void swiglu_ffn_bwd_hidden_kerne
         }
         asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
         // ---- row-wise out of the tile: lane -> token 16 * i + lane / 4, 16-byte piece lane % 4 of each 64-byte run --------
-        const int64_t unit0 = s * step_stride;
+        const int64_t unit0 = (step0 + s) * step_stride;
 #pragma unroll
         for (int i = 0; i < 2; ++i) {
           const uint8_t* src = tile + (i * 16 + lane / 4) * kTileRow + (lane % 4) * 16;
@@ -264,11 +266,17 @@ int launch_bwd_hidden(const FfnBwdParams& p, bool gate_first, hipStream_t s, con
   const size_t lds_bytes = bwd_lds_bytes(D, p.F);
   const int64_t grid = (p.M + kTokPerWg - 1) / kTokPerWg;
   if (grid > 0x7fffffffLL) return set_error(TAAC_ERR_UNSUPPORTED, "%s: too many workgroups", name);
+  // The hidden units are divided over workgroups too where the token tiles are few: about four workgroups per compute unit, at
+  // least four steps each (a workgroup's rows arrive in front of its first step).
+  const int cus = compute_units();
+  const int64_t by_grid = (4 * static_cast<int64_t>(cus > 0 ? cus : 1)) / grid, by_steps = p.F / kUnits / 4;
+  const int64_t most = by_grid < by_steps ? by_grid : by_steps;
+  const uint32_t splits = most < 1 ? 1u : static_cast<uint32_t>(most);
   auto go = [&](auto kernel) -> int {
     if (hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize,
                             static_cast<int>(lds_bytes)) != hipSuccess)
       return set_error(TAAC_ERR_LAUNCH, "%s: cannot reserve %zu bytes of LDS", name, lds_bytes);
-    hipLaunchKernelGGL(kernel, dim3(static_cast<uint32_t>(grid)), dim3(kWaves * kWave), lds_bytes, s, p);
+    hipLaunchKernelGGL(kernel, dim3(static_cast<uint32_t>(grid), splits), dim3(kWaves * kWave), lds_bytes, s, p);
     return check_launch(name);
   };
   return gate_first ? go(swiglu_ffn_bwd_hidden_kernel<D, true>) : go(swiglu_ffn_bwd_hidden_kernel<D, false>);

@@ -10,19 +10,19 @@ namespace {
 // dx = dres + rstd * (g - x_hat * mean(g * x_hat)),  g = (dy W) * norm_w,  x_hat = x * rstd.
 //
 // The product is the narrow output of a long contraction (K = 2F or 3D, D features): a workgroup takes 64 * TG tokens x all
-// features, so dy is read once and complete rows meet in the workgroup; 2 * TG wavefronts, TG token groups of 64 x 2 feature
-// halves. K is walked in slabs of 32: both operands' slabs go from global memory straight into LDS (16 rows x 64 bytes per
-// transfer) into a ring of four stages, three slabs ahead; the four 16-byte pieces of a row are XOR-swizzled by (row / 4) % 4, so
-// that the 16 lanes of a fragment read hit distinct banks. Rows beyond the count repeat the last row and are not stored.
+// features, so dy is read once and complete rows meet in the workgroup; TG token groups of 64 x FG feature groups, a wavefront
+// each. K is walked in slabs: both operands' slabs go from global memory straight into LDS (1 KB per transfer) into a ring of
+// stages, RING - 1 slabs ahead; the 16-byte pieces of a row are XOR-swizzled by its number, so that the 16 lanes of a fragment
+// read hit distinct banks. Rows beyond the count repeat the last row and are not stored.
 // The epilogue replaces a store of dh = dy W, the norm's backward over x and dh, and the residual add: 3 of the 8 passes over
 // [M, D] that the layer-by-layer backward makes here. The gradient of the norm's weight is left to the weight-gradient kernels,
 // which hold sum_m dy[m, n] x_hat[m, k] anyway (d norm_w[k] = sum_n w[n, k] of it).
 // The epilogue's rows pass through LDS: read and written as a lane's own eight bytes of 32 rows at once, they cost 46 us per
 // 256-token workgroup whatever K (294 912 tokens, D = 256: K = 768 337 -> 220 us, K = 2048 515 -> 400 us).
-// Bound: HBM (dy, K * 2 bytes per token); 64-token workgroups (TG = 1) where 256-token ones would leave compute units idle.
+// Bound: HBM (dy, K * 2 bytes per token). Where 256-token workgroups would leave compute units idle a workgroup takes 64 tokens,
+// and a slab's chain (barrier, fragment reads, products, transfers) is the time: eight wavefronts and slabs of 64 columns instead
+// of two and 32, 6 100 tokens, D = 256: K = 2048 43 -> 24 us.
 // ------------------------------------------------------------------------------------------------------------------
-constexpr int kSlab = 32;
-constexpr int kRing = 4;
 
 struct DgradParams {
   const bf16_t* dy;
@@ -38,15 +38,20 @@ struct DgradParams {
   bool panels;           // dy in panel order
 };
 
-template <int D, int TG>
-__global__ __launch_bounds__(TG * 2 * kWave, 2) void dgrad_norm_kernel(const DgradParams p) {
-  constexpr int NWAVES = 2 * TG;
+// TG: token groups of 64; FG: feature groups (wavefronts = TG * FG); SLAB: columns of dy per stage, RING stages.
+template <int D, int TG, int FG, int SLAB, int RING>
+__global__ __launch_bounds__(TG * FG * kWave, 2) void dgrad_norm_kernel(const DgradParams p) {
+  constexpr int NWAVES = TG * FG;
   constexpr int TOK = 64 * TG;
-  constexpr int NI = D / 64;                    // 32-feature blocks per wavefront
-  constexpr int kTokBytes = TOK * kSlab * 2, kStage = kTokBytes + D * kSlab * 2;
-  constexpr int WT = D / 16 / NWAVES;           // weight transfers per wavefront and slab
-  constexpr int PW = 2 + WT;                    // all transfers: TOK / 16 = 2 * NWAVES token rows' worth
-  static_assert(D % (16 * NWAVES) == 0, "every wavefront stages the same number of pieces");
+  constexpr int NI = D / FG / 32;               // 32-feature blocks per wavefront
+  constexpr int kRowB = SLAB * 2;               // bytes of a staged row
+  constexpr int kTokBytes = TOK * kRowB, kStage = kTokBytes + D * kRowB;
+  constexpr int LPR = SLAB / 8, RPX = kWave / LPR;  // lanes per row and rows per transfer
+  constexpr int AT = TOK / RPX / NWAVES, WT = D / RPX / NWAVES;  // transfers per wavefront and slab: rows of dy, of the weight
+  constexpr int PW = AT + WT;
+  static_assert(TOK % (RPX * NWAVES) == 0 && D % (RPX * NWAVES) == 0, "every wavefront stages the same number of pieces");
+  static_assert((SLAB == 32 || SLAB == 64) && SLAB % kPanelCols == 0 && kPanelRows % TOK == 0, "a slab of a workgroup lies in whole panel rows");
+  static_assert(RING == 3 || RING == 4, "waits are written for these");
   extern __shared__ __attribute__((aligned(1024))) uint8_t smem[];
 
   int64_t rows = p.M;
@@ -61,43 +66,44 @@ __global__ __launch_bounds__(TG * 2 * kWave, 2) void dgrad_norm_kernel(const Dgr
   const int lane = tid % kWave;
   const int l32 = lane % 32, hh = lane / 32;
   const int wt = wave % TG, wn = wave / TG;
-  const int nslabs = p.K / kSlab;
+  const int nslabs = p.K / SLAB;
 
-  const bf16_t* a_src[2];
+  // piece order of a staged row: the 16 rows that a fragment read touches together fall on distinct banks
+  auto swizzle = [](int row) { return SLAB == 32 ? (row >> 2) & 3 : (row >> 1) & 7; };
+  const bf16_t* a_src[AT];
   const bf16_t* w_src[WT];
 #pragma unroll
-  for (int i = 0; i < 2; ++i) {
-    const int row = 16 * (2 * wave + i) + lane / 4;
+  for (int i = 0; i < AT; ++i) {
+    const int row = RPX * (AT * wave + i) + lane / LPR, piece = (lane % LPR) ^ swizzle(row);
     const int64_t arow = m0 + row < rows ? m0 + row : rows - 1;
-    a_src[i] = p.dy + (p.panels ? panel_row(arow, p.K) : arow * p.K) + ((lane % 4) ^ ((row >> 2) & 3)) * 8;
+    a_src[i] = p.dy + (p.panels ? panel_row(arow, p.K) + piece / 4 * kPanel + piece % 4 * 8 : arow * p.K + piece * 8);
   }
 #pragma unroll
   for (int i = 0; i < WT; ++i) {
-    const int row = 16 * (WT * wave + i) + lane / 4;
-    w_src[i] = p.w_t + static_cast<int64_t>(row) * p.K + ((lane % 4) ^ ((row >> 2) & 3)) * 8;
+    const int row = RPX * (WT * wave + i) + lane / LPR;
+    w_src[i] = p.w_t + static_cast<int64_t>(row) * p.K + ((lane % LPR) ^ swizzle(row)) * 8;
   }
   // every workgroup starts its walk over K at a different slab: with all of them on the same columns of a matrix whose row pitch
   // is a power of two their requests crowd the same memory channels
   const int rot = static_cast<int>((blockIdx.x * 5u) % static_cast<uint32_t>(nslabs));
-  static_assert(kSlab == kPanelCols && kPanelRows % TOK == 0, "a slab of a workgroup lies in one panel");
-  const int64_t slab_stride = p.panels ? kPanel : kSlab;
+  const int64_t slab_stride = p.panels ? SLAB / kPanelCols * kPanel : SLAB;
   auto stage = [&](int slab) {
-    uint8_t* base = smem + (slab % kRing) * kStage;
+    uint8_t* base = smem + (slab % RING) * kStage;
     const int turned = slab + rot;
     const int at = turned >= nslabs ? turned - nslabs : turned;
     const int64_t a0 = at * slab_stride;
-    const int k0 = at * kSlab;
+    const int k0 = at * SLAB;
 #pragma unroll
-    for (int i = 0; i < 2; ++i) lds_dma16(a_src[i] + a0, base + (2 * wave + i) * 1024);
+    for (int i = 0; i < AT; ++i) lds_dma16(a_src[i] + a0, base + (AT * wave + i) * 1024);
 #pragma unroll
     for (int i = 0; i < WT; ++i) lds_dma16(w_src[i] + k0, base + kTokBytes + (WT * wave + i) * 1024);
   };
-  const int swz = (l32 >> 2) & 3;
-  int piece_off[2];
+  const int swz = swizzle(l32);  // of any row l32 + a multiple of 32
+  int piece_off[SLAB / 16];
 #pragma unroll
-  for (int ks = 0; ks < 2; ++ks) piece_off[ks] = ((2 * ks + hh) ^ swz) * 16;
-  const int a_row_off = (wt * 64 + l32) * (kSlab * 2);
-  const int w_row_off = kTokBytes + (wn * (D / 2) + l32) * (kSlab * 2);
+  for (int ks = 0; ks < SLAB / 16; ++ks) piece_off[ks] = ((2 * ks + hh) ^ swz) * 16;
+  const int a_row_off = (wt * 64 + l32) * kRowB;
+  const int w_row_off = kTokBytes + (wn * (D / FG) + l32) * kRowB;
 
   f32x16 acc[NI][2];
 #pragma unroll
@@ -108,37 +114,37 @@ __global__ __launch_bounds__(TG * 2 * kWave, 2) void dgrad_norm_kernel(const Dgr
       for (int j = 0; j < 16; ++j) acc[ni][mi][j] = 0.f;
 
 #pragma unroll
-  for (int q = 0; q < kRing - 1; ++q)
+  for (int q = 0; q < RING - 1; ++q)
     if (q < nslabs) stage(q);
-  if (nslabs > 2) vm_wait<2 * PW>();
+  if (RING == 4 && nslabs > 2) vm_wait<2 * PW>();
   else if (nslabs > 1) vm_wait<PW>();
   else vm_wait<0>();
   __syncthreads();
   for (int s = 0; s < nslabs; ++s) {
-    if (s + kRing - 1 < nslabs) stage(s + kRing - 1);  // the slot last read in slab s - 1, which every wavefront has left
-    const uint8_t* st = smem + (s % kRing) * kStage;
+    if (s + RING - 1 < nslabs) stage(s + RING - 1);  // the slot last read in slab s - 1, which every wavefront has left
+    const uint8_t* st = smem + (s % RING) * kStage;
 #pragma unroll
-    for (int ks = 0; ks < kSlab / 16; ++ks) {
+    for (int ks = 0; ks < SLAB / 16; ++ks) {
       bf16x8 wf[NI], af[2];
 #pragma unroll
-      for (int mi = 0; mi < 2; ++mi) af[mi] = *reinterpret_cast<const bf16x8*>(st + a_row_off + mi * 32 * (kSlab * 2) + piece_off[ks]);
+      for (int mi = 0; mi < 2; ++mi) af[mi] = *reinterpret_cast<const bf16x8*>(st + a_row_off + mi * 32 * kRowB + piece_off[ks]);
 #pragma unroll
-      for (int ni = 0; ni < NI; ++ni) wf[ni] = *reinterpret_cast<const bf16x8*>(st + w_row_off + ni * 32 * (kSlab * 2) + piece_off[ks]);
+      for (int ni = 0; ni < NI; ++ni) wf[ni] = *reinterpret_cast<const bf16x8*>(st + w_row_off + ni * 32 * kRowB + piece_off[ks]);
 #pragma unroll
       for (int ni = 0; ni < NI; ++ni)
 #pragma unroll
         for (int mi = 0; mi < 2; ++mi) acc[ni][mi] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(wf[ni], af[mi], acc[ni][mi], 0, 0, 0);
     }
     if (s + 1 < nslabs) {
-      // the transfers of slab s + 1 were issued three slabs ago; behind them are those of slabs s + 2 and s + 3
-      if (s + 3 < nslabs) vm_wait<2 * PW>();
+      // the transfers of slab s + 1 were issued RING - 1 slabs ago; behind them are those of slab s + 2 (and s + 3)
+      if (RING == 4 && s + 3 < nslabs) vm_wait<2 * PW>();
       else if (s + 2 < nslabs) vm_wait<PW>();
       else vm_wait<0>();
     }
     __syncthreads();
   }
 
-  // acc[ni][mi][jq * 4 + e]: feature wn * D / 2 + ni * 32 + jq * 8 + hh * 4 + e of token wt * 64 + mi * 32 + l32.
+  // acc[ni][mi][jq * 4 + e]: feature wn * D / FG + ni * 32 + jq * 8 + hh * 4 + e of token wt * 64 + mi * 32 + l32.
   // A lane holds eight bytes out of each 32 features of one row, so x, dres and dx pass through LDS, 32 * TG tokens (one mi) at a
   // time over the ring's memory: whole rows in and out of memory, the 16-byte pieces of a tile row XOR-swizzled by row % 16.
   constexpr int TILE_ROWS = 32 * TG, kRowBytes = D * 2, kTile = TILE_ROWS * kRowBytes;
@@ -147,10 +153,10 @@ __global__ __launch_bounds__(TG * 2 * kWave, 2) void dgrad_norm_kernel(const Dgr
   constexpr int PIECES = D / 8;
   uint8_t* x_tile = smem;
   uint8_t* res_tile = smem + kTile;
-  float* red = reinterpret_cast<float*>(smem + 2 * kTile);  // [2 feature halves][TILE_ROWS] sums of g * x
+  float* red = reinterpret_cast<float*>(smem + 2 * kTile);  // [FG][TILE_ROWS] sums of g * x
   const int trow = wt * 32 + l32;
   auto token_of = [&](int tile_row, int mi) { return m0 + tile_row / 32 * 64 + mi * 32 + tile_row % 32; };
-  auto lane_piece = [&](int ni, int jq) { return trow * kRowBytes + (((wn * (D / 16) + ni * 4 + jq) ^ (trow & 15)) * 16) + hh * 8; };
+  auto lane_piece = [&](int ni, int jq) { return trow * kRowBytes + (((wn * (D / FG / 8) + ni * 4 + jq) ^ (trow & 15)) * 16) + hh * 8; };
 #pragma unroll
   for (int mi = 0; mi < 2; ++mi) {
     if (mi > 0) __syncthreads();  // the tiles have been stored
@@ -172,7 +178,7 @@ __global__ __launch_bounds__(TG * 2 * kWave, 2) void dgrad_norm_kernel(const Dgr
 #pragma unroll
       for (int jq = 0; jq < 4; ++jq) {
         const bf16x4 xv = *reinterpret_cast<const bf16x4*>(x_tile + lane_piece(ni, jq));
-        const bf16x4 wv = *reinterpret_cast<const bf16x4*>(p.norm_w + wn * (D / 2) + ni * 32 + jq * 8 + hh * 4);
+        const bf16x4 wv = *reinterpret_cast<const bf16x4*>(p.norm_w + wn * (D / FG) + ni * 32 + jq * 8 + hh * 4);
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
           const float g = acc[ni][mi][jq * 4 + e] * static_cast<float>(wv[e]);
@@ -186,7 +192,10 @@ __global__ __launch_bounds__(TG * 2 * kWave, 2) void dgrad_norm_kernel(const Dgr
     if (hh == 0) red[wn * TILE_ROWS + trow] = both;
     __syncthreads();
     // mean(g * x_hat) * x_hat = (sum of g * x) / D * rstd^2 * x
-    const float proj = (red[trow] + red[TILE_ROWS + trow]) * (1.0f / D) * scale * scale;
+    float sum = red[trow];
+#pragma unroll
+    for (int f = 1; f < FG; ++f) sum += red[f * TILE_ROWS + trow];
+    const float proj = sum * (1.0f / D) * scale * scale;
 #pragma unroll
     for (int ni = 0; ni < NI; ++ni)
 #pragma unroll
@@ -212,17 +221,18 @@ __global__ __launch_bounds__(TG * 2 * kWave, 2) void dgrad_norm_kernel(const Dgr
   }
 }
 
-template <int D, int TG>
+template <int D, int TG, int FG, int SLAB, int RING>
 int launch_dgrad(const DgradParams& p, hipStream_t s, const char* name) {
-  constexpr size_t ring = static_cast<size_t>(kRing) * (64 * TG + D) * kSlab * 2;
-  constexpr size_t tiles = 2 * static_cast<size_t>(32 * TG) * (D * 2 + sizeof(float));
+  constexpr size_t ring = static_cast<size_t>(RING) * (64 * TG + D) * SLAB * 2;
+  constexpr size_t tiles = static_cast<size_t>(32 * TG) * (2 * D * 2 + FG * sizeof(float));
   constexpr size_t lds = ring > tiles ? ring : tiles;
-  if (hipFuncSetAttribute(reinterpret_cast<const void*>(dgrad_norm_kernel<D, TG>), hipFuncAttributeMaxDynamicSharedMemorySize,
-                          static_cast<int>(lds)) != hipSuccess)
+  auto kernel = dgrad_norm_kernel<D, TG, FG, SLAB, RING>;
+  if (hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds)) !=
+      hipSuccess)
     return set_error(TAAC_ERR_LAUNCH, "%s: cannot reserve %zu bytes of LDS", name, lds);
   const int64_t grid = (p.M + 64 * TG - 1) / (64 * TG);
   if (grid > 0x7fffffffLL) return set_error(TAAC_ERR_UNSUPPORTED, "%s: too many workgroups", name);
-  hipLaunchKernelGGL((dgrad_norm_kernel<D, TG>), dim3(static_cast<uint32_t>(grid)), dim3(TG * 2 * kWave), lds, s, p);
+  hipLaunchKernelGGL(kernel, dim3(static_cast<uint32_t>(grid)), dim3(TG * FG * kWave), lds, s, p);
   return check_launch(name);
 }
 
@@ -236,6 +246,7 @@ int launch_dgrad(const DgradParams& p, hipStream_t s, const char* name) {
 // Bound: HBM - the operands are read once per 256 features of the other side.
 // ------------------------------------------------------------------------------------------------------------------
 constexpr int kChunk = 64;
+constexpr int kXcds = 8;
 
 struct WgradParams {
   WgradItem item[kWgradItems];
@@ -252,13 +263,17 @@ template <int TN, int TK, int WN, int WK>
 __global__ __launch_bounds__(WN * WK * kWave, 2) void wgrad_block_kernel(const WgradParams p) {
   constexpr int THREADS = WN * WK * kWave;
   constexpr int BN = TN / WN / 32, BK = TK / WK / 32;   // 32 x 32 blocks of a wavefront
-  constexpr int ROWN = TN * 2 + 32, ROWK = TK * 2 + 32;  // LDS row bytes
+  constexpr int ROWN = TN * 2 + 64, ROWK = TK * 2 + 64;  // LDS row bytes
   constexpr int SLABN = kChunk * ROWN, SLABK = kChunk * ROWK;
   constexpr int PN = kChunk * (TN / 8) / THREADS, PK = kChunk * (TK / 8) / THREADS;  // 16-byte pieces per thread and chunk
   constexpr int RN = THREADS / (TN / 8), RK = THREADS / (TK / 8);                    // rows between a thread's pieces
   extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
 
-  const int tile = static_cast<int>(blockIdx.x), split = static_cast<int>(blockIdx.y);
+  // Workgroups are handed to the eight XCDs in turn; the tiles of a split, which read the same rows, go to one XCD and meet in its L2.
+  const int tiles = p.first_tile[p.n_items];
+  const int n_wg = static_cast<int>(gridDim.x), xcd = static_cast<int>(blockIdx.x) % kXcds, slot = static_cast<int>(blockIdx.x) / kXcds;
+  const int unit = xcd * (n_wg / kXcds) + (xcd < n_wg % kXcds ? xcd : n_wg % kXcds) + slot;
+  const int tile = unit % tiles, split = unit / tiles;
   int which = 0;
 #pragma unroll
   for (int i = 1; i < kWgradItems; ++i)
@@ -450,10 +465,14 @@ __global__ __launch_bounds__(kReduceThreads) void wgrad_reduce_kernel(const Redu
     if (!ok || row >= N) continue;
     const int64_t at = static_cast<int64_t>(row) * K + col;
     f32x4 s = {0.f, 0.f, 0.f, 0.f};
-    for (int k = 0; k < p.splits; ++k) {
-      const f32x4 v = *reinterpret_cast<const f32x4*>(src + k * nk + at);
+    for (int k = 0; k < p.splits; k += 8) {  // eight partials requested at once, added in order
+      f32x4 v[8];
 #pragma unroll
-      for (int e = 0; e < 4; ++e) s[e] += v[e];
+      for (int j = 0; j < 8; ++j) v[j] = *reinterpret_cast<const f32x4*>(src + (k + j < p.splits ? k + j : k) * nk + at);
+#pragma unroll
+      for (int j = 0; j < 8; ++j)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) s[e] += k + j < p.splits ? v[j][e] : 0.f;
     }
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
@@ -547,8 +566,13 @@ int dgrad_norm(const char* name, const void* dy, bool dy_panels, int32_t K, cons
   p.panels = dy_panels;
   const int cus = compute_units();
   const bool small = M < 128 * static_cast<int64_t>(cus);
-  if (D == 256) return small ? launch_dgrad<256, 1>(p, s, name) : launch_dgrad<256, 4>(p, s, name);
-  return small ? launch_dgrad<128, 1>(p, s, name) : launch_dgrad<128, 4>(p, s, name);
+  // Two 128-token workgroups share a compute unit, so that one's epilogue runs beside the other's products: worth the second pass
+  // over the weights where the contraction is short, and where 256-token workgroups would be less than two rounds (294 912
+  // tokens, D = 256, 128- / 256-token workgroups: K = 768 207 / 222 us, K = 2048 420 / 400; 51 584 rows: 347 / 430 us over both).
+  if (small) return D == 256 ? launch_dgrad<256, 1, 8, 64, 3>(p, s, name) : launch_dgrad<128, 1, 4, 64, 3>(p, s, name);
+  if (D == 128) return launch_dgrad<128, 4, 2, 32, 4>(p, s, name);
+  if (K <= 1024 || M < 512 * static_cast<int64_t>(cus)) return launch_dgrad<256, 2, 2, 32, 3>(p, s, name);
+  return launch_dgrad<256, 4, 2, 32, 4>(p, s, name);
 }
 
 int64_t wgrad_scratch_floats(int64_t M, const int32_t (*shapes)[2], int items) {
@@ -605,7 +629,7 @@ int wgrad_block(const char* name, const WgradItem* items, int n_items, int64_t M
   p.n_items = q.n_items = n_items;
   q.partial = scratch;
   q.norm_partial = vectors;
-  const dim3 grid(tiles, pl.splits);
+  const dim3 grid(tiles * pl.splits);
   auto go = [&](auto kernel, int threads, size_t lds) -> int {
     if (hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds)) !=
         hipSuccess)
@@ -613,7 +637,7 @@ int wgrad_block(const char* name, const WgradItem* items, int n_items, int64_t M
     hipLaunchKernelGGL(kernel, grid, dim3(threads), lds, s, p);
     return check_launch(name);
   };
-  const size_t lds = 2 * 2 * static_cast<size_t>(kChunk) * (pl.tn * 2 + 32);
+  const size_t lds = 2 * 2 * static_cast<size_t>(kChunk) * (pl.tn * 2 + 64);
   const int rc = pl.tn == 256 ? go(wgrad_block_kernel<256, 256, 2, 4>, 512, lds) : go(wgrad_block_kernel<128, 128, 2, 2>, 256, lds);
   if (rc != TAAC_OK) return rc;
   if (dtype == TAAC_F32)
