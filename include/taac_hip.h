@@ -842,6 +842,16 @@ int taac_embedding_bag_mean_bwd(const void* values, int index_is_int64, int64_t 
                                 void* workspace, int dtype, void* stream);
 
 /*
+ * The same gradient with a workspace whose size the library names (for every dtype, fp32 included): the call may then sort the
+ * slots by the row they name instead of adding them up in memory. taac_embedding_bag_mean_bwd_bytes: the bytes needed, possibly 0,
+ * or -1 for bad arguments. grad_out, grad_weight and the workspace 16-byte aligned.
+ */
+int64_t taac_embedding_bag_mean_bwd_bytes(int64_t num_embeddings, int32_t emb_dim, int64_t bags, int32_t bag_size, int dtype);
+int taac_embedding_bag_mean_bwd_sized(const void* values, int index_is_int64, int64_t bags, int32_t bag_size,
+                                      const void* grad_out, void* grad_weight, int64_t num_embeddings, int32_t emb_dim,
+                                      void* workspace, int64_t workspace_bytes, int dtype, void* stream);
+
+/*
  * Weights of one backbone block; every pointer is a device pointer to bf16 data in torch nn.Linear layout.
  * Field names follow the reference's parameter names (experiments/symbiosis/backbone.py:24-56).
  * Biases may be NULL (treated as zero). query_norm_weight / key_norm_weight are the attention layer's

@@ -258,6 +258,11 @@ SIGNATURES: dict[str, tuple[object, list[object]]] = {
         c_int,
         [c_void_p, c_int, c_int64, c_int32, c_void_p, c_void_p, c_int64, c_int32, c_void_p, c_int, c_void_p],
     ),
+    "taac_embedding_bag_mean_bwd_bytes": (c_int64, [c_int64, c_int32, c_int64, c_int32, c_int]),
+    "taac_embedding_bag_mean_bwd_sized": (
+        c_int,
+        [c_void_p, c_int, c_int64, c_int32, c_void_p, c_void_p, c_int64, c_int32, c_void_p, c_int64, c_int, c_void_p],
+    ),
     "taac_candidate_readout_fwd": (
         c_int,
         [c_void_p, c_void_p, c_void_p, c_int32, c_int32, c_int32, c_int32, c_int32, c_void_p, c_void_p, c_float,

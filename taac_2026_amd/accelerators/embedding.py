@@ -73,12 +73,14 @@ def hip_embedding_bag_mean_backward_kernel(values: torch.Tensor, grad_out: torch
     grad_out = grad_out.contiguous()
     emb_dim = grad_out.shape[1]
     grad_weight = torch.empty(num_embeddings, emb_dim, dtype=grad_out.dtype, device=grad_out.device)
-    workspace = None
-    if grad_out.dtype != torch.float32:
-        workspace = torch.empty(num_embeddings, emb_dim, dtype=torch.float32, device=grad_out.device)
-    status = library.taac_embedding_bag_mean_bwd(
+    if grad_out.data_ptr() % 16:
+        grad_out = grad_out.clone()
+    dtype = _native.dtype_code(grad_out.dtype)
+    needed = library.taac_embedding_bag_mean_bwd_bytes(num_embeddings, emb_dim, values.shape[0], values.shape[1], dtype)
+    workspace = torch.empty(max(needed, 0), dtype=torch.uint8, device=grad_out.device)
+    status = library.taac_embedding_bag_mean_bwd_sized(
         values.data_ptr(), int(values.dtype == torch.int64), values.shape[0], values.shape[1], grad_out.data_ptr(),
-        grad_weight.data_ptr(), num_embeddings, emb_dim, _native.ptr(workspace), _native.dtype_code(grad_out.dtype),
+        grad_weight.data_ptr(), num_embeddings, emb_dim, workspace.data_ptr(), max(needed, 0), dtype,
         _native.current_stream(grad_out.device),
     )
     _native.check(status, "embedding_bag_mean backward")

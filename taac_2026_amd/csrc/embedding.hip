@@ -6,6 +6,8 @@
 // table row is fetched as one contiguous run of 16-byte requests and the output row is written once. The ids of a bag
 // are read four at a time and the (up to four) rows they name are requested before any of them is accumulated, fp32
 // accumulation, one rounding.
+#include <type_traits>
+
 #include "common.h"
 
 namespace taac {
@@ -225,6 +227,302 @@ void launch_bag_bwd(const void* values, int64_t bags, int bag_size, const void* 
                      sums, n, e, lanes);
 }
 
+// ---- the same gradient without sums in memory -------------------------------------------------------------------------------
+// The kernels above add every slot's row to an fp32 copy of the table in memory: the copy is cleared, hit by one atomic per
+// slot and feature, and read again to be rounded (1 000 000 x 64 in fp16, 786 000 slots: 37 + 176 + 95 us). Here the slots are
+// sorted by the row they name - a count per row, a start per row, the slots placed - and a row's sum is formed in registers and
+// written once, rounded. The order within a row, and the order of the rows' segments, is whatever the atomics gave: no scan over
+// workgroups (1 000 000 x 64, the same slots: count 57, start 13, place 19, rows 48 us). Rows named more than kHot times are cut into chunks that workgroups of their own sum up; the row then adds those.
+// Bound: the table's gradient (written once) and the gathered rows of grad_out.
+constexpr int kHot = 64;        // longest row that one lane group sums by itself
+constexpr int kHotChunk = 256;  // entries of a chunk, at least
+constexpr int kHotParts = 64;   // chunks of a row, at most
+constexpr int kRowsPerThread = 8;
+constexpr int kLocalRows = 16384;  // largest table whose counts a workgroup keeps in LDS
+constexpr int kLocalThreads = 1024;
+
+struct BagEntry {
+  int32_t bag;
+  float inv;  // 1 / number of valid ids of the bag
+};
+struct HotChunk {
+  int32_t first, count, chunks;  // entries; chunks of the row (in its first chunk)
+};
+struct SortedBags {
+  int32_t* counts;   // [n]; of a hot row after the start kernel: -1 - its first chunk
+  int32_t* cursors;  // entries, chunks (behind counts: cleared with them)
+  int32_t* start;    // [n]
+  int32_t* rank;     // [slots]
+  BagEntry* entries; // [slots]
+  HotChunk* chunks;  // [slots / kHot]
+  float* partial;    // [slots / kHot][emb_dim]
+  int64_t bytes;
+};
+SortedBags sorted_layout(char* base, int64_t n, int64_t slots, int emb_dim) {
+  SortedBags b{};
+  char* at = base;
+  auto take = [&](int64_t bytes) {
+    char* here = at;
+    at += (bytes + 255) & ~static_cast<int64_t>(255);
+    return here;
+  };
+  b.counts = reinterpret_cast<int32_t*>(take((n + 2) * 4));
+  b.cursors = b.counts + n;
+  b.start = reinterpret_cast<int32_t*>(take(n * 4));
+  b.rank = reinterpret_cast<int32_t*>(take(slots * 4));
+  b.entries = reinterpret_cast<BagEntry*>(take(slots * static_cast<int64_t>(sizeof(BagEntry))));
+  b.chunks = reinterpret_cast<HotChunk*>(take(slots / kHot * static_cast<int64_t>(sizeof(HotChunk))));
+  b.partial = reinterpret_cast<float*>(take(slots / kHot * emb_dim * 4));
+  b.bytes = at - base;
+  return b;
+}
+
+__global__ __launch_bounds__(kBlock) void bag_clear_kernel(int32_t* __restrict__ counts, int64_t n) {
+  const int64_t i = (static_cast<int64_t>(blockIdx.x) * kBlock + threadIdx.x) * 4;
+#pragma unroll
+  for (int e = 0; e < 4; ++e)
+    if (i + e < n) counts[i + e] = 0;
+}
+
+template <typename I>
+__global__ __launch_bounds__(kBlock) void bag_count_kernel(const I* __restrict__ values, int64_t slots, int64_t n, SortedBags b) {
+  const int64_t i = static_cast<int64_t>(blockIdx.x) * kBlock + threadIdx.x;
+  if (i >= slots) return;
+  const int64_t id = static_cast<int64_t>(values[i]);
+  if (id > 0 && id < n) b.rank[i] = atomicAdd(b.counts + id, 1);
+}
+
+// The same for a small table, whose rows are named so often that the adds to one row would queue up in memory: a workgroup counts its
+// share of the slots in LDS and reserves each row's places with one add.
+template <typename I>
+__global__ __launch_bounds__(kLocalThreads) void bag_count_local_kernel(const I* __restrict__ values, int64_t slots, int32_t n,
+                                                                        SortedBags b) {
+  extern __shared__ int32_t local[];
+  const int64_t per = (slots + gridDim.x - 1) / gridDim.x, begin = per * blockIdx.x, end = begin + per < slots ? begin + per : slots;
+  for (int32_t r = threadIdx.x; r < n; r += kLocalThreads) local[r] = 0;
+  __syncthreads();
+  for (int64_t i = begin + threadIdx.x; i < end; i += kLocalThreads) {
+    const int64_t id = static_cast<int64_t>(values[i]);
+    if (id > 0 && id < n) b.rank[i] = atomicAdd(local + id, 1);
+  }
+  __syncthreads();
+  for (int32_t r = threadIdx.x; r < n; r += kLocalThreads) {
+    const int32_t c = local[r];
+    if (c > 0) local[r] = atomicAdd(b.counts + r, c);
+  }
+  __syncthreads();
+  for (int64_t i = begin + threadIdx.x; i < end; i += kLocalThreads) {
+    const int64_t id = static_cast<int64_t>(values[i]);
+    if (id > 0 && id < n) b.rank[i] += local[id];
+  }
+}
+
+// Starts of the rows' segments: a scan inside the workgroup, one add to the common cursor for all of its rows.
+__global__ __launch_bounds__(kBlock) void bag_start_kernel(int64_t n, SortedBags b) {
+  __shared__ int32_t wave_sum[kBlock / kWave];
+  __shared__ int32_t base;
+  const int64_t r0 = (static_cast<int64_t>(blockIdx.x) * kBlock + threadIdx.x) * kRowsPerThread;
+  const int lane = threadIdx.x % kWave, wave = threadIdx.x / kWave;
+  int32_t c[kRowsPerThread], mine = 0;
+#pragma unroll
+  for (int e = 0; e < kRowsPerThread; ++e) {
+    c[e] = r0 + e < n ? b.counts[r0 + e] : 0;
+    mine += c[e];
+  }
+  int32_t upto = mine;
+#pragma unroll
+  for (int d = 1; d < kWave; d *= 2) {
+    const int32_t v = __shfl_up(upto, d);
+    if (lane >= d) upto += v;
+  }
+  if (lane == kWave - 1) wave_sum[wave] = upto;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    int32_t total = 0;
+    for (int w = 0; w < kBlock / kWave; ++w) total += wave_sum[w];
+    base = total > 0 ? atomicAdd(b.cursors, total) : 0;
+  }
+  __syncthreads();
+  int32_t at = base + upto - mine;
+  for (int w = 0; w < wave; ++w) at += wave_sum[w];
+#pragma unroll
+  for (int e = 0; e < kRowsPerThread; ++e) {
+    if (r0 + e >= n) break;
+    b.start[r0 + e] = at;
+    if (c[e] > kHot) {
+      const int32_t by_parts = (c[e] + kHotParts - 1) / kHotParts, len = by_parts > kHotChunk ? by_parts : kHotChunk;
+      const int32_t chunks = (c[e] + len - 1) / len;  // at most c / kHot
+      const int32_t first = atomicAdd(b.cursors + 1, chunks);
+      for (int32_t k = 0; k < chunks; ++k)
+        b.chunks[first + k] = HotChunk{at + k * len, c[e] - k * len < len ? c[e] - k * len : len, chunks};
+      b.counts[r0 + e] = -1 - first;
+    }
+    at += c[e];
+  }
+}
+
+// One bag per `lanes` lanes (a power of two up to 64).
+template <typename I>
+__global__ __launch_bounds__(kBlock) void bag_place_kernel(const I* __restrict__ values, int64_t bags, int bag_size, int64_t n,
+                                                           int lanes, SortedBags b) {
+  const int lane = threadIdx.x % lanes;
+  const int64_t bag = static_cast<int64_t>(blockIdx.x) * (kBlock / lanes) + threadIdx.x / lanes;
+  if (bag >= bags) return;  // whole lane group
+  const I* ids = values + bag * bag_size;
+  int count = 0;
+  for (int j = lane; j < bag_size; j += lanes) {
+    const int64_t id = static_cast<int64_t>(ids[j]);
+    count += id > 0 && id < n ? 1 : 0;
+  }
+  for (int d = lanes / 2; d > 0; d /= 2) count += __shfl_xor(count, d);
+  const float inv = 1.0f / static_cast<float>(count > 0 ? count : 1);
+  for (int j = lane; j < bag_size; j += lanes) {
+    const int64_t id = static_cast<int64_t>(ids[j]);
+    if (id > 0 && id < n) b.entries[b.start[id] + b.rank[bag * bag_size + j]] = BagEntry{static_cast<int32_t>(bag), inv};
+  }
+}
+
+// Adds entries first, first + step, ... (below end) to acc, four in flight.
+template <typename T>
+__device__ __forceinline__ void add_entries(const BagEntry* entries, const T* __restrict__ grad, int emb_dim, bool live,
+                                            int32_t first, int32_t end, int32_t step, float (&acc)[Piece<T>::N]) {
+  typedef typename Piece<T>::vec vec_t;
+  constexpr int N = Piece<T>::N;
+  for (int32_t i = first; i < end; i += 4 * step) {
+    BagEntry e[4];
+    vec_t g[4];
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      const bool in = i + k * step < end;
+      e[k] = entries[in ? i + k * step : i];
+      if (!in) e[k].bag = -1;
+    }
+#pragma unroll
+    for (int k = 0; k < 4; ++k)
+      if (live && e[k].bag >= 0) g[k] = *reinterpret_cast<const vec_t*>(grad + static_cast<int64_t>(e[k].bag) * emb_dim);
+#pragma unroll
+    for (int k = 0; k < 4; ++k)
+      if (live && e[k].bag >= 0) {
+#pragma unroll
+        for (int c = 0; c < N; ++c) acc[c] = fmaf(static_cast<float>(g[k][c]), e[k].inv, acc[c]);
+      }
+  }
+}
+
+template <typename T, int G>
+__global__ __launch_bounds__(kBlock) void bag_hot_kernel(const T* __restrict__ grad_out, int emb_dim, SortedBags b) {
+  constexpr int N = Piece<T>::N, GROUPS = kBlock / G;
+  __shared__ float red[GROUPS][G * N];
+  const int lane = threadIdx.x % G, group = threadIdx.x / G;
+  const bool live = lane * N < emb_dim;
+  const int32_t n_chunks = b.cursors[1];
+  for (int32_t c = blockIdx.x; c < n_chunks; c += gridDim.x) {
+    const HotChunk chunk = b.chunks[c];
+    float acc[N];
+#pragma unroll
+    for (int e = 0; e < N; ++e) acc[e] = 0.f;
+    add_entries<T>(b.entries, grad_out + lane * N, emb_dim, live, chunk.first + group, chunk.first + chunk.count, GROUPS, acc);
+#pragma unroll
+    for (int e = 0; e < N; ++e) red[group][lane * N + e] = acc[e];
+    __syncthreads();
+    for (int col = threadIdx.x; col < emb_dim; col += kBlock) {
+      float s = 0.f;
+#pragma unroll
+      for (int g = 0; g < GROUPS; ++g) s += red[g][col];
+      b.partial[static_cast<int64_t>(c) * emb_dim + col] = s;
+    }
+    __syncthreads();
+  }
+}
+
+template <typename T, int G>
+__global__ __launch_bounds__(kBlock) void bag_rows_kernel(const T* __restrict__ grad_out, T* __restrict__ grad_weight, int64_t n,
+                                                          int emb_dim, SortedBags b) {
+  typedef typename Piece<T>::vec vec_t;
+  constexpr int N = Piece<T>::N;
+  const int lane = threadIdx.x % G;
+  const int64_t row = static_cast<int64_t>(blockIdx.x) * (kBlock / G) + threadIdx.x / G;
+  if (row >= n) return;
+  const bool live = lane * N < emb_dim;
+  const int32_t count = b.counts[row], start = b.start[row];
+  float acc[N];
+#pragma unroll
+  for (int e = 0; e < N; ++e) acc[e] = 0.f;
+  if (count >= 0) {
+    add_entries<T>(b.entries, grad_out + lane * N, emb_dim, live, start, start + count, 1, acc);
+  } else if (live) {
+    const int32_t first = -1 - count, chunks = b.chunks[first].chunks;
+#pragma unroll 4
+    for (int32_t k = 0; k < chunks; ++k) {
+      const float* part = b.partial + static_cast<int64_t>(first + k) * emb_dim + lane * N;
+#pragma unroll
+      for (int e = 0; e < N; ++e) acc[e] += part[e];
+    }
+  }
+  if (!live) return;
+  vec_t o;
+#pragma unroll
+  for (int e = 0; e < N; ++e) o[e] = static_cast<T>(acc[e]);
+  __builtin_nontemporal_store(o, reinterpret_cast<vec_t*>(grad_weight + row * emb_dim + lane * N));
+}
+
+// Whether the sorted form runs: rows of up to 64 whole pieces, 32-bit positions, and enough work that its six launches (against
+// three, or two for fp32) do not decide. Measured back to back, sums in memory / sorted, us, skewed ids, a quarter padding -
+// 16-bit: 1 000 000 x 64, 262 144 x 4 slots 316 / 146, 1 024 x 4 slots 154 / 42; 100 000 x 64, 1 024 x 4 24 / 19; 20 000 x 64,
+// 256 x 4 11.7 / 18.9; 30 000 x 128, 65 536 x 3 95 / 78; 50 000 x 32, 30 000 x 2 24 / 35; 1 000 x 32, 524 288 x 12 4 384 / 229 (3 053
+// with the counts in memory), 1 000 x 16, 65 536 x 4 354 / 48, 1 000 x 64, 4 096 x 4 19 / 33.
+// fp32, which the other form sums in place: 1 000 000 x 64, 262 144 x 4 219 / 184, 1 024 x 4 43 / 61; 2 000 000 x 64, 524 288 x 4 420 / 334.
+bool sorted_bags(int64_t n, int64_t slots, int emb_dim, int dtype) {
+  const int piece = dtype == TAAC_F32 ? 4 : 8;
+  if (emb_dim % piece != 0 || emb_dim / piece > kWave || slots <= 0 || n > 0x3fffffffLL || slots > 0x3fffffffLL) return false;
+  const int64_t enough = 1 << 22;
+  if (dtype == TAAC_F32) return slots * emb_dim >= enough && 2 * slots >= n;
+  return slots * emb_dim >= enough || n * emb_dim >= enough;
+}
+
+template <typename T, typename I>
+int launch_sorted(const I* values, int64_t bags, int bag_size, const T* grad_out, T* grad_weight, int64_t n, int emb_dim, char* workspace,
+                  hipStream_t s, const char* name) {
+  const int64_t slots = bags * bag_size;
+  const SortedBags b = sorted_layout(workspace, n, slots, emb_dim);
+  auto blocks = [](int64_t threads) { return dim3(static_cast<uint32_t>((threads + kBlock - 1) / kBlock)); };
+  hipLaunchKernelGGL(bag_clear_kernel, blocks((n + 2 + 3) / 4), dim3(kBlock), 0, s, b.counts, n + 2);
+  const int64_t share = std::max<int64_t>(4 * n, 4 * kLocalThreads);  // slots of a workgroup, so that its counts pay
+  if (n <= kLocalRows && slots >= 4 * share) {
+    auto kernel = bag_count_local_kernel<I>;
+    const size_t lds = static_cast<size_t>(n) * 4;
+    if (hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, kLocalRows * 4) != hipSuccess)
+      return set_error(TAAC_ERR_LAUNCH, "%s: cannot reserve %zu bytes of LDS", name, lds);
+    const uint32_t grid = static_cast<uint32_t>(std::min<int64_t>(slots / share, 512));
+    hipLaunchKernelGGL(kernel, dim3(grid), dim3(kLocalThreads), lds, s, values, slots, static_cast<int32_t>(n), b);
+  } else {
+    hipLaunchKernelGGL(bag_count_kernel<I>, blocks(slots), dim3(kBlock), 0, s, values, slots, n, b);
+  }
+  hipLaunchKernelGGL(bag_start_kernel, blocks((n + kRowsPerThread - 1) / kRowsPerThread), dim3(kBlock), 0, s, n, b);
+  int lanes = 1;
+  while (lanes < bag_size && lanes < kWave) lanes *= 2;
+  hipLaunchKernelGGL(bag_place_kernel<I>, blocks(bags * lanes), dim3(kBlock), 0, s, values, bags, bag_size, n, lanes, b);
+  int rc = check_launch(name);
+  if (rc != TAAC_OK) return rc;
+  auto go = [&](auto g_tag) {
+    constexpr int G = decltype(g_tag)::value;
+    const int64_t most = slots / kHot;  // chunks, at most
+    if (most > 0)
+      hipLaunchKernelGGL((bag_hot_kernel<T, G>), dim3(static_cast<uint32_t>(std::min<int64_t>(most, 2048))), dim3(kBlock), 0, s, grad_out,
+                         emb_dim, b);
+    hipLaunchKernelGGL((bag_rows_kernel<T, G>), blocks(n * G), dim3(kBlock), 0, s, grad_out, grad_weight, n, emb_dim, b);
+    return check_launch(name);
+  };
+  const int pieces = emb_dim / Piece<T>::N;
+  if (pieces <= 1) return go(std::integral_constant<int, 1>{});
+  if (pieces <= 2) return go(std::integral_constant<int, 2>{});
+  if (pieces <= 4) return go(std::integral_constant<int, 4>{});
+  if (pieces <= 8) return go(std::integral_constant<int, 8>{});
+  if (pieces <= 16) return go(std::integral_constant<int, 16>{});
+  if (pieces <= 32) return go(std::integral_constant<int, 32>{});
+  return go(std::integral_constant<int, 64>{});
+}
+
 }  // namespace
 }  // namespace taac
 
@@ -294,4 +592,44 @@ extern "C" int taac_embedding_bag_mean_bwd(const void* values, int index_is_int6
       hipLaunchKernelGGL((round_sums_kernel<f16_t>), dim3(blocks), dim3(kBlock), 0, s, sums, static_cast<f16_t*>(grad_weight), count);
   }
   return check_launch(name);
+}
+
+extern "C" int64_t taac_embedding_bag_mean_bwd_bytes(int64_t num_embeddings, int32_t emb_dim, int64_t bags, int32_t bag_size, int dtype) {
+  using namespace taac;
+  if (num_embeddings <= 0 || emb_dim <= 0 || bags < 0 || bag_size < 0 || (dtype != TAAC_F32 && dtype != TAAC_BF16 && dtype != TAAC_F16)) return -1;
+  const int64_t slots = bags * bag_size;
+  if (sorted_bags(num_embeddings, slots, emb_dim, dtype)) return sorted_layout(nullptr, num_embeddings, slots, emb_dim).bytes;
+  return dtype == TAAC_F32 ? 0 : num_embeddings * emb_dim * 4;
+}
+
+extern "C" int taac_embedding_bag_mean_bwd_sized(const void* values, int index_is_int64, int64_t bags, int32_t bag_size,
+                                                 const void* grad_out, void* grad_weight, int64_t num_embeddings, int32_t emb_dim,
+                                                 void* workspace, int64_t workspace_bytes, int dtype, void* stream) {
+  using namespace taac;
+  const char* name = "taac_embedding_bag_mean_bwd_sized";
+  const int64_t need = taac_embedding_bag_mean_bwd_bytes(num_embeddings, emb_dim, bags, bag_size, dtype);
+  if (need < 0) return set_error(TAAC_ERR_INVALID_VALUE, "%s: bad dimensions or dtype", name);
+  if (workspace_bytes < need || (need > 0 && !workspace))
+    return set_error(TAAC_ERR_INVALID_VALUE, "%s: the workspace must hold taac_embedding_bag_mean_bwd_bytes", name);
+  const int64_t slots = bags * bag_size;
+  if (!sorted_bags(num_embeddings, slots, emb_dim, dtype) || !aligned16(grad_out) || !aligned16(grad_weight)) {
+    if (dtype != TAAC_F32 && workspace_bytes < num_embeddings * emb_dim * 4)
+      return set_error(TAAC_ERR_UNSUPPORTED, "%s: grad_out and grad_weight must be 16-byte aligned", name);
+    return taac_embedding_bag_mean_bwd(values, index_is_int64, bags, bag_size, grad_out, grad_weight, num_embeddings, emb_dim, workspace,
+                                       dtype, stream);
+  }
+  if (!values || !grad_out || !grad_weight) return set_error(TAAC_ERR_INVALID_VALUE, "%s: null tensor pointer", name);
+  if ((reinterpret_cast<uintptr_t>(workspace) & 15) != 0)
+    return set_error(TAAC_ERR_INVALID_VALUE, "%s: the workspace must be 16-byte aligned", name);
+  hipStream_t s = as_stream(stream);
+  char* ws = static_cast<char*>(workspace);
+#define TAAC_BAG_SORTED(T)                                                                                                        \
+  (index_is_int64 ? launch_sorted<T, int64_t>(static_cast<const int64_t*>(values), bags, bag_size, static_cast<const T*>(grad_out), \
+                                              static_cast<T*>(grad_weight), num_embeddings, emb_dim, ws, s, name)                 \
+                  : launch_sorted<T, int32_t>(static_cast<const int32_t*>(values), bags, bag_size, static_cast<const T*>(grad_out), \
+                                              static_cast<T*>(grad_weight), num_embeddings, emb_dim, ws, s, name))
+  if (dtype == TAAC_F32) return TAAC_BAG_SORTED(float);
+  if (dtype == TAAC_BF16) return TAAC_BAG_SORTED(bf16_t);
+  return TAAC_BAG_SORTED(f16_t);
+#undef TAAC_BAG_SORTED
 }

@@ -173,3 +173,36 @@ def test_backward_skips_ids_outside_the_table_and_needs_no_gradient_when_frozen(
     assert empty.shape == (16, 16) and empty.abs().max().item() == 0.0
     weight = torch.randn(16, 16, generator=g).to(device)
     assert not embedding_bag_mean(weight, values.clamp(0, 15).to(device)).requires_grad
+
+
+@pytest.mark.parametrize("dtype,index_dtype,rows,dim,bags,bag_size", [
+    (torch.float16, torch.int64, 20_000, 256, 301, 5),        # more rows than slots; bags that are no power of two
+    (torch.bfloat16, torch.int32, 1_000, 32, 40_000, 4),      # counts in LDS, every row in several chunks
+    (torch.float16, torch.int64, 3, 512, 3_000, 5),           # the widest row (64 pieces), two rows hold everything
+    (torch.float32, torch.int64, 70_001, 20, 60_000, 4),      # five of eight lanes hold a piece
+    (torch.float32, torch.int32, 17_000, 4, 400_000, 3),      # one piece; counts in memory
+    (torch.bfloat16, torch.int64, 600_000, 8, 40, 70),        # bags of more than 64 slots
+])
+def test_backward_of_sorted_slots(device, dtype, index_dtype, rows, dim, bags, bag_size):
+    """The sorted form against float64: an element's error is at most (terms + 2) * 2^-24 of the sum of its terms' magnitudes
+    (float32 products and sums, 2^-24 each), and half a unit in the last place of the result."""
+    from taac_2026_amd.accelerators.embedding import hip_embedding_bag_mean_backward_kernel
+
+    g = torch.Generator().manual_seed(rows + dim)
+    values = (torch.rand(bags, bag_size, generator=g) ** 2 * rows).long().clamp_(max=rows - 1)
+    values[torch.rand(bags, bag_size, generator=g) < 0.25] = 0
+    values[0] = 0
+    values[1, 0], values[2, 0] = -5, rows                     # outside the table: skipped
+    grad_out = torch.randn(bags, dim, generator=g).to(dtype)
+    got = hip_embedding_bag_mean_backward_kernel(values.to(index_dtype).to(device), grad_out.to(device), rows).cpu().double()
+    valid = (values > 0) & (values < rows)
+    scaled = grad_out.double() / valid.sum(1).clamp_min(1)[:, None]
+    bag_of, slot_of = valid.nonzero(as_tuple=True)
+    ids = values[bag_of, slot_of]
+    want = torch.zeros(rows, dim, dtype=torch.float64).index_add_(0, ids, scaled[bag_of])
+    size = torch.zeros(rows, dim, dtype=torch.float64).index_add_(0, ids, scaled[bag_of].abs())
+    terms = torch.zeros(rows, dtype=torch.float64).index_add_(0, ids, torch.ones_like(ids, dtype=torch.float64))
+    half_ulp = {torch.float16: 2.0 ** -11, torch.bfloat16: 2.0 ** -8, torch.float32: 2.0 ** -24}[dtype]   # 11, 8, 24 significant bits
+    tiny = 2.0 ** -25 if dtype == torch.float16 else 0.0      # half the spacing of float16's subnormal numbers
+    bound = (terms + 2)[:, None] * 2.0 ** -24 * size
+    assert ((got - want).abs() <= bound + half_ulp * (want.abs() + bound) + tiny).all()
