@@ -253,6 +253,17 @@ int taac_mask_pack_bits(const void* mask, int64_t rows, int32_t cols, uint32_t* 
 int taac_mask_block_any(const uint32_t* struct_bits, int32_t Tq, int32_t Tk, uint8_t* block_any, void* stream);
 
 /*
+ * Every form of a role mask in one launch: structural[q, k] = the role of query q sees the role of key k, or q == k (bytes, bits
+ * and block_any as taac_mask_pack_bits / taac_mask_block_any give them), key_valid[b, k] = key k of sample b is not padded, with
+ * key 0 valid where all are (bytes and bits). roles: int32 or int64 [T]; visible: host memory, per query role 0..7 bit r = keys of
+ * role r, bit 31 = every key; a query of another role sees only itself. padding: bytes [B, T], nonzero = padded.
+ * Replaces: the mask's tensor expressions (experiments/symbiosis/attention.py:21-60).
+ */
+int taac_role_mask(const void* roles, int roles_int64, const uint32_t visible[8], const uint8_t* padding, int32_t B, int32_t T,
+                   uint8_t* structural, uint32_t* struct_bits, uint8_t* block_any, uint8_t* key_valid, uint32_t* valid_bits,
+                   void* stream);
+
+/*
  * Training pair of taac_flash_attn_fwd (key-length mask, optional causal triangle; head_dim <= 64 for the backward).
  * taac_flash_attn_train_fwd additionally writes lse: fp32 [B, H, Tq] contiguous, the natural-log sum of exp of the
  * scaled scores of every query row (-inf for rows without a visible key and for padded rows).

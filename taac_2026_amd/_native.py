@@ -114,6 +114,10 @@ SIGNATURES: dict[str, tuple[object, list[object]]] = {
     ),
     "taac_mask_compact": (c_int, [c_void_p, c_int32, c_int32, c_int32, c_int64, c_void_p, c_void_p, c_void_p, c_void_p]),
     "taac_mask_pack_bits": (c_int, [c_void_p, c_int64, c_int32, c_void_p, c_void_p]),
+    "taac_role_mask": (
+        c_int,
+        [c_void_p, c_int, c_void_p, c_void_p, c_int32, c_int32, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p],
+    ),
     "taac_mask_block_any": (c_int, [c_void_p, c_int32, c_int32, c_void_p, c_void_p]),
     "taac_flash_attn_train_fwd": (
         c_int,

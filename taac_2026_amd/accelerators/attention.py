@@ -139,6 +139,30 @@ def build_structured_mask(
     )
 
 
+def build_role_mask(role_ids: torch.Tensor, visible: ctypes.Array, padding_mask: torch.Tensor) -> StructuredAttentionMask:
+    """``structural[q, k]`` = the role of query q sees that of key k (``visible``: eight words, one per query role, bit r = keys
+    of role r, bit 31 = every key) or q == k; the valid keys are those ``padding_mask`` (B, T) leaves, position 0 where it leaves
+    none. One launch for every form of the mask. ``role_ids``: int32 / int64 (T,)."""
+    name = "hip build_role_mask"
+    require_cuda_tensors(name, role_ids, padding_mask)
+    batch, tokens = padding_mask.shape
+    if role_ids.shape != (tokens,) or role_ids.dtype not in (torch.int32, torch.int64) or padding_mask.dtype is not torch.bool:
+        raise ValueError(f"{name}: role_ids must be int32 or int64 (tokens,), padding_mask bool (batch, tokens)")
+    role_ids, padding = role_ids.contiguous(), padding_mask.contiguous()
+    device, words = padding.device, (tokens + 31) // 32
+    structural = torch.empty(tokens, tokens, dtype=torch.bool, device=device)
+    struct_bits = torch.empty(tokens, words, dtype=torch.int32, device=device)
+    block_any = torch.empty((tokens + 127) // 128, (tokens + 63) // 64, dtype=torch.uint8, device=device)
+    key_valid = torch.empty(batch, tokens, dtype=torch.bool, device=device)
+    valid_bits = torch.empty(batch, words, dtype=torch.int32, device=device)
+    status = _native.load_library().taac_role_mask(
+        role_ids.data_ptr(), int(role_ids.dtype == torch.int64), visible, padding.data_ptr(), batch, tokens,
+        structural.data_ptr(), struct_bits.data_ptr(), block_any.data_ptr(), key_valid.data_ptr(), valid_bits.data_ptr(),
+        _native.current_stream(device))
+    _native.check(status, "role_mask")
+    return StructuredAttentionMask(struct_bits, block_any, valid_bits, None, structural, key_valid, None, 0, padding_mask)
+
+
 def plan_structured_attention_mask(q: torch.Tensor, k: torch.Tensor, attn_mask: torch.Tensor) -> StructuredAttentionMask:
     """Factor a (B, H | 1, Tq, Tk) bool mask into ``structural[i, j] & key_valid[b, j]`` with optional self-only query
     rows, verifying the factorisation exactly; ``RuntimeError`` when the mask has no such form. This reads the full mask

@@ -1459,6 +1459,75 @@ __global__ __launch_bounds__(kWave) void block_any_kernel(const uint32_t* __rest
   if (threadIdx.x == 0) block_any[blockIdx.x] = any ? 1 : 0;
 }
 
+// All forms of a role mask in one launch. Workgroups below nqc * nkc take a 128-query x 64-key block of the structure, one 32-key word
+// per thread; the ones behind them a sample's padding per wavefront. (As elementwise tensor expressions with the three packing
+// launches behind them: some 50 launches of 2 us and a 0.1 ms hole in front of the first block.)
+struct RoleMaskParams {
+  const void* roles;
+  bool roles_int64;
+  uint32_t visible[8];      // per query role: bit r = sees keys of role r, bit 31 = sees every key
+  const uint8_t* padding;   // [B, T]
+  int32_t B, T, nqc, nkc, wpr;
+  uint8_t* structural;      // [T, T]
+  uint32_t* struct_bits;    // [T, wpr]
+  uint8_t* block_any;       // [nqc, nkc]
+  uint8_t* key_valid;       // [B, T]
+  uint32_t* valid_bits;     // [B, wpr]
+};
+constexpr int kMaskThreads = 256;
+static_assert(2 * kQB == kMaskThreads && kKC == 64, "one word of a block per thread");
+__global__ __launch_bounds__(kMaskThreads) void role_mask_kernel(const RoleMaskParams p) {
+  const int tid = threadIdx.x, T = p.T;
+  const int blocks = p.nqc * p.nkc;
+  auto role = [&](int t) -> uint32_t {  // 8: none of the eight
+    const int64_t r = p.roles_int64 ? static_cast<const int64_t*>(p.roles)[t] : static_cast<const int32_t*>(p.roles)[t];
+    return r >= 0 && r < 8 ? static_cast<uint32_t>(r) : 8u;
+  };
+  if (static_cast<int>(blockIdx.x) < blocks) {
+    __shared__ uint8_t key_roles[kKC];
+    const int qc = blockIdx.x / p.nkc, kc = blockIdx.x % p.nkc;
+    if (tid < kKC) key_roles[tid] = kc * kKC + tid < T ? static_cast<uint8_t>(role(kc * kKC + tid)) : 255;
+    __syncthreads();
+    const int q = qc * kQB + tid / 2, w = 2 * kc + tid % 2;
+    uint32_t word = 0u;
+    if (q < T && w < p.wpr) {
+      const uint32_t r = role(q);
+      const uint32_t sees = r < 8 ? p.visible[r] : 0u;
+      for (int c = 0; c < 32; ++c) {
+        const int k = w * 32 + c, kr = key_roles[tid % 2 * 32 + c];
+        if (kr == 255) break;  // beyond the last key
+        const bool on = (sees >> 31) != 0u || (kr < 8 && ((sees >> kr) & 1u)) || k == q;
+        word |= (on ? 1u : 0u) << c;
+      }
+      p.struct_bits[static_cast<int64_t>(q) * p.wpr + w] = word;
+    }
+    const bool any = __syncthreads_or(word != 0u) != 0;
+    if (tid == 0) p.block_any[blockIdx.x] = any ? 1 : 0;
+    // bytes of the block, consecutive threads on consecutive keys: a wavefront holds the 64 keys of one row at a time
+    const int lane = tid % kWave, wave = tid / kWave;
+    for (int i = 0; i < kWave / 2; ++i) {
+      const int row = qc * kQB + wave * (kWave / 2) + i, k = kc * kKC + lane;
+      const uint32_t bits = static_cast<uint32_t>(__shfl(static_cast<int>(word), 2 * i + lane / 32));
+      if (row < T && k < T) p.structural[static_cast<int64_t>(row) * T + k] = (bits >> (lane % 32)) & 1u;
+    }
+    return;
+  }
+  const int b = (static_cast<int>(blockIdx.x) - blocks) * (kMaskThreads / kWave) + tid / kWave, lane = tid % kWave;
+  if (b >= p.B) return;
+  const uint8_t* pad = p.padding + static_cast<int64_t>(b) * T;
+  bool mine = false;
+  for (int t = lane; t < T; t += kWave) mine |= pad[t] == 0;
+  const bool all_padded = __builtin_amdgcn_ballot_w64(mine) == 0;  // then position 0 counts as valid: no softmax row is empty
+  for (int t0 = 0; t0 < T; t0 += kWave) {
+    const int t = t0 + lane;
+    const bool valid = t < T && (pad[t] == 0 || (all_padded && t == 0));
+    if (t < T) p.key_valid[static_cast<int64_t>(b) * T + t] = valid ? 1 : 0;
+    const uint64_t bits = __builtin_amdgcn_ballot_w64(valid);
+    const int w = t0 / 32 + lane;
+    if (lane < 2 && w < p.wpr) p.valid_bits[static_cast<int64_t>(b) * p.wpr + w] = static_cast<uint32_t>(bits >> (32 * lane));
+  }
+}
+
 struct MaskArgs {
   const uint32_t* struct_bits = nullptr;
   int64_t struct_stride = 0;
@@ -1827,6 +1896,35 @@ extern "C" int taac_mask_block_any(const uint32_t* struct_bits, int32_t Tq, int3
   const int nqc = (Tq + kQB - 1) / kQB, nkc = (Tk + kKC - 1) / kKC;
   hipLaunchKernelGGL(block_any_kernel, dim3(nqc * nkc), dim3(kWave), 0, as_stream(stream), struct_bits, Tq,
                      (Tk + 31) / 32, nkc, block_any);
+  return check_launch(name);
+}
+
+extern "C" int taac_role_mask(const void* roles, int roles_int64, const uint32_t visible[8], const uint8_t* padding, int32_t B, int32_t T,
+                              uint8_t* structural, uint32_t* struct_bits, uint8_t* block_any, uint8_t* key_valid,
+                              uint32_t* valid_bits, void* stream) {
+  using namespace taac;
+  const char* name = "taac_role_mask";
+  if (B <= 0 || T <= 0) return set_error(TAAC_ERR_INVALID_VALUE, "%s: B and T must be positive", name);
+  if (!roles || !visible || !padding || !structural || !struct_bits || !block_any || !key_valid || !valid_bits)
+    return set_error(TAAC_ERR_INVALID_VALUE, "%s: null pointer", name);
+  RoleMaskParams p{};
+  p.roles = roles;
+  p.roles_int64 = roles_int64 != 0;
+  for (int r = 0; r < 8; ++r) p.visible[r] = visible[r];
+  p.padding = padding;
+  p.B = B;
+  p.T = T;
+  p.nqc = (T + kQB - 1) / kQB;
+  p.nkc = (T + kKC - 1) / kKC;
+  p.wpr = (T + 31) / 32;
+  p.structural = structural;
+  p.struct_bits = struct_bits;
+  p.block_any = block_any;
+  p.key_valid = key_valid;
+  p.valid_bits = valid_bits;
+  const int64_t grid = static_cast<int64_t>(p.nqc) * p.nkc + (B + kMaskThreads / kWave - 1) / (kMaskThreads / kWave);
+  if (grid > 0x7fffffffLL) return set_error(TAAC_ERR_UNSUPPORTED, "%s: too many workgroups", name);
+  hipLaunchKernelGGL(role_mask_kernel, dim3(static_cast<uint32_t>(grid)), dim3(kMaskThreads), 0, as_stream(stream), p);
   return check_launch(name);
 }
 

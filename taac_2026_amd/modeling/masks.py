@@ -10,12 +10,13 @@ part is a few (T, T) elementwise torch expressions on the inputs' device; the B 
 
 from __future__ import annotations
 
+import ctypes
 import math
 
 import torch
 import torch.nn as nn
 
-from taac_2026_amd.accelerators.attention import StructuredAttentionMask, build_structured_mask
+from taac_2026_amd.accelerators.attention import StructuredAttentionMask, build_role_mask, build_structured_mask
 from taac_2026_amd.modeling.sequence import safe_key_padding_mask
 
 # Token roles of the TokenFormer package (experiments/tokenformer/model.py:32-37).
@@ -88,6 +89,18 @@ def metadata_structural_mask(role_ids: torch.Tensor) -> torch.Tensor:
     return structural | torch.eye(token_count, dtype=torch.bool, device=role_ids.device)
 
 
+def _role_bits(*roles: int) -> int:
+    return sum(1 << role for role in roles)
+
+
+# The same table for the kernel: one word per query role, bit r = keys of role r, bit 31 = every key.
+_EVERY_KEY = 1 << 31
+_FIELD_KEYS = _role_bits(ROLE_CLS, ROLE_CANDIDATE, ROLE_USER, ROLE_ITEM, ROLE_DENSE, ROLE_MISSING, ROLE_STATS)
+_SEQUENCE_KEYS = _role_bits(ROLE_CLS, ROLE_CANDIDATE, ROLE_ITEM, ROLE_SEQUENCE, ROLE_MISSING, ROLE_STATS)
+_VISIBLE = (ctypes.c_uint32 * 8)(_EVERY_KEY, _EVERY_KEY, _FIELD_KEYS, _FIELD_KEYS, _FIELD_KEYS, _FIELD_KEYS, _SEQUENCE_KEYS,
+                                 _EVERY_KEY)
+
+
 class MetadataAttentionMask(nn.Module):
     """``forward(padding_mask (B, T), role_ids (T,)) -> StructuredAttentionMask``; disabled: every valid key is visible.
     (The reference module takes its token batch object and reads these two fields from it.)"""
@@ -98,6 +111,10 @@ class MetadataAttentionMask(nn.Module):
 
     def forward(self, padding_mask: torch.Tensor, role_ids: torch.Tensor) -> StructuredAttentionMask:
         token_count = padding_mask.shape[1]
+        if (self.enabled and padding_mask.is_cuda and padding_mask.dtype is torch.bool and padding_mask.numel() > 0
+                and role_ids.device == padding_mask.device and role_ids.shape == (token_count,)
+                and role_ids.dtype in (torch.int32, torch.int64)):
+            return build_role_mask(role_ids, _VISIBLE, padding_mask)
         if self.enabled:
             structural = metadata_structural_mask(role_ids)
         else:

@@ -495,3 +495,21 @@ def test_reference_block_trains_with_its_default_dropout(device):
             assert parameter.grad is not None and torch.isfinite(parameter.grad).all(), name
     assert torch.equal(results[0][0], results[1][0]) and torch.equal(results[0][1], results[1][1])
     assert torch.isfinite(results[0][0]).all() and torch.isfinite(results[0][1]).all()
+
+
+@pytest.mark.parametrize("tokens", [1, 31, 33, 64, 65, 127, 128, 129, 300])
+@pytest.mark.parametrize("dtype", [torch.int32, torch.int64])
+def test_role_mask_in_one_launch_equals_the_tensor_expressions(device, tokens, dtype):
+    from taac_2026_amd.accelerators.attention import build_structured_mask
+    from taac_2026_amd.modeling.masks import metadata_structural_mask
+    from taac_2026_amd.modeling.sequence import safe_key_padding_mask
+
+    g = torch.Generator().manual_seed(tokens)
+    roles = torch.randint(-1, 10, (tokens,), generator=g).to(dtype).to(device)   # some are none of the eight
+    padding = (torch.rand(6, tokens, generator=g) < 0.5).to(device)
+    padding[1], padding[2] = True, False                                           # nothing valid, everything valid
+    got = MetadataAttentionMask(enabled=True)(padding, roles)
+    want = build_structured_mask(metadata_structural_mask(roles), ~safe_key_padding_mask(padding))
+    for field in ("structural", "struct_bits", "block_any", "key_valid", "valid_bits"):
+        assert torch.equal(getattr(got, field), getattr(want, field)), field
+    assert got.self_bits is None and got.query_self is None and got.padding_source is padding
