@@ -549,6 +549,13 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu((DP ==
 #pragma unroll
     for (int j = 0; j < 16; ++j) dkacc[mb][j] = dvacc[mb][j] = 0.f;
   const float c = p.scale * 1.4426950408889634f;
+  // With mask bits the products dP start from -D: four registers less at their peak, without which the kernel spills (d = 32, masked
+  // blocks of 128 x 403 tokens 87 -> 71 us). Without them the statistics' way into the accumulators only delays the first product
+  // (1024 x 512 tokens 490 -> 512 us). The 1 / sqrt(d) of dS multiplies dK at the end; in fp16, whose range the unscaled dS could
+  // leave, it multiplies every element.
+  constexpr bool START_D = MODE == kMaskBits;
+  const float ds_scale = std::is_same<T, bf16_t>::value ? 1.0f : p.scale;
+  const float dk_scale = std::is_same<T, bf16_t>::value ? p.scale : 1.0f;
   const int64_t stat0 = (static_cast<int64_t>(b) * p.H + h) * p.Tq;
 
   if (k_begin < len) {  // workgroup-uniform: a block of padding keys gets zero gradients without any work
@@ -571,12 +578,12 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu((DP ==
       }
     };
     // the row statistics travel through registers: base-2 log-sum-exp (+inf: the row carries nothing, exp2(x - inf) = 0)
-    // and D_i / sqrt(d)
+    // and -D_i
     auto commit_stats = [&](int buffer) {
       if (tid < kChunk) {
         float* stats = reinterpret_cast<float*>(smem + buffer * BUF_BYTES + 2 * TILE_BYTES);
         stats[tid] = lse_next > -INFINITY ? lse_next * 1.4426950408889634f : INFINITY;
-        stats[kChunk + tid] = delta_next * p.scale;
+        stats[kChunk + tid] = -delta_next;
       }
       if (BITS)
         reinterpret_cast<uint32_t*>(smem + buffer * BUF_BYTES + 2 * TILE_BYTES + 2 * kChunk * 4)[tid] = word_next;
@@ -615,6 +622,14 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu((DP ==
         f32x16 sacc, dpacc;
 #pragma unroll
         for (int j = 0; j < 16; ++j) sacc[j] = dpacc[j] = 0.f;
+        if (START_D) {
+#pragma unroll
+          for (int jq = 0; jq < 4; ++jq) {
+            const f32x4 d4 = *reinterpret_cast<const f32x4*>(&sDelta[qt * 32 + jq * 8 + hh * 4]);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) dpacc[jq * 4 + e] = d4[e];
+          }
+        }
 #pragma unroll
         for (int s = 0; s < KSTEPS; ++s) {
           const uint32_t off = qt * 32 * ROWB + (row_off ^ (s * 32));
@@ -632,12 +647,14 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu((DP ==
           for (int j = 0; j < 16; ++j)
             if (kj > qc0 + qt * 32 + (j / 4) * 8 + hh * 4 + (j % 4)) sacc[j] = -INFINITY;
         }
+        auto scaled = [&](float x) { return std::is_same<T, bf16_t>::value ? x : x * ds_scale; };
         vec_t pb[2], dsb[2];
 #pragma unroll
         for (int jq = 0; jq < 4; ++jq) {
           const int r0 = qt * 32 + jq * 8 + hh * 4;  // four consecutive queries of the chunk
           const f32x4 l4 = *reinterpret_cast<const f32x4*>(&sLse[r0]);
-          const f32x4 d4 = *reinterpret_cast<const f32x4*>(&sDelta[r0]);  // already times 1 / sqrt(d)
+          [[maybe_unused]] f32x4 d4 = {0.f, 0.f, 0.f, 0.f};
+          if (!START_D) d4 = *reinterpret_cast<const f32x4*>(&sDelta[r0]);
           [[maybe_unused]] u32x4 w4 = {0u, 0u, 0u, 0u};
           if (BITS) w4 = *reinterpret_cast<const u32x4*>(&sWords[r0]);
 #pragma unroll
@@ -648,14 +665,14 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu((DP ==
               // the lane owns key kj; register j is query qc0 + r0 + e: bit l32 of that row's word for the wavefront's keys
               prob = (key_seen && ((w4[e] >> l32) & 1u) != 0u) ? prob : 0.f;
               pb[j / 8][j % 8] = static_cast<T>(prob);
-              dsb[j / 8][j % 8] = static_cast<T>(prob * fmaf(dpacc[j], p.scale, -d4[e]));
+              dsb[j / 8][j % 8] = static_cast<T>(prob * scaled(dpacc[j]));
             } else if (MODE == kMaskBitsDropout) {
               const int qrow = qc0 + r0 + e;
               prob = (key_seen && ((w4[e] >> l32) & 1u) != 0u) ? prob : 0.f;
               const bool keep = qrow < p.Tq && kj < p.Tk &&
                                 p.drop_mask[b * p.mask_bs + h * p.mask_hs + static_cast<int64_t>(qrow) * p.Tk + kj] != 0;
               pb[j / 8][j % 8] = static_cast<T>(keep ? prob * p.drop_scale : 0.f);
-              dsb[j / 8][j % 8] = static_cast<T>(prob * fmaf(keep ? dpacc[j] * p.drop_scale : 0.f, p.scale, -d4[e]));
+              dsb[j / 8][j % 8] = static_cast<T>(prob * scaled((keep ? dpacc[j] * p.drop_scale : 0.f) + d4[e]));
             } else if (MODE != kMaskNone) {
               // the lane owns key kj; register j is query qc0 + r0 + e: one mask byte per register
               const int qrow = qc0 + r0 + e;
@@ -663,15 +680,15 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu((DP ==
                                 p.drop_mask[b * p.mask_bs + h * p.mask_hs + static_cast<int64_t>(qrow) * p.Tk + kj] != 0;
               if (DROPOUT) {
                 pb[j / 8][j % 8] = static_cast<T>(keep ? prob * p.drop_scale : 0.f);
-                dsb[j / 8][j % 8] = static_cast<T>(prob * fmaf(keep ? dpacc[j] * p.drop_scale : 0.f, p.scale, -d4[e]));
+                dsb[j / 8][j % 8] = static_cast<T>(prob * scaled((keep ? dpacc[j] * p.drop_scale : 0.f) + d4[e]));
               } else {
                 prob = keep ? prob : 0.f;
                 pb[j / 8][j % 8] = static_cast<T>(prob);
-                dsb[j / 8][j % 8] = static_cast<T>(prob * fmaf(dpacc[j], p.scale, -d4[e]));
+                dsb[j / 8][j % 8] = static_cast<T>(prob * scaled(dpacc[j] + d4[e]));
               }
             } else {
               pb[j / 8][j % 8] = static_cast<T>(prob);
-              dsb[j / 8][j % 8] = static_cast<T>(prob * fmaf(dpacc[j], p.scale, -d4[e]));
+              dsb[j / 8][j % 8] = static_cast<T>(prob * scaled(dpacc[j] + d4[e]));
             }
           }
         }
@@ -679,6 +696,12 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu((DP ==
       });
       if (DMA && more) commit_stats(buf);  // the next chunk's statistics: the barrier above publishes them
     }
+  }
+  if (dk_scale != 1.0f) {
+#pragma unroll
+    for (int mb = 0; mb < MB; ++mb)
+#pragma unroll
+      for (int j = 0; j < 16; ++j) dkacc[mb][j] *= dk_scale;
   }
   if (!k_ok) {  // a key in the padding receives no gradient
 #pragma unroll
