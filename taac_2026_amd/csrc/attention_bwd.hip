@@ -57,9 +57,9 @@ struct AttnBwdParams {
 };
 
 // First row of (sample b, head h).
-template <typename T>
+template <bool COMPACT, typename T>
 __device__ __forceinline__ T* head_rows(T* base, const int64_t (&strides)[4], const AttnBwdParams& p, int b, int h) {
-  const int64_t row0 = p.row_offsets != nullptr ? p.row_offsets[b] * strides[2] : b * strides[0];
+  const int64_t row0 = COMPACT ? p.row_offsets[b] * strides[2] : b * strides[0];
   return base + row0 + h * strides[1];
 }
 
@@ -292,7 +292,9 @@ __device__ __forceinline__ uint32_t keep_bytes4(const uint8_t* row, int key0, in
 // kMaskBitsDropout: the bit form for the pairs AND the byte keep mask of dropout (both pointers).
 constexpr int kMaskNone = 0, kMaskDropout = 1, kMaskVisible = 2, kMaskBits = 3, kMaskBitsDropout = 4;
 
-template <typename T, int DP, bool DMA, int MODE = kMaskNone>
+// COMPACT: samples are addressed by row_offsets (decided at run time it costs the other form 1.5 %: every pointer's chain of scalar
+// loads stands in front of a workgroup's first rows; 2048 x 4 x 256 x 64: 270 -> 274 and 306 -> 310 us).
+template <typename T, int DP, bool DMA, int MODE = kMaskNone, bool COMPACT = false>
 __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(DP == 32 ? 4 : 3))) void attn_bwd_dq_kernel(const AttnBwdParams p) {
   constexpr bool DROPOUT = MODE == kMaskDropout || MODE == kMaskBitsDropout;
   constexpr bool BITS = MODE == kMaskBits || MODE == kMaskBitsDropout;
@@ -309,12 +311,12 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(DP == 
   const int bh = static_cast<int>(logical / p.nblk);
   const int h = bh % p.H, b = bh / p.H;
   const int tid = threadIdx.x, wave = tid / kWave, lane = tid % kWave, l32 = lane % 32, hh = lane / 32;
-  const T* qb = head_rows(static_cast<const T*>(p.q), p.qs, p, b, h);
-  const T* kb = head_rows(static_cast<const T*>(p.k), p.ks, p, b, h);
-  const T* vb = head_rows(static_cast<const T*>(p.v), p.vs, p, b, h);
-  const T* ob = head_rows(static_cast<const T*>(p.o), p.os, p, b, h);
-  const T* dob = head_rows(static_cast<const T*>(p.dout), p.dos, p, b, h);
-  T* dqb = head_rows(static_cast<T*>(p.dq), p.dqs, p, b, h);
+  const T* qb = head_rows<COMPACT>(static_cast<const T*>(p.q), p.qs, p, b, h);
+  const T* kb = head_rows<COMPACT>(static_cast<const T*>(p.k), p.ks, p, b, h);
+  const T* vb = head_rows<COMPACT>(static_cast<const T*>(p.v), p.vs, p, b, h);
+  const T* ob = head_rows<COMPACT>(static_cast<const T*>(p.o), p.os, p, b, h);
+  const T* dob = head_rows<COMPACT>(static_cast<const T*>(p.dout), p.dos, p, b, h);
+  T* dqb = head_rows<COMPACT>(static_cast<T*>(p.dq), p.dqs, p, b, h);
 
   int len = p.Tk;
   if (p.key_lengths != nullptr) {
@@ -488,10 +490,10 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(DP == 
     }
   }
   __syncthreads();  // the staging buffers now hold the output tiles
-  store_owned<T, DP>(dqacc, smem + wave * (32 * OROW), dqb, p.dqs[2], q_begin + wave * 32, p.row_offsets != nullptr ? len : p.Tq, p.d, lane);
+  store_owned<T, DP>(dqacc, smem + wave * (32 * OROW), dqb, p.dqs[2], q_begin + wave * 32, COMPACT ? len : p.Tq, p.d, lane);
 }
 
-template <typename T, int DP, bool DMA, int MODE = kMaskNone>
+template <typename T, int DP, bool DMA, int MODE = kMaskNone, bool COMPACT = false>
 __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu((DP == 32 ? 4 : 3) - (DMA ? 0 : 1)))) void attn_bwd_dkv_kernel(const AttnBwdParams p) {
   constexpr bool DROPOUT = MODE == kMaskDropout || MODE == kMaskBitsDropout;
   constexpr bool BITS = MODE == kMaskBits || MODE == kMaskBitsDropout;
@@ -513,12 +515,12 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu((DP ==
   const int bh = static_cast<int>(logical / p.nblk);
   const int h = bh % p.H, b = bh / p.H;
   const int tid = threadIdx.x, wave = tid / kWave, lane = tid % kWave, l32 = lane % 32, hh = lane / 32;
-  const T* qb = head_rows(static_cast<const T*>(p.q), p.qs, p, b, h);
-  const T* kb = head_rows(static_cast<const T*>(p.k), p.ks, p, b, h);
-  const T* vb = head_rows(static_cast<const T*>(p.v), p.vs, p, b, h);
-  const T* dob = head_rows(static_cast<const T*>(p.dout), p.dos, p, b, h);
-  T* dkb = head_rows(static_cast<T*>(p.dk), p.dks, p, b, h);
-  T* dvb = head_rows(static_cast<T*>(p.dv), p.dvs, p, b, h);
+  const T* qb = head_rows<COMPACT>(static_cast<const T*>(p.q), p.qs, p, b, h);
+  const T* kb = head_rows<COMPACT>(static_cast<const T*>(p.k), p.ks, p, b, h);
+  const T* vb = head_rows<COMPACT>(static_cast<const T*>(p.v), p.vs, p, b, h);
+  const T* dob = head_rows<COMPACT>(static_cast<const T*>(p.dout), p.dos, p, b, h);
+  T* dkb = head_rows<COMPACT>(static_cast<T*>(p.dk), p.dks, p, b, h);
+  T* dvb = head_rows<COMPACT>(static_cast<T*>(p.dv), p.dvs, p, b, h);
 
   int len = p.Tk;
   if (p.key_lengths != nullptr) {
@@ -551,11 +553,10 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu((DP ==
   const float c = p.scale * 1.4426950408889634f;
   // With mask bits the products dP start from -D: four registers less at their peak, without which the kernel spills (d = 32, masked
   // blocks of 128 x 403 tokens 87 -> 71 us). Without them the statistics' way into the accumulators only delays the first product
-  // (1024 x 512 tokens 490 -> 512 us). The 1 / sqrt(d) of dS multiplies dK at the end; in fp16, whose range the unscaled dS could
-  // leave, it multiplies every element.
+  // (1024 x 512 tokens 490 -> 512 us). The 1 / sqrt(d) of dS then multiplies dK at the end; in fp16, whose range the unscaled dS
+  // could leave, it multiplies every element.
   constexpr bool START_D = MODE == kMaskBits;
-  const float ds_scale = std::is_same<T, bf16_t>::value ? 1.0f : p.scale;
-  const float dk_scale = std::is_same<T, bf16_t>::value ? p.scale : 1.0f;
+  constexpr bool LATE_SCALE = START_D && std::is_same<T, bf16_t>::value;
   const int64_t stat0 = (static_cast<int64_t>(b) * p.H + h) * p.Tq;
 
   if (k_begin < len) {  // workgroup-uniform: a block of padding keys gets zero gradients without any work
@@ -578,12 +579,12 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu((DP ==
       }
     };
     // the row statistics travel through registers: base-2 log-sum-exp (+inf: the row carries nothing, exp2(x - inf) = 0)
-    // and -D_i
+    // and -D_i, times 1 / sqrt(d) where that is not left to the end
     auto commit_stats = [&](int buffer) {
       if (tid < kChunk) {
         float* stats = reinterpret_cast<float*>(smem + buffer * BUF_BYTES + 2 * TILE_BYTES);
         stats[tid] = lse_next > -INFINITY ? lse_next * 1.4426950408889634f : INFINITY;
-        stats[kChunk + tid] = -delta_next;
+        stats[kChunk + tid] = START_D ? -delta_next : -delta_next * p.scale;
       }
       if (BITS)
         reinterpret_cast<uint32_t*>(smem + buffer * BUF_BYTES + 2 * TILE_BYTES + 2 * kChunk * 4)[tid] = word_next;
@@ -647,7 +648,6 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu((DP ==
           for (int j = 0; j < 16; ++j)
             if (kj > qc0 + qt * 32 + (j / 4) * 8 + hh * 4 + (j % 4)) sacc[j] = -INFINITY;
         }
-        auto scaled = [&](float x) { return std::is_same<T, bf16_t>::value ? x : x * ds_scale; };
         vec_t pb[2], dsb[2];
 #pragma unroll
         for (int jq = 0; jq < 4; ++jq) {
@@ -665,14 +665,14 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu((DP ==
               // the lane owns key kj; register j is query qc0 + r0 + e: bit l32 of that row's word for the wavefront's keys
               prob = (key_seen && ((w4[e] >> l32) & 1u) != 0u) ? prob : 0.f;
               pb[j / 8][j % 8] = static_cast<T>(prob);
-              dsb[j / 8][j % 8] = static_cast<T>(prob * scaled(dpacc[j]));
+              dsb[j / 8][j % 8] = static_cast<T>(prob * (LATE_SCALE ? dpacc[j] : dpacc[j] * p.scale));
             } else if (MODE == kMaskBitsDropout) {
               const int qrow = qc0 + r0 + e;
               prob = (key_seen && ((w4[e] >> l32) & 1u) != 0u) ? prob : 0.f;
               const bool keep = qrow < p.Tq && kj < p.Tk &&
                                 p.drop_mask[b * p.mask_bs + h * p.mask_hs + static_cast<int64_t>(qrow) * p.Tk + kj] != 0;
               pb[j / 8][j % 8] = static_cast<T>(keep ? prob * p.drop_scale : 0.f);
-              dsb[j / 8][j % 8] = static_cast<T>(prob * scaled((keep ? dpacc[j] * p.drop_scale : 0.f) + d4[e]));
+              dsb[j / 8][j % 8] = static_cast<T>(prob * fmaf(keep ? dpacc[j] * p.drop_scale : 0.f, p.scale, d4[e]));
             } else if (MODE != kMaskNone) {
               // the lane owns key kj; register j is query qc0 + r0 + e: one mask byte per register
               const int qrow = qc0 + r0 + e;
@@ -680,15 +680,15 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu((DP ==
                                 p.drop_mask[b * p.mask_bs + h * p.mask_hs + static_cast<int64_t>(qrow) * p.Tk + kj] != 0;
               if (DROPOUT) {
                 pb[j / 8][j % 8] = static_cast<T>(keep ? prob * p.drop_scale : 0.f);
-                dsb[j / 8][j % 8] = static_cast<T>(prob * scaled((keep ? dpacc[j] * p.drop_scale : 0.f) + d4[e]));
+                dsb[j / 8][j % 8] = static_cast<T>(prob * fmaf(keep ? dpacc[j] * p.drop_scale : 0.f, p.scale, d4[e]));
               } else {
                 prob = keep ? prob : 0.f;
                 pb[j / 8][j % 8] = static_cast<T>(prob);
-                dsb[j / 8][j % 8] = static_cast<T>(prob * scaled(dpacc[j] + d4[e]));
+                dsb[j / 8][j % 8] = static_cast<T>(prob * fmaf(dpacc[j], p.scale, d4[e]));
               }
             } else {
               pb[j / 8][j % 8] = static_cast<T>(prob);
-              dsb[j / 8][j % 8] = static_cast<T>(prob * scaled(dpacc[j] + d4[e]));
+              dsb[j / 8][j % 8] = static_cast<T>(prob * fmaf(dpacc[j], p.scale, d4[e]));
             }
           }
         }
@@ -697,11 +697,11 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu((DP ==
       if (DMA && more) commit_stats(buf);  // the next chunk's statistics: the barrier above publishes them
     }
   }
-  if (dk_scale != 1.0f) {
+  if (LATE_SCALE) {
 #pragma unroll
     for (int mb = 0; mb < MB; ++mb)
 #pragma unroll
-      for (int j = 0; j < 16; ++j) dkacc[mb][j] *= dk_scale;
+      for (int j = 0; j < 16; ++j) dkacc[mb][j] *= p.scale;
   }
   if (!k_ok) {  // a key in the padding receives no gradient
 #pragma unroll
@@ -711,7 +711,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu((DP ==
   }
   __syncthreads();
   uint8_t* tile = smem + wave * (32 * OROW);
-  const int k_store_end = p.row_offsets != nullptr ? len : p.Tk;
+  const int k_store_end = COMPACT ? len : p.Tk;
   store_owned<T, DP>(dkacc, tile, dkb, p.dks[2], k_begin + wave * 32, k_store_end, p.d, lane);
   asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
   store_owned<T, DP>(dvacc, tile, dvb, p.dvs[2], k_begin + wave * 32, k_store_end, p.d, lane);
@@ -729,22 +729,30 @@ bool small_offsets(int64_t rows, int64_t stride) {
   return stride < (1 << 22) && rows < (1 << 22) && rows * stride * 2 < (1ll << 31);
 }
 
-template <typename T, int DP, int MODE>
-void launch_bwd_mode(AttnBwdParams p, bool register_staging, hipStream_t s) {
+template <typename T, int DP, int MODE, bool COMPACT>
+void launch_bwd_form(AttnBwdParams p, bool register_staging, hipStream_t s) {
   // TAAC_ATTN_REGISTER_STAGING keeps the register-staged kernels for full head dims too (comparison route of the caller).
   const bool direct = p.d == DP && !register_staging;
   p.nblk = static_cast<uint32_t>((p.Tq + kOwn - 1) / kOwn);
   p.total = p.nblk * p.B * p.H;
   if (direct && small_offsets(p.Tk, p.ks[2]) && small_offsets(p.Tk, p.vs[2]))
-    hipLaunchKernelGGL((attn_bwd_dq_kernel<T, DP, true, MODE>), dim3(p.total), dim3(kThreads), 0, s, p);
+    hipLaunchKernelGGL((attn_bwd_dq_kernel<T, DP, true, MODE, COMPACT>), dim3(p.total), dim3(kThreads), 0, s, p);
   else
-    hipLaunchKernelGGL((attn_bwd_dq_kernel<T, DP, false, MODE>), dim3(p.total), dim3(kThreads), 0, s, p);
+    hipLaunchKernelGGL((attn_bwd_dq_kernel<T, DP, false, MODE, COMPACT>), dim3(p.total), dim3(kThreads), 0, s, p);
   p.nblk = static_cast<uint32_t>((p.Tk + kOwn - 1) / kOwn);
   p.total = p.nblk * p.B * p.H;
   if (direct && small_offsets(p.Tq, p.qs[2]) && small_offsets(p.Tq, p.dos[2]))
-    hipLaunchKernelGGL((attn_bwd_dkv_kernel<T, DP, true, MODE>), dim3(p.total), dim3(kThreads), 0, s, p);
+    hipLaunchKernelGGL((attn_bwd_dkv_kernel<T, DP, true, MODE, COMPACT>), dim3(p.total), dim3(kThreads), 0, s, p);
   else
-    hipLaunchKernelGGL((attn_bwd_dkv_kernel<T, DP, false, MODE>), dim3(p.total), dim3(kThreads), 0, s, p);
+    hipLaunchKernelGGL((attn_bwd_dkv_kernel<T, DP, false, MODE, COMPACT>), dim3(p.total), dim3(kThreads), 0, s, p);
+}
+
+template <typename T, int DP, int MODE>
+void launch_bwd_mode(const AttnBwdParams& p, bool register_staging, hipStream_t s) {
+  if constexpr (std::is_same<T, bf16_t>::value && (MODE == kMaskNone || MODE == kMaskBits)) {  // what attention_compact_bwd asks for
+    if (p.row_offsets != nullptr) return launch_bwd_form<T, DP, MODE, true>(p, register_staging, s);
+  }
+  launch_bwd_form<T, DP, MODE, false>(p, register_staging, s);
 }
 
 template <typename T, int DP>
