@@ -36,6 +36,20 @@ def _bf16(parameter: torch.Tensor | None) -> torch.Tensor | None:
     return parameter if parameter.dtype == torch.bfloat16 else parameter.to(torch.bfloat16)
 
 
+def _part(block: nn.Module, name: str) -> nn.Module | None:
+    """``getattr(block, name)`` of a submodule, by its registry where it is there (attribute lookups on modules are most of what the
+    host does in ``PCVRBackbone.forward``)."""
+    return block._modules[name] if name in block._modules else getattr(block, name)
+
+
+def _held(module: nn.Module | None, name: str) -> torch.Tensor | None:
+    """``getattr(module, name)`` of a parameter, by its registry where it is there. It is not where the value is computed or a view
+    that a wrapper puts in its place (parametrisations, weight norm, flattened shards, data-parallel replicas)."""
+    if module is None:
+        return None
+    return module._parameters[name] if name in module._parameters else getattr(module, name)
+
+
 def _compute_dtype(tokens: torch.Tensor) -> torch.dtype:
     """The 16-bit type a layer computes in: float16 tokens stay float16 (tiled kernels, forward only), everything else
     runs in bfloat16."""
@@ -546,28 +560,24 @@ class PCVRBackbone(nn.Module):
         keep_alive: list[torch.Tensor] = []
 
         def dev(module: nn.Module | None, name: str) -> int | None:
-            # (the registries directly: attribute lookups on modules and no-op conversions of 42 parameters are most of what
-            # the host does in this call)
-            parameter = None if module is None else module._parameters[name]
-            if parameter is None:
+            tensor = _held(module, name)
+            if tensor is None:
                 return None
-            if parameter.dtype is torch.bfloat16 and parameter.is_contiguous():
-                return parameter.data_ptr()
-            tensor = _bf16(parameter).detach().contiguous()
-            keep_alive.append(tensor)
+            if tensor.dtype is not torch.bfloat16 or not tensor.is_contiguous():
+                tensor = _bf16(tensor).detach().contiguous()
+            keep_alive.append(tensor)  # (a computed value has no other owner)
             return tensor.data_ptr()
 
         packed = (_native.BlockWeights * len(self.blocks))()
         for slot, block in zip(packed, self.blocks):
-            parts = block._modules
-            slot.attn_norm_weight = dev(parts["attn_norm"], "weight")
-            slot.qkv_weight, slot.qkv_bias = dev(parts["qkv"], "weight"), dev(parts["qkv"], "bias")
-            slot.out_weight, slot.out_bias = dev(parts["out"], "weight"), dev(parts["out"], "bias")
-            slot.ffn_norm_weight = dev(parts["ffn_norm"], "weight")
-            slot.up_weight, slot.up_bias = dev(parts["up"], "weight"), dev(parts["up"], "bias")
-            slot.down_weight, slot.down_bias = dev(parts["down"], "weight"), dev(parts["down"], "bias")
-            slot.query_norm_weight = dev(parts.get("query_norm"), "weight")
-            slot.key_norm_weight = dev(parts.get("key_norm"), "weight")
+            slot.attn_norm_weight = dev(_part(block, "attn_norm"), "weight")
+            slot.qkv_weight, slot.qkv_bias = dev(_part(block, "qkv"), "weight"), dev(_part(block, "qkv"), "bias")
+            slot.out_weight, slot.out_bias = dev(_part(block, "out"), "weight"), dev(_part(block, "out"), "bias")
+            slot.ffn_norm_weight = dev(_part(block, "ffn_norm"), "weight")
+            slot.up_weight, slot.up_bias = dev(_part(block, "up"), "weight"), dev(_part(block, "up"), "bias")
+            slot.down_weight, slot.down_bias = dev(_part(block, "down"), "weight"), dev(_part(block, "down"), "bias")
+            slot.query_norm_weight = dev(_part(block, "query_norm"), "weight")
+            slot.key_norm_weight = dev(_part(block, "key_norm"), "weight")
         table = None
         if self.rope_base is not None:
             table = rope_table(tokens, self.d_model // self.num_heads, self.rope_base, torch.bfloat16, emb.device)
@@ -624,10 +634,7 @@ class PCVRBackbone(nn.Module):
             return (torch.sigmoid(logits.float()), emb * valid) if return_hidden else torch.sigmoid(logits.float())
         params: list[torch.Tensor | None] = []
         for block in self.blocks:
-            parts = block._modules                    # (the registries directly, as in forward)
-            for part, parameter in self._TRAINED:
-                module = parts.get(part)
-                params.append(None if module is None else module._parameters[parameter])
+            params += [_held(_part(block, part), parameter) for part, parameter in self._TRAINED]
         params += [self.head.weight, self.head.bias]
         hidden, _, probabilities = InteractionStackFunction.apply(
             emb, key_lengths, None,

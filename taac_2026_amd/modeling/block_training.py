@@ -391,7 +391,7 @@ class InteractionStackFunction(torch.autograd.Function):
 def uniform_parameters(params: list) -> list:
     """``params`` as they are when all are bf16 or all float32; else rounded to bf16 (autograd carries the gradients back)."""
     dtypes = {p.dtype for p in params if p is not None}
-    if len(dtypes) == 1:
+    if dtypes in ({torch.bfloat16}, {torch.float32}):
         return params
     return [p if p is None or p.dtype == torch.bfloat16 else p.to(torch.bfloat16) for p in params]
 

@@ -9,6 +9,7 @@ from __future__ import annotations
 import pytest
 import torch
 import torch.nn.functional as F
+import torch.nn.utils.parametrize
 
 from oracle import reference as oracle
 from taac_2026_amd.api import MetadataAttentionMask, PCVRBackbone, UnifiedInteractionBlock, run_interaction_blocks
@@ -100,3 +101,33 @@ def test_a_stack_is_its_blocks_one_after_the_other(device):
 
     for got, want in zip(run(False), run(True)):
         assert torch.equal(got, want)
+
+
+def test_computed_weights_are_taken_where_a_module_holds_no_parameter(device):
+    """A parametrised weight is not in its module's registry: it is computed at each access. The network takes it like the plain
+    network with the same value, and its gradient reaches what it is computed from."""
+    class Double(torch.nn.Module):
+        def forward(self, weight):
+            return weight * 2.0
+
+    g = torch.Generator().manual_seed(5)
+    plain = PCVRBackbone(d_model=128, num_heads=4, d_ff=128, n_blocks=2).to(torch.bfloat16).to(device)
+    computed = PCVRBackbone(d_model=128, num_heads=4, d_ff=128, n_blocks=2).to(torch.bfloat16).to(device)
+    computed.load_state_dict(plain.state_dict())
+    with torch.no_grad():
+        for block, other in zip(plain.blocks, computed.blocks):
+            for module, target in ((block.qkv, other.qkv), (block.down, other.down), (block.ffn_norm, other.ffn_norm)):
+                module.weight.mul_(2.0)                                   # exact in bf16
+                torch.nn.utils.parametrize.register_parametrization(target, "weight", Double(), unsafe=True)
+    emb = torch.randn(3, 40, 128, generator=g).to(torch.bfloat16).to(device)
+    lengths = torch.tensor([40, 0, 17], dtype=torch.int32, device=device)
+    with torch.no_grad():
+        assert torch.equal(computed(emb, lengths), plain(emb, lengths))
+    got, want = computed(emb, lengths), plain(emb, lengths)
+    assert torch.equal(got, want)
+    got.sum().backward()
+    want.sum().backward()
+    for block, other in zip(plain.blocks, computed.blocks):
+        assert torch.equal(other.up.weight.grad, block.up.weight.grad)
+        for module, target in ((block.qkv, other.qkv), (block.down, other.down), (block.ffn_norm, other.ffn_norm)):
+            assert torch.equal(target.parametrizations.weight.original.grad, module.weight.grad * 2.0)
