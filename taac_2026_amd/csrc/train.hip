@@ -684,7 +684,7 @@ extern "C" int taac_stack_train_bwd(const void* grad_out, const void* grad_attn_
   if (!shape_ok(z)) return set_error(TAAC_ERR_UNSUPPORTED, "%s: shape not covered (see taac_stack_train_bytes)", name);
   if (param_dtype != TAAC_BF16 && param_dtype != TAAC_F32)
     return set_error(TAAC_ERR_INVALID_VALUE, "%s: parameters are bf16 or fp32", name);
-  if (!key_lengths || !saved || !scratch || (grad_p != nullptr && (!p || !grad_head_w || !grad_head_b)) ||
+  if (!key_lengths || !saved || !scratch || (grad_p != nullptr && (!p || !grad_head_w)) ||
       (grad_p == nullptr && grad_out == nullptr && grad_attn_tokens == nullptr) ||
       (struct_bits && (!rows_given || !count_given || !valid_bits)))
     return set_error(TAAC_ERR_INVALID_VALUE, "%s: null pointer", name);
@@ -715,7 +715,7 @@ extern "C" int taac_stack_train_bwd(const void* grad_out, const void* grad_attn_
     hipLaunchKernelGGL(head_bwd_kernel, dim3(B), dim3(kThreads), 0, s, sv.x_last, grad_p, p, offsets, sv.head_w, dy, dw_part, db_part, D);
     if ((rc = check_launch(name)) != TAAC_OK) return rc;
     vectors[n_vectors++] = VectorItem{dw_part, grad_head_w, B, D, D};
-    vectors[n_vectors++] = VectorItem{db_part, grad_head_b, B, 1, 1};
+    if (grad_head_b != nullptr) vectors[n_vectors++] = VectorItem{db_part, grad_head_b, B, 1, 1};
     have_dy = true;
   }
   if (grad_out != nullptr) {

@@ -131,3 +131,19 @@ def test_computed_weights_are_taken_where_a_module_holds_no_parameter(device):
         assert torch.equal(other.up.weight.grad, block.up.weight.grad)
         for module, target in ((block.qkv, other.qkv), (block.down, other.down), (block.ffn_norm, other.ffn_norm)):
             assert torch.equal(target.parametrizations.weight.original.grad, module.weight.grad * 2.0)
+
+
+def test_a_head_without_bias_trains(device):
+    """No bias = a bias of zero: the same probabilities and gradients, bit for bit."""
+    g = torch.Generator().manual_seed(6)
+    emb = torch.randn(3, 40, 128, generator=g).to(torch.bfloat16).to(device)
+    lengths = torch.tensor([40, 0, 17], dtype=torch.int32, device=device)
+    zero, none = (PCVRBackbone(d_model=128, num_heads=4, d_ff=128, n_blocks=1).to(torch.bfloat16).to(device) for _ in range(2))
+    none.load_state_dict(zero.state_dict())
+    none.head.bias = None
+    got, want = none(emb, lengths), zero(emb, lengths)
+    assert torch.equal(got, want)
+    got.sum().backward()
+    want.sum().backward()
+    for name, parameter in none.named_parameters():
+        assert torch.equal(parameter.grad, zero.get_parameter(name).grad), name
