@@ -528,7 +528,13 @@ __global__ __launch_bounds__(256) void sum_vectors_kernel(const VectorParams p) 
   }
 }
 
-// 256 x 256 tiles where the layers are that wide, 128 x 128 tiles of four wavefronts for the narrow model.
+// 256 x 256 tiles where the layers are that wide and the batch fills the chip with them; 128 x 128 tiles of four wavefronts, two
+// workgroups per compute unit, for the narrow model and for small batches: there a tile's chain over its chunks and its store are the
+// time, not the operands, which L2 holds, and four times as many tiles need fewer splits and partial sums. Gradients and their
+// reduction, us per block, 256- / 128-wide tiles, F = 1024 (F = 512), by positions of which 6 in 10 hold tokens: 1 024 50 / 27,
+// 3 216 39 / 28, 9 648 49 / 42 (45 / 36), 15 360 (48 / 46), 16 384 58 / 59 (49 / 47); from 42 496 on the step is 1 - 7 % slower.
+// At least 512 tokens a split: with 1 024 it is 37 instead of 27 at 1 024 positions and, D = 128, 35 instead of 25; 256 lies within 4 us
+// either way.
 struct WgradPlan {
   int tn, tk, tiles, splits;
 };
@@ -536,13 +542,13 @@ WgradPlan plan_of(int64_t M, const int32_t (*shapes)[2], int items) {
   WgradPlan pl{};
   int min_side = 1 << 30;
   for (int i = 0; i < items; ++i) min_side = shapes[i][0] < min_side ? shapes[i][0] : (shapes[i][1] < min_side ? shapes[i][1] : min_side);
-  pl.tn = pl.tk = min_side >= 256 ? 256 : 128;
+  const int cus = compute_units() > 0 ? compute_units() : 1;
+  pl.tn = pl.tk = min_side >= 256 && M >= 64 * static_cast<int64_t>(cus) ? 256 : 128;
   for (int i = 0; i < items; ++i) pl.tiles += ((shapes[i][0] + pl.tn - 1) / pl.tn) * ((shapes[i][1] + pl.tk - 1) / pl.tk);
-  // about one workgroup per compute unit (two of the small ones), but no split of fewer than 1 024 tokens: a split costs a pass
+  // about one workgroup per compute unit (two of the small ones), but no split of fewer than 512 tokens: a split costs a pass
   // over its partial tile
-  const int cus = compute_units();
-  const int want = (pl.tn == 256 ? 1 : 2) * (cus > 0 ? cus : 1) / pl.tiles;
-  const int64_t most = (M + 1023) / 1024;
+  const int want = (pl.tn == 256 ? 1 : 2) * cus / pl.tiles;
+  const int64_t most = (M + 511) / 512;
   pl.splits = want < 1 ? 1 : want;
   if (pl.splits > most) pl.splits = most < 1 ? 1 : static_cast<int>(most);
   return pl;

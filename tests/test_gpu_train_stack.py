@@ -27,6 +27,7 @@ def _near(name: str, got: torch.Tensor, want: torch.Tensor, blocks: int) -> None
     (256, 4, 96, 2, [0, 65, 64, 1], 65, True, torch.float32),             # around a 64-token tile; F not a multiple of a gradient tile
     (128, 4, 160, 2, [31, 33, 0], 33, False, torch.float32),
     (128, 2, 256, 1, [257, 3], 257, True, torch.bfloat16),                # rows of a sample over two workgroups of the index
+    (256, 4, 96, 1, [(11 * i) % 66 for i in range(40)], 65, False, torch.float32),      # several splits of the small gradient tiles
     (256, 8, 512, 1, [(7 * i) % 33 for i in range(1100)], 32, False, torch.bfloat16),   # 256-token workgroups, some past the count
     (128, 4, 128, 1, [(5 * i) % 41 for i in range(900)], 40, False, torch.float32),
 ])
