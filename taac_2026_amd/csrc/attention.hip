@@ -65,8 +65,8 @@ struct AttnParams {
   int64_t qs[4], ks[4], vs[4], os[4];
   float scale_log2;  // log2(e) / sqrt(d)
   int32_t zero_pad;
-  const int32_t* row_offsets;  // direct-transfer kernel: sample b's rows start at row row_offsets[b] of q, k, v and o (a compact
-                               // tensor of the batch's valid tokens) instead of at b times the batch strides; or null
+  const int32_t* row_offsets;  // sample b's rows start at row row_offsets[b] of q, k, v and o (a compact tensor of the batch's valid
+                               // tokens) instead of at b times the batch strides; or null
   uint32_t nqc;    // query chunks per (batch, head)
   uint32_t total;  // workgroups
   uint32_t nqc_magic, h_magic;  // floor(2^32 / nqc), floor(2^32 / H) (0 for a divisor of 1): divisions without a divide
@@ -75,6 +75,13 @@ struct AttnParams {
   int32_t pair_blocks;
   uint32_t nqg, nqg_magic, total_g;
 };
+
+// First row of (sample b, head h).
+template <bool COMPACT, typename T>
+__device__ __forceinline__ T* head_rows(T* base, const int64_t (&strides)[4], const AttnParams& p, int b, int h) {
+  const int64_t row0 = COMPACT ? p.row_offsets[b] * strides[2] : b * strides[0];
+  return base + row0 + h * strides[1];
+}
 
 // x / d and x % d for a divisor known to the host: q = mulhi(x, floor(2^32 / d)) is at most two short of the quotient.
 __device__ __forceinline__ void magic_divmod(uint32_t x, uint32_t d, uint32_t magic, uint32_t& q, uint32_t& r) {
@@ -176,7 +183,8 @@ struct QueryFeatureFactors {
   }
 };
 
-template <typename T, int DP, bool CAUSAL, bool SCALED, bool MASKED, bool DROPOUT = false>
+// COMPACT: samples are addressed by row_offsets.
+template <typename T, int DP, bool CAUSAL, bool SCALED, bool MASKED, bool DROPOUT = false, bool COMPACT = false>
 __global__ __launch_bounds__(kThreads) void flash_attn_fwd_kernel(const AttnParams p) {
   static_assert(!(DROPOUT && SCALED && !MASKED), "dropout comes with the masks of the training path, not with row factors");
   static_assert(!(MASKED && CAUSAL), "a structured mask carries its own causal triangle");
@@ -208,10 +216,10 @@ __global__ __launch_bounds__(kThreads) void flash_attn_fwd_kernel(const AttnPara
   const int l32 = lane % 32;
   const int hh = lane / 32;
 
-  const T* qb = static_cast<const T*>(p.q) + b * p.qs[0] + h * p.qs[1];
-  const T* kb = static_cast<const T*>(p.k) + b * p.ks[0] + h * p.ks[1];
-  const T* vb = static_cast<const T*>(p.v) + b * p.vs[0] + h * p.vs[1];
-  T* ob = static_cast<T*>(p.o) + b * p.os[0] + h * p.os[1];
+  const T* qb = head_rows<COMPACT>(static_cast<const T*>(p.q), p.qs, p, b, h);
+  const T* kb = head_rows<COMPACT>(static_cast<const T*>(p.k), p.ks, p, b, h);
+  const T* vb = head_rows<COMPACT>(static_cast<const T*>(p.v), p.vs, p, b, h);
+  T* ob = head_rows<COMPACT>(static_cast<T*>(p.o), p.os, p, b, h);
 
   int len = p.Tk;
   if (p.key_lengths != nullptr) {
@@ -1353,19 +1361,20 @@ __global__ __launch_bounds__(kSparseWaves * kWave) void flash_attn_fwd_sparse_ke
   }
 }
 
+// Whether the direct-transfer kernel can address the tensors - 32-bit source offsets with a 24-bit row multiply: row strides below
+// 4 M elements, sequences below 2^31 bytes (the same for the query and output rows).
+bool small_offsets(const AttnParams& p) {
+  return p.ks[2] < (1 << 22) && p.vs[2] < (1 << 22) && p.Tk < (1 << 22) && static_cast<int64_t>(p.Tk) * p.ks[2] * 2 < (1ll << 31) &&
+         static_cast<int64_t>(p.Tk) * p.vs[2] * 2 < (1ll << 31) && p.qs[2] >= 0 && p.os[2] >= 0 && p.qs[2] < (1 << 22) &&
+         p.os[2] < (1 << 22) && p.Tq < (1 << 22) && static_cast<int64_t>(p.Tq) * p.qs[2] * 2 < (1ll << 31) &&
+         static_cast<int64_t>(p.Tq) * p.os[2] * 2 < (1ll << 31);
+}
+
 template <typename T, int DP>
 void launch(const AttnParams& p, bool causal, bool register_staging, hipStream_t s) {
   const bool scaled = p.q_row_scale != nullptr || p.k_row_scale != nullptr || p.q_col_scale != nullptr;
   // TAAC_ATTN_REGISTER_STAGING keeps the general kernel for full head dims too (comparison route of the caller).
   const bool dma_staging = !register_staging;
-  // 32-bit source offsets with a 24-bit row multiply: row strides below 8 M elements, sequences below 2^31 bytes
-  // (the same for the query and output rows)
-  const bool small_offsets = p.ks[2] < (1 << 22) && p.vs[2] < (1 << 22) && p.Tk < (1 << 22) &&
-                             static_cast<int64_t>(p.Tk) * p.ks[2] * 2 < (1ll << 31) &&
-                             static_cast<int64_t>(p.Tk) * p.vs[2] * 2 < (1ll << 31) &&
-                             p.qs[2] >= 0 && p.os[2] >= 0 && p.qs[2] < (1 << 22) && p.os[2] < (1 << 22) && p.Tq < (1 << 22) &&
-                             static_cast<int64_t>(p.Tq) * p.qs[2] * 2 < (1ll << 31) &&
-                             static_cast<int64_t>(p.Tq) * p.os[2] * 2 < (1ll << 31);
   if constexpr (DP == 32 || DP == 64) {
     if (p.compact_keys != nullptr) {  // the entry point has checked the shape
       const int64_t groups = static_cast<int64_t>((p.Tq + 31) / 32) * ((static_cast<int64_t>(p.B) * p.H + kSparseWaves - 1) / kSparseWaves);
@@ -1380,7 +1389,7 @@ void launch(const AttnParams& p, bool causal, bool register_staging, hipStream_t
     // structure bits ride along when they are all there is to the mask: per sample, no validity or self rows, no chunk map
     const bool structure_only = p.struct_bits != nullptr && p.valid_bits == nullptr && p.self_bits == nullptr &&
                                 p.block_any == nullptr;
-    if (p.d == DP && (p.struct_bits == nullptr || structure_only) && dma_staging && small_offsets && p.drop_mask == nullptr) {
+    if (p.d == DP && (p.struct_bits == nullptr || structure_only) && dma_staging && small_offsets(p) && p.drop_mask == nullptr) {
       if (structure_only && scaled)
         hipLaunchKernelGGL((flash_attn_fwd_dma_kernel<T, DP, false, true, true>), dim3(p.total_g), dim3(kThreads), 0, s, p);
       else if (structure_only)
@@ -1394,6 +1403,12 @@ void launch(const AttnParams& p, bool causal, bool register_staging, hipStream_t
       else
         hipLaunchKernelGGL((flash_attn_fwd_dma_kernel<T, DP, false, false, false>), dim3(p.total_g), dim3(kThreads), 0, s, p);
       return;
+    }
+    if constexpr (std::is_same<T, bf16_t>::value) {
+      if (p.row_offsets != nullptr) {  // samples too long for 32-bit offsets; the entry point has checked that there is no mask
+        hipLaunchKernelGGL((flash_attn_fwd_kernel<T, DP, false, false, false, false, true>), dim3(p.total), dim3(kThreads), 0, s, p);
+        return;
+      }
     }
   }
   if (p.drop_mask != nullptr && p.struct_bits != nullptr)
@@ -1637,6 +1652,14 @@ int attention_entry(const char* name, const void* q, const void* k, const void* 
   p.nqg_magic = magic_of(p.nqg);
   p.total_g = p.nqg * static_cast<uint32_t>(B) * static_cast<uint32_t>(H);
 
+  // The compact layout has two kernels: direct transfers (with or without structure bits), and the general one without a mask.
+  if (row_offsets != nullptr &&
+      (dtype != TAAC_BF16 || (d != 32 && d != 64) || is_causal != 0 || register_staging || drop_mask != nullptr ||
+       q_row_scale != nullptr || k_row_scale != nullptr || q_col_scale != nullptr || mask.valid_bits != nullptr ||
+       mask.self_bits != nullptr || mask.block_any != nullptr || mask.compact_keys != nullptr ||
+       (mask.struct_bits != nullptr && !small_offsets(p))))
+    return set_error(TAAC_ERR_UNSUPPORTED, "%s: no kernel addresses samples by their row offsets in this form", name);
+
   hipStream_t s = as_stream(stream);
   if (dtype == TAAC_BF16)
     launch_dp<bf16_t>(p, is_causal != 0, register_staging, s);
@@ -1652,7 +1675,6 @@ namespace taac {
 int attention_compact_fwd(const char* name, const void* qk, const void* v, int64_t ld_qk, int64_t ld_v, const int32_t* lengths,
                           const int32_t* row_offsets, const uint32_t* struct_bits, int64_t struct_stride, void* o, int64_t ld_o,
                           float* lse, int32_t B, int32_t H, int32_t T, int32_t dh, hipStream_t s) {
-  if (dh != 32 && dh != 64) return set_error(TAAC_ERR_UNSUPPORTED, "%s: head dims 32 and 64", name);
   MaskArgs mask;
   mask.struct_bits = struct_bits;
   mask.struct_stride = struct_stride;

@@ -148,3 +148,60 @@ def test_a_head_without_bias_trains(device):
     want.sum().backward()
     for name, parameter in none.named_parameters():
         assert torch.equal(parameter.grad, zero.get_parameter(name).grad), name
+
+
+def _network(d_model, heads, d_ff, n_blocks, seed):
+    """A network whose parameters are bf16 values, and its parameters as float64 leaves."""
+    g = torch.Generator().manual_seed(seed)
+    model = PCVRBackbone(d_model=d_model, num_heads=heads, d_ff=d_ff, n_blocks=n_blocks)
+    with torch.no_grad():
+        for parameter in model.parameters():
+            spread = torch.randn(parameter.shape, generator=g)
+            center = 1.0 if parameter.ndim == 1 and parameter.mean() > 0.5 else 0.0
+            parameter.copy_((center + spread * (0.1 if parameter.ndim == 1 else parameter.shape[1] ** -0.5)).to(torch.bfloat16))
+    return model, {name: value.detach().double().requires_grad_(True) for name, value in model.named_parameters()}
+
+
+def _oracle_hidden(reference, emb, lengths, heads, n_blocks):
+    padding = torch.arange(emb.shape[1])[None, :] >= lengths[:, None]
+    mask = (~padding)[:, None, None, :].expand(emb.shape[0], 1, emb.shape[1], emb.shape[1])
+    x = emb
+    for i in range(n_blocks):
+        block = {name.split(".", 2)[2]: value for name, value in reference.items() if name.startswith(f"blocks.{i}.")}
+        x, _ = oracle.interaction_block(x, padding, mask, block, num_heads=heads)
+    return x * (~padding).double().unsqueeze(-1)
+
+
+def test_samples_beyond_the_offsets_of_the_direct_transfers(device):
+    """q | k | v rows of 768 values and 1 398 102 positions: the offsets inside a sample may need more than 31 bits, so the
+    attention takes its general kernels. Every sample is still its own (few valid tokens, so that the oracle stays small)."""
+    tokens, short, lengths = 1_398_102, 71, torch.tensor([71, 33], dtype=torch.int32)
+    if torch.cuda.get_device_properties(device).total_memory < 100 * 2 ** 30:
+        pytest.skip("about 30 GB of tensors")
+    g = torch.Generator().manual_seed(11)
+    model, reference = _network(256, 4, 32, 1, seed=12)
+    model = model.to(torch.bfloat16).to(device).train()
+    emb = torch.randn(2, short, 256, generator=g).to(torch.bfloat16)
+    grad = torch.randn(2, short, 256, generator=g).to(torch.bfloat16)
+    emb_d = torch.zeros(2, tokens, 256, dtype=torch.bfloat16, device=device)
+    emb_d[:, :short] = emb.to(device)
+    emb_d.requires_grad_(True)
+    _, hidden = model(emb_d, lengths.to(device), return_hidden=True)
+    grad_d = torch.zeros_like(hidden)
+    grad_d[:, :short] = grad.to(device)
+    hidden.backward(grad_d)
+    del grad_d
+
+    emb_r = emb.double().requires_grad_(True)
+    want = _oracle_hidden(reference, emb_r, lengths, 4, 1)
+    want.backward(grad.double())
+    for b in range(2):
+        _near(f"hidden of sample {b}", hidden[b, :short], want[b].detach(), 1)
+        _near(f"tokens of sample {b}", emb_d.grad[b, :short], emb_r.grad[b], 1)
+    assert not hidden[:, short:].any() and not emb_d.grad[:, short:].any()
+    for name, parameter in model.named_parameters():
+        if not name.startswith("head."):
+            _near(name, parameter.grad, reference[name].grad, 1)
+    del hidden, emb_d, parameter
+    model.zero_grad(set_to_none=True)
+    torch.cuda.empty_cache()
