@@ -24,7 +24,7 @@ from taac_2026_amd.accelerators.attention import StructuredAttentionMask, front_
 from taac_2026_amd.accelerators.linear import (attention_out_ffn, front_rows, norm_linear, qkv_projection, silu_mlp,
                                                swiglu_ffn, swiglu_ffn_backward_supported, swiglu_ffn_dropout, valid_rows)
 from taac_2026_amd.accelerators.tensor_validation import require_cuda_tensors, require_inference
-from taac_2026_amd.modeling.block_training import (InteractionStackFunction, run_training_block, run_training_stack,
+from taac_2026_amd.modeling.block_training import (InteractionStackFunction, block_form, run_training_block, run_training_stack,
                                                    training_route_applies, uniform_parameters)
 from taac_2026_amd.modeling.normalization import RMSNorm
 from taac_2026_amd.modeling.sequence import scaled_dot_product_attention
@@ -612,34 +612,63 @@ class PCVRBackbone(nn.Module):
 
     def _forward_training(self, emb: torch.Tensor, key_lengths: torch.Tensor, return_hidden: bool):
         """The same network under autograd: blocks and readout as one function over the valid tokens
-        (:class:`InteractionStackFunction`), without a host synchronisation."""
+        (:class:`InteractionStackFunction`), without a host synchronisation. Blocks that differ in their hidden size or their query /
+        key norms are one function per run of equal ones, and a head of another form than ``Linear(D, 1)`` reads the final hidden
+        state."""
         name = "hip PCVRBackbone"
         if emb.ndim != 3 or emb.shape[-1] != self.d_model or emb.dtype != torch.bfloat16:
             raise ValueError(f"{name} expects bfloat16 embeddings of shape (batch, tokens, {self.d_model})")
         if key_lengths.shape != (emb.shape[0],):
             raise ValueError("key_lengths must have shape (batch,)")
         head_dim = self.d_model // self.num_heads
-        if self.rope_base is not None or self.d_model not in (128, 256) or head_dim not in (32, 64) or self.d_ff % 32 != 0 \
+
+        def covered(d_ff: int) -> bool:
+            return d_ff % 32 == 0 and swiglu_ffn_backward_supported(self.d_model, d_ff)
+
+        if key_lengths.dtype != torch.int32 or not key_lengths.is_contiguous():
+            key_lengths = key_lengths.to(torch.int32).contiguous()
+        params: list[torch.Tensor | None] = []
+        runs: list[list] = []  # [form, number of blocks]
+        for block in self.blocks:
+            own = [_held(_part(block, part), parameter) for part, parameter in self._TRAINED]
+            form = block_form(name, own, self.d_model, emb.device)
+            params += own
+            if runs and runs[-1][0] == form:
+                runs[-1][1] += 1
+            else:
+                runs.append([form, 1])
+        if self.rope_base is not None or self.d_model not in (128, 256) or head_dim not in (32, 64) \
                 or any(p.dtype not in (torch.bfloat16, torch.float32) for p in self.parameters()) \
-                or not swiglu_ffn_backward_supported(self.d_model, self.d_ff):
+                or not all(map(covered, {self.d_ff, *(form[0] for form, _ in runs)})):
             raise RuntimeError(f"{name}: the training route covers bf16 (or float32 master) parameters, d_model 128 / 256, "
                                "head dims 32 / 64, d_ff a multiple of 32 within the backward kernel's bound "
                                "(taac_swiglu_ffn_bwd_packed_bytes) and no rotary embedding")
-        if key_lengths.dtype != torch.int32 or not key_lengths.is_contiguous():
-            key_lengths = key_lengths.to(torch.int32).contiguous()
-        if emb.numel() == 0 or len(self.blocks) == 0:  # nothing in front of the readout
+        if emb.numel() == 0 or not runs:  # nothing in front of the readout
             valid = (torch.arange(emb.shape[1], device=emb.device)[None, :] < key_lengths[:, None]).to(emb.dtype).unsqueeze(-1)
-            pooled = (emb * valid).sum(dim=1) / valid.sum(dim=1).clamp_min(1.0)
-            logits = torch.nn.functional.linear(pooled, _bf16(self.head.weight), _bf16(self.head.bias)).squeeze(-1)
-            return (torch.sigmoid(logits.float()), emb * valid) if return_hidden else torch.sigmoid(logits.float())
-        params: list[torch.Tensor | None] = []
-        for block in self.blocks:
-            params += [_held(_part(block, part), parameter) for part, parameter in self._TRAINED]
-        params += [self.head.weight, self.head.bias]
-        hidden, _, probabilities = InteractionStackFunction.apply(
-            emb, key_lengths, None,
-            (self.num_heads, self.eps, self.eps, self.eps, True, bool(return_hidden), True, False, True), *uniform_parameters(params))
+            hidden = emb * valid
+            probabilities = self._read_out(hidden, key_lengths)
+            return (probabilities, hidden) if return_hidden else probabilities
+        *params, head_w, head_b = uniform_parameters([*params, self.head.weight, self.head.bias])
+        rides = head_w.shape == (1, self.d_model) and (head_b is None or head_b.shape == (1,)) and head_w.device == emb.device \
+            and (head_b is None or head_b.device == emb.device)
+        hidden, first = emb, 0
+        for i, (_, count) in enumerate(runs):
+            head = (head_w, head_b) if rides and i == len(runs) - 1 else ()
+            hidden, _, probabilities = InteractionStackFunction.apply(
+                hidden, key_lengths, None,
+                (self.num_heads, self.eps, self.eps, self.eps, True, not head or bool(return_hidden), True, False, bool(head)),
+                *params[first:first + count * len(self._TRAINED)], *head)
+            first += count * len(self._TRAINED)
+        if not rides:
+            probabilities = self._read_out(hidden, key_lengths)
         return (probabilities, hidden) if return_hidden else probabilities
+
+    def _read_out(self, hidden: torch.Tensor, key_lengths: torch.Tensor) -> torch.Tensor:
+        """Masked mean (``masked_mean``, modeling/sequence.py:54-60), head and sigmoid as tensor operations; padded rows are zeros."""
+        count = key_lengths.clamp(0, hidden.shape[1]).to(hidden.dtype).unsqueeze(-1)
+        pooled = hidden.sum(dim=1) / count.clamp_min(1.0)
+        logits = torch.nn.functional.linear(pooled, _bf16(self.head.weight), _bf16(self.head.bias)).squeeze(-1)
+        return torch.sigmoid(logits.float())
 
     FP8_MAXIMA = ("qkv.weight", "out.weight", "up.weight", "down.weight", "attn_norm", "attention", "ffn_norm", "hidden")
 

@@ -18,6 +18,7 @@ with self-only queries.
 from __future__ import annotations
 
 import ctypes
+import functools
 import importlib
 
 import torch
@@ -388,6 +389,36 @@ class InteractionStackFunction(torch.autograd.Function):
         return (grad_tokens, None, None, None, *grads)
 
 
+_OPTIONAL = (2, 4, 7, 9, 10, 11)  # slots a block may do without (the query and key norm weights only together)
+
+
+@functools.lru_cache(maxsize=64)
+def _block_shapes(width: int, hidden: int) -> tuple:
+    """Shapes of a block's parameters, in the order of taac_block_weights."""
+    return ((width,), (3 * width, width), (3 * width,), (width, width), (width,), (width,), (2 * hidden, width), (2 * hidden,),
+            (width, hidden), (width,), (width,), (width,))
+
+
+def block_form(name: str, params: list, width: int, device: torch.device) -> tuple[int, bool]:
+    """``(F, query / key norms)`` of a block of ``width`` features. The native call takes addresses, so a parameter of another shape
+    or on another device than ``device`` is refused here."""
+    down = params[8]
+    hidden = down.shape[1] if down is not None and down.ndim == 2 else 0
+    ordinal = -1 if device.type == "cpu" else device.index
+    for slot, (p, shape) in enumerate(zip(params, _block_shapes(width, hidden))):
+        if p is None:
+            if slot not in _OPTIONAL:
+                raise ValueError(f"{name}: a block has no weight where its layers need one")
+        elif p.shape != shape:
+            raise ValueError(f"{name}: a parameter of shape {tuple(p.shape)} does not fit a block of {width} features "
+                             f"and {hidden} hidden units")
+        elif p.get_device() != ordinal:
+            raise RuntimeError(f"{name} requires all tensors to live on the same device")
+    if (params[10] is None) != (params[11] is None):
+        raise ValueError(f"{name}: query and key norm come together")
+    return hidden, params[10] is not None
+
+
 def uniform_parameters(params: list) -> list:
     """``params`` as they are when all are bf16 or all float32; else rounded to bf16 (autograd carries the gradients back)."""
     dtypes = {p.dtype for p in params if p is not None}
@@ -454,6 +485,8 @@ def run_training_block(block, tokens: torch.Tensor, key_lengths: torch.Tensor | 
                        mask=None, padding_mask: torch.Tensor | None = None):
     """One block through :class:`InteractionStackFunction` (:class:`InteractionBlockFunction` under self-only queries)."""
     attention, ffn = block.attention, block.ffn
+    params = _block_parameters(block)
+    block_form("hip UnifiedInteractionBlock", params, tokens.shape[-1], tokens.device)
     if mask is not None and mask.query_self is not None:
         def bf16(parameter):
             return parameter if parameter is None or parameter.dtype == torch.bfloat16 else parameter.to(torch.bfloat16)
@@ -461,25 +494,28 @@ def run_training_block(block, tokens: torch.Tensor, key_lengths: torch.Tensor | 
         return InteractionBlockFunction.apply(
             tokens, mask, padding_mask, bool(return_attention_tokens), attention.num_heads, block.attn_norm.eps,
             block.ffn_norm.eps, ffn.gate_first, 1e-6 if attention.query_norm is None else attention.query_norm.eps,
-            *map(bf16, _block_parameters(block)))
+            *map(bf16, params))
     index = None if mask is None else _RowIndex.for_mask(mask, padding_mask, tokens.shape[1])
     output, attn_tokens, _ = InteractionStackFunction.apply(
         tokens, key_lengths if index is None else index.lengths, index,
-        (*_block_config(block), True, False, bool(return_attention_tokens), False), *uniform_parameters(_block_parameters(block)))
+        (*_block_config(block), True, False, bool(return_attention_tokens), False), *uniform_parameters(params))
     return output, attn_tokens
 
 
 def run_training_stack(blocks, tokens: torch.Tensor, mask, padding_mask: torch.Tensor) -> torch.Tensor | None:
     """All ``blocks`` as one function, or None when they do not form one (different settings, hooks, self-only queries)."""
-    config = _block_config(blocks[0])
+    config, form = _block_config(blocks[0]), None
     params: list = []
     for block in blocks:
         if (block._forward_hooks or block._forward_pre_hooks or block._backward_hooks or block._backward_pre_hooks
                 or _block_config(block) != config):
             return None
-        params += _block_parameters(block)
-        if params[-_SLOTS + 8].shape != params[8].shape or (params[-1] is None) != (params[11] is None):
+        own = _block_parameters(block)
+        own_form = block_form("hip UnifiedInteractionBlock", own, tokens.shape[-1], tokens.device)
+        if form not in (None, own_form):
             return None
+        form = own_form
+        params += own
     index = _RowIndex.for_mask(mask, padding_mask, tokens.shape[1])
     return InteractionStackFunction.apply(tokens, index.lengths, index, (*config, True, False, False, False),
                                           *uniform_parameters(params))[0]

@@ -205,3 +205,67 @@ def test_samples_beyond_the_offsets_of_the_direct_transfers(device):
     del hidden, emb_d, parameter
     model.zero_grad(set_to_none=True)
     torch.cuda.empty_cache()
+
+
+def test_a_head_of_several_outputs_trains(device):
+    """``Linear(D, 3)`` in the place of the head: probabilities and gradients against the oracle, every row of the head's too."""
+    g = torch.Generator().manual_seed(21)
+    tokens, lengths = 40, torch.tensor([40, 0, 17, 33], dtype=torch.int32)
+    model, reference = _network(128, 4, 128, 2, seed=22)
+    model.head = torch.nn.Linear(128, 3)
+    with torch.no_grad():
+        for parameter in model.head.parameters():
+            parameter.copy_((0.3 * torch.randn(parameter.shape, generator=g)).to(torch.bfloat16))
+    reference.update({f"head.{name}": value.detach().double().requires_grad_(True) for name, value in model.head.named_parameters()})
+    emb, grad = torch.randn(4, tokens, 128, generator=g).to(torch.bfloat16), torch.randn(4, 3, generator=g)
+    model = model.to(torch.bfloat16).to(device).train()
+    emb_d, emb_r = emb.to(device).requires_grad_(True), emb.double().requires_grad_(True)
+    got = model(emb_d, lengths.to(device))
+    got.backward(grad.to(device))
+    want = _oracle_hidden(reference, emb_r, lengths, 4, 2).sum(1) / lengths.clamp_min(1).double().unsqueeze(-1)
+    want = torch.sigmoid(F.linear(want, reference["head.weight"], reference["head.bias"]))
+    want.backward(grad.double())
+    assert got.shape == (4, 3)
+    _near("p", got, want.detach(), 2)
+    _near("tokens", emb_d.grad, emb_r.grad, 2)
+    for name, parameter in model.named_parameters():
+        _near(name, parameter.grad, reference[name].grad, 2)
+    for row in range(3):
+        _near(f"head.weight[{row}]", model.head.weight.grad[row], reference["head.weight"].grad[row], 2)
+
+
+def test_blocks_of_different_hidden_sizes_train(device):
+    """A network whose middle block was replaced by a narrower one: each block with its own shapes."""
+    g = torch.Generator().manual_seed(23)
+    tokens, lengths = 45, torch.tensor([45, 0, 17, 33, 1], dtype=torch.int32)
+    model, reference = _network(256, 8, 256, 3, seed=24)
+    other, _ = _network(256, 8, 96, 1, seed=25)
+    model.blocks[1] = other.blocks[0]
+    reference = {name: value.detach().double().requires_grad_(True) for name, value in model.named_parameters()}
+    emb, grad = torch.randn(5, tokens, 256, generator=g).to(torch.bfloat16), torch.randn(5, generator=g)
+    model = model.to(torch.bfloat16).to(device).train()
+    emb_d, emb_r = emb.to(device).requires_grad_(True), emb.double().requires_grad_(True)
+    got, hidden = model(emb_d, lengths.to(device), return_hidden=True)
+    grad_hidden = torch.randn(5, tokens, 256, generator=g).to(torch.bfloat16)
+    torch.autograd.backward([got, hidden], [grad.to(device), grad_hidden.to(device)])
+    want_hidden = _oracle_hidden(reference, emb_r, lengths, 8, 3)
+    pooled = want_hidden.sum(1) / lengths.clamp_min(1).double().unsqueeze(-1)
+    want = torch.sigmoid(F.linear(pooled, reference["head.weight"], reference["head.bias"]).squeeze(-1))
+    torch.autograd.backward([want, want_hidden], [grad.double(), grad_hidden.double()])
+    _near("p", got, want.detach(), 3)
+    _near("hidden", hidden, want_hidden.detach(), 3)
+    _near("tokens", emb_d.grad, emb_r.grad, 3)
+    for name, parameter in model.named_parameters():
+        _near(name, parameter.grad, reference[name].grad, 3)
+
+
+def test_a_layer_of_another_shape_is_refused(device):
+    model = PCVRBackbone(d_model=128, num_heads=4, d_ff=128, n_blocks=2)
+    model.blocks[1].up = torch.nn.Linear(128, 2 * 96)  # narrower than its down projection
+    model = model.to(torch.bfloat16).to(device).train()
+    lengths = torch.tensor([5, 0], dtype=torch.int32, device=device)
+    with pytest.raises(ValueError, match="does not fit a block"):
+        model(torch.zeros(2, 8, 128, dtype=torch.bfloat16, device=device), lengths)
+    model.blocks[1].up = torch.nn.Linear(128, 2 * 128).to(torch.bfloat16)  # left on the host
+    with pytest.raises(RuntimeError, match="same device"):
+        model(torch.zeros(2, 8, 128, dtype=torch.bfloat16, device=device), lengths)

@@ -222,3 +222,33 @@ def test_hash_compress_ids_against_the_rule_stated_per_element():
     assert got.max().item() <= 8 and (got[values > 0] >= 1).all()
     assert hash_compress_ids(values, 0).tolist() == [[0] * values.shape[1]]
     assert hash_compress_ids(values.to(torch.int32)[:, :10], 3).dtype == torch.int32
+
+
+def test_parameters_that_do_not_form_a_block_are_refused():
+    """The training route hands addresses to the library: shapes and devices are looked at first."""
+    from taac_2026_amd.modeling.block_training import block_form
+
+    cpu, width, hidden = torch.device("cpu"), 128, 96
+    shapes = [(width,), (3 * width, width), (3 * width,), (width, width), (width,), (width,), (2 * hidden, width), (2 * hidden,),
+              (width, hidden), (width,), (width,), (width,)]
+    params = [torch.empty(shape, dtype=torch.bfloat16) for shape in shapes]
+    assert block_form("block", params, width, cpu) == (hidden, True)
+    plain = [None if slot in (2, 4, 7, 9, 10, 11) else p for slot, p in enumerate(params)]
+    assert block_form("block", plain, width, cpu) == (hidden, False)
+    for slot, shape in enumerate(shapes):
+        wrong = list(params)
+        wrong[slot] = torch.empty((shape[0] - 32, *shape[1:]))
+        with pytest.raises(ValueError, match="does not fit a block"):
+            block_form("block", wrong, width, cpu)
+        wrong[slot] = None
+        if plain[slot] is not None or slot in (10, 11):
+            with pytest.raises(ValueError):
+                block_form("block", wrong, width, cpu)
+        else:
+            assert block_form("block", wrong, width, cpu) == (hidden, True)
+    narrow = list(params)
+    narrow[8] = torch.empty(width, hidden - 32)  # the down projection of a narrower feed-forward
+    with pytest.raises(ValueError, match="does not fit a block"):
+        block_form("block", narrow, width, cpu)
+    with pytest.raises(RuntimeError, match="same device"):
+        block_form("block", params, width, torch.device("meta", 0))
