@@ -84,13 +84,11 @@ __device__ __forceinline__ void linear_pack_piece(const TW* __restrict__ w, bf16
 // Feed-forward backward (ffn_bwd.hip). Blob: step s (32 hidden units), sub-step u (k-steps 8 u .. 8 u + 7) holds fragments (block b, k-step 8 u + j) at index
 // b * 8 + j; block 0 = rows 32 s .. of the first half of w_up, block 1 = the same rows of its second half, block 2 =
 // columns 32 s .. of w_down (rows of its transpose). Lane (l32, hh) of a fragment holds k = 16 ks + 8 hh .. + 7 of row l32.
-// norm_w (optional, [D]): weight of the RMSNorm in front of the up projection, folded into blocks 0 and 1.
 constexpr int kBwdUnits = 32;   // hidden units per step
 constexpr int kBwdSubK = 8;     // k-steps (of 16 features) per sub-step
 template <typename TW>
 __device__ __forceinline__ void ffn_bwd_pack_piece(const TW* __restrict__ w_up, const TW* __restrict__ w_down,
-                                                   bf16x8* __restrict__ packed, int D, int F, int64_t gid,
-                                                   const TW* __restrict__ norm_w = nullptr) {
+                                                   bf16x8* __restrict__ packed, int D, int F, int64_t gid) {
   const int NSUB = D / 16 / kBwdSubK, NFRAG = 3 * kBwdSubK;
   const int lane = static_cast<int>(gid % 64);
   const int f = static_cast<int>((gid / 64) % NFRAG);
@@ -103,11 +101,6 @@ __device__ __forceinline__ void ffn_bwd_pack_piece(const TW* __restrict__ w_up, 
   bf16x8 v;
   if (b < 2) {
     v = weight_piece(w_up + (b * static_cast<int64_t>(F) + unit) * D + k0);
-    if (norm_w != nullptr) {
-      const bf16x8 g = weight_piece(norm_w + k0);
-#pragma unroll
-      for (int e = 0; e < 8; ++e) v[e] = static_cast<bf16_t>(static_cast<float>(v[e]) * static_cast<float>(g[e]));
-    }
   } else {
 #pragma unroll
     for (int e = 0; e < 8; ++e) v[e] = static_cast<bf16_t>(w_down[static_cast<int64_t>(k0 + e) * F + unit]);

@@ -34,7 +34,7 @@ inline int64_t align256(int64_t v) { return (v + 255) & ~static_cast<int64_t>(25
 // ---- weights of a block, as the kernels read them -----------------------------------------------------------------------
 struct PackedBlock {
   int64_t qkv, out, ffn;          // forward blobs (norm weights folded)
-  int64_t ffn_bwd;                // feed-forward backward blob (norm weight folded)
+  int64_t ffn_bwd;                // feed-forward backward blob
   int64_t up_t, qkv_t, out_t;     // [D, 2F] and [D, 3D] row-major transposes, blob of the out projection's transpose
   int64_t vectors;                // bf16: attn_norm D | qkv_bias 3D | out_bias D | ffn_norm D | up_bias 2F | down_bias D | query D | key D
   int64_t bytes;
@@ -170,7 +170,7 @@ __global__ __launch_bounds__(kRowThreads) void train_setup_kernel(const TrainSet
   gid -= d2;
   if (gid < 3 * df) return ffn_pack_piece(up, down, blob(p.pb.ffn), D, F, p.gate_first, gid, ffn_norm, p.fold_act);
   gid -= 3 * df;
-  if (gid < 3 * df) return ffn_bwd_pack_piece(up, down, blob(p.pb.ffn_bwd), D, F, gid, ffn_norm);
+  if (gid < 3 * df) return ffn_bwd_pack_piece(up, down, blob(p.pb.ffn_bwd), D, F, gid);
   gid -= 3 * df;
   int64_t at;
   if (gid < 2 * df) {
@@ -730,7 +730,7 @@ extern "C" int taac_stack_train_bwd(const void* grad_out, const void* grad_attn_
     const taac_block_weights& g = grads[i];
     bf16_t* dx1 = sc.dx1;
     if (have_dy) {
-      if ((rc = ffn_bwd_hidden_count(name, b.x1, b.rstd_ffn, dy, pk + sv.pb.ffn_bwd, v.up_bias, sc.hidden, sc.grad_pre, M, D, F,
+      if ((rc = ffn_bwd_hidden_count(name, b.x1, b.rstd_ffn, v.ffn_norm, dy, pk + sv.pb.ffn_bwd, v.up_bias, sc.hidden, sc.grad_pre, M, D, F,
                                      gate_first != 0, count, s)) != TAAC_OK)
         return rc;
       if ((rc = dgrad_norm(name, sc.grad_pre, true, 2 * F, pk + sv.pb.up_t, b.x1, b.rstd_ffn, v.ffn_norm, dy, dx1, M, D, count, s)) != TAAC_OK)

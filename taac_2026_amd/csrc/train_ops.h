@@ -40,11 +40,11 @@ int attention_compact_bwd(const char* name, const void* qk, const void* v, int64
                           const void* dout, int64_t ld_do, const float* lse, const int32_t* lengths, const int32_t* row_offsets,
                           const uint32_t* struct_bits, int64_t struct_stride, void* dqkv, int64_t ld_dqkv, float* delta, int32_t B,
                           int32_t H, int32_t T, int32_t dh, hipStream_t s);
-// hidden [M, F] and the gradient of the up projection [M, 2F] from x (in front of the norm; rstd its factor) and the gradient dy
-// of the feed-forward output. Both results are in panel order.
-int ffn_bwd_hidden_count(const char* name, const void* x, const float* rstd, const void* dy, const void* packed, const void* b_up,
-                         void* hidden, void* grad_pre, int64_t M, int32_t D, int32_t F, bool gate_first, const int32_t* count,
-                         hipStream_t s);
+// hidden [M, F] and the gradient of the up projection [M, 2F] from x (in front of the norm; rstd its factor, norm_w [D] its weight)
+// and the gradient dy of the feed-forward output. Both results are in panel order.
+int ffn_bwd_hidden_count(const char* name, const void* x, const float* rstd, const void* norm_w, const void* dy, const void* packed,
+                         const void* b_up, void* hidden, void* grad_pre, int64_t M, int32_t D, int32_t F, bool gate_first,
+                         const int32_t* count, hipStream_t s);
 
 // dx = dres + d rmsnorm(x) applied to dy W (train_dense.hip): dy [M, K], w_t [D, K] (the layer's weight transposed), x [M, D] the
 // rows in front of the norm, rstd its factor, norm_w [D] its weight. dx may be dres. dy_panels: dy is in panel order.

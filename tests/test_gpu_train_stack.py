@@ -269,3 +269,31 @@ def test_a_layer_of_another_shape_is_refused(device):
     model.blocks[1].up = torch.nn.Linear(128, 2 * 128).to(torch.bfloat16)  # left on the host
     with pytest.raises(RuntimeError, match="same device"):
         model(torch.zeros(2, 8, 128, dtype=torch.bfloat16, device=device), lengths)
+
+
+@pytest.mark.parametrize("d_model,dtype", [(256, torch.bfloat16), (128, torch.float32)])
+def test_the_feed_forward_backward_rounds_no_product_of_two_weights(device, d_model, dtype):
+    """Rows that the norm maps to +-1, a norm weight and up weights whose products all lie 0.3 % above the bf16 value below them: the
+    hidden state of the backward is off by that much wherever the two are multiplied and rounded in front of the product, and the
+    down projection's gradient, which is linear in it, shrinks. Otherwise normalised rows and products are exact and the hidden
+    state is rounded once, 2^-9 of each value at most: no further may the gradient be off along the true one."""
+    g = torch.Generator().manual_seed(31)
+    batch, tokens, d_ff = 40, 65, 256
+    model, _ = _network(d_model, 4, d_ff, 1, seed=32)
+    block = model.blocks[0]
+    with torch.no_grad():
+        for parameter in (block.out.weight, block.out.bias, block.up.bias):
+            parameter.zero_()
+        block.ffn_norm.weight.fill_(1 + 9 / 128)
+        block.up.weight.copy_(torch.where(torch.rand(block.up.weight.shape, generator=g) < 0.5, -1.0, 1.0) * (1 + 7 / 128) / 16)
+    reference = {name: value.detach().double().requires_grad_(True) for name, value in model.named_parameters()}
+    emb = torch.where(torch.rand(batch, tokens, d_model, generator=g) < 0.5, -1.0, 1.0).to(torch.bfloat16)
+    grad = torch.randn(batch, tokens, d_model, generator=g).to(torch.bfloat16)
+    lengths = torch.full((batch,), tokens, dtype=torch.int32)
+    model = model.to(dtype).to(device).train()
+    _, hidden = model(emb.to(device), lengths.to(device), return_hidden=True)
+    hidden.backward(grad.to(device))
+    _oracle_hidden(reference, emb.double(), lengths, 4, 1).backward(grad.double())
+    got, want = model.blocks[0].down.weight.grad.cpu().double(), reference["blocks.0.down.weight"].grad
+    along = float((got * want).sum() / (want * want).sum())
+    assert abs(along - 1.0) <= 2.0 ** -9, along
