@@ -522,20 +522,13 @@ class PCVRBackbone(nn.Module):
         self.blocks = nn.ModuleList(_PlainBlock(d_model, num_heads, d_ff, qk_norm) for _ in range(n_blocks))
         self.head = nn.Linear(d_model, 1)
         self.reset_parameters()
-        self._workspace: torch.Tensor | None = None
+        self._fp8_maxima: torch.Tensor | None = None
 
     def reset_parameters(self) -> None:
         for module in self.modules():
             if isinstance(module, nn.Linear):
                 nn.init.xavier_uniform_(module.weight)
                 nn.init.zeros_(module.bias)
-
-    def _get_workspace(self, nbytes: int, device: torch.device) -> torch.Tensor:
-        ws = self._workspace
-        if ws is None or ws.numel() < nbytes or ws.device != device:
-            ws = torch.empty(nbytes, dtype=torch.uint8, device=device)
-            self._workspace = ws
-        return ws
 
     def forward(self, emb: torch.Tensor, key_lengths: torch.Tensor, *, return_hidden: bool = False,
                 dense_tokens: bool = False, split_out_ffn: bool = False, fp8: bool = False, row_major_qkv: bool = False):
@@ -583,7 +576,10 @@ class PCVRBackbone(nn.Module):
             table = rope_table(tokens, self.d_model // self.num_heads, self.rope_base, torch.bfloat16, emb.device)
 
         nbytes = library.taac_backbone_workspace_bytes(batch, tokens, self.d_model, self.d_ff, len(self.blocks))
-        workspace = self._get_workspace(int(nbytes), emb.device)
+        self._fp8_maxima = None  # (holds the workspace of the last fp8 forward)
+        # From the allocator's pool of the current stream on every call, not held by the module: calls on other streams or threads,
+        # which may run at the same time, have theirs (it holds arrival counters besides the activations).
+        workspace = torch.empty(int(nbytes), dtype=torch.uint8, device=emb.device)
         hidden = torch.empty_like(emb) if return_hidden else None
         flags = ((_native.BACKBONE_DENSE_TOKENS if dense_tokens else 0) | (_native.BACKBONE_SPLIT_OUT_FFN if split_out_ffn else 0)
                  | (_native.BACKBONE_FP8 if fp8 else 0) | (_native.BACKBONE_ROW_MAJOR_QKV if row_major_qkv else 0))
@@ -596,7 +592,6 @@ class PCVRBackbone(nn.Module):
             _native.current_stream(emb.device),
         )
         _native.check(status, "backbone_fwd")
-        self._fp8_maxima = None
         if fp8:
             offset = library.taac_backbone_fp8_scales_offset(batch, tokens, self.d_model, self.d_ff, len(self.blocks))
             count = (len(self.blocks) + 1) * 8
@@ -676,9 +671,10 @@ class PCVRBackbone(nn.Module):
         """Per block, the per-tensor maxima (scale = maximum / 448) the last ``fp8=True`` forward quantised with: the four
         weights, the two normalised streams, the attention output and the gated hidden state (host tensors; waits for
         the forward)."""
-        if getattr(self, "_fp8_maxima", None) is None:
+        maxima = getattr(self, "_fp8_maxima", None)
+        if maxima is None:
             raise RuntimeError("hip PCVRBackbone: no fp8 forward has run on this module")
-        table = self._fp8_maxima[:len(self.blocks)].cpu()
+        table = maxima[:len(self.blocks)].cpu()
         return [dict(zip(self.FP8_MAXIMA, row)) for row in table]
 
 

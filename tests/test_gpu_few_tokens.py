@@ -3,6 +3,8 @@ kernels that large batches take (a capped grid selects those) and, through them,
 
 from __future__ import annotations
 
+import threading
+
 import pytest
 import torch
 
@@ -118,3 +120,43 @@ def test_backbone_with_hidden_units_divided_over_workgroups(device, test_hooks, 
         for _ in range(3):
             again, h_again = model(emb, lengths, return_hidden=True)
             assert torch.equal(again, p) and torch.equal(h_again, h)
+
+
+def test_calls_in_flight_on_several_streams_do_not_share_memory(device):
+    """One module, two threads with a stream each: every call has the arrival counters, partial sums and activations of its own
+    workspace, so that the results are those of the calls one after the other, bit for bit."""
+    model = PCVRBackbone(d_model=256, num_heads=8, d_ff=1024, n_blocks=2).to(device=device, dtype=torch.bfloat16).eval()
+    g = torch.Generator().manual_seed(9)
+    requests = [(_bf16(g, 1 + i % 3, 100, 256).to(device),
+                 torch.randint(1, 101, (1 + i % 3,), generator=g, dtype=torch.int32).to(device)) for i in range(24)]
+    with torch.no_grad():
+        want = [model(emb, lengths, return_hidden=True) for emb, lengths in requests]
+    torch.cuda.synchronize()
+    got: list = [None] * len(requests)
+
+    def serve(first: int) -> None:
+        with torch.no_grad(), torch.cuda.stream(torch.cuda.Stream(device)):
+            for i in range(first, len(requests), 2):
+                got[i] = model(*requests[i], return_hidden=True)
+            torch.cuda.current_stream(device).synchronize()
+
+    threads = [threading.Thread(target=serve, args=(first,)) for first in range(2)]
+    for thread in threads:
+        thread.start()
+    for thread in threads:
+        thread.join()
+    for (p, hidden), (want_p, want_hidden) in zip(got, want):
+        assert torch.equal(p, want_p) and torch.equal(hidden, want_hidden)
+    # two calls on one stream, the first of which has not run yet, and one on another stream in between
+    busy, other = torch.cuda.Stream(device), torch.cuda.Stream(device)
+    torch.cuda.synchronize()
+    with torch.no_grad():
+        with torch.cuda.stream(busy):
+            torch.cuda._sleep(20_000_000)
+            first = model(*requests[0])
+        with torch.cuda.stream(other):
+            second = model(*requests[1])
+        with torch.cuda.stream(busy):
+            third = model(*requests[2])
+    torch.cuda.synchronize()
+    assert all(torch.equal(p, want[i][0]) for i, p in enumerate((first, second, third)))
