@@ -502,13 +502,20 @@ def run_training_block(block, tokens: torch.Tensor, key_lengths: torch.Tensor | 
     return output, attn_tokens
 
 
+def _called_plainly(block: torch.nn.Module) -> bool:
+    """Whether calling ``block`` does nothing but run its class's ``forward``: no hooks, its own or of all modules, no ``forward`` of
+    the instance, no compiled call."""
+    return not (block._forward_hooks or block._forward_pre_hooks or block._backward_hooks or block._backward_pre_hooks
+                or "forward" in block.__dict__ or block._compiled_call_impl is not None
+                or type(block).__call__ is not torch.nn.Module.__call__ or torch.nn.modules.module._has_any_global_hook())
+
+
 def run_training_stack(blocks, tokens: torch.Tensor, mask, padding_mask: torch.Tensor) -> torch.Tensor | None:
     """All ``blocks`` as one function, or None when they do not form one (different settings, hooks, self-only queries)."""
     config, form = _block_config(blocks[0]), None
     params: list = []
     for block in blocks:
-        if (block._forward_hooks or block._forward_pre_hooks or block._backward_hooks or block._backward_pre_hooks
-                or _block_config(block) != config):
+        if not _called_plainly(block) or _block_config(block) != config:
             return None
         own = _block_parameters(block)
         own_form = block_form("hip UnifiedInteractionBlock", own, tokens.shape[-1], tokens.device)

@@ -297,3 +297,20 @@ def test_the_feed_forward_backward_rounds_no_product_of_two_weights(device, d_mo
     got, want = model.blocks[0].down.weight.grad.cpu().double(), reference["blocks.0.down.weight"].grad
     along = float((got * want).sum() / (want * want).sum())
     assert abs(along - 1.0) <= 2.0 ** -9, along
+
+
+def test_hooks_of_all_modules_and_replaced_forwards_see_every_block_of_a_stack(device):
+    roles = torch.tensor([0, 1, 2, 3, 6, 6, 6, 7]).to(device)
+    blocks = [UnifiedInteractionBlock(128, 4, 1).to(torch.bfloat16).to(device).train() for _ in range(3)]
+    padding = torch.zeros(2, roles.numel(), dtype=torch.bool, device=device)
+    x = torch.randn(2, roles.numel(), 128, device=device).to(torch.bfloat16).requires_grad_(True)
+    mask = MetadataAttentionMask(enabled=True)(padding, roles)
+    seen: list = []
+    handle = torch.nn.modules.module.register_module_forward_hook(lambda module, args, out: seen.append(module))
+    try:
+        run_interaction_blocks(blocks, x, padding, mask)
+    finally:
+        handle.remove()
+    assert [module for module in seen if module in blocks] == blocks
+    blocks[1].forward = lambda tokens, *args, **kwargs: (tokens * 0, None)
+    assert not run_interaction_blocks(blocks[:2], x, padding, mask).any()

@@ -260,3 +260,20 @@ def test_tensors_on_the_host_have_no_stream():
 
     with pytest.raises(ValueError, match="cuda device"):
         _native.current_stream(torch.device("cpu"))
+
+
+def test_a_stack_is_one_function_only_where_its_blocks_are_called_plainly():
+    from taac_2026_amd.api import UnifiedInteractionBlock
+    from taac_2026_amd.modeling.block_training import _called_plainly
+
+    block = UnifiedInteractionBlock(128, 4, 1)
+    assert _called_plainly(block)
+    of_all = torch.nn.modules.module
+    for register in (block.register_forward_hook, block.register_full_backward_pre_hook, of_all.register_module_forward_hook,
+                     of_all.register_module_forward_pre_hook, of_all.register_module_full_backward_hook):
+        handle = register(lambda *args: None)
+        assert not _called_plainly(block)
+        handle.remove()
+        assert _called_plainly(block)
+    block.forward = lambda *args, **kwargs: None
+    assert not _called_plainly(block)
