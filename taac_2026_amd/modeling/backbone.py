@@ -466,7 +466,7 @@ def run_interaction_blocks(blocks, tokens: torch.Tensor, padding_mask: torch.Ten
     ``MetadataAttentionMask`` the row indices and the mask gathered per sample are built by the first block and shared
     by the others. The padding mask must not be modified while the loop runs. With tensors that take a gradient the blocks
     run as one function where ``UnifiedInteractionBlock`` would take its training route."""
-    stream = tokens
+    stream, blocks = tokens, list(blocks)
     if (len(blocks) > 0 and torch.is_grad_enabled() and isinstance(attention_mask, StructuredAttentionMask)
             and attention_mask.query_self is None
             and all(type(block).forward is UnifiedInteractionBlock.forward and not block._fused_route(tokens)

@@ -277,3 +277,15 @@ def test_a_stack_is_one_function_only_where_its_blocks_are_called_plainly():
         assert _called_plainly(block)
     block.forward = lambda *args, **kwargs: None
     assert not _called_plainly(block)
+
+
+def test_a_block_loop_takes_any_iterable():
+    calls = []
+
+    def block(stream, *args, **kwargs):
+        calls.append(kwargs)
+        return stream + 1, None
+
+    tokens = torch.zeros(1, 2, 4)
+    out = api.run_interaction_blocks((block for _ in range(3)), tokens, torch.zeros(1, 2, dtype=torch.bool), None)
+    assert torch.equal(out, tokens + 3) and [call["inplace"] for call in calls] == [False, True, True]
