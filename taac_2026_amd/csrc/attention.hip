@@ -612,7 +612,9 @@ __global__ __launch_bounds__(kThreads) void flash_attn_fwd_kernel(const AttnPara
 // MASKED: per-sample structure bits on top (struct_bits with a sample stride, every listed key valid, no chunk map): the
 // form in which samples with their valid tokens moved to the front arrive. The lane's two words of a chunk are fetched
 // with the chunk's transfers; tiles that are fully visible to the wavefront skip the bit tests.
-template <typename T, int DP, bool CAUSAL, bool SCALED, bool MASKED>
+// COMPACT: samples are addressed by row_offsets (a form of its own: decided at run time, the loads of the pointers' strides stand in
+// front of a workgroup's first rows in the other form too).
+template <typename T, int DP, bool CAUSAL, bool SCALED, bool MASKED, bool COMPACT = false>
 __global__ __launch_bounds__(kThreads) void flash_attn_fwd_dma_kernel(const AttnParams p) {
   static_assert(!(MASKED && CAUSAL), "a structured mask carries its own causal triangle");
   typedef typename Vec8<T>::type vec_t;
@@ -646,13 +648,10 @@ __global__ __launch_bounds__(kThreads) void flash_attn_fwd_dma_kernel(const Attn
   const int qc_a = static_cast<int>(qg_u);
   const int qc_b = p.pair_blocks ? static_cast<int>(p.nqc) - 1 - qc_a : qc_a;
 
-  // first row of the sample: one scalar load in the compact layout, a product otherwise
-  const bool compact = p.row_offsets != nullptr;
-  const int64_t row0 = compact ? p.row_offsets[b] : b;
-  const T* qb = static_cast<const T*>(p.q) + row0 * (compact ? p.qs[2] : p.qs[0]) + h * p.qs[1];
-  const T* kb = static_cast<const T*>(p.k) + row0 * (compact ? p.ks[2] : p.ks[0]) + h * p.ks[1];
-  const T* vb = static_cast<const T*>(p.v) + row0 * (compact ? p.vs[2] : p.vs[0]) + h * p.vs[1];
-  T* ob = static_cast<T*>(p.o) + row0 * (compact ? p.os[2] : p.os[0]) + h * p.os[1];
+  const T* qb = head_rows<COMPACT>(static_cast<const T*>(p.q), p.qs, p, b, h);
+  const T* kb = head_rows<COMPACT>(static_cast<const T*>(p.k), p.ks, p, b, h);
+  const T* vb = head_rows<COMPACT>(static_cast<const T*>(p.v), p.vs, p, b, h);
+  T* ob = head_rows<COMPACT>(static_cast<T*>(p.o), p.os, p, b, h);
 
   int len = p.Tk;
   if (p.key_lengths != nullptr) {
@@ -1386,6 +1385,17 @@ void launch(const AttnParams& p, bool causal, bool register_staging, hipStream_t
                            dim3(kSparseWaves * kWave), 0, s, p);
       return;
     }
+    if constexpr (std::is_same<T, bf16_t>::value) {
+      if (p.row_offsets != nullptr) {  // the entry point has checked the form; samples too long for 32-bit offsets have no mask
+        if (p.struct_bits != nullptr)
+          hipLaunchKernelGGL((flash_attn_fwd_dma_kernel<T, DP, false, false, true, true>), dim3(p.total_g), dim3(kThreads), 0, s, p);
+        else if (small_offsets(p))
+          hipLaunchKernelGGL((flash_attn_fwd_dma_kernel<T, DP, false, false, false, true>), dim3(p.total_g), dim3(kThreads), 0, s, p);
+        else
+          hipLaunchKernelGGL((flash_attn_fwd_kernel<T, DP, false, false, false, false, true>), dim3(p.total), dim3(kThreads), 0, s, p);
+        return;
+      }
+    }
     // structure bits ride along when they are all there is to the mask: per sample, no validity or self rows, no chunk map
     const bool structure_only = p.struct_bits != nullptr && p.valid_bits == nullptr && p.self_bits == nullptr &&
                                 p.block_any == nullptr;
@@ -1403,12 +1413,6 @@ void launch(const AttnParams& p, bool causal, bool register_staging, hipStream_t
       else
         hipLaunchKernelGGL((flash_attn_fwd_dma_kernel<T, DP, false, false, false>), dim3(p.total_g), dim3(kThreads), 0, s, p);
       return;
-    }
-    if constexpr (std::is_same<T, bf16_t>::value) {
-      if (p.row_offsets != nullptr) {  // samples too long for 32-bit offsets; the entry point has checked that there is no mask
-        hipLaunchKernelGGL((flash_attn_fwd_kernel<T, DP, false, false, false, false, true>), dim3(p.total), dim3(kThreads), 0, s, p);
-        return;
-      }
     }
   }
   if (p.drop_mask != nullptr && p.struct_bits != nullptr)
