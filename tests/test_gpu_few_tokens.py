@@ -3,6 +3,7 @@ kernels that large batches take (a capped grid selects those) and, through them,
 
 from __future__ import annotations
 
+import copy
 import threading
 
 import pytest
@@ -147,6 +148,7 @@ def test_calls_in_flight_on_several_streams_do_not_share_memory(device):
         thread.join()
     for (p, hidden), (want_p, want_hidden) in zip(got, want):
         assert torch.equal(p, want_p) and torch.equal(hidden, want_hidden)
+    assert len(model._workspaces) == 3 and len(copy.deepcopy(model)._workspaces) == 0
     # two calls on one stream, the first of which has not run yet, and one on another stream in between
     busy, other = torch.cuda.Stream(device), torch.cuda.Stream(device)
     torch.cuda.synchronize()
@@ -160,3 +162,29 @@ def test_calls_in_flight_on_several_streams_do_not_share_memory(device):
             third = model(*requests[2])
     torch.cuda.synchronize()
     assert all(torch.equal(p, want[i][0]) for i, p in enumerate((first, second, third)))
+
+
+def test_a_captured_call_has_its_own_memory(device):
+    """A forward recorded into a graph, replayed between eager calls of the same module on other inputs and streams: every result is
+    that of the eager call on the same input."""
+    model = PCVRBackbone(d_model=256, num_heads=8, d_ff=1024, n_blocks=2).to(device=device, dtype=torch.bfloat16).eval()
+    g = torch.Generator().manual_seed(10)
+    lengths = torch.tensor([100, 37], dtype=torch.int32, device=device)
+    inputs = [_bf16(g, 2, 100, 256).to(device) for _ in range(4)]
+    other = torch.cuda.Stream(device)
+    with torch.no_grad():
+        want = [model(emb, lengths) for emb in inputs]
+        static = inputs[0].clone()
+        torch.cuda.synchronize()
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph):
+            p = model(static, lengths)
+        for i, emb in enumerate(inputs):
+            static.copy_(emb)
+            torch.cuda.synchronize()
+            with torch.cuda.stream(other):
+                eager = model(inputs[i - 1], lengths)
+            graph.replay()
+            again = model(inputs[i - 2], lengths)
+            torch.cuda.synchronize()
+            assert torch.equal(p, want[i]) and torch.equal(eager, want[i - 1]) and torch.equal(again, want[i - 2])
