@@ -84,7 +84,7 @@ __global__ __launch_bounds__(kBlock) void token_dots_head_kernel(const float* __
   }
 }
 
-// Batches of more than kMaxScanBatch samples: exclusive prefix sums of the per-sample valid counts (one workgroup; B is walked
+// Batches too large for one launch (row_index.h): exclusive prefix sums of the per-sample valid counts (one workgroup; B is walked
 // in slabs of kBlock with a running carry), then the rows (valid_rows_kernel / valid_rows_bits_kernel).
 __global__ __launch_bounds__(kBlock) void length_offsets_kernel(const int32_t* __restrict__ lengths,
                                                                 const uint32_t* __restrict__ bits, int B, int T,
@@ -363,7 +363,7 @@ extern "C" int taac_valid_rows(const int32_t* key_lengths, int32_t B, int32_t T,
     return set_error(TAAC_ERR_UNSUPPORTED, "%s: B * T must fit 32-bit row numbers", name);
   if (!rows || !n_rows || (B > 0 && !key_lengths)) return set_error(TAAC_ERR_INVALID_VALUE, "%s: null pointer", name);
   if (B > 65535) return set_error(TAAC_ERR_UNSUPPORTED, "%s: at most 65535 samples", name);
-  if (B > 0 && T > 0 && B <= kMaxScanBatch) {
+  if (B > 0 && T > 0 && row_index_in_one_launch(B, T, false)) {
     const uint32_t units = static_cast<uint32_t>(B) * ((T + kRowThreads - 1) / kRowThreads);
     hipLaunchKernelGGL(valid_rows_scan_kernel, dim3(units), dim3(kRowThreads), 0, as_stream(stream), key_lengths, B, T, rows, n_rows);
     return check_launch(name);
@@ -386,7 +386,7 @@ extern "C" int taac_valid_rows_from_bits(const uint32_t* valid_bits, int32_t B, 
     return set_error(TAAC_ERR_UNSUPPORTED, "%s: B * T must fit 32-bit row numbers", name);
   if (!rows || !n_rows || (B > 0 && T > 0 && !valid_bits)) return set_error(TAAC_ERR_INVALID_VALUE, "%s: null pointer", name);
   if (B > 65535) return set_error(TAAC_ERR_UNSUPPORTED, "%s: at most 65535 samples", name);
-  if (B > 0 && T > 0 && B <= kMaxScanBatch) {
+  if (B > 0 && T > 0 && row_index_in_one_launch(B, T, true)) {
     const uint32_t units = static_cast<uint32_t>(B) * ((T + kRowThreads - 1) / kRowThreads);
     hipLaunchKernelGGL(valid_rows_bits_scan_kernel, dim3(units), dim3(kRowThreads), 0, as_stream(stream), valid_bits, B, T, rows, n_rows);
     return check_launch(name);

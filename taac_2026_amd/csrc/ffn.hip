@@ -1296,7 +1296,7 @@ int backbone_setup(const taac_block_weights* blocks, int n, int32_t D, int32_t F
     if (base == 0) {
       p.counters = counters;
       p.n_counters = n_counters;
-      if (rows != nullptr && B <= kMaxScanBatch) {
+      if (rows != nullptr && row_index_in_one_launch(B, T, false)) {
         p.rows = rows;
         p.n_rows = n_rows;
         p.row_units = static_cast<uint32_t>(B) * (T > kRowThreads ? (T + kRowThreads - 1) / kRowThreads : 1);

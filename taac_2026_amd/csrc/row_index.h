@@ -1,6 +1,6 @@
 // Valid-row index of a padded batch, one workgroup per (sample, 256 positions): every workgroup forms the prefix sum of the
-// samples in front of its own itself (B lengths, a few loads per thread and an L2 hit after the first workgroup), so the
-// index takes one launch instead of a scan followed by a fill.
+// samples in front of its own itself (up to B lengths, or B rows of validity words, spread over its threads), so the index takes one
+// launch instead of a scan followed by a fill.
 #pragma once
 
 #include "common.h"
@@ -9,7 +9,16 @@ namespace taac {
 namespace {
 
 constexpr int kRowThreads = 256;
-constexpr int kMaxScanBatch = 8192;  // above, the prefix sums cost more than a launch: length_offsets_kernel + fill
+
+// Whether it does: the prefix sums' work grows with the square of the batch, the scan's (length_offsets_kernel: one workgroup, 256
+// samples at a time) with the batch, so the line lies where the loads of all workgroups per sample - B x slabs x words of a sample
+// (one for lengths) - pass a constant. One launch / scan and fill, us. Lengths: 64 x 512 4.2 / 7.6, 8192 x 512 26 / 42, 16384 x 512
+// 81 / 80, 2048 x 2048 15 / 19, 4096 x 2048 33 / 34, 8192 x 2048 90 / 66, 16384 x 32 44 / 71, 32768 x 32 143 / 138. Bits: 64 x 512
+// 4.6 / 9.3, 256 x 512 5.8 / 9.6, 1024 x 512 35 / 17, 8192 x 512 2003 / 101, 64 x 2048 11 / 12, 256 x 2048 39 / 19, 16384 x 32 61 / 73.
+inline bool row_index_in_one_launch(int64_t B, int64_t T, bool bits) {
+  const int64_t slabs = T > kRowThreads ? (T + kRowThreads - 1) / kRowThreads : 1, words = bits ? (T + 31) / 32 : 1;
+  return B * slabs * words <= 16384;
+}
 
 __device__ __forceinline__ int32_t clamped_length(const int32_t* __restrict__ lengths, int b, int T) {
   const int32_t len = lengths[b];

@@ -558,7 +558,8 @@ extern "C" int taac_stack_train_fwd(const void* tokens, const int32_t* key_lengt
   const int32_t* count = rows_given != nullptr ? count_given : sv.count;
   const int32_t* offsets = rows + M;
   int rc = TAAC_OK;
-  if (rows_given == nullptr && B > kMaxScanBatch && (rc = taac_valid_rows(key_lengths, B, T, sv.rows, sv.count, stream)) != TAAC_OK)
+  const bool index_in_setup = rows_given == nullptr && row_index_in_one_launch(B, T, false);
+  if (rows_given == nullptr && !index_in_setup && (rc = taac_valid_rows(key_lengths, B, T, sv.rows, sv.count, stream)) != TAAC_OK)
     return rc;
   for (int first = 0; first < n_blocks; first += kSetupBlocks) {
     TrainSetup t{};
@@ -597,7 +598,7 @@ extern "C" int taac_stack_train_fwd(const void* tokens, const int32_t* key_lengt
     t.B = B;
     t.T = T;
     if (first == 0) {
-      if (rows_given == nullptr && B <= kMaxScanBatch) {
+      if (index_in_setup) {
         t.rows = sv.rows;
         t.n_rows = sv.count;
         t.row_units = static_cast<uint32_t>(B) * (T > kRowThreads ? (T + kRowThreads - 1) / kRowThreads : 1);

@@ -337,3 +337,46 @@ def test_valid_rows_from_a_padding_mask(device):
     assert int(by_len[1].item()) == int(by_mask[1].item()) == 14 and torch.equal(by_len[0][:14], by_mask[0][:14])
     with pytest.raises(ValueError, match="key_lengths or padding_mask"):
         valid_rows(None, 9)
+
+
+@pytest.mark.parametrize("bits,tokens,batch", [(False, 1, 16384), (False, 257, 8192), (True, 512, 512), (True, 33, 8192)])
+def test_valid_rows_on_both_sides_of_the_one_launch_form(device, bits, tokens, batch):
+    """The largest batch whose index takes one launch, and the next one: the same rows, count and offsets as the padding gives."""
+    from taac_2026_amd.api import valid_rows
+
+    g = torch.Generator().manual_seed(tokens)
+    for size in (batch, batch + 1):
+        lengths = torch.randint(-1, tokens + 2, (size,), generator=g, dtype=torch.int32)
+        padding = torch.arange(tokens)[None, :] >= lengths[:, None]
+        if bits:
+            padding |= torch.rand(size, tokens, generator=g) < 0.3
+        rows, count = valid_rows(None, tokens, padding_mask=padding.to(device)) if bits else valid_rows(lengths.to(device), tokens)
+        expected = (~padding).flatten().nonzero().flatten()
+        assert int(count.item()) == expected.numel()
+        assert torch.equal(rows[:expected.numel()].cpu().long(), expected)
+        offsets = rows[size * tokens:size * tokens + size + 1].cpu().long()
+        assert torch.equal(offsets, torch.cat([torch.zeros(1, dtype=torch.long), (~padding).sum(1).cumsum(0)]))
+
+
+@pytest.mark.parametrize("batch", [16384, 16385])
+def test_backbone_on_both_sides_of_the_one_launch_index(device, batch):
+    """Batches whose row index is part of the set-up launch, or not: each sample's result is that of its own small batch, up to the
+    order of the fp32 sums of the kernels that few tokens take."""
+    model = PCVRBackbone(d_model=128, num_heads=4, d_ff=64, n_blocks=1).to(torch.bfloat16).to(device)
+    g = torch.Generator().manual_seed(3)
+    emb = torch.randn(batch, 3, 128, generator=g).to(torch.bfloat16).to(device)
+    lengths = torch.randint(0, 4, (batch,), generator=g, dtype=torch.int32).to(device)
+    pick = torch.tensor([0, 1, 777, 8191, 8192, batch - 2, batch - 1], device=device)
+    with torch.no_grad():
+        served = model(emb, lengths)
+        torch.testing.assert_close(served[pick], model(emb[pick], lengths[pick]), rtol=0, atol=2e-3)
+    emb.requires_grad_(True)
+    trained = model(emb, lengths)
+    torch.testing.assert_close(trained.detach(), served, rtol=0, atol=2e-3)
+    trained[pick].sum().backward()
+    own = emb.detach()[pick].requires_grad_(True)
+    model(own, lengths[pick]).sum().backward()
+    torch.testing.assert_close(emb.grad[pick].float(), own.grad.float(), rtol=2 ** -5, atol=2 ** -5 * float(own.grad.abs().max()))
+    rest = torch.ones(batch, dtype=torch.bool, device=device)
+    rest[pick] = False
+    assert not emb.grad[rest].any()
