@@ -475,6 +475,9 @@ __global__ __launch_bounds__(kBlock) void bag_rows_kernel(const T* __restrict__ 
 bool sorted_bags(int64_t n, int64_t slots, int emb_dim, int dtype) {
   const int piece = dtype == TAAC_F32 ? 4 : 8;
   if (emb_dim % piece != 0 || emb_dim / piece > kWave || slots <= 0 || n > 0x3fffffffLL || slots > 0x3fffffffLL) return false;
+  int lanes = 1;
+  while (lanes < emb_dim / piece) lanes *= 2;
+  if (n * lanes > 0xffffff00LL) return false;  // threads of a launch over the rows
   const int64_t enough = 1 << 22;
   if (dtype == TAAC_F32) return slots * emb_dim >= enough && 2 * slots >= n;
   return slots * emb_dim >= enough || n * emb_dim >= enough;

@@ -342,3 +342,12 @@ def test_status_mapping_to_python_exceptions():
     with pytest.raises(RuntimeError, match="head_dim"):
         _native.check(status, "flash_attention")
     _native.check(_native.TAAC_OK, "anything")
+
+
+def test_the_sorted_embedding_gradient_stays_within_a_launch():
+    """A table whose rows times lanes pass 2^32 threads takes the form that adds up in memory (fp32: no workspace)."""
+    library = _native.load_library()
+    size = lambda rows, dim, dtype: library.taac_embedding_bag_mean_bwd_bytes(rows, dim, 2 ** 22, 16, dtype)  # noqa: E731
+    assert size(2 ** 26 - 4, 256, _native.TAAC_F32) > 0 and size(2 ** 26, 256, _native.TAAC_F32) == 0
+    assert size(2 ** 26, 128, _native.TAAC_F32) > 0 and size(2 ** 26 - 1, 129, _native.TAAC_F32) == 0
+    assert size(2 ** 26, 512, _native.TAAC_BF16) == 2 ** 26 * 512 * 4
