@@ -1648,7 +1648,8 @@ int attention_entry(const char* name, const void* q, const void* k, const void* 
   p.nqt_magic = magic_of(static_cast<uint32_t>((Tq + 31) / 32));
   // Pairs of query blocks per workgroup where blocks differ in work or may be empty (key lengths, a causal triangle);
   // with neither, every block is the same and single blocks fill the last round of the launch better. Nor in launches that the
-  // chip takes in one round anyway (up to five workgroups per compute unit): there a pair only makes the longest workgroup longer.
+  // chip takes in one round anyway (up to four workgroups per compute unit; five fit): there a pair only makes the longest workgroup
+  // longer.
   const int cus = compute_units();
   if (cus <= 0) return set_error(TAAC_ERR_LAUNCH, "%s: cannot query the device", name);
   p.pair_blocks = (p.nqc > 1 && (key_lengths != nullptr || is_causal != 0) && total > 4 * static_cast<int64_t>(cus)) ? 1 : 0;

@@ -218,7 +218,9 @@ __device__ __forceinline__ f32x4 load_through(const f32x4* src) {
 // 49.9 -> 21.5 us; 8192 tokens: 55.6 -> 27.8; its line is at ffn_few_rows).
 // splits > 1 (see TsParams): for batches that leave most of the chip idle even so, the hidden units of a tile are also divided over
 // workgroups, eight at most (one request of 512 positions, eight splits, with the requests below ordered by need: the whole
-// 4-block call 164 -> 140 us; fences instead of the write-through accesses: 156).
+// 4-block call 164 -> 140 us; fences instead of the write-through accesses: 156). Sixteen lose where tiles and F admit them: a
+// wavefront then has one 16-unit chunk behind the same latency chains (at most 16 / 8 / 4 splits, F = 1024 160 / 140 / 135 us,
+// F = 512 136 / 136 / 127, F = 2048 169 / 151 / 153).
 // LDS: [4 partials of 32 x D floats][x1 (32 padded rows of D bf16)][first-layer bias 2F][4 x 32 row sums]
 // ------------------------------------------------------------------------------------------------------------------
 template <int D, bool OUTP, bool FOLD>

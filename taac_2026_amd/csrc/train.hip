@@ -9,13 +9,13 @@
 // known on the device; every kernel reads the count, grids and buffers are sized by B * T, the host never waits.
 //
 // The forward keeps per block: the input stream x, q | k | v, the attention output and its log-sum-exp, the stream x1 between the
-// two halves, and the factors of the two norms. The backward of a block is seven launches:
+// two halves, and the factors of the two norms. The backward of a block is eight launches, nine with query / key norms:
 //   feed-forward backward (hidden state, gradient of the up projection)  -> x1, dy
 //   input gradient of the up projection + norm backward + residual       -> dx1
 //   out projection's input gradient                                       -> datt
-//   attention backward (two kernels; + the query / key norms' backward)  -> dq | dk | dv
+//   attention backward (two launches; + the query / key norms')           -> dq | dk | dv
 //   input gradient of the q | k | v projection + norm backward + residual -> dx
-//   the four weight gradients, and the reduction of their splits
+//   the four weight gradients, and the reduction of their splits (two launches)
 // The normalised rows never exist in memory: the weight gradients multiply x by the norm's factor as they stage it and apply the
 // norm's weight to the columns of the result; the gradient of that weight falls out of the same sums (train_ops.h).
 #include <vector>

@@ -238,11 +238,12 @@ int launch_dgrad(const DgradParams& p, hipStream_t s, const char* name) {
 
 // ------------------------------------------------------------------------------------------------------------------
 // Weight gradients. Both operands are [tokens, features] row-major and the MFMA needs eight consecutive tokens of one feature
-// per lane from each, so 64-token chunks of both slabs pass through registers into one of two LDS buffers (rows padded by 32
+// per lane from each, so 64-token chunks of both slabs pass through registers into one of two LDS buffers (rows padded by 64
 // bytes: the four rows and pieces a 16-lane group of a transposed read touches fall on distinct banks) while the chunk before is
 // multiplied, and both fragments are read with ds_read_b64_tr_b16. A workgroup owns a TN x TK tile of one layer's gradient over its
-// share of the tokens; all tiles of all layers form one launch of about one workgroup per compute unit (a workgroup fills one with
-// its LDS), so a block's partial sums are one chip's worth of tiles (64 MB at D = 256) instead of one per layer.
+// share of the tokens; all tiles of all layers form one launch of about one workgroup per compute unit (two of the 128 x 128 tiles;
+// a workgroup of the large ones fills one with its LDS), so a block's partial sums are one chip's worth of tiles (64 MB at D = 256)
+// instead of one per layer.
 // Bound: HBM - the operands are read once per 256 features of the other side.
 // ------------------------------------------------------------------------------------------------------------------
 constexpr int kChunk = 64;

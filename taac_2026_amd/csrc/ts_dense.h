@@ -64,11 +64,11 @@ struct TsParams {
   // the rounded output), so that a mean-pooling linear head behind the layer need not read the rows again.
   const bf16_t* head_w;     // [D] or null
   float* token_dots;        // [M] (rows like out), written for the tokens the kernel stores
+  float* rstd_out;          // [M]: the per-token factor of the norm in front (of the up projection; of the linear layer), or null
+  bf16_t* x1_out;           // OUTP: the tokens between the two halves of the block, [M, D] rows like out; or null
   // Few-token feed-forward with the hidden units of a 32-token tile divided over `splits` workgroups (0: one): every workgroup
   // leaves its fp32 partial in split_partials [tile][splits][32 x D] and counts itself in split_counters [tile] (zero before
   // the launch); the last one to arrive adds the partials up in order, finishes the tile and sets the counter back to zero.
-  float* rstd_out;          // [M]: the per-token factor of the norm in front (of the up projection; of the linear layer), or null
-  bf16_t* x1_out;           // OUTP: the tokens between the two halves of the block, [M, D] rows like out; or null
   int32_t splits;
   float* split_partials;
   uint32_t* split_counters;
@@ -92,7 +92,7 @@ __host__ __device__ __forceinline__ int up_unit_of_slot(int m16) {
   return 8 * ((m16 >> 2) & 1) + 4 * (m16 >> 3) + (m16 & 3);
 }
 
-// Constants of the gate's activation when the packed up projection carries them (see ffn_pack_piece in ffn.hip).
+// Constants of the gate's activation when the packed up projection carries them (see ffn_pack_piece in pack.h).
 constexpr float kFoldGate = -1.4426950408889634f, kFoldValue = -0.6931471805599453f;
 
 // ---- shared pieces ---------------------------------------------------------------------------------------------------
