@@ -22,6 +22,18 @@ def _near(name: str, got: torch.Tensor, want: torch.Tensor, blocks: int) -> None
     assert (got - want).norm() <= 2.0 ** -5 * blocks * want.norm() + 1e-9, (name, (got - want).norm() / want.norm())
 
 
+def _near_rows(name: str, got: torch.Tensor, want: torch.Tensor, lengths: torch.Tensor, blocks: int) -> None:
+    """Row by row: a row at a remainder that is missing, stale or another one is off by its whole norm, which the norm over all rows
+    does not show. The same bound on the row's norm, with that of a typical row besides (a row that is small because its terms
+    cancel has their roundings); padded rows are zeros."""
+    got, want = got.detach().cpu().double(), want.double()
+    valid = torch.arange(got.shape[1])[None, :] < lengths[:, None]
+    assert not got[~valid].any(), name
+    size, error = want[valid].norm(dim=-1), (got - want)[valid].norm(dim=-1)
+    bound = 2.0 ** -5 * blocks * (size + size.square().mean().sqrt())
+    assert (error <= bound).all(), (name, (error / bound).max())
+
+
 @pytest.mark.parametrize("d_model,heads,d_ff,n_blocks,lengths,tokens,qk_norm,dtype", [
     (256, 8, 1024, 1, [1], 1, False, torch.bfloat16),                     # one token
     (256, 4, 96, 2, [0, 65, 64, 1], 65, True, torch.float32),             # around a 64-token tile; F not a multiple of a gradient tile
@@ -67,6 +79,8 @@ def test_training_stack_at_the_edges_of_its_tiles(device, d_model, heads, d_ff, 
     _near("p", p, want_p.detach(), n_blocks)
     _near("hidden", hidden, (x * keep).detach(), n_blocks)
     _near("tokens", emb_d.grad, emb_r.grad, n_blocks)
+    _near_rows("hidden", hidden, (x * keep).detach(), lengths, n_blocks)
+    _near_rows("tokens", emb_d.grad, emb_r.grad, lengths, n_blocks)
     for name, parameter in model.named_parameters():
         assert parameter.grad.dtype == dtype
         _near(name, parameter.grad, reference[name].grad, n_blocks)
@@ -314,3 +328,29 @@ def test_hooks_of_all_modules_and_replaced_forwards_see_every_block_of_a_stack(d
     assert [module for module in seen if module in blocks] == blocks
     blocks[1].forward = lambda tokens, *args, **kwargs: (tokens * 0, None)
     assert not run_interaction_blocks(blocks[:2], x, padding, mask).any()
+
+
+def test_training_stack_with_the_kernels_of_large_batches(device):
+    """More positions than 512 per compute unit: the input gradient of the up projection takes its 256-token workgroups, the last of
+    which holds a remainder. The samples are short and the oracle sees their first positions only."""
+    batch, tokens, short = 2049, 64, 9
+    assert batch * tokens > 512 * torch.cuda.get_device_properties(device).multi_processor_count
+    lengths = torch.tensor([(7 * i) % short for i in range(batch)], dtype=torch.int32)
+    assert int(lengths.sum()) % 256 not in (0, 255)
+    g = torch.Generator().manual_seed(41)
+    model, reference = _network(256, 8, 1024, 1, seed=42)
+    emb, grad = (torch.randn(batch, tokens, 256, generator=g).to(torch.bfloat16) for _ in range(2))
+    model = model.to(torch.bfloat16).to(device).train()
+    emb_d = emb.to(device).requires_grad_(True)
+    _, hidden = model(emb_d, lengths.to(device), return_hidden=True)
+    hidden.backward(grad.to(device))
+    emb_r = emb[:, :short].double().requires_grad_(True)
+    want = _oracle_hidden(reference, emb_r, lengths, 8, 1)
+    want.backward(grad[:, :short].double())
+    assert not hidden[:, short:].any() and not emb_d.grad[:, short:].any()
+    for name, got, right in (("hidden", hidden[:, :short], want.detach()), ("tokens", emb_d.grad[:, :short], emb_r.grad)):
+        _near(name, got, right, 1)
+        _near_rows(name, got, right, lengths, 1)
+    for name, parameter in model.named_parameters():
+        if not name.startswith("head."):
+            _near(name, parameter.grad, reference[name].grad, 1)
