@@ -662,8 +662,9 @@ class PCVRBackbone(nn.Module):
                 runs[-1][1] += 1
             else:
                 runs.append([form, 1])
+        params += [self.head.weight, self.head.bias]
         if self.rope_base is not None or self.d_model not in (128, 256) or head_dim not in (32, 64) \
-                or any(p.dtype not in (torch.bfloat16, torch.float32) for p in self.parameters()) \
+                or not {p.dtype for p in params if p is not None} <= {torch.bfloat16, torch.float32} \
                 or not all(map(covered, {self.d_ff, *(form[0] for form, _ in runs)})):
             raise RuntimeError(f"{name}: the training route covers bf16 (or float32 master) parameters, d_model 128 / 256, "
                                "head dims 32 / 64, d_ff a multiple of 32 within the backward kernel's bound "
@@ -673,7 +674,7 @@ class PCVRBackbone(nn.Module):
             hidden = emb * valid
             probabilities = self._read_out(hidden, key_lengths)
             return (probabilities, hidden) if return_hidden else probabilities
-        *params, head_w, head_b = uniform_parameters([*params, self.head.weight, self.head.bias])
+        *params, head_w, head_b = uniform_parameters(params)
         rides = head_w.shape == (1, self.d_model) and (head_b is None or head_b.shape == (1,)) and head_w.device == emb.device \
             and (head_b is None or head_b.device == emb.device)
         hidden, first = emb, 0
