@@ -369,10 +369,12 @@ def ptr(tensor: torch.Tensor | None) -> int | None:
 def current_stream(device: torch.device) -> int:
     """The raw stream of the calling thread on ``device`` (without a ``torch.cuda.Stream`` object around it: 0.2 instead of 2.5
     us per operator call). The library only takes device addresses: a stream of another kind of device is refused."""
-    if device.type != "cuda":
-        raise ValueError(f"expected a cuda device, got {device}")
     index = device.index
-    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device() if index is None else index)
+    if index is None:  # not a tensor on a GPU, whose device has an ordinal
+        if device.type != "cuda":
+            raise ValueError(f"expected a cuda device, got {device}")
+        index = torch.cuda.current_device()
+    return torch._C._cuda_getCurrentRawStream(index)
 
 
 __all__ = [
