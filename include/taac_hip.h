@@ -271,9 +271,9 @@ int taac_role_mask(const void* roles, int roles_int64, const uint32_t visible[8]
  *   dv = P^T dout,  dS = P * (dout v^T - D) / sqrt(d),  dq = dS k,  dk = dS^T q
  * for the same mask arguments as the forward. o is the forward's output, dout its gradient (logical (B, H, Tq, d) like
  * q, own strides); dq / dk / dv have the logical shapes of q / k / v and their own element strides (same rules as the
- * forward). delta: workspace, fp32 [B, H, Tq]. With zero_padded_queries the padded query rows carry no gradient (dq
+ * forward). delta: workspace, fp32 [B, H, Tq] (written or not). With zero_padded_queries the padded query rows carry no gradient (dq
  * rows are zero); gradients of keys at or beyond key_lengths[b] are zero. Every output element has one writer and a
- * fixed summation order (two kernels, each recomputing the scores), so results are reproducible run to run.
+ * fixed summation order, so results are reproducible run to run.
  * Replaces: the TileLang training forward (accelerators/attention/kernels/tilelang.py:287-390) and backward
  * preprocess + backward kernels (:405-435, 598-699), which accumulate dq with floating-point atomics.
  */

@@ -3,8 +3,9 @@
 // With S = Q K^T / sqrt(d), P = exp(S - lse) (lse saved by the training forward), D_i = sum_d O[i, d] dO[i, d]:
 //   dV = P^T dO,   dP = dO V^T,   dS = P * (dP - D) / sqrt(d),   dQ = dS K,   dK = dS^T Q
 // (the recipe of the reference's backward kernels, accelerators/attention/kernels/tilelang.py:405-435, 598-699).
-// Two kernels, both recomputing S and dP from the inputs, so that every output element has exactly one writer and a
-// fixed summation order (the reference accumulates dQ with floating-point atomics):
+// Every output element has exactly one writer and a fixed summation order (the reference accumulates dQ with
+// floating-point atomics). Where a workgroup can hold a sample's keys, attn_bwd_fused_kernel forms all three gradients
+// at once; otherwise two kernels, both recomputing S and dP from the inputs:
 //   attn_bwd_dq_kernel   one workgroup per (batch, head, 128 queries): a lane owns one query, the keys stream through
 //                        LDS in chunks of 64; also writes D for the second kernel.
 //   attn_bwd_dkv_kernel  one workgroup per (batch, head, 128 keys): a lane owns one key, the queries stream through LDS.
@@ -717,6 +718,382 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu((DP ==
   store_owned<T, DP>(dvacc, tile, dvb, p.dvs[2], k_begin + wave * 32, k_store_end, p.d, lane);
 }
 
+template <typename T>
+struct Mfma16;
+template <>
+struct Mfma16<bf16_t> {
+  static __device__ __forceinline__ f32x4 run(bf16x8 a, bf16x8 b, f32x4 c) {
+    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
+  }
+};
+template <>
+struct Mfma16<f16_t> {
+  static __device__ __forceinline__ f32x4 run(f16x8 a, f16x8 b, f32x4 c) {
+    return __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b, c, 0, 0, 0);
+  }
+};
+
+// acc + a[e] * b[e] + a[e + 1] * b[e + 1] in float32.
+__device__ __forceinline__ float dot2(bf16x8 a, bf16x8 b, int e, float acc) {
+  typedef __attribute__((__vector_size__(2 * sizeof(__bf16)))) __bf16 bf16x2;
+  return __builtin_amdgcn_fdot2_f32_bf16(bf16x2{a[e], a[e + 1]}, bf16x2{b[e], b[e + 1]}, acc, false);
+}
+__device__ __forceinline__ float dot2(f16x8 a, f16x8 b, int e, float acc) {
+  typedef __attribute__((__vector_size__(2 * sizeof(_Float16)))) _Float16 f16x2;
+  return __builtin_amdgcn_fdot2(f16x2{a[e], a[e + 1]}, f16x2{b[e], b[e + 1]}, acc, false);
+}
+
+// dQ, dK and dV of one (batch, head) in one workgroup, for samples whose keys it can hold: S, dP and the exponentials are
+// formed once instead of twice (five products per pair of tiles instead of seven) and every tensor is read once.
+// Wavefront w owns the 32-key tiles w, w + 4, ... (NT of them: their dK / dV accumulators and V fragments stay in
+// registers, NT * DP = 64 or 128), K lies in LDS as a whole, the queries stream through LDS in chunks of 32 rows. A lane
+// owns a key, so P and dS come out of the first products as the B operands of dV and dK; dQ contracts over the keys
+// instead: the dS tiles of all wavefronts meet in LDS ([key][query], 16 bits as every operand) and each wavefront forms
+// its own 16 queries x 16 features (DP = 64: twice) of dQ over all key tiles, so dQ, too, has one writer per element and
+// a fixed order.
+template <int DP, int NT, bool BITS>
+struct FusedLayout {
+  static constexpr int kRows = 32;                                     // streamed queries per step
+  static constexpr int ROWB = DP * 2, TILE_BYTES = kRows * ROWB;
+  static constexpr int kWaves = kThreads / kWave, kTiles = kWaves * NT;  // key tiles of 32 rows
+  static constexpr int K_BYTES = kTiles * TILE_BYTES, DS_BYTES = kTiles * kRows * 64;
+  static constexpr int WORD_BYTES = BITS ? kTiles * kRows * 4 : 0;      // [tile][row]
+  static constexpr int BUF_BYTES = 2 * TILE_BYTES + WORD_BYTES;         // Q, dO, words
+  static constexpr int STAT_BYTES = 2 * kTiles * kRows * 4;             // log-sum-exp and -D of every query
+  static constexpr int BYTES = K_BYTES + DS_BYTES + 2 * BUF_BYTES + STAT_BYTES;
+};
+
+template <typename T, int DP, int NT, int MODE, bool COMPACT>
+__global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(NT * DP == 128 ? 2 : 3, NT * DP == 128 ? 2 : 3)))
+void attn_bwd_fused_kernel(const AttnBwdParams p) {
+  constexpr bool BITS = MODE == kMaskBits;
+  static_assert(MODE == kMaskNone || BITS, "the other masks are read per element by the two kernels above");
+  typedef typename Vec8<T>::type vec_t;
+  typedef typename Vec8<T>::half_type vec4_t;
+  typedef FusedLayout<DP, NT, BITS> L;
+  constexpr int KSTEPS = DP / 16, MB = DP / 32, C8 = DP / 8, kRows = L::kRows, ROWB = L::ROWB, TILE_BYTES = L::TILE_BYTES;
+  constexpr int kWaves = L::kWaves;
+  [[maybe_unused]] constexpr int kWords = L::kTiles * kRows;
+  // In bf16 dS stays without its 1 / sqrt(d), which multiplies dK and dQ at the end; fp16 could leave its range that way.
+  constexpr bool LATE_SCALE = std::is_same<T, bf16_t>::value;
+  __shared__ __attribute__((aligned(1024))) uint8_t smem[L::BYTES];
+  uint8_t* const k_image = smem;
+  uint8_t* const ds_image = smem + L::K_BYTES;
+  uint8_t* const buffers = smem + L::K_BYTES + L::DS_BYTES;
+
+  const int bh = static_cast<int>(xcd_remap(blockIdx.x, p.total));
+  const int h = bh % p.H, b = bh / p.H;
+  const int tid = threadIdx.x, wave = tid / kWave, lane = tid % kWave, l32 = lane % 32, hh = lane / 32;
+  const T* qb = head_rows<COMPACT>(static_cast<const T*>(p.q), p.qs, p, b, h);
+  const T* kb = head_rows<COMPACT>(static_cast<const T*>(p.k), p.ks, p, b, h);
+  const T* vb = head_rows<COMPACT>(static_cast<const T*>(p.v), p.vs, p, b, h);
+  const T* ob = head_rows<COMPACT>(static_cast<const T*>(p.o), p.os, p, b, h);
+  const T* dob = head_rows<COMPACT>(static_cast<const T*>(p.dout), p.dos, p, b, h);
+  T* dqb = head_rows<COMPACT>(static_cast<T*>(p.dq), p.dqs, p, b, h);
+  T* dkb = head_rows<COMPACT>(static_cast<T*>(p.dk), p.dks, p, b, h);
+  T* dvb = head_rows<COMPACT>(static_cast<T*>(p.dv), p.dvs, p, b, h);
+
+  int len = p.Tk;
+  if (p.key_lengths != nullptr) {
+    len = p.key_lengths[b];
+    len = len < 0 ? 0 : (len > p.Tk ? p.Tk : len);
+  }
+  const int q_valid = p.zero_pad ? (len < p.Tq ? len : p.Tq) : p.Tq;
+  // The wavefront's key tiles are own, own + 4, ...: with a number of tiles that 4 does not divide the wavefronts with one tile more
+  // lie on other SIMDs in other workgroups.
+  const int own = (wave + bh + bh / 32) % (kThreads / kWave);
+  const int n_tiles = (len + 31) / 32;           // at most L::kTiles: the host checks Tk
+  const int q_end = n_tiles > 0 ? q_valid : 0;   // rows of dQ at or beyond it are zero
+  const float c = p.scale * 1.4426950408889634f;
+  const int64_t stat0 = (static_cast<int64_t>(b) * p.H + h) * p.Tq;
+  [[maybe_unused]] const int wpr = (p.Tk + 31) / 32;
+
+  f32x16 dkacc[NT][MB], dvacc[NT][MB];
+#pragma unroll
+  for (int t = 0; t < NT; ++t)
+#pragma unroll
+    for (int mb = 0; mb < MB; ++mb)
+#pragma unroll
+      for (int j = 0; j < 16; ++j) dkacc[t][mb][j] = dvacc[t][mb][j] = 0.f;
+
+  if (q_end > 0) {
+    // ---- a chunk of Q and dO: 1 KB transfers straight into LDS, dealt to the wavefronts; rows at or beyond q_valid
+    // repeat the last valid one (their probabilities are zeros). Row r of a tile: 16-byte piece x lies at x ^ row_swizzle(r).
+    auto transfer = [&](const T* base, int64_t stride, int row0, int row_end, int slot, uint8_t* tile) {
+      const int r = slot * (kWave / C8) + lane / C8;
+      const int piece = (lane % C8) ^ row_swizzle<DP>(r);
+      int row = row0 + r;
+      row = row < row_end ? row : row_end - 1;
+      lds_dma16_offset(base, __umul24(static_cast<uint32_t>(row), static_cast<uint32_t>(stride) * 2u) + static_cast<uint32_t>(piece * 16),
+                       tile + slot * 1024);
+    };
+    constexpr int kSlots = TILE_BYTES / 1024;  // per operand of a chunk: 2 or 4
+    auto fetch_chunk = [&](int qc0, uint8_t* buf) {
+#pragma unroll
+      for (int i = 0; i < 2 * kSlots / kWaves; ++i) {
+        const int slot = wave + i * kWaves;  // wavefront-uniform
+        if (slot < kSlots)
+          transfer(qb, p.qs[2], qc0, q_valid, slot, buf);
+        else
+          transfer(dob, p.dos[2], qc0, q_valid, slot - kSlots, buf + TILE_BYTES);
+      }
+    };
+    // words of the chunk's rows for every key tile, [tile][row], one per lane and transfer; rows and tiles that do not exist repeat
+    // the last one (their probabilities are zeros, or nobody reads them)
+    auto fetch_words = [&](int qc0, uint8_t* buf) {
+#pragma unroll
+      for (int i = 0; i < (kWords + kThreads - 1) / kThreads; ++i) {
+        const int slot0 = i * kThreads + wave * kWave;
+        if (slot0 < kWords) {  // wavefront-uniform
+          const int slot = slot0 + lane;
+          int tile = slot / kRows, qi = qc0 + slot % kRows;
+          tile = tile < n_tiles ? tile : n_tiles - 1;
+          qi = qi < q_valid ? qi : q_valid - 1;
+          lds_dma4(p.bit_words + b * p.bits_bs + static_cast<int64_t>(qi) * wpr + tile, buf + 2 * TILE_BYTES + slot0 * 4);
+        }
+      }
+    };
+    // The statistics of all queries: D from one 16-byte piece of O and dO per thread, summed over the C8 threads of a row; base-2
+    // log-sum-exp, +inf for a row that carries nothing: exp2(x - inf) = 0. Rows of the last chunk at or beyond q_valid among them.
+    float* const stats = reinterpret_cast<float*>(buffers + 2 * L::BUF_BYTES);
+    constexpr int kStatRows = kThreads / C8, kStatUnroll = 4;  // rows per pass, passes in flight
+    auto row_stats = [&](int row0) {
+      const int piece = (tid % C8) * 8;
+      vec_t of[kStatUnroll], dof[kStatUnroll];
+      float lse[kStatUnroll];
+#pragma unroll
+      for (int u = 0; u < kStatUnroll; ++u) {
+        const int row = row0 + u * kStatRows + tid / C8;
+        lse[u] = -INFINITY;
+        if (row < q_valid) {
+          of[u] = *reinterpret_cast<const vec_t*>(ob + row * p.os[2] + piece);
+          dof[u] = *reinterpret_cast<const vec_t*>(dob + row * p.dos[2] + piece);
+          lse[u] = p.lse[stat0 + row];
+        } else {
+#pragma unroll
+          for (int e = 0; e < 8; ++e) of[u][e] = dof[u][e] = static_cast<T>(0.f);
+        }
+      }
+#pragma unroll
+      for (int u = 0; u < kStatUnroll; ++u) {
+        const int row = row0 + u * kStatRows + tid / C8;
+        if (row0 + u * kStatRows >= q_valid) break;  // uniform
+        float delta = 0.f;
+#pragma unroll
+        for (int e = 0; e < 8; e += 2) delta = dot2(of[u], dof[u], e, delta);
+        delta = group_sum<C8>(delta);
+        if (piece == 0 && row < L::kTiles * kRows) {
+          stats[row] = lse[u] > -INFINITY ? lse[u] * 1.4426950408889634f : INFINITY;
+          stats[L::kTiles * kRows + row] = -delta;
+        }
+      }
+    };
+
+    if (BITS) fetch_words(0, buffers);
+    for (int slot = wave; slot < n_tiles * kSlots; slot += kWaves)
+      transfer(kb, p.ks[2], 0, len, slot, k_image);
+    fetch_chunk(0, buffers);
+    vec_t vf[NT][KSTEPS];
+#pragma unroll
+    for (int t = 0; t < NT; ++t) {
+      const int key = (own + t * kWaves) * 32 + l32;
+      load_owned<T, DP>(vb, p.vs[2], key, key < len, p.d, hh, vf[t]);
+    }
+    for (int row0 = 0; row0 < q_valid; row0 += kStatUnroll * kStatRows) row_stats(row0);
+    // bit t: the lane's key of the wavefront's tile t is valid as a key
+    [[maybe_unused]] uint32_t seen = ~0u;
+    if (BITS && p.key_valid != nullptr) {
+      seen = 0u;
+#pragma unroll
+      for (int t = 0; t < NT; ++t) {
+        const int tile = own + t * kWaves;
+        if (tile < n_tiles)
+          seen |= ((reinterpret_cast<const uint32_t*>(p.key_valid)[static_cast<int64_t>(b) * wpr + tile] >> l32) & 1u) << t;
+      }
+    }
+
+    const uint32_t row_off = streamed_row_offset<DP>(l32, hh);
+    const uint32_t col_off = streamed_column_offset<DP>(lane);
+    // dS in LDS: rows of 32 queries per key, the 8-byte piece x of key r at x ^ (r / 4) % 8 - writes of one piece by 32 keys and the
+    // transposed reads below cover the banks evenly.
+    const uint32_t ds_write = static_cast<uint32_t>(l32 * 64);
+    const int g16 = lane / 16, i16 = lane % 16, q_half = wave % 2, d_col = wave / 2;
+    uint32_t ds_read[2], k_read[2];
+#pragma unroll
+    for (int half = 0; half < 2; ++half) {
+      const int key = 8 * g16 + 4 * half + i16 / 4;  // of the tile: one transposed read holds keys 8 g16 + 4 half + 0..3
+      const int piece = 4 * q_half + i16 % 4;        // four queries
+      ds_read[half] = lds_offset(ds_image) + static_cast<uint32_t>(key * 64 + ((piece ^ (key / 4)) * 8));
+      const int piece16 = 2 * d_col + (i16 % 4) / 2;  // eight features
+      k_read[half] = lds_offset(k_image) + static_cast<uint32_t>(key * ROWB + ((piece16 ^ row_swizzle<DP>(key)) * 16) + (i16 % 2) * 8);
+    }
+
+    vm_wait<0>();
+    int buf = 0;
+    for (int qc0 = 0; qc0 < q_valid; qc0 += kRows) {
+      const bool more = qc0 + kRows < q_valid;
+      const int q_tile = qc0 / kRows;
+      const int tiles = p.causal ? (n_tiles < q_tile + 1 ? n_tiles : q_tile + 1) : n_tiles;  // key tiles these queries see
+      uint8_t* const chunk = buffers + buf * L::BUF_BYTES;
+      uint8_t* const next = buffers + (buf ^ 1) * L::BUF_BYTES;
+      __syncthreads();  // the chunk and its statistics have landed (every wavefront awaited its own transfers); dS is free
+      if (more) {
+        if (BITS) fetch_words(qc0 + kRows, next);
+        fetch_chunk(qc0 + kRows, next);
+      }
+      const float* s_lse = stats + qc0;
+      const float* s_delta = s_lse + L::kTiles * kRows;
+      [[maybe_unused]] const uint32_t* s_words = reinterpret_cast<const uint32_t*>(chunk + 2 * TILE_BYTES);
+      const uint32_t col_addr = lds_offset(chunk) + col_off;
+      static_for<NT>([&](auto t_tag) {
+        constexpr int t = decltype(t_tag)::value;
+        const int tile = own + t * kWaves;
+        if (tile >= tiles) return;  // wavefront-uniform
+        f32x16 sacc, dpacc;
+#pragma unroll
+        for (int j = 0; j < 16; ++j) sacc[j] = 0.f;
+#pragma unroll
+        for (int jq = 0; jq < 4; ++jq) {
+          const f32x4 d4 = *reinterpret_cast<const f32x4*>(&s_delta[jq * 8 + hh * 4]);
+#pragma unroll
+          for (int e = 0; e < 4; ++e) dpacc[jq * 4 + e] = d4[e];
+        }
+#pragma unroll
+        for (int s = 0; s < KSTEPS; ++s) {
+          const uint32_t off = row_off ^ (s * 32);
+          const vec_t qa = *reinterpret_cast<const vec_t*>(chunk + off);
+          const vec_t kf = *reinterpret_cast<const vec_t*>(k_image + tile * TILE_BYTES + off);
+          sacc = Mfma32<T>::run(qa, kf, sacc);
+        }
+#pragma unroll
+        for (int s = 0; s < KSTEPS; ++s) {
+          const vec_t da = *reinterpret_cast<const vec_t*>(chunk + TILE_BYTES + (row_off ^ (s * 32)));
+          dpacc = Mfma32<T>::run(da, vf[t][s], dpacc);
+        }
+        const int key = tile * 32 + l32;
+        // pairs that do not exist get a score of -inf; only the tile at the end of the keys and the one on the causal diagonal test
+        if (tile * 32 + 32 > len || (BITS && p.key_valid != nullptr)) {  // wavefront-uniform
+          const bool beyond = key >= len || (BITS && ((seen >> t) & 1u) == 0u);
+#pragma unroll
+          for (int j = 0; j < 16; ++j) sacc[j] = beyond ? -INFINITY : sacc[j];
+        }
+        if (p.causal && tile == q_tile) {
+          const int first = l32 - hh * 4;  // query row (j / 4) * 8 + hh * 4 + j % 4 lies before key l32
+#pragma unroll
+          for (int j = 0; j < 16; ++j) sacc[j] = first > (j / 4) * 8 + (j % 4) ? -INFINITY : sacc[j];
+        }
+        vec_t pb[2], dsb[2];
+#pragma unroll
+        for (int jq = 0; jq < 4; ++jq) {
+          const f32x4 l4 = *reinterpret_cast<const f32x4*>(&s_lse[jq * 8 + hh * 4]);
+          [[maybe_unused]] u32x4 w4 = {0u, 0u, 0u, 0u};
+          if (BITS) w4 = *reinterpret_cast<const u32x4*>(&s_words[tile * kRows + jq * 8 + hh * 4]);
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            const int j = jq * 4 + e;
+            float prob = __builtin_amdgcn_exp2f(fmaf(sacc[j], c, -l4[e]));
+            if (BITS)  // all ones where the word has the lane's bit
+              prob = __builtin_bit_cast(float, __builtin_bit_cast(uint32_t, prob) & __builtin_amdgcn_sbfe(w4[e], l32, 1));
+            pb[j / 8][j % 8] = static_cast<T>(prob);
+            dsb[j / 8][j % 8] = static_cast<T>(prob * (LATE_SCALE ? dpacc[j] : dpacc[j] * p.scale));
+          }
+        }
+        uint8_t* const ds_tile = ds_image + tile * (kRows * 64) + ds_write;
+#pragma unroll
+        for (int jq = 0; jq < 4; ++jq) {
+          vec4_t quad;
+#pragma unroll
+          for (int e = 0; e < 4; ++e) quad[e] = dsb[jq / 2][(jq % 2) * 4 + e];
+          *reinterpret_cast<vec4_t*>(ds_tile + ((2 * jq + hh) ^ (l32 / 4)) * 8) = quad;
+        }
+        accumulate_columns2<T, DP, 0>(dvacc[t], pb, col_addr + TILE_BYTES, dkacc[t], dsb, col_addr);
+      });
+      __syncthreads();  // the dS tiles of every wavefront are in LDS
+      f32x4 dqacc[MB];
+#pragma unroll
+      for (int m = 0; m < MB; ++m) dqacc[m] = f32x4{0.f, 0.f, 0.f, 0.f};
+      auto contract = [&](int tile, auto n_tag) {  // key tiles tile .. tile + n - 1
+        constexpr int n = decltype(n_tag)::value;
+        u32x2 fs[n][2], fk[n][MB][2];
+        const uint32_t ds0 = ds_read[0] + tile * (kRows * 64), ds1 = ds_read[1] + tile * (kRows * 64);
+        const uint32_t k0 = k_read[0] + tile * TILE_BYTES, k1 = k_read[1] + tile * TILE_BYTES;
+        static_for<n>([&](auto i_tag) {
+          constexpr int i = decltype(i_tag)::value;
+          lds_read_tr16<i * kRows * 64>(fs[i][0], ds0);
+          lds_read_tr16<i * kRows * 64>(fs[i][1], ds1);
+          static_for<MB>([&](auto m_tag) {
+            constexpr int m = decltype(m_tag)::value;
+            lds_read_tr16<i * TILE_BYTES>(fk[i][m][0], k0 ^ (m * 64));
+            lds_read_tr16<i * TILE_BYTES>(fk[i][m][1], k1 ^ (m * 64));
+          });
+        });
+        static_for<n>([&](auto i_tag) {
+          constexpr int i = decltype(i_tag)::value;
+          constexpr int kLater = (n - 1 - i) * (2 + 2 * MB), kLeft = kLater < 15 ? kLater : 15;  // 4-bit count
+          if constexpr (MB == 1)
+            asm volatile("s_waitcnt lgkmcnt(%4)" : "+v"(fs[i][0]), "+v"(fs[i][1]), "+v"(fk[i][0][0]), "+v"(fk[i][0][1]) : "n"(kLeft) : "memory");
+          else
+            asm volatile("s_waitcnt lgkmcnt(%6)"
+                         : "+v"(fs[i][0]), "+v"(fs[i][1]), "+v"(fk[i][0][0]), "+v"(fk[i][0][1]), "+v"(fk[i][MB - 1][0]), "+v"(fk[i][MB - 1][1])
+                         : "n"(kLeft) : "memory");
+          const u32x4 sbits = {fs[i][0][0], fs[i][0][1], fs[i][1][0], fs[i][1][1]};
+#pragma unroll
+          for (int m = 0; m < MB; ++m) {
+            const u32x4 kbits = {fk[i][m][0][0], fk[i][m][0][1], fk[i][m][1][0], fk[i][m][1][1]};
+            dqacc[m] = Mfma16<T>::run(__builtin_bit_cast(vec_t, kbits), __builtin_bit_cast(vec_t, sbits), dqacc[m]);
+          }
+        });
+      };
+      int tile = 0;
+      if constexpr (MB == 1)
+        for (; tile + 4 <= tiles; tile += 4) contract(tile, std::integral_constant<int, 4>{});
+      for (; tile + 2 <= tiles; tile += 2) contract(tile, std::integral_constant<int, 2>{});
+      if (tiles & 1) contract(tile, std::integral_constant<int, 1>{});
+      vm_wait<0>();  // the next chunk's transfers, before this chunk's stores join the queue
+      const int q_row = qc0 + 16 * q_half + i16;
+      if (q_row < q_valid) {
+#pragma unroll
+        for (int m = 0; m < MB; ++m) {
+          vec4_t out;
+#pragma unroll
+          for (int e = 0; e < 4; ++e) out[e] = static_cast<T>(LATE_SCALE ? dqacc[m][e] * p.scale : dqacc[m][e]);
+          *reinterpret_cast<vec4_t*>(dqb + q_row * p.dqs[2] + 32 * m + 16 * d_col + 4 * g16) = out;
+        }
+      }
+      buf ^= 1;
+    }
+    __syncthreads();  // the images now hold the output tiles
+    uint8_t* out_tile = smem + wave * (32 * (ROWB + 16));
+    const int k_store_end = COMPACT ? len : p.Tk;
+#pragma unroll
+    for (int t = 0; t < NT; ++t) {
+      const int key0 = (own + t * kWaves) * 32;
+      if (key0 >= n_tiles * 32) break;
+      if (LATE_SCALE) {
+#pragma unroll
+        for (int mb = 0; mb < MB; ++mb)
+#pragma unroll
+          for (int j = 0; j < 16; ++j) dkacc[t][mb][j] *= p.scale;
+      }
+      store_owned<T, DP>(dkacc[t], out_tile, dkb, p.dks[2], key0, k_store_end, p.d, lane);
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+      store_owned<T, DP>(dvacc[t], out_tile, dvb, p.dvs[2], key0, k_store_end, p.d, lane);
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    }
+  }
+  if (!COMPACT) {  // rows without a gradient
+    vec_t zero;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) zero[e] = static_cast<T>(0.f);
+    const int piece = (tid % C8) * 8;
+    for (int row = q_end + tid / C8; row < p.Tq; row += kThreads / C8) *reinterpret_cast<vec_t*>(dqb + row * p.dqs[2] + piece) = zero;
+    for (int row = (q_end > 0 ? n_tiles * 32 : 0) + tid / C8; row < p.Tk; row += kThreads / C8) {
+      *reinterpret_cast<vec_t*>(dkb + row * p.dks[2] + piece) = zero;
+      *reinterpret_cast<vec_t*>(dvb + row * p.dvs[2] + piece) = zero;
+    }
+  }
+}
+
 bool strides_ok(const int64_t* st) {
   if (!st || st[3] != 1) return false;
   for (int i = 0; i < 3; ++i)
@@ -729,10 +1106,38 @@ bool small_offsets(int64_t rows, int64_t stride) {
   return stride < (1 << 22) && rows < (1 << 22) && rows * stride * 2 < (1ll << 31);
 }
 
+// The fused kernel where a workgroup can hold a sample's keys (512 of 32 features, 256 of 64) and there are enough (sample, head)
+// pairs: it has one workgroup per pair where the two kernels have one per 128 rows. Both sides in us, lengths ~ U{16..rows}:
+//   up to 128 rows (as many workgroups either way):  8 x 48 x 32, 256 pairs 9.0 -> 6.3, 16384 pairs 113 -> 113; 128 x 64 15.5 -> 11.5
+//   256 x 32:  256 pairs 17.3 -> 18.5, 512 pairs 25.3 -> 24.1, 4096 pairs 134 -> 99;  256 x 64:  256 pairs 26.8 -> 27.5, 512 pairs 46 -> 37,
+//   8192 pairs 493 -> 343;  512 x 32:  512 pairs 52 -> 60 (causal 46 -> 42), 1024 pairs 101 -> 96, 16384 pairs 1443 -> 1024.
+// Mask bits over more than 256 rows of 32 features stay with the two kernels: the words' registers are the ones that the four key
+// tiles of a wavefront need (300 rows, 1024 pairs: 65 -> 74; 512 rows 131 -> 130).
+template <typename T, int DP, int MODE, bool COMPACT>
+bool launch_bwd_fused(AttnBwdParams p, hipStream_t s) {
+  constexpr int kSmall = 64 / DP, kLarge = 128 / DP;  // key tiles per wavefront
+  constexpr int kRowsSmall = kSmall * kOwn, kRowsLarge = DP == 32 && MODE == kMaskBits ? kRowsSmall : kLarge * kOwn;
+  const int64_t pairs = static_cast<int64_t>(p.B) * p.H;
+  const int32_t rows = p.Tq > p.Tk ? p.Tq : p.Tk;
+  const int64_t enough = rows <= kOwn ? 1 : (DP == 32 && rows > kRowsSmall && !p.causal ? 1024 : 512);
+  if (rows > kRowsLarge || pairs < enough) return false;
+  if (!small_offsets(p.Tq, p.qs[2]) || !small_offsets(p.Tq, p.dos[2]) || !small_offsets(p.Tk, p.ks[2])) return false;
+  p.nblk = 1;
+  p.total = static_cast<uint32_t>(pairs);
+  if (rows <= kRowsSmall)
+    hipLaunchKernelGGL((attn_bwd_fused_kernel<T, DP, kSmall, MODE, COMPACT>), dim3(p.total), dim3(kThreads), 0, s, p);
+  else if constexpr (kRowsLarge > kRowsSmall)
+    hipLaunchKernelGGL((attn_bwd_fused_kernel<T, DP, kLarge, MODE, COMPACT>), dim3(p.total), dim3(kThreads), 0, s, p);
+  return true;
+}
+
 template <typename T, int DP, int MODE, bool COMPACT>
 void launch_bwd_form(AttnBwdParams p, bool register_staging, hipStream_t s) {
   // TAAC_ATTN_REGISTER_STAGING keeps the register-staged kernels for full head dims too (comparison route of the caller).
   const bool direct = p.d == DP && !register_staging;
+  if constexpr (MODE == kMaskNone || MODE == kMaskBits) {
+    if (direct && launch_bwd_fused<T, DP, MODE, COMPACT>(p, s)) return;
+  }
   p.nblk = static_cast<uint32_t>((p.Tq + kOwn - 1) / kOwn);
   p.total = p.nblk * p.B * p.H;
   if (direct && small_offsets(p.Tk, p.ks[2]) && small_offsets(p.Tk, p.vs[2]))

@@ -46,6 +46,18 @@ __device__ __forceinline__ void lds_dma16_offset(const void* base, uint32_t lane
       : "memory", "m0");
 }
 
+// 4 bytes per lane from global memory straight into LDS; lane l lands at lds_wave_base + 4 * l.
+__device__ __forceinline__ void lds_dma4(const void* gsrc, void* lds_wave_base) {
+  const uint32_t base = __builtin_amdgcn_readfirstlane(lds_offset(lds_wave_base));
+  asm volatile(
+      "s_mov_b32 m0, %1\n\t"
+      "s_nop 0\n\t"
+      "global_load_lds_dword %0, off"
+      :
+      : "v"(gsrc), "s"(base)
+      : "memory", "m0");
+}
+
 // Transposed 64-bit read: element e of lane j of a 16-lane group receives element j % 4 of the 8-byte row whose address
 // lane 4 * e + j / 4 of that group supplies.
 template <int OFFSET>

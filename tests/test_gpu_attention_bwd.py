@@ -174,3 +174,117 @@ def test_dropout_draws_its_own_mask_and_rejects_what_it_does_not_cover(device):
         flash_attention(q, k, v, dropout_p=0.5, training=False)
     with pytest.raises(ValueError, match="dropout_mask must be uint8"):
         flash_attention(q, k, v, dropout_p=0.5, training=True, dropout_mask=torch.ones(2, 2, 64, 63, dtype=torch.uint8, device=device))
+
+
+def _native_backward(q, k, v, out, grad_out, lse, lengths, causal, zero_pad, *, staged=False, words=None, visible=None, key_valid=None):
+    """dq, dk, dv through the C ABI (poisoned with NaN before the call); ``staged``: the register-staged kernels; ``words``:
+    mask bits with optional validity words; ``visible``: the same mask as bytes."""
+    from taac_2026_amd import _native
+
+    library = _native.load_library()
+    grads = [torch.full_like(t, float("nan")) for t in (q, k, v)]
+    delta = torch.empty_like(lse)
+    (batch, heads, rows, dim), keys = q.shape, k.shape[2]
+    strides = [_native.Int64x4(*t.stride()) for t in (q, k, v, out, grad_out, *grads)]
+    head = [t.data_ptr() for t in (q, k, v, out, grad_out, lse)] + [_native.ptr(lengths)]
+    outs = [t.data_ptr() for t in (*grads, delta)]
+    tail = [_native.dtype_code(q.dtype), _native.current_stream(q.device)]
+    if words is not None:
+        status = library.taac_flash_attn_bits_bwd(*head, words.data_ptr(), words.stride(0), _native.ptr(key_valid), None, 1.0, *outs,
+                                                  batch, heads, rows, keys, dim, *strides, int(zero_pad), *tail)
+    elif visible is not None:
+        status = library.taac_flash_attn_mask_bwd(*head, visible.data_ptr(), rows * keys, 0, None, *outs, batch, heads, rows, keys, dim,
+                                                  *strides, int(zero_pad), *tail)
+    else:
+        status = library.taac_flash_attn_bwd(*head, *outs, batch, heads, rows, keys, dim, *strides, int(causal) | (2 if staged else 0),
+                                             int(zero_pad), *tail)
+    _native.check(status, "backward")
+    return grads
+
+
+def _log_sum_exp(q, k, visible):
+    """out-independent statistics in float64: log-sum-exp of the visible scaled scores and the probabilities."""
+    scores = (q.double() @ k.double().transpose(-1, -2)) / q.shape[-1] ** 0.5
+    scores = scores.masked_fill(~visible, float("-inf"))
+    return torch.logsumexp(scores, dim=-1), torch.nan_to_num(torch.softmax(scores, dim=-1), nan=0.0)
+
+
+def _exact_gradients(q, k, v, out, grad_out, probabilities):
+    """The closed form in float64, with D from the saved output as the kernels take it, and the same sums over the terms'
+    absolute values."""
+    def gradients(q, k, v, out, g, sign):
+        d = (g * out).sum(-1, keepdim=True)
+        ds = probabilities * (g @ v.transpose(-1, -2) - sign * d) * q.shape[-1] ** -0.5
+        return ds @ k, ds.transpose(-1, -2) @ q, probabilities.transpose(-1, -2) @ g
+
+    tensors = [t.double() for t in (q, k, v, out, grad_out)]
+    return list(zip(gradients(*tensors, 1.0), gradients(*(t.abs() for t in tensors), -1.0)))
+
+
+def _check_gradients(got, other, exact, dtype):
+    # a term's probability or dS is rounded to 16 bits and so is the sum: 2^-8 of it (bf16: 8 bits) or 2^-11 (fp16: 11 bits) each
+    unit = 2.0 ** -7 if dtype == torch.bfloat16 else 2.0 ** -10
+    for name, a, s, (e, size) in zip(("dq", "dk", "dv"), got, other, exact):
+        assert not torch.isnan(a).any(), name
+        assert (a[size == 0] == 0).all(), name  # padding and samples without a key
+        error, error_other = (a.double() - e), (s.double() - e)
+        assert (error.abs() <= unit * size + 1e-6).all(), name
+        assert error.norm() <= 1.05 * error_other.norm() + 1e-6 * size.norm(), (name, error.norm(), error_other.norm())
+
+
+# One workgroup per (sample, head): one to four key tiles per wavefront, their last ones partly filled, and sizes on both sides of
+# what such a workgroup holds; pairs as many as the dispatch asks for.
+@pytest.mark.parametrize("rows,keys,dim,batch,heads", [
+    (1, 1, 32, 3, 2), (31, 31, 64, 3, 2), (33, 33, 32, 3, 2), (128, 128, 64, 5, 2), (100, 37, 32, 3, 2), (20, 128, 64, 3, 2),
+    (129, 129, 32, 64, 8), (256, 256, 32, 64, 8), (257, 257, 32, 128, 8), (490, 490, 32, 128, 8), (512, 512, 32, 128, 8),
+    (129, 129, 64, 128, 4), (256, 256, 64, 128, 4), (257, 257, 64, 128, 4)])
+@pytest.mark.parametrize("dtype,causal,zero_pad", [(torch.bfloat16, False, True), (torch.float16, True, False), (torch.bfloat16, True, True)])
+def test_backward_with_all_keys_in_one_workgroup(device, rows, keys, dim, batch, heads, dtype, causal, zero_pad):
+    if rows != keys and zero_pad:
+        pytest.skip("zero_padded_queries needs as many queries as keys")
+    g = torch.Generator(device=device).manual_seed(rows * 3 + dim)
+    # the projection layout: heads next to each other in a row
+    draw = lambda n: torch.randn(batch, n, heads, dim, generator=g, device=device).to(dtype).transpose(1, 2)  # noqa: E731
+    q, k, v, grad_out = draw(rows), draw(keys), draw(keys), draw(rows)
+    lengths = torch.randint(0, keys + 1, (batch,), generator=g, device=device, dtype=torch.int32)
+    lengths[0], lengths[1], lengths[2] = keys, 0, max(1, keys - 1)
+    index = torch.arange(keys, device=device)
+    visible = (index < lengths[:, None])[:, None, None, :].expand(batch, 1, rows, keys)
+    if causal:
+        visible = visible & (index <= torch.arange(rows, device=device)[:, None])
+    if zero_pad:
+        visible = visible & (torch.arange(rows, device=device) < lengths[:, None])[:, None, :, None]
+    lse, p = _log_sum_exp(q, k, visible)
+    out = (p @ v.double()).to(dtype)
+    exact = _exact_gradients(q, k, v, out, grad_out, p)
+    args = (q, k, v, out, grad_out, lse.float().contiguous(), lengths, causal, zero_pad)
+    got, staged = _native_backward(*args), _native_backward(*args, staged=True)
+    _check_gradients(got, staged, exact, dtype)
+    assert all(torch.equal(a, b) for a, b in zip(got, _native_backward(*args)))
+
+
+@pytest.mark.parametrize("rows,dim,batch,heads,valid", [(40, 32, 3, 2, True), (128, 64, 3, 2, False), (250, 32, 64, 8, True),
+                                                        (300, 32, 128, 8, False), (129, 64, 128, 4, False), (255, 64, 128, 4, True)])
+def test_mask_bits_backward_with_all_keys_in_one_workgroup(device, rows, dim, batch, heads, valid):
+    g = torch.Generator(device=device).manual_seed(rows + dim)
+    draw = lambda: torch.randn(batch, heads, rows, dim, generator=g, device=device).to(torch.bfloat16)  # noqa: E731
+    q, k, v, grad_out = draw(), draw(), draw(), draw()
+    lengths = torch.randint(1, rows + 1, (batch,), generator=g, device=device, dtype=torch.int32)
+    words_per_row = (rows + 31) // 32
+    bits = torch.rand(batch, rows, words_per_row * 32, generator=g, device=device) < 0.4
+    weights = (1 << torch.arange(32, device=device, dtype=torch.int64))
+    pack = lambda t: (t.reshape(*t.shape[:-1], words_per_row, 32) * weights).sum(-1).to(torch.int32).contiguous()  # noqa: E731
+    words = pack(bits)
+    key_valid = torch.rand(batch, words_per_row * 32, generator=g, device=device) < 0.8
+    index = torch.arange(rows, device=device)
+    visible = bits[:, :, :rows] & (index < lengths[:, None])[:, None, :]
+    if valid:
+        visible = visible & key_valid[:, None, :rows]
+    alive = visible & (index < lengths[:, None])[:, :, None]
+    lse, p = _log_sum_exp(q, k, alive[:, None])
+    out = (p @ v.double()).to(torch.bfloat16)
+    exact = _exact_gradients(q, k, v, out, grad_out, p)
+    args = (q, k, v, out, grad_out, lse.float().contiguous(), lengths, False, True)
+    got = _native_backward(*args, words=words, key_valid=pack(key_valid) if valid else None)
+    dense = _native_backward(*args, visible=visible.to(torch.uint8).contiguous())
+    _check_gradients(got, dense, exact, torch.bfloat16)
