@@ -231,8 +231,16 @@ void launch_bag_bwd(const void* values, int64_t bags, int bag_size, const void* 
 // The kernels above add every slot's row to an fp32 copy of the table in memory: the copy is cleared, hit by one atomic per
 // slot and feature, and read again to be rounded (1 000 000 x 64 in fp16, 786 000 slots: 37 + 176 + 95 us). Here the slots are
 // sorted by the row they name - a count per row, a start per row, the slots placed - and a row's sum is formed in registers and
-// written once, rounded. The order within a row, and the order of the rows' segments, is whatever the atomics gave: no scan over
-// workgroups (1 000 000 x 64, the same slots: count 57, start 13, place 19, rows 48 us). Rows named more than kHot times are cut into chunks that workgroups of their own sum up; the row then adds those.
+// written once, rounded. The order within a row, and the order of the rows' segments, is whatever the atomics gave. Rows named
+// more than kHot times are cut into chunks that workgroups of their own sum up; the row then adds those.
+// The sort is bound by its atomics (one per slot on counts of every row in memory: 57 us of 94 for the above) and its scattered
+// accesses. It therefore goes over kBuckets sets of rows: a workgroup counts its share of the slots per set in LDS and reserves
+// its places with one add per set, places the slots set by set, and one workgroup per set then counts, scans and places by row
+// in LDS. The sets are dealt out in runs of kRun rows, so that popular neighbours spread over all of them. Measured for the
+// above: counts 10, places 13, sort 13 us; the whole gradient 145 -> 91 us, 40 000 x 64 with 400 000 x 10 slots 691 -> 216, 2 000 000 x 16
+// with 524 288 x 12 528 -> 260. 4096 slots a share: with half as many the adds on the sets' cursors cost more (98 us) than the
+// second workgroup per compute unit gives.
+// A small table with many slots is counted as a whole in LDS instead.
 // Bound: the table's gradient (written once) and the gathered rows of grad_out.
 constexpr int kHot = 64;        // longest row that one lane group sums by itself
 constexpr int kHotChunk = 256;  // entries of a chunk, at least
@@ -240,6 +248,12 @@ constexpr int kHotParts = 64;   // chunks of a row, at most
 constexpr int kRowsPerThread = 8;
 constexpr int kLocalRows = 16384;  // largest table whose counts a workgroup keeps in LDS
 constexpr int kLocalThreads = 1024;
+constexpr int kBuckets = 256;       // sets of rows
+constexpr int kRun = 8;             // consecutive rows of a set
+constexpr int kBucketRows = kLocalThreads * kRowsPerThread;  // rows of a set that are counted at once
+constexpr int kCursors = 64 + kBuckets;  // places of the cursors in front of the counts, whole cache lines
+constexpr int kBucketShare = 4096;  // slots of a workgroup, at least
+constexpr int kBucketShares = 512;  // workgroups, at most (about)
 
 struct BagEntry {
   int32_t bag;
@@ -249,16 +263,32 @@ struct HotChunk {
   int32_t first, count, chunks;  // entries; chunks of the row (in its first chunk)
 };
 struct SortedBags {
-  int32_t* counts;   // [n]; of a hot row after the start kernel: -1 - its first chunk
-  int32_t* cursors;  // entries, chunks (behind counts: cleared with them)
-  int32_t* start;    // [n]
-  int32_t* rank;     // [slots]
+  int32_t* cursors;  // entries, chunks; per set its entries (cleared together)
+  int32_t* counts;   // [rows], behind the cursors; of a hot row after the start kernel: -1 - its first chunk
+  int32_t* start;    // [rows]
+  int32_t* rank;     // [slots]: place within the row (whole table in LDS), row within the set
   BagEntry* entries; // [slots]
+  BagEntry* by_set;  // [slots]: entries set by set
+  int32_t* offsets;  // [shares][kBuckets]: where a share's entries of a set begin, within the set
   HotChunk* chunks;  // [slots / kHot]
   float* partial;    // [slots / kHot][emb_dim]
+  int32_t set_rows;  // rows of a set, a multiple of kRun; 0: not sorted by sets, rows in their order
+  int32_t share_bags, shares;
   int64_t bytes;
+
+  // Position of a row in counts and start.
+  __device__ __forceinline__ int64_t position(int64_t row) const {
+    if (set_rows == 0) return row;
+    const uint32_t r = static_cast<uint32_t>(row), run = r / kRun;  // fewer than 2^30 rows
+    return static_cast<int64_t>(run % kBuckets) * set_rows + run / kBuckets * kRun + r % kRun;
+  }
 };
-SortedBags sorted_layout(char* base, int64_t n, int64_t slots, int emb_dim) {
+// Whether the counts of the whole table are formed in LDS: every workgroup clears and adds up all of them, and in the sets' form the
+// adds of few rows queue up in LDS. In LDS / by sets, us: 1 000 x 32, 524 288 x 12 slots 229 / 564; 1 000 x 16, 65 536 x 4 49.6 / 52.5;
+// 16 000 x 128, 30 000 x 12 126 / 62.
+bool counts_in_lds(int64_t n, int64_t slots) { return n <= kLocalRows && slots >= 256 * std::max<int64_t>(n, kLocalThreads); }
+
+SortedBags sorted_layout(char* base, int64_t n, int64_t bags, int bag_size, int emb_dim) {
   SortedBags b{};
   char* at = base;
   auto take = [&](int64_t bytes) {
@@ -266,11 +296,24 @@ SortedBags sorted_layout(char* base, int64_t n, int64_t slots, int emb_dim) {
     at += (bytes + 255) & ~static_cast<int64_t>(255);
     return here;
   };
-  b.counts = reinterpret_cast<int32_t*>(take((n + 2) * 4));
-  b.cursors = b.counts + n;
-  b.start = reinterpret_cast<int32_t*>(take(n * 4));
+  const int64_t slots = bags * bag_size;
+  int64_t rows = n;
+  if (!counts_in_lds(n, slots)) {
+    b.set_rows = static_cast<int32_t>((n + kRun * kBuckets - 1) / (kRun * kBuckets) * kRun);
+    rows = static_cast<int64_t>(b.set_rows) * kBuckets;
+    const int64_t share = std::max<int64_t>(kBucketShare, slots / kBucketShares);
+    b.share_bags = static_cast<int32_t>(std::max<int64_t>(1, share / bag_size));
+    b.shares = static_cast<int32_t>((bags + b.share_bags - 1) / b.share_bags);
+  }
+  b.cursors = reinterpret_cast<int32_t*>(take((kCursors + rows) * 4));
+  b.counts = b.cursors + kCursors;
+  b.start = reinterpret_cast<int32_t*>(take(rows * 4));
   b.rank = reinterpret_cast<int32_t*>(take(slots * 4));
   b.entries = reinterpret_cast<BagEntry*>(take(slots * static_cast<int64_t>(sizeof(BagEntry))));
+  if (b.set_rows > 0) {
+    b.by_set = reinterpret_cast<BagEntry*>(take(slots * static_cast<int64_t>(sizeof(BagEntry))));
+    b.offsets = reinterpret_cast<int32_t*>(take(static_cast<int64_t>(b.shares) * kBuckets * 4));
+  }
   b.chunks = reinterpret_cast<HotChunk*>(take(slots / kHot * static_cast<int64_t>(sizeof(HotChunk))));
   b.partial = reinterpret_cast<float*>(take(slots / kHot * emb_dim * 4));
   b.bytes = at - base;
@@ -284,16 +327,7 @@ __global__ __launch_bounds__(kBlock) void bag_clear_kernel(int32_t* __restrict__
     if (i + e < n) counts[i + e] = 0;
 }
 
-template <typename I>
-__global__ __launch_bounds__(kBlock) void bag_count_kernel(const I* __restrict__ values, int64_t slots, int64_t n, SortedBags b) {
-  const int64_t i = static_cast<int64_t>(blockIdx.x) * kBlock + threadIdx.x;
-  if (i >= slots) return;
-  const int64_t id = static_cast<int64_t>(values[i]);
-  if (id > 0 && id < n) b.rank[i] = atomicAdd(b.counts + id, 1);
-}
-
-// The same for a small table, whose rows are named so often that the adds to one row would queue up in memory: a workgroup counts its
-// share of the slots in LDS and reserves each row's places with one add.
+// A table small enough that a workgroup counts its share of the slots in LDS and reserves each row's places with one add.
 template <typename I>
 __global__ __launch_bounds__(kLocalThreads) void bag_count_local_kernel(const I* __restrict__ values, int64_t slots, int32_t n,
                                                                         SortedBags b) {
@@ -317,18 +351,10 @@ __global__ __launch_bounds__(kLocalThreads) void bag_count_local_kernel(const I*
   }
 }
 
-// Starts of the rows' segments: a scan inside the workgroup, one add to the common cursor for all of its rows.
-__global__ __launch_bounds__(kBlock) void bag_start_kernel(int64_t n, SortedBags b) {
-  __shared__ int32_t wave_sum[kBlock / kWave];
-  __shared__ int32_t base;
-  const int64_t r0 = (static_cast<int64_t>(blockIdx.x) * kBlock + threadIdx.x) * kRowsPerThread;
+// Exclusive sum of `mine` over the workgroup's threads; `total`: of all of them. wave_sum: one value per wavefront.
+template <int WAVES>
+__device__ __forceinline__ int32_t block_scan(int32_t mine, int32_t* wave_sum, int32_t& total) {
   const int lane = threadIdx.x % kWave, wave = threadIdx.x / kWave;
-  int32_t c[kRowsPerThread], mine = 0;
-#pragma unroll
-  for (int e = 0; e < kRowsPerThread; ++e) {
-    c[e] = r0 + e < n ? b.counts[r0 + e] : 0;
-    mine += c[e];
-  }
   int32_t upto = mine;
 #pragma unroll
   for (int d = 1; d < kWave; d *= 2) {
@@ -337,27 +363,163 @@ __global__ __launch_bounds__(kBlock) void bag_start_kernel(int64_t n, SortedBags
   }
   if (lane == kWave - 1) wave_sum[wave] = upto;
   __syncthreads();
-  if (threadIdx.x == 0) {
-    int32_t total = 0;
-    for (int w = 0; w < kBlock / kWave; ++w) total += wave_sum[w];
-    base = total > 0 ? atomicAdd(b.cursors, total) : 0;
+  int32_t before = 0;
+  total = 0;
+#pragma unroll
+  for (int w = 0; w < WAVES; ++w) {
+    const int32_t v = wave_sum[w];
+    before += w < wave ? v : 0;
+    total += v;
   }
+  return before + upto - mine;
+}
+
+// A row of `count` entries from `at` on: more than kHot of them are cut into chunks. Returns what counts[] then holds.
+__device__ __forceinline__ int32_t row_chunks(const SortedBags& b, int32_t at, int32_t count) {
+  if (count <= kHot) return count;
+  const int32_t by_parts = (count + kHotParts - 1) / kHotParts, len = by_parts > kHotChunk ? by_parts : kHotChunk;
+  const int32_t chunks = (count + len - 1) / len;  // at most count / kHot
+  const int32_t first = atomicAdd(b.cursors + 1, chunks);
+  for (int32_t k = 0; k < chunks; ++k)
+    b.chunks[first + k] = HotChunk{at + k * len, count - k * len < len ? count - k * len : len, chunks};
+  return -1 - first;
+}
+
+// Starts of the rows' segments: a scan inside the workgroup, one add to the common cursor for all of its rows.
+__global__ __launch_bounds__(kBlock) void bag_start_kernel(int64_t n, SortedBags b) {
+  __shared__ int32_t wave_sum[kBlock / kWave];
+  __shared__ int32_t base;
+  const int64_t r0 = (static_cast<int64_t>(blockIdx.x) * kBlock + threadIdx.x) * kRowsPerThread;
+  int32_t c[kRowsPerThread], mine = 0;
+#pragma unroll
+  for (int e = 0; e < kRowsPerThread; ++e) {
+    c[e] = r0 + e < n ? b.counts[r0 + e] : 0;
+    mine += c[e];
+  }
+  int32_t total;
+  int32_t at = block_scan<kBlock / kWave>(mine, wave_sum, total);
+  if (threadIdx.x == 0) base = total > 0 ? atomicAdd(b.cursors, total) : 0;
   __syncthreads();
-  int32_t at = base + upto - mine;
-  for (int w = 0; w < wave; ++w) at += wave_sum[w];
+  at += base;
 #pragma unroll
   for (int e = 0; e < kRowsPerThread; ++e) {
     if (r0 + e >= n) break;
     b.start[r0 + e] = at;
-    if (c[e] > kHot) {
-      const int32_t by_parts = (c[e] + kHotParts - 1) / kHotParts, len = by_parts > kHotChunk ? by_parts : kHotChunk;
-      const int32_t chunks = (c[e] + len - 1) / len;  // at most c / kHot
-      const int32_t first = atomicAdd(b.cursors + 1, chunks);
-      for (int32_t k = 0; k < chunks; ++k)
-        b.chunks[first + k] = HotChunk{at + k * len, c[e] - k * len < len ? c[e] - k * len : len, chunks};
-      b.counts[r0 + e] = -1 - first;
-    }
+    if (c[e] > kHot) b.counts[r0 + e] = row_chunks(b, at, c[e]);
     at += c[e];
+  }
+}
+
+// ---- by sets of rows ----
+__device__ __forceinline__ uint32_t bucket_of(int64_t id) { return static_cast<uint32_t>(id) / kRun % kBuckets; }
+
+// Entries of every set: a share's are counted in LDS and reserved with one add, whose result is where they begin in the set.
+template <typename I>
+__global__ __launch_bounds__(kLocalThreads) void bag_set_count_kernel(const I* __restrict__ values, int64_t slots, int bag_size, int64_t n,
+                                                                      SortedBags b) {
+  __shared__ int32_t count[kBuckets];
+  constexpr int kAhead = 4;
+  for (int t = threadIdx.x; t < kBuckets; t += kLocalThreads) count[t] = 0;
+  __syncthreads();
+  const int64_t per = static_cast<int64_t>(b.share_bags) * bag_size, begin = per * blockIdx.x, end = begin + per < slots ? begin + per : slots;
+  for (int64_t i = begin + threadIdx.x; i < end; i += kAhead * kLocalThreads) {
+    int64_t id[kAhead];
+#pragma unroll
+    for (int k = 0; k < kAhead; ++k) id[k] = i + k * kLocalThreads < end ? static_cast<int64_t>(values[i + k * kLocalThreads]) : 0;
+#pragma unroll
+    for (int k = 0; k < kAhead; ++k)
+      if (id[k] > 0 && id[k] < n) atomicAdd(count + bucket_of(id[k]), 1);
+  }
+  __syncthreads();
+  for (int t = threadIdx.x; t < kBuckets; t += kLocalThreads) {
+    const int32_t c = count[t];
+    b.offsets[static_cast<int64_t>(blockIdx.x) * kBuckets + t] = c > 0 ? atomicAdd(b.cursors + 2 + t, c) : 0;
+  }
+}
+
+// The slots set by set, in the shares of the kernel above; one bag per `lanes` lanes (a power of two up to 64).
+template <typename I>
+__global__ __launch_bounds__(kLocalThreads) void bag_set_place_kernel(const I* __restrict__ values, int64_t bags, int bag_size, int64_t n,
+                                                                      int lanes, SortedBags b) {
+  __shared__ int32_t next[kBuckets];
+  __shared__ int32_t wave_sum[kLocalThreads / kWave];
+  const int t = threadIdx.x;
+  int32_t total;
+  const int32_t set_begin = block_scan<kLocalThreads / kWave>(t < kBuckets ? b.cursors[2 + t] : 0, wave_sum, total);
+  if (t < kBuckets) next[t] = set_begin + b.offsets[static_cast<int64_t>(blockIdx.x) * kBuckets + t];
+  __syncthreads();
+  const int lane = t % lanes;
+  const int64_t first = static_cast<int64_t>(blockIdx.x) * b.share_bags;
+  const int64_t last = first + b.share_bags < bags ? first + b.share_bags : bags;
+  for (int64_t bag = first + t / lanes; bag < last; bag += kLocalThreads / lanes) {  // whole lane groups
+    const I* ids = values + bag * bag_size;
+    int count = 0;
+    for (int j = lane; j < bag_size; j += lanes) {
+      const int64_t id = static_cast<int64_t>(ids[j]);
+      count += id > 0 && id < n ? 1 : 0;
+    }
+    for (int d = lanes / 2; d > 0; d /= 2) count += __shfl_xor(count, d);
+    const float inv = 1.0f / static_cast<float>(count > 0 ? count : 1);
+    for (int j = lane; j < bag_size; j += lanes) {
+      const int64_t id = static_cast<int64_t>(ids[j]);
+      if (id > 0 && id < n) {
+        const int32_t at = atomicAdd(next + bucket_of(id), 1);
+        b.by_set[at] = BagEntry{static_cast<int32_t>(bag), inv};
+        b.rank[at] = static_cast<int32_t>(static_cast<uint32_t>(id) / (kRun * kBuckets) * kRun + static_cast<uint32_t>(id) % kRun);
+      }
+    }
+  }
+}
+
+// One workgroup per set: counts, starts and places of its rows in LDS, kBucketRows of them at a time.
+__global__ __launch_bounds__(kLocalThreads) void bag_set_sort_kernel(SortedBags b) {
+  __shared__ int32_t next[kBucketRows];
+  __shared__ int32_t wave_sum[kLocalThreads / kWave];
+  const int t = threadIdx.x, set = blockIdx.x;
+  int32_t begin;
+  block_scan<kLocalThreads / kWave>(t < set ? b.cursors[2 + t] : 0, wave_sum, begin);  // set < kBuckets <= threads
+  const int32_t end = begin + b.cursors[2 + set];
+  int32_t at0 = begin;
+  for (int32_t r0 = 0; r0 < b.set_rows; r0 += kBucketRows) {
+    const int32_t mine0 = t * kRowsPerThread;
+    __syncthreads();  // the places and sums of the rows before are done with
+#pragma unroll
+    for (int e = 0; e < kRowsPerThread; ++e) next[t + e * kLocalThreads] = 0;
+    __syncthreads();
+    for (int32_t i = begin + t; i < end; i += kLocalThreads) {
+      const uint32_t r = static_cast<uint32_t>(b.rank[i] - r0);
+      if (r < static_cast<uint32_t>(kBucketRows)) atomicAdd(next + r, 1);
+    }
+    __syncthreads();
+    int32_t c[kRowsPerThread], mine = 0, total;
+#pragma unroll
+    for (int e = 0; e < kRowsPerThread; ++e) {
+      c[e] = next[mine0 + e];
+      mine += c[e];
+    }
+    int32_t at = at0 + block_scan<kLocalThreads / kWave>(mine, wave_sum, total);
+    if (r0 + mine0 < b.set_rows) {  // kRowsPerThread divides set_rows
+      int32_t starts[kRowsPerThread];
+#pragma unroll
+      for (int e = 0; e < kRowsPerThread; ++e) {
+        starts[e] = next[mine0 + e] = at;
+        const int32_t entries = c[e];
+        c[e] = row_chunks(b, at, entries);
+        at += entries;
+      }
+      const int64_t row = static_cast<int64_t>(set) * b.set_rows + r0 + mine0;
+#pragma unroll
+      for (int e = 0; e < kRowsPerThread; e += 4) {
+        *reinterpret_cast<int4*>(b.start + row + e) = int4{starts[e], starts[e + 1], starts[e + 2], starts[e + 3]};
+        *reinterpret_cast<int4*>(b.counts + row + e) = int4{c[e], c[e + 1], c[e + 2], c[e + 3]};
+      }
+    }
+    __syncthreads();
+    for (int32_t i = begin + t; i < end; i += kLocalThreads) {
+      const uint32_t r = static_cast<uint32_t>(b.rank[i] - r0);
+      if (r < static_cast<uint32_t>(kBucketRows)) b.entries[atomicAdd(next + r, 1)] = b.by_set[i];
+    }
+    at0 += total;
   }
 }
 
@@ -444,7 +606,8 @@ __global__ __launch_bounds__(kBlock) void bag_rows_kernel(const T* __restrict__ 
   const int64_t row = static_cast<int64_t>(blockIdx.x) * (kBlock / G) + threadIdx.x / G;
   if (row >= n) return;
   const bool live = lane * N < emb_dim;
-  const int32_t count = b.counts[row], start = b.start[row];
+  const int64_t position = b.position(row);
+  const int32_t count = b.counts[position], start = b.start[position];
   float acc[N];
 #pragma unroll
   for (int e = 0; e < N; ++e) acc[e] = 0.f;
@@ -468,10 +631,10 @@ __global__ __launch_bounds__(kBlock) void bag_rows_kernel(const T* __restrict__ 
 
 // Whether the sorted form runs: rows of up to 64 whole pieces, 32-bit positions, and enough work that its six launches (against
 // three, or two for fp32) do not decide. Measured back to back, sums in memory / sorted, us, skewed ids, a quarter padding -
-// 16-bit: 1 000 000 x 64, 262 144 x 4 slots 316 / 146, 1 024 x 4 slots 154 / 42; 100 000 x 64, 1 024 x 4 24 / 19; 20 000 x 64,
+// 16-bit: 1 000 000 x 64, 262 144 x 4 slots 316 / 91, 1 024 x 4 slots 154 / 40; 100 000 x 64, 1 024 x 4 24 / 19; 20 000 x 64,
 // 256 x 4 11.7 / 18.9; 30 000 x 128, 65 536 x 3 95 / 78; 50 000 x 32, 30 000 x 2 24 / 35; 1 000 x 32, 524 288 x 12 4 384 / 229 (3 053
 // with the counts in memory), 1 000 x 16, 65 536 x 4 354 / 48, 1 000 x 64, 4 096 x 4 19 / 33.
-// fp32, which the other form sums in place: 1 000 000 x 64, 262 144 x 4 219 / 184, 1 024 x 4 43 / 61; 2 000 000 x 64, 524 288 x 4 420 / 334.
+// fp32, which the other form sums in place: 1 000 000 x 64, 262 144 x 4 219 / 130, 1 024 x 4 43 / 61; 2 000 000 x 64, 524 288 x 4 420 / 237.
 bool sorted_bags(int64_t n, int64_t slots, int emb_dim, int dtype) {
   const int piece = dtype == TAAC_F32 ? 4 : 8;
   if (emb_dim % piece != 0 || emb_dim / piece > kWave || slots <= 0 || n > 0x3fffffffLL || slots > 0x3fffffffLL) return false;
@@ -487,24 +650,27 @@ template <typename T, typename I>
 int launch_sorted(const I* values, int64_t bags, int bag_size, const T* grad_out, T* grad_weight, int64_t n, int emb_dim, char* workspace,
                   hipStream_t s, const char* name) {
   const int64_t slots = bags * bag_size;
-  const SortedBags b = sorted_layout(workspace, n, slots, emb_dim);
+  const SortedBags b = sorted_layout(workspace, n, bags, bag_size, emb_dim);
   auto blocks = [](int64_t threads) { return dim3(static_cast<uint32_t>((threads + kBlock - 1) / kBlock)); };
-  hipLaunchKernelGGL(bag_clear_kernel, blocks((n + 2 + 3) / 4), dim3(kBlock), 0, s, b.counts, n + 2);
-  const int64_t share = std::max<int64_t>(4 * n, 4 * kLocalThreads);  // slots of a workgroup, so that its counts pay
-  if (n <= kLocalRows && slots >= 4 * share) {
+  int lanes = 1;
+  while (lanes < bag_size && lanes < kWave) lanes *= 2;
+  const int64_t cleared = kCursors + (b.set_rows > 0 ? 0 : n);
+  hipLaunchKernelGGL(bag_clear_kernel, blocks((cleared + 3) / 4), dim3(kBlock), 0, s, b.cursors, cleared);
+  if (b.set_rows > 0) {
+    hipLaunchKernelGGL(bag_set_count_kernel<I>, dim3(b.shares), dim3(kLocalThreads), 0, s, values, slots, bag_size, n, b);
+    hipLaunchKernelGGL(bag_set_place_kernel<I>, dim3(b.shares), dim3(kLocalThreads), 0, s, values, bags, bag_size, n, lanes, b);
+    hipLaunchKernelGGL(bag_set_sort_kernel, dim3(kBuckets), dim3(kLocalThreads), 0, s, b);
+  } else {
+    const int64_t share = std::max<int64_t>(4 * n, 4 * kLocalThreads);  // slots of a workgroup, so that its counts pay
     auto kernel = bag_count_local_kernel<I>;
     const size_t lds = static_cast<size_t>(n) * 4;
     if (hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, kLocalRows * 4) != hipSuccess)
       return set_error(TAAC_ERR_LAUNCH, "%s: cannot reserve %zu bytes of LDS", name, lds);
     const uint32_t grid = static_cast<uint32_t>(std::min<int64_t>(slots / share, 512));
     hipLaunchKernelGGL(kernel, dim3(grid), dim3(kLocalThreads), lds, s, values, slots, static_cast<int32_t>(n), b);
-  } else {
-    hipLaunchKernelGGL(bag_count_kernel<I>, blocks(slots), dim3(kBlock), 0, s, values, slots, n, b);
+    hipLaunchKernelGGL(bag_start_kernel, blocks((n + kRowsPerThread - 1) / kRowsPerThread), dim3(kBlock), 0, s, n, b);
+    hipLaunchKernelGGL(bag_place_kernel<I>, blocks(bags * lanes), dim3(kBlock), 0, s, values, bags, bag_size, n, lanes, b);
   }
-  hipLaunchKernelGGL(bag_start_kernel, blocks((n + kRowsPerThread - 1) / kRowsPerThread), dim3(kBlock), 0, s, n, b);
-  int lanes = 1;
-  while (lanes < bag_size && lanes < kWave) lanes *= 2;
-  hipLaunchKernelGGL(bag_place_kernel<I>, blocks(bags * lanes), dim3(kBlock), 0, s, values, bags, bag_size, n, lanes, b);
   int rc = check_launch(name);
   if (rc != TAAC_OK) return rc;
   auto go = [&](auto g_tag) {
@@ -601,7 +767,7 @@ extern "C" int64_t taac_embedding_bag_mean_bwd_bytes(int64_t num_embeddings, int
   using namespace taac;
   if (num_embeddings <= 0 || emb_dim <= 0 || bags < 0 || bag_size < 0 || (dtype != TAAC_F32 && dtype != TAAC_BF16 && dtype != TAAC_F16)) return -1;
   const int64_t slots = bags * bag_size;
-  if (sorted_bags(num_embeddings, slots, emb_dim, dtype)) return sorted_layout(nullptr, num_embeddings, slots, emb_dim).bytes;
+  if (sorted_bags(num_embeddings, slots, emb_dim, dtype)) return sorted_layout(nullptr, num_embeddings, bags, bag_size, emb_dim).bytes;
   return dtype == TAAC_F32 ? 0 : num_embeddings * emb_dim * 4;
 }
 

@@ -182,6 +182,11 @@ def test_backward_skips_ids_outside_the_table_and_needs_no_gradient_when_frozen(
     (torch.float32, torch.int64, 70_001, 20, 60_000, 4),      # five of eight lanes hold a piece
     (torch.float32, torch.int32, 17_000, 4, 400_000, 3),      # one piece; counts in memory
     (torch.bfloat16, torch.int64, 600_000, 8, 40, 70),        # bags of more than 64 slots
+    (torch.bfloat16, torch.int64, 1_000, 32, 70_000, 4),      # enough slots per row that every workgroup counts the whole table
+    (torch.float32, torch.int32, 2_200_001, 4, 700_000, 2),   # sets of more rows than are counted at once, the last one partly filled
+    (torch.bfloat16, torch.int32, 2_049, 64, 2_000, 33),      # one run of rows more than there are sets; few rows in chunks
+    (torch.float16, torch.int64, 8, 64, 20_000, 4),           # one run: all slots in one set
+    (torch.float16, torch.int64, 40_000, 128, 9, 6_000),      # a bag larger than a workgroup's share
 ])
 def test_backward_of_sorted_slots(device, dtype, index_dtype, rows, dim, bags, bag_size):
     """The sorted form against float64: an element's error is at most (terms + 2) * 2^-24 of the sum of its terms' magnitudes
