@@ -962,6 +962,23 @@ int taac_stack_train_bwd(const void* grad_out, const void* grad_attn_tokens, con
                          void* grad_head_b, int zero_padded_rows, const void* saved, void* scratch, void* grad_tokens,
                          void* stream);
 
+/*
+ * Inference of a stack of n_blocks interaction blocks (experiments/symbiosis/backbone.py:51-68; no rotary embedding) under padding of
+ * any pattern and a structured mask, as one call: per block taac_norm_linear(_qk)_fwd into the front layout, taac_row_rstd,
+ * taac_flash_attn_masked_fwd and taac_attn_out_ffn_fwd, with the same values as those calls.
+ * tokens: bf16 [B, T, D]; padding: uint8 [B, T], non-zero = padded: such rows of out repeat tokens. rows / n_rows: the other rows
+ * (taac_valid_rows_from_bits); front_rows / lengths: taac_front_rows of them; struct_bits, struct_sample_stride:
+ * taac_mask_front_bits. blocks: qkv_weight = taac_linear_pack_weights_norm, out_weight = taac_linear_pack_weights, up_weight = the
+ * feed-forward's blob (gate first, norm folded; norm_folded: its TAAC_FOLDED_* bits), down_weight unused; the others bf16, 16-byte
+ * aligned; query / key norm weights in all blocks or in none. workspace: taac_stack_fwd_bytes bytes (-1: shape not covered), 256-byte
+ * aligned. out: bf16 [B, T, D], not tokens.
+ */
+int64_t taac_stack_fwd_bytes(int32_t B, int32_t T, int32_t D, int32_t n_blocks, int qk_norm);
+int taac_stack_fwd(const void* tokens, const uint8_t* padding, const int32_t* rows, const int32_t* n_rows, const int32_t* front_rows,
+                   const int32_t* lengths, const uint32_t* struct_bits, int64_t struct_sample_stride, const taac_block_weights* blocks,
+                   int32_t n_blocks, int32_t B, int32_t T, int32_t D, int32_t H, int32_t F, float attn_eps, float ffn_eps, float qk_eps,
+                   int norm_folded, void* workspace, int64_t workspace_bytes, void* out, void* stream);
+
 #ifdef __cplusplus
 }
 #endif

@@ -296,6 +296,11 @@ SIGNATURES: dict[str, tuple[object, list[object]]] = {
         [c_void_p, c_void_p, ctypes.POINTER(BlockWeights), c_int32, c_void_p, c_void_p, c_int32, c_int32, c_int32,
          c_int32, c_int32, c_float, c_void_p, c_int, c_void_p, c_int64, c_void_p, c_void_p, c_void_p],
     ),
+    "taac_stack_fwd_bytes": (c_int64, [c_int32] * 4 + [c_int]),
+    "taac_stack_fwd": (
+        c_int,
+        [c_void_p] * 7 + [c_int64, c_void_p] + [c_int32] * 6 + [c_float] * 3 + [c_int, c_void_p, c_int64, c_void_p, c_void_p],
+    ),
     "taac_stack_train_bytes": (c_int64, [c_int32] * 6 + [c_int, c_int]),
     "taac_stack_train_fwd": (
         c_int,

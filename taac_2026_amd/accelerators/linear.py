@@ -519,6 +519,17 @@ def pack_linear_weight(weight: torch.Tensor, norm_weight: torch.Tensor | None = 
     return packed
 
 
+def packed_block(name: str, params: list, d_model: int, hidden: int) -> tuple[list, int]:
+    """Parameters of an interaction block in the order of ``taac_block_weights`` (bf16) with the cached blobs of its dense layers in the
+    weights' places, and the ``TAAC_FOLDED_*`` bits of the feed-forward's."""
+    attn_norm, qkv, qkv_bias, out, out_bias, ffn_norm, up, up_bias, down, down_bias, query_norm, key_norm = params
+    fold = _fold_choice(name, None, d_model, hidden)
+    blobs = (_packed_linear(qkv, attn_norm), _packed_cache.get((out,), lambda: pack_linear_weight(out)),
+             _packed_ffn(up, down, True, ffn_norm, fold))
+    return ([attn_norm, blobs[0], qkv_bias, blobs[1], out_bias, ffn_norm, blobs[2], up_bias, None, down_bias, query_norm, key_norm],
+            _folded_flags(ffn_norm, fold))
+
+
 def _packed_linear(weight: torch.Tensor, norm_weight: torch.Tensor | None) -> torch.Tensor:
     """Cached blob of a layer, with the weight of the norm in front of it folded in when there is one."""
     if norm_weight is None:

@@ -793,3 +793,142 @@ extern "C" int taac_mask_front_bits(const uint32_t* struct_bits, int32_t T, cons
                      struct_bits, T, rows, B, out_bits);
   return check_launch(name);
 }
+
+namespace taac {
+namespace {
+
+// Workspace of taac_stack_fwd for M = B * T rows.
+struct StackLayout {
+  bf16_t *qkv, *attended;
+  float *sumsq, *scales, *products;  // query / key norms: [2 D / 64][M], [2][M], [n_blocks][D]
+  int64_t bytes;
+};
+StackLayout stack_layout(char* base, int64_t M, int32_t D, int32_t n_blocks, bool qk_norm) {
+  StackLayout l{};
+  int64_t at = 0;
+  auto take = [&](int64_t bytes) {
+    char* here = base + at;
+    at += align256(bytes);
+    return here;
+  };
+  l.qkv = reinterpret_cast<bf16_t*>(take(M * 3 * D * 2));
+  l.attended = reinterpret_cast<bf16_t*>(take(M * D * 2));
+  if (qk_norm) {
+    l.sumsq = reinterpret_cast<float*>(take(M * (2 * D / 64) * 4));
+    l.scales = reinterpret_cast<float*>(take(2 * M * 4));
+    l.products = reinterpret_cast<float*>(take(static_cast<int64_t>(n_blocks) * D * 4));
+  }
+  l.bytes = at;
+  return l;
+}
+
+constexpr int kProductBlocks = 16;
+struct StackSetup {
+  const bf16_t* tokens;
+  bf16_t* out;
+  const uint8_t* padding;  // [M]
+  float* scales;           // [2 M], or null
+  float* products;         // of blocks first_block .., n_blocks of them
+  int64_t M;
+  int32_t D, n_blocks;
+  const bf16_t* query[kProductBlocks];
+  const bf16_t* key[kProductBlocks];
+};
+
+// What a stack needs in front of its blocks: the padded rows of the output (they pass through; the blocks write the others), ones in
+// the norm factors (rows outside the index are read by nobody, but a lane that holds such a row multiplies by it) and the products of
+// the query and key norm weights.
+__global__ __launch_bounds__(kBlock) void stack_setup_kernel(const StackSetup p) {
+  const int64_t i = static_cast<int64_t>(blockIdx.x) * kBlock + threadIdx.x;
+  const int pieces = p.D / 8;
+  if (p.tokens != nullptr && i < p.M * pieces) {
+    if (p.padding[i / pieces] != 0) reinterpret_cast<bf16x8*>(p.out)[i] = reinterpret_cast<const bf16x8*>(p.tokens)[i];
+  }
+  if (p.scales != nullptr && i < 2 * p.M) p.scales[i] = 1.f;
+  if (i < static_cast<int64_t>(p.n_blocks) * p.D) {
+    const int block = static_cast<int>(i / p.D), col = static_cast<int>(i % p.D);
+    p.products[i] = static_cast<float>(p.query[block][col]) * static_cast<float>(p.key[block][col]);
+  }
+}
+
+}  // namespace
+}  // namespace taac
+
+extern "C" int64_t taac_stack_fwd_bytes(int32_t B, int32_t T, int32_t D, int32_t n_blocks, int qk_norm) {
+  if (B <= 0 || T <= 0 || (D != 128 && D != 256) || n_blocks <= 0) return -1;
+  return taac::stack_layout(nullptr, static_cast<int64_t>(B) * T, D, n_blocks, qk_norm != 0).bytes;
+}
+
+extern "C" int taac_stack_fwd(const void* tokens, const uint8_t* padding, const int32_t* rows, const int32_t* n_rows,
+                              const int32_t* front_rows, const int32_t* lengths, const uint32_t* struct_bits,
+                              int64_t struct_sample_stride, const taac_block_weights* blocks, int32_t n_blocks, int32_t B, int32_t T,
+                              int32_t D, int32_t H, int32_t F, float attn_eps, float ffn_eps, float qk_eps, int norm_folded,
+                              void* workspace, int64_t workspace_bytes, void* out, void* stream) {
+  using namespace taac;
+  const char* name = "taac_stack_fwd";
+  if (B <= 0 || T <= 0 || n_blocks <= 0 || H <= 0 || F <= 0)
+    return set_error(TAAC_ERR_INVALID_VALUE, "%s: B, T, n_blocks, H and F must be positive", name);
+  if ((D != 128 && D != 256) || D % H != 0) return set_error(TAAC_ERR_UNSUPPORTED, "%s: D must be 128 or 256 and H divide it", name);
+  if (!tokens || !padding || !rows || !n_rows || !front_rows || !lengths || !struct_bits || !blocks || !out || !workspace)
+    return set_error(TAAC_ERR_INVALID_VALUE, "%s: null pointer", name);
+  if (!aligned16(tokens) || !aligned16(out) || (reinterpret_cast<uintptr_t>(workspace) & 255u) != 0)
+    return set_error(TAAC_ERR_INVALID_VALUE, "%s: tokens and out must be 16-byte, the workspace 256-byte aligned", name);
+  if (tokens == out) return set_error(TAAC_ERR_INVALID_VALUE, "%s: out must not be tokens", name);
+  const bool qk_norm = blocks[0].query_norm_weight != nullptr;
+  for (int i = 0; i < n_blocks; ++i)
+    if ((blocks[i].query_norm_weight != nullptr) != qk_norm || (blocks[i].key_norm_weight != nullptr) != qk_norm)
+      return set_error(TAAC_ERR_INVALID_VALUE, "%s: query and key norms in all blocks or in none", name);
+  const int64_t M = static_cast<int64_t>(B) * T;
+  if (M > 0x3fffffffLL) return set_error(TAAC_ERR_UNSUPPORTED, "%s: at most 2^30 rows", name);
+  const StackLayout l = stack_layout(static_cast<char*>(workspace), M, D, n_blocks, qk_norm);
+  if (workspace_bytes < l.bytes) return set_error(TAAC_ERR_INVALID_VALUE, "%s: the workspace must hold taac_stack_fwd_bytes", name);
+  hipStream_t s = as_stream(stream);
+  for (int first = 0; first == 0 || (qk_norm && first < n_blocks); first += kProductBlocks) {
+    StackSetup setup{};
+    setup.M = M;
+    setup.D = D;
+    if (first == 0) {
+      setup.tokens = static_cast<const bf16_t*>(tokens);
+      setup.out = static_cast<bf16_t*>(out);
+      setup.padding = padding;
+      setup.scales = l.scales;
+    }
+    if (qk_norm) {
+      setup.products = l.products + static_cast<int64_t>(first) * D;
+      setup.n_blocks = n_blocks - first < kProductBlocks ? n_blocks - first : kProductBlocks;
+      for (int i = 0; i < setup.n_blocks; ++i) {
+        setup.query[i] = static_cast<const bf16_t*>(blocks[first + i].query_norm_weight);
+        setup.key[i] = static_cast<const bf16_t*>(blocks[first + i].key_norm_weight);
+      }
+    }
+    const int64_t wide = first == 0 ? M * (D / 8) : 0, products = static_cast<int64_t>(setup.n_blocks) * D;  // (2 M <= M D / 8)
+    const int64_t threads = wide > products ? wide : products;
+    hipLaunchKernelGGL(stack_setup_kernel, dim3(static_cast<uint32_t>((threads + kBlock - 1) / kBlock)), dim3(kBlock), 0, s, setup);
+    const int rc = check_launch(name);
+    if (rc != TAAC_OK) return rc;
+  }
+  const int32_t dh = D / H;
+  const int64_t qkv_strides[4] = {static_cast<int64_t>(T) * 3 * D, dh, 3 * static_cast<int64_t>(D), 1};
+  const int64_t out_strides[4] = {static_cast<int64_t>(T) * D, dh, D, 1};
+  for (int i = 0; i < n_blocks; ++i) {
+    const taac_block_weights& w = blocks[i];
+    const void* x = i == 0 ? tokens : out;
+    int rc = qk_norm ? taac_norm_linear_qk_fwd(x, D, w.attn_norm_weight, attn_eps, nullptr, w.qkv_bias, w.qkv_weight, l.qkv, 3 * D, M, D, H,
+                                               T, nullptr, nullptr, l.sumsq, front_rows, n_rows, rows, 1, stream)
+                     : taac_norm_linear_fwd(x, D, w.attn_norm_weight, attn_eps, nullptr, w.qkv_bias, w.qkv_weight, nullptr, 3 * D, l.qkv,
+                                            3 * D, M, 3 * D, D, front_rows, n_rows, rows, 1, stream);
+    if (rc != TAAC_OK) return rc;
+    if (qk_norm) {
+      rc = taac_row_rstd(l.sumsq, M, D, qk_eps, l.scales, front_rows, n_rows, stream);
+      if (rc != TAAC_OK) return rc;
+    }
+    rc = taac_flash_attn_masked_fwd(l.qkv, l.qkv + D, l.qkv + 2 * D, lengths, struct_bits, struct_sample_stride, nullptr, nullptr, nullptr,
+                                    l.scales, qk_norm ? l.scales + M : nullptr, qk_norm ? l.products + static_cast<int64_t>(i) * D : nullptr,
+                                    l.attended, B, H, T, T, dh, qkv_strides, qkv_strides, qkv_strides, out_strides, 2, TAAC_BF16, stream);
+    if (rc != TAAC_OK) return rc;
+    rc = taac_attn_out_ffn_fwd(l.attended, D, w.out_bias, w.out_weight, x, D, w.ffn_norm_weight, ffn_eps, w.up_bias, w.down_bias, w.up_weight,
+                               out, D, M, D, F, rows, n_rows, front_rows, norm_folded, stream);
+    if (rc != TAAC_OK) return rc;
+  }
+  return TAAC_OK;
+}

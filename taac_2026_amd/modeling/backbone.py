@@ -22,11 +22,12 @@ import torch.nn as nn
 
 from taac_2026_amd import _native
 from taac_2026_amd.accelerators.attention import StructuredAttentionMask, front_structured_mask, qk_norm_rope, rope_table
-from taac_2026_amd.accelerators.linear import (attention_out_ffn, front_rows, norm_linear, qkv_projection, silu_mlp,
+from taac_2026_amd.accelerators.linear import (attention_out_ffn, front_rows, norm_linear, packed_block, qkv_projection, silu_mlp,
                                                swiglu_ffn, swiglu_ffn_backward_supported, swiglu_ffn_dropout, valid_rows)
 from taac_2026_amd.accelerators.tensor_validation import require_cuda_tensors, require_inference
-from taac_2026_amd.modeling.block_training import (InteractionStackFunction, block_form, run_training_block, run_training_stack,
-                                                   training_route_applies, uniform_parameters)
+from taac_2026_amd.modeling.block_training import (InteractionStackFunction, _block_config, block_form, _block_parameters, _called_plainly,
+                                                   run_training_block, run_training_stack, _addresses, training_route_applies,
+                                                   uniform_parameters)
 from taac_2026_amd.modeling.normalization import RMSNorm
 from taac_2026_amd.modeling.sequence import scaled_dot_product_attention
 
@@ -68,6 +69,19 @@ def _as(parameter: torch.Tensor | None, dtype: torch.dtype) -> torch.Tensor | No
 
 def _dense(layer: nn.Linear, x: torch.Tensor, *, residual: torch.Tensor | None = None) -> torch.Tensor:
     return norm_linear(x, _as(layer.weight, x.dtype), _as(layer.bias, x.dtype), residual=residual)
+
+
+def _front_index(structured: StructuredAttentionMask, padding_mask: torch.Tensor, batch: int) -> tuple:
+    """``(index, front, lengths, mask)`` of the front layout: the valid rows, where they go, the samples' numbers of them and the mask's
+    structure gathered per sample. Kept in the mask's cache; rebuilt when the padding mask was written to."""
+    entry = structured.cache.get("front")
+    if entry is None or entry[0] != padding_mask._version:
+        token_count = padding_mask.shape[1]
+        index = valid_rows(None, token_count, padding_mask=padding_mask)
+        entry = (padding_mask._version, index, *front_rows(index, batch, token_count),
+                 front_structured_mask(structured, index, batch))
+        structured.cache["front"] = entry
+    return entry[1:]
 
 
 class SwiGLUFeedForward(nn.Module):
@@ -304,6 +318,12 @@ class UnifiedInteractionBlock(nn.Module):
             return False
         return not (torch.is_grad_enabled() and (tokens.requires_grad or any(p.requires_grad for p in self.parameters())))
 
+    def _front_layout(self, structured, padding_mask: torch.Tensor, token_count: int) -> bool:
+        """Whether the fused route under this mask (and no key lengths) moves every sample's valid tokens to the front."""
+        return (structured is not None and structured.padding_source is padding_mask and structured.query_self is None
+                and not structured.sample_stride and structured.structural.shape == (token_count, token_count)
+                and self.token_layout != "positions")
+
     def _forward_fused(self, tokens, padding_mask, attention_mask, key_lengths, return_attention_tokens, inplace):
         batch, token_count, d_model = tokens.shape
         x = tokens.contiguous()
@@ -318,17 +338,8 @@ class UnifiedInteractionBlock(nn.Module):
         # The indices and the gathered mask depend on the mask object only: the blocks of a stack, which all receive it,
         # share them through its cache.
         front = lengths = None
-        if (structured is not None and key_lengths is None and structured.padding_source is padding_mask
-                and structured.query_self is None and not structured.sample_stride
-                and structured.structural.shape == (token_count, token_count)
-                and self.token_layout != "positions"):
-            entry = structured.cache.get("front")
-            if entry is None or entry[0] != padding_mask._version:  # rebuilt when the padding mask was written to
-                index = valid_rows(None, token_count, padding_mask=padding_mask)
-                entry = (padding_mask._version, index, *front_rows(index, batch, token_count),
-                         front_structured_mask(structured, index, batch))
-                structured.cache["front"] = entry
-            _, index, front, lengths, structured = entry
+        if key_lengths is None and self._front_layout(structured, padding_mask, token_count):
+            index, front, lengths, structured = _front_index(structured, padding_mask, batch)
         elif key_lengths is not None:
             index = valid_rows(key_lengths, token_count)
         elif structured is not None and structured.padding_source is padding_mask:
@@ -478,9 +489,59 @@ def run_interaction_blocks(blocks, tokens: torch.Tensor, padding_mask: torch.Ten
         output = run_training_stack(blocks, tokens, attention_mask, padding_mask)
         if output is not None:
             return output
+    output = _run_fused_stack(blocks, tokens, padding_mask, attention_mask)
+    if output is not None:
+        return output
     for position, block in enumerate(blocks):
         stream, _ = block(stream, padding_mask, attention_mask, return_attention_tokens=False, inplace=position > 0)
     return stream
+
+
+def _run_fused_stack(blocks: list, tokens: torch.Tensor, padding_mask: torch.Tensor, mask) -> torch.Tensor | None:
+    """``blocks`` on their fused route as one native call (same kernels, same values), or None when they do not form one: other
+    settings, another route, layout or gate order, hooks. Called one by one the wrappers around a block's four kernels take the host
+    about 130 us, more than the kernels below some 20 000 tokens."""
+    if not isinstance(mask, StructuredAttentionMask) or not blocks or tokens.ndim != 3 or tokens.numel() == 0:
+        return None
+    batch, token_count, width = tokens.shape
+    if padding_mask.shape != (batch, token_count):
+        return None
+    config, form, table, keep = None, None, [], []
+    for block in blocks:
+        if (type(block).forward is not UnifiedInteractionBlock.forward or type(block)._forward_fused is not UnifiedInteractionBlock._forward_fused
+                or not _called_plainly(block) or not block._fused_route(tokens) or not block._front_layout(mask, padding_mask, token_count)
+                or block.attention.rope_base is not None or not block.ffn.gate_first or getattr(block, "nlir_gate", None) is not None):
+            return None
+        own_config = _block_config(block)
+        params = [_bf16(p) for p in _block_parameters(block)]
+        own_form = block_form("hip UnifiedInteractionBlock", params, width, tokens.device)
+        if config not in (None, own_config) or form not in (None, own_form):
+            return None
+        config, form = own_config, own_form
+        table.append(params)
+    heads, attn_eps, ffn_eps, qk_eps, _ = config
+    hidden, qk_norm = form
+    if width % heads:
+        return None
+    packed = []
+    for params in table:
+        blobs, norm_folded = packed_block("hip UnifiedInteractionBlock", params, width, hidden)
+        packed += blobs
+    x, padding = tokens.contiguous(), padding_mask.contiguous()
+    if x.data_ptr() & 15:
+        x = x.clone()
+    index, front, lengths, front_mask = _front_index(mask, padding_mask, batch)
+    output = torch.empty(x.shape, dtype=x.dtype, device=x.device)
+    library = _native.load_library()
+    nbytes = library.taac_stack_fwd_bytes(batch, token_count, width, len(blocks), int(qk_norm))
+    workspace = torch.empty(nbytes, dtype=torch.uint8, device=x.device)
+    status = library.taac_stack_fwd(
+        x.data_ptr(), padding.data_ptr(), index[0].data_ptr(), index[1].data_ptr(), front.data_ptr(), lengths.data_ptr(),
+        front_mask.struct_bits.data_ptr(), int(front_mask.sample_stride), _addresses(packed, keep), len(blocks), batch, token_count,
+        width, heads, hidden, attn_eps, ffn_eps, qk_eps, norm_folded, workspace.data_ptr(), nbytes, output.data_ptr(),
+        _native.current_stream(x.device))
+    _native.check(status, "interaction blocks")
+    return output
 
 
 class _PlainBlock(nn.Module):

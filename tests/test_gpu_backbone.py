@@ -380,3 +380,37 @@ def test_backbone_on_both_sides_of_the_one_launch_index(device, batch):
     rest = torch.ones(batch, dtype=torch.bool, device=device)
     rest[pick] = False
     assert not emb.grad[rest].any()
+
+
+@pytest.mark.parametrize("width,heads,n_blocks,qk_norm,batch,tokens", [
+    (256, 8, 1, True, 5, 33), (128, 2, 17, True, 3, 70), (128, 4, 3, False, 1, 8), (256, 4, 2, True, 40, 257)])
+def test_fused_stack_equals_single_blocks(device, width, heads, n_blocks, qk_norm, batch, tokens):
+    """The one-call stack against the blocks called one by one, bit for bit (17 blocks: more than one set-up launch), with a sample of
+    padding only; blocks that a hook watches are called."""
+    from taac_2026_amd.api import MetadataAttentionMask, UnifiedInteractionBlock, run_interaction_blocks
+
+    g = torch.Generator().manual_seed(tokens)
+    blocks = torch.nn.ModuleList(UnifiedInteractionBlock(width, heads, 2, qk_norm=qk_norm) for _ in range(n_blocks))
+    with torch.no_grad():
+        for name, p in blocks.named_parameters():
+            p.copy_(torch.randn(p.shape, generator=g) * (0.5 / p.shape[-1] ** 0.5 if p.ndim == 2 else 0.1)
+                    + (1.0 if name.endswith("norm.weight") else 0.0))
+    blocks = blocks.to(device).to(torch.bfloat16).eval()
+    x = torch.randn(batch, tokens, width, generator=g).to(torch.bfloat16).to(device)
+    padding = torch.rand(batch, tokens, generator=g).to(device) < 0.4
+    padding[:, :2] = False
+    if batch > 1:
+        padding[1] = True
+    roles = torch.tensor([0, 1, 2, 7] + [6] * (tokens - 4), device=device)
+    mask_module, kept = MetadataAttentionMask(enabled=True), x.clone()
+    with torch.no_grad():
+        got = run_interaction_blocks(blocks, x, padding, mask_module(padding, roles))
+        mask, stream = mask_module(padding, roles), x
+        for block in blocks:
+            stream, _ = block(stream, padding, mask, return_attention_tokens=False)
+        assert torch.equal(got, stream) and torch.equal(x, kept) and torch.equal(got[padding], x[padding])
+        calls = []
+        handle = blocks[-1].register_forward_hook(lambda *_: calls.append(1))
+        assert torch.equal(run_interaction_blocks(blocks, x, padding, mask), got) and calls == [1]
+        handle.remove()
+        assert run_interaction_blocks(blocks, x[:, ::2], padding[:, ::2].contiguous(), None).shape == x[:, ::2].shape  # no mask: block by block
