@@ -35,7 +35,7 @@ inline int64_t align256(int64_t v) { return (v + 255) & ~static_cast<int64_t>(25
 struct PackedBlock {
   int64_t qkv, out, ffn;          // forward blobs (norm weights folded)
   int64_t ffn_bwd;                // feed-forward backward blob
-  int64_t up_t, qkv_t, out_t;     // [D, 2F] and [D, 3D] row-major transposes, blob of the out projection's transpose
+  int64_t up_t, qkv_t, out_t;     // transposes [D, 2F] and [D, 3D] in dgrad_norm's order, blob of the out projection's transpose
   int64_t vectors;                // bf16: attn_norm D | qkv_bias 3D | out_bias D | ffn_norm D | up_bias 2F | down_bias D | query D | key D
   int64_t bytes;
 };
@@ -124,8 +124,8 @@ __device__ __forceinline__ void vector_piece(const TrainSetup& p, int blk, bf16_
   segment(p.key_norm[blk], D);
 }
 
-// Piece of the transpose [cols, rows] of a row-major weight [rows, cols]: column d, rows c .. c + 7. Consecutive pieces take
-// consecutive columns, so that the eight strided reads of a wavefront are eight contiguous runs.
+// Piece of the transpose [cols, rows] of a row-major weight [rows, cols], in the order of dgrad_norm's weight: column d, rows c .. c + 7.
+// Consecutive pieces take consecutive columns, so that the eight strided reads of a wavefront are eight contiguous runs.
 template <typename TW>
 __device__ __forceinline__ bf16x8 transposed_piece(const TW* w, int rows, int cols, int64_t piece, int64_t* dst) {
   const int d = static_cast<int>(piece % cols);
@@ -133,7 +133,7 @@ __device__ __forceinline__ bf16x8 transposed_piece(const TW* w, int rows, int co
   bf16x8 v;
 #pragma unroll
   for (int e = 0; e < 8; ++e) v[e] = static_cast<bf16_t>(static_cast<float>(w[static_cast<int64_t>(c + e) * cols + d]));
-  *dst = static_cast<int64_t>(d) * rows + c;
+  *dst = transposed_weight_at(d, c, cols);
   return v;
 }
 

@@ -22,6 +22,9 @@ namespace {
 // Bound: HBM (dy, K * 2 bytes per token). Where 256-token workgroups would leave compute units idle a workgroup takes 64 tokens,
 // and a slab's chain (barrier, fragment reads, products, transfers) is the time: eight wavefronts and slabs of 64 columns instead
 // of two and 32, 6 100 tokens, D = 256: K = 2048 43 -> 24 us.
+// The weight lies in panels of 32 columns (transposed_weight_at): a slab of it is one or two runs of memory. As rows of K columns its
+// D pieces of 64 or 128 bytes were a power of two apart and came from the same memory channels: 285 000 tokens, D = 256: K = 2048
+// 401 -> 379 us, K = 768 207 -> 197; 30 000 tokens, both 42.6 -> 38.5.
 // ------------------------------------------------------------------------------------------------------------------
 
 struct DgradParams {
@@ -81,10 +84,9 @@ __global__ __launch_bounds__(TG * FG * kWave, 2) void dgrad_norm_kernel(const Dg
 #pragma unroll
   for (int i = 0; i < WT; ++i) {
     const int row = RPX * (WT * wave + i) + lane / LPR;
-    w_src[i] = p.w_t + static_cast<int64_t>(row) * p.K + ((lane % LPR) ^ swizzle(row)) * 8;
+    w_src[i] = p.w_t + transposed_weight_at(row, ((lane % LPR) ^ swizzle(row)) * 8, D);
   }
-  // every workgroup starts its walk over K at a different slab: with all of them on the same columns of a matrix whose row pitch
-  // is a power of two their requests crowd the same memory channels
+  // every workgroup starts its walk over K at a different slab, so that they do not all ask the same memory channels at once
   const int rot = static_cast<int>((blockIdx.x * 5u) % static_cast<uint32_t>(nslabs));
   const int64_t slab_stride = p.panels ? SLAB / kPanelCols * kPanel : SLAB;
   auto stage = [&](int slab) {
@@ -92,11 +94,11 @@ __global__ __launch_bounds__(TG * FG * kWave, 2) void dgrad_norm_kernel(const Dg
     const int turned = slab + rot;
     const int at = turned >= nslabs ? turned - nslabs : turned;
     const int64_t a0 = at * slab_stride;
-    const int k0 = at * SLAB;
+    const int64_t w0 = transposed_weight_at(0, static_cast<int64_t>(at) * SLAB, D);
 #pragma unroll
     for (int i = 0; i < AT; ++i) lds_dma16(a_src[i] + a0, base + (AT * wave + i) * 1024);
 #pragma unroll
-    for (int i = 0; i < WT; ++i) lds_dma16(w_src[i] + k0, base + kTokBytes + (WT * wave + i) * 1024);
+    for (int i = 0; i < WT; ++i) lds_dma16(w_src[i] + w0, base + kTokBytes + (WT * wave + i) * 1024);
   };
   const int swz = swizzle(l32);  // of any row l32 + a multiple of 32
   int piece_off[SLAB / 16];

@@ -46,7 +46,11 @@ int ffn_bwd_hidden_count(const char* name, const void* x, const float* rstd, con
                          const void* b_up, void* hidden, void* grad_pre, int64_t M, int32_t D, int32_t F, bool gate_first,
                          const int32_t* count, hipStream_t s);
 
-// dx = dres + d rmsnorm(x) applied to dy W (train_dense.hip): dy [M, K], w_t [D, K] (the layer's weight transposed), x [M, D] the
+// Element (row d, column c) of a weight transposed to [D, K], in the order in which dgrad_norm reads it: panels of 32 columns, D rows
+// of 64 bytes each, one behind the other.
+__host__ __device__ inline int64_t transposed_weight_at(int64_t d, int64_t c, int64_t D) { return c / 32 * (D * 32) + d * 32 + c % 32; }
+
+// dx = dres + d rmsnorm(x) applied to dy W (train_dense.hip): dy [M, K], w_t [D, K] (the layer's weight transposed, in panels), x [M, D] the
 // rows in front of the norm, rstd its factor, norm_w [D] its weight. dx may be dres. dy_panels: dy is in panel order.
 int dgrad_norm(const char* name, const void* dy, bool dy_panels, int32_t K, const void* w_t, const void* x, const float* rstd, const void* norm_w,
                const void* dres, void* dx, int64_t M, int32_t D, const int32_t* count, hipStream_t s);
