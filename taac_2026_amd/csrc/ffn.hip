@@ -212,6 +212,8 @@ __device__ __forceinline__ void load_residual(const bf16_t* residual, int64_t ld
 //
 // KEEP (with OUTP): the training forward; x1 and the norm's factor are stored for the backward (p.x1_out, p.rstd_out). A variant
 // of its own: with a run-time test the serving kernel takes 532 instead of 475 us per block of 285 k tokens (D = 256, F = 1024).
+// x1 leaves 64 features at a time behind its projection: stored as a whole in front of the main loop, where nothing hid it, the block took
+// 557 us instead of 476 (30 000 tokens: 86 instead of 67).
 // ------------------------------------------------------------------------------------------------------------------
 template <int D, int TT, int NWAVES, int CPB, bool DEFER, bool OUTP, bool GATE = false, bool GLU = true, bool FOLD = false, bool KEEP = false>
 __global__ __launch_bounds__(NWAVES * kWave, TT == 1 ? 2 : 1) void swiglu_ffn_kernel(const TsParams p) {
@@ -560,21 +562,40 @@ __global__ __launch_bounds__(NWAVES * kWave, TT == 1 ? 2 : 1) void swiglu_ffn_ke
               }
               acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ident[0], hf[t][2 * rb], acc, 0, 0, 0);
               acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ident[1], hf[t][2 * rb + 1], acc, 0, 0, 0);
+              [[maybe_unused]] uint32_t x1_bits[8];  // pairs of x1, in accumulator order
 #pragma unroll
               for (int j = 0; j < 16; j += 2) {
                 const bf16x2 pair = {static_cast<bf16_t>(acc[j]), static_cast<bf16_t>(acc[j + 1])};
                 uint32_t bits = __builtin_bit_cast(uint32_t, pair);
                 asm("" : "+v"(bits));  // opaque: the optimiser otherwise splits the pair into two conversions again
+                x1_bits[j / 2] = bits;
                 acc[j] = __builtin_bit_cast(float, bits << 16);
                 acc[j + 1] = __builtin_bit_cast(float, bits & 0xffff0000u);
                 const bf16x2 rounded = __builtin_bit_cast(bf16x2, bits);
                 ss[t] = __builtin_amdgcn_fdot2_f32_bf16(rounded, rounded, ss[t], false);
               }
+              if constexpr (KEEP) {
+                // Two of the chunk's kKeepStores stores: eight features of a token per lane (the 4-feature runs of the accumulator and of
+                // the other half-wavefront's, exchanged), under way while the next chunk is projected.
+#pragma unroll
+                for (int k = 0; k < 2; ++k) {
+                  const auto r0 = __builtin_amdgcn_permlane32_swap(x1_bits[4 * k], x1_bits[4 * k + 2], false, false);
+                  const auto r1 = __builtin_amdgcn_permlane32_swap(x1_bits[4 * k + 1], x1_bits[4 * k + 3], false, false);
+                  const u32x4 run = {static_cast<uint32_t>(r0[0]), static_cast<uint32_t>(r1[0]), static_cast<uint32_t>(r0[1]),
+                                     static_cast<uint32_t>(r1[1])};
+                  *reinterpret_cast<u32x4*>(p.x1_out + hrow_index[t] * D + c * kNC + rb * 32 + k * 16 + hh * 8) = run;
+                }
+              }
             }
         }
       }
-      // the next chunk has landed (and, with the first wait, the first step of the feed-forward weights)
-      vm_wait<0>();
+      // the next chunk has landed (and, with the first wait, the first step of the feed-forward weights); x1's stores, issued behind
+      // its transfers, may still be under way
+      constexpr int kKeepStores = 4 * TT;
+      if (KEEP && active)
+        vm_wait<kKeepStores>();
+      else
+        vm_wait<0>();
       __syncthreads();
     });
     if (active) {
@@ -620,24 +641,6 @@ __global__ __launch_bounds__(NWAVES * kWave, TT == 1 ? 2 : 1) void swiglu_ffn_ke
         });
         if constexpr (KEEP) {
           if (hh == 0) p.rstd_out[hrow_index[t]] = scale;
-          // x1 itself in the same fragment form: 16-byte stores, two lanes per 32-byte run of a row
-          bf16_t* x1row = p.x1_out + hrow_index[t] * D + hh * 8;
-          static_for<KS>([&](auto kc) {
-            constexpr int ks = decltype(kc)::value;
-            constexpr int mb = ks / 2, jq = 2 * (ks % 2);
-            bf16x4 lo, hi;
-#pragma unroll
-            for (int e = 0; e < 4; ++e) {
-              lo[e] = static_cast<bf16_t>(oacc[t][mb][jq * 4 + e]);
-              hi[e] = static_cast<bf16_t>(oacc[t][mb][(jq + 1) * 4 + e]);
-            }
-            const u32x2 ul = __builtin_bit_cast(u32x2, lo), uh = __builtin_bit_cast(u32x2, hi);
-            const auto r0 = __builtin_amdgcn_permlane32_swap(ul[0], uh[0], false, false);
-            const auto r1 = __builtin_amdgcn_permlane32_swap(ul[1], uh[1], false, false);
-            const u32x4 frag = {static_cast<uint32_t>(r0[0]), static_cast<uint32_t>(r1[0]), static_cast<uint32_t>(r0[1]),
-                                static_cast<uint32_t>(r1[1])};
-            *reinterpret_cast<bf16x8*>(x1row + ks * 16) = __builtin_bit_cast(bf16x8, frag);
-          });
         }
       }
     }

@@ -354,3 +354,28 @@ def test_training_stack_with_the_kernels_of_large_batches(device):
     for name, parameter in model.named_parameters():
         if not name.startswith("head."):
             _near(name, parameter.grad, reference[name].grad, 1)
+
+
+@pytest.mark.parametrize("d_model,heads,batch,tokens,full", [(256, 8, 140, 130, False), (256, 4, 600, 130, True), (128, 4, 300, 130, False)])
+def test_tokens_between_the_halves_of_a_large_batch(device, d_model, heads, batch, tokens, full):
+    """The persistent feed-forward kernel of the training forward stores the tokens between a block's halves while it projects: against
+    the inference route, which writes them with a kernel of their own, over slices of a few wavefronts and, with enough tokens, over
+    whole tiles and a remainder. Both round the projection and the sum once (2^-8 of values below 8: 2^-5 each); on the whole the
+    two differ by one rounding."""
+    g = torch.Generator(device=device).manual_seed(batch)
+    block = UnifiedInteractionBlock(d_model, heads, 2)
+    with torch.no_grad():
+        for name, p in block.named_parameters():
+            p.copy_(torch.randn(p.shape, generator=torch.Generator().manual_seed(len(name))) * (p.shape[-1] ** -0.5 if p.ndim == 2 else 0.1)
+                    + (1.0 if name.endswith("norm.weight") else 0.0))
+    block = block.to(torch.bfloat16).to(device)
+    x = torch.randn(batch, tokens, d_model, generator=g, device=device).to(torch.bfloat16)
+    lengths = torch.randint(tokens - 1 if full else 0, tokens + 1, (batch,), generator=g, device=device, dtype=torch.int32)
+    padding = torch.arange(tokens, device=device) >= lengths[:, None]
+    with torch.no_grad():
+        out, between = block.eval()(x, padding, None, key_lengths=lengths)
+    got_out, got_between = block.train()(x.clone().requires_grad_(True), padding, None, key_lengths=lengths)
+    for got, want in ((got_between, between), (got_out, out)):
+        a, b = got[~padding].float(), want[~padding].float()
+        assert b.abs().max() < 8 and (a - b).abs().max() <= 2.0 ** -4 and (a - b).norm() <= 2.0 ** -8 * b.norm()
+        assert torch.equal(got[padding], x[padding])
