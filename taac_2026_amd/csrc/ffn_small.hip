@@ -190,19 +190,21 @@ __global__ __launch_bounds__(D, 2) void norm_linear_small_kernel(const TsParams 
 // Data that other workgroups of the same launch read: accesses at the scope of the whole chip, which go through the L2 of the die
 // to the memory all dies share. (Ordinary stores with a fence behind them write back and drop everything the die's L2 holds:
 // 8 us per launch.)
-__device__ __forceinline__ void store_through(f32x4* dst, const f32x4& v) {
-  const u32x4 bits = __builtin_bit_cast(u32x4, v);
-  uint64_t* d = reinterpret_cast<uint64_t*>(dst);
-  __hip_atomic_store(d, static_cast<uint64_t>(bits[0]) | static_cast<uint64_t>(bits[1]) << 32, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-  __hip_atomic_store(d + 1, static_cast<uint64_t>(bits[2]) | static_cast<uint64_t>(bits[3]) << 32, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-__device__ __forceinline__ f32x4 load_through(const f32x4* src) {
-  const uint64_t* s = reinterpret_cast<const uint64_t*>(src);
-  const uint64_t lo = __hip_atomic_load(s, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-  const uint64_t hi = __hip_atomic_load(s + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-  const u32x4 bits = {static_cast<uint32_t>(lo), static_cast<uint32_t>(lo >> 32), static_cast<uint32_t>(hi), static_cast<uint32_t>(hi >> 32)};
-  return __builtin_bit_cast(f32x4, bits);
-}
+// Sixteen bytes per lane and access: as atomic accesses, eight bytes at most, twice as many requests leave the compute unit and the
+// last workgroup of a tile takes 5 us for its 256 KB (512 tokens, D = 256, F = 1024, eight splits: 19.7 -> 17.0 us for the kernel).
+// Ordering is the caller's: a wait and a barrier in front of the count that publishes the stores, a barrier behind it for the loads.
+constexpr int kThroughL2 = 16;  // the sc1 bit of a buffer access: coherent at the scope of the chip
+struct SharedPartials {
+  __amdgpu_buffer_rsrc_t rsrc;
+  __device__ __forceinline__ SharedPartials(float* base, int bytes)
+      : rsrc(__builtin_amdgcn_make_buffer_rsrc(base, 0, bytes, 0x00020000)) {}
+  __device__ __forceinline__ void store(int at, const f32x4& v) const {
+    __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, v), rsrc, at, 0, kThroughL2);
+  }
+  __device__ __forceinline__ f32x4 load(int at) const {
+    return __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(rsrc, at, 0, kThroughL2));
+  }
+};
 
 // ------------------------------------------------------------------------------------------------------------------
 // The feed-forward half for few tokens: [out projection + residual ->] RMSNorm -> up -> SiLU-gate -> down -> + residual of
@@ -218,9 +220,10 @@ __device__ __forceinline__ f32x4 load_through(const f32x4* src) {
 // 49.9 -> 21.5 us; 8192 tokens: 55.6 -> 27.8; its line is at ffn_few_rows).
 // splits > 1 (see TsParams): for batches that leave most of the chip idle even so, the hidden units of a tile are also divided over
 // workgroups, eight at most (one request of 512 positions, eight splits, with the requests below ordered by need: the whole
-// 4-block call 164 -> 140 us; fences instead of the write-through accesses: 156). Sixteen lose where tiles and F admit them: a
-// wavefront then has one 16-unit chunk behind the same latency chains (at most 16 / 8 / 4 splits, F = 1024 160 / 140 / 135 us,
-// F = 512 136 / 136 / 127, F = 2048 169 / 151 / 153).
+// 4-block call 164 -> 140 us; fences instead of the write-through accesses: 156; those accesses 16 bytes wide instead
+// of 8: 128 -> 119). Sixteen lose where tiles and F admit them: a wavefront then has one 16-unit chunk behind the same latency
+// chains (at most 16 / 8 / 4 splits, with 8-byte accesses, F = 1024 160 / 140 / 135 us, F = 512 136 / 136 / 127, F = 2048
+// 169 / 151 / 153).
 // LDS: [4 partials of 32 x D floats][x1 (32 padded rows of D bf16)][first-layer bias 2F][4 x 32 row sums]
 // ------------------------------------------------------------------------------------------------------------------
 template <int D, bool OUTP, bool FOLD>
@@ -421,12 +424,13 @@ __global__ __launch_bounds__(4 * kWave, 1) void swiglu_ffn_small_kernel(const Ts
   if (splits > 1) {
     // The partial of this workgroup becomes visible to the chip, then the workgroup counts itself: whoever counts last finds all
     // partials of the tile (nobody waits for anybody). They are added in the order of the splits: the same result every run.
-    f32x4* parts = reinterpret_cast<f32x4*>(p.split_partials) + static_cast<int64_t>(blockIdx.x) * splits * (kPart / 16);
-    f32x4* mine = parts + static_cast<int64_t>(blockIdx.y) * (kPart / 16);
+    const SharedPartials parts(p.split_partials + static_cast<int64_t>(blockIdx.x) * splits * (kPart / 4), splits * kPart);
+    const int lane_at = (wave * MBW * 4 * kWave + lane) * 16;  // of a partial: [feature block][register quad][lane]
+    const int mine = static_cast<int>(blockIdx.y) * kPart + lane_at;
 #pragma unroll
     for (int m = 0; m < MBW; ++m)
 #pragma unroll
-      for (int jq = 0; jq < 4; ++jq) store_through(mine + ((wave * MBW + m) * 4 + jq) * kWave + lane, total[m][jq]);
+      for (int jq = 0; jq < 4; ++jq) parts.store(mine + (m * 4 + jq) * (kWave * 16), total[m][jq]);
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // this wavefront's partials have reached the chip's common memory
     __syncthreads();
     uint32_t* arrived = reinterpret_cast<uint32_t*>(sums);
@@ -443,17 +447,28 @@ __global__ __launch_bounds__(4 * kWave, 1) void swiglu_ffn_small_kernel(const Ts
       for (int jq = 0; jq < 4; ++jq)
 #pragma unroll
         for (int e = 0; e < 4; ++e) total[m][jq][e] = 0.f;
-    for (int w = 0; w < splits; ++w) {
-      const f32x4* other = parts + static_cast<int64_t>(w) * (kPart / 16);
+    auto add_partials = [&](int first_split, auto ahead) {
+      constexpr int kAhead = decltype(ahead)::value;  // partials in flight
+      f32x4 v[kAhead][MBW][4];
 #pragma unroll
-      for (int m = 0; m < MBW; ++m)
+      for (int u = 0; u < kAhead; ++u)
 #pragma unroll
-        for (int jq = 0; jq < 4; ++jq) {
-          const f32x4 v = load_through(other + ((wave * MBW + m) * 4 + jq) * kWave + lane);
+        for (int m = 0; m < MBW; ++m)
 #pragma unroll
-          for (int e = 0; e < 4; ++e) total[m][jq][e] += v[e];
-        }
-    }
+          for (int jq = 0; jq < 4; ++jq)
+            v[u][m][jq] = parts.load((first_split + u) * kPart + lane_at + (m * 4 + jq) * (kWave * 16));
+#pragma unroll
+      for (int u = 0; u < kAhead; ++u)
+#pragma unroll
+        for (int m = 0; m < MBW; ++m)
+#pragma unroll
+          for (int jq = 0; jq < 4; ++jq)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) total[m][jq][e] += v[u][m][jq][e];
+    };
+    // 2, 4 or 8 splits (ffn_splits). Eight partials, 64 KB per wavefront: 17.0 us for the kernel with four in flight, 17.5 with two.
+    if (splits == 2) add_partials(0, std::integral_constant<int, 2>{});
+    for (int w = 0; w + 4 <= splits; w += 4) add_partials(w, std::integral_constant<int, 4>{});
   }
   const bool live = tok0 + l32 < count;
   if (OUTP && p.x1_out != nullptr) {
