@@ -60,6 +60,7 @@ struct Fp8TsParams {
   float* amax_out;          // STATS: receives max |bf16(rmsnorm(out, out_norm_w))| (max |out| without a weight)
   const bf16_t* out_norm_w; // [N] or null
   float out_eps;
+  int32_t whole_tiles;      // a workgroup takes whole tiles; otherwise the steps of a tile may be divided (see the launchers)
 };
 
 __device__ __forceinline__ float clamp448(float x) { return __builtin_fminf(__builtin_fmaxf(x, -448.f), 448.f); }
@@ -93,7 +94,7 @@ __device__ __forceinline__ void lds_wait_halves(u32x4& a, u32x4& b) {
 // per-tensor scale of the layer that consumes the output - without a pass of its own over it.
 // NORM: the rows are RMS-normalised (weight p.norm_w) before they are quantised.
 template <int kK, int EPI, bool A_FP8, bool STATS, bool NORM = false>
-__global__ __launch_bounds__(kWaves * kWave, 2) void linear_fp8_ts_kernel(const Fp8TsParams p, const int /*max_tiles*/) {
+__global__ __launch_bounds__(kWaves * kWave, 2) void linear_fp8_ts_kernel(const Fp8TsParams p) {
   static_assert(!NORM || (kK == 256 && !A_FP8), "the normalisation is built for bf16 rows of 256 features");
   constexpr bool RES = EPI == TAAC_EPI_RESIDUAL;
   constexpr int kTT = tiles_per_wave(kK, EPI);
@@ -133,10 +134,23 @@ __global__ __launch_bounds__(kWaves * kWave, 2) void linear_fp8_ts_kernel(const 
     count = n < p.M ? n : p.M;
   }
   const int num_tiles = static_cast<int>((count + kTokPerWg - 1) / kTokPerWg);
-  const int my_tiles = (num_tiles - static_cast<int>(blockIdx.x) + static_cast<int>(gridDim.x) - 1) /
-                       static_cast<int>(gridDim.x);
-  if (my_tiles <= 0) return;  // whole workgroup: no tile for it (fewer tokens than the grid was sized for)
-  const int total = my_tiles * nsteps_tile;
+  // The steps of all tiles in order, divided evenly and in one run over the workgroups: a step needs nothing of another step of
+  // its tile but the token rows, which a workgroup that starts inside a tile loads as well. Whole tiles, in turn over the
+  // workgroups, leave most of the chip idle where they are few or in a last round of few (256 -> 768 features of normalised rows,
+  // the number of rows on the device, whole tiles / divided: 580 rows 56 / 20 us, 9 200 56 / 22, 37 000 56 / 45, 73 000 57 / 55,
+  // 146 000 122 / 102, 293 000 178 / 164).
+  int first_tile = blockIdx.x, tile_stride = gridDim.x, first_chunk = 0, total;
+  if (p.whole_tiles) {
+    total = (num_tiles - first_tile + tile_stride - 1) / tile_stride * nsteps_tile;
+  } else {
+    const int64_t steps = static_cast<int64_t>(num_tiles) * nsteps_tile;
+    const int64_t first = steps * blockIdx.x / gridDim.x;
+    total = static_cast<int>(steps * (blockIdx.x + 1) / gridDim.x - first);
+    first_tile = static_cast<int>(first / nsteps_tile);
+    first_chunk = static_cast<int>(first % nsteps_tile);
+    tile_stride = 1;
+  }
+  if (total <= 0) return;  // whole workgroup: nothing for it (fewer tokens than the grid was sized for)
   // memory row of token `tok`; tokens at or beyond the count repeat the last one (same values, benign duplicate stores)
   auto row_of = [&](int64_t tok) -> int64_t {
     tok = tok < count ? tok : count - 1;
@@ -172,7 +186,7 @@ __global__ __launch_bounds__(kWaves * kWave, 2) void linear_fp8_ts_kernel(const 
     }
   };
   auto rows_of_tile = [&](int idx) -> int64_t {
-    return (static_cast<int64_t>(blockIdx.x) + static_cast<int64_t>(idx) * gridDim.x) * kTokPerWg + wave * (32 * kTT);
+    return (static_cast<int64_t>(first_tile) + static_cast<int64_t>(idx) * tile_stride) * kTokPerWg + wave * (32 * kTT);
   };
   // Residual pieces in the layout of the epilogue stores: piece t*NSTT + i = token 32*t + ROWS_PER_STORE*i +
   // lane / PIECES, features 8 * (lane % PIECES) .. +7 of the step's OUTC features.
@@ -261,9 +275,9 @@ __global__ __launch_bounds__(kWaves * kWave, 2) void linear_fp8_ts_kernel(const 
   bf16x8 res_cur[NST], res_next[NST];
   int tile_idx = 0;
   int64_t tok_wave = rows_of_tile(0);
-  stage(0, 0);
-  if (total > 1) stage(nsteps_tile > 1 ? 1 : 0, 1);
-  if (RES) request_residual(tok_wave, 0, res_cur);
+  stage(first_chunk, 0);
+  if (total > 1) stage((first_chunk + 1) % nsteps_tile, 1);
+  if (RES) request_residual(tok_wave, first_chunk, res_cur);
   stage_bias(p.bias, bias_lds, p.N, tid, kWaves * kWave);
   if constexpr (NORM) {
     stage_bias(p.norm_w, normw_lds, kK, tid, kWaves * kWave);
@@ -280,9 +294,9 @@ __global__ __launch_bounds__(kWaves * kWave, 2) void linear_fp8_ts_kernel(const 
   for (int i = 0; i < NST; ++i) st_ss[i] = st_mw[i] = 0.f;
 
   uint8_t* tile_lds = tiles + wave * kTileWave;
-  int chunk = 0;                    // step inside the tile
+  int chunk = first_chunk;          // step inside the tile
   int buf = 0;                      // ring slot of step s
-  int chunk2 = 2 % nsteps_tile;     // step s + 2 inside its tile
+  int chunk2 = (first_chunk + 2) % nsteps_tile;  // step s + 2 inside its tile
   for (int s = 0; s < total; ++s) {
     const bool has_next = s + 1 < total;
     const bool stage_ahead = s + 2 < total;
@@ -439,26 +453,33 @@ __global__ __launch_bounds__(kWaves * kWave, 2) void linear_fp8_ts_kernel(const 
 // Launches the token-stationary kernel when the shape fits it: K = 256 (any epilogue, weight rows a multiple of 64) or
 // K = 1024 (no SiLU-gate, weight rows a multiple of 32), 16-byte aligned rows. Returns TAAC_OK after a launch, a negative
 // status on a launch error and 1 when the shape is not covered (the caller then uses the tiled kernel).
+// Whether the output may overwrite rows that another step of the same tile still has to read (rows in place, at any column).
+bool rows_in_place(const Fp8TsParams& p, int a_bytes) {
+  const intptr_t apart = reinterpret_cast<intptr_t>(p.out) - reinterpret_cast<intptr_t>(p.a);
+  const int64_t pitch = p.ldo * 2;
+  return p.lda * a_bytes == pitch && apart < pitch && apart > -pitch;
+}
+
 template <int K>
-int launch_fp8_ts_for_k(const Fp8TsParams& p, int a_is_fp8, int epilogue, hipStream_t s, const char* name) {
+int launch_fp8_ts_for_k(Fp8TsParams p, int a_is_fp8, int epilogue, hipStream_t s, const char* name) {
   const size_t lds_bytes = static_cast<size_t>(3 * step_bytes(K)) + static_cast<size_t>(kWaves) * 32 * tile_row_bytes(K) +
                            static_cast<size_t>(p.N) * 2;
   if (lds_bytes > 160 * 1024) return 1;
   const int tok_per_wg = kWaves * 32 * tiles_per_wave(K, epilogue);
   const int64_t tiles64 = (p.M + tok_per_wg - 1) / tok_per_wg;
   if (tiles64 > 0x3fffffffLL) return 1;
-  const int num_tiles = static_cast<int>(tiles64);
   const int cus = compute_units();
   if (cus <= 0) return set_error(TAAC_ERR_LAUNCH, "%s: cannot query the device", name);
-  int grid = num_tiles < cus ? num_tiles : cus;
+  p.whole_tiles = rows_in_place(p, a_is_fp8 ? 1 : 2);
+  const int64_t most = p.whole_tiles ? tiles64 : tiles64 * (epilogue == TAAC_EPI_SWIGLU ? p.N / 64 : p.N / (row_blocks(K) * 32));
+  int grid = static_cast<int>(most < cus ? most : cus);
   if (const int limit = test_max_workgroups(); limit > 0 && limit < grid) grid = limit;  // taac_test_hooks
 #define TAAC_FP8_TS_LAUNCH(EPI, AF8)                                                                                \
   do {                                                                                                              \
     if (hipFuncSetAttribute(reinterpret_cast<const void*>(linear_fp8_ts_kernel<K, EPI, AF8, false>),                       \
                             hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds_bytes)) != hipSuccess) \
       return set_error(TAAC_ERR_LAUNCH, "%s: cannot reserve %zu bytes of LDS", name, lds_bytes);                    \
-    hipLaunchKernelGGL((linear_fp8_ts_kernel<K, EPI, AF8, false>), dim3(grid), dim3(kWaves * kWave), lds_bytes, s, p,      \
-                       num_tiles);                                                                                  \
+    hipLaunchKernelGGL((linear_fp8_ts_kernel<K, EPI, AF8, false>), dim3(grid), dim3(kWaves * kWave), lds_bytes, s, p);     \
     return check_launch(name);                                                                                      \
   } while (0)
   if (epilogue == TAAC_EPI_NONE) {
@@ -571,18 +592,18 @@ extern "C" int taac_norm_linear_fp8_fwd(const void* x, int64_t ldx, const void* 
   if (lds_bytes > 160 * 1024) return set_error(TAAC_ERR_UNSUPPORTED, "%s: N=%d does not fit the LDS", name, N);
   const int tok_per_wg = kWaves * 32 * tiles_per_wave(256, epilogue);
   const int64_t tiles64 = (M + tok_per_wg - 1) / tok_per_wg;
-  const int num_tiles = static_cast<int>(tiles64);
   const int cus = compute_units();
   if (cus <= 0) return set_error(TAAC_ERR_LAUNCH, "%s: cannot query the device", name);
-  int grid = num_tiles < cus ? num_tiles : cus;
+  p.whole_tiles = amax_out != nullptr || rows_in_place(p, 2);  // (the statistics of a token run over all its features)
+  const int64_t most = p.whole_tiles ? tiles64 : tiles64 * (N / 64);
+  int grid = static_cast<int>(most < cus ? most : cus);
   if (const int limit = test_max_workgroups(); limit > 0 && limit < grid) grid = limit;  // taac_test_hooks
 #define TAAC_NL_FP8(EPI, ST, NM)                                                                                          \
   do {                                                                                                                    \
     if (hipFuncSetAttribute(reinterpret_cast<const void*>(linear_fp8_ts_kernel<256, EPI, false, ST, NM>),                 \
                             hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds_bytes)) != hipSuccess)       \
       return set_error(TAAC_ERR_LAUNCH, "%s: cannot reserve %zu bytes of LDS", name, lds_bytes);                          \
-    hipLaunchKernelGGL((linear_fp8_ts_kernel<256, EPI, false, ST, NM>), dim3(grid), dim3(kWaves * kWave), lds_bytes, s, p, \
-                       num_tiles);                                                                                        \
+    hipLaunchKernelGGL((linear_fp8_ts_kernel<256, EPI, false, ST, NM>), dim3(grid), dim3(kWaves * kWave), lds_bytes, s, p); \
     return check_launch(name);                                                                                            \
   } while (0)
 #define TAAC_NL_FP8_EPI(EPI)                              \

@@ -159,3 +159,34 @@ def test_norm_linear_fp8_fuses_norm_rows_and_the_next_scale(device, test_hooks, 
     assert amax_plain.item() == got[valid].float().abs().max().item()
     expected_next = rms_norm(got[valid].to(device), nxt).float().abs().max().item()
     assert abs(amax_out.item() - expected_next) <= 2 ** -7 * expected_next
+
+
+@pytest.mark.parametrize("m,n", [(1, 64), (513, 768), (1500, 256), (3000, 832)])
+def test_dense_layer_with_its_steps_divided_over_workgroups(device, test_hooks, m, n):
+    """The steps of the tiles run over the workgroups in one sequence, so a workgroup may start and end inside a tile: every
+    number of workgroups gives the same bits, and rows written in place still see their whole input."""
+    g = torch.Generator().manual_seed(m)
+    bf = lambda t: t.to(torch.bfloat16)  # noqa: E731
+    x, w, b, nw = _to(device, bf(torch.randn(m, 256, generator=g)), bf(torch.randn(n, 256, generator=g) / 16),
+                      bf(torch.randn(n, generator=g)), bf(1 + 0.1 * torch.randn(256, generator=g)))
+    res = bf(torch.randn(m, n, generator=g)).to(device)
+    with torch.no_grad():
+        wq, wa = quantize_fp8(w)
+        ax, an = amax(x), amax(rms_norm(x, nw))
+
+        def layers():
+            out = [norm_linear_fp8(x, wq, an, wa, b, norm_weight=nw)[0], linear_fp8(x, wq, ax, wa, b, residual=res),
+                   linear_fp8(x, wq, ax, wa, b, swiglu=True)]
+            if n == 256:
+                held = x.clone()
+                out.append(norm_linear_fp8(held, wq, an, wa, b, norm_weight=nw, out=held)[0])
+            return out
+
+        test_hooks(max_workgroups=1)
+        want = layers()
+        if n == 256:
+            assert torch.equal(want[3], want[0])
+        for workgroups in (None, 2, 5, 11, 100):
+            test_hooks(max_workgroups=workgroups)
+            for got, one in zip(layers(), want):
+                assert torch.equal(got, one)
