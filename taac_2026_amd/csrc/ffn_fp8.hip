@@ -327,7 +327,11 @@ __global__ __launch_bounds__(NW* kWave, 2) void swiglu_ffn_fp8_kernel(const FfnF
     for (int i = 0; i < TPW; ++i) lds_dma16_offset(src + i * 1024, lane_off, dst + i * 1024);
   };
 
-  stage(0, 0);
+  // Pass 1 reduces every hidden unit by itself: its chunks may be divided over blockIdx.y.
+  const int nchunks = nsteps / 2;
+  const int c_begin = PASS2 ? 0 : nchunks * static_cast<int>(blockIdx.y) / static_cast<int>(gridDim.y);
+  const int c_end = PASS2 ? nchunks : nchunks * (static_cast<int>(blockIdx.y) + 1) / static_cast<int>(gridDim.y);
+  stage(2 * c_begin, 0);
   const float amax_x = fmaxf(*p.amax_x, 1e-12f);
   const float amax_up = fmaxf(*p.amax_up, 1e-12f);
   const float dq1 = (amax_x / 448.0f) * (amax_up / 448.0f);
@@ -497,8 +501,7 @@ __global__ __launch_bounds__(NW* kWave, 2) void swiglu_ffn_fp8_kernel(const FfnF
     });
   };
 
-  const int nchunks = nsteps / 2;
-  for (int c = 0; c < nchunks; ++c) {
+  for (int c = c_begin; c < c_end; ++c) {
     // bias fragments of the chunk's four sub-chunks: one dword per lane (row slot l32), k = 0, 1 of the lower half-wavefront
     uint32_t brow[4] = {0u, 0u, 0u, 0u};
     if (BIAS && active) {
@@ -515,7 +518,7 @@ __global__ __launch_bounds__(NW* kWave, 2) void swiglu_ffn_fp8_kernel(const FfnF
     vm_wait<0>();  // the next step's weights (the only vector-memory operations of the loop)
     __syncthreads();
     // second half: buffer 1; the step after it (or, after the last one, the pending down fragments) goes to buffer 0
-    if (c + 1 < nchunks)
+    if (c + 1 < c_end)
       stage(2 * c + 2, 0);
     else if (PASS2)
       stage_tail(0);
@@ -650,14 +653,14 @@ __global__ void f8_clear_kernel(float* a, float* b) {
 bool f8_ptr_ok(const void* p, uintptr_t mask) { return (reinterpret_cast<uintptr_t>(p) & mask) == 0; }
 
 template <typename K>
-int f8_launch(K kernel, const FfnFp8Params& p, int waves, int tokens_per_wg, size_t lds_bytes, hipStream_t s,
+int f8_launch(K kernel, const FfnFp8Params& p, int waves, int tokens_per_wg, int splits, size_t lds_bytes, hipStream_t s,
               const char* name) {
   if (hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize,
                           static_cast<int>(lds_bytes)) != hipSuccess)
     return set_error(TAAC_ERR_LAUNCH, "%s: cannot reserve %zu bytes of LDS", name, lds_bytes);
   const int64_t grid = (p.M + tokens_per_wg - 1) / tokens_per_wg;
   if (grid > 0x7fffffffLL) return set_error(TAAC_ERR_UNSUPPORTED, "%s: too many workgroups", name);
-  hipLaunchKernelGGL(kernel, dim3(static_cast<uint32_t>(grid)), dim3(waves * kWave), lds_bytes, s, p);
+  hipLaunchKernelGGL(kernel, dim3(static_cast<uint32_t>(grid), static_cast<uint32_t>(splits)), dim3(waves * kWave), lds_bytes, s, p);
   return check_launch(name);
 }
 
@@ -904,11 +907,19 @@ extern "C" int taac_swiglu_ffn_fp8_fwd(const void* x, int64_t ldx, const void* n
     hipLaunchKernelGGL(f8_clear_kernel, dim3(1), dim3(kWave), 0, s, amax_hidden, amax_next);
     if ((rc = check_launch(name)) != TAAC_OK) return rc;
   }
+  // Pass 1 divides the hidden units of its 256-token tiles as well: until every compute unit has a workgroup, and in two wherever
+  // the tiles are no more than two a unit (of which padding usually leaves fewer). Positions, of which 56 % hold tokens, us for
+  // 1 / 2 / 4 / 8 / 16 parts: 1 024 47 / 33 / 25 / 21 / 19, 16 384 50 / 35 / 27 / 30 / 46, 65 536 51 / 47 / 48 / 64 / 104,
+  // 131 072 70 / 65 / 74 / 106 / 182, 262 144 100 / 105 / 133.
+  const int64_t cus = compute_units(), tiles1 = (M + 4 * 64 - 1) / (4 * 64);
+  int splits1 = tiles1 <= 2 * cus ? 2 : 1;
+  while (2 * splits1 * tiles1 <= cus) splits1 *= 2;
+  if (splits1 > F / kF8Chunk) splits1 = F / kF8Chunk;
 // pass 1: 4 wavefronts x 2 tiles; pass 2: 4 wavefronts x 1 tile; two workgroups per compute unit
 #define TAAC_F8_FFN(DD, BB)                                                                                             \
   do {                                                                                                                  \
-    if ((rc = f8_launch(swiglu_ffn_fp8_kernel<DD, 2, 4, false, BB>, p, 4, 4 * 64, lds1, s, name)) != TAAC_OK) return rc; \
-    return f8_launch(swiglu_ffn_fp8_kernel<DD, 1, 4, true, BB>, p, 4, 4 * 32, lds2, s, name);                           \
+    if ((rc = f8_launch(swiglu_ffn_fp8_kernel<DD, 2, 4, false, BB>, p, 4, 4 * 64, splits1, lds1, s, name)) != TAAC_OK) return rc; \
+    return f8_launch(swiglu_ffn_fp8_kernel<DD, 1, 4, true, BB>, p, 4, 4 * 32, 1, lds2, s, name);                           \
   } while (0)
   if (D == 256) {
     if (b_up != nullptr) TAAC_F8_FFN(256, true);

@@ -190,3 +190,18 @@ def test_dense_layer_with_its_steps_divided_over_workgroups(device, test_hooks, 
             test_hooks(max_workgroups=workgroups)
             for got, one in zip(layers(), want):
                 assert torch.equal(got, one)
+
+
+@pytest.mark.parametrize("m,f", [(1, 64), (300, 192), (700, 1024), (20000, 1024), (40000, 128)])
+def test_scale_of_a_hidden_state_divided_over_workgroups(device, m, f):
+    """The first pass takes a tile's hidden units in one to sixteen parts, by the number of rows: the maximum it leaves is that of
+    the rows taken 131 073 at a time (no parts, the same rows repeated), to the bit, and so is every row of the result."""
+    x, nw, uw, ub, dw, db = _to(device, *_case(m, 256, f, seed=f))
+    with torch.no_grad():
+        packed = pack_ffn_weights_fp8(uw, dw)
+        ax = amax(rms_norm(x, nw))
+        many = x.repeat(-(-131073 // m), 1)
+        got, got_max, _ = swiglu_ffn_fp8(x, packed, ub, db, ax, hidden_size=f, norm_weight=nw)
+        want, want_max, _ = swiglu_ffn_fp8(many, packed, ub, db, ax, hidden_size=f, norm_weight=nw)
+    assert got_max.item() == want_max.item()
+    assert torch.equal(got, want[:m])
