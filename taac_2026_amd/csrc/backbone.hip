@@ -625,11 +625,12 @@ extern "C" int taac_backbone_fwd(const void* emb, const int32_t* key_lengths, co
       if ((rc = taac_norm_linear_fp8_fwd(h, D, nullptr, eps, fp8_out(i), w.out_bias, sc + 5, sc + 1, cur, D, x, D, M, D, D,
                                          rows, n_rows, w.ffn_norm_weight, eps, sc + 6, stream)) != TAAC_OK)
         return rc;
-      if ((rc = taac_swiglu_ffn_fp8_fwd(x, D, w.ffn_norm_weight, eps, fp8_ffn(i), w.up_bias, w.down_bias, sc + 6, sc + 2,
-                                        sc + 3, sc + 7, x, D, x_out, D, M, D, F, 1, rows, n_rows,
-                                        last ? nullptr : blocks[i + 1].attn_norm_weight, eps, last ? nullptr : sc + 8 + 4,
-                                        stream)) != TAAC_OK)
+      if ((rc = swiglu_ffn_fp8_readout(x, D, w.ffn_norm_weight, eps, fp8_ffn(i), w.up_bias, w.down_bias, sc + 6, sc + 2, sc + 3,
+                                       sc + 7, x, D, x_out, D, M, D, F, 1, rows, n_rows,
+                                       last ? nullptr : blocks[i + 1].attn_norm_weight, eps, last ? nullptr : sc + 8 + 4,
+                                       ride ? w_head : nullptr, ride ? token_dots : nullptr, stream)) != TAAC_OK)
         return rc;
+      dots_ready = ride;
       cur = x_out;
       continue;
     }

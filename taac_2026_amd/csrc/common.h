@@ -76,6 +76,14 @@ int launch_linear_fp8_ts(const void* a, int a_is_fp8, int64_t lda, const void* w
                          int64_t M, int32_t N, int32_t K, int epilogue, int gate_first, hipStream_t s,
                          const char* name);
 
+// taac_swiglu_ffn_fp8_fwd that also writes the dot product of every stored row with head_w [D] (16-byte aligned; no amax_next
+// then) to token_dots[row]; null: no readout.
+int swiglu_ffn_fp8_readout(const void* x, int64_t ldx, const void* norm_weight, float eps, const void* packed_weights,
+                           const void* b_up, const void* b_down, const float* amax_x, const float* amax_up,
+                           const float* amax_down, float* amax_hidden, const void* residual, int64_t ldr, void* out, int64_t ldo,
+                           int64_t M, int32_t D, int32_t F, int gate_first, const int32_t* rows, const int32_t* n_rows,
+                           const void* next_norm_weight, float next_eps, float* amax_next, const void* head_w, float* token_dots,
+                           void* stream);
 // FP8 preparation of a backbone (ffn_fp8.hip): per block four weight scales (qkv, out, up, down; zeroed by the caller), the row-major e4m3
 // copies of the qkv / out weights and the packed feed-forward blob.
 int prepare_backbone_fp8(const taac_block_weights* blocks, int n, int32_t D, int32_t F, float* const* scales,

@@ -271,6 +271,8 @@ __device__ __forceinline__ void f8_stage_up_bias(const bf16_t* b_up, uint32_t* d
 // ---- the kernel -------------------------------------------------------------------------------------------------------
 // PASS2 = false: up projection + activation, max |hid| -> amax_hidden.   PASS2 = true: the whole layer.
 // A wavefront owns TT tiles of 32 tokens; every weight fragment read from LDS feeds TT MFMAs. NW wavefronts per workgroup.
+// HEAD: the readout rides on pass 2, which leaves every stored row's dot product with next_norm_w (the readout's weight there) in
+// amax_next[row] and reduces no maximum. (As a test inside one kernel it costs the layers without a readout 1 us of 107.)
 // BIAS: an up-projection bias is present. The activation works on the raw accumulators a = (projection + bias) / dq:
 //   silu(g) * u = a_g * a_u * dq^2 / (1 + exp2(-log2(e) * dq * a_g)),
 // the constant factors are applied once (to the maximum in pass 1, folded into the quantisation factor in pass 2).
@@ -279,7 +281,7 @@ __device__ __forceinline__ void f8_stage_up_bias(const bf16_t* b_up, uint32_t* d
 // under the matrix unit. The down projection of a chunk follows one chunk late (its B operand, the quantised hidden state
 // of the previous chunk, is complete once the first sub-chunk of the current chunk has been issued).
 // LDS: [2 weight buffers][b_down (D) | norm weight (D) | next norm weight (D)][16 floats][BIAS: bias pairs (2F dwords)]
-template <int D, int TT, int NW, bool PASS2, bool BIAS>
+template <int D, int TT, int NW, bool PASS2, bool BIAS, bool HEAD = false>
 __global__ __launch_bounds__(NW* kWave, 2) void swiglu_ffn_fp8_kernel(const FfnFp8Params p) {
   constexpr int KS = D / 64;                    // k-steps of the up projection = up fragments per sub-chunk
   constexpr int MB = D / 32;                    // row blocks of the down projection
@@ -591,7 +593,7 @@ __global__ __launch_bounds__(NW* kWave, 2) void swiglu_ffn_fp8_kernel(const FfnF
 
       // ---- epilogue in accumulator order: register jq * 4 + e of row block mb is feature mb * 32 + jq * 8 + hh * 4 + e of
       // token l32. out = bf16(acc * dq2 + b_down + residual), 8-byte pieces.
-      const bool want_next = p.amax_next != nullptr;
+      const bool want_next = !HEAD && p.amax_next != nullptr;
 #pragma unroll
       for (int t = 0; t < TT; ++t) {
         const int64_t tok = tok0 + t * 32 + l32;
@@ -600,6 +602,7 @@ __global__ __launch_bounds__(NW* kWave, 2) void swiglu_ffn_fp8_kernel(const FfnF
         const bf16_t* res_row = p.residual != nullptr ? p.residual + row * p.ldr + hh * 4 : nullptr;
         bf16_t* out_row = p.out + row * p.ldo + hh * 4;
         float ss = 0.f;
+        [[maybe_unused]] float dot = 0.f;
 #pragma unroll
         for (int mb = 0; mb < MB; ++mb) {
           bf16x4 rv[4];
@@ -625,8 +628,17 @@ __global__ __launch_bounds__(NW* kWave, 2) void swiglu_ffn_fp8_kernel(const FfnF
                 ss = fmaf(r, r, ss);
               }
             }
+            if constexpr (HEAD) {
+              const bf16x4 hw = *reinterpret_cast<const bf16x4*>(nextw_lds + mb * 32 + jq * 8 + hh * 4);
+#pragma unroll
+              for (int e = 0; e < 4; ++e) dot = fmaf(static_cast<float>(ov[e]), static_cast<float>(hw[e]), dot);
+            }
             if (live) *reinterpret_cast<bf16x4*>(out_row + mb * 32 + jq * 8) = ov;
           }
+        }
+        if constexpr (HEAD) {
+          dot = f8_pair_sum(dot);
+          if (live && hh == 0) p.amax_next[row] = dot;
         }
         if (want_next) {
           // amax of what the next layer will quantise: bf16(rmsnorm(out) * w) with its norm weight, or |out| itself. The
@@ -657,7 +669,7 @@ __global__ __launch_bounds__(NW* kWave, 2) void swiglu_ffn_fp8_kernel(const FfnF
         }
       }
     }
-    if (p.amax_next != nullptr) f8_block_atomic_max(nmax, p.amax_next, red, wave, lane, NW);
+    if (!HEAD && p.amax_next != nullptr) f8_block_atomic_max(nmax, p.amax_next, red, wave, lane, NW);
   }
 }
 
@@ -860,14 +872,14 @@ extern "C" int taac_ffn_fp8_pack_weights(const void* w_up, const void* w_down, c
   return check_launch(name);
 }
 
-extern "C" int taac_swiglu_ffn_fp8_fwd(const void* x, int64_t ldx, const void* norm_weight, float eps,
-                                       const void* packed_weights, const void* b_up, const void* b_down,
-                                       const float* amax_x, const float* amax_up, const float* amax_down,
-                                       float* amax_hidden, const void* residual, int64_t ldr, void* out, int64_t ldo,
-                                       int64_t M, int32_t D, int32_t F, int gate_first, const int32_t* rows,
-                                       const int32_t* n_rows, const void* next_norm_weight, float next_eps,
-                                       float* amax_next, void* stream) {
-  using namespace taac;
+namespace taac {
+int swiglu_ffn_fp8_readout(const void* x, int64_t ldx, const void* norm_weight, float eps,
+                           const void* packed_weights, const void* b_up, const void* b_down,
+                           const float* amax_x, const float* amax_up, const float* amax_down,
+                           float* amax_hidden, const void* residual, int64_t ldr, void* out, int64_t ldo,
+                           int64_t M, int32_t D, int32_t F, int gate_first, const int32_t* rows,
+                           const int32_t* n_rows, const void* next_norm_weight, float next_eps,
+                           float* amax_next, const void* head_w, float* token_dots, void* stream) {
   const char* name = "taac_swiglu_ffn_fp8_fwd";
   if (M < 0 || D <= 0 || F <= 0) return set_error(TAAC_ERR_INVALID_VALUE, "%s: M must be >= 0, D and F > 0", name);
   if (taac_ffn_fp8_packed_bytes(D, F) < 0)
@@ -934,16 +946,37 @@ extern "C" int taac_swiglu_ffn_fp8_fwd(const void* x, int64_t ldx, const void* n
   while (2 * splits1 * tiles1 <= cus) splits1 *= 2;
   if (splits1 > F / kF8Chunk) splits1 = F / kF8Chunk;
 // pass 1: 4 wavefronts x 2 tiles; pass 2: 4 wavefronts x 1 tile; two workgroups per compute unit
-#define TAAC_F8_FFN(DD, BB)                                                                                             \
-  do {                                                                                                                  \
-    if ((rc = f8_launch(swiglu_ffn_fp8_kernel<DD, 2, 4, false, BB>, p, 4, 4 * 64, splits1, lds1, s, name)) != TAAC_OK) return rc; \
-    return f8_launch(swiglu_ffn_fp8_kernel<DD, 1, 4, true, BB>, p, 4, 4 * 32, 1, lds2, s, name);                           \
+#define TAAC_F8_FFN(DD, BB, HEAD)                                                                                          \
+  do {                                                                                                                     \
+    if ((rc = f8_launch(swiglu_ffn_fp8_kernel<DD, 2, 4, false, BB>, p, 4, 4 * 64, splits1, lds1, s, name)) != TAAC_OK)     \
+      return rc;                                                                                                           \
+    return f8_launch(swiglu_ffn_fp8_kernel<DD, 1, 4, true, BB, HEAD>, p, 4, 4 * 32, 1, lds2, s, name);                     \
   } while (0)
-  if (D == 256) {
-    if (b_up != nullptr) TAAC_F8_FFN(256, true);
-    TAAC_F8_FFN(256, false);
+  if (head_w != nullptr) {
+    if (D != 256) return set_error(TAAC_ERR_UNSUPPORTED, "%s: a readout rides on layers of width 256 (got %d)", name, D);
+    p.next_norm_w = static_cast<const bf16_t*>(head_w);
+    p.amax_next = token_dots;
+    if (b_up != nullptr) TAAC_F8_FFN(256, true, true);
+    TAAC_F8_FFN(256, false, true);
   }
-  if (b_up != nullptr) TAAC_F8_FFN(128, true);
-  TAAC_F8_FFN(128, false);
+  if (D == 256) {
+    if (b_up != nullptr) TAAC_F8_FFN(256, true, false);
+    TAAC_F8_FFN(256, false, false);
+  }
+  if (b_up != nullptr) TAAC_F8_FFN(128, true, false);
+  TAAC_F8_FFN(128, false, false);
 #undef TAAC_F8_FFN
+}
+}  // namespace taac
+
+extern "C" int taac_swiglu_ffn_fp8_fwd(const void* x, int64_t ldx, const void* norm_weight, float eps,
+                                       const void* packed_weights, const void* b_up, const void* b_down,
+                                       const float* amax_x, const float* amax_up, const float* amax_down,
+                                       float* amax_hidden, const void* residual, int64_t ldr, void* out, int64_t ldo,
+                                       int64_t M, int32_t D, int32_t F, int gate_first, const int32_t* rows,
+                                       const int32_t* n_rows, const void* next_norm_weight, float next_eps,
+                                       float* amax_next, void* stream) {
+  return taac::swiglu_ffn_fp8_readout(x, ldx, norm_weight, eps, packed_weights, b_up, b_down, amax_x, amax_up, amax_down, amax_hidden,
+                                      residual, ldr, out, ldo, M, D, F, gate_first, rows, n_rows, next_norm_weight, next_eps,
+                                      amax_next, nullptr, nullptr, stream);
 }

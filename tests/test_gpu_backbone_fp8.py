@@ -162,6 +162,24 @@ def test_fp8_backbone_skips_padded_positions_and_repeats_bit_for_bit(device):
     assert (h_ref[~valid] == 0).all()
 
 
+@pytest.mark.parametrize("bias", [False, True])
+@pytest.mark.parametrize("batch,n_sequence,dense", [(1, 3, False), (5, 130, False), (5, 130, True), (70, 480, False)])
+def test_readout_that_rides_on_the_last_fp8_layer(device, batch, n_sequence, dense, bias):
+    """The probabilities come out of the last layer's epilogue: they are those of the hidden state it stored. Bound: 512 tokens of
+    256 products each, summed in float32 (2**-24 relative a sum, under 400 sums a chain), through a slope of at most 1/4."""
+    inputs = workloads.backbone_inputs(batch=batch, n_feature_tokens=32, n_sequence_tokens=n_sequence, n_blocks=2, d_ff=128,
+                                       min_sequence_len=1, seed=batch + n_sequence)
+    if bias:
+        inputs = _with_biases(inputs, seed=batch)
+    p, hidden, _ = _run(inputs, device, fp8=True, dense_tokens=dense)
+    valid = torch.arange(inputs.emb.shape[1])[None, :] < inputs.key_lengths[:, None]
+    weight = inputs.head_weight[0].double()
+    terms = hidden.double() * weight * valid[..., None] / valid.sum(1)[:, None, None]
+    want = torch.sigmoid(terms.sum((1, 2)) + inputs.head_bias.double())
+    atol = 400 * 2 ** -24 * (1 + terms.abs().sum((1, 2)).max().item()) / 4
+    torch.testing.assert_close(p.double(), want, rtol=0, atol=atol)
+
+
 def test_fp8_backbone_rejects_what_it_does_not_cover(device):
     inputs = workloads.backbone_inputs(batch=2, n_feature_tokens=8, n_sequence_tokens=24, d_model=128, num_heads=4, d_ff=256, min_sequence_len=4,
                                        n_blocks=1, seed=1)
