@@ -667,8 +667,8 @@ extern "C" int taac_backbone_fwd(const void* emb, const int32_t* key_lengths, co
       }
       if (planes)
         rc = norm_linear_qk_heads(cur, D, w.attn_norm_weight, eps, w.qkv_bias, pk_qkv, qkv, M, D, heads, T, q_weight,
-                                  k_weight, rope_cos_sin, qk_norm ? qk_sumsq : nullptr, qk_norm ? qk_rstd : nullptr, rows,
-                                  n_rows, w.attn_norm_weight != nullptr, stream);
+                                  k_weight, rope_cos_sin, qk_norm ? qk_rstd : nullptr, rows, n_rows, w.attn_norm_weight != nullptr,
+                                  stream);
       else
         rc = taac_norm_linear_qk_fwd(cur, D, w.attn_norm_weight, eps, nullptr, w.qkv_bias, pk_qkv, qkv, 3 * D, M, D, heads,
                                      T, weights_in_epilogue ? qk_weight : nullptr, rope_cos_sin,
@@ -676,7 +676,7 @@ extern "C" int taac_backbone_fwd(const void* emb, const int32_t* key_lengths, co
                                      stream);
       if (rc != TAAC_OK) return rc;
       if (qk_norm) {
-        if (!(planes && dense_few_rows(M, D)) &&
+        if (!planes &&
             (rc = taac_row_rstd(qk_sumsq, M, D, eps, qk_rstd, rows, n_rows, stream)) != TAAC_OK)
           return rc;
         q_scale = qk_rstd;
@@ -801,7 +801,7 @@ namespace {
 // Workspace of taac_stack_fwd for M = B * T rows.
 struct StackLayout {
   bf16_t *qkv, *attended;
-  float *sumsq, *scales, *products;  // query / key norms: [2 D / 64][M], [2][M], [n_blocks][D]
+  float *scales, *products;  // query / key norms: [2][M], [n_blocks][D]
   int64_t bytes;
 };
 StackLayout stack_layout(char* base, int64_t M, int32_t D, int32_t n_blocks, bool qk_norm) {
@@ -815,7 +815,6 @@ StackLayout stack_layout(char* base, int64_t M, int32_t D, int32_t n_blocks, boo
   l.qkv = reinterpret_cast<bf16_t*>(take(M * 3 * D * 2));
   l.attended = reinterpret_cast<bf16_t*>(take(M * D * 2));
   if (qk_norm) {
-    l.sumsq = reinterpret_cast<float*>(take(M * (2 * D / 64) * 4));
     l.scales = reinterpret_cast<float*>(take(2 * M * 4));
     l.products = reinterpret_cast<float*>(take(static_cast<int64_t>(n_blocks) * D * 4));
   }
@@ -914,15 +913,11 @@ extern "C" int taac_stack_fwd(const void* tokens, const uint8_t* padding, const 
   for (int i = 0; i < n_blocks; ++i) {
     const taac_block_weights& w = blocks[i];
     const void* x = i == 0 ? tokens : out;
-    int rc = qk_norm ? taac_norm_linear_qk_fwd(x, D, w.attn_norm_weight, attn_eps, nullptr, w.qkv_bias, w.qkv_weight, l.qkv, 3 * D, M, D, H,
-                                               T, nullptr, nullptr, l.sumsq, front_rows, n_rows, rows, 1, stream)
+    int rc = qk_norm ? norm_linear_qk_factors(name, x, D, w.attn_norm_weight, attn_eps, w.qkv_bias, w.qkv_weight, l.qkv, 3 * D, M, D, H,
+                                              T, qk_eps, l.scales, front_rows, n_rows, rows, 1, stream)
                      : taac_norm_linear_fwd(x, D, w.attn_norm_weight, attn_eps, nullptr, w.qkv_bias, w.qkv_weight, nullptr, 3 * D, l.qkv,
                                             3 * D, M, 3 * D, D, front_rows, n_rows, rows, 1, stream);
     if (rc != TAAC_OK) return rc;
-    if (qk_norm) {
-      rc = taac_row_rstd(l.sumsq, M, D, qk_eps, l.scales, front_rows, n_rows, stream);
-      if (rc != TAAC_OK) return rc;
-    }
     rc = taac_flash_attn_masked_fwd(l.qkv, l.qkv + D, l.qkv + 2 * D, lengths, struct_bits, struct_sample_stride, nullptr, nullptr, nullptr,
                                     l.scales, qk_norm ? l.scales + M : nullptr, qk_norm ? l.products + static_cast<int64_t>(i) * D : nullptr,
                                     l.attended, B, H, T, T, dh, qkv_strides, qkv_strides, qkv_strides, out_strides, 2, TAAC_BF16, stream);

@@ -867,6 +867,7 @@ __global__ __launch_bounds__(8 * kWave, 2) void norm_linear_kernel(const TsParam
   // QK: (memory row, position in the sample) of the wavefront's tokens, kept in LDS behind the bias and norm weights
   // (written and read by the same wavefront only), instead of in registers.
   int2* rowinfo = reinterpret_cast<int2*>(reinterpret_cast<uint8_t*>(bias_lds) + ((p.N + D) * 2 + 15) / 16 * 16) + wave * kWave;
+  [[maybe_unused]] float* norm_ss = reinterpret_cast<float*>(rowinfo + (NWAVES - wave) * kWave) + wave * kWave;  // qk_rstd: running sums
   // QK == 0: a float32 copy of the bias in the same place (the epilogue adds it in float32: read as it is needed, the
   // widening of 64 values per step and wavefront is done once per workgroup instead)
   float* bias_f32 = reinterpret_cast<float*>(reinterpret_cast<uint8_t*>(bias_lds) + ((p.N + D) * 2 + 15) / 16 * 16);
@@ -881,12 +882,15 @@ __global__ __launch_bounds__(8 * kWave, 2) void norm_linear_kernel(const TsParam
   const int wg = static_cast<int>(blockIdx.x);
   const int full_rounds = num_tiles / G;
   const int R = num_tiles % G;
+  // With the factors of the query and key norm (qk_rstd) a segment is one or more of the parts q, k, v, so that a workgroup meets all
+  // chunks of a factor.
+  const int unit = QK != 0 && p.qk_rstd != nullptr ? D / kNC : 1, units = nchunks / unit;
   int S = R > 0 ? G / R : 1;
-  S = S < nchunks ? S : nchunks;
+  S = S < units ? S : units;
   const bool has_tail = R > 0 && wg < R * S;
   const int tail_tile = full_rounds * G + wg / S;
-  const int tail_begin = has_tail ? ((wg % S) * nchunks) / S : 0;
-  const int tail_len = has_tail ? (((wg % S) + 1) * nchunks) / S - tail_begin : 0;
+  const int tail_begin = has_tail ? ((wg % S) * units) / S * unit : 0;
+  const int tail_len = has_tail ? (((wg % S) + 1) * units) / S * unit - tail_begin : 0;
   const int full_total = full_rounds * nchunks;
   const int total = full_total + tail_len;
   if (total == 0) return;  // whole workgroup: nothing assigned to it
@@ -1122,7 +1126,9 @@ __global__ __launch_bounds__(8 * kWave, 2) void norm_linear_kernel(const TsParam
     if constexpr (QK == 0) read_chunk_bias(bias_f32 + chunk * kNC, hh, bvf);
     if constexpr (QK != 0) {
       // Query and key chunks: the sum of squares of the rounded projection goes to qk_sumsq (one value per token and
-      // chunk; the statistic of the norm over the model width is their sum). QK == 2 also multiplies the features by
+      // chunk; the statistic of the norm over the model width is their sum), or is summed over the part's chunks in LDS and leaves as
+      // the norm's factor in qk_rstd (a launch of its own behind the projection took 5 us a block:
+      // 45 900 positions of the narrow network 256 -> 247 us a call). QK == 2 also multiplies the features by
       // the norm weight and rotates them. The per-token factor rsqrt(mean + eps) commutes with both and is applied by
       // the attention kernel. Value chunks are stored as they are.
       constexpr bool XF = QK == 2;
@@ -1141,11 +1147,22 @@ __global__ __launch_bounds__(8 * kWave, 2) void norm_linear_kernel(const TsParam
 #pragma unroll
       for (int t = 0; t < TT; ++t) {
         read_chunk_bias(bias_lds + chunk * kNC, hh, bv);  // per tile: not held while the pieces are processed
-        if (qk_chunk && p.qk_sumsq != nullptr) {
+        if (qk_chunk && (p.qk_sumsq != nullptr || p.qk_rstd != nullptr)) {
           float ss = tile_to_lds_sumsq(tile_lds, acc0[t], acc1[t], bv, l32, hh, rstd[t]);
           ss = half_wave_pair_sum(ss);
           const int row = rowinfo[t * 32 + l32].x;
-          if (hh == 0) p.qk_sumsq[static_cast<int64_t>(chunk) * p.M + row] = ss;
+          if (p.qk_rstd != nullptr) {
+            constexpr int parts = D / kNC;  // chunks of the query, and of the key
+            if (hh == 0) {
+              if (chunk % parts > 0) ss += norm_ss[t * 32 + l32];
+              if (chunk % parts < parts - 1)
+                norm_ss[t * 32 + l32] = ss;
+              else
+                p.qk_rstd[static_cast<int64_t>(chunk / parts) * p.M + row] = rsqrtf(ss * (1.0f / D) + p.qk_eps);
+            }
+          } else {
+            if (hh == 0) p.qk_sumsq[static_cast<int64_t>(chunk) * p.M + row] = ss;
+          }
         } else {
           tile_to_lds(tile_lds, acc0[t], acc1[t], bv, l32, hh, rstd[t]);
         }
@@ -1642,7 +1659,7 @@ struct QkExtras {
   const void* k_weight = nullptr;
   const void* cos_sin = nullptr;
   float* qk_sumsq = nullptr;
-  float* qk_rstd = nullptr;  // with qk_sumsq: written by the few-token form instead
+  float* qk_rstd = nullptr;  // [2][M] factors of the query and key norm, written instead of qk_sumsq
   float qk_eps = 0.f;
   int32_t qk_chunks = 0, head_dim = 0, tokens_per_sample = 0;
   bool enabled = false;
@@ -1678,8 +1695,9 @@ int norm_linear_launch(const char* name, const void* x, int64_t ldx, const void*
       !ptr_ok(bias, 15) || !ptr_ok(packed_weights, 15) || !ptr_ok(qk.q_weight, 15) || !ptr_ok(qk.k_weight, 15) || !ptr_ok(qk.cos_sin, 15) ||
       !ptr_ok(qk.qk_sumsq, 3))
     return set_error(TAAC_ERR_UNSUPPORTED, "%s: tensor base pointers must be 16-byte aligned", name);
-  // behind the 16-bit bias and norm weight: the query / key epilogue's row table, or the float32 copy of the bias
-  const size_t rowinfo_bytes = qk.enabled ? 16 + 8 * static_cast<size_t>(kWave) * sizeof(int2) : 16 + static_cast<size_t>(N) * 4;
+  // behind the 16-bit bias and norm weight: the query / key epilogue's row table and running sums, or the float32 copy of the bias
+  const size_t rowinfo_bytes = qk.enabled ? 16 + 8 * static_cast<size_t>(kWave) * (sizeof(int2) + (qk.qk_rstd != nullptr ? 4 : 0))
+                                          : 16 + static_cast<size_t>(N) * 4;
   const size_t lds_bytes = static_cast<size_t>(3 * 2 * (K / 16)) * kFrag + 8 * static_cast<size_t>(kStageWave) +
                            static_cast<size_t>(N + K) * 2 + rowinfo_bytes;
   if (lds_bytes > kMaxLdsBytes)
@@ -1718,7 +1736,6 @@ int norm_linear_launch(const char* name, const void* x, int64_t ldx, const void*
   const bool qk_transform = qk.enabled && (qk.q_weight != nullptr || qk.cos_sin != nullptr);
   if (dense_few_rows(M, K) && packed_weights && (norm_weight == nullptr || norm_folded))
     return norm_linear_small(p, K, qk_transform ? 2 : (qk.enabled ? 1 : 0), s, name);
-  p.qk_rstd = nullptr;
   // Without a residual two token tiles per wavefront fit the register file: every weight fragment read from LDS then
   // feeds two MFMAs, which halves the LDS reads (and their share of the power budget) per token.
   const int tt = residual ? 1 : 2;
@@ -1806,13 +1823,12 @@ namespace taac {
 int norm_linear_qk_heads(const void* x, int64_t ldx, const void* norm_weight, float eps, const void* bias,
                          const void* packed_weights, void* out, int64_t M, int32_t d_model, int32_t num_heads,
                          int32_t tokens_per_sample, const void* q_weight, const void* k_weight, const void* cos_sin,
-                         float* qk_sumsq, float* qk_rstd, const int32_t* rows, const int32_t* n_rows, int norm_folded, void* stream) {
+                         float* qk_rstd, const int32_t* rows, const int32_t* n_rows, int norm_folded, void* stream) {
   QkExtras qk;
   qk.enabled = true;
   qk.q_weight = q_weight;
   qk.k_weight = k_weight;
   qk.cos_sin = cos_sin;
-  qk.qk_sumsq = qk_sumsq;
   qk.qk_rstd = qk_rstd;
   qk.qk_eps = eps;
   qk.qk_chunks = 2 * d_model / kNC;
@@ -1821,6 +1837,21 @@ int norm_linear_qk_heads(const void* x, int64_t ldx, const void* norm_weight, fl
   return norm_linear_launch("taac_backbone_fwd", x, ldx, norm_weight, eps, nullptr, bias, packed_weights, nullptr, 0, out,
                             3 * d_model, M, 3 * d_model, d_model, rows, n_rows, nullptr, qk, norm_folded, stream,
                             d_model / num_heads);
+}
+
+int norm_linear_qk_factors(const char* name, const void* x, int64_t ldx, const void* norm_weight, float eps, const void* bias,
+                           const void* packed_weights, void* out, int64_t ldo, int64_t M, int32_t d_model, int32_t num_heads,
+                           int32_t tokens_per_sample, float qk_eps, float* qk_rstd, const int32_t* rows, const int32_t* n_rows,
+                           const int32_t* x_rows, int norm_folded, void* stream) {
+  QkExtras qk;
+  qk.enabled = true;
+  qk.qk_rstd = qk_rstd;
+  qk.qk_eps = qk_eps;
+  qk.qk_chunks = 2 * d_model / kNC;
+  qk.head_dim = d_model / num_heads;
+  qk.tokens_per_sample = tokens_per_sample;
+  return norm_linear_launch(name, x, ldx, norm_weight, eps, nullptr, bias, packed_weights, nullptr, 0, out, ldo, M, 3 * d_model,
+                            d_model, rows, n_rows, x_rows, qk, norm_folded, stream);
 }
 
 // taac_attn_out_ffn_fwd (attn_plane = 0) / taac_attn_out_ffn_heads_fwd (attn_plane = head_dim) that also leaves, for every

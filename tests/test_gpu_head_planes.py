@@ -149,6 +149,24 @@ def test_backbone_plane_route_equals_its_row_major_route(device, d_model, heads,
         assert torch.equal(hidden, hidden_rows)
 
 
+@pytest.mark.parametrize("workgroups", [1, 2, 5, 7])
+@pytest.mark.parametrize("d_model,rope_base", [(256, None), (256, 10000.0), (128, None)])
+def test_norm_factors_of_the_projection_equal_those_of_their_own_kernel(device, test_hooks, workgroups, d_model, rope_base):
+    """The plane route's projection sums the query / key statistic over its chunks and stores the factors (a divided last round
+    of tiles is then cut between q, k and v); the row-major route leaves the sums to a kernel of their own. Same order, same bits."""
+    test_hooks(max_workgroups=workgroups)
+    inputs = workloads.backbone_inputs(batch=9, n_feature_tokens=8, n_sequence_tokens=233, d_model=d_model, num_heads=4, d_ff=128,
+                                       n_blocks=2, min_sequence_len=1, seed=workgroups)
+    model = PCVRBackbone(d_model=d_model, num_heads=4, d_ff=128, n_blocks=2, qk_norm=True, rope_base=rope_base)
+    model = model.to(device=device, dtype=torch.bfloat16).eval()
+    emb, lengths = 50 * inputs.emb.to(device), inputs.key_lengths.to(device)
+    with torch.no_grad():
+        planes = model(emb, lengths, return_hidden=True)
+        rows = model(emb, lengths, return_hidden=True, row_major_qkv=True)
+    assert torch.isfinite(planes[0]).all()
+    assert torch.equal(planes[0], rows[0]) and torch.equal(planes[1], rows[1])
+
+
 @pytest.mark.parametrize("d_model,heads,d_ff", [(256, 8, 1024), (128, 2, 256), (128, 8, 256)])  # head widths 32, 64, 16 (rows)
 @pytest.mark.parametrize("dense_tokens", [False, True])
 def test_readout_riding_on_the_last_block_equals_the_readout_kernel(device, d_model, heads, d_ff, dense_tokens):
