@@ -964,8 +964,8 @@ int taac_stack_train_bwd(const void* grad_out, const void* grad_attn_tokens, con
 
 /*
  * Inference of a stack of n_blocks interaction blocks (experiments/symbiosis/backbone.py:51-68; no rotary embedding) under padding of
- * any pattern and a structured mask, as one call: per block taac_norm_linear(_qk)_fwd into the front layout, taac_row_rstd,
- * taac_flash_attn_masked_fwd and taac_attn_out_ffn_fwd, with the same values as those calls.
+ * any pattern and a structured mask, as one call: per block taac_norm_linear(_qk)_fwd into the front layout (with
+ * the factors of taac_row_rstd), taac_flash_attn_masked_fwd and taac_attn_out_ffn_fwd, with the same values as those calls.
  * tokens: bf16 [B, T, D]; padding: uint8 [B, T], non-zero = padded: such rows of out repeat tokens. rows / n_rows: the other rows
  * (taac_valid_rows_from_bits); front_rows / lengths: taac_front_rows of them; struct_bits, struct_sample_stride:
  * taac_mask_front_bits. blocks: qkv_weight = taac_linear_pack_weights_norm, out_weight = taac_linear_pack_weights, up_weight = the
