@@ -288,3 +288,26 @@ def test_mask_bits_backward_with_all_keys_in_one_workgroup(device, rows, dim, ba
     got = _native_backward(*args, words=words, key_valid=pack(key_valid) if valid else None)
     dense = _native_backward(*args, visible=visible.to(torch.uint8).contiguous())
     _check_gradients(got, dense, exact, torch.bfloat16)
+
+
+@pytest.mark.parametrize("rows,dim,batch,heads,bits", [(128, 32, 8, 4, False), (200, 32, 64, 8, False), (400, 32, 128, 8, False),
+                                                       (250, 64, 128, 4, False), (200, 32, 64, 8, True)])
+def test_one_workgroup_rounds_as_the_two_kernels_do(device, rows, dim, batch, heads, bits):
+    """dS is rounded to bf16 with its scale on every route, so two routes differ where their float32 sums fall on different sides of a
+    rounding boundary only: about one dS in 2^12, by 2^-8 of it, 2^-14 of a gradient's norm. (Rounded before a scale that is no
+    power of two they are 2^-8.3 apart.) Mask bits against the same mask as bytes."""
+    g = torch.Generator(device=device).manual_seed(rows)
+    q, k, v, grad_out = (torch.randn(batch, heads, rows, dim, generator=g, device=device).to(torch.bfloat16) for _ in range(4))
+    lengths = torch.randint(1, rows + 1, (batch,), generator=g, device=device, dtype=torch.int32)
+    index = torch.arange(rows, device=device)
+    inside = index < lengths[:, None]
+    lse, p = _log_sum_exp(q, k, (inside[:, None, :] & inside[:, :, None])[:, None])
+    args = (q, k, v, (p @ v.double()).to(torch.bfloat16), grad_out, lse.float().contiguous(), lengths, False, True)
+    if bits:
+        words = torch.full((batch, rows, (rows + 31) // 32), -1, dtype=torch.int32, device=device)
+        got = _native_backward(*args, words=words)
+        other = _native_backward(*args, visible=torch.ones(batch, rows, rows, dtype=torch.uint8, device=device))
+    else:
+        got, other = _native_backward(*args), _native_backward(*args, staged=True)
+    for name, a, b in zip(("dq", "dk", "dv"), got, other):
+        assert (a.double() - b.double()).norm() <= 2.0 ** -12 * b.double().norm(), name
