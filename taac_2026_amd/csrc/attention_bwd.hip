@@ -1066,7 +1066,6 @@ void attn_bwd_fused_kernel(const AttnBwdParams p) {
     }
     __syncthreads();  // the images now hold the output tiles
     uint8_t* out_tile = smem + wave * (32 * (ROWB + 16));
-    const int k_store_end = COMPACT ? len : p.Tk;
 #pragma unroll
     for (int t = 0; t < NT; ++t) {
       const int key0 = (own + t * kWaves) * 32;
@@ -1077,19 +1076,19 @@ void attn_bwd_fused_kernel(const AttnBwdParams p) {
 #pragma unroll
           for (int j = 0; j < 16; ++j) dkacc[t][mb][j] *= p.scale;
       }
-      store_owned<T, DP>(dkacc[t], out_tile, dkb, p.dks[2], key0, k_store_end, p.d, lane);
+      store_owned<T, DP>(dkacc[t], out_tile, dkb, p.dks[2], key0, len, p.d, lane);
       asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-      store_owned<T, DP>(dvacc[t], out_tile, dvb, p.dvs[2], key0, k_store_end, p.d, lane);
+      store_owned<T, DP>(dvacc[t], out_tile, dvb, p.dvs[2], key0, len, p.d, lane);
       asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
     }
   }
-  if (!COMPACT) {  // rows without a gradient
+  if (!COMPACT) {  // rows without a gradient: keys of the padding too, whose sums hold 0 x inf where a gradient is not finite
     vec_t zero;
 #pragma unroll
     for (int e = 0; e < 8; ++e) zero[e] = static_cast<T>(0.f);
     const int piece = (tid % C8) * 8;
     for (int row = q_end + tid / C8; row < p.Tq; row += kThreads / C8) *reinterpret_cast<vec_t*>(dqb + row * p.dqs[2] + piece) = zero;
-    for (int row = (q_end > 0 ? n_tiles * 32 : 0) + tid / C8; row < p.Tk; row += kThreads / C8) {
+    for (int row = (q_end > 0 ? len : 0) + tid / C8; row < p.Tk; row += kThreads / C8) {
       *reinterpret_cast<vec_t*>(dkb + row * p.dks[2] + piece) = zero;
       *reinterpret_cast<vec_t*>(dvb + row * p.dvs[2] + piece) = zero;
     }

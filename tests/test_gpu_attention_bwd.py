@@ -311,3 +311,24 @@ def test_one_workgroup_rounds_as_the_two_kernels_do(device, rows, dim, batch, he
         got, other = _native_backward(*args), _native_backward(*args, staged=True)
     for name, a, b in zip(("dq", "dk", "dv"), got, other):
         assert (a.double() - b.double()).norm() <= 2.0 ** -12 * b.double().norm(), name
+
+
+@pytest.mark.parametrize("value", [float("inf"), float("nan")])
+@pytest.mark.parametrize("rows,dim,batch,heads,bits", [(40, 32, 4, 2, False), (100, 64, 4, 2, True), (250, 32, 64, 8, True),
+                                                       (400, 32, 128, 8, False), (200, 64, 128, 4, False), (400, 32, 4, 2, True)])
+def test_padding_keys_receive_zeros_whatever_the_gradient(device, rows, dim, batch, heads, bits, value):
+    """A gradient that is not finite reaches the keys its query sees, not the padding in the same tile; other samples are untouched."""
+    g = torch.Generator(device=device).manual_seed(rows)
+    q, k, v, grad_out = (torch.randn(batch, heads, rows, dim, generator=g, device=device).to(torch.bfloat16) for _ in range(4))
+    lengths = torch.randint(rows // 4, rows + 1, (batch,), generator=g, device=device, dtype=torch.int32)
+    lengths[0] = rows - 5
+    grad_out[0, :, 3, 1] = value
+    index = torch.arange(rows, device=device)
+    inside = index < lengths[:, None]
+    lse, p = _log_sum_exp(q, k, (inside[:, None, :] & inside[:, :, None])[:, None])
+    words = torch.full((batch, rows, (rows + 31) // 32), -1, dtype=torch.int32, device=device) if bits else None
+    got = _native_backward(q, k, v, (p @ v.double()).to(torch.bfloat16), grad_out, lse.float().contiguous(), lengths, False, True, words=words)
+    for name, t in zip(("dq", "dk", "dv"), got):
+        assert (t.transpose(1, 2)[~inside] == 0).all(), name
+        assert torch.isfinite(t[1:]).all(), name
+    assert not torch.isfinite(got[2][0, :, :rows - 5]).all()
