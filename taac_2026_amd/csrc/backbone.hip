@@ -1,5 +1,6 @@
 // Forward driver of the unified token backbone (pre-norm blocks + pCVR readout) and the readout kernel.
 // The driver only sequences the library's own entry points on one stream over a caller-provided workspace.
+#include <algorithm>
 #include <cstdlib>
 #include <vector>
 
@@ -428,10 +429,11 @@ inline int64_t packed_block_bytes(int32_t D, int32_t F) {
   return align256(static_cast<int64_t>(3) * D * D * 2) + align256(static_cast<int64_t>(D) * D * 2) +
          align256(static_cast<int64_t>(3) * D * F * 2);
 }
-// Query / key norm scratch of the fused path: per-chunk sums of squares [2D / 64, M], factors [2, M], per block the product
-// of the query and key norm weights (fp32 [D]) or, with a rotary table, the two weights side by side (bf16 [2D]).
+// Query / key norm scratch of the fused path: per-chunk sums of squares [2D / 64, M] and the counters behind them, factors [2, M], per
+// block the product of the query and key norm weights (fp32 [D]) or, with a rotary table, the two weights side by side (bf16 [2D]).
+inline int64_t qk_sums_bytes(int64_t M, int32_t D) { return align256((2 * D / 64) * M * 4); }
 inline int64_t qk_norm_bytes(int64_t M, int32_t D, int32_t n_blocks) {
-  return align256((2 * D / 64) * M * 4) + align256(2 * M * 4) + align256(static_cast<int64_t>(D) * 4 * n_blocks);
+  return qk_sums_bytes(M, D) + align256(kQkCounters * 4) + align256(2 * M * 4) + align256(static_cast<int64_t>(D) * 4 * n_blocks);
 }
 // FP8 mode (TAAC_BACKBONE_FP8; D = 256, F a multiple of 64): per block the e4m3 qkv / out weights, the packed feed-forward
 // blob and 8 scales (weights: qkv, out, up, down; activations: block input, attention output, feed-forward input, gated
@@ -512,7 +514,8 @@ extern "C" int taac_backbone_fwd(const void* emb, const int32_t* key_lengths, co
   int32_t* n_rows = nullptr;
   char* after_packed = packed + static_cast<int64_t>(n_blocks) * packed_block_bytes(D, F);
   float* qk_sumsq = reinterpret_cast<float*>(after_packed + row_index_bytes(B, T));
-  float* qk_rstd = reinterpret_cast<float*>(reinterpret_cast<char*>(qk_sumsq) + align256((2 * D / 64) * M * 4));
+  uint32_t* qk_counters = reinterpret_cast<uint32_t*>(reinterpret_cast<char*>(qk_sumsq) + qk_sums_bytes(M, D));
+  float* qk_rstd = reinterpret_cast<float*>(reinterpret_cast<char*>(qk_counters) + align256(kQkCounters * 4));
   bf16_t* qk_weight = reinterpret_cast<bf16_t*>(reinterpret_cast<char*>(qk_rstd) + align256(2 * M * 4));
   if (rope_cos_sin != nullptr && !aligned16(rope_cos_sin))
     return set_error(TAAC_ERR_UNSUPPORTED, "%s: the rotary table must be 16-byte aligned", name);
@@ -558,8 +561,9 @@ extern "C" int taac_backbone_fwd(const void* emb, const int32_t* key_lengths, co
     }
     if ((rc = backbone_setup(blocks, n_blocks, D, F, fp8 ? nullptr : pk.data(), pk.data() + n_blocks, pk.data() + 2 * n_blocks,
                              fold_act, qk_norms && rope_cos_sin == nullptr ? norm_product : nullptr, key_lengths, B, T, rows,
-                             n_rows, sparse ? hidden_out : nullptr, split_counters,
-                             ffn_split > 1 ? static_cast<int32_t>(tiles) : 0, as_stream(stream), name)) != TAAC_OK)
+                             n_rows, sparse ? hidden_out : nullptr, ffn_split > 1 ? split_counters : qk_counters,
+                             ffn_split > 1 ? static_cast<int32_t>(tiles) : (dense_few_rows(M, D) ? 0 : kQkCounters),
+                             as_stream(stream), name)) != TAAC_OK)
       return rc;
   }
   // FP8 mode: scales and e4m3 weights of all blocks (three launches), then the scale of the first block's input
@@ -667,8 +671,8 @@ extern "C" int taac_backbone_fwd(const void* emb, const int32_t* key_lengths, co
       }
       if (planes)
         rc = norm_linear_qk_heads(cur, D, w.attn_norm_weight, eps, w.qkv_bias, pk_qkv, qkv, M, D, heads, T, q_weight,
-                                  k_weight, rope_cos_sin, qk_norm ? qk_rstd : nullptr, rows, n_rows, w.attn_norm_weight != nullptr,
-                                  stream);
+                                  k_weight, rope_cos_sin, qk_norm ? qk_sumsq : nullptr, qk_norm ? qk_rstd : nullptr, qk_counters, rows,
+                                  n_rows, w.attn_norm_weight != nullptr, stream);
       else
         rc = taac_norm_linear_qk_fwd(cur, D, w.attn_norm_weight, eps, nullptr, w.qkv_bias, pk_qkv, qkv, 3 * D, M, D, heads,
                                      T, weights_in_epilogue ? qk_weight : nullptr, rope_cos_sin,
@@ -801,7 +805,8 @@ namespace {
 // Workspace of taac_stack_fwd for M = B * T rows.
 struct StackLayout {
   bf16_t *qkv, *attended;
-  float *scales, *products;  // query / key norms: [2][M], [n_blocks][D]
+  float *sumsq, *scales, *products;  // query / key norms: [2 D / 64][M], [2][M], [n_blocks][D]
+  uint32_t* counters;                // [kQkCounters]
   int64_t bytes;
 };
 StackLayout stack_layout(char* base, int64_t M, int32_t D, int32_t n_blocks, bool qk_norm) {
@@ -815,6 +820,8 @@ StackLayout stack_layout(char* base, int64_t M, int32_t D, int32_t n_blocks, boo
   l.qkv = reinterpret_cast<bf16_t*>(take(M * 3 * D * 2));
   l.attended = reinterpret_cast<bf16_t*>(take(M * D * 2));
   if (qk_norm) {
+    l.sumsq = reinterpret_cast<float*>(take(qk_sums_bytes(M, D)));
+    l.counters = reinterpret_cast<uint32_t*>(take(kQkCounters * 4));
     l.scales = reinterpret_cast<float*>(take(2 * M * 4));
     l.products = reinterpret_cast<float*>(take(static_cast<int64_t>(n_blocks) * D * 4));
   }
@@ -827,7 +834,8 @@ struct StackSetup {
   const bf16_t* tokens;
   bf16_t* out;
   const uint8_t* padding;  // [M]
-  float* scales;           // [2 M], or null
+  float* scales;           // [2 M], or null; with the counters
+  uint32_t* counters;      // [kQkCounters]
   float* products;         // of blocks first_block .., n_blocks of them
   int64_t M;
   int32_t D, n_blocks;
@@ -836,8 +844,8 @@ struct StackSetup {
 };
 
 // What a stack needs in front of its blocks: the padded rows of the output (they pass through; the blocks write the others), ones in
-// the norm factors (rows outside the index are read by nobody, but a lane that holds such a row multiplies by it) and the products of
-// the query and key norm weights.
+// the norm factors (rows outside the index are read by nobody, but a lane that holds such a row multiplies by it), zeros in the counters
+// and the products of the query and key norm weights.
 __global__ __launch_bounds__(kBlock) void stack_setup_kernel(const StackSetup p) {
   const int64_t i = static_cast<int64_t>(blockIdx.x) * kBlock + threadIdx.x;
   const int pieces = p.D / 8;
@@ -845,6 +853,7 @@ __global__ __launch_bounds__(kBlock) void stack_setup_kernel(const StackSetup p)
     if (p.padding[i / pieces] != 0) reinterpret_cast<bf16x8*>(p.out)[i] = reinterpret_cast<const bf16x8*>(p.tokens)[i];
   }
   if (p.scales != nullptr && i < 2 * p.M) p.scales[i] = 1.f;
+  if (p.scales != nullptr && i < kQkCounters) p.counters[i] = 0u;
   if (i < static_cast<int64_t>(p.n_blocks) * p.D) {
     const int block = static_cast<int>(i / p.D), col = static_cast<int>(i % p.D);
     p.products[i] = static_cast<float>(p.query[block][col]) * static_cast<float>(p.key[block][col]);
@@ -892,6 +901,7 @@ extern "C" int taac_stack_fwd(const void* tokens, const uint8_t* padding, const 
       setup.out = static_cast<bf16_t*>(out);
       setup.padding = padding;
       setup.scales = l.scales;
+      setup.counters = l.counters;
     }
     if (qk_norm) {
       setup.products = l.products + static_cast<int64_t>(first) * D;
@@ -901,8 +911,8 @@ extern "C" int taac_stack_fwd(const void* tokens, const uint8_t* padding, const 
         setup.key[i] = static_cast<const bf16_t*>(blocks[first + i].key_norm_weight);
       }
     }
-    const int64_t wide = first == 0 ? M * (D / 8) : 0, products = static_cast<int64_t>(setup.n_blocks) * D;  // (2 M <= M D / 8)
-    const int64_t threads = wide > products ? wide : products;
+    const int64_t wide = first == 0 ? std::max<int64_t>(M * (D / 8), kQkCounters) : 0;  // (2 M <= M D / 8)
+    const int64_t threads = std::max<int64_t>(wide, static_cast<int64_t>(setup.n_blocks) * D);
     hipLaunchKernelGGL(stack_setup_kernel, dim3(static_cast<uint32_t>((threads + kBlock - 1) / kBlock)), dim3(kBlock), 0, s, setup);
     const int rc = check_launch(name);
     if (rc != TAAC_OK) return rc;
@@ -914,7 +924,7 @@ extern "C" int taac_stack_fwd(const void* tokens, const uint8_t* padding, const 
     const taac_block_weights& w = blocks[i];
     const void* x = i == 0 ? tokens : out;
     int rc = qk_norm ? norm_linear_qk_factors(name, x, D, w.attn_norm_weight, attn_eps, w.qkv_bias, w.qkv_weight, l.qkv, 3 * D, M, D, H,
-                                              T, qk_eps, l.scales, front_rows, n_rows, rows, 1, stream)
+                                              T, qk_eps, l.sumsq, l.scales, l.counters, front_rows, n_rows, rows, 1, stream)
                      : taac_norm_linear_fwd(x, D, w.attn_norm_weight, attn_eps, nullptr, w.qkv_bias, w.qkv_weight, nullptr, 3 * D, l.qkv,
                                             3 * D, M, 3 * D, D, front_rows, n_rows, rows, 1, stream);
     if (rc != TAAC_OK) return rc;

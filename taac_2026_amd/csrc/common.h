@@ -52,17 +52,20 @@ int ffn_splits(int64_t M, int32_t D, int32_t F);
 int64_t ffn_split_bytes(int64_t M, int32_t D, int32_t F);
 // RMSNorm + q | k | v projection with the query / key epilogue (ffn.hip; the arguments of taac_norm_linear_qk_fwd with
 // packed weights, the two norm weights apart) whose output is a stack of per-head planes [3 * num_heads][M][head_dim],
-// head_dim 32 or 64; qk_rstd [2, M]: null, or receives the factors of taac_row_rstd.
+// head_dim 32 or 64; qk_rstd [2, M]: null, or receives the factors of taac_row_rstd; qk_sumsq [2 d_model / 64, M] and qk_counters
+// [kQkCounters], zeros that stay zeros, are then scratch.
+constexpr int kQkCounters = 512;
 int norm_linear_qk_heads(const void* x, int64_t ldx, const void* norm_weight, float eps, const void* bias,
                          const void* packed_weights, void* out, int64_t M, int32_t d_model, int32_t num_heads,
                          int32_t tokens_per_sample, const void* q_weight, const void* k_weight, const void* cos_sin,
-                         float* qk_rstd, const int32_t* rows, const int32_t* n_rows, int norm_folded, void* stream);
+                         float* qk_sumsq, float* qk_rstd, uint32_t* qk_counters, const int32_t* rows, const int32_t* n_rows,
+                         int norm_folded, void* stream);
 // taac_norm_linear_qk_fwd with packed weights and neither norm weight nor rotation, whose statistic leaves as the factors of
-// taac_row_rstd with qk_eps: qk_rstd [2, M].
+// taac_row_rstd with qk_eps: qk_rstd [2, M]; scratch as above.
 int norm_linear_qk_factors(const char* name, const void* x, int64_t ldx, const void* norm_weight, float eps, const void* bias,
                            const void* packed_weights, void* out, int64_t ldo, int64_t M, int32_t d_model, int32_t num_heads,
-                           int32_t tokens_per_sample, float qk_eps, float* qk_rstd, const int32_t* rows, const int32_t* n_rows,
-                           const int32_t* x_rows, int norm_folded, void* stream);
+                           int32_t tokens_per_sample, float qk_eps, float* qk_sumsq, float* qk_rstd, uint32_t* qk_counters,
+                           const int32_t* rows, const int32_t* n_rows, const int32_t* x_rows, int norm_folded, void* stream);
 // Whether the dense layers over at most M rows of D features run as the few-token kernels of ffn_small.hip.
 bool dense_few_rows(int64_t M, int32_t D);
 // Out projection + feed-forward half of a block (ffn.hip; attn_plane: 0 = rows of ld_attn elements, 32 / 64 = per-head

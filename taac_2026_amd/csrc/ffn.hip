@@ -882,15 +882,21 @@ __global__ __launch_bounds__(8 * kWave, 2) void norm_linear_kernel(const TsParam
   const int wg = static_cast<int>(blockIdx.x);
   const int full_rounds = num_tiles / G;
   const int R = num_tiles % G;
-  // With the factors of the query and key norm (qk_rstd) a segment is one or more of the parts q, k, v, so that a workgroup meets all
-  // chunks of a factor.
-  const int unit = QK != 0 && p.qk_rstd != nullptr ? D / kNC : 1, units = nchunks / unit;
   int S = R > 0 ? G / R : 1;
-  S = S < units ? S : units;
+  S = S < nchunks ? S : nchunks;
+  // A factor of the query or key norm (qk_rstd) is a sum over the chunks of its part. A workgroup that holds the whole part sums in
+  // LDS; where the segments cut the parts, their sums meet in memory (below the loop), which costs about a chunk: four or five
+  // segments are made three, the parts themselves. Whole parts everywhere leave most of the chip idle (four blocks, D = 256, sums and
+  // a kernel of their own for the factors / whole parts / meeting, us a call: 14 tiles 241 / 273 / 236, 21 342 / 369 / 337, 42 462 / 464 /
+  // 453, 256 + 5 1863 / 1888 / 1856, 256 + 10 1881 / 1904 / 1872; 48 490 / 482 / 484, 64 555 / 548 / 553).
+  const bool factors = QK != 0 && p.qk_rstd != nullptr;
+  if (factors && S > 3 && S < 6) S = 3;
   const bool has_tail = R > 0 && wg < R * S;
   const int tail_tile = full_rounds * G + wg / S;
-  const int tail_begin = has_tail ? ((wg % S) * units) / S * unit : 0;
-  const int tail_len = has_tail ? (((wg % S) + 1) * units) / S * unit - tail_begin : 0;
+  const int tail_begin = has_tail ? ((wg % S) * nchunks) / S : 0;
+  const int tail_len = has_tail ? (((wg % S) + 1) * nchunks) / S - tail_begin : 0;
+  constexpr int kParts = D / kNC;  // chunks of the query, and of the key
+  const bool meet = factors && has_tail && S != 1 && S != 3;
   const int full_total = full_rounds * nchunks;
   const int total = full_total + tail_len;
   if (total == 0) return;  // whole workgroup: nothing assigned to it
@@ -1151,17 +1157,17 @@ __global__ __launch_bounds__(8 * kWave, 2) void norm_linear_kernel(const TsParam
           float ss = tile_to_lds_sumsq(tile_lds, acc0[t], acc1[t], bv, l32, hh, rstd[t]);
           ss = half_wave_pair_sum(ss);
           const int row = rowinfo[t * 32 + l32].x;
-          if (p.qk_rstd != nullptr) {
-            constexpr int parts = D / kNC;  // chunks of the query, and of the key
-            if (hh == 0) {
-              if (chunk % parts > 0) ss += norm_ss[t * 32 + l32];
-              if (chunk % parts < parts - 1)
-                norm_ss[t * 32 + l32] = ss;
-              else
-                p.qk_rstd[static_cast<int64_t>(chunk / parts) * p.M + row] = rsqrtf(ss * (1.0f / D) + p.qk_eps);
-            }
-          } else {
+          if (p.qk_rstd == nullptr) {
             if (hh == 0) p.qk_sumsq[static_cast<int64_t>(chunk) * p.M + row] = ss;
+          } else if (meet && s >= full_total) {  // read by another workgroup of this launch: through to the chip's common memory
+            if (hh == 0)
+              __hip_atomic_store(p.qk_sumsq + static_cast<int64_t>(chunk) * p.M + row, ss, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+          } else if (hh == 0) {
+            if (chunk % kParts > 0) ss += norm_ss[t * 32 + l32];
+            if (chunk % kParts < kParts - 1)
+              norm_ss[t * 32 + l32] = ss;
+            else
+              p.qk_rstd[static_cast<int64_t>(chunk / kParts) * p.M + row] = rsqrtf(ss * (1.0f / D) + p.qk_eps);
           }
         } else {
           tile_to_lds(tile_lds, acc0[t], acc1[t], bv, l32, hh, rstd[t]);
@@ -1247,6 +1253,43 @@ __global__ __launch_bounds__(8 * kWave, 2) void norm_linear_kernel(const TsParam
       }
     }
     buf = buf == 2 ? 0 : buf + 1;
+  }
+  if constexpr (QK != 0) {
+    if (meet) {  // workgroup-uniform
+      // The workgroup counts the chunks whose sums it has stored; whoever completes a part finds all of them and forms the factors, in
+      // the order of the chunks as everywhere (nobody waits for anybody), and sets the counter back.
+      uint32_t* const arrived = reinterpret_cast<uint32_t*>(smem);
+      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // this wavefront's sums have reached the chip's common memory
+      __syncthreads();                                  // everyone's have, and the weight buffers are free
+      int own[2];
+#pragma unroll
+      for (int part = 0; part < 2; ++part) {
+        const int first = part * kParts, begin = tail_begin > first ? tail_begin : first;
+        const int end = tail_begin + tail_len < first + kParts ? tail_begin + tail_len : first + kParts;
+        own[part] = end > begin ? end - begin : 0;
+        if (tid == part && own[part] > 0)
+          arrived[part] = __hip_atomic_fetch_add(p.qk_counters + 2 * (wg / S) + part, static_cast<uint32_t>(own[part]), __ATOMIC_RELAXED,
+                                                 __HIP_MEMORY_SCOPE_AGENT);
+      }
+      __syncthreads();
+#pragma unroll
+      for (int part = 0; part < 2; ++part) {
+        if (own[part] == 0 || arrived[part] + static_cast<uint32_t>(own[part]) != kParts) continue;
+        if (tid == part) p.qk_counters[2 * (wg / S) + part] = 0u;
+        static_assert(kTokPerWg == NWAVES * kWave, "one token per thread");
+        const int64_t tok = static_cast<int64_t>(tail_tile) * kTokPerWg + tid;
+        if (tok >= count) continue;
+        const int64_t row = token_row(p, count, tok);
+        float sums[kParts], ss = 0.f;
+#pragma unroll
+        for (int c = 0; c < kParts; ++c)
+          sums[c] = __hip_atomic_load(p.qk_sumsq + static_cast<int64_t>(part * kParts + c) * p.M + row, __ATOMIC_RELAXED,
+                                      __HIP_MEMORY_SCOPE_AGENT);
+#pragma unroll
+        for (int c = 0; c < kParts; ++c) ss += sums[c];
+        p.qk_rstd[part * p.M + row] = rsqrtf(ss * (1.0f / D) + p.qk_eps);
+      }
+    }
   }
 }
 
@@ -1659,7 +1702,8 @@ struct QkExtras {
   const void* k_weight = nullptr;
   const void* cos_sin = nullptr;
   float* qk_sumsq = nullptr;
-  float* qk_rstd = nullptr;  // [2][M] factors of the query and key norm, written instead of qk_sumsq
+  float* qk_rstd = nullptr;  // [2][M] factors of the query and key norm; qk_sumsq and qk_counters are then scratch
+  uint32_t* qk_counters = nullptr;
   float qk_eps = 0.f;
   int32_t qk_chunks = 0, head_dim = 0, tokens_per_sample = 0;
   bool enabled = false;
@@ -1726,6 +1770,7 @@ int norm_linear_launch(const char* name, const void* x, int64_t ldx, const void*
   p.qk_w = static_cast<const bf16_t*>(qk.q_weight);
   p.qk_wk = static_cast<const bf16_t*>(qk.k_weight);
   p.qk_rstd = qk.qk_rstd;
+  p.qk_counters = qk.qk_counters;
   p.qk_eps = qk.qk_eps;
   p.cos_sin = static_cast<const bf16_t*>(qk.cos_sin);
   p.qk_sumsq = qk.qk_sumsq;
@@ -1748,6 +1793,7 @@ int norm_linear_launch(const char* name, const void* x, int64_t ldx, const void*
   // it has, so the grid is not held to one workgroup per tile (one request of 512 tokens ran on one compute unit: q | k | v
   // projection 44 -> 12.6 us, 45 900 positions of the narrow network 31 -> 18 us).
   int grid = static_cast<int64_t>(num_tiles) * (N / kNC) < cus ? num_tiles * (N / kNC) : cus;
+  if (qk.qk_rstd != nullptr && grid > kQkCounters) grid = kQkCounters;  // two counters for each of up to grid / 2 divided tiles
   // taac_test_hooks: cap the number of persistent workgroups so that small inputs exercise the multi-tile path.
   if (const int limit = test_max_workgroups(); limit > 0 && limit < grid) grid = limit;
 #define TAAC_LIN_LAUNCH(KK, TT, RR, QQ)                                                                           \
@@ -1823,13 +1869,16 @@ namespace taac {
 int norm_linear_qk_heads(const void* x, int64_t ldx, const void* norm_weight, float eps, const void* bias,
                          const void* packed_weights, void* out, int64_t M, int32_t d_model, int32_t num_heads,
                          int32_t tokens_per_sample, const void* q_weight, const void* k_weight, const void* cos_sin,
-                         float* qk_rstd, const int32_t* rows, const int32_t* n_rows, int norm_folded, void* stream) {
+                         float* qk_sumsq, float* qk_rstd, uint32_t* qk_counters, const int32_t* rows, const int32_t* n_rows,
+                         int norm_folded, void* stream) {
   QkExtras qk;
   qk.enabled = true;
   qk.q_weight = q_weight;
   qk.k_weight = k_weight;
   qk.cos_sin = cos_sin;
+  qk.qk_sumsq = qk_sumsq;
   qk.qk_rstd = qk_rstd;
+  qk.qk_counters = qk_counters;
   qk.qk_eps = eps;
   qk.qk_chunks = 2 * d_model / kNC;
   qk.head_dim = d_model / num_heads;
@@ -1841,11 +1890,13 @@ int norm_linear_qk_heads(const void* x, int64_t ldx, const void* norm_weight, fl
 
 int norm_linear_qk_factors(const char* name, const void* x, int64_t ldx, const void* norm_weight, float eps, const void* bias,
                            const void* packed_weights, void* out, int64_t ldo, int64_t M, int32_t d_model, int32_t num_heads,
-                           int32_t tokens_per_sample, float qk_eps, float* qk_rstd, const int32_t* rows, const int32_t* n_rows,
-                           const int32_t* x_rows, int norm_folded, void* stream) {
+                           int32_t tokens_per_sample, float qk_eps, float* qk_sumsq, float* qk_rstd, uint32_t* qk_counters,
+                           const int32_t* rows, const int32_t* n_rows, const int32_t* x_rows, int norm_folded, void* stream) {
   QkExtras qk;
   qk.enabled = true;
+  qk.qk_sumsq = qk_sumsq;
   qk.qk_rstd = qk_rstd;
+  qk.qk_counters = qk_counters;
   qk.qk_eps = qk_eps;
   qk.qk_chunks = 2 * d_model / kNC;
   qk.head_dim = d_model / num_heads;
@@ -1892,7 +1943,8 @@ bool ffn_few_rows(int64_t M, int32_t D) { return test_max_workgroups() == 0 && M
 
 // Whether a projection over at most M rows of D features runs as the few-token kernel. Measured for q | k | v (launches
 // back to back, few-token / persistent kernel, us): D = 256 - 512 rows 6.0 / 13.6, 4096 9.9 / 14.1, 8192 14.4 / 15.6,
-// 16384 24.5 / 21.4; D = 128 - 512 rows 3.8 / 8.7, 8192 6.3 / 9.2, 16384 9.6 / 10.4, 24576 12.6 / 12.4. Below the line a tile's
+// 16384 24.5 / 21.4; D = 128 - 512 rows 3.8 / 8.7, 8192 6.3 / 9.2, 16384 9.6 / 10.4, 24576 12.6 / 12.4. With query / key norms, four
+// whole blocks: D = 256 - 8192 rows 230 / 238, 10240 330 / 332, 16384 387 / 386; D = 128 - 16384 170 / 182, 20480 222 / 213. Below the line a tile's
 // latency chain decides, above it the weights, which every 32-token workgroup fetches from L2 for itself.
 bool dense_few_rows(int64_t M, int32_t D) {
   return test_max_workgroups() == 0 && M * D <= 10240 * 256;  // taac_test_hooks: a capped grid keeps the persistent kernels

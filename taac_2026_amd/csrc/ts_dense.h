@@ -43,7 +43,9 @@ struct TsParams {
   const bf16_t* qk_wk;      // [D] norm weight of the key features, with qk_w
   const bf16_t* cos_sin;    // rotary table [tokens_per_sample][head_dim] of (cos, sin) pairs, or null
   float* qk_sumsq;          // [qk_chunks][M] sum of squares of a token's 64 features of one chunk
-  float* qk_rstd;           // few-token form: [2][M] factors of the query and key norm (instead of qk_sumsq), or null
+  float* qk_rstd;           // [2][M] factors of the query and key norm, or null. Given, it takes the place of qk_sumsq, which the
+                            // persistent kernel then uses for the token tiles whose chunks it divides over workgroups
+  uint32_t* qk_counters;    // persistent kernel, with qk_rstd: [kQkCounters], zero before the launch and behind it
   float qk_eps;
   int32_t qk_chunks;        // leading 64-feature chunks that belong to the query and key projections
   int32_t head_dim, tokens_per_sample;

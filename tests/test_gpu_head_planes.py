@@ -149,11 +149,12 @@ def test_backbone_plane_route_equals_its_row_major_route(device, d_model, heads,
         assert torch.equal(hidden, hidden_rows)
 
 
-@pytest.mark.parametrize("workgroups", [1, 2, 5, 7])
+@pytest.mark.parametrize("workgroups", [1, 2, 5, 7, 10, 13, 18, 23, 36, 37])
 @pytest.mark.parametrize("d_model,rope_base", [(256, None), (256, 10000.0), (128, None)])
 def test_norm_factors_of_the_projection_equal_those_of_their_own_kernel(device, test_hooks, workgroups, d_model, rope_base):
-    """The plane route's projection sums the query / key statistic over its chunks and stores the factors (a divided last round
-    of tiles is then cut between q, k and v); the row-major route leaves the sums to a kernel of their own. Same order, same bits."""
+    """The plane route's projection sums the query / key statistic over its chunks and stores the factors - the three tiles here in
+    one to twelve segments, where these cut q, k or v with the sums meeting in memory, in both blocks; the row-major route leaves
+    the sums to a kernel of their own. Same order, same bits."""
     test_hooks(max_workgroups=workgroups)
     inputs = workloads.backbone_inputs(batch=9, n_feature_tokens=8, n_sequence_tokens=233, d_model=d_model, num_heads=4, d_ff=128,
                                        n_blocks=2, min_sequence_len=1, seed=workgroups)
