@@ -1108,20 +1108,31 @@ bool small_offsets(int64_t rows, int64_t stride) {
 }
 
 // The fused kernel where a workgroup can hold a sample's keys (512 of 32 features, 256 of 64) and there are enough (sample, head)
-// pairs: it has one workgroup per pair where the two kernels have one per 128 rows. Both sides in us, lengths ~ U{16..rows}:
-//   up to 128 rows (as many workgroups either way):  8 x 48 x 32, 256 pairs 9.0 -> 6.3, 16384 pairs 113 -> 113; 128 x 64 15.5 -> 11.5
-//   256 x 32:  256 pairs 17.3 -> 18.5, 512 pairs 25.3 -> 24.1, 4096 pairs 134 -> 99;  256 x 64:  256 pairs 26.8 -> 27.5, 512 pairs 46 -> 37,
-//   8192 pairs 493 -> 343;  512 x 32:  512 pairs 52 -> 60 (causal 46 -> 42), 1024 pairs 101 -> 96, 16384 pairs 1443 -> 1024.
-// Mask bits over more than 256 rows of 32 features stay with the two kernels: the words' registers are the ones that the four key
-// tiles of a wavefront need (300 rows, 1024 pairs: 65 -> 74; 512 rows 131 -> 130).
+// pairs: it has one workgroup per pair where the two kernels have one per 128 rows. Two kernels / fused in us, lengths ~ U{16..rows}:
+//   up to 128 rows (as many workgroups either way):  48 x 32, 256 pairs 8.8 / 6.8, 8192 pairs 58 / 54;  128 x 64, 256 pairs 15.7 / 12.6,
+//   16384 pairs 453 / 330.
+//   256 x 32:  256 pairs 20.0 / 20.5, 512 pairs 27.7 / 24.9, 4096 pairs 165 / 122;  256 x 64:  256 pairs 27.1 / 28.7, 512 pairs 48 / 38,
+//   8192 pairs 517 / 371.
+//   More rows of 32 features, four key tiles per wavefront and half the wavefronts in flight. In three blocks of 128 the two kernels
+//   hold their own: 300 rows, 1024 pairs 55 / 54 and 50 / 53 (two draws of the lengths), 2048 pairs 85 / 92, 3584 pairs 169 / 164, 8192
+//   pairs 356 / 321. In four: 400 rows, 1024 pairs 85 / 70, 8192 pairs 688 / 451; 480 rows, 1024 pairs 101 / 101; 512 rows, 1024 pairs 108 /
+//   117 and 102 / 99, 1536 pairs 152 / 148 and 140 / 132, 8192 pairs 814 / 624. Causal, 300 rows, 512 pairs 31 / 28, 512 rows 65 / 54.
+// Mask bits, 32 features: as above up to 256 rows (256 rows, 512 pairs 34 / 30, 8192 pairs 368 / 297), but the kernel spills, and where
+// it could gain little, up to 128 rows, it loses once a tensor is more than some 25 MB: 48 rows, 8192 pairs 68 / 65, 12288 pairs 100 / 108;
+// 96 rows, 4096 pairs 52 / 50, 8192 pairs 108 / 133; 128 rows, 3072 pairs 52 / 48, 6144 pairs 97 / 124. Over more rows they stay with the
+// two kernels: the words' registers are the ones that the four key tiles of a wavefront need. 300 rows, 1024 pairs 67 / 74, 4096 pairs 239 /
+// 274; 350 rows, 4096 pairs 280 / 319. (It would gain from 400 rows and 2048 pairs on: 403 rows, 1024 pairs 117 / 116, 4096 pairs 436 / 360;
+// 512 rows, 1024 pairs 145 / 152, 4096 pairs 535 / 471.)
 template <typename T, int DP, int MODE, bool COMPACT>
 bool launch_bwd_fused(AttnBwdParams p, hipStream_t s) {
   constexpr int kSmall = 64 / DP, kLarge = 128 / DP;  // key tiles per wavefront
   constexpr int kRowsSmall = kSmall * kOwn, kRowsLarge = DP == 32 && MODE == kMaskBits ? kRowsSmall : kLarge * kOwn;
   const int64_t pairs = static_cast<int64_t>(p.B) * p.H;
   const int32_t rows = p.Tq > p.Tk ? p.Tq : p.Tk;
-  const int64_t enough = rows <= kOwn ? 1 : (DP == 32 && rows > kRowsSmall && !p.causal ? 1024 : 512);
+  int64_t enough = rows <= kOwn ? 1 : 512;
+  if (DP == 32 && rows > kRowsSmall && !p.causal) enough = rows <= 3 * kOwn ? 3584 : (rows <= 480 ? 1024 : 1536);
   if (rows > kRowsLarge || pairs < enough) return false;
+  if (DP == 32 && MODE == kMaskBits && rows <= kOwn && rows * pairs > 400000) return false;
   if (!small_offsets(p.Tq, p.qs[2]) || !small_offsets(p.Tq, p.dos[2]) || !small_offsets(p.Tk, p.ks[2])) return false;
   p.nblk = 1;
   p.total = static_cast<uint32_t>(pairs);

@@ -237,7 +237,8 @@ def _check_gradients(got, other, exact, dtype):
 @pytest.mark.parametrize("rows,keys,dim,batch,heads", [
     (1, 1, 32, 3, 2), (31, 31, 64, 3, 2), (33, 33, 32, 3, 2), (128, 128, 64, 5, 2), (100, 37, 32, 3, 2), (20, 128, 64, 3, 2),
     (129, 129, 32, 64, 8), (256, 256, 32, 64, 8), (257, 257, 32, 128, 8), (490, 490, 32, 128, 8), (512, 512, 32, 128, 8),
-    (129, 129, 64, 128, 4), (256, 256, 64, 128, 4), (257, 257, 64, 128, 4)])
+    (129, 129, 64, 128, 4), (256, 256, 64, 128, 4), (257, 257, 64, 128, 4), (257, 257, 32, 448, 8), (384, 384, 32, 448, 8),
+    (385, 385, 32, 128, 8), (512, 512, 32, 192, 8)])
 @pytest.mark.parametrize("dtype,causal,zero_pad", [(torch.bfloat16, False, True), (torch.float16, True, False), (torch.bfloat16, True, True)])
 def test_backward_with_all_keys_in_one_workgroup(device, rows, keys, dim, batch, heads, dtype, causal, zero_pad):
     if rows != keys and zero_pad:
