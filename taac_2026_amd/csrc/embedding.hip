@@ -236,11 +236,13 @@ void launch_bag_bwd(const void* values, int64_t bags, int bag_size, const void* 
 // The sort is bound by its atomics (one per slot on counts of every row in memory: 57 us of 94 for the above) and its scattered
 // accesses. It therefore goes over kBuckets sets of rows: a workgroup counts its share of the slots per set in LDS and reserves
 // its places with one add per set, places the slots set by set, and one workgroup per set then counts, scans and places by row
-// in LDS. The sets are dealt out in runs of kRun rows, so that popular neighbours spread over all of them. Measured for the
+// in LDS. The sets are dealt out in runs of kRun rows, so that popular neighbours spread over all of them, in single rows where the
+// table is small enough that its counts stay in L2 (16 000 rows, 262 144 slots under a 1 / id popularity 89 -> 61 us). A set is one
+// workgroup's work, however many slots name it: see bag_sort for what that costs. Measured for the
 // above: counts 10, places 13, sort 13 us; the whole gradient 145 -> 91 us, 40 000 x 64 with 400 000 x 10 slots 691 -> 216, 2 000 000 x 16
 // with 524 288 x 12 528 -> 260. 4096 slots a share: with half as many the adds on the sets' cursors cost more (98 us) than the
 // second workgroup per compute unit gives.
-// A small table with many slots is counted as a whole in LDS instead.
+// A small table with many slots is counted as a whole in LDS instead, one of very many rows with many slots in memory.
 // Bound: the table's gradient (written once) and the gathered rows of grad_out.
 constexpr int kHot = 64;        // longest row that one lane group sums by itself
 constexpr int kHotChunk = 256;  // entries of a chunk, at least
@@ -249,11 +251,12 @@ constexpr int kRowsPerThread = 8;
 constexpr int kLocalRows = 16384;  // largest table whose counts a workgroup keeps in LDS
 constexpr int kLocalThreads = 1024;
 constexpr int kBuckets = 256;       // sets of rows
-constexpr int kRun = 8;             // consecutive rows of a set
+constexpr int kRun = 8;             // consecutive rows of a set; its rows are a multiple of that
 constexpr int kBucketRows = kLocalThreads * kRowsPerThread;  // rows of a set that are counted at once
 constexpr int kCursors = 64 + kBuckets;  // places of the cursors in front of the counts, whole cache lines
 constexpr int kBucketShare = 4096;  // slots of a workgroup, at least
 constexpr int kBucketShares = 512;  // workgroups, at most (about)
+constexpr int kTogether = 32;       // lanes of a wavefront that name one row and add together, at least
 
 struct BagEntry {
   int32_t bag;
@@ -273,20 +276,39 @@ struct SortedBags {
   HotChunk* chunks;  // [slots / kHot]
   float* partial;    // [slots / kHot][emb_dim]
   int32_t set_rows;  // rows of a set, a multiple of kRun; 0: not sorted by sets, rows in their order
+  int32_t run_log2;  // consecutive rows of a set
   int32_t share_bags, shares;
   int64_t bytes;
 
   // Position of a row in counts and start.
   __device__ __forceinline__ int64_t position(int64_t row) const {
     if (set_rows == 0) return row;
-    const uint32_t r = static_cast<uint32_t>(row), run = r / kRun;  // fewer than 2^30 rows
-    return static_cast<int64_t>(run % kBuckets) * set_rows + run / kBuckets * kRun + r % kRun;
+    const uint32_t r = static_cast<uint32_t>(row);  // fewer than 2^30 rows
+    return static_cast<int64_t>(set_of(r)) * set_rows + row_in_set(r);
+  }
+  __device__ __forceinline__ uint32_t set_of(uint32_t row) const { return (row >> run_log2) % kBuckets; }
+  __device__ __forceinline__ uint32_t row_in_set(uint32_t row) const {
+    return ((row >> run_log2) / kBuckets << run_log2) + (row & ((1u << run_log2) - 1));
   }
 };
-// Whether the counts of the whole table are formed in LDS: every workgroup clears and adds up all of them, and in the sets' form the
-// adds of few rows queue up in LDS. In LDS / by sets, us: 1 000 x 32, 524 288 x 12 slots 229 / 564; 1 000 x 16, 65 536 x 4 49.6 / 52.5;
-// 16 000 x 128, 30 000 x 12 126 / 62.
-bool counts_in_lds(int64_t n, int64_t slots) { return n <= kLocalRows && slots >= 256 * std::max<int64_t>(n, kLocalThreads); }
+enum class BagSort { kLocal, kSets, kMemory };
+// Where the counts of the rows are formed, by size alone. Gradient in us, ids with u^2 / 1 / id popularity / 30 % of the slots on one id.
+// kLocal, the whole table in LDS: every workgroup clears and adds up all rows, but its adds to a popular row meet few others. kSets: the
+// workgroup of the set with the popular row sorts all slots that name it.
+//   3 rows, 65 536 slots in LDS 32 (u^2), by sets 100; 200 rows, 65 536 33 / 37; 1 024 rows, 65 536 44 / 43 / 39, by sets 41 / 42 / 54;
+//   262 144 50 / 68 / 68, 48 / 68 / 119.  4 096 rows: 262 144 73 / 75 / 70, 51 / 63 / 116; 524 288 87 / 96 / 99, 83 / 97 / 206; 786 432
+//   95 / 104 / 107, 95 / 126 / 284.  16 000 rows: 262 144 101 / 118 / 109, 47 / 62 / 113; 1 048 576 138 / 156 / 150, 93 / 139 / 344; 2 048 000
+//   163 / 185 / 215, 137 / 239 / 712.  The line stands where u^2 gains at most a sixth by sets and one popular row would cost threefold.
+// kMemory, a returning add per slot: an id that many slots name queues up there (1 000 000 rows, 1 048 576 slots, 10 % of them on one id: in
+// memory 1 003, by sets 181; all of them 9 078, 1 106), but a set of more rows than LDS holds walks its slots again for each kBucketRows of
+// them. u^2, in memory / by sets: 10 000 000 rows, 30 000 000 slots 2 480 / 2 250; 50 000 000 rows, 6 291 456 1 499 / 1 436, 30 000 000 3 040 /
+// 4 400; 100 000 000 rows, 6 291 456 1 850 / 1 850; 200 000 000 rows, 1 048 576 2 480 / 1 860, 6 291 456 3 260 / 3 700, 30 000 000 5 380 /
+// 11 900; 10^9 rows, 1 048 576 9 670 / 9 600, 6 291 456 12 500 / 29 700.
+BagSort bag_sort(int64_t n, int64_t slots) {
+  if (n <= kLocalThreads || (n <= kLocalRows && slots >= 128 * n)) return BagSort::kLocal;
+  const int64_t walks = (n + kBuckets * kBucketRows - 1) / (static_cast<int64_t>(kBuckets) * kBucketRows);
+  return slots * walks <= 300000000 ? BagSort::kSets : BagSort::kMemory;
+}
 
 SortedBags sorted_layout(char* base, int64_t n, int64_t bags, int bag_size, int emb_dim) {
   SortedBags b{};
@@ -298,8 +320,9 @@ SortedBags sorted_layout(char* base, int64_t n, int64_t bags, int bag_size, int 
   };
   const int64_t slots = bags * bag_size;
   int64_t rows = n;
-  if (!counts_in_lds(n, slots)) {
+  if (bag_sort(n, slots) == BagSort::kSets) {
     b.set_rows = static_cast<int32_t>((n + kRun * kBuckets - 1) / (kRun * kBuckets) * kRun);
+    b.run_log2 = n <= kLocalRows ? 0 : 3;
     rows = static_cast<int64_t>(b.set_rows) * kBuckets;
     const int64_t share = std::max<int64_t>(kBucketShare, slots / kBucketShares);
     b.share_bags = static_cast<int32_t>(std::max<int64_t>(1, share / bag_size));
@@ -325,6 +348,15 @@ __global__ __launch_bounds__(kBlock) void bag_clear_kernel(int32_t* __restrict__
 #pragma unroll
   for (int e = 0; e < 4; ++e)
     if (i + e < n) counts[i + e] = 0;
+}
+
+// One returning add in memory per slot.
+template <typename I>
+__global__ __launch_bounds__(kBlock) void bag_count_kernel(const I* __restrict__ values, int64_t slots, int64_t n, SortedBags b) {
+  const int64_t i = static_cast<int64_t>(blockIdx.x) * kBlock + threadIdx.x;
+  if (i >= slots) return;
+  const int64_t id = static_cast<int64_t>(values[i]);
+  if (id > 0 && id < n) b.rank[i] = atomicAdd(b.counts + id, 1);
 }
 
 // A table small enough that a workgroup counts its share of the slots in LDS and reserves each row's places with one add.
@@ -411,8 +443,6 @@ __global__ __launch_bounds__(kBlock) void bag_start_kernel(int64_t n, SortedBags
 }
 
 // ---- by sets of rows ----
-__device__ __forceinline__ uint32_t bucket_of(int64_t id) { return static_cast<uint32_t>(id) / kRun % kBuckets; }
-
 // Entries of every set: a share's are counted in LDS and reserved with one add, whose result is where they begin in the set.
 template <typename I>
 __global__ __launch_bounds__(kLocalThreads) void bag_set_count_kernel(const I* __restrict__ values, int64_t slots, int bag_size, int64_t n,
@@ -428,7 +458,7 @@ __global__ __launch_bounds__(kLocalThreads) void bag_set_count_kernel(const I* _
     for (int k = 0; k < kAhead; ++k) id[k] = i + k * kLocalThreads < end ? static_cast<int64_t>(values[i + k * kLocalThreads]) : 0;
 #pragma unroll
     for (int k = 0; k < kAhead; ++k)
-      if (id[k] > 0 && id[k] < n) atomicAdd(count + bucket_of(id[k]), 1);
+      if (id[k] > 0 && id[k] < n) atomicAdd(count + b.set_of(static_cast<uint32_t>(id[k])), 1);
   }
   __syncthreads();
   for (int t = threadIdx.x; t < kBuckets; t += kLocalThreads) {
@@ -463,12 +493,35 @@ __global__ __launch_bounds__(kLocalThreads) void bag_set_place_kernel(const I* _
     for (int j = lane; j < bag_size; j += lanes) {
       const int64_t id = static_cast<int64_t>(ids[j]);
       if (id > 0 && id < n) {
-        const int32_t at = atomicAdd(next + bucket_of(id), 1);
+        const int32_t at = atomicAdd(next + b.set_of(static_cast<uint32_t>(id)), 1);
         b.by_set[at] = BagEntry{static_cast<int32_t>(bag), inv};
-        b.rank[at] = static_cast<int32_t>(static_cast<uint32_t>(id) / (kRun * kBuckets) * kRun + static_cast<uint32_t>(id) % kRun);
+        b.rank[at] = static_cast<int32_t>(b.row_in_set(static_cast<uint32_t>(id)));
       }
     }
   }
+}
+
+// next[r] += 1 for every lane that takes part; returns its value before. Where a popular row fills the set, the lanes that name it add
+// together: as adds to one address they queue up, two clocks each (1 000 000 rows, 1 048 576 slots, half of them on one id: 787 -> 579 us).
+template <bool RETURN>
+__device__ __forceinline__ int32_t add_row(int32_t* next, uint32_t r, bool takes_part) {
+  const uint64_t open = __ballot(takes_part);
+  int32_t at = 0;
+  if (__popcll(open) >= kTogether) {  // wavefront-uniform, as all of this
+    const int lane = threadIdx.x % kWave, first = __ffsll(static_cast<unsigned long long>(open)) - 1;
+    const uint32_t row = __builtin_amdgcn_readlane(r, first);
+    const uint64_t same = __ballot(r == row);
+    if (__popcll(same) >= kTogether) {
+      if (lane == first) at = atomicAdd(next + row, __popcll(same));
+      if (RETURN) at = __builtin_amdgcn_readlane(at, first) + __popcll(same & ((1ull << lane) - 1));
+      takes_part = takes_part && r != row;
+    }
+  }
+  if (takes_part) {
+    const int32_t own = atomicAdd(next + r, 1);
+    if (RETURN) at = own;
+  }
+  return at;
 }
 
 // One workgroup per set: counts, starts and places of its rows in LDS, kBucketRows of them at a time.
@@ -486,9 +539,9 @@ __global__ __launch_bounds__(kLocalThreads) void bag_set_sort_kernel(SortedBags 
 #pragma unroll
     for (int e = 0; e < kRowsPerThread; ++e) next[t + e * kLocalThreads] = 0;
     __syncthreads();
-    for (int32_t i = begin + t; i < end; i += kLocalThreads) {
-      const uint32_t r = static_cast<uint32_t>(b.rank[i] - r0);
-      if (r < static_cast<uint32_t>(kBucketRows)) atomicAdd(next + r, 1);
+    for (int32_t i0 = begin; i0 < end; i0 += kLocalThreads) {  // whole wavefronts
+      const uint32_t r = i0 + t < end ? static_cast<uint32_t>(b.rank[i0 + t] - r0) : ~0u;
+      add_row<false>(next, r, r < static_cast<uint32_t>(kBucketRows));
     }
     __syncthreads();
     int32_t c[kRowsPerThread], mine = 0, total;
@@ -515,9 +568,11 @@ __global__ __launch_bounds__(kLocalThreads) void bag_set_sort_kernel(SortedBags 
       }
     }
     __syncthreads();
-    for (int32_t i = begin + t; i < end; i += kLocalThreads) {
-      const uint32_t r = static_cast<uint32_t>(b.rank[i] - r0);
-      if (r < static_cast<uint32_t>(kBucketRows)) b.entries[atomicAdd(next + r, 1)] = b.by_set[i];
+    for (int32_t i0 = begin; i0 < end; i0 += kLocalThreads) {
+      const uint32_t r = i0 + t < end ? static_cast<uint32_t>(b.rank[i0 + t] - r0) : ~0u;
+      const bool takes_part = r < static_cast<uint32_t>(kBucketRows);
+      const int32_t place = add_row<true>(next, r, takes_part);
+      if (takes_part) b.entries[place] = b.by_set[i0 + t];
     }
     at0 += total;
   }
@@ -660,14 +715,18 @@ int launch_sorted(const I* values, int64_t bags, int bag_size, const T* grad_out
     hipLaunchKernelGGL(bag_set_count_kernel<I>, dim3(b.shares), dim3(kLocalThreads), 0, s, values, slots, bag_size, n, b);
     hipLaunchKernelGGL(bag_set_place_kernel<I>, dim3(b.shares), dim3(kLocalThreads), 0, s, values, bags, bag_size, n, lanes, b);
     hipLaunchKernelGGL(bag_set_sort_kernel, dim3(kBuckets), dim3(kLocalThreads), 0, s, b);
-  } else {
+  } else if (bag_sort(n, slots) == BagSort::kLocal) {
     const int64_t share = std::max<int64_t>(4 * n, 4 * kLocalThreads);  // slots of a workgroup, so that its counts pay
     auto kernel = bag_count_local_kernel<I>;
     const size_t lds = static_cast<size_t>(n) * 4;
     if (hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, kLocalRows * 4) != hipSuccess)
       return set_error(TAAC_ERR_LAUNCH, "%s: cannot reserve %zu bytes of LDS", name, lds);
-    const uint32_t grid = static_cast<uint32_t>(std::min<int64_t>(slots / share, 512));
+    const uint32_t grid = static_cast<uint32_t>(std::min<int64_t>(std::max<int64_t>(slots / share, 1), 512));
     hipLaunchKernelGGL(kernel, dim3(grid), dim3(kLocalThreads), lds, s, values, slots, static_cast<int32_t>(n), b);
+  } else {
+    hipLaunchKernelGGL(bag_count_kernel<I>, blocks(slots), dim3(kBlock), 0, s, values, slots, n, b);
+  }
+  if (b.set_rows == 0) {
     hipLaunchKernelGGL(bag_start_kernel, blocks((n + kRowsPerThread - 1) / kRowsPerThread), dim3(kBlock), 0, s, n, b);
     hipLaunchKernelGGL(bag_place_kernel<I>, blocks(bags * lanes), dim3(kBlock), 0, s, values, bags, bag_size, n, lanes, b);
   }

@@ -180,13 +180,22 @@ def test_backward_skips_ids_outside_the_table_and_needs_no_gradient_when_frozen(
     (torch.bfloat16, torch.int32, 1_000, 32, 40_000, 4),      # counts in LDS, every row in several chunks
     (torch.float16, torch.int64, 3, 512, 3_000, 5),           # the widest row (64 pieces), two rows hold everything
     (torch.float32, torch.int64, 70_001, 20, 60_000, 4),      # five of eight lanes hold a piece
-    (torch.float32, torch.int32, 17_000, 4, 400_000, 3),      # one piece; counts in memory
+    (torch.float32, torch.int32, 17_000, 4, 400_000, 3),      # one piece; sets of runs of eight rows
     (torch.bfloat16, torch.int64, 600_000, 8, 40, 70),        # bags of more than 64 slots
-    (torch.bfloat16, torch.int64, 1_000, 32, 70_000, 4),      # enough slots per row that every workgroup counts the whole table
+    (torch.bfloat16, torch.int64, 1_000, 32, 70_000, 4),      # the same with every workgroup's share at its largest
     (torch.float32, torch.int32, 2_200_001, 4, 700_000, 2),   # sets of more rows than are counted at once, the last one partly filled
-    (torch.bfloat16, torch.int32, 2_049, 64, 2_000, 33),      # one run of rows more than there are sets; few rows in chunks
-    (torch.float16, torch.int64, 8, 64, 20_000, 4),           # one run: all slots in one set
+    (torch.bfloat16, torch.int32, 2_049, 64, 2_000, 33),      # sets of eight rows, or nine, one of them with a popular one
+    (torch.float16, torch.int64, 8, 64, 20_000, 4),           # a table of a few rows
     (torch.float16, torch.int64, 40_000, 128, 9, 6_000),      # a bag larger than a workgroup's share
+    (torch.float32, torch.int32, 1_000, 32, 140_000, 2),      # counts in LDS for the other types
+    (torch.float16, torch.int32, 3, 64, 70_000, 4),
+    (torch.bfloat16, torch.int64, 1_024, 64, 9_000, 8),       # the largest table that is always counted there, and one row more
+    (torch.bfloat16, torch.int64, 1_025, 64, 9_000, 8),
+    (torch.bfloat16, torch.int32, 2_000, 32, 64_000, 4),      # as many slots as that takes for more rows, and one bag less
+    (torch.bfloat16, torch.int32, 2_000, 32, 63_999, 4),
+    (torch.float16, torch.int64, 16_384, 16, 300_000, 7),     # the largest table in LDS, and the smallest in runs of eight rows
+    (torch.float16, torch.int64, 16_385, 16, 300_000, 7),
+    (torch.float32, torch.int32, 40_000_000, 4, 5_000_000, 4),  # too many rows and slots for the sets: counts in memory
 ])
 def test_backward_of_sorted_slots(device, dtype, index_dtype, rows, dim, bags, bag_size):
     """The sorted form against float64: an element's error is at most (terms + 2) * 2^-24 of the sum of its terms' magnitudes
