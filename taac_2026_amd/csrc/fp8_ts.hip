@@ -3,8 +3,9 @@
 // with q(a) formed while the token rows are loaded (bf16 activations) or taken as given (e4m3 activations), and the
 // epilogues of taac_linear_fp8 (none / + residual / SiLU-gate).
 //
-// Same scheme as the bf16 token-stationary linear kernel: a persistent workgroup of 8 wavefronts owns 512 tokens at a
-// time (two 32-token tiles per wavefront; one with the residual epilogue); each wavefront quantises its rows once into MFMA B-operand fragments
+// Same scheme as the bf16 token-stationary linear kernel: a persistent workgroup of 8 wavefronts works on tiles of 512 tokens
+// (two 32-token tiles per wavefront; one with the residual epilogue), on a run of the steps of consecutive tiles that may begin and end
+// inside one, or on whole tiles where a row has to be seen as a whole (whole_tiles); each wavefront quantises its rows once into MFMA B-operand fragments
 // (v_mfma_scale_f32_32x32x64_f8f6f4: lane (l32, hh) holds the 32 bytes k = 64*ks + 32*hh .. +31 of token l32) and keeps
 // them in 64 registers; the e4m3 weights stream L2 -> LDS by DMA, 64 weight rows per step, through a ring of three
 // buffers two steps ahead of their use. A fragment (32 rows x 64 k) is 2 KB in LDS: two 1 KB halves, each written by
@@ -450,9 +451,6 @@ __global__ __launch_bounds__(kWaves * kWave, 2) void linear_fp8_ts_kernel(const 
   }
 }
 
-// Launches the token-stationary kernel when the shape fits it: K = 256 (any epilogue, weight rows a multiple of 64) or
-// K = 1024 (no SiLU-gate, weight rows a multiple of 32), 16-byte aligned rows. Returns TAAC_OK after a launch, a negative
-// status on a launch error and 1 when the shape is not covered (the caller then uses the tiled kernel).
 // Whether the output may overwrite rows that another step of the same tile still has to read (rows in place, at any column).
 bool rows_in_place(const Fp8TsParams& p, int a_bytes) {
   const intptr_t apart = reinterpret_cast<intptr_t>(p.out) - reinterpret_cast<intptr_t>(p.a);
@@ -460,6 +458,9 @@ bool rows_in_place(const Fp8TsParams& p, int a_bytes) {
   return p.lda * a_bytes == pitch && apart < pitch && apart > -pitch;
 }
 
+// Launches the token-stationary kernel when the shape fits it: K = 256 (any epilogue, weight rows a multiple of 64) or
+// K = 1024 (no SiLU-gate, weight rows a multiple of 32), 16-byte aligned rows. Returns TAAC_OK after a launch, a negative
+// status on a launch error and 1 when the shape is not covered (the caller then uses the tiled kernel).
 template <int K>
 int launch_fp8_ts_for_k(Fp8TsParams p, int a_is_fp8, int epilogue, hipStream_t s, const char* name) {
   const size_t lds_bytes = static_cast<size_t>(3 * step_bytes(K)) + static_cast<size_t>(kWaves) * 32 * tile_row_bytes(K) +
