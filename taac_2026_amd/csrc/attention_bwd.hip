@@ -733,16 +733,6 @@ struct Mfma16<f16_t> {
   }
 };
 
-// acc + a[e] * b[e] + a[e + 1] * b[e + 1] in float32.
-__device__ __forceinline__ float dot2(bf16x8 a, bf16x8 b, int e, float acc) {
-  typedef __attribute__((__vector_size__(2 * sizeof(__bf16)))) __bf16 bf16x2;
-  return __builtin_amdgcn_fdot2_f32_bf16(bf16x2{a[e], a[e + 1]}, bf16x2{b[e], b[e + 1]}, acc, false);
-}
-__device__ __forceinline__ float dot2(f16x8 a, f16x8 b, int e, float acc) {
-  typedef __attribute__((__vector_size__(2 * sizeof(_Float16)))) _Float16 f16x2;
-  return __builtin_amdgcn_fdot2(f16x2{a[e], a[e + 1]}, f16x2{b[e], b[e + 1]}, acc, false);
-}
-
 // dQ, dK and dV of one (batch, head) in one workgroup, for samples whose keys it can hold: S, dP and the exponentials are
 // formed once instead of twice (five products per pair of tiles instead of seven) and every tensor is read once.
 // Wavefront w owns the 32-key tiles w, w + 4, ... (NT of them: their dK / dV accumulators and V fragments stay in
@@ -750,7 +740,10 @@ __device__ __forceinline__ float dot2(f16x8 a, f16x8 b, int e, float acc) {
 // owns a key, so P and dS come out of the first products as the B operands of dV and dK; dQ contracts over the keys
 // instead: the dS tiles of all wavefronts meet in LDS ([key][query], 16 bits as every operand) and each wavefront forms
 // its own 16 queries x 16 features (DP = 64: twice) of dQ over all key tiles, so dQ, too, has one writer per element and
-// a fixed order.
+// a fixed order. Every sum is formed in the order of the two kernels and every value rounded as there, so that without a mask the
+// gradients are theirs to the bit, whichever route a batch's size takes. (D added up over eight lanes a row, the start value of dP, and
+// 1 / sqrt(d) at the end save three instructions per pair, 1024 x 8 x 512 x 32 604 instead of 638 us, 2048 x 4 x 256 x 64 371 instead of
+// 383, but move a quarter of dQ and dK at d = 32 by a rounding, which a few layers make 0.2 % of every gradient.)
 template <int DP, int NT, bool BITS>
 struct FusedLayout {
   static constexpr int kRows = 32;                                     // streamed queries per step
@@ -774,10 +767,10 @@ void attn_bwd_fused_kernel(const AttnBwdParams p) {
   constexpr int KSTEPS = DP / 16, MB = DP / 32, C8 = DP / 8, kRows = L::kRows, ROWB = L::ROWB, TILE_BYTES = L::TILE_BYTES;
   constexpr int kWaves = L::kWaves;
   [[maybe_unused]] constexpr int kWords = L::kTiles * kRows;
-  // dS is rounded with its 1 / sqrt(d), as in the two kernels. Where that is a power of two and bf16's range holds the rest, it
-  // multiplies dK and dQ at the end instead: the same bits. (With 1 / sqrt(32) at the end as well the gradients are others by 0.3 % and
-  // no closer to float64: dQ of 512 x 250 x 32 0.002391 against 0.002387; 1024 x 8 x 512 x 32 608 against 621 us.)
-  constexpr bool LATE_SCALE = DP == 64 && std::is_same<T, bf16_t>::value;
+  // With mask bits, where the kernel spills, the products dP start from -D, and a scale that is a power of two multiplies dK and dQ at the
+  // end, the same bits in bf16's range: 512 x 8 x 250 x 32 167 instead of 186 us. (The two kernels start dK's products so and round its dS
+  // before the scale: dQ and dK are each within a rounding of theirs, no further from float64.)
+  constexpr bool START_D = BITS, LATE_SCALE = BITS && DP == 64 && std::is_same<T, bf16_t>::value;
   __shared__ __attribute__((aligned(1024))) uint8_t smem[L::BYTES];
   uint8_t* const k_image = smem;
   uint8_t* const ds_image = smem + L::K_BYTES;
@@ -855,38 +848,34 @@ void attn_bwd_fused_kernel(const AttnBwdParams p) {
         }
       }
     };
-    // The statistics of all queries: D from one 16-byte piece of O and dO per thread, summed over the C8 threads of a row; base-2
-    // log-sum-exp, +inf for a row that carries nothing: exp2(x - inf) = 0. Rows of the last chunk at or beyond q_valid among them.
+    // The statistics of all queries: base-2 log-sum-exp, +inf for a row that carries nothing: exp2(x - inf) = 0, and -D, two threads a
+    // row. Rows of the last chunk at or beyond q_valid among them.
     float* const stats = reinterpret_cast<float*>(buffers + 2 * L::BUF_BYTES);
-    constexpr int kStatRows = kThreads / C8, kStatUnroll = 4;  // rows per pass, passes in flight
+    constexpr int kStatRows = kThreads / 2, kStatUnroll = 2;  // rows per pass, passes in flight
     auto row_stats = [&](int row0) {
-      const int piece = (tid % C8) * 8;
-      vec_t of[kStatUnroll], dof[kStatUnroll];
+      const int half = tid % 2;
+      vec_t of[kStatUnroll][KSTEPS], dof[kStatUnroll][KSTEPS];
       float lse[kStatUnroll];
 #pragma unroll
       for (int u = 0; u < kStatUnroll; ++u) {
-        const int row = row0 + u * kStatRows + tid / C8;
-        lse[u] = -INFINITY;
-        if (row < q_valid) {
-          of[u] = *reinterpret_cast<const vec_t*>(ob + row * p.os[2] + piece);
-          dof[u] = *reinterpret_cast<const vec_t*>(dob + row * p.dos[2] + piece);
-          lse[u] = p.lse[stat0 + row];
-        } else {
-#pragma unroll
-          for (int e = 0; e < 8; ++e) of[u][e] = dof[u][e] = static_cast<T>(0.f);
-        }
+        const int row = row0 + u * kStatRows + tid / 2;
+        lse[u] = row < q_valid ? p.lse[stat0 + row] : -INFINITY;
+        load_owned<T, DP>(ob, p.os[2], row, row < q_valid, p.d, half, of[u]);
+        load_owned<T, DP>(dob, p.dos[2], row, row < q_valid, p.d, half, dof[u]);
       }
 #pragma unroll
       for (int u = 0; u < kStatUnroll; ++u) {
-        const int row = row0 + u * kStatRows + tid / C8;
+        const int row = row0 + u * kStatRows + tid / 2;
         if (row0 + u * kStatRows >= q_valid) break;  // uniform
         float delta = 0.f;
 #pragma unroll
-        for (int e = 0; e < 8; e += 2) delta = dot2(of[u], dof[u], e, delta);
-        delta = group_sum<C8>(delta);
-        if (piece == 0 && row < L::kTiles * kRows) {
+        for (int s = 0; s < KSTEPS; ++s)
+#pragma unroll
+          for (int e = 0; e < 8; ++e) delta = fmaf(static_cast<float>(of[u][s][e]), static_cast<float>(dof[u][s][e]), delta);
+        delta = group_sum<2>(delta);
+        if (half == 0 && row < L::kTiles * kRows) {
           stats[row] = lse[u] > -INFINITY ? lse[u] * 1.4426950408889634f : INFINITY;
-          stats[L::kTiles * kRows + row] = -delta;
+          stats[L::kTiles * kRows + row] = START_D ? -delta : -delta * p.scale;
         }
       }
     };
@@ -923,7 +912,9 @@ void attn_bwd_fused_kernel(const AttnBwdParams p) {
     uint32_t ds_read[2], k_read[2];
 #pragma unroll
     for (int half = 0; half < 2; ++half) {
-      const int key = 8 * g16 + 4 * half + i16 / 4;  // of the tile: one transposed read holds keys 8 g16 + 4 half + 0..3
+      // of the tile: one transposed read holds four keys, in the order in which accumulate_columns has them (the matrix unit adds a
+      // product's terms in theirs)
+      const int key = 16 * (g16 / 2) + 4 * (g16 % 2) + 8 * half + i16 / 4;
       const int piece = 4 * q_half + i16 % 4;        // four queries
       ds_read[half] = lds_offset(ds_image) + static_cast<uint32_t>(key * 64 + ((piece ^ (key / 4)) * 8));
       const int piece16 = 2 * d_col + (i16 % 4) / 2;  // eight features
@@ -953,12 +944,14 @@ void attn_bwd_fused_kernel(const AttnBwdParams p) {
         if (tile >= tiles) return;  // wavefront-uniform
         f32x16 sacc, dpacc;
 #pragma unroll
-        for (int j = 0; j < 16; ++j) sacc[j] = 0.f;
+        for (int j = 0; j < 16; ++j) sacc[j] = dpacc[j] = 0.f;
+        if (START_D) {
 #pragma unroll
-        for (int jq = 0; jq < 4; ++jq) {
-          const f32x4 d4 = *reinterpret_cast<const f32x4*>(&s_delta[jq * 8 + hh * 4]);
+          for (int jq = 0; jq < 4; ++jq) {
+            const f32x4 d4 = *reinterpret_cast<const f32x4*>(&s_delta[jq * 8 + hh * 4]);
 #pragma unroll
-          for (int e = 0; e < 4; ++e) dpacc[jq * 4 + e] = d4[e];
+            for (int e = 0; e < 4; ++e) dpacc[jq * 4 + e] = d4[e];
+          }
         }
 #pragma unroll
         for (int s = 0; s < KSTEPS; ++s) {
@@ -988,6 +981,8 @@ void attn_bwd_fused_kernel(const AttnBwdParams p) {
 #pragma unroll
         for (int jq = 0; jq < 4; ++jq) {
           const f32x4 l4 = *reinterpret_cast<const f32x4*>(&s_lse[jq * 8 + hh * 4]);
+          [[maybe_unused]] f32x4 d4 = {0.f, 0.f, 0.f, 0.f};
+          if (!START_D) d4 = *reinterpret_cast<const f32x4*>(&s_delta[jq * 8 + hh * 4]);
           [[maybe_unused]] u32x4 w4 = {0u, 0u, 0u, 0u};
           if (BITS) w4 = *reinterpret_cast<const u32x4*>(&s_words[tile * kRows + jq * 8 + hh * 4]);
 #pragma unroll
@@ -997,7 +992,7 @@ void attn_bwd_fused_kernel(const AttnBwdParams p) {
             if (BITS)  // all ones where the word has the lane's bit
               prob = __builtin_bit_cast(float, __builtin_bit_cast(uint32_t, prob) & __builtin_amdgcn_sbfe(w4[e], l32, 1));
             pb[j / 8][j % 8] = static_cast<T>(prob);
-            dsb[j / 8][j % 8] = static_cast<T>(prob * (LATE_SCALE ? dpacc[j] : dpacc[j] * p.scale));
+            dsb[j / 8][j % 8] = static_cast<T>(prob * (!START_D ? fmaf(dpacc[j], p.scale, d4[e]) : LATE_SCALE ? dpacc[j] : dpacc[j] * p.scale));
           }
         }
         uint8_t* const ds_tile = ds_image + tile * (kRows * 64) + ds_write;
@@ -1112,11 +1107,11 @@ bool small_offsets(int64_t rows, int64_t stride) {
 //   up to 128 rows (as many workgroups either way):  48 x 32, 256 pairs 8.8 / 6.8, 8192 pairs 58 / 54;  128 x 64, 256 pairs 15.7 / 12.6,
 //   16384 pairs 453 / 330.
 //   256 x 32:  256 pairs 20.0 / 20.5, 512 pairs 27.7 / 24.9, 4096 pairs 165 / 122;  256 x 64:  256 pairs 27.1 / 28.7, 512 pairs 48 / 38,
-//   8192 pairs 517 / 371.
+//   8192 pairs 523 / 387.
 //   More rows of 32 features, four key tiles per wavefront and half the wavefronts in flight. In three blocks of 128 the two kernels
 //   hold their own: 300 rows, 1024 pairs 55 / 54 and 50 / 53 (two draws of the lengths), 2048 pairs 85 / 92, 3584 pairs 169 / 164, 8192
-//   pairs 356 / 321. In four: 400 rows, 1024 pairs 85 / 70, 8192 pairs 688 / 451; 480 rows, 1024 pairs 101 / 101; 512 rows, 1024 pairs 108 /
-//   117 and 102 / 99, 1536 pairs 152 / 148 and 140 / 132, 8192 pairs 814 / 624. Causal, 300 rows, 512 pairs 31 / 28, 512 rows 65 / 54.
+//   pairs 358 / 326. In four: 400 rows, 1024 pairs 85 / 70, 8192 pairs 687 / 462; 480 rows, 1024 pairs 102 / 103; 512 rows, 1024 pairs 108 /
+//   117 and 102 / 99, 1536 pairs 152 / 150 and 139 / 132, 8192 pairs 809 / 638. Causal, 300 rows, 512 pairs 31 / 28, 512 rows 65 / 54.
 // Mask bits, 32 features: as above up to 256 rows (256 rows, 512 pairs 34 / 30, 8192 pairs 368 / 297), but the kernel spills, and where
 // it could gain little, up to 128 rows, it loses once a tensor is more than some 25 MB: 48 rows, 8192 pairs 68 / 65, 12288 pairs 100 / 108;
 // 96 rows, 4096 pairs 52 / 50, 8192 pairs 108 / 133; 128 rows, 3072 pairs 52 / 48, 6144 pairs 97 / 124. Over more rows they stay with the
