@@ -232,8 +232,8 @@ def _check_gradients(got, other, exact, dtype):
         assert error.norm() <= 1.05 * error_other.norm() + 1e-6 * size.norm(), (name, error.norm(), error_other.norm())
 
 
-# One workgroup per (sample, head): one to four key tiles per wavefront, their last ones partly filled, and sizes on both sides of
-# what such a workgroup holds; pairs as many as the dispatch asks for.
+# One workgroup per (sample, head): one to four key tiles per wavefront, their last ones partly filled, sizes and pairs on both sides of
+# what such a workgroup holds and of what the dispatch asks for.
 @pytest.mark.parametrize("rows,keys,dim,batch,heads", [
     (1, 1, 32, 3, 2), (31, 31, 64, 3, 2), (33, 33, 32, 3, 2), (128, 128, 64, 5, 2), (100, 37, 32, 3, 2), (20, 128, 64, 3, 2),
     (129, 129, 32, 64, 8), (256, 256, 32, 64, 8), (257, 257, 32, 128, 8), (490, 490, 32, 128, 8), (512, 512, 32, 128, 8),
