@@ -740,10 +740,14 @@ struct Mfma16<f16_t> {
 // owns a key, so P and dS come out of the first products as the B operands of dV and dK; dQ contracts over the keys
 // instead: the dS tiles of all wavefronts meet in LDS ([key][query], 16 bits as every operand) and each wavefront forms
 // its own 16 queries x 16 features (DP = 64: twice) of dQ over all key tiles, so dQ, too, has one writer per element and
-// a fixed order. Every sum is formed in the order of the two kernels and every value rounded as there, so that without a mask the
-// gradients are theirs to the bit, whichever route a batch's size takes. (D added up over eight lanes a row, the start value of dP, and
-// 1 / sqrt(d) at the end save three instructions per pair, 1024 x 8 x 512 x 32 604 instead of 638 us, 2048 x 4 x 256 x 64 371 instead of
-// 383, but move a quarter of dQ and dK at d = 32 by a rounding, which a few layers make 0.2 % of every gradient.)
+// a fixed order. Every sum is formed in the order of the two kernels and every value rounded as there, so that the
+// gradients are theirs to the bit, whichever route a batch's size takes. (Without a mask, D added up over eight lanes a row, the start
+// value of dP, and 1 / sqrt(d) at the end save three instructions per pair, 1024 x 8 x 512 x 32 604 instead of 638 us, 2048 x 4 x 256 x 64
+// 371 instead of 383, but move a quarter of dQ and dK at d = 32 by a rounding, which a few layers make 0.2 % of every gradient.)
+// Under mask bits the two kernels round the dS of dQ and that of dK differently (START_D there), so that dP is formed twice, one behind the
+// other. Two wavefronts a SIMD instead of three leave the registers for it: with three, 16 to 36 of them are spilled (256 rows, 8192 pairs
+// of 32 features 340 instead of 290 us; 64 rows of 64 features 192 instead of 123). One dP and the scale at the end moved dK, at d = 64 dQ,
+// by roundings: 312 and 133 us there, with three wavefronts.
 template <int DP, int NT, bool BITS>
 struct FusedLayout {
   static constexpr int kRows = 32;                                     // streamed queries per step
@@ -752,12 +756,14 @@ struct FusedLayout {
   static constexpr int K_BYTES = kTiles * TILE_BYTES, DS_BYTES = kTiles * kRows * 64;
   static constexpr int WORD_BYTES = BITS ? kTiles * kRows * 4 : 0;      // [tile][row]
   static constexpr int BUF_BYTES = 2 * TILE_BYTES + WORD_BYTES;         // Q, dO, words
-  static constexpr int STAT_BYTES = 2 * kTiles * kRows * 4;             // log-sum-exp and -D of every query
+  static constexpr int STAT_BYTES = (BITS ? 3 : 2) * kTiles * kRows * 4;  // log-sum-exp and -D / sqrt(d) of every query; -D
   static constexpr int BYTES = K_BYTES + DS_BYTES + 2 * BUF_BYTES + STAT_BYTES;
+  static constexpr int kWavesPerSimd = NT * DP == 128 || BITS ? 2 : 3;
 };
 
 template <typename T, int DP, int NT, int MODE, bool COMPACT>
-__global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(NT * DP == 128 ? 2 : 3, NT * DP == 128 ? 2 : 3)))
+__global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(FusedLayout<DP, NT, MODE == kMaskBits>::kWavesPerSimd,
+                                                                          FusedLayout<DP, NT, MODE == kMaskBits>::kWavesPerSimd)))
 void attn_bwd_fused_kernel(const AttnBwdParams p) {
   constexpr bool BITS = MODE == kMaskBits;
   static_assert(MODE == kMaskNone || BITS, "the other masks are read per element by the two kernels above");
@@ -767,10 +773,7 @@ void attn_bwd_fused_kernel(const AttnBwdParams p) {
   constexpr int KSTEPS = DP / 16, MB = DP / 32, C8 = DP / 8, kRows = L::kRows, ROWB = L::ROWB, TILE_BYTES = L::TILE_BYTES;
   constexpr int kWaves = L::kWaves;
   [[maybe_unused]] constexpr int kWords = L::kTiles * kRows;
-  // With mask bits, where the kernel spills, the products dP start from -D, and a scale that is a power of two multiplies dK and dQ at the
-  // end, the same bits in bf16's range: 512 x 8 x 250 x 32 167 instead of 186 us. (The two kernels start dK's products so and round its dS
-  // before the scale: dQ and dK are each within a rounding of theirs, no further from float64.)
-  constexpr bool START_D = BITS, LATE_SCALE = BITS && DP == 64 && std::is_same<T, bf16_t>::value;
+  constexpr bool LATE_SCALE = BITS && std::is_same<T, bf16_t>::value;
   __shared__ __attribute__((aligned(1024))) uint8_t smem[L::BYTES];
   uint8_t* const k_image = smem;
   uint8_t* const ds_image = smem + L::K_BYTES;
@@ -848,8 +851,8 @@ void attn_bwd_fused_kernel(const AttnBwdParams p) {
         }
       }
     };
-    // The statistics of all queries: base-2 log-sum-exp, +inf for a row that carries nothing: exp2(x - inf) = 0, and -D, two threads a
-    // row. Rows of the last chunk at or beyond q_valid among them.
+    // The statistics of all queries: base-2 log-sum-exp, +inf for a row that carries nothing: exp2(x - inf) = 0, and -D / sqrt(d) (with
+    // mask bits -D, too), two threads a row. Rows of the last chunk at or beyond q_valid among them.
     float* const stats = reinterpret_cast<float*>(buffers + 2 * L::BUF_BYTES);
     constexpr int kStatRows = kThreads / 2, kStatUnroll = 2;  // rows per pass, passes in flight
     auto row_stats = [&](int row0) {
@@ -875,7 +878,8 @@ void attn_bwd_fused_kernel(const AttnBwdParams p) {
         delta = group_sum<2>(delta);
         if (half == 0 && row < L::kTiles * kRows) {
           stats[row] = lse[u] > -INFINITY ? lse[u] * 1.4426950408889634f : INFINITY;
-          stats[L::kTiles * kRows + row] = START_D ? -delta : -delta * p.scale;
+          stats[L::kTiles * kRows + row] = -delta * p.scale;
+          if (BITS) stats[2 * L::kTiles * kRows + row] = -delta;
         }
       }
     };
@@ -945,14 +949,6 @@ void attn_bwd_fused_kernel(const AttnBwdParams p) {
         f32x16 sacc, dpacc;
 #pragma unroll
         for (int j = 0; j < 16; ++j) sacc[j] = dpacc[j] = 0.f;
-        if (START_D) {
-#pragma unroll
-          for (int jq = 0; jq < 4; ++jq) {
-            const f32x4 d4 = *reinterpret_cast<const f32x4*>(&s_delta[jq * 8 + hh * 4]);
-#pragma unroll
-            for (int e = 0; e < 4; ++e) dpacc[jq * 4 + e] = d4[e];
-          }
-        }
 #pragma unroll
         for (int s = 0; s < KSTEPS; ++s) {
           const uint32_t off = row_off ^ (s * 32);
@@ -981,8 +977,7 @@ void attn_bwd_fused_kernel(const AttnBwdParams p) {
 #pragma unroll
         for (int jq = 0; jq < 4; ++jq) {
           const f32x4 l4 = *reinterpret_cast<const f32x4*>(&s_lse[jq * 8 + hh * 4]);
-          [[maybe_unused]] f32x4 d4 = {0.f, 0.f, 0.f, 0.f};
-          if (!START_D) d4 = *reinterpret_cast<const f32x4*>(&s_delta[jq * 8 + hh * 4]);
+          const f32x4 d4 = *reinterpret_cast<const f32x4*>(&s_delta[jq * 8 + hh * 4]);
           [[maybe_unused]] u32x4 w4 = {0u, 0u, 0u, 0u};
           if (BITS) w4 = *reinterpret_cast<const u32x4*>(&s_words[tile * kRows + jq * 8 + hh * 4]);
 #pragma unroll
@@ -992,7 +987,8 @@ void attn_bwd_fused_kernel(const AttnBwdParams p) {
             if (BITS)  // all ones where the word has the lane's bit
               prob = __builtin_bit_cast(float, __builtin_bit_cast(uint32_t, prob) & __builtin_amdgcn_sbfe(w4[e], l32, 1));
             pb[j / 8][j % 8] = static_cast<T>(prob);
-            dsb[j / 8][j % 8] = static_cast<T>(prob * (!START_D ? fmaf(dpacc[j], p.scale, d4[e]) : LATE_SCALE ? dpacc[j] : dpacc[j] * p.scale));
+            dsb[j / 8][j % 8] = static_cast<T>(prob * fmaf(dpacc[j], p.scale, d4[e]));
+            if (BITS) sacc[j] = prob;
           }
         }
         uint8_t* const ds_tile = ds_image + tile * (kRows * 64) + ds_write;
@@ -1002,6 +998,21 @@ void attn_bwd_fused_kernel(const AttnBwdParams p) {
 #pragma unroll
           for (int e = 0; e < 4; ++e) quad[e] = dsb[jq / 2][(jq % 2) * 4 + e];
           *reinterpret_cast<vec4_t*>(ds_tile + ((2 * jq + hh) ^ (l32 / 4)) * 8) = quad;
+        }
+        if constexpr (BITS) {  // dK's dS: the products start from -D, 1 / sqrt(d) comes at the end (fp16: before the rounding)
+#pragma unroll
+          for (int jq = 0; jq < 4; ++jq) {
+            const f32x4 d4 = *reinterpret_cast<const f32x4*>(&s_delta[L::kTiles * kRows + jq * 8 + hh * 4]);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) dpacc[jq * 4 + e] = d4[e];
+          }
+#pragma unroll
+          for (int s = 0; s < KSTEPS; ++s) {
+            const vec_t da = *reinterpret_cast<const vec_t*>(chunk + TILE_BYTES + (row_off ^ (s * 32)));
+            dpacc = Mfma32<T>::run(da, vf[t][s], dpacc);
+          }
+#pragma unroll
+          for (int j = 0; j < 16; ++j) dsb[j / 8][j % 8] = static_cast<T>(sacc[j] * (LATE_SCALE ? dpacc[j] : dpacc[j] * p.scale));
         }
         accumulate_columns2<T, DP, 0>(dvacc[t], pb, col_addr + TILE_BYTES, dkacc[t], dsb, col_addr);
       });
@@ -1053,7 +1064,7 @@ void attn_bwd_fused_kernel(const AttnBwdParams p) {
         for (int m = 0; m < MB; ++m) {
           vec4_t out;
 #pragma unroll
-          for (int e = 0; e < 4; ++e) out[e] = static_cast<T>(LATE_SCALE ? dqacc[m][e] * p.scale : dqacc[m][e]);
+          for (int e = 0; e < 4; ++e) out[e] = static_cast<T>(dqacc[m][e]);
           *reinterpret_cast<vec4_t*>(dqb + q_row * p.dqs[2] + 32 * m + 16 * d_col + 4 * g16) = out;
         }
       }
@@ -1112,12 +1123,12 @@ bool small_offsets(int64_t rows, int64_t stride) {
 //   hold their own: 300 rows, 1024 pairs 55 / 54 and 50 / 53 (two draws of the lengths), 2048 pairs 85 / 92, 3584 pairs 169 / 164, 8192
 //   pairs 358 / 326. In four: 400 rows, 1024 pairs 85 / 70, 8192 pairs 687 / 462; 480 rows, 1024 pairs 102 / 103; 512 rows, 1024 pairs 108 /
 //   117 and 102 / 99, 1536 pairs 152 / 150 and 139 / 132, 8192 pairs 809 / 638. Causal, 300 rows, 512 pairs 31 / 28, 512 rows 65 / 54.
-// Mask bits, 32 features: as above up to 256 rows (256 rows, 512 pairs 34 / 30, 8192 pairs 368 / 297), but the kernel spills, and where
-// it could gain little, up to 128 rows, it loses once a tensor is more than some 25 MB: 48 rows, 8192 pairs 68 / 65, 12288 pairs 100 / 108;
-// 96 rows, 4096 pairs 52 / 50, 8192 pairs 108 / 133; 128 rows, 3072 pairs 52 / 48, 6144 pairs 97 / 124. Over more rows they stay with the
-// two kernels: the words' registers are the ones that the four key tiles of a wavefront need. 300 rows, 1024 pairs 67 / 74, 4096 pairs 239 /
-// 274; 350 rows, 4096 pairs 280 / 319. (It would gain from 400 rows and 2048 pairs on: 403 rows, 1024 pairs 117 / 116, 4096 pairs 436 / 360;
-// 512 rows, 1024 pairs 145 / 152, 4096 pairs 535 / 471.)
+// Mask bits: 64 features, 64 rows, 256 pairs 12.6 / 8.7, 8192 pairs 175 / 123, 256 rows, 512 pairs 59 / 45, 8192 pairs 674 / 534; 32 features,
+// 160 rows, 512 pairs 24.4 / 19.8, 256 rows, 512 pairs 34 / 31, 8192 pairs 370 / 290. Up to 128 rows of 32 features there is little to gain,
+// and the second dP loses it where the workgroups are several to a compute unit: 64 rows, 512 pairs 10.8 / 8.4, 1536 pairs 20.2 / 20.1, 3072
+// pairs 32.6 / 35.5; 96 rows, 2048 pairs 31.2 / 30.1, 4096 pairs 52 / 55; 128 rows, 2048 pairs 36.8 / 35.2. Over 256 rows of 32 features
+// they stay with the two kernels: the words' registers are the ones that the four key tiles of a wavefront need (already with one dP, 300
+// rows, 1024 pairs 67 / 74, 4096 pairs 239 / 274; 403 rows 117 / 116, 436 / 360).
 template <typename T, int DP, int MODE, bool COMPACT>
 bool launch_bwd_fused(AttnBwdParams p, hipStream_t s) {
   constexpr int kSmall = 64 / DP, kLarge = 128 / DP;  // key tiles per wavefront
@@ -1127,7 +1138,7 @@ bool launch_bwd_fused(AttnBwdParams p, hipStream_t s) {
   int64_t enough = rows <= kOwn ? 1 : 512;
   if (DP == 32 && rows > kRowsSmall && !p.causal) enough = rows <= 3 * kOwn ? 3584 : (rows <= 480 ? 1024 : 1536);
   if (rows > kRowsLarge || pairs < enough) return false;
-  if (DP == 32 && MODE == kMaskBits && rows <= kOwn && rows * pairs > 400000) return false;
+  if (DP == 32 && MODE == kMaskBits && rows <= kOwn && pairs > (rows <= 64 ? 1536 : 2048)) return false;
   if (!small_offsets(p.Tq, p.qs[2]) || !small_offsets(p.Tq, p.dos[2]) || !small_offsets(p.Tk, p.ks[2])) return false;
   p.nblk = 1;
   p.total = static_cast<uint32_t>(pairs);

@@ -291,13 +291,10 @@ def test_mask_bits_backward_with_all_keys_in_one_workgroup(device, rows, dim, ba
     _check_gradients(got, dense, exact, torch.bfloat16)
 
 
-@pytest.mark.parametrize("rows,dim,batch,heads,bits", [(128, 32, 8, 4, False), (200, 32, 64, 8, False), (400, 32, 128, 8, False),
-                                                       (250, 64, 128, 4, False), (77, 64, 8, 4, False), (200, 32, 64, 8, True)])
-def test_one_workgroup_rounds_as_the_two_kernels_do(device, rows, dim, batch, heads, bits):
-    """Without a mask every sum has the order and every value the rounding of the two kernels: the same bits, so that a gradient does not
-    depend on how many samples a batch has. With mask bits dP starts from -D: against the same mask as bytes the two differ where
-    float32 sums fall on different sides of a rounding boundary, about one dS in 2^12, by 2^-8 of it, 2^-14 of a gradient's norm.
-    (Rounded before a scale that is no power of two they are 2^-8.3 apart.)"""
+@pytest.mark.parametrize("rows,dim,batch,heads", [(128, 32, 8, 4), (200, 32, 64, 8), (400, 32, 128, 8), (250, 64, 128, 4), (77, 64, 8, 4)])
+def test_one_workgroup_rounds_as_the_two_kernels_do(device, rows, dim, batch, heads):
+    """Every sum has the order and every value the rounding of the two kernels: the same bits, so that a gradient does not depend on how
+    many samples a batch has."""
     g = torch.Generator(device=device).manual_seed(rows)
     q, k, v, grad_out = (torch.randn(batch, heads, rows, dim, generator=g, device=device).to(torch.bfloat16) for _ in range(4))
     lengths = torch.randint(1, rows + 1, (batch,), generator=g, device=device, dtype=torch.int32)
@@ -305,17 +302,37 @@ def test_one_workgroup_rounds_as_the_two_kernels_do(device, rows, dim, batch, he
     inside = index < lengths[:, None]
     lse, p = _log_sum_exp(q, k, (inside[:, None, :] & inside[:, :, None])[:, None])
     args = (q, k, v, (p @ v.double()).to(torch.bfloat16), grad_out, lse.float().contiguous(), lengths, False, True)
-    if bits:
-        words = torch.full((batch, rows, (rows + 31) // 32), -1, dtype=torch.int32, device=device)
-        got = _native_backward(*args, words=words)
-        other = _native_backward(*args, visible=torch.ones(batch, rows, rows, dtype=torch.uint8, device=device))
-    else:
-        got, other = _native_backward(*args), _native_backward(*args, staged=True)
-    for name, a, b in zip(("dq", "dk", "dv"), got, other):
-        if bits:
-            assert (a.double() - b.double()).norm() <= 2.0 ** -12 * b.double().norm(), name
-        else:
-            assert torch.equal(a, b), name
+    for name, a, b in zip(("dq", "dk", "dv"), _native_backward(*args), _native_backward(*args, staged=True)):
+        assert torch.equal(a, b), name
+
+
+@pytest.mark.parametrize("dtype,rows,dim,batch,heads,part", [
+    (torch.bfloat16, 129, 32, 64, 8, 63), (torch.float16, 256, 32, 64, 8, 21), (torch.bfloat16, 250, 64, 130, 4, 65),
+    (torch.float16, 160, 64, 130, 4, 65), (torch.bfloat16, 64, 32, 388, 4, 194), (torch.bfloat16, 97, 32, 260, 8, 52)])
+@pytest.mark.parametrize("valid", [False, True])
+def test_mask_bits_backward_of_a_batch_and_of_its_parts(device, dtype, rows, dim, batch, heads, part, valid):
+    """On one side of the dispatch's lines a batch, on the other its parts: a sample's gradients have the same bits."""
+    g = torch.Generator(device=device).manual_seed(rows)
+    q, k, v, grad_out = (torch.randn(batch, heads, rows, dim, generator=g, device=device).to(dtype) for _ in range(4))
+    lengths = torch.randint(1, rows + 1, (batch,), generator=g, device=device, dtype=torch.int32)
+    n_words = (rows + 31) // 32
+    words, key_valid = (torch.randint(-2 ** 31, 2 ** 31, (batch, n, n_words), generator=g, device=device).to(torch.int32) for n in (rows, 1))
+    on = lambda t: ((t.unsqueeze(-1) >> torch.arange(32, device=device)) & 1).flatten(-2)[..., :rows] != 0  # noqa: E731
+    inside = torch.arange(rows, device=device) < lengths[:, None]
+    visible = on(words) & inside[:, None, :] & inside[:, :, None]
+    if valid:
+        visible = visible & on(key_valid)
+    lse, p = _log_sum_exp(q, k, visible[:, None])
+    out, lse = (p @ v.double()).to(dtype), lse.float().contiguous()
+
+    def gradients(s):
+        return _native_backward(q[s], k[s], v[s], out[s], grad_out[s], lse[s], lengths[s], False, True, words=words[s],
+                                key_valid=key_valid[s] if valid else None)
+
+    whole = gradients(slice(0, batch))
+    parts = [gradients(slice(i, i + part)) for i in range(0, batch, part)]
+    for name, a, *pieces in zip(("dq", "dk", "dv"), whole, *parts):
+        assert torch.equal(a, torch.cat(pieces)), name
 
 
 @pytest.mark.parametrize("value", [float("inf"), float("nan")])
