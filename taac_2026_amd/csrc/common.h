@@ -47,7 +47,7 @@ bool ffn_act_fold_supported(int32_t D, int32_t F);
 bool ffn_few_rows(int64_t M, int32_t D);
 // Workgroups that share the hidden units of a token tile when the gated feed-forward over at most M rows runs as the few-token
 // kernel and is given the scratch memory for it (ffn_split_bytes; the counters behind the partials zeroed once): a power of
-// two as long as the tiles leave that many compute units idle and every wavefront has two chunks of hidden units. 1 otherwise.
+// two as long as the tiles leave that many compute units idle. 1 otherwise.
 int ffn_splits(int64_t M, int32_t D, int32_t F);
 int64_t ffn_split_bytes(int64_t M, int32_t D, int32_t F);
 // RMSNorm + q | k | v projection with the query / key epilogue (ffn.hip; the arguments of taac_norm_linear_qk_fwd with

@@ -221,9 +221,11 @@ struct SharedPartials {
 // splits > 1 (see TsParams): for batches that leave most of the chip idle even so, the hidden units of a tile are also divided over
 // workgroups, eight at most (one request of 512 positions, eight splits, with the requests below ordered by need: the whole
 // 4-block call 164 -> 140 us; fences instead of the write-through accesses: 156; those accesses 16 bytes wide instead
-// of 8: 128 -> 119). Every wavefront keeps two 16-unit chunks: one alone has the same latency chains in front of and behind it (at most
-// 8 / 4 / 2 splits, one request of 512 positions, D = 256: F = 512 137 / 132 / 134 us, F = 1024 142 / 141 / 150, F = 2048 156 / 161 /
-// 183; D = 128: F = 512 99 / 96 / 95, F = 1024 102 / 100 / 104; sixteen, with 8-byte accesses, F = 1024 160 against 140 for eight).
+// of 8: 128 -> 119). Sixteen lose where tiles and F admit them: a wavefront then has one 16-unit chunk behind the same latency
+// chains (with 8-byte accesses, F = 1024 160 against 140 us for eight, F = 2048 169 against 151). At F = 512 eight leave it one chunk, too,
+// and cost 4 % (at most 8 / 4 / 2 splits, one request of 512 positions, D = 256: F = 512 137 / 132 / 134 us, F = 1024 142 / 141 / 150,
+// F = 2048 156 / 161 / 183; D = 128: F = 512 99 / 96 / 95, F = 1024 102 / 100 / 104); another number would add the units in another
+// order and move every output by roundings.
 // LDS: [4 partials of 32 x D floats][x1 (32 padded rows of D bf16)][first-layer bias 2F][4 x 32 row sums]
 // ------------------------------------------------------------------------------------------------------------------
 template <int D, bool OUTP, bool FOLD>
@@ -527,7 +529,7 @@ int ffn_splits(int64_t M, int32_t D, int32_t F) {
   const int cus = compute_units();
   int splits = 1;
   if (ffn_few_rows(M, D))
-    while (splits < 8 && 2 * splits * tiles <= cus && 2 * splits * 8 * kHU <= F) splits *= 2;  // two chunks for each wavefront
+    while (splits < 8 && 2 * splits * tiles <= cus && 2 * splits * 4 * kHU <= F) splits *= 2;
   return splits;
 }
 

@@ -107,7 +107,7 @@ def test_feed_forward_matches_the_persistent_kernel(device, test_hooks, m, d, f,
                                                                (32, 120, 256, 8, 512), (20, 120, 128, 4, 256), (7, 61, 256, 8, 128),
                                                                (2, 300, 256, 8, 512), (7, 61, 256, 8, 384), (1, 20, 128, 4, 1024)])
 def test_backbone_with_hidden_units_divided_over_workgroups(device, test_hooks, batch, sequence, d_model, heads, d_ff):
-    """Batches small enough for 2 to 8 workgroups per token tile (as many as leave a wavefront two chunks of hidden units), against the persistent kernels and from run to run (the
+    """Batches small enough for 2 to 8 workgroups per token tile, against the persistent kernels and from run to run (the
     partial sums are added in a fixed order, whoever arrives last). Bound of the hidden state: roundings of the blocks'
     outputs flip by one bf16 step (2**-8 relative) and travel through the following blocks."""
     inputs = workloads.backbone_inputs(batch=batch, n_feature_tokens=8, n_sequence_tokens=sequence, d_model=d_model,
