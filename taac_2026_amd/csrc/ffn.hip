@@ -1933,13 +1933,14 @@ int attn_out_ffn_count(const char* name, const void* attn, const void* out_bias,
                    split_scratch, count, x1_out, rstd_out);
 }
 
-// Whether the gated feed-forward over at most M rows of D features runs as the few-token kernel: as long as its 32-token
-// workgroups are at most two rounds of the chip. M counts padded rows; with half of them valid (9 648 rows, 6 100 tokens,
-// training) 26.9 / 64.8 us. Measured with the out projection in front, launches back to back, few-token /
-// persistent kernel, us: D = 256, F = 1024 - 512 rows 21.5 / 49.9, 8192 27.8 / 55.6, 16384 53.8 / 57.7, 24576 72.5 / 58.2;
-// F = 512 - 8192 18.8 / 34.7, 16384 34.4 / 36.4; D = 128 (two workgroups per compute unit), F = 512 - 512 rows 9.2 / 19.5,
-// 16384 16.8 / 21.9, 24576 23.0 / 22.2.
-bool ffn_few_rows(int64_t M, int32_t D) { return test_max_workgroups() == 0 && M * D <= 16384 * 256; }
+// Whether the gated feed-forward over at most M rows of D features runs as the few-token kernel. M counts padded rows. With the out
+// projection in front, one launch, few-token / persistent kernel, us, all rows valid and 55 % of them: D = 256, F = 1024 - 512 rows
+// 17.6 / 50.9, 8103 23.0 / 56.2 and 19.6 / 52.4, 16384 32.4 / 57.6 and 26.1 / 52.2, 24576 54.1 / 59.0 and 29.2 / 55.8, 32768 60.9 /
+// 62.6 and 55.2 / 54.5, 49152 89.6 / 89.1 and 55.3 / 57.6, 65536 117 / 103 and 86.4 / 81.4; F = 512 - 24576 37.6 / 39.6 and 20.1 / 35.3,
+// 32768 40.8 / 41.0 and 36.3 / 36.1, 49152 58.9 / 56.1 and 37.0 / 37.8. D = 128, F = 512 - 512 8.2 / 20.2, 16384 14.4 / 22.2 and 12.7 /
+// 21.3, 49152 30.8 / 33.1 and 19.2 / 23.7, 65536 37.8 / 35.7 and 27.9 / 30.4; F = 256 - 49152 23.3 / 23.7 and 15.5 / 17.4, 65536 29.0 /
+// 25.8 and 21.6 / 21.4.
+bool ffn_few_rows(int64_t M, int32_t D) { return test_max_workgroups() == 0 && M <= (D == 256 ? 24576 : 49152); }
 
 // Whether a projection over at most M rows of D features runs as the few-token kernel. Measured for q | k | v (launches
 // back to back, few-token / persistent kernel, us): D = 256 - 512 rows 6.0 / 13.6, 4096 9.9 / 14.1, 8192 14.4 / 15.6,

@@ -190,8 +190,8 @@ __global__ __launch_bounds__(D, 2) void norm_linear_small_kernel(const TsParams 
 // Data that other workgroups of the same launch read: accesses at the scope of the whole chip, which go through the L2 of the die
 // to the memory all dies share. (Ordinary stores with a fence behind them write back and drop everything the die's L2 holds:
 // 8 us per launch.)
-// Sixteen bytes per lane and access: as atomic accesses, eight bytes at most, twice as many requests leave the compute unit and the
-// last workgroup of a tile takes 5 us for its 256 KB (512 tokens, D = 256, F = 1024, eight splits: 19.7 -> 17.0 us for the kernel).
+// Sixteen bytes per lane and access: as atomic accesses, eight bytes at most, twice as many requests leave the compute unit (eight
+// partials of 32 KB: 2.7 us more).
 // Ordering is the caller's: a wait and a barrier in front of the count that publishes the stores, a barrier behind it for the loads.
 constexpr int kThroughL2 = 16;  // the sc1 bit of a buffer access: coherent at the scope of the chip
 struct SharedPartials {
@@ -208,94 +208,149 @@ struct SharedPartials {
 
 // ------------------------------------------------------------------------------------------------------------------
 // The feed-forward half for few tokens: [out projection + residual ->] RMSNorm -> up -> SiLU-gate -> down -> + residual of
-// 32 tokens per workgroup (the products, blobs and roundings of swiglu_ffn_kernel). Four wavefronts share the tokens and divide
-// the HIDDEN units: wavefront w takes the 16-unit chunks w, w + 4, ...; each holds a [D, 32] partial of the down projection
-// in its accumulators, and the four partials meet once, in LDS, where every wavefront adds up its share of the features in a
-// fixed order. The projection in front is divided by output features; its result reaches the other wavefronts through LDS.
-// A wavefront is alone on its SIMD and reads its fragments from L2 through a ring as deep as a chunk (24 KB in flight at
-// D = 256, 96 KB per compute unit).
-// Bound: the 1.6 MB of weights a compute unit pulls from L2 for its 32 tokens (0.7 us per chunk and wavefront, 64 bytes per
-// clock of the compute unit: 11 us) behind and in front of which lie 9.5 us of latency chains; the persistent kernel has one
-// or two of its eight wavefronts at work there and takes 50 us whatever the number of tokens (512 tokens, D = 256, F = 1024:
-// 49.9 -> 21.5 us; 8192 tokens: 55.6 -> 27.8; its line is at ffn_few_rows).
+// 32 or 64 tokens per workgroup (the products, blobs and roundings of swiglu_ffn_kernel). The wavefronts, one per 32 features, share
+// the tokens. The projection and the down projection are divided by OUTPUT features, the up projection by HIDDEN units; the
+// normalised tokens and the hidden state, as operand fragments, meet in LDS. (With the down projection divided by hidden units, too,
+// every wavefront holds a partial of all features: four times the accumulators, 128 KB of partials through LDS, and one wavefront
+// per SIMD, whose instructions then stand between its products.)
+//
+// A wavefront's weights are one stream of fragments, L2 -> registers, through a ring of KS fragments (16 KB in flight at
+// D = 256, 128 KB per workgroup): projection, then the up fragments of its 16-unit chunks, then the down fragments of its
+// features; a slot is requested again as soon as its product is issued.
+// Bound, one tile: the weights a compute unit pulls from L2 at 64 bytes a clock (1.6 MB at D = 256, F = 1024: 24 000 of the kernel's
+// 38 000 cycles; the rest is the chain row index -> rows -> projection -> norm in front, and the stores). Two tiles halve that and are
+// bound by the products and the activation, which add: 1.7 us per 1000 tokens at D = 256, F = 1024.
+// One launch, us, this form / the one with partials of all features: D = 256, F = 1024 - 4096 rows 19.9 / 25.1, 8103 rows 23.0 /
+// 27.8, 16384 rows 32.4 / 53.8, 9648 rows, 6100 valid 20.4 / 26.9; F = 512 - 8103 rows 15.1 / 18.8; D = 128, F = 512 - 512 rows 8.2 / 9.2.
 // splits > 1 (see TsParams): for batches that leave most of the chip idle even so, the hidden units of a tile are also divided over
-// workgroups, eight at most (one request of 512 positions, eight splits, with the requests below ordered by need: the whole
-// 4-block call 164 -> 140 us; fences instead of the write-through accesses: 156; those accesses 16 bytes wide instead
-// of 8: 128 -> 119). Sixteen lose where tiles and F admit them: a wavefront then has one 16-unit chunk behind the same latency
-// chains (with 8-byte accesses, F = 1024 160 against 140 us for eight, F = 2048 169 against 151). At F = 512 eight leave it one chunk, too,
-// and cost 4 % (at most 8 / 4 / 2 splits, one request of 512 positions, D = 256: F = 512 137 / 132 / 134 us, F = 1024 142 / 141 / 150,
-// F = 2048 156 / 161 / 183; D = 128: F = 512 99 / 96 / 95, F = 1024 102 / 100 / 104); another number would add the units in another
-// order and move every output by roundings.
-// LDS: [4 partials of 32 x D floats][x1 (32 padded rows of D bf16)][first-layer bias 2F][4 x 32 row sums]
+// workgroups; the exchange costs 4 - 5 us, and the rule is at ffn_splits.
 // ------------------------------------------------------------------------------------------------------------------
-template <int D, bool OUTP, bool FOLD>
-__global__ __launch_bounds__(4 * kWave, 1) void swiglu_ffn_small_kernel(const TsParams p) {
-  constexpr int NW = 4;
+constexpr int kSlab = 64;  // 16-unit chunks whose hidden state lies in LDS at a time (F = 1024 in one piece)
+
+// LDS of the kernel for workgroups of TT token tiles and `chunks` chunks of hidden units: first the normalised rows of a tile that are
+// kept (one tile: read once, but the hidden state need not wait for it; two tiles, D = 256: the second one's fragments, for which there
+// are no registers), then the tokens as they come in (and the other normalised rows), whose place the hidden state takes. The
+// biases and sums come behind.
+__host__ __device__ constexpr int small_kept_bytes(int D, int TT) { return TT == 1 || D == 256 ? 32 * (D * 2 + 16) : 0; }
+__host__ __device__ constexpr int small_tile_bytes(int D, int TT, int chunks) {
+  const int rows = 32 * (D * 2 + 16), hidden = TT * (chunks < kSlab ? chunks : kSlab) * kFrag;
+  const int tokens = 2 * TT * rows - small_kept_bytes(D, TT);
+  return small_kept_bytes(D, TT) + (hidden > tokens ? hidden : tokens);
+}
+
+// Workgroups that a compute unit holds: of the one-tile form, and of the form that takes one or two tiles.
+__host__ __device__ constexpr int small_one_residents(int D) { return D == 256 ? 1 : 3; }
+__host__ __device__ constexpr int small_pair_residents(int D) { return D == 256 ? 1 : 2; }
+
+// Groups of one chunk per wavefront that a workgroup of the kernel takes at most.
+__host__ __device__ constexpr int small_groups(int D, int F, int splits) {
+  return ((F / kHU + D / 32 - 1) / (D / 32) + splits - 1) / splits;
+}
+
+// What a workgroup asks for before it knows the number of tokens: the row index of its tiles and the projection's weights.
+template <int D, int TT>
+struct SmallTokens {
+  static constexpr int kPieces = D / 8;                             // 16-byte pieces of a row
+  static constexpr int kStep = D / 32 * kWave / kPieces;            // rows that the threads load a piece each of
+  static constexpr int kPasses = 32 * TT / kStep;
+  SmallRows<kPasses> in;  // rows of x, by pieces
+  SmallRows<TT> out;      // rows of residual / out: token l32 of each tile
+  __device__ __forceinline__ void request(const TsParams& p, int64_t tok0, int tid, int l32) {
+    in.request(p, p.x_rows != nullptr ? p.x_rows : p.rows, [&](int i) { return tok0 + i * kStep + tid / kPieces; });
+    out.request(p, p.rows, [&](int t) { return tok0 + t * 32 + l32; });
+  }
+};
+
+template <int D, int TT, bool OUTP, bool FOLD, bool SLABS>
+__device__ __forceinline__ void ffn_small_tile(const TsParams& p, uint8_t* smem, int64_t count, int tile, int split,
+                                               SmallTokens<D, TT>& tokens, bf16x8 (&ring)[D / 16]) {
   constexpr int KS = D / 16, MB = D / 32;
+  constexpr int NW = MB;                      // wavefronts
   constexpr int CFRAG = KS + MB;
-  constexpr int MBW = MB / NW;              // 32-feature blocks a wavefront projects in front and adds up behind
-  constexpr int kRow = D * 2 + 16;          // bytes per row of the x1 tile
-  constexpr int kPart = MB * 4 * kWave * 16;  // bytes of one partial
-  extern __shared__ __attribute__((aligned(1024))) uint8_t smem[];
-  uint8_t* x1_lds = smem + NW * kPart;
-  bf16_t* bias_lds = reinterpret_cast<bf16_t*>(x1_lds + 32 * kRow);
-  float* sums = reinterpret_cast<float*>(bias_lds + 2 * p.F);  // [NW][32]
+  constexpr int kRow = D * 2 + 16;            // bytes per row of a token tile
+  constexpr int kPart = MB * 4 * kWave * 16;  // bytes of one split's partial
+  constexpr int XT = D == 256 ? 1 : TT;       // tiles whose normalised tokens stay in registers
+  constexpr int kKept = small_kept_bytes(D, TT);
+  static_assert(KS == 2 * NW, "a ring holds the down fragments of two groups of chunks");
+  static_assert(TT == 1 || !SLABS, "two tiles: one slab");
+  const int F = p.F;
+  const int nchunks = F / kHU;
+  const int splits = TT == 1 && p.splits > 1 ? p.splits : 1;
+  const int shift = __builtin_ctz(splits);  // a power of two (ffn_splits)
+  const int groups = ((nchunks + NW - 1) / NW + splits - 1) >> shift;
+  // normalised rows of a tile; rows as they come in, then between the halves; hidden state
+  auto normed_lds = [&](int t) {
+    if constexpr (TT == 1) return smem;
+    if (kKept > 0) return t == 1 ? smem : smem + kKept;
+    return smem + t * 32 * kRow;
+  };
+  uint8_t* x_lds = smem + (TT == 1 ? kKept : kKept + (kKept > 0 ? 1 : 2) * 32 * kRow);
+  uint8_t* hidden_lds = smem + kKept;
+  float* bias_lds = reinterpret_cast<float*>(smem + small_tile_bytes(D, TT, groups * NW));
+  bf16_t* end_lds = reinterpret_cast<bf16_t*>(bias_lds + 2 * F);  // down-projection bias, readout weight
+  float* sums = reinterpret_cast<float*>(end_lds + 2 * D);  // [TT][NW][32]
 
   const int tid = threadIdx.x;
   const int wave = __builtin_amdgcn_readfirstlane(tid / kWave);
   const int lane = tid % kWave;
   const int l32 = lane % 32, hh = lane / 32;
-  const int F = p.F;
-  const int nchunks = F / kHU;
+  const int lane16 = lane * 16;
+  const int64_t tok0 = static_cast<int64_t>(tile) * (32 * TT);
 
-  // Requests in the order in which their values are needed (they arrive in that order): row index and count, the projection's
-  // weights behind them, then - one latency later - the token rows, and last what is used after the projection.
-  const int64_t tok0 = static_cast<int64_t>(blockIdx.x) * 32;
-  SmallRows<1> xr, orow;
-  xr.request(p, p.x_rows != nullptr ? p.x_rows : p.rows, [&](int) { return tok0 + l32; });
-  orow.request(p, p.rows, [&](int) { return tok0 + l32; });
-  const int64_t count = token_count(p);
-  __builtin_amdgcn_sched_barrier(0);
-  [[maybe_unused]] bf16x8 w0[OUTP ? MBW * KS : 1];
-  if constexpr (OUTP) {
-    const char* src = reinterpret_cast<const char*>(p.w0) + static_cast<int64_t>(wave * MBW * KS) * kFrag;
+  // Weights: buffer accesses, whose address is a lane offset, a scalar offset and a constant (no vector arithmetic per load).
+  // Group k of the workgroup holds the NW chunks from (k * splits + split) * NW on, the wavefront's own one at + wave.
+  const int blob_bytes = nchunks * CFRAG * kFrag;
+  const auto blob = __builtin_amdgcn_make_buffer_rsrc(const_cast<bf16_t*>(p.w1), 0, blob_bytes, 0x00020000);
+  auto request = [&](int at, int constant) {
+    return __builtin_bit_cast(bf16x8, __builtin_amdgcn_raw_buffer_load_b128(blob, lane16 + constant, at, 0));
+  };
+  auto first_chunk = [&](int group) { return ((group << shift) + split) * NW; };
+  auto own_chunk = [&](int group) {
+    const int chunk = first_chunk(group) + wave;
+    return chunk < nchunks ? chunk : nchunks - 1;
+  };
+  auto up_at = [&](int group) { return own_chunk(group) * (CFRAG * kFrag); };
+  const int blob_end = blob_bytes - kFrag;  // (the last fragment stands in for those that are requested and not used)
+  auto request_up = [&](int at, auto ic) {
+    constexpr int i = decltype(ic)::value;
+    return request(at + i / 4 * (4 * kFrag), i % 4 * kFrag);
+  };
+  auto request_down = [&](int group, int j) {
+    const int at = (first_chunk(group) + j) * (CFRAG * kFrag) + (KS + wave) * kFrag;
+    return request(at < blob_end ? at : blob_end, 0);
+  };
+  int64_t xrow[SmallTokens<D, TT>::kPasses], row[TT];  // row: of token l32 of a tile in residual / out
+  tokens.in.resolve(count, xrow);
+  tokens.out.resolve(count, row);
+  // The token rows are loaded once per workgroup, contiguous pieces by neighbouring lanes (as operand fragments by every wavefront,
+  // 32 bytes of 32 rows an access, they cost the compute unit 16 times the requests), and become fragments in LDS.
+  constexpr int kPasses = SmallTokens<D, TT>::kPasses, kStep = SmallTokens<D, TT>::kStep, kPieces = SmallTokens<D, TT>::kPieces;
+  const int piece = tid % kPieces;
+  bf16x8 xp[kPasses];
+  {
+    const int col = piece * 8;
+    const int sh = p.x_plane_shift;
+    const bf16_t* base = p.x + (sh > 0 ? ((static_cast<int64_t>(col >> sh) * p.M) << sh) + (col & ((1 << sh) - 1)) : col);
+    const int64_t stride = sh > 0 ? static_cast<int64_t>(1) << sh : p.ldx;
 #pragma unroll
-    for (int i = 0; i < MBW * KS; ++i) w0[i] = *reinterpret_cast<const bf16x8*>(src + i * kFrag + lane * 16);
-    __builtin_amdgcn_sched_barrier(0);
+    for (int i = 0; i < kPasses; ++i) xp[i] = *reinterpret_cast<const bf16x8*>(base + xrow[i] * stride);
   }
-  if (tok0 >= count) return;  // whole workgroup
-  int64_t xrow[1], orows[1];
-  xr.resolve(count, xrow);
-  orow.resolve(count, orows);
-  const int64_t row = orows[0];  // of token l32 in residual / out
-  bf16x8 xf[1][KS];
-  load_token_rows_at<D, 1>(p, xrow, hh, xf);
-  // Four features per register quad of the lane's blocks, in accumulator order. A vector that is absent is read from the weights
+  // Four features per register quad of the lane's block, in accumulator order. A vector that is absent is read from the weights
   // instead (finite, in bounds for D values) and cleared where it is used: no branch between the loads.
-  auto feature_vectors = [&](const bf16_t* v, bf16x4 (&dst)[MBW][4]) {
+  auto feature_vectors = [&](const bf16_t* v, bf16x4 (&dst)[4]) {
     const bf16_t* src = v != nullptr ? v : p.w1;
 #pragma unroll
-    for (int m = 0; m < MBW; ++m)
-#pragma unroll
-      for (int jq = 0; jq < 4; ++jq)
-        dst[m][jq] = *reinterpret_cast<const bf16x4*>(src + (wave * MBW + m) * 32 + jq * 8 + hh * 4);
+    for (int jq = 0; jq < 4; ++jq) dst[jq] = *reinterpret_cast<const bf16x4*>(src + wave * 32 + jq * 8 + hh * 4);
   };
-  [[maybe_unused]] bf16x4 hv[MBW][4], b0v[MBW][4];  // block input, projection bias
-  if constexpr (OUTP) {
-    feature_vectors(p.residual + row * p.ldr, hv);
-    feature_vectors(p.b0, b0v);
-  }
-  __builtin_amdgcn_sched_barrier(0);
-  const int splits = p.splits > 1 ? p.splits : 1;
-  const int first_chunk = static_cast<int>(blockIdx.y) * NW + wave, stride = NW * splits;
-  const int first = first_chunk < nchunks ? first_chunk : nchunks - 1;
-  const char* ffn_blob = reinterpret_cast<const char*>(p.w1) + lane * 16;
-  bf16x8 ring[CFRAG];
-  auto load_chunk_frag = [&](int chunk, int i) {
-    return *reinterpret_cast<const bf16x8*>(ffn_blob + (static_cast<int64_t>(chunk) * CFRAG + i) * kFrag);
-  };
+  [[maybe_unused]] bf16x4 hv[TT][4], b0v[4];  // block input (then x1, in accumulator order), projection bias
+  auto block_input = [&]() {
+    if constexpr (OUTP) {
 #pragma unroll
-  for (int i = 0; i < CFRAG; ++i) ring[i] = load_chunk_frag(first, i);
+      for (int t = 0; t < TT; ++t) feature_vectors(p.residual + row[t] * p.ldr, hv[t]);
+      feature_vectors(p.b0, b0v);
+    }
+  };
+  if constexpr (TT == 1) block_input();
   // first-layer bias, gated half first; FOLD: with the constants the packed layer carries. 8 entries per thread and round.
   auto bias_piece = [&](int i) {
     const bool gated = i < F;  // F is a multiple of 32: a piece lies in one half
@@ -303,233 +358,391 @@ __global__ __launch_bounds__(4 * kWave, 1) void swiglu_ffn_small_kernel(const Ts
   };
   auto store_bias = [&](int i, bf16x8 v) {
     const float c = p.b1 == nullptr ? 0.f : (!FOLD ? 1.f : (i < F ? kFoldGate : kFoldValue));
+    f32x4 lo, hi;  // widened once, here, not per chunk
 #pragma unroll
-    for (int e = 0; e < 8; ++e) v[e] = static_cast<bf16_t>(static_cast<float>(v[e]) * c);
-    if (i < 2 * F) *reinterpret_cast<bf16x8*>(bias_lds + i) = v;
+    for (int e = 0; e < 4; ++e) {
+      lo[e] = static_cast<float>(static_cast<bf16_t>(static_cast<float>(v[e]) * c));
+      hi[e] = static_cast<float>(static_cast<bf16_t>(static_cast<float>(v[4 + e]) * c));
+    }
+    if (i < 2 * F) {
+      *reinterpret_cast<f32x4*>(bias_lds + i) = lo;
+      *reinterpret_cast<f32x4*>(bias_lds + i + 4) = hi;
+    }
   };
   const bf16x8 bias_regs = bias_piece(tid * 8 < 2 * F ? tid * 8 : 0);
-  bf16x4 b2v[MBW][4], hwv[MBW][4];  // for the end of the kernel: down-projection bias, readout weight
-  feature_vectors(p.b2, b2v);
-  feature_vectors(p.head_w, hwv);
+  const bf16_t* end_src = tid < D / 8 ? p.b2 : p.head_w;
+  bf16x8 end_regs = *reinterpret_cast<const bf16x8*>((end_src != nullptr ? end_src : p.w1) + tid % (D / 8) * 8);
   __builtin_amdgcn_sched_barrier(0);
+  // Groups in which the wavefront has a chunk: all but perhaps the last one of the workgroup. (A wavefront without a chunk in a slab
+  // goes through the motions with the last chunk: what it leaves in its place of the hidden state is not used.)
+  const int all_own = first_chunk(groups - 1) + wave < nchunks ? groups : groups - 1;
+  constexpr int kSlabGroups = kSlab / NW;
+  auto ring_up = [&](int group) {
+    const int at = up_at(group);
+    static_for<KS>([&](auto ic) { ring[decltype(ic)::value] = request_up(at, ic); });
+  };
+  if constexpr (!OUTP) ring_up(0);
+#pragma unroll
+  for (int i = 0; i < kPasses; ++i) *reinterpret_cast<bf16x8*>(x_lds + (i * kStep + tid / kPieces) * kRow + piece * 16) = xp[i];
+  if constexpr (TT > 1) {  // (no registers for it next to the rows)
+    __builtin_amdgcn_sched_barrier(0);
+    block_input();
+  }
+  __syncthreads();
+  auto fragment = [&](const uint8_t* rows, int ks) {
+    return *reinterpret_cast<const bf16x8*>(rows + l32 * kRow + (ks * 16 + hh * 8) * 2);
+  };
+  bf16x8 xf[XT][KS];
+#pragma unroll
+  for (int t = 0; t < XT; ++t)
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks) xf[t][ks] = fragment(x_lds + t * 32 * kRow, ks);
+  // Fragment ks of tile t: from the registers, or read from `far`, two products ahead.
+  auto products = [&](f32x16 (&acc)[TT], const uint8_t* far, auto reload) {
+    bf16x8 ahead[2];
+    if constexpr (XT < TT) {
+#pragma unroll
+      for (int ks = 0; ks < 2; ++ks) ahead[ks] = fragment(far, ks);
+    }
+    static_for<KS>([&](auto ic) {
+      constexpr int i = decltype(ic)::value;
+#pragma unroll
+      for (int t = 0; t < XT; ++t) acc[t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ring[i], xf[t][i], acc[t], 0, 0, 0);
+      if constexpr (XT < TT) {
+        acc[1] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ring[i], ahead[i % 2], acc[1], 0, 0, 0);
+        if constexpr (i + 2 < KS) ahead[i % 2] = fragment(far, i + 2);
+      }
+      reload(ic);
+      __builtin_amdgcn_sched_barrier(0);
+    });
+  };
 
   if constexpr (OUTP) {
     const float b0_on = p.b0 != nullptr ? 1.f : 0.f;
-    float ss = 0.f;
+    f32x16 acc[TT];
 #pragma unroll
-    for (int m = 0; m < MBW; ++m) {
-      f32x16 acc;
+    for (int t = 0; t < TT; ++t)
 #pragma unroll
-      for (int j = 0; j < 16; ++j) acc[j] = 0.f;
+      for (int j = 0; j < 16; ++j) acc[t][j] = 0.f;
+    const int at = up_at(0);
+    products(acc, x_lds + 32 * kRow, [&](auto ic) { ring[decltype(ic)::value] = request_up(at, ic); });
 #pragma unroll
-      for (int ks = 0; ks < KS; ++ks) acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(w0[m * KS + ks], xf[0][ks], acc, 0, 0, 0);
+    for (int t = 0; t < TT; ++t) {
+      float ss = 0.f;
 #pragma unroll
       for (int jq = 0; jq < 4; ++jq) {
         bf16x4 x1;
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
-          const float lin = static_cast<float>(static_cast<bf16_t>(fmaf(static_cast<float>(b0v[m][jq][e]), b0_on, acc[jq * 4 + e])));
-          x1[e] = static_cast<bf16_t>(lin + static_cast<float>(hv[m][jq][e]));
+          const float lin = static_cast<float>(static_cast<bf16_t>(fmaf(static_cast<float>(b0v[jq][e]), b0_on, acc[t][jq * 4 + e])));
+          x1[e] = static_cast<bf16_t>(lin + static_cast<float>(hv[t][jq][e]));
           const float r = static_cast<float>(x1[e]);
           ss = fmaf(r, r, ss);
         }
-        *reinterpret_cast<bf16x4*>(x1_lds + l32 * kRow + ((wave * MBW + m) * 32 + jq * 8 + hh * 4) * 2) = x1;
+        hv[t][jq] = x1;
       }
+      ss = half_wave_pair_sum(ss);
+      if (hh == 0) sums[(t * NW + wave) * 32 + l32] = ss;
     }
-    ss = half_wave_pair_sum(ss);
-    if (hh == 0) sums[wave * 32 + l32] = ss;
   }
   store_bias(tid * 8, bias_regs);
   for (int i = (NW * kWave + tid) * 8; i < 2 * F; i += NW * kWave * 8) store_bias(i, bias_piece(i));
-  __syncthreads();
+  if (tid < 2 * (D / 8)) {
+    if (end_src == nullptr) {
+#pragma unroll
+      for (int e = 0; e < 8; ++e) end_regs[e] = static_cast<bf16_t>(0.f);
+    }
+    *reinterpret_cast<bf16x8*>(end_lds + tid * 8) = end_regs;
+  }
   if constexpr (OUTP) {
-    float total = 0.f;
+    __syncthreads();
+    const bool keep = p.x1_out != nullptr && split == 0;
 #pragma unroll
-    for (int w = 0; w < NW; ++w) total += sums[w * 32 + l32];
-    const float scale = p.norm_w != nullptr ? rsqrtf(total * (1.0f / D) + p.eps) : 1.0f;
-    if (p.rstd_out != nullptr && wave == 0 && hh == 0 && tok0 + l32 < count) p.rstd_out[row] = scale;
+    for (int t = 0; t < TT; ++t) {
+      float sum = 0.f;
 #pragma unroll
-    for (int ks = 0; ks < KS; ++ks) {
-      xf[0][ks] = *reinterpret_cast<const bf16x8*>(x1_lds + l32 * kRow + (ks * 16 + hh * 8) * 2);
+      for (int w = 0; w < NW; ++w) sum += sums[(t * NW + w) * 32 + l32];
+      const float scale = p.norm_w != nullptr ? rsqrtf(sum * (1.0f / D) + p.eps) : 1.0f;
+      if (p.rstd_out != nullptr && split == 0 && wave == 0 && hh == 0 && tok0 + t * 32 + l32 < count) p.rstd_out[row[t]] = scale;
 #pragma unroll
-      for (int e = 0; e < 8; ++e) xf[0][ks][e] = static_cast<bf16_t>(static_cast<float>(xf[0][ks][e]) * scale);
-    }
-  } else if (p.norm_w != nullptr) {
-    float rstd[1];
-    token_rstd<D, 1>(p.eps, xf, rstd);
+      for (int jq = 0; jq < 4; ++jq) {  // every wavefront normalises the features it has projected
+        const int at = l32 * kRow + (wave * 32 + jq * 8 + hh * 4) * 2;
+        bf16x4 v;
 #pragma unroll
-    for (int ks = 0; ks < KS; ++ks)
-#pragma unroll
-      for (int e = 0; e < 8; ++e) xf[0][ks][e] = static_cast<bf16_t>(static_cast<float>(xf[0][ks][e]) * rstd[0]);
-  }
-
-  f32x16 oacc[MB];
-#pragma unroll
-  for (int mb = 0; mb < MB; ++mb)
-#pragma unroll
-    for (int j = 0; j < 16; ++j) oacc[mb][j] = 0.f;
-  for (int chunk = first_chunk; chunk < nchunks; chunk += stride) {
-    const int next = chunk + stride < nchunks ? chunk + stride : chunk;  // the last chunk is requested once more, and not used
-    const bf16x8 bg = *reinterpret_cast<const bf16x8*>(bias_lds + chunk * kHU + hh * 8);
-    const bf16x8 bu = *reinterpret_cast<const bf16x8*>(bias_lds + F + chunk * kHU + hh * 8);
-    f32x16 gu;
-#pragma unroll
-    for (int e = 0; e < 8; ++e) {
-      gu[e] = static_cast<float>(bg[e]);
-      gu[8 + e] = static_cast<float>(bu[e]);
-    }
-    static_for<KS>([&](auto ic) {
-      constexpr int i = decltype(ic)::value;
-      gu = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ring[i], xf[0][i], gu, 0, 0, 0);
-      ring[i] = load_chunk_frag(next, i);
-      __builtin_amdgcn_sched_barrier(0);
-    });
-    bf16x8 hb;
-#pragma unroll
-    for (int e = 0; e < 8; ++e) {
-      if constexpr (FOLD)
-        hb[e] = static_cast<bf16_t>(gu[e] * gu[8 + e] * __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(gu[e])));
-      else
-        hb[e] = static_cast<bf16_t>(silu_f(gu[e]) * gu[8 + e]);
-    }
-    static_for<MB>([&](auto ic) {
-      constexpr int i = decltype(ic)::value;
-      oacc[i] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ring[KS + i], hb, oacc[i], 0, 0, 0);
-      ring[KS + i] = load_chunk_frag(next, KS + i);
-      __builtin_amdgcn_sched_barrier(0);
-    });
-  }
-
-  // ---- the four partials: [wavefront][feature block][register quad][lane] -------------------------------------------------
-#pragma unroll
-  for (int mb = 0; mb < MB; ++mb)
-#pragma unroll
-    for (int jq = 0; jq < 4; ++jq) {
-      const f32x4 v = {oacc[mb][jq * 4], oacc[mb][jq * 4 + 1], oacc[mb][jq * 4 + 2], oacc[mb][jq * 4 + 3]};
-      *reinterpret_cast<f32x4*>(smem + wave * kPart + ((mb * 4 + jq) * kWave + lane) * 16) = v;
-    }
-  __syncthreads();
-  f32x4 total[MBW][4];
-#pragma unroll
-  for (int m = 0; m < MBW; ++m)
-#pragma unroll
-    for (int jq = 0; jq < 4; ++jq) {
-      const int piece = ((wave * MBW + m) * 4 + jq) * kWave + lane;
-      total[m][jq] = *reinterpret_cast<const f32x4*>(smem + piece * 16);
-#pragma unroll
-      for (int w = 1; w < NW; ++w) {
-        const f32x4 v = *reinterpret_cast<const f32x4*>(smem + w * kPart + piece * 16);
-#pragma unroll
-        for (int e = 0; e < 4; ++e) total[m][jq][e] += v[e];
+        for (int e = 0; e < 4; ++e) v[e] = static_cast<bf16_t>(static_cast<float>(hv[t][jq][e]) * scale);
+        *reinterpret_cast<bf16x4*>(normed_lds(t) + at) = v;
+        if (keep) *reinterpret_cast<bf16x4*>(x_lds + t * 32 * kRow + at) = hv[t][jq];
       }
     }
-  if (splits > 1) {
+    __syncthreads();
+#pragma unroll
+    for (int t = 0; t < XT; ++t)
+#pragma unroll
+      for (int ks = 0; ks < KS; ++ks) xf[t][ks] = fragment(normed_lds(t), ks);
+    if (keep) {
+#pragma unroll
+      for (int i = 0; i < kPasses; ++i) {
+        const int t = i * kStep + tid / kPieces;
+        if (tok0 + t >= count) continue;
+        const int64_t r = p.rows != nullptr ? static_cast<int64_t>(p.rows[tok0 + t]) : tok0 + t;
+        *reinterpret_cast<bf16x8*>(p.x1_out + r * D + piece * 8) = *reinterpret_cast<const bf16x8*>(x_lds + t * kRow + piece * 16);
+      }
+      if constexpr (TT == 1) __syncthreads();  // the hidden state takes the place of x1
+    }
+  } else {
+    // the rows are whole in every wavefront; the second tile's, where it stays in LDS, is normalised by the first
+    if constexpr (XT < TT) {
+      if (wave == 0) {
+        bf16x8 far[1][KS];
+        float rstd[1] = {1.0f};
+#pragma unroll
+        for (int ks = 0; ks < KS; ++ks) far[0][ks] = fragment(x_lds + 32 * kRow, ks);
+        if (p.norm_w != nullptr) token_rstd<D, 1>(p.eps, far, rstd);
+#pragma unroll
+        for (int ks = 0; ks < KS; ++ks) {
+#pragma unroll
+          for (int e = 0; e < 8; ++e) far[0][ks][e] = static_cast<bf16_t>(static_cast<float>(far[0][ks][e]) * rstd[0]);
+          *reinterpret_cast<bf16x8*>(normed_lds(1) + l32 * kRow + (ks * 16 + hh * 8) * 2) = far[0][ks];
+        }
+      }
+    }
+    if (p.norm_w != nullptr) {
+      float rstd[XT];
+      token_rstd<D, XT>(p.eps, xf, rstd);
+#pragma unroll
+      for (int t = 0; t < XT; ++t)
+#pragma unroll
+        for (int ks = 0; ks < KS; ++ks)
+#pragma unroll
+          for (int e = 0; e < 8; ++e) xf[t][ks][e] = static_cast<bf16_t>(static_cast<float>(xf[t][ks][e]) * rstd[t]);
+    }
+    if constexpr (TT == 1) __syncthreads();  // as below, and the biases
+  }
+  if constexpr (TT > 1) __syncthreads();  // the hidden state takes the place of the tokens
+
+  f32x16 total[TT];
+#pragma unroll
+  for (int t = 0; t < TT; ++t)
+#pragma unroll
+    for (int j = 0; j < 16; ++j) total[t][j] = 0.f;
+  for (int slab = 0; slab < (SLABS ? groups : 1); slab += kSlabGroups) {
+    const int slab_end = SLABS && slab + kSlabGroups < groups ? slab + kSlabGroups : groups;
+    const int own_end = slab_end < all_own ? slab_end : all_own;
+    auto up_chunk = [&](int group, auto last_c) {
+      constexpr bool last = decltype(last_c)::value;
+      const int unit = own_chunk(group) * kHU + hh * 8;
+      const int next = up_at(group + 1);
+      f32x16 gu[TT];
+#pragma unroll
+      for (int t = 0; t < TT; ++t)
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          const f32x4 b = *reinterpret_cast<const f32x4*>(bias_lds + (q < 2 ? 0 : F) + unit + q % 2 * 4);
+#pragma unroll
+          for (int e = 0; e < 4; ++e) gu[t][q * 4 + e] = b[e];
+        }
+      products(gu, normed_lds(TT - 1), [&](auto ic) {
+        constexpr int i = decltype(ic)::value;
+        ring[i] = last ? request_down(slab + i / NW, i % NW) : request_up(next, ic);
+      });
+#pragma unroll
+      for (int t = 0; t < TT; ++t) {
+        bf16x8 hb;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+          if constexpr (FOLD)
+            hb[e] = static_cast<bf16_t>(gu[t][e] * gu[t][8 + e] * __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(gu[t][e])));
+          else
+            hb[e] = static_cast<bf16_t>(silu_f(gu[t][e]) * gu[t][8 + e]);
+        }
+        *reinterpret_cast<bf16x8*>(hidden_lds + (((group - slab) * NW + wave) * TT + t) * kFrag + lane16) = hb;
+      }
+    };
+    for (int group = slab; group + 1 < own_end; ++group) up_chunk(group, std::false_type{});
+    up_chunk(own_end > slab ? own_end - 1 : slab, std::true_type{});
+    __syncthreads();
+    // two groups a round; only the last group of a workgroup may be a partial one
+    auto down_groups = [&](int group, auto last_c) {
+      constexpr bool last = decltype(last_c)::value;
+      static_for<KS / 4>([&](auto quad_c) {
+        constexpr int q = decltype(quad_c)::value;
+        const int g = group + q * 4 / NW;
+        if (last && g >= slab_end) return;
+        bf16x8 hb[4][TT];
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+#pragma unroll
+          for (int t = 0; t < TT; ++t)
+            hb[j][t] = *reinterpret_cast<const bf16x8*>(hidden_lds + (((group - slab) * NW + q * 4 + j) * TT + t) * kFrag + lane16);
+        static_for<4>([&](auto jc) {
+          constexpr int j = decltype(jc)::value, i = q * 4 + j;
+          if (!last || first_chunk(g) + i % NW < nchunks) {
+#pragma unroll
+            for (int t = 0; t < TT; ++t) total[t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ring[i], hb[j][t], total[t], 0, 0, 0);
+          }
+          if constexpr (!last) ring[i] = request_down(g + 2, i % NW);
+          __builtin_amdgcn_sched_barrier(0);
+        });
+      });
+    };
+    int group = slab;
+    for (; group + 2 < slab_end; group += 2) down_groups(group, std::false_type{});
+    down_groups(group, std::true_type{});
+    if constexpr (SLABS) {
+      if (slab_end < groups) {  // the ring starts anew
+        ring_up(slab_end);
+        __syncthreads();  // the hidden state of this slab has been read
+      }
+    }
+  }
+
+  if (TT == 1 && splits > 1) {
     // The partial of this workgroup becomes visible to the chip, then the workgroup counts itself: whoever counts last finds all
     // partials of the tile (nobody waits for anybody). They are added in the order of the splits: the same result every run.
-    const SharedPartials parts(p.split_partials + static_cast<int64_t>(blockIdx.x) * splits * (kPart / 4), splits * kPart);
-    const int lane_at = (wave * MBW * 4 * kWave + lane) * 16;  // of a partial: [feature block][register quad][lane]
-    const int mine = static_cast<int>(blockIdx.y) * kPart + lane_at;
+    const SharedPartials parts(p.split_partials + static_cast<int64_t>(tile) * splits * (kPart / 4), splits * kPart);
+    const int lane_at = wave * (4 * kWave * 16) + lane16;  // of a partial: [feature block][register quad][lane]
+    const int at = split * kPart + lane_at;
 #pragma unroll
-    for (int m = 0; m < MBW; ++m)
-#pragma unroll
-      for (int jq = 0; jq < 4; ++jq) parts.store(mine + (m * 4 + jq) * (kWave * 16), total[m][jq]);
+    for (int jq = 0; jq < 4; ++jq)
+      parts.store(at + jq * (kWave * 16), f32x4{total[0][jq * 4], total[0][jq * 4 + 1], total[0][jq * 4 + 2], total[0][jq * 4 + 3]});
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // this wavefront's partials have reached the chip's common memory
     __syncthreads();
     uint32_t* arrived = reinterpret_cast<uint32_t*>(sums);
     if (tid == 0)
-      *arrived = __hip_atomic_fetch_add(p.split_counters + blockIdx.x, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      *arrived = __hip_atomic_fetch_add(p.split_counters + tile, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     __syncthreads();
     const bool last = *arrived == static_cast<uint32_t>(splits - 1);
     __syncthreads();  // (the row sums of the readout reuse the word)
     if (!last) return;
-    if (tid == 0) p.split_counters[blockIdx.x] = 0u;
+    if (tid == 0) p.split_counters[tile] = 0u;
 #pragma unroll
-    for (int m = 0; m < MBW; ++m)
+    for (int j = 0; j < 16; ++j) total[0][j] = 0.f;
+    auto add_partials = [&](auto number) {  // all in flight at once
+      constexpr int n = decltype(number)::value;
+      f32x4 v[n][4];
 #pragma unroll
-      for (int jq = 0; jq < 4; ++jq)
+      for (int u = 0; u < n; ++u)
 #pragma unroll
-        for (int e = 0; e < 4; ++e) total[m][jq][e] = 0.f;
-    auto add_partials = [&](int first_split, auto ahead) {
-      constexpr int kAhead = decltype(ahead)::value;  // partials in flight
-      f32x4 v[kAhead][MBW][4];
+        for (int jq = 0; jq < 4; ++jq) v[u][jq] = parts.load(u * kPart + lane_at + jq * (kWave * 16));
 #pragma unroll
-      for (int u = 0; u < kAhead; ++u)
+      for (int u = 0; u < n; ++u)
 #pragma unroll
-        for (int m = 0; m < MBW; ++m)
+        for (int jq = 0; jq < 4; ++jq)
 #pragma unroll
-          for (int jq = 0; jq < 4; ++jq)
-            v[u][m][jq] = parts.load((first_split + u) * kPart + lane_at + (m * 4 + jq) * (kWave * 16));
-#pragma unroll
-      for (int u = 0; u < kAhead; ++u)
-#pragma unroll
-        for (int m = 0; m < MBW; ++m)
-#pragma unroll
-          for (int jq = 0; jq < 4; ++jq)
-#pragma unroll
-            for (int e = 0; e < 4; ++e) total[m][jq][e] += v[u][m][jq][e];
+          for (int e = 0; e < 4; ++e) total[0][jq * 4 + e] += v[u][jq][e];
     };
-    // 2, 4 or 8 splits (ffn_splits). Eight partials, 64 KB per wavefront: 17.0 us for the kernel with four in flight, 17.5 with two.
-    if (splits == 2) add_partials(0, std::integral_constant<int, 2>{});
-    for (int w = 0; w + 4 <= splits; w += 4) add_partials(w, std::integral_constant<int, 4>{});
+    if (splits == 2)  // 2 or 4 (ffn_splits)
+      add_partials(std::integral_constant<int, 2>{});
+    else
+      add_partials(std::integral_constant<int, 4>{});
   }
-  const bool live = tok0 + l32 < count;
-  if (OUTP && p.x1_out != nullptr) {
-    for (int idx = tid; idx < 32 * (D / 8); idx += NW * kWave) {
-      const int t = idx / (D / 8), c = idx % (D / 8) * 8;
-      if (tok0 + t >= count) continue;
-      const int64_t r = p.rows != nullptr ? static_cast<int64_t>(p.rows[tok0 + t]) : tok0 + t;
-      *reinterpret_cast<bf16x8*>(p.x1_out + r * D + c) = *reinterpret_cast<const bf16x8*>(x1_lds + t * kRow + c * 2);
-    }
-  }
-  const float b2_on = p.b2 != nullptr ? 1.f : 0.f;
-  float hdot = 0.f;
+  bf16x4 result[TT][4];
 #pragma unroll
-  for (int m = 0; m < MBW; ++m)
+  for (int t = 0; t < TT; ++t) {
+    float hdot = 0.f;
 #pragma unroll
     for (int jq = 0; jq < 4; ++jq) {
-      const int col = (wave * MBW + m) * 32 + jq * 8 + hh * 4;
-      f32x4 s = total[m][jq];
+      const int col = wave * 32 + jq * 8 + hh * 4;
+      const bf16x4 b2v = *reinterpret_cast<const bf16x4*>(end_lds + col), hwv = *reinterpret_cast<const bf16x4*>(end_lds + D + col);
+      f32x4 s;
 #pragma unroll
-      for (int e = 0; e < 4; ++e) s[e] = fmaf(static_cast<float>(b2v[m][jq][e]), b2_on, s[e]);
+      for (int e = 0; e < 4; ++e) s[e] = total[t][jq * 4 + e] + static_cast<float>(b2v[e]);
       bf16x4 o;
       if constexpr (OUTP) {  // x1 + down, rounded once
-        const bf16x4 x1 = *reinterpret_cast<const bf16x4*>(x1_lds + l32 * kRow + col * 2);
 #pragma unroll
-        for (int e = 0; e < 4; ++e) o[e] = static_cast<bf16_t>(s[e] + static_cast<float>(x1[e]));
+        for (int e = 0; e < 4; ++e) o[e] = static_cast<bf16_t>(s[e] + static_cast<float>(hv[t][jq][e]));
       } else {
 #pragma unroll
         for (int e = 0; e < 4; ++e) o[e] = static_cast<bf16_t>(s[e]);
         if (p.residual != nullptr) {
-          const bf16x4 r = *reinterpret_cast<const bf16x4*>(p.residual + row * p.ldr + col);
+          const bf16x4 r = *reinterpret_cast<const bf16x4*>(p.residual + row[t] * p.ldr + col);
 #pragma unroll
           for (int e = 0; e < 4; ++e) o[e] = static_cast<bf16_t>(static_cast<float>(o[e]) + static_cast<float>(r[e]));
         }
       }
-      if (live) *reinterpret_cast<bf16x4*>(p.out + row * p.ldo + col) = o;
+      result[t][jq] = o;
 #pragma unroll
-      for (int e = 0; e < 4; ++e) hdot = fmaf(static_cast<float>(o[e]), static_cast<float>(hwv[m][jq][e]), hdot);
+      for (int e = 0; e < 4; ++e) hdot = fmaf(static_cast<float>(o[e]), static_cast<float>(hwv[e]), hdot);
     }
-  if (p.head_w != nullptr) {
-    hdot = half_wave_pair_sum(hdot);
-    if (hh == 0) sums[wave * 32 + l32] = hdot;
-    __syncthreads();
-    if (wave == 0 && hh == 0 && live) {
-      float d = 0.f;
-#pragma unroll
-      for (int w = 0; w < NW; ++w) d += sums[w * 32 + l32];
-      p.token_dots[row] = d;
+    if (p.head_w != nullptr) {
+      hdot = half_wave_pair_sum(hdot);
+      if (hh == 0) sums[(t * NW + wave) * 32 + l32] = hdot;
     }
   }
+  if (p.head_w != nullptr) {  // (in front of the stores: the barrier would wait for them)
+    __syncthreads();
+    if (wave < TT && hh == 0 && tok0 + wave * 32 + l32 < count) {
+      float d = 0.f;
+#pragma unroll
+      for (int w = 0; w < NW; ++w) d += sums[(wave * NW + w) * 32 + l32];
+      p.token_dots[TT == 1 || wave == 0 ? row[0] : row[TT - 1]] = d;
+    }
+  }
+#pragma unroll
+  for (int t = 0; t < TT; ++t) {
+    if (tok0 + t * 32 + l32 >= count) continue;
+#pragma unroll
+    for (int jq = 0; jq < 4; ++jq)
+      *reinterpret_cast<bf16x4*>(p.out + row[t] * p.ldo + wave * 32 + jq * 8 + hh * 4) = result[t][jq];
+  }
+}
+
+// Forms of the kernel: one tile, one slab / one tile, several slabs (F > 1024) / one or two tiles, one slab. The last is for more
+// rows than the chip has places for one-tile workgroups: the number of tokens, known on the device only, decides whether its
+// workgroups take two tiles (D = 256, F = 1024: 12288 rows, all valid, 28.0 us, 39.3 with one tile in two rounds; 6758 valid 21.2, one tile
+// in one round).
+enum { kSmallOne, kSmallSlabs, kSmallPair };
+
+template <int D, bool OUTP, bool FOLD, int FORM>
+__global__ __launch_bounds__(D / 32 * kWave, D == 256 || FORM == kSmallPair ? 2 : 3) void swiglu_ffn_small_kernel(const TsParams p) {
+  constexpr int KS = D / 16;
+  extern __shared__ __attribute__((aligned(1024))) uint8_t smem[];
+  const int tid = threadIdx.x;
+  const int wave = __builtin_amdgcn_readfirstlane(tid / kWave);
+  const int lane = tid % kWave;
+  // Workgroup i runs on die i % 8: with two or four splits a die reads only its own share of the hidden units' weights.
+  const int shift = __builtin_ctz(p.splits > 1 ? p.splits : 1);
+  const int tile = static_cast<int>(blockIdx.x) >> shift, split = static_cast<int>(blockIdx.x) & ((1 << shift) - 1);
+  // Requests in the order in which their values are needed (they arrive in that order): row index and count, the projection's
+  // weights behind them, then - one latency later - the token rows, and what is used after the projection.
+  SmallTokens<D, 1> one;
+  [[maybe_unused]] SmallTokens<D, 2> two;
+  one.request(p, static_cast<int64_t>(tile) * 32, tid, lane % 32);
+  if constexpr (FORM == kSmallPair) two.request(p, static_cast<int64_t>(tile) * 64, tid, lane % 32);
+  const int64_t count = token_count(p);
+  __builtin_amdgcn_sched_barrier(0);
+  bf16x8 ring[KS];
+  if constexpr (OUTP) {
+    const auto w0 = __builtin_amdgcn_make_buffer_rsrc(const_cast<bf16_t*>(p.w0), 0, D * D * 2, 0x00020000);
+    static_for<KS>([&](auto ic) {
+      constexpr int i = decltype(ic)::value;
+      ring[i] = __builtin_bit_cast(bf16x8, __builtin_amdgcn_raw_buffer_load_b128(w0, lane * 16 + i % 4 * kFrag,
+                                                                                 wave * (KS * kFrag) + i / 4 * (4 * kFrag), 0));
+    });
+    __builtin_amdgcn_sched_barrier(0);
+  }
+  if constexpr (FORM == kSmallPair) {
+    if (count > static_cast<int64_t>(p.units) * (32 * small_pair_residents(D))) {
+      if (static_cast<int64_t>(tile) * 64 < count) ffn_small_tile<D, 2, OUTP, FOLD, false>(p, smem, count, tile, 0, two, ring);
+      return;
+    }
+  }
+  if (static_cast<int64_t>(tile) * 32 < count)
+    ffn_small_tile<D, 1, OUTP, FOLD, FORM == kSmallSlabs>(p, smem, count, tile, split, one, ring);
 }
 
 }  // namespace
 
+// Two or four workgroups per token tile as long as the tiles leave them a compute unit each, every wavefront keeps two chunks of
+// hidden units, and the weights are worth the exchange. Whole 4-block calls, 1 / 2 / 4 / 8 splits, us: D = 256, F = 1024 - 1 x 512
+// positions 146 / 125 / 116 / 119, 8 x 256 139 / 121 / 119; F = 512 (two chunks at two splits) - 1 x 512 115 / 112 / 108, 4 x 512
+// 116 / 115 / 116; D = 128, F = 512 - 1 x 512 86 / 84 / 82, 8 x 256 81 / 80 / 80; F = 256 - 78 / 79 / 79, 74 / 75 / 77.
 int ffn_splits(int64_t M, int32_t D, int32_t F) {
   const int64_t tiles = (M + 31) / 32;
   const int cus = compute_units();
   int splits = 1;
-  if (ffn_few_rows(M, D))
-    while (splits < 8 && 2 * splits * tiles <= cus && 2 * splits * 4 * kHU <= F) splits *= 2;
+  if (ffn_few_rows(M, D) && F >= 512)
+    while (splits < 4 && 2 * splits * tiles <= cus && 2 * splits * 2 * (D / 32) * kHU <= F) splits *= 2;
   return splits;
 }
 
@@ -561,16 +774,30 @@ int norm_linear_small(const TsParams& p, int32_t K, int qk_mode, hipStream_t s, 
 }
 
 int swiglu_ffn_small(const TsParams& p, int32_t D, bool with_proj, bool act_folded, hipStream_t s, const char* name) {
-  const size_t lds_bytes = static_cast<size_t>(4) * 32 * D * 4 + 32 * (D * 2 + 16) + static_cast<size_t>(2) * p.F * 2 + 4 * 32 * 4;
+  const int splits = p.splits > 1 ? p.splits : 1;
+  const int64_t tiles = (p.M + 31) / 32;
+  const int chunks = small_groups(D, p.F, splits) * (D / 32);
+  const int form = chunks > kSlab ? kSmallSlabs : (tiles > small_one_residents(D) * p.units ? kSmallPair : kSmallOne);
+  const int tt = form == kSmallPair ? 2 : 1;
+  int tile_bytes = small_tile_bytes(D, 1, chunks);
+  if (tt == 2 && small_tile_bytes(D, 2, chunks) > tile_bytes) tile_bytes = small_tile_bytes(D, 2, chunks);
+  const size_t lds_bytes = tile_bytes + static_cast<size_t>(2) * p.F * 4 + 4 * D + static_cast<size_t>(tt) * (D / 32) * 32 * 4;
   if (lds_bytes > 160 * 1024) return 1;
-  const dim3 grid(static_cast<uint32_t>((p.M + 31) / 32), p.splits > 1 ? p.splits : 1);
-#define TAAC_SMALL(DD, OO, FF)                                                                                        \
+  const int64_t pairs = (p.M + 63) / 64, residents = small_pair_residents(D) * p.units;  // (these take one tile while that suffices)
+  const dim3 grid(static_cast<uint32_t>(form == kSmallPair ? (pairs > residents ? pairs : residents) : tiles * splits));
+#define TAAC_SMALL_LAUNCH(DD, OO, FF, FORM)                                                                           \
   do {                                                                                                                \
-    if (hipFuncSetAttribute(reinterpret_cast<const void*>(swiglu_ffn_small_kernel<DD, OO, FF>),                       \
+    if (hipFuncSetAttribute(reinterpret_cast<const void*>(swiglu_ffn_small_kernel<DD, OO, FF, FORM>),                 \
                             hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds_bytes)) != hipSuccess)   \
       return set_error(TAAC_ERR_LAUNCH, "%s: cannot reserve %zu bytes of LDS", name, lds_bytes);                      \
-    hipLaunchKernelGGL((swiglu_ffn_small_kernel<DD, OO, FF>), grid, dim3(4 * kWave), lds_bytes, s, p);                \
+    hipLaunchKernelGGL((swiglu_ffn_small_kernel<DD, OO, FF, FORM>), grid, dim3(DD / 32 * kWave), lds_bytes, s, p);    \
     return check_launch(name);                                                                                        \
+  } while (0)
+#define TAAC_SMALL(DD, OO, FF)                                        \
+  do {                                                                \
+    if (form == kSmallSlabs) TAAC_SMALL_LAUNCH(DD, OO, FF, kSmallSlabs); \
+    if (form == kSmallPair) TAAC_SMALL_LAUNCH(DD, OO, FF, kSmallPair);   \
+    TAAC_SMALL_LAUNCH(DD, OO, FF, kSmallOne);                         \
   } while (0)
 #define TAAC_SMALL_D(DD)                        \
   do {                                          \
@@ -583,6 +810,7 @@ int swiglu_ffn_small(const TsParams& p, int32_t D, bool with_proj, bool act_fold
   TAAC_SMALL_D(128);
 #undef TAAC_SMALL_D
 #undef TAAC_SMALL
+#undef TAAC_SMALL_LAUNCH
 }
 
 }  // namespace taac

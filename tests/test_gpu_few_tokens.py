@@ -102,6 +102,32 @@ def test_feed_forward_matches_the_persistent_kernel(device, test_hooks, m, d, f,
         assert torch.equal(held, attention_out_ffn(x, wo, bo, res, wu, bu, wd, bd, norm_weight=nw))
 
 
+@pytest.mark.parametrize("d,f,rows_over,valid", [(256, 64, 1, 1.0), (256, 1024, 33, 1.0), (256, 96, 1, 0.5), (256, 64, 33, 0.99), (128, 32, 1, 1.0),
+                                                 (128, 512, 65, 0.8), (128, 32, 1, 0.4), (256, 1056, None, 1.0), (128, 2080, None, 0.7)])
+def test_forms_of_the_few_token_feed_forward(device, test_hooks, d, f, rows_over, valid):
+    """Rows just over the places that the chip has for one-tile workgroups (one per compute unit at D = 256, three at 128), with so many
+    valid that workgroups take two tiles, the last of them a remainder, or one; hidden sizes over one slab of 1024 units, with a
+    remainder (rows_over None: 70 rows). Bound: as in the test above. Rows that are not listed stay as they are."""
+    places = torch.cuda.get_device_properties(device).multi_processor_count * (1 if d == 256 else 3)
+    m = 70 if rows_over is None else 32 * places + rows_over
+    g = torch.Generator().manual_seed(m + f)
+    x, res, nw = _bf16(g, m, d).to(device), _bf16(g, m, d).to(device), (1 + _bf16(g, d, scale=0.1)).to(device)
+    wo, bo = _bf16(g, d, d, scale=d ** -0.5).to(device), _bf16(g, d, scale=0.1).to(device)
+    wu, bu = _bf16(g, 2 * f, d, scale=d ** -0.5).to(device), _bf16(g, 2 * f, scale=0.1).to(device)
+    wd, bd = _bf16(g, d, f, scale=f ** -0.5).to(device), _bf16(g, d, scale=0.1).to(device)
+    listed = valid_rows(torch.tensor([int(m * valid)], dtype=torch.int32, device=device), m)
+    with torch.no_grad():
+        for fused in (True, False):
+            def call():
+                out = torch.full_like(res, 7.0)
+                if fused:
+                    return attention_out_ffn(x, wo, bo, res, wu, bu, wd, bd, norm_weight=nw, token_rows=listed, out=out)
+                return swiglu_ffn(x, wu, bu, wd, bd, residual=res, norm_weight=nw, token_rows=listed, out=out)
+            small, large = _both(test_hooks, call)
+            torch.testing.assert_close(small.float(), large.float(), rtol=2 ** -7, atol=2 ** -6)
+            assert (small[int(m * valid):] == 7.0).all()
+
+
 @pytest.mark.parametrize("batch,sequence,d_model,heads,d_ff", [(1, 20, 256, 8, 1024), (1, 480, 256, 8, 1024), (5, 90, 256, 4, 64),
                                                                (16, 120, 256, 8, 512), (3, 61, 128, 4, 256),
                                                                (32, 120, 256, 8, 512), (20, 120, 128, 4, 256), (7, 61, 256, 8, 128),
