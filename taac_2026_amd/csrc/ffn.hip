@@ -1779,7 +1779,7 @@ int norm_linear_launch(const char* name, const void* x, int64_t ldx, const void*
   p.tokens_per_sample = qk.tokens_per_sample;
   hipStream_t s = as_stream(stream);
   const bool qk_transform = qk.enabled && (qk.q_weight != nullptr || qk.cos_sin != nullptr);
-  if (dense_few_rows(M, K) && packed_weights && (norm_weight == nullptr || norm_folded))
+  if (dense_few_rows(M, K, qk_transform) && packed_weights && (norm_weight == nullptr || norm_folded))
     return norm_linear_small(p, K, qk_transform ? 2 : (qk.enabled ? 1 : 0), s, name);
   // Without a residual two token tiles per wavefront fit the register file: every weight fragment read from LDS then
   // feeds two MFMAs, which halves the LDS reads (and their share of the power budget) per token.
@@ -1942,13 +1942,15 @@ int attn_out_ffn_count(const char* name, const void* attn, const void* out_bias,
 // 25.8 and 21.6 / 21.4.
 bool ffn_few_rows(int64_t M, int32_t D) { return test_max_workgroups() == 0 && M <= (D == 256 ? 24576 : 49152); }
 
-// Whether a projection over at most M rows of D features runs as the few-token kernel. Measured for q | k | v (launches
-// back to back, few-token / persistent kernel, us): D = 256 - 512 rows 6.0 / 13.6, 4096 9.9 / 14.1, 8192 14.4 / 15.6,
-// 16384 24.5 / 21.4; D = 128 - 512 rows 3.8 / 8.7, 8192 6.3 / 9.2, 16384 9.6 / 10.4, 24576 12.6 / 12.4. With query / key norms, four
-// whole blocks: D = 256 - 8192 rows 230 / 238, 10240 330 / 332, 16384 387 / 386; D = 128 - 16384 170 / 182, 20480 222 / 213. Below the line a tile's
-// latency chain decides, above it the weights, which every 32-token workgroup fetches from L2 for itself.
-bool dense_few_rows(int64_t M, int32_t D) {
-  return test_max_workgroups() == 0 && M * D <= 10240 * 256;  // taac_test_hooks: a capped grid keeps the persistent kernels
+// Whether a projection over at most M rows of D features runs as the few-token kernel (transform: with the query / key norm weight or
+// rotation in its epilogue). One launch, few-token / persistent kernel, us, all rows valid and 55 % of them, q | k | v: D = 256 - 512 rows
+// 5.1 / 14.6, 8103 10.6 / 16.2 and 7.6 / 15.4, 16384 17.2 / 22.0 and 11.3 / 16.4, 32768 25.4 / 25.9 and 16.4 / 20.6; with the factors of the query /
+// key norms 32768 27.2 / 29.5 and 18.1 / 23.5; rotated 8103 14.9 / 19.4, 24576 32.6 / 33.4 and 20.0 / 25.6, 32768 38.8 / 35.0 and 24.8 / 27.3;
+// a residual in N = 256 32768 14.9 / 15.8. D = 128 - 512 rows 4.0 / 9.4, 49152 14.4 / 16.0 and 10.8 / 13.4, with the factors 18.8 / 18.4 and
+// 13.1 / 14.9, rotated 22.8 / 23.9 and 16.0 / 18.6; 65536 17.4 / 18.2, 23.4 / 20.7, 28.1 / 25.7. Above the line every compute unit has its tiles
+// and the persistent kernel's weights, shared through LDS, cost it less.
+bool dense_few_rows(int64_t M, int32_t D, bool transform) {
+  return test_max_workgroups() == 0 && M <= (D != 256 ? 49152 : transform ? 24576 : 32768);  // (taac_test_hooks: a capped grid)
 }
 
 // Whether the kernels take the activation's constants from the packed weights at this shape: the gated form with the

@@ -43,18 +43,29 @@ struct SmallRows {
   }
 };
 
-// [RMSNorm (weight folded) ->] linear [-> + residual], K = D, weights in fragment order. A workgroup takes 32 tokens
-// (blockIdx.x) and D output features (blockIdx.y), 64 per wavefront. QK as in norm_linear_kernel: the features of the query
+// [RMSNorm (weight folded) ->] linear [-> + residual], K = D, weights in fragment order. A workgroup holds the weights of D output
+// features (blockIdx.y), 64 per wavefront, in registers and takes the 32-token tiles blockIdx.x, + gridDim.x, ...: the grid has no more
+// workgroups than the chip has places, so that those without a tile (the number of tokens is known on the device only) do not
+// stand in front of others. The rows of a tile are loaded once, contiguous pieces by neighbouring lanes, and become
+// fragments in LDS. QK as in norm_linear_kernel: the features of the query
 // (blockIdx.y = 0) and of the key (1) leave their sum of squares behind - as the norm's factor per token in qk_rstd when that
 // is given (the workgroup holds all features of the part), per 64-feature chunk in qk_sumsq otherwise - and with QK == 2 are
 // multiplied by the norm weight and rotated. Same values as norm_linear_kernel, bit for bit (same products in the same order).
-// q | k | v of one request (512 tokens, D = 256): 6.0 us, the persistent kernel 13.6; its line is at dense_few_rows.
+// Bound by latency: count and row index -> rows -> LDS -> products -> store, 8 700 cycles of a lone workgroup; next to that a compute unit
+// pulls 128 KB of weights per workgroup. q | k | v at D = 256, us, with the rows as fragments in every wavefront, the weights in
+// front of them and a workgroup per tile / as it is: 512 rows 6.7 / 5.1, 8103 rows, 55 % valid 12.7 / 7.6, 16384 25.2 / 17.2; the lines are at
+// dense_few_rows.
 template <int D, bool RES, int QK>
 __global__ __launch_bounds__(D, 2) void norm_linear_small_kernel(const TsParams p) {
   constexpr int NW = D / kNC;  // wavefronts
   constexpr int KS = D / 16;
   constexpr int NFRAG = 2 * KS;
+  constexpr int kRow = D * 2 + 16;                      // bytes per row of the token tile
+  constexpr int kPieces = D / 8, kStep = D / kPieces;   // 16-byte pieces of a row; rows that the threads load a piece each of
+  constexpr int kPasses = 32 / kStep;
   __shared__ __attribute__((aligned(16))) uint8_t tiles[NW * kStageWave];
+  __shared__ __attribute__((aligned(16))) uint8_t x_lds[2][32 * kRow];
+  __shared__ __attribute__((aligned(16))) bf16_t bias_lds[NW][kNC];
   [[maybe_unused]] __shared__ float part_ss[NW][32];
   const int tid = threadIdx.x;
   const int wave = __builtin_amdgcn_readfirstlane(tid / kWave);
@@ -65,81 +76,61 @@ __global__ __launch_bounds__(D, 2) void norm_linear_small_kernel(const TsParams 
   const int my_chunk = part * NW + wave;
   const bool active = my_chunk < nchunks;  // N need not be a multiple of D
   const int chunk = active ? my_chunk : nchunks - 1;
+  const int piece = tid % kPieces;
 
-  // The weights depend on nothing: requested first, in flight behind the row count and the row index.
+  // Memory rows: of x for the pieces a thread loads; of out / residual for token 8 * i + lane / 8.
+  int tok0 = static_cast<int>(blockIdx.x) * 32;
+  const int stride = static_cast<int>(gridDim.x) * 32;
+  const int32_t *in_index = p.x_rows != nullptr ? p.x_rows : p.rows, *out_index = p.rows;
+  const int last = static_cast<int>(p.M) - 1;  // (few rows: 32 bits)
+  int32_t in[kPasses], out[4];
+  auto request_rows = [&](int first) {  // what lies beyond the count is not used
+#pragma unroll
+    for (int i = 0; i < kPasses; ++i) in[i] = first + i * kStep + tid / kPieces;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) out[i] = first + i * 8 + lane / 8;
+    if (in_index != nullptr) {
+#pragma unroll
+      for (int i = 0; i < kPasses; ++i) in[i] = in_index[in[i] < last ? in[i] : last];
+    }
+    if (out_index != nullptr) {
+#pragma unroll
+      for (int i = 0; i < 4; ++i) out[i] = out_index[out[i] < last ? out[i] : last];
+    }
+  };
+  request_rows(tok0);
+  const int count = static_cast<int>(token_count(p));
+  __builtin_amdgcn_sched_barrier(0);
+  // The weights depend on nothing. Half of them is in flight behind the row count and the row index, the rest behind the rows: all of
+  // them in front (64 KB per wavefront group at 64 bytes a clock) would hold the rows up.
   const char* wsrc = reinterpret_cast<const char*>(p.w1) + static_cast<int64_t>(chunk) * NFRAG * kFrag;
   bf16x8 w[NFRAG];
 #pragma unroll
-  for (int i = 0; i < NFRAG; ++i) w[i] = *reinterpret_cast<const bf16x8*>(wsrc + i * kFrag + lane * 16);
+  for (int i = 0; i < KS; ++i) w[i] = *reinterpret_cast<const bf16x8*>(wsrc + i * kFrag + lane * 16);
   __builtin_amdgcn_sched_barrier(0);
-  const int64_t tok0 = static_cast<int64_t>(blockIdx.x) * 32;
-  SmallRows<1> xr;  // memory rows: of x for token l32; of out / residual for token 8 * i + lane / 8
-  SmallRows<4> pr;
-  xr.request(p, p.x_rows != nullptr ? p.x_rows : p.rows, [&](int) { return tok0 + l32; });
-  pr.request(p, p.rows, [&](int i) { return tok0 + i * 8 + lane / 8; });
-  const int64_t count = token_count(p);
   if (tok0 >= count) return;  // whole workgroup
-  int64_t xrow[1], prow[4];
-  xr.resolve(count, xrow);
-  pr.resolve(count, prow);
-  bf16x8 xf[1][KS];
-  load_token_rows_at<D, 1>(p, xrow, hh, xf);
-  const bf16_t* bias = p.b1 != nullptr ? p.b1 + chunk * kNC : nullptr;
-  bf16x4 bv[8];
+  bf16x8 xp[kPasses];
+  auto load_rows = [&](int first) {
+    int col = piece * 8;
+    asm volatile("" : "+v"(col));
+    const int sh = p.x_plane_shift;  // feature planes: see load_token_rows_at
+    const bf16_t* base = p.x + (sh > 0 ? ((static_cast<int64_t>(col >> sh) * p.M) << sh) + (col & ((1 << sh) - 1)) : col);
+    const int64_t row_stride = sh > 0 ? static_cast<int64_t>(1) << sh : p.ldx;
 #pragma unroll
-  for (int q = 0; q < 8; ++q)
-#pragma unroll
-    for (int e = 0; e < 4; ++e) bv[q][e] = static_cast<bf16_t>(0.f);
-  if (bias != nullptr) read_chunk_bias(bias, hh, bv);
-  bf16x8 res[4];
-  if constexpr (RES) {
-#pragma unroll
-    for (int i = 0; i < 4; ++i)
-      res[i] = *reinterpret_cast<const bf16x8*>(p.residual + prow[i] * p.ldr + chunk * kNC + (lane % 8) * 8);
-  }
-
-  f32x16 acc0, acc1;
-#pragma unroll
-  for (int j = 0; j < 16; ++j) acc0[j] = acc1[j] = 0.f;
-#pragma unroll
-  for (int ks = 0; ks < KS; ++ks) {
-    acc0 = __builtin_amdgcn_mfma_f32_32x32x16_bf16(w[ks], xf[0][ks], acc0, 0, 0, 0);
-    acc1 = __builtin_amdgcn_mfma_f32_32x32x16_bf16(w[KS + ks], xf[0][ks], acc1, 0, 0, 0);
-  }
-  float rstd[1] = {1.0f};
-  if (p.norm_w != nullptr) token_rstd<D, 1>(p.eps, xf, rstd);  // the norm's weight is part of the packed layer
-  if (p.rstd_out != nullptr && part == 0 && wave == 0 && hh == 0 && tok0 + l32 < count)
-    p.rstd_out[token_row(p, count, tok0 + l32)] = rstd[0];
-
-  uint8_t* tile = tiles + wave * kStageWave;
-  [[maybe_unused]] const bool qk_part = QK != 0 && chunk < p.qk_chunks;  // the same for all wavefronts of a part
-  if constexpr (QK != 0) {
-    if (qk_part && (p.qk_sumsq != nullptr || p.qk_rstd != nullptr)) {
-      const float ss = half_wave_pair_sum(tile_to_lds_sumsq(tile, acc0, acc1, bv, l32, hh, rstd[0]));
-      if (p.qk_rstd != nullptr) {
-        if (hh == 0) part_ss[wave][l32] = ss;
-        __syncthreads();
-        if (wave == 0 && hh == 0) {
-          float total = 0.f;
-#pragma unroll
-          for (int c = 0; c < NW; ++c) total += part_ss[c][l32];
-          const int64_t tok = tok0 + l32;
-          const int64_t row = token_row(p, count, tok);
-          if (tok < count) p.qk_rstd[part * p.M + row] = rsqrtf(total * (1.0f / D) + p.qk_eps);
-        }
-      } else {
-        const int64_t row = token_row(p, count, tok0 + l32);
-        if (hh == 0 && tok0 + l32 < count) p.qk_sumsq[static_cast<int64_t>(chunk) * p.M + row] = ss;
-      }
-    } else {
-      tile_to_lds(tile, acc0, acc1, bv, l32, hh, rstd[0]);
+    for (int i = 0; i < kPasses; ++i) {
+      const int64_t row = first + i * kStep + tid / kPieces < count ? in[i] : 0;  // row 0 stands in beyond the count
+      xp[i] = *reinterpret_cast<const bf16x8*>(base + row * row_stride);
     }
-  } else {
-    tile_to_lds(tile, acc0, acc1, bv, l32, hh, rstd[0]);
-  }
-  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-  if (!active) return;  // no barrier below
+  };
+  load_rows(tok0);
+  __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+  for (int i = KS; i < NFRAG; ++i) w[i] = *reinterpret_cast<const bf16x8*>(wsrc + i * kFrag + lane * 16);
+  bf16_t* bias = bias_lds[wave];
+  bias[lane] = p.b1 != nullptr ? p.b1[chunk * kNC + lane] : static_cast<bf16_t>(0.f);
+  uint8_t* tile = tiles + wave * kStageWave;
   const int col8 = chunk * kNC + (lane % 8) * 8;
+  [[maybe_unused]] const bool qk_part = QK != 0 && chunk < p.qk_chunks;  // the same for all wavefronts of a part
   [[maybe_unused]] bf16x8 wn;
   [[maybe_unused]] bool rotate = false;
   if constexpr (QK == 2) {
@@ -149,41 +140,123 @@ __global__ __launch_bounds__(D, 2) void norm_linear_small_kernel(const TsParams 
       wn = *reinterpret_cast<const bf16x8*>(part == 0 ? p.qk_w + col8 : p.qk_wk + (col8 - D));
     rotate = qk_part && p.cos_sin != nullptr;
   }
+
+  for (int buf = 0; tok0 < count; tok0 += stride, buf ^= 1) {
+    int32_t prow[4];
 #pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const int row = i * 8 + lane / 8;
-    bf16x8 v = *reinterpret_cast<const bf16x8*>(tile + row * kStageRow + (lane % 8) * 16);
+    for (int i = 0; i < 4; ++i) prow[i] = tok0 + i * 8 + lane / 8 < count ? out[i] : 0;
+#pragma unroll
+    for (int i = 0; i < kPasses; ++i) *reinterpret_cast<bf16x8*>(x_lds[buf] + (i * kStep + tid / kPieces) * kRow + piece * 16) = xp[i];
+    bf16x8 res[4];
     if constexpr (RES) {
 #pragma unroll
-      for (int e = 0; e < 8; ++e) v[e] = static_cast<bf16_t>(static_cast<float>(v[e]) + static_cast<float>(res[i][e]));
+      for (int i = 0; i < 4; ++i)
+        res[i] = *reinterpret_cast<const bf16x8*>(p.residual + static_cast<int64_t>(prow[i]) * p.ldr + chunk * kNC + (lane % 8) * 8);
     }
-    if constexpr (QK == 2) {
-      if (qk_part) {
-        float f[8];
+    __syncthreads();  // (two tiles in turn: whoever writes the next one has seen everybody leave the one before)
+    f32x16 acc0, acc1;
 #pragma unroll
-        for (int e = 0; e < 8; ++e) f[e] = static_cast<float>(v[e]) * static_cast<float>(wn[e]);
-        if (rotate) {
-          const int pos = static_cast<int>(input_row(p, count, tok0 + row) % p.tokens_per_sample);
-          const bf16x8 cs = *reinterpret_cast<const bf16x8*>(p.cos_sin + static_cast<int64_t>(pos) * p.head_dim + col8 % p.head_dim);
+    for (int j = 0; j < 16; ++j) acc0[j] = acc1[j] = 0.f;
+    typedef __attribute__((__vector_size__(2 * sizeof(__bf16)))) __bf16 bf16x2;
+    float rstd = 1.0f, norm_ss = 0.f;
+    constexpr int kAhead = 4;  // fragments in flight (all of them do not fit next to the weights)
+    auto fragment = [&](int ks) { return *reinterpret_cast<const bf16x8*>(x_lds[buf] + l32 * kRow + (ks * 16 + hh * 8) * 2); };
+    bf16x8 xf[kAhead];
 #pragma unroll
-          for (int e = 0; e < 8; e += 2) {
-            const float even = f[e], odd = f[e + 1];
-            const float cv = static_cast<float>(cs[e]), sv = static_cast<float>(cs[e + 1]);
-            f[e] = even * cv - odd * sv;
-            f[e + 1] = even * sv + odd * cv;
+    for (int ks = 0; ks < kAhead; ++ks) xf[ks] = fragment(ks);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks) {
+      const bf16x8 x = xf[ks % kAhead];
+      if (ks + kAhead < KS) xf[ks % kAhead] = fragment(ks + kAhead);
+      acc0 = __builtin_amdgcn_mfma_f32_32x32x16_bf16(w[ks], x, acc0, 0, 0, 0);
+      acc1 = __builtin_amdgcn_mfma_f32_32x32x16_bf16(w[KS + ks], x, acc1, 0, 0, 0);
+#pragma unroll
+      for (int e = 0; e < 8; e += 2) {  // as token_rstd
+        const bf16x2 pair = {x[e], x[e + 1]};
+        norm_ss = __builtin_amdgcn_fdot2_f32_bf16(pair, pair, norm_ss, false);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    if (p.norm_w != nullptr) {  // the norm's weight is part of the packed layer
+      norm_ss += __shfl_xor(norm_ss, 32, kWave);
+      rstd = rsqrtf(norm_ss * (1.0f / D) + p.eps);
+    }
+    if (p.rstd_out != nullptr && part == 0 && wave == 0 && hh == 0 && tok0 + l32 < count)
+      p.rstd_out[token_row(p, count, tok0 + l32)] = rstd;
+
+    bf16x4 bv[8];
+    read_chunk_bias(bias, hh, bv);
+    if constexpr (QK != 0) {
+      if (qk_part && (p.qk_sumsq != nullptr || p.qk_rstd != nullptr)) {
+        const float ss = half_wave_pair_sum(tile_to_lds_sumsq(tile, acc0, acc1, bv, l32, hh, rstd));
+        if (p.qk_rstd != nullptr) {
+          if (hh == 0) part_ss[wave][l32] = ss;
+          __syncthreads();
+          if (wave == 0 && hh == 0) {
+            float total = 0.f;
+#pragma unroll
+            for (int c = 0; c < NW; ++c) total += part_ss[c][l32];
+            const int64_t tok = tok0 + l32;
+            const int64_t row = token_row(p, count, tok);
+            if (tok < count) p.qk_rstd[part * p.M + row] = rsqrtf(total * (1.0f / D) + p.qk_eps);
+          }
+        } else {
+          const int64_t row = token_row(p, count, tok0 + l32);
+          if (hh == 0 && tok0 + l32 < count) p.qk_sumsq[static_cast<int64_t>(chunk) * p.M + row] = ss;
+        }
+      } else {
+        tile_to_lds(tile, acc0, acc1, bv, l32, hh, rstd);
+      }
+    } else {
+      tile_to_lds(tile, acc0, acc1, bv, l32, hh, rstd);
+    }
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    if (active) {
+      int col = col8;
+      asm volatile("" : "+v"(col));  // (addresses formed ahead of the loop would be spilled)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const int row = i * 8 + lane / 8;
+        bf16x8 v = *reinterpret_cast<const bf16x8*>(tile + row * kStageRow + (lane % 8) * 16);
+        if constexpr (RES) {
+#pragma unroll
+          for (int e = 0; e < 8; ++e) v[e] = static_cast<bf16_t>(static_cast<float>(v[e]) + static_cast<float>(res[i][e]));
+        }
+        if constexpr (QK == 2) {
+          if (qk_part) {
+            float f[8];
+#pragma unroll
+            for (int e = 0; e < 8; ++e) f[e] = static_cast<float>(v[e]) * static_cast<float>(wn[e]);
+            if (rotate) {
+              const int pos = static_cast<int>(input_row(p, count, tok0 + row) % p.tokens_per_sample);
+              const bf16x8 cs = *reinterpret_cast<const bf16x8*>(p.cos_sin + static_cast<int64_t>(pos) * p.head_dim + col % p.head_dim);
+#pragma unroll
+              for (int e = 0; e < 8; e += 2) {
+                const float even = f[e], odd = f[e + 1];
+                const float cv = static_cast<float>(cs[e]), sv = static_cast<float>(cs[e + 1]);
+                f[e] = even * cv - odd * sv;
+                f[e + 1] = even * sv + odd * cv;
+              }
+            }
+#pragma unroll
+            for (int e = 0; e < 8; ++e) v[e] = static_cast<bf16_t>(f[e]);
           }
         }
-#pragma unroll
-        for (int e = 0; e < 8; ++e) v[e] = static_cast<bf16_t>(f[e]);
+        if (tok0 + row >= count) continue;
+        // feature planes: column c lies in plane c >> shift, at c % 2^shift of the row
+        const int64_t at = p.out_plane_shift > 0
+                               ? (((static_cast<int64_t>(col >> p.out_plane_shift) * p.M + prow[i]) << p.out_plane_shift) +
+                                  (col & ((1 << p.out_plane_shift) - 1)))
+                               : static_cast<int64_t>(prow[i]) * p.ldo + col;
+        *reinterpret_cast<bf16x8*>(p.out + at) = v;
       }
     }
-    if (tok0 + row >= count) continue;
-    // feature planes: column col8 lies in plane col8 >> shift, at col8 % 2^shift of the row
-    const int64_t at = p.out_plane_shift > 0
-                           ? (((static_cast<int64_t>(col8 >> p.out_plane_shift) * p.M + prow[i]) << p.out_plane_shift) +
-                              (col8 & ((1 << p.out_plane_shift) - 1)))
-                           : prow[i] * p.ldo + col8;
-    *reinterpret_cast<bf16x8*>(p.out + at) = v;
+    // (not a tile ahead: next to the weights there are no registers for the rows, and reloads of spilled ones wait for all loads)
+    if (tok0 + stride < count) {
+      request_rows(tok0 + stride);
+      load_rows(tok0 + stride);
+    }
   }
 }
 
@@ -754,7 +827,10 @@ int64_t ffn_split_bytes(int64_t M, int32_t D, int32_t F) {
 }
 
 int norm_linear_small(const TsParams& p, int32_t K, int qk_mode, hipStream_t s, const char* name) {
-  const dim3 grid(static_cast<uint32_t>((p.M + 31) / 32), static_cast<uint32_t>((p.N + K - 1) / K));
+  // Places for workgroups: two per compute unit at K = 256 (registers), six at 128.
+  const int64_t tiles = (p.M + 31) / 32, parts = (p.N + K - 1) / K, places = static_cast<int64_t>(compute_units()) * (K == 256 ? 2 : 6);
+  const int64_t columns = places / parts > 0 ? places / parts : 1;
+  const dim3 grid(static_cast<uint32_t>(tiles < columns ? tiles : columns), static_cast<uint32_t>(parts));
 #define TAAC_SMALL(KK, RR, QQ)                                                                    \
   do {                                                                                            \
     hipLaunchKernelGGL((norm_linear_small_kernel<KK, RR, QQ>), grid, dim3(KK), 0, s, p);          \

@@ -71,6 +71,27 @@ def test_query_key_epilogue_equals_the_persistent_kernel(device, test_hooks, d_m
                 assert torch.equal(small, large)
 
 
+@pytest.mark.parametrize("m,k,heads,valid", [(5475, 256, 8, 1.0), (12001, 256, 4, 0.7), (16417, 128, 4, 1.0), (32768, 256, 8, 0.3)])
+def test_projection_of_several_tiles_per_workgroup(device, test_hooks, m, k, heads, valid):
+    """More tiles than columns of workgroups (two workgroups per compute unit and part at K = 256, six at 128), or columns beyond
+    the valid tokens: bit for bit the persistent kernel's rows, and no others written."""
+    g = torch.Generator().manual_seed(m)
+    x, w, b = _bf16(g, 1, m, k).to(device), _bf16(g, 3 * k, k, scale=k ** -0.5).to(device), _bf16(g, 3 * k).to(device)
+    nw, res = (1 + _bf16(g, k, scale=0.1)).to(device), _bf16(g, m, 3 * k).to(device)
+    rows = valid_rows(torch.tensor([int(m * valid)], dtype=torch.int32, device=device), m)
+    with torch.no_grad():
+        def call():
+            blank = torch.full((m, 3 * k), 7.0, dtype=torch.bfloat16, device=device)
+            qk = qkv_projection(x, w, b, num_heads=heads, norm_weight=nw, query_weight=nw, key_weight=nw, rope_base=1e4, token_rows=rows,
+                                out=blank.clone())
+            return [norm_linear(x[0], w, b, norm_weight=nw, token_rows=rows, out=blank.clone()),
+                    norm_linear(x[0], w, b, residual=res, token_rows=rows, out=blank.clone()), *(t for t in qk if t is not None)]
+        small, large = _both(test_hooks, call)
+        for a, c in zip(small, large):
+            assert torch.equal(a, c)
+        assert (small[0][int(m * valid):] == 7.0).all()
+
+
 @pytest.mark.parametrize("m,d,f", [(1, 256, 32), (33, 128, 32), (31, 256, 96), (64, 128, 512), (100, 256, 1024), (8192, 256, 64)])
 @pytest.mark.parametrize("gate_first", [True, False])
 def test_feed_forward_matches_the_persistent_kernel(device, test_hooks, m, d, f, gate_first):
