@@ -96,15 +96,16 @@ __device__ __forceinline__ uint32_t pack2(T lo, T hi) {
 //   rows as MFMA A operands (lane l32 reads one piece of row l32: 16 consecutive rows of one piece cover all banks);
 //   columns as MFMA A operands through ds_read_b64_tr_b16: a 16-lane group reads 32 contiguous bytes of four
 //   consecutive rows and every lane receives four rows of one feature (see streamed_column_offset below).
-// +32 rows leave the swizzle unchanged, +16 rows too, +8 rows flip kSwizzleBit8 of it.
+// +32 rows leave the swizzle unchanged, +16 rows too, +8 rows flip SwizzleStep::kRows8 of the address. Four rows further it is another
+// pair of pieces, for the transposed reads of eight consecutive rows (attn_bwd_fused_kernel's dQ).
 template <int DP>
 __device__ __forceinline__ int row_swizzle(int r) {
   static_assert(DP == 32 || DP == 64, "row swizzles are written for 64- and 128-byte rows");
-  return DP == 32 ? (r >> 2) & 3 : ((r >> 1) & 7) ^ (((r >> 1) & 1) << 2);
+  return DP == 32 ? ((r >> 1) & 2) | ((r >> 3) & 1) : ((r >> 1) & 7) ^ (((r >> 1) & 1) << 2);
 }
 template <int DP>
 struct SwizzleStep {
-  static constexpr uint32_t kRows8 = (DP == 32 ? 2 : 4) * 16;  // address bits that +8 rows flip
+  static constexpr uint32_t kRows8 = (DP == 32 ? 1 : 4) * 16;  // address bits that +8 rows flip
 };
 
 // Staging of one streamed operand. DMA: the chunk goes from global memory straight into LDS (one 1 KB transfer per
@@ -718,6 +719,29 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu((DP ==
   store_owned<T, DP>(dvacc, tile, dvb, p.dvs[2], k_begin + wave * 32, k_store_end, p.d, lane);
 }
 
+// A transposed read (lds_read_tr16) that the compiler waits for.
+template <typename T>
+__device__ __forceinline__ typename Vec8<T>::half_type read_tr16(uint32_t addr) {
+  typedef short s16x4 __attribute__((ext_vector_type(4)));
+  typedef __attribute__((address_space(3))) s16x4* lds_ptr;
+  return __builtin_bit_cast(typename Vec8<T>::half_type, __builtin_amdgcn_ds_read_tr16_b64_v4i16(reinterpret_cast<lds_ptr>(addr)));
+}
+
+// The fragments of read_columns, awaited by the compiler.
+template <typename T, int DP>
+__device__ __forceinline__ void fetch_columns(typename Vec8<T>::half_type (&frag)[2][2], uint32_t addr) {
+#pragma unroll
+  for (int s2 = 0; s2 < 2; ++s2) {
+    frag[s2][0] = read_tr16<T>(addr + s2 * (16 * DP * 2));
+    frag[s2][1] = read_tr16<T>((addr ^ SwizzleStep<DP>::kRows8) + s2 * (16 * DP * 2) + 8 * DP * 2);
+  }
+}
+
+template <typename H>
+__device__ __forceinline__ auto join(H lo, H hi) {
+  return __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
+}
+
 template <typename T>
 struct Mfma16;
 template <>
@@ -748,6 +772,14 @@ struct Mfma16<f16_t> {
 // other. Two wavefronts a SIMD instead of three leave the registers for it: with three, 16 to 36 of them are spilled (256 rows, 8192 pairs
 // of 32 features 340 instead of 290 us; 64 rows of 64 features 192 instead of 123). One dP and the scale at the end moved dK, at d = 64 dQ,
 // by roundings: 312 and 133 us there, with three wavefronts.
+// A pair of tiles is some 490 cycles of vector instructions and 320 of products, but also a chain from LDS reads to products to exponentials to
+// products, which two or three wavefronts a SIMD do not cover. Left alone, the compiler puts each read in front of the instruction that takes
+// it: nine memory latencies per pair. With 32 features the operands, the rows' values and the columns of the second products are therefore
+// requested behind scheduling fences ahead of their use, and dQ's contraction requests the next two tiles in front of the products of two (as
+// nested branches: one behind the other they hold both groups' registers across all of them, and spill). 64 features leave the registers for
+// the rows' values alone, and without mask bits. K's and dS's pieces lie so that a transposed read has no two lanes on one bank (both had two, a
+// quarter of the LDS cycles). 1024 x 8 x 512 x 32, lengths ~ U{64..512} 718 -> 670 us, all 512 1215 -> 1115, causal (600 samples) 297 -> 272;
+// 1024 x 8 x 256 x 32 203 -> 191; 2048 x 4 x 256 x 64 369 -> 353; 110 rows of 64 151 -> 146.
 template <int DP, int NT, bool BITS>
 struct FusedLayout {
   static constexpr int kRows = 32;                                     // streamed queries per step
@@ -759,6 +791,9 @@ struct FusedLayout {
   static constexpr int STAT_BYTES = (BITS ? 3 : 2) * kTiles * kRows * 4;  // log-sum-exp and -D / sqrt(d) of every query; -D
   static constexpr int BYTES = K_BYTES + DS_BYTES + 2 * BUF_BYTES + STAT_BYTES;
   static constexpr int kWavesPerSimd = NT * DP == 128 || BITS ? 2 : 3;
+  // What a pair of tiles reads from LDS is requested ahead of its use, as far as the registers go (see the loop over the tiles).
+  static constexpr bool kOperandsAhead = DP == 32;
+  static constexpr bool kRowsAhead = DP == 32 || (NT == 2 && !BITS);
 };
 
 template <typename T, int DP, int NT, int MODE, bool COMPACT>
@@ -799,7 +834,7 @@ void attn_bwd_fused_kernel(const AttnBwdParams p) {
   const int q_valid = p.zero_pad ? (len < p.Tq ? len : p.Tq) : p.Tq;
   // The wavefront's key tiles are own, own + 4, ...: with a number of tiles that 4 does not divide the wavefronts with one tile more
   // lie on other SIMDs in other workgroups.
-  const int own = (wave + bh + bh / 32) % (kThreads / kWave);
+  const int own = __builtin_amdgcn_readfirstlane((wave + bh + bh / 32) % (kThreads / kWave));
   const int n_tiles = (len + 31) / 32;           // at most L::kTiles: the host checks Tk
   const int q_end = n_tiles > 0 ? q_valid : 0;   // rows of dQ at or beyond it are zero
   const float c = p.scale * 1.4426950408889634f;
@@ -909,8 +944,9 @@ void attn_bwd_fused_kernel(const AttnBwdParams p) {
 
     const uint32_t row_off = streamed_row_offset<DP>(l32, hh);
     const uint32_t col_off = streamed_column_offset<DP>(lane);
-    // dS in LDS: rows of 32 queries per key, the 8-byte piece x of key r at x ^ (r / 4) % 8 - writes of one piece by 32 keys and the
-    // transposed reads below cover the banks evenly.
+    // dS in LDS: rows of 32 queries per key, the 8-byte piece x of key r at x ^ ds_swizzle(r): one piece of 32 keys (a write) and four
+    // pieces of eight consecutive keys (half of a transposed read below) cover all 64 banks.
+    auto ds_swizzle = [](int r) { return ((r >> 3) & 3) | (r & 4); };
     const uint32_t ds_write = static_cast<uint32_t>(l32 * 64);
     const int g16 = lane / 16, i16 = lane % 16, q_half = wave % 2, d_col = wave / 2;
     uint32_t ds_read[2], k_read[2];
@@ -920,7 +956,7 @@ void attn_bwd_fused_kernel(const AttnBwdParams p) {
       // product's terms in theirs)
       const int key = 16 * (g16 / 2) + 4 * (g16 % 2) + 8 * half + i16 / 4;
       const int piece = 4 * q_half + i16 % 4;        // four queries
-      ds_read[half] = lds_offset(ds_image) + static_cast<uint32_t>(key * 64 + ((piece ^ (key / 4)) * 8));
+      ds_read[half] = lds_offset(ds_image) + static_cast<uint32_t>(key * 64 + ((piece ^ ds_swizzle(key)) * 8));
       const int piece16 = 2 * d_col + (i16 % 4) / 2;  // eight features
       k_read[half] = lds_offset(k_image) + static_cast<uint32_t>(key * ROWB + ((piece16 ^ row_swizzle<DP>(key)) * 16) + (i16 % 2) * 8);
     }
@@ -949,18 +985,27 @@ void attn_bwd_fused_kernel(const AttnBwdParams p) {
         f32x16 sacc, dpacc;
 #pragma unroll
         for (int j = 0; j < 16; ++j) sacc[j] = dpacc[j] = 0.f;
+        vec_t qa[KSTEPS], kf[KSTEPS], da[KSTEPS];
 #pragma unroll
         for (int s = 0; s < KSTEPS; ++s) {
-          const uint32_t off = row_off ^ (s * 32);
-          const vec_t qa = *reinterpret_cast<const vec_t*>(chunk + off);
-          const vec_t kf = *reinterpret_cast<const vec_t*>(k_image + tile * TILE_BYTES + off);
-          sacc = Mfma32<T>::run(qa, kf, sacc);
+          qa[s] = *reinterpret_cast<const vec_t*>(chunk + (row_off ^ (s * 32)));
+          kf[s] = *reinterpret_cast<const vec_t*>(k_image + tile * TILE_BYTES + (row_off ^ (s * 32)));
         }
 #pragma unroll
-        for (int s = 0; s < KSTEPS; ++s) {
-          const vec_t da = *reinterpret_cast<const vec_t*>(chunk + TILE_BYTES + (row_off ^ (s * 32)));
-          dpacc = Mfma32<T>::run(da, vf[t][s], dpacc);
-        }
+        for (int s = 0; s < KSTEPS; ++s) da[s] = *reinterpret_cast<const vec_t*>(chunk + TILE_BYTES + (row_off ^ (s * 32)));
+        f32x4 l4[2], d4[2];
+        [[maybe_unused]] u32x4 w4[2];
+        auto row_values = [&](int jq) {  // of the four queries of the accumulators' quarter jq
+          l4[jq % 2] = *reinterpret_cast<const f32x4*>(&s_lse[jq * 8 + hh * 4]);
+          d4[jq % 2] = *reinterpret_cast<const f32x4*>(&s_delta[jq * 8 + hh * 4]);
+          if (BITS) w4[jq % 2] = *reinterpret_cast<const u32x4*>(&s_words[tile * kRows + jq * 8 + hh * 4]);
+        };
+        if (L::kRowsAhead) row_values(0);
+        if (L::kOperandsAhead) __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int s = 0; s < KSTEPS; ++s) sacc = Mfma32<T>::run(qa[s], kf[s], sacc);
+#pragma unroll
+        for (int s = 0; s < KSTEPS; ++s) dpacc = Mfma32<T>::run(da[s], vf[t][s], dpacc);
         const int key = tile * 32 + l32;
         // pairs that do not exist get a score of -inf; only the tile at the end of the keys and the one on the causal diagonal test
         if (tile * 32 + 32 > len || (BITS && p.key_valid != nullptr)) {  // wavefront-uniform
@@ -974,20 +1019,26 @@ void attn_bwd_fused_kernel(const AttnBwdParams p) {
           for (int j = 0; j < 16; ++j) sacc[j] = first > (j / 4) * 8 + (j % 4) ? -INFINITY : sacc[j];
         }
         vec_t pb[2], dsb[2];
+        [[maybe_unused]] vec4_t fd[2][2], fq[2][2];  // columns of dO and Q: the operands of dV and dK
 #pragma unroll
         for (int jq = 0; jq < 4; ++jq) {
-          const f32x4 l4 = *reinterpret_cast<const f32x4*>(&s_lse[jq * 8 + hh * 4]);
-          const f32x4 d4 = *reinterpret_cast<const f32x4*>(&s_delta[jq * 8 + hh * 4]);
-          [[maybe_unused]] u32x4 w4 = {0u, 0u, 0u, 0u};
-          if (BITS) w4 = *reinterpret_cast<const u32x4*>(&s_words[tile * kRows + jq * 8 + hh * 4]);
+          if (!L::kRowsAhead)
+            row_values(jq);
+          else if (jq < 3)
+            row_values(jq + 1);
+          if (L::kOperandsAhead && !BITS) {
+            if (jq == 2) fetch_columns<T, DP>(fd, col_addr + TILE_BYTES);
+            if (jq == 3) fetch_columns<T, DP>(fq, col_addr);
+          }
+          if (L::kRowsAhead) __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
           for (int e = 0; e < 4; ++e) {
             const int j = jq * 4 + e;
-            float prob = __builtin_amdgcn_exp2f(fmaf(sacc[j], c, -l4[e]));
+            float prob = __builtin_amdgcn_exp2f(fmaf(sacc[j], c, -l4[jq % 2][e]));
             if (BITS)  // all ones where the word has the lane's bit
-              prob = __builtin_bit_cast(float, __builtin_bit_cast(uint32_t, prob) & __builtin_amdgcn_sbfe(w4[e], l32, 1));
+              prob = __builtin_bit_cast(float, __builtin_bit_cast(uint32_t, prob) & __builtin_amdgcn_sbfe(w4[jq % 2][e], l32, 1));
             pb[j / 8][j % 8] = static_cast<T>(prob);
-            dsb[j / 8][j % 8] = static_cast<T>(prob * fmaf(dpacc[j], p.scale, d4[e]));
+            dsb[j / 8][j % 8] = static_cast<T>(prob * fmaf(dpacc[j], p.scale, d4[jq % 2][e]));
             if (BITS) sacc[j] = prob;
           }
         }
@@ -997,7 +1048,7 @@ void attn_bwd_fused_kernel(const AttnBwdParams p) {
           vec4_t quad;
 #pragma unroll
           for (int e = 0; e < 4; ++e) quad[e] = dsb[jq / 2][(jq % 2) * 4 + e];
-          *reinterpret_cast<vec4_t*>(ds_tile + ((2 * jq + hh) ^ (l32 / 4)) * 8) = quad;
+          *reinterpret_cast<vec4_t*>(ds_tile + ((2 * jq + hh) ^ ds_swizzle(l32)) * 8) = quad;
         }
         if constexpr (BITS) {  // dK's dS: the products start from -D, 1 / sqrt(d) comes at the end (fp16: before the rounding)
 #pragma unroll
@@ -1008,55 +1059,65 @@ void attn_bwd_fused_kernel(const AttnBwdParams p) {
           }
 #pragma unroll
           for (int s = 0; s < KSTEPS; ++s) {
-            const vec_t da = *reinterpret_cast<const vec_t*>(chunk + TILE_BYTES + (row_off ^ (s * 32)));
-            dpacc = Mfma32<T>::run(da, vf[t][s], dpacc);
+            const vec_t again = *reinterpret_cast<const vec_t*>(chunk + TILE_BYTES + (row_off ^ (s * 32)));
+            dpacc = Mfma32<T>::run(again, vf[t][s], dpacc);
           }
 #pragma unroll
           for (int j = 0; j < 16; ++j) dsb[j / 8][j % 8] = static_cast<T>(sacc[j] * (LATE_SCALE ? dpacc[j] : dpacc[j] * p.scale));
         }
-        accumulate_columns2<T, DP, 0>(dvacc[t], pb, col_addr + TILE_BYTES, dkacc[t], dsb, col_addr);
+        if constexpr (!L::kOperandsAhead) {
+          accumulate_columns2<T, DP, 0>(dvacc[t], pb, col_addr + TILE_BYTES, dkacc[t], dsb, col_addr);
+        } else {
+          if (BITS) {
+            fetch_columns<T, DP>(fd, col_addr + TILE_BYTES);
+            fetch_columns<T, DP>(fq, col_addr);
+          }
+#pragma unroll
+          for (int s2 = 0; s2 < 2; ++s2) {
+            dvacc[t][0] = Mfma32<T>::run(join(fd[s2][0], fd[s2][1]), pb[s2], dvacc[t][0]);
+            dkacc[t][0] = Mfma32<T>::run(join(fq[s2][0], fq[s2][1]), dsb[s2], dkacc[t][0]);
+          }
+        }
       });
       __syncthreads();  // the dS tiles of every wavefront are in LDS
       f32x4 dqacc[MB];
 #pragma unroll
       for (int m = 0; m < MB; ++m) dqacc[m] = f32x4{0.f, 0.f, 0.f, 0.f};
-      auto contract = [&](int tile, auto n_tag) {  // key tiles tile .. tile + n - 1
-        constexpr int n = decltype(n_tag)::value;
-        u32x2 fs[n][2], fk[n][MB][2];
-        const uint32_t ds0 = ds_read[0] + tile * (kRows * 64), ds1 = ds_read[1] + tile * (kRows * 64);
-        const uint32_t k0 = k_read[0] + tile * TILE_BYTES, k1 = k_read[1] + tile * TILE_BYTES;
-        static_for<n>([&](auto i_tag) {
-          constexpr int i = decltype(i_tag)::value;
-          lds_read_tr16<i * kRows * 64>(fs[i][0], ds0);
-          lds_read_tr16<i * kRows * 64>(fs[i][1], ds1);
-          static_for<MB>([&](auto m_tag) {
-            constexpr int m = decltype(m_tag)::value;
-            lds_read_tr16<i * TILE_BYTES>(fk[i][m][0], k0 ^ (m * 64));
-            lds_read_tr16<i * TILE_BYTES>(fk[i][m][1], k1 ^ (m * 64));
-          });
-        });
-        static_for<n>([&](auto i_tag) {
-          constexpr int i = decltype(i_tag)::value;
-          constexpr int kLater = (n - 1 - i) * (2 + 2 * MB), kLeft = kLater < 15 ? kLater : 15;  // 4-bit count
-          if constexpr (MB == 1)
-            asm volatile("s_waitcnt lgkmcnt(%4)" : "+v"(fs[i][0]), "+v"(fs[i][1]), "+v"(fk[i][0][0]), "+v"(fk[i][0][1]) : "n"(kLeft) : "memory");
-          else
-            asm volatile("s_waitcnt lgkmcnt(%6)"
-                         : "+v"(fs[i][0]), "+v"(fs[i][1]), "+v"(fk[i][0][0]), "+v"(fk[i][0][1]), "+v"(fk[i][MB - 1][0]), "+v"(fk[i][MB - 1][1])
-                         : "n"(kLeft) : "memory");
-          const u32x4 sbits = {fs[i][0][0], fs[i][0][1], fs[i][1][0], fs[i][1][1]};
+      // In groups of key tiles, the next group's operands requested in front of this group's products. What lies beyond the last tile
+      // is read (the images have kTiles tiles) but not multiplied.
+      constexpr int kGroup = 2 / MB, kGroups = L::kTiles / kGroup;
+      vec4_t fs[2][kGroup][2], fk[2][kGroup][MB][2];
+      auto fetch_group = [&](auto g_tag) {
+        constexpr int g = decltype(g_tag)::value;
+#pragma unroll
+        for (int i = 0; i < kGroup; ++i) {
+          constexpr int first = g * kGroup;
+          fs[g % 2][i][0] = read_tr16<T>(ds_read[0] + (first + i) * (kRows * 64));
+          fs[g % 2][i][1] = read_tr16<T>(ds_read[1] + (first + i) * (kRows * 64));
 #pragma unroll
           for (int m = 0; m < MB; ++m) {
-            const u32x4 kbits = {fk[i][m][0][0], fk[i][m][0][1], fk[i][m][1][0], fk[i][m][1][1]};
-            dqacc[m] = Mfma16<T>::run(__builtin_bit_cast(vec_t, kbits), __builtin_bit_cast(vec_t, sbits), dqacc[m]);
+            fk[g % 2][i][m][0] = read_tr16<T>((k_read[0] ^ (m * 64)) + (first + i) * TILE_BYTES);
+            fk[g % 2][i][m][1] = read_tr16<T>((k_read[1] ^ (m * 64)) + (first + i) * TILE_BYTES);
           }
-        });
+        }
       };
-      int tile = 0;
-      if constexpr (MB == 1)
-        for (; tile + 4 <= tiles; tile += 4) contract(tile, std::integral_constant<int, 4>{});
-      for (; tile + 2 <= tiles; tile += 2) contract(tile, std::integral_constant<int, 2>{});
-      if (tiles & 1) contract(tile, std::integral_constant<int, 1>{});
+      fetch_group(std::integral_constant<int, 0>{});
+      auto contract = [&](auto self, auto g_tag) -> void {
+        constexpr int g = decltype(g_tag)::value;
+        if constexpr (g + 1 < kGroups) fetch_group(std::integral_constant<int, g + 1>{});
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int i = 0; i < kGroup; ++i)
+          if (i == 0 || g * kGroup + i < tiles) {
+#pragma unroll
+            for (int m = 0; m < MB; ++m)
+              dqacc[m] = Mfma16<T>::run(join(fk[g % 2][i][m][0], fk[g % 2][i][m][1]), join(fs[g % 2][i][0], fs[g % 2][i][1]), dqacc[m]);
+          }
+        if constexpr (g + 1 < kGroups) {
+          if ((g + 1) * kGroup < tiles) self(self, std::integral_constant<int, g + 1>{});
+        }
+      };
+      contract(contract, std::integral_constant<int, 0>{});
       vm_wait<0>();  // the next chunk's transfers, before this chunk's stores join the queue
       const int q_row = qc0 + 16 * q_half + i16;
       if (q_row < q_valid) {

@@ -306,6 +306,24 @@ def test_one_workgroup_rounds_as_the_two_kernels_do(device, rows, dim, batch, he
         assert torch.equal(a, b), name
 
 
+@pytest.mark.parametrize("rows,dim,batch,heads", [(512, 32, 192, 8), (256, 32, 64, 8), (256, 64, 128, 4), (128, 64, 8, 4)])
+@pytest.mark.parametrize("causal", [False, True])
+def test_one_workgroup_with_every_number_of_key_tiles(device, rows, dim, batch, heads, causal):
+    """Lengths over the whole range, on both sides of every key tile's edge: groups of tiles that are whole, half or not there."""
+    g = torch.Generator(device=device).manual_seed(rows + causal)
+    q, k, v, grad_out = (torch.randn(batch, heads, rows, dim, generator=g, device=device).to(torch.bfloat16) for _ in range(4))
+    edges = torch.arange(32, rows + 1, 32, device=device)
+    edges = torch.cat([edges, edges - 31, (edges + 1).clamp_max(rows), edges - 1])
+    lengths = edges[torch.arange(batch, device=device) % edges.numel()].to(torch.int32)
+    index = torch.arange(rows, device=device)
+    inside = index < lengths[:, None]
+    seen = inside[:, None, :] & inside[:, :, None] & ((index[None, :] <= index[:, None]) | (not causal))
+    lse, p = _log_sum_exp(q, k, seen[:, None])
+    args = (q, k, v, (p @ v.double()).to(torch.bfloat16), grad_out, lse.float().contiguous(), lengths, causal, True)
+    for name, a, b in zip(("dq", "dk", "dv"), _native_backward(*args), _native_backward(*args, staged=True)):
+        assert torch.equal(a, b), name
+
+
 @pytest.mark.parametrize("dtype,rows,dim,batch,heads,part", [
     (torch.bfloat16, 129, 32, 64, 8, 63), (torch.float16, 256, 32, 64, 8, 21), (torch.bfloat16, 250, 64, 130, 4, 65),
     (torch.float16, 160, 64, 130, 4, 65), (torch.bfloat16, 64, 32, 388, 4, 194), (torch.bfloat16, 97, 32, 260, 8, 52)])
