@@ -26,7 +26,7 @@ from taac_2026_amd.accelerators.linear import (attention_out_ffn, front_rows, no
                                                swiglu_ffn, swiglu_ffn_backward_supported, swiglu_ffn_dropout, valid_rows)
 from taac_2026_amd.accelerators.tensor_validation import require_cuda_tensors, require_inference
 from taac_2026_amd.modeling.block_training import (InteractionStackFunction, _block_config, block_form, _block_parameters, _called_plainly,
-                                                   run_training_block, run_training_stack, _addresses, training_route_applies,
+                                                   _every_parameter, _held, _part, run_training_block, run_training_stack, _addresses, training_route_applies,
                                                    uniform_parameters)
 from taac_2026_amd.modeling.normalization import RMSNorm
 from taac_2026_amd.modeling.sequence import scaled_dot_product_attention
@@ -39,20 +39,6 @@ def _bf16(parameter: torch.Tensor | None) -> torch.Tensor | None:
     if parameter is None:
         return None
     return parameter if parameter.dtype == torch.bfloat16 else parameter.to(torch.bfloat16)
-
-
-def _part(block: nn.Module, name: str) -> nn.Module | None:
-    """``getattr(block, name)`` of a submodule, by its registry where it is there (attribute lookups on modules are most of what the
-    host does in ``PCVRBackbone.forward``)."""
-    return block._modules[name] if name in block._modules else getattr(block, name)
-
-
-def _held(module: nn.Module | None, name: str) -> torch.Tensor | None:
-    """``getattr(module, name)`` of a parameter, by its registry where it is there. It is not where the value is computed or a view
-    that a wrapper puts in its place (parametrisations, weight norm, flattened shards, data-parallel replicas)."""
-    if module is None:
-        return None
-    return module._parameters[name] if name in module._parameters else getattr(module, name)
 
 
 def _compute_dtype(tokens: torch.Tensor) -> torch.dtype:
@@ -316,7 +302,7 @@ class UnifiedInteractionBlock(nn.Module):
             return False
         if self.training and (self.attention.dropout > 0.0 or self.ffn.dropout.p > 0.0):
             return False
-        return not (torch.is_grad_enabled() and (tokens.requires_grad or any(p.requires_grad for p in self.parameters())))
+        return not (torch.is_grad_enabled() and (tokens.requires_grad or any(p.requires_grad for p in _every_parameter(self))))
 
     def _front_layout(self, structured, padding_mask: torch.Tensor, token_count: int) -> bool:
         """Whether the fused route under this mask (and no key lengths) moves every sample's valid tokens to the front."""

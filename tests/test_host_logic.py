@@ -289,3 +289,26 @@ def test_a_block_loop_takes_any_iterable():
     tokens = torch.zeros(1, 2, 4)
     out = api.run_interaction_blocks((block for _ in range(3)), tokens, torch.zeros(1, 2, dtype=torch.bool), None)
     assert torch.equal(out, tokens + 3) and [call["inplace"] for call in calls] == [False, True, True]
+
+
+@pytest.mark.parametrize("changed", ["as built", "parametrised", "shared norm", "no bias"])
+def test_block_parameters_are_the_attributes_values(changed):
+    """The lists that a call takes off a block's registries hold what the attributes give."""
+    from taac_2026_amd.modeling.backbone import UnifiedInteractionBlock
+    from taac_2026_amd.modeling.block_training import _block_config, _block_parameters, _every_parameter
+
+    block = UnifiedInteractionBlock(128, 4, 2, qk_norm=True)
+    if changed == "parametrised":
+        torch.nn.utils.parametrizations.weight_norm(block.attention.qkv)
+    elif changed == "shared norm":
+        block.ffn_norm = block.attn_norm
+    elif changed == "no bias":
+        block.ffn.up.bias = None
+    attention, ffn = block.attention, block.ffn
+    by_name = [block.attn_norm.weight, attention.qkv.weight, attention.qkv.bias, attention.out.weight, attention.out.bias,
+               block.ffn_norm.weight, ffn.up.weight, ffn.up.bias, ffn.down.weight, ffn.down.bias, attention.query_norm.weight,
+               attention.key_norm.weight]
+    for got, expected in zip(_block_parameters(block), by_name, strict=True):
+        assert got is expected or torch.equal(got, expected)
+    assert {id(p) for p in _every_parameter(block)} == {id(p) for p in block.parameters()}
+    assert _block_config(block) == (4, block.attn_norm.eps, block.ffn_norm.eps, attention.query_norm.eps, True)
