@@ -597,6 +597,13 @@ __global__ __launch_bounds__(kThreads) void flash_attn_fwd_kernel(const AttnPara
   }
 }
 
+// `score` where bit `at` of the word is set, else -inf: a signed one-bit field is all ones or nothing and picks the bits (two
+// instructions; a test, a compare and a select are three).
+__device__ __forceinline__ float where_bit_else_minus_inf(float score, uint32_t word, int at) {
+  const uint32_t seen = static_cast<uint32_t>(__builtin_amdgcn_sbfe(static_cast<int>(word), at, 1));
+  return __builtin_bit_cast(float, (seen & __builtin_bit_cast(uint32_t, score)) | (~seen & 0xff800000u));
+}
+
 // ------------------------------------------------------------------------------------------------------------------
 // The plain case at head dims 32 and 64 (key-length / causal masking only, no row factors, no structured mask): K and V
 // chunks go from global memory straight into LDS (one 1 KB transfer per wavefront and operand, no staging registers,
@@ -612,8 +619,10 @@ __global__ __launch_bounds__(kThreads) void flash_attn_fwd_kernel(const AttnPara
 // scores of those keys are masked), since uninitialised memory could hold NaNs that a zero probability would not cancel.
 // ------------------------------------------------------------------------------------------------------------------
 // MASKED: per-sample structure bits on top (struct_bits with a sample stride, every listed key valid, no chunk map): the
-// form in which samples with their valid tokens moved to the front arrive. The lane's two words of a chunk are fetched
-// with the chunk's transfers; tiles that are fully visible to the wavefront skip the bit tests.
+// form in which samples with their valid tokens moved to the front arrive. The words of a chunk arrive in LDS with the chunk's
+// transfers; tiles of which the wavefront sees every key skip the bit tests. Under a role mask, 384 samples of up to 512 tokens, 8 heads of
+// 32 (4 of 64), with the query / key factors, 163 us (132) with the words in registers and three instructions per hidden score, 138 (117) with them in LDS and
+// two, 133 (112) without the tests where only keys behind the length are hidden.
 // COMPACT: samples are addressed by row_offsets (a form of its own: decided at run time, the loads of the pointers' strides stand in
 // front of a workgroup's first rows in the other form too).
 template <typename T, int DP, bool CAUSAL, bool SCALED, bool MASKED, bool COMPACT = false>
@@ -636,7 +645,10 @@ __global__ __launch_bounds__(kThreads) void flash_attn_fwd_dma_kernel(const Attn
   // 16 KB: with three a compute unit holds three workgroups, with two it holds as many as the registers allow), chunk c + 1
   // is requested once every wavefront has left chunk c - 1.
   constexpr int NBUF = DP == 64 ? 2 : 3;
-  __shared__ __attribute__((aligned(1024))) uint8_t smem[NBUF * BUF_BYTES > OT_BYTES ? NBUF * BUF_BYTES : OT_BYTES];
+  // MASKED: behind the chunk buffers the words of the wavefronts' queries for every buffer's chunk, [buffer][wavefront][word][query]
+  constexpr int WORD_BYTES = kWave * 4, WORDS_AT = NBUF * BUF_BYTES;
+  constexpr int STAGE_BYTES = NBUF * BUF_BYTES + (MASKED ? NBUF * (kThreads / kWave) * WORD_BYTES : 0);
+  __shared__ __attribute__((aligned(1024))) uint8_t smem[STAGE_BYTES > OT_BYTES ? STAGE_BYTES : OT_BYTES];
 
   // A workgroup takes two query blocks of one (sample, head), g and nqc - 1 - g (one, for the middle block of an odd
   // count): under key lengths the first is the one more likely to hold valid queries, so few workgroups find nothing to
@@ -761,20 +773,15 @@ __global__ __launch_bounds__(kThreads) void flash_attn_fwd_dma_kernel(const Attn
   const bool scale_keys = SCALED && p.k_row_scale != nullptr;
   vec_t kreg[SCALED ? PPT : 1];
   float kfac[SCALED ? PPT : 1];
-  // mask words of the two chunks in flight (even / odd chunk) and of the chunk being consumed
-  uint32_t mw_even[2] = {0u, 0u}, mw_odd[2] = {0u, 0u}, mw[2] = {0u, 0u};
+  // The chunk's two mask words of the wavefront's 32 queries travel into LDS as well, a word per lane. (In registers, picked by the
+  // chunk's parity, they were waited for - and with them everything else just requested - where they were requested.)
+  [[maybe_unused]] const uint32_t* const bit_rows = MASKED ? p.struct_bits + b * p.struct_stride + static_cast<int64_t>(q_begin) * p.wpr : nullptr;
+  [[maybe_unused]] const uint32_t bit_row = MASKED ? __umul24(static_cast<uint32_t>(q_row_read - q_begin), static_cast<uint32_t>(p.wpr)) : 0u;
   auto issue = [&](int chunk, int buffer) {
     if (MASKED) {
-#pragma unroll
-      for (int kt = 0; kt < 2; ++kt) {
-        const int w = chunk * 2 + kt;
-        const uint32_t word = (qi < q_valid && w < p.wpr)
-                                  ? p.struct_bits[b * p.struct_stride + static_cast<int64_t>(qi) * p.wpr + w] : 0u;
-        if (chunk & 1)
-          mw_odd[kt] = word;
-        else
-          mw_even[kt] = word;
-      }
+      const int w = chunk * 2 + hh;
+      lds_dma4_offset(bit_rows, (bit_row + static_cast<uint32_t>(w < p.wpr ? w : p.wpr - 1)) * 4u,
+                      smem + WORDS_AT + (buffer * (kThreads / kWave) + wave) * WORD_BYTES);
     }
 #pragma unroll
     for (int i = 0; i < PPT; ++i) {
@@ -782,9 +789,12 @@ __global__ __launch_bounds__(kThreads) void flash_attn_fwd_dma_kernel(const Attn
       row = row < kv_end ? row : kv_end - 1;  // kv_end >= 1 here
       uint8_t* dst = smem + buffer * BUF_BYTES + i * (kThreads * 16) + wave * (kWave * 16);
       if (scale_keys) {
-        kreg[SCALED ? i : 0] = *reinterpret_cast<const vec_t*>(reinterpret_cast<const uint8_t*>(kb) +
-                                                              __umul24(static_cast<uint32_t>(row), k_row_bytes) + k_piece_off);
-        kfac[SCALED ? i : 0] = p.k_row_scale[static_cast<int64_t>(b) * p.Tk + row];
+        // (opaque 32-bit offsets of uniform bases: reassociated, the addresses take six registers more)
+        uint32_t k_off = __umul24(static_cast<uint32_t>(row), k_row_bytes) + k_piece_off, f_off = static_cast<uint32_t>(row) * 4u;
+        asm volatile("" : "+v"(k_off), "+v"(f_off));
+        kreg[SCALED ? i : 0] = *reinterpret_cast<const vec_t*>(reinterpret_cast<const uint8_t*>(kb) + k_off);
+        kfac[SCALED ? i : 0] =
+            *reinterpret_cast<const float*>(reinterpret_cast<const uint8_t*>(p.k_row_scale + static_cast<int64_t>(b) * p.Tk) + f_off);
       } else {
         lds_dma16_offset(kb, __umul24(static_cast<uint32_t>(row), k_row_bytes) + k_piece_off, dst);
       }
@@ -830,7 +840,7 @@ __global__ __launch_bounds__(kThreads) void flash_attn_fwd_dma_kernel(const Attn
   int buf = 0;
   // transfers (and mask words) of one chunk per wavefront: what may stay in flight while the chunk before it is awaited.
   // With key factors the keys pass through registers and are waited for when they are committed: wait for everything.
-  constexpr int kInFlight = 2 * PPT + (MASKED ? 2 : 0);
+  constexpr int kInFlight = 2 * PPT + (MASKED ? 1 : 0);
   // One chunk: wait for its transfers, publish them, start the next chunk's, then (NT > 0) take the chunk's first NT key
   // tiles into the running softmax. NT is a compile-time property of the call site: a wavefront sees whole chunks first,
   // then at most one chunk of which only the first tile holds visible keys, then chunks that only the other wavefronts of
@@ -844,10 +854,8 @@ __global__ __launch_bounds__(kThreads) void flash_attn_fwd_dma_kernel(const Attn
     else
       vm_wait<0>();
     __syncthreads();  // ... everyone's have, and everyone is done reading the buffer of the chunk before
-    if (MASKED) {
-      mw[0] = (chunk & 1) ? mw_odd[0] : mw_even[0];
-      mw[1] = (chunk & 1) ? mw_odd[1] : mw_even[1];
-    }
+    [[maybe_unused]] const uint32_t* const words =
+        reinterpret_cast<const uint32_t*>(smem + WORDS_AT + (buf * (kThreads / kWave) + wave) * WORD_BYTES) + l32;
     // the chunk requested now: two ahead into the buffer (buf + 2) % 3, or the next one into the buffer left last
     const bool more = NBUF == 3 ? chunk + 2 < nchunks : (chunk >= 1 && chunk + 1 < nchunks);
     const int ahead = NBUF == 3 ? (buf == 0 ? 2 : buf - 1) : 1 - buf;
@@ -904,16 +912,22 @@ __global__ __launch_bounds__(kThreads) void flash_attn_fwd_dma_kernel(const Attn
       }
       if (MASKED) {
         // Accumulator register j of the lane is key (j / 4) * 8 + hh * 4 + j % 4 of the tile: bit of the lane's word.
+        uint32_t mw[NT];
         bool all_visible = true;
 #pragma unroll
-        for (int kt = 0; kt < NT; ++kt) all_visible = all_visible && mw[kt] == 0xffffffffu;
+        for (int kt = 0; kt < NT; ++kt) {
+          mw[kt] = words[kt * 32];
+          // (NT tiles hold keys in front of kv_end; what lies behind it is masked already)
+          const int left = kv_end - kc0 - kt * 32;
+          const uint32_t beyond = left < 32 ? 0xffffffffu << left : 0u;
+          all_visible = all_visible && (mw[kt] | beyond) == 0xffffffffu;
+        }
         if (__builtin_amdgcn_ballot_w64(!all_visible) != 0) {  // wavefront-uniform
 #pragma unroll
           for (int kt = 0; kt < NT; ++kt) {
             const uint32_t bits = mw[kt] >> (hh * 4);
 #pragma unroll
-            for (int j = 0; j < 16; ++j)
-              if (((bits >> ((j / 4) * 8 + (j % 4))) & 1u) == 0u) sacc[kt][j] = -INFINITY;
+            for (int j = 0; j < 16; ++j) sacc[kt][j] = where_bit_else_minus_inf(sacc[kt][j], bits, (j / 4) * 8 + (j % 4));
           }
         }
       }

@@ -58,6 +58,18 @@ __device__ __forceinline__ void lds_dma4(const void* gsrc, void* lds_wave_base) 
       : "memory", "m0");
 }
 
+// lds_dma4 with the source given as a wavefront-uniform base (scalar registers) + a 32-bit per-lane byte offset.
+__device__ __forceinline__ void lds_dma4_offset(const void* base, uint32_t lane_offset, void* lds_wave_base) {
+  const uint32_t lds_base = __builtin_amdgcn_readfirstlane(lds_offset(lds_wave_base));
+  asm volatile(
+      "s_mov_b32 m0, %2\n\t"
+      "s_nop 0\n\t"
+      "global_load_lds_dword %0, %1"
+      :
+      : "v"(lane_offset), "s"(base), "s"(lds_base)
+      : "memory", "m0");
+}
+
 // Transposed 64-bit read: element e of lane j of a 16-lane group receives element j % 4 of the 8-byte row whose address
 // lane 4 * e + j / 4 of that group supplies.
 template <int OFFSET>

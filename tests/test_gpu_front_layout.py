@@ -153,6 +153,38 @@ def test_attention_over_the_front_layout_matches_the_masked_attention_over_posit
     torch.testing.assert_close(got, expected, rtol=2e-2, atol=2e-2)
 
 
+@pytest.mark.parametrize("tokens,dim", [(512, 32), (197, 32), (31, 32), (300, 64), (65, 64)])
+@pytest.mark.parametrize("dtype,factors", [(torch.bfloat16, True), (torch.bfloat16, False), (torch.float16, True)])
+def test_attention_over_the_front_layout_at_the_edges_of_tiles(device, tokens, dim, dtype, factors):
+    """Lengths on both sides of every key tile's edge, under a mask with tiles that are seen whole, in part and not at all. Scores,
+    probabilities and output are rounded to 16 bits once each: 2e-2 as in the tests above."""
+    edges = [n + d for n in range(0, tokens + 1, 32) for d in (-1, 0, 1) if 1 <= n + d <= tokens] + [tokens]
+    batch, heads = len(edges), 2
+    g = torch.Generator(device=device).manual_seed(tokens + dim)
+    lengths = torch.tensor(edges, device=device)
+    at = torch.arange(tokens, device=device)
+    padding = at >= lengths[:, None]
+    structural = torch.ones(tokens, tokens, dtype=torch.bool, device=device)
+    structural[4:, :10] = False                                                # most queries do not see the first keys
+    structural[12:40, 40:] = False                                             # some see nothing behind them
+    structural[40:60] &= torch.rand(structural[40:60].shape, generator=g, device=device) < 0.5
+    structural |= at[:, None] == at
+    q, k, v = (torch.randn(batch, heads, tokens, dim, generator=g, device=device).to(dtype) for _ in range(3))
+    scales = [0.5 + torch.rand(batch, tokens, generator=g, device=device) if factors else None for _ in range(2)]
+    seen = structural & ~padding[:, None, None, :]
+    q_eff, k_eff = (t.double() if f is None else t.double() * f[:, None, :, None] for t, f in zip((q, k), scales))
+    scores = (q_eff @ k_eff.transpose(-1, -2) / dim ** 0.5).masked_fill(~seen, float("-inf"))
+    expected = torch.softmax(scores, dim=-1) @ v.double()
+    index = valid_rows(None, tokens, padding_mask=padding)
+    _, front_lengths = front_rows(index, batch, tokens)
+    front_mask = front_structured_mask(build_structured_mask(structural, ~padding), index, batch)
+    padded = padding[:, None, :, None]
+    q, k, v = (t.masked_fill(padded, float("nan")) for t in (q, k, v))  # rows beyond a sample's length are never used
+    got = flash_attention(q, k, v, key_lengths=front_lengths, structured_mask=front_mask, zero_padded_queries=2,
+                          q_row_scale=scales[0], k_row_scale=scales[1])
+    torch.testing.assert_close(got.double().masked_fill(padded, 0.0), expected.masked_fill(padded, 0.0), rtol=2e-2, atol=2e-2)
+
+
 @pytest.mark.parametrize("tokens,dim", [(150, 32), (96, 64)])
 def test_attention_over_the_front_layout_takes_a_gradient(device, tokens, dim):
     """The same comparison for the backward: gradients of attention over the front layout (structure bits per sample,
