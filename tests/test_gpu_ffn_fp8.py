@@ -161,6 +161,28 @@ def test_norm_linear_fp8_fuses_norm_rows_and_the_next_scale(device, test_hooks, 
     assert abs(amax_out.item() - expected_next) <= 2 ** -7 * expected_next
 
 
+@pytest.mark.parametrize("n", [64, 256, 320])
+@pytest.mark.parametrize("with_residual", [False, True])
+def test_memory_rows_of_a_tile_are_kept_over_its_steps(device, test_hooks, n, with_residual):
+    """Rows through an index in steps divided over the workgroups, a tile after the other in one of them: the bits of the layer on the
+    gathered rows, and nothing beside them."""
+    batch, tokens, k = 13, 190, 256
+    g = torch.Generator(device=device).manual_seed(n)
+    x, res = (torch.randn(batch * tokens, width, generator=g, device=device).to(torch.bfloat16) for width in (k, n))
+    w = (torch.randn(n, k, generator=g, device=device) / 16).to(torch.bfloat16)
+    lengths = torch.randint(0, tokens + 1, (batch,), generator=g, device=device, dtype=torch.int32)
+    valid = (torch.arange(tokens, device=device)[None, :] < lengths[:, None]).flatten()
+    with torch.no_grad():
+        wq, wa = quantize_fp8(w)
+        ax = amax(x[valid])
+        want = linear_fp8(x[valid], wq, ax, wa, None, residual=res[valid] if with_residual else None)
+        for workgroups in (1, 3, 8, None):
+            test_hooks(max_workgroups=workgroups)
+            out = torch.full((batch * tokens, n), float("nan"), dtype=torch.bfloat16, device=device)
+            norm_linear_fp8(x, wq, ax, wa, None, residual=res if with_residual else None, token_rows=valid_rows(lengths, tokens), out=out)
+            assert torch.equal(out[valid], want) and torch.isnan(out[~valid].float()).all()
+
+
 @pytest.mark.parametrize("m,n", [(1, 64), (513, 768), (1500, 256), (3000, 832)])
 def test_dense_layer_with_its_steps_divided_over_workgroups(device, test_hooks, m, n):
     """The steps of the tiles run over the workgroups in one sequence, so a workgroup may start and end inside a tile: every
