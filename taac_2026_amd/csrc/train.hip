@@ -235,10 +235,13 @@ __global__ __launch_bounds__(kThreads) void scatter_kernel(const bf16x8* __restr
   } else {
     const uint32_t* bits = valid_bits + static_cast<int64_t>(b) * ((T + 31) / 32);
     const uint32_t word = bits[t / 32];
-    if ((word >> (t % 32)) & 1u) {
-      rank = __popc(word & ((1u << (t % 32)) - 1u));
-      for (int w = 0; w < t / 32; ++w) rank += __popc(bits[w]);
-    }
+    // The words in front of the row's are counted by the row's lanes together (`pieces` of them, a power of two within a wavefront): by each
+    // alone it is a load behind the other, 128 x 403 tokens of 256 features 19.4 -> 14.8 us.
+    const int lane = static_cast<int>(idx % pieces);
+    int before = 0;
+    for (int w = lane; w < t / 32; w += pieces) before += __popc(bits[w]);
+    for (int off = 1; off < pieces; off <<= 1) before += __shfl_xor(before, off, kWave);
+    if ((word >> (t % 32)) & 1u) rank = before + __popc(word & ((1u << (t % 32)) - 1u));
   }
   bf16x8 v;
   if (rank >= 0) {
@@ -363,20 +366,24 @@ __global__ __launch_bounds__(kThreads) void qk_norm_bwd_kernel(const bf16_t* __r
   }
   constexpr int R = 2;
   constexpr int64_t kStep = GPB / 2;
-  for (int64_t m0 = (static_cast<int64_t>(blockIdx.x) * R) * kStep + gid / 2; m0 < rows; m0 += static_cast<int64_t>(gridDim.x) * R * kStep) {
-    bf16x8 xv[R], gv[R];
-    bool ok[R];
+  // The rows of the next step are requested in front of this step's: behind its stores they would wait for those as well (loads and
+  // stores complete in one order), a memory latency and the stores in every step (29 000
+  // rows of 256, us: 23.2 -> 17.8).
+  const int64_t stride = static_cast<int64_t>(gridDim.x) * R * kStep;
+  const int64_t first = (static_cast<int64_t>(blockIdx.x) * R) * kStep + gid / 2;
+  auto request = [&](int64_t m0, bf16x8 (&xv)[R], bf16x8 (&gv)[R]) {
 #pragma unroll
     for (int r = 0; r < R; ++r) {
       const int64_t m = m0 + r * kStep;
-      ok[r] = m < rows;
-      const int64_t at = (ok[r] ? m : m0) * (3 * D) + part * D + lane * 8;
+      const int64_t at = (m < rows ? m : first) * (3 * D) + part * D + lane * 8;  // (its values are not used then)
       xv[r] = *reinterpret_cast<const bf16x8*>(qkv + at);
       gv[r] = *reinterpret_cast<const bf16x8*>(dqkv + at);
     }
+  };
+  auto step = [&](int64_t m0, const bf16x8 (&xv)[R], const bf16x8 (&gv)[R]) {
 #pragma unroll
     for (int r = 0; r < R; ++r) {
-      if (!ok[r]) continue;  // the same for the whole lane group
+      if (m0 + r * kStep >= rows) continue;  // the same for the whole lane group
       float ss = 0.f, sg = 0.f;
 #pragma unroll
       for (int e = 0; e < 8; ++e) {
@@ -394,6 +401,18 @@ __global__ __launch_bounds__(kThreads) void qk_norm_bwd_kernel(const bf16_t* __r
         dw[e] = fmaf(g, x * rstd, dw[e]);
       }
       *reinterpret_cast<bf16x8*>(dqkv + (m0 + r * kStep) * (3 * D) + part * D + lane * 8) = o;
+    }
+  };
+  if (first < rows) {
+    bf16x8 xa[R], ga[R], xb[R], gb[R];
+    request(first, xa, ga);
+    for (int64_t m0 = first; m0 < rows; m0 += 2 * stride) {
+      request(m0 + stride, xb, gb);
+      __builtin_amdgcn_sched_barrier(0);
+      step(m0, xa, ga);
+      request(m0 + 2 * stride, xa, ga);
+      __builtin_amdgcn_sched_barrier(0);
+      step(m0 + stride, xb, gb);
     }
   }
 #pragma unroll

@@ -379,3 +379,31 @@ def test_tokens_between_the_halves_of_a_large_batch(device, d_model, heads, batc
         a, b = got[~padding].float(), want[~padding].float()
         assert b.abs().max() < 8 and (a - b).abs().max() <= 2.0 ** -4 and (a - b).norm() <= 2.0 ** -8 * b.norm()
         assert torch.equal(got[padding], x[padding])
+
+
+@pytest.mark.parametrize("d_model,heads,batch,tokens", [(256, 8, 900, 25), (128, 4, 1500, 27)])
+def test_query_and_key_norms_of_several_steps_a_workgroup(device, d_model, heads, batch, tokens):
+    """More rows than the workgroups of the norms' backward take at once: two whole steps and a part of a third."""
+    lengths = [(11 * i) % (tokens + 1) for i in range(batch)]
+    test_training_stack_at_the_edges_of_its_tiles(device, d_model, heads, 64, 1, lengths, tokens, True, torch.bfloat16)
+
+
+@pytest.mark.parametrize("width,tokens", [(128, 1), (128, 545), (128, 700), (256, 96), (256, 1056)])
+def test_rows_go_back_to_where_scattered_padding_left_them(device, width, tokens):
+    """Under a role mask with padding inside the samples: the training stack's output has the rows of the inference kernels' (same values but
+    for roundings; a row at another's place is off by its norm), and padded rows carry the gradient that arrives."""
+    g = torch.Generator(device=device).manual_seed(tokens)
+    blocks = torch.nn.ModuleList([UnifiedInteractionBlock(width, width // 32, 2)]).to(device).to(torch.bfloat16)
+    x, grad = (torch.randn(3, tokens, width, generator=g, device=device).to(torch.bfloat16) for _ in range(2))
+    padding = torch.rand(3, tokens, generator=g, device=device) < torch.tensor([0.2, 0.8, 0.5], device=device)[:, None]
+    padding[:, 0] = False
+    mask = MetadataAttentionMask(enabled=True)(padding, torch.randint(0, 8, (tokens,), generator=g, device=device))
+    leaf = x.clone().requires_grad_(True)
+    out = run_interaction_blocks(blocks, leaf, padding, mask)
+    out.backward(grad)
+    with torch.no_grad():
+        want = run_interaction_blocks(blocks, x, padding, mask).float()
+    error = (out.detach().float() - want).norm(dim=-1)
+    assert (error <= 2.0 ** -4 * want.norm(dim=-1)).all()
+    assert torch.equal(out.detach()[padding], x[padding]) and torch.equal(leaf.grad[padding], grad[padding])
+    assert ((leaf.grad - grad)[~padding].float().norm(dim=-1) > 0).all()
