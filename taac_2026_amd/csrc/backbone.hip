@@ -164,16 +164,25 @@ __global__ __launch_bounds__(kBlock) void front_rows_kernel(const int32_t* __res
   front_rows[i] = b * T + static_cast<int32_t>(i - offsets[b]);
 }
 
-// One workgroup per (sample b, 32 front rows): the sample's key positions go to LDS once; a wavefront then takes 8
-// rows, holds a row's structure words across its lanes (lane l: words l and l + 64) and, 64 keys per step, lets lane j
-// pick the word of its key from them with a lane permute; a ballot gathers the bits. Only rows below the sample's
-// number of valid tokens n_b are written, and of those the words that hold a key below n_b (the attention kernel reads
-// nothing else), bits at or beyond n_b as zeros.
-constexpr int kFrontRowsPerBlock = 32;
+// One workgroup per (sample b, kFrontRowsPerBlock front rows). The front keys are the sample's valid positions in ascending order, so a
+// front row is its structure row with the bits of the invalid positions squeezed out: one lane takes a word of 32 positions, moves each
+// kept bit down by the number of dropped ones below it - by 1, 2, 4, 8 and 16 where that number has the digit; which bits move in which
+// step depends on the validity word alone, so a lane works it out once for all its rows - and ORs the piece into the row's words
+// in LDS from the bit on at which the valid positions in front of the word end. Only rows below the sample's number of valid tokens n_b are written,
+// and of those the words that hold a key below n_b's 64-key group (the attention kernel reads nothing else), bits at or beyond n_b as zeros.
+// Bound by the chain of loads in front of it (offsets, positions, structure words). Before, a lane picked the word of its key by a
+// lane permute and a ballot gathered 64 bits. Before / now, us, samples x positions, 30 % of them invalid: 16 x 403 6.2 / 3.7,
+// 512 x 403 23.1 / 11.3 (none invalid 36.3 / 16.1, 80 % 7.8 / 6.8), 512 x 200 10.5 / 7.5, 64 x 2048 60.9 / 20.6, 32 x 4096
+// 105.5 / 39.3. Rows of a workgroup: 32 / 64 / 128, 512 x 403 16.0 / 11.3 / 12.6, 16 x 403 3.6 / 3.7 / 4.6, 32 x 4096 37.4 / 39.3 / 44.9.
+constexpr int kFrontRowsPerBlock = 64;
+constexpr int kFrontWords = 4096 / 32;
+constexpr int kFrontRowsAtOnce = 4;
 __global__ __launch_bounds__(kBlock) void mask_front_bits_kernel(const uint32_t* __restrict__ struct_bits, int T,
                                                                  const int32_t* __restrict__ rows, int B,
                                                                  uint32_t* __restrict__ out) {
-  __shared__ uint16_t kpos[4096];
+  __shared__ uint32_t valid[kFrontWords];
+  __shared__ uint32_t position[kFrontRowsPerBlock];
+  extern __shared__ uint32_t front[];  // [kFrontRowsPerBlock][wpr]
   const int wpr = (T + 31) / 32;
   const int slabs = (T + kFrontRowsPerBlock - 1) / kFrontRowsPerBlock;
   const int b = blockIdx.x / slabs, r0 = (blockIdx.x % slabs) * kFrontRowsPerBlock;
@@ -181,35 +190,76 @@ __global__ __launch_bounds__(kBlock) void mask_front_bits_kernel(const uint32_t*
   const int32_t off = offsets[b];
   const int n = offsets[b + 1] - off;
   if (r0 >= n) return;  // workgroup-uniform
-  for (int j = threadIdx.x; j < n; j += kBlock) kpos[j] = static_cast<uint16_t>(rows[off + j] - b * T);
+  const int here = n - r0 < kFrontRowsPerBlock ? n - r0 : kFrontRowsPerBlock;
+  if (threadIdx.x < kFrontWords) valid[threadIdx.x] = 0u;
+  for (int i = threadIdx.x; i < here * wpr; i += kBlock) front[i] = 0u;
   __syncthreads();
-  const int lane = threadIdx.x % kWave, wave = threadIdx.x / kWave;
-  constexpr int kRowsPerWave = kFrontRowsPerBlock / (kBlock / kWave);
-  // the structure words of the wavefront's rows first (independent loads), then the gathers
-  uint32_t w_lo[kRowsPerWave], w_hi[kRowsPerWave];
-#pragma unroll
-  for (int i = 0; i < kRowsPerWave; ++i) {
-    const int r = r0 + wave * kRowsPerWave + i;
-    const uint32_t* src = struct_bits + static_cast<int64_t>(kpos[r < n ? r : 0]) * wpr;
-    w_lo[i] = (r < n && lane < wpr) ? src[lane] : 0u;
-    w_hi[i] = (r < n && lane + kWave < wpr) ? src[lane + kWave] : 0u;
+  for (int j = threadIdx.x; j < n; j += kBlock) {
+    const uint32_t at = static_cast<uint32_t>(rows[off + j] - b * T);
+    if (at < static_cast<uint32_t>(T)) atomicOr(&valid[at / 32], 1u << (at % 32));
+    if (j >= r0 && j < r0 + here) position[j - r0] = at < static_cast<uint32_t>(T) ? at : 0u;
   }
-  for (int j0 = 0; j0 < n; j0 += kWave) {
-    const int j = j0 + lane;
-    const int key = j < n ? kpos[j] : 0;
-    const int src_lane = (key >> 5) & (kWave - 1);
-    const bool upper = (key >> 5) >= kWave;
+  __syncthreads();
+  // lanes of a row: wpr rounded up to a power of two
+  const int shift = wpr <= 1 ? 0 : 32 - __builtin_clz(static_cast<unsigned>(wpr - 1));
+  const int word = threadIdx.x & ((1 << shift) - 1), row0 = threadIdx.x >> shift, rows_at_once = kBlock >> shift;
+  uint32_t words[kFrontRowsAtOnce];
+  auto request = [&](int first) {
 #pragma unroll
-    for (int i = 0; i < kRowsPerWave; ++i) {
-      const int r = r0 + wave * kRowsPerWave + i;
-      if (r >= n) break;  // wavefront-uniform
-      const uint32_t lo = __shfl(w_lo[i], src_lane, kWave);
-      const uint32_t word = wpr > kWave ? (upper ? __shfl(w_hi[i], src_lane, kWave) : lo) : lo;
-      const uint64_t bits = __builtin_amdgcn_ballot_w64(j < n && ((word >> (key & 31)) & 1u) != 0u);
-      uint32_t* dst = out + (static_cast<int64_t>(b) * T + r) * wpr;
-      if (lane < 2 && j0 / 32 + lane < wpr) dst[j0 / 32 + lane] = static_cast<uint32_t>(bits >> (32 * lane));
+    for (int i = 0; i < kFrontRowsAtOnce; ++i) {
+      const int r = first + i * rows_at_once;
+      words[i] = (word < wpr && r < here) ? struct_bits[static_cast<int64_t>(position[r]) * wpr + word] : 0u;
+    }
+  };
+  request(row0);
+  // valid positions in front of the lane's word: every wavefront scans all words, two a lane
+  const int lane = threadIdx.x % kWave;
+  const int even = __popc(valid[2 * lane]);
+  int upto = even + __popc(valid[2 * lane + 1]);
+  const int pair = upto;
+#pragma unroll
+  for (int step = 1; step < kWave; step <<= 1) {
+    const int below = __shfl_up(upto, step, kWave);
+    if (lane >= step) upto += below;
+  }
+  const int pairs_before = __shfl(upto - pair, word / 2, kWave), even_before = __shfl(even, word / 2, kWave);
+  const int before = pairs_before + ((word & 1) ? even_before : 0);
+  // moved[k]: the bits that move down by 2^k. `odd`: at each bit, whether the number of dropped bits below it that are still to
+  // be counted is odd; those at odd counts are then taken out, which halves the counts for the next step.
+  const uint32_t keep = valid[word];
+  uint32_t moved[5], kept = keep, dropped_below = ~keep << 1;
+#pragma unroll
+  for (int k = 0; k < 5; ++k) {
+    uint32_t odd = dropped_below;
+#pragma unroll
+    for (int step = 1; step < 32; step <<= 1) odd ^= odd << step;
+    moved[k] = odd & kept;
+    kept = (kept ^ moved[k]) | (moved[k] >> (1 << k));
+    dropped_below &= ~odd;
+  }
+  for (int first = row0; first < here; first += kFrontRowsAtOnce * rows_at_once) {
+    if (first != row0) request(first);
+#pragma unroll
+    for (int i = 0; i < kFrontRowsAtOnce; ++i) {
+      const int r = first + i * rows_at_once;
+      uint32_t bits = words[i] & keep;
+#pragma unroll
+      for (int k = 0; k < 5; ++k) {
+        const uint32_t moving = bits & moved[k];
+        bits = (bits ^ moving) | (moving >> (1 << k));
+      }
+      const uint64_t piece = static_cast<uint64_t>(bits) << (before % 32);
+      const uint32_t lo = static_cast<uint32_t>(piece), hi = static_cast<uint32_t>(piece >> 32);
+      uint32_t* dst = front + r * wpr + before / 32;
+      if (lo != 0u) atomicOr(dst, lo);  // a bit that is set stands for a key below n: within the row's words
+      if (hi != 0u) atomicOr(dst + 1, hi);
     }
   }
+  __syncthreads();
+  const int written = (n + kWave - 1) / kWave * 2 < wpr ? (n + kWave - 1) / kWave * 2 : wpr;
+  if (word < written)
+    for (int r = row0; r < here; r += rows_at_once)
+      out[(static_cast<int64_t>(b) * T + r0 + r) * wpr + word] = front[r * wpr + word];
 }
 
 }  // namespace
@@ -794,7 +844,8 @@ extern "C" int taac_mask_front_bits(const uint32_t* struct_bits, int32_t T, cons
   if (!struct_bits || !rows || !out_bits) return set_error(TAAC_ERR_INVALID_VALUE, "%s: null pointer", name);
   const int64_t blocks = static_cast<int64_t>(B) * ((T + kFrontRowsPerBlock - 1) / kFrontRowsPerBlock);
   if (blocks > 0x7fffffffLL) return set_error(TAAC_ERR_UNSUPPORTED, "%s: too many rows", name);
-  hipLaunchKernelGGL(mask_front_bits_kernel, dim3(static_cast<uint32_t>(blocks)), dim3(kBlock), 0, as_stream(stream),
+  hipLaunchKernelGGL(mask_front_bits_kernel, dim3(static_cast<uint32_t>(blocks)), dim3(kBlock),
+                     kFrontRowsPerBlock * ((T + 31) / 32) * sizeof(uint32_t), as_stream(stream),
                      struct_bits, T, rows, B, out_bits);
   return check_launch(name);
 }

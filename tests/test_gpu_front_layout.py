@@ -8,6 +8,7 @@ import pytest
 import torch
 
 from oracle import reference as oracle
+from taac_2026_amd import _native
 from taac_2026_amd.api import (
     build_structured_mask,
     flash_attention,
@@ -221,3 +222,32 @@ def test_attention_over_the_front_layout_takes_a_gradient(device, tokens, dim):
         want = want.transpose(1, 2).reshape(batch * tokens, heads, dim)[rows]
         assert torch.isfinite(got).all(), name
         torch.testing.assert_close(got, want, rtol=3e-2, atol=3e-2, msg=lambda m, n=name: f"{n}: {m}")
+
+
+@pytest.mark.parametrize("batch,tokens", [(3, 1), (4, 31), (4, 32), (4, 64), (4, 65), (40, 403), (4, 513), (3, 2049), (3, 4096)])
+def test_front_structured_mask_bits_at_the_edges_of_words(device, batch, tokens):
+    g = torch.Generator().manual_seed(tokens)
+    padding = _padding(batch, tokens, seed=tokens + 2)
+    for b in range(3, batch):  # ends, runs, single positions
+        padding[b] = b % 2 == 0
+        cut = torch.randint(0, tokens + 1, (2,), generator=g).sort().values.tolist()
+        padding[b, cut[0]:cut[1]] = b % 2 == 1
+    structural = torch.rand(tokens, tokens, generator=g) < 0.5
+    mask = build_structured_mask(structural.to(device), (~padding).to(device))
+    rows, _ = valid_rows(None, tokens, padding_mask=padding.to(device))
+    words = (tokens + 31) // 32
+    untouched = -0x5A5A5A5B
+    out = torch.full((batch * tokens, words), untouched, dtype=torch.int32, device=device)
+    _native.check(_native.load_library().taac_mask_front_bits(mask.struct_bits.data_ptr(), tokens, rows.data_ptr(), batch,
+                                                              out.data_ptr(), _native.current_stream(out.device)), "front bits")
+    out = out.cpu().view(batch, tokens, words)
+    shifts = torch.arange(32)
+    for b in range(batch):
+        positions = (~padding[b]).nonzero().flatten()
+        n = positions.numel()
+        written = min(words, 2 * ((n + 63) // 64))
+        want = torch.zeros(n, words * 32, dtype=torch.bool)
+        want[:, :n] = structural[positions][:, positions]
+        got = ((out[b, :n, :written, None] >> shifts) & 1).bool().view(n, written * 32)
+        assert torch.equal(got, want[:, :written * 32]), b
+        assert (out[b, n:] == untouched).all() and (out[b, :, written:] == untouched).all(), b
