@@ -5,7 +5,7 @@
 // model.py:215-222, 291, 309, 316-317; experiments/symbiosis/pooling.py:16-32) and masked_mean
 // (modeling/sequence.py:54-60) without writing the normalised tokens, the pooled vector or the hidden layer to memory.
 //
-// One workgroup of 256 lanes per sample. The sample's valid token rows are read exactly once: a row is owned by 32
+// One workgroup of 256 or 1024 lanes per sample. The sample's valid token rows are read exactly once: a row is owned by 32
 // consecutive lanes (128-bit loads, up to four per lane), 16 to 32 rows in flight per workgroup; the token norm's
 // statistic is a 32-lane shuffle reduction, the normalised row is accumulated in fp32 registers. Because the token
 // norm's weight is per feature it commutes with the mean and is applied once to the pooled sum. The classifier is two
@@ -188,18 +188,39 @@ __global__ __launch_bounds__(kReadoutBlock) void candidate_readout_kernel(const 
   // ---- classifier: hidden = silu(W1 e + b1), logits = W2 hidden + b2 ------------------------------------------------
   float* s_hidden = s_red;  // the partial sums are dead (barriers above); the host sizes the region for both uses
   const int kvec = K / 8;
-  for (int j = g; j < p.hidden; j += kRowGroups) {
-    const bf16_t* wrow = p.fc1_w + static_cast<int64_t>(j) * K;
-    float dot = 0.f;
-    for (int piece = l32; piece < kvec; piece += kRowLanes) {
-      const bf16x8 w = *reinterpret_cast<const bf16x8*>(wrow + piece * 8);
+  // A chain of loads from L2: four weight rows of a group at once (the lanes of a row beyond the last read the first again and drop
+  // its product); one at a time / four, us, 256 lanes, samples x tokens at width 256: 1 x 100 35.5 / 26.6, 1024 x 100 49.5 / 39.7;
+  // 1024 lanes: 384 x 514 44.8 / 41.5, 256 x 514 at width 512 55.3 / 45.5. Eight, or the pieces unrolled, take registers
+  // that the second workgroup of a compute unit needs (384 x 514 59).
+  constexpr int kHiddenAtOnce = 4;
+  for (int j0 = g; j0 < p.hidden; j0 += kRowGroups * kHiddenAtOnce) {
+    const bf16_t* wrow[kHiddenAtOnce];
+    float dot[kHiddenAtOnce];
 #pragma unroll
-      for (int e = 0; e < 8; ++e) dot = fmaf(static_cast<float>(w[e]), s_pooled[piece * 8 + e], dot);
+    for (int i = 0; i < kHiddenAtOnce; ++i) {
+      const int j = j0 + i * kRowGroups;
+      wrow[i] = p.fc1_w + static_cast<int64_t>(j < p.hidden ? j : j0) * K;
+      dot[i] = 0.f;
     }
-    dot = group_sum<kRowLanes>(dot);
-    if (l32 == 0) {
-      const float z = dot + (p.fc1_b != nullptr ? static_cast<float>(p.fc1_b[j]) : 0.f);
-      s_hidden[j] = z / (1.0f + expf(-z));
+    for (int piece = l32; piece < kvec; piece += kRowLanes) {
+      bf16x8 w[kHiddenAtOnce];
+#pragma unroll
+      for (int i = 0; i < kHiddenAtOnce; ++i) w[i] = *reinterpret_cast<const bf16x8*>(wrow[i] + piece * 8);
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        const float x = s_pooled[piece * 8 + e];
+#pragma unroll
+        for (int i = 0; i < kHiddenAtOnce; ++i) dot[i] = fmaf(static_cast<float>(w[i][e]), x, dot[i]);
+      }
+    }
+#pragma unroll
+    for (int i = 0; i < kHiddenAtOnce; ++i) {
+      const int j = j0 + i * kRowGroups;
+      dot[i] = group_sum<kRowLanes>(dot[i]);
+      if (l32 == 0 && j < p.hidden) {
+        const float z = dot[i] + (p.fc1_b != nullptr ? static_cast<float>(p.fc1_b[j]) : 0.f);
+        s_hidden[j] = z / (1.0f + expf(-z));
+      }
     }
   }
   __syncthreads();
@@ -268,10 +289,14 @@ extern "C" int taac_candidate_readout_fwd(const void* tokens, const int32_t* key
   p.apply_sigmoid = apply_sigmoid ? 1 : 0;
   hipStream_t s = as_stream(stream);
   const int nv = (D / 8 + kRowLanes - 1) / kRowLanes;
-  // Long sequences get 1024-lane workgroups: a sample's rows are spread over 32 lane groups, and because only two such
-  // workgroups fit a compute unit at a time the rest are handed out as others finish, which evens out samples of very
-  // different lengths. Short sequences keep 256 lanes (more workgroups per compute unit, cheaper reduction).
-  const bool wide = T >= 128;
+  // 1024 lanes for long sequences: a sample's rows are spread over 32 lane groups, and because only two such workgroups fit a compute
+  // unit at a time the rest are handed out as others finish, which evens out samples of very different lengths. Also for batches
+  // whose samples then all run at once, two a compute unit: there the classifier is a chain of loads, and a quarter of the steps is
+  // left. 256 / 1024 lanes, us, samples x tokens at width 256: 1 x 100 26.6 / 12.8, 256 x 60 26.2 / 14.0, 400 x 60 27.2 / 19.9,
+  // 512 x 120 30.9 / 21.8; beyond, short sequences keep 256 lanes (more workgroups per compute unit, cheaper reduction): 640 x 60
+  // 30.5 / 29.0, 1024 x 30 33.3 / 38.0, 1024 x 100 39.7 / 40.7, 2048 x 60 60.7 / 72. 512 x 60 at width 128 16.3 / 12.4, 512 72 / 57,
+  // 1024 230 / 172.
+  const bool wide = T >= 128 || B <= 2 * compute_units();
   const int threads = wide ? 1024 : 256;
   const int groups = threads / kRowLanes;
   const int region = groups * D > p.hidden ? groups * D : p.hidden;

@@ -167,3 +167,29 @@ def test_errors(device):
         candidate_readout(torch.zeros(1, 4, 12, dtype=torch.bfloat16, device=device), cls_index=0)
     with pytest.raises(RuntimeError, match="CUDA"):
         candidate_readout(x.cpu(), cls_index=0)
+
+
+@pytest.mark.parametrize("batch,tokens,d,hidden,actions", [(4, 127, 256, 33, 1), (4, 128, 256, 129, 2), (512, 9, 64, 30, 1),
+                                                           (513, 9, 64, 30, 1), (600, 40, 256, 65, 3), (3, 257, 256, 256, 1),
+                                                           (3, 300, 128, 100, 35), (3, 200, 512, 31, 1), (3, 161, 1000, 260, 1)])
+def test_rows_that_do_not_count_leave_no_trace(device, batch, tokens, d, hidden, actions):
+    """Both workgroup sizes (few samples or many), hidden layers that end inside a step, and padding rows of NaN and infinity."""
+    x, wt, wp, w1, b1, w2, b2, pad = _draw(batch, tokens, d, hidden, actions, seed=tokens + hidden)
+    pad[2, 0] = True
+    x[pad] = float("nan")
+    x[0, ::2] = float("inf")
+    cls_index = 1
+    pad[1:, cls_index] = False
+    x[:, cls_index] = torch.randn(batch, d, generator=torch.Generator().manual_seed(7)).to(torch.bfloat16)
+    finite = x.masked_fill(pad[..., None], 0.0)
+    finite[:, cls_index] = x[:, cls_index]
+    want_emb, want_logits = oracle.candidate_readout(finite, pad, cls_index=cls_index, candidate_index=None,
+                                                     token_norm_weight=wt, pool_norm_weight=wp, eps=1e-6,
+                                                     classifier=(w1, b1, w2, b2))
+    to = lambda t: t.to(device)
+    with torch.no_grad():
+        logits, emb = candidate_readout(to(x), cls_index=cls_index, padding_mask=to(pad), token_norm_weight=to(wt),
+                                        pool_norm_weight=to(wp), fc1_weight=to(w1), fc1_bias=to(b1), fc2_weight=to(w2),
+                                        fc2_bias=to(b2), return_embedding=True)
+    torch.testing.assert_close(emb.cpu().float(), want_emb, **TOL)
+    torch.testing.assert_close(logits.cpu(), want_logits, **TOL)
