@@ -443,14 +443,17 @@ def _held(module: torch.nn.Module | None, name: str) -> torch.Tensor | None:
 
 
 def _every_parameter(module: torch.nn.Module):
-    """``module.parameters()`` without their names, which take longer than the call that they are looked at for; one that several
-    modules share comes several times."""
-    modules = [module]
+    """``module.parameters()`` without their names, which take longer than the call that they are looked at for; every module once
+    (modules may be shared, or hold one that holds them), a parameter that several modules share several times."""
+    modules, seen = [module], {module}
     for m in modules:
         for p in m._parameters.values():
             if p is not None:
                 yield p
-        modules.extend(child for child in m._modules.values() if child is not None)
+        for child in m._modules.values():
+            if child is not None and child not in seen:
+                seen.add(child)
+                modules.append(child)
 
 
 def _block_parameters(block) -> list:

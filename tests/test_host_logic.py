@@ -2,6 +2,7 @@
 
 from __future__ import annotations
 
+import itertools
 import json
 from pathlib import Path
 
@@ -312,3 +313,15 @@ def test_block_parameters_are_the_attributes_values(changed):
         assert got is expected or torch.equal(got, expected)
     assert {id(p) for p in _every_parameter(block)} == {id(p) for p in block.parameters()}
     assert _block_config(block) == (4, block.attn_norm.eps, block.ffn_norm.eps, attention.query_norm.eps, True)
+
+
+def test_parameters_of_modules_that_hold_each_other():
+    """A block whose submodule refers back to it: every module is looked at once, as ``parameters()`` does."""
+    from taac_2026_amd.modeling.backbone import UnifiedInteractionBlock
+    from taac_2026_amd.modeling.block_training import _every_parameter
+
+    block = UnifiedInteractionBlock(128, 4, 2)
+    block.ffn.owner = block
+    expected = list(block.parameters())
+    taken = list(itertools.islice(_every_parameter(block), len(expected) + 1))
+    assert {id(p) for p in taken} == {id(p) for p in expected} and len(taken) == len(expected)
