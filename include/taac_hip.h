@@ -695,7 +695,8 @@ int taac_front_rows(const int32_t* rows, const int32_t* n_rows, int32_t B, int32
  * the r-th valid token of sample b, bit j = struct_bits[position(b, r), position(b, j)] for j below the sample's
  * number of valid tokens n_b and zeros up to the end of the 64-key group of key n_b - 1. Nothing else is written (rows
  * at or beyond n_b, words beyond that group): the attention call below does not read it. struct_bits:
- * [T, ceil(T / 32)] (taac_mask_pack_bits), rows: the index of taac_valid_rows_from_bits. Use with key_lengths =
+ * [T, ceil(T / 32)] (taac_mask_pack_bits), rows: the index of taac_valid_rows_from_bits, whose positions of a sample ascend (an
+ * index in another order gives the bits of that order, slower). Use with key_lengths =
  * the lengths of taac_front_rows, zero_padded_queries = 1 or 2, struct_sample_stride = T * ceil(T / 32) and
  * valid_bits = block_any = NULL in taac_flash_attn_masked_fwd. T <= 4096.
  */

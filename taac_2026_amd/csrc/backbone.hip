@@ -166,9 +166,11 @@ __global__ __launch_bounds__(kBlock) void front_rows_kernel(const int32_t* __res
 
 // One workgroup per (sample b, kFrontRowsPerBlock front rows). The front keys are the sample's valid positions in ascending order, so a
 // front row is its structure row with the bits of the invalid positions squeezed out: one lane takes a word of 32 positions, moves each
-// kept bit down by the number of dropped ones below it - by 1, 2, 4, 8 and 16 where that number has the digit; which bits move in which
+// kept bit down by the number of dropped ones below it - by 1, 2, 4, 8 and 16 where that number has the digit ("compress" in
+// H. S. Warren, Hacker's Delight, 2nd edition, section 7-4); which bits move in which
 // step depends on the validity word alone, so a lane works it out once for all its rows - and ORs the piece into the row's words
-// in LDS from the bit on at which the valid positions in front of the word end. Only rows below the sample's number of valid tokens n_b are written,
+// in LDS from the bit on at which the valid positions in front of the word end. An index that lists a sample's positions in another
+// order is gathered bit by bit (nothing in this library makes one; the look at the order is up to 0.4 us, 512 x 403). Only rows below the sample's number of valid tokens n_b are written,
 // and of those the words that hold a key below n_b's 64-key group (the attention kernel reads nothing else), bits at or beyond n_b as zeros.
 // Bound by the chain of loads in front of it (offsets, positions, structure words). Before, a lane picked the word of its key by a
 // lane permute and a ballot gathered 64 bits. Before / now, us, samples x positions, 30 % of them invalid: 16 x 403 6.2 / 3.7,
@@ -181,7 +183,7 @@ __global__ __launch_bounds__(kBlock) void mask_front_bits_kernel(const uint32_t*
                                                                  const int32_t* __restrict__ rows, int B,
                                                                  uint32_t* __restrict__ out) {
   __shared__ uint32_t valid[kFrontWords];
-  __shared__ uint32_t position[kFrontRowsPerBlock];
+  __shared__ uint32_t position[kFrontRowsPerBlock], descends;
   extern __shared__ uint32_t front[];  // [kFrontRowsPerBlock][wpr]
   const int wpr = (T + 31) / 32;
   const int slabs = (T + kFrontRowsPerBlock - 1) / kFrontRowsPerBlock;
@@ -192,14 +194,30 @@ __global__ __launch_bounds__(kBlock) void mask_front_bits_kernel(const uint32_t*
   if (r0 >= n) return;  // workgroup-uniform
   const int here = n - r0 < kFrontRowsPerBlock ? n - r0 : kFrontRowsPerBlock;
   if (threadIdx.x < kFrontWords) valid[threadIdx.x] = 0u;
+  if (threadIdx.x == 0) descends = 0u;
   for (int i = threadIdx.x; i < here * wpr; i += kBlock) front[i] = 0u;
   __syncthreads();
+  const int written = (n + kWave - 1) / kWave * 2 < wpr ? (n + kWave - 1) / kWave * 2 : wpr;
   for (int j = threadIdx.x; j < n; j += kBlock) {
-    const uint32_t at = static_cast<uint32_t>(rows[off + j] - b * T);
+    const int32_t row = rows[off + j];
+    if (j + 1 < n && row >= rows[off + j + 1]) descends = 1u;
+    const uint32_t at = static_cast<uint32_t>(row - b * T);
     if (at < static_cast<uint32_t>(T)) atomicOr(&valid[at / 32], 1u << (at % 32));
     if (j >= r0 && j < r0 + here) position[j - r0] = at < static_cast<uint32_t>(T) ? at : 0u;
   }
   __syncthreads();
+  if (descends != 0u) {
+    for (int i = threadIdx.x; i < here * written; i += kBlock) {
+      const int r = i / written, first = i % written * 32;
+      uint32_t bits = 0u;
+      for (int k = 0; k < 32 && first + k < n; ++k) {
+        const uint32_t at = static_cast<uint32_t>(rows[off + first + k] - b * T);
+        if (at < static_cast<uint32_t>(T)) bits |= ((struct_bits[static_cast<int64_t>(position[r]) * wpr + at / 32] >> (at % 32)) & 1u) << k;
+      }
+      out[(static_cast<int64_t>(b) * T + r0 + r) * wpr + first / 32] = bits;
+    }
+    return;
+  }
   // lanes of a row: wpr rounded up to a power of two
   const int shift = wpr <= 1 ? 0 : 32 - __builtin_clz(static_cast<unsigned>(wpr - 1));
   const int word = threadIdx.x & ((1 << shift) - 1), row0 = threadIdx.x >> shift, rows_at_once = kBlock >> shift;
@@ -256,7 +274,6 @@ __global__ __launch_bounds__(kBlock) void mask_front_bits_kernel(const uint32_t*
     }
   }
   __syncthreads();
-  const int written = (n + kWave - 1) / kWave * 2 < wpr ? (n + kWave - 1) / kWave * 2 : wpr;
   if (word < written)
     for (int r = row0; r < here; r += rows_at_once)
       out[(static_cast<int64_t>(b) * T + r0 + r) * wpr + word] = front[r * wpr + word];

@@ -251,3 +251,34 @@ def test_front_structured_mask_bits_at_the_edges_of_words(device, batch, tokens)
         got = ((out[b, :n, :written, None] >> shifts) & 1).bool().view(n, written * 32)
         assert torch.equal(got, want[:, :written * 32]), b
         assert (out[b, n:] == untouched).all() and (out[b, :, written:] == untouched).all(), b
+
+
+@pytest.mark.parametrize("batch,tokens", [(2, 2), (3, 33), (4, 200), (2, 1030), (1, 4096)])
+def test_front_structured_mask_bits_of_an_index_in_another_order(device, batch, tokens):
+    """The index decides the order of a sample's rows and keys: the last two swapped, all reversed, and any."""
+    g = torch.Generator().manual_seed(tokens)
+    padding = torch.rand(batch, tokens, generator=g) < 0.3
+    padding[:, :2] = False
+    structural = torch.rand(tokens, tokens, generator=g) < 0.5
+    mask = build_structured_mask(structural.to(device), (~padding).to(device))
+    rows, lengths = valid_rows(None, tokens, padding_mask=padding.to(device))
+    counts = (~padding).sum(dim=1).tolist()
+    words = (tokens + 31) // 32
+    for order in ("swapped", "reversed", "any"):
+        index, at = rows.cpu().clone(), 0
+        positions = []
+        for b, n in enumerate(counts):
+            mine = index[at:at + n].clone()
+            if order == "swapped":
+                mine[-2:] = mine[-2:].flip(0)
+            else:
+                mine = mine.flip(0) if order == "reversed" else mine[torch.randperm(n, generator=g)]
+            index[at:at + n] = mine
+            positions.append(mine.long() - b * tokens)
+            at += n
+        front = front_structured_mask(mask, (index.to(device), lengths), batch)
+        out = front.struct_bits.cpu().view(batch, tokens, words)
+        for b, p in enumerate(positions):
+            n = p.numel()
+            got = ((out[b, :n, :, None] >> torch.arange(32)) & 1).bool().view(n, words * 32)[:, :n]
+            assert torch.equal(got, structural[p][:, p]), (order, b)
