@@ -289,14 +289,18 @@ extern "C" int taac_candidate_readout_fwd(const void* tokens, const int32_t* key
   p.apply_sigmoid = apply_sigmoid ? 1 : 0;
   hipStream_t s = as_stream(stream);
   const int nv = (D / 8 + kRowLanes - 1) / kRowLanes;
-  // 1024 lanes for long sequences: a sample's rows are spread over 32 lane groups, and because only two such workgroups fit a compute
-  // unit at a time the rest are handed out as others finish, which evens out samples of very different lengths. Also for batches
-  // whose samples then all run at once, two a compute unit: there the classifier is a chain of loads, and a quarter of the steps is
-  // left. 256 / 1024 lanes, us, samples x tokens at width 256: 1 x 100 26.6 / 12.8, 256 x 60 26.2 / 14.0, 400 x 60 27.2 / 19.9,
+  // 1024 lanes for long sequences: a sample's rows are spread over 32 lane groups, and because only two such workgroups (from D = 585 on
+  // one) fit a compute unit at a time the rest are handed out as others finish, which evens out samples of very different lengths. With
+  // a classifier also for batches of up to two samples a compute unit: there it is a chain of loads, and a quarter of the steps is left.
+  // 256 / 1024 lanes, us, samples x tokens at width 256: 1 x 100 26.6 / 12.8, 256 x 60 26.2 / 14.0, 400 x 60 27.2 / 19.9,
   // 512 x 120 30.9 / 21.8; beyond, short sequences keep 256 lanes (more workgroups per compute unit, cheaper reduction): 640 x 60
   // 30.5 / 29.0, 1024 x 30 33.3 / 38.0, 1024 x 100 39.7 / 40.7, 2048 x 60 60.7 / 72. 512 x 60 at width 128 16.3 / 12.4, 512 72 / 57,
-  // 1024 230 / 172.
-  const bool wide = T >= 128 || B <= 2 * compute_units();
+  // 1024 230 / 172. Pooling alone has no such chain, only the rows: width 256, 64 x 8 5.3 / 6.0, 256 x 31 6.8 / 6.2, 257 x 31 6.8 / 7.4, 512 x 96
+  // 11.8 / 9.8; 512, 512 x 80 17.7 / 18.9, 512 x 96 19.7 / 19.9; 1024, 256 x 31 13.6 / 10.6, 400 x 8 10.9 / 17.1, 400 x 96 33.1 / 29.4.
+  // The mean is added up in 8 or 32 partial sums accordingly: its last bits depend on T and, between these lines, on B.
+  const int cus = compute_units();
+  const int from = classifier ? 1 : (B <= cus ? 24 : 96);
+  const bool wide = T >= 128 || (T >= from && B <= 2 * cus);
   const int threads = wide ? 1024 : 256;
   const int groups = threads / kRowLanes;
   const int region = groups * D > p.hidden ? groups * D : p.hidden;

@@ -193,3 +193,15 @@ def test_rows_that_do_not_count_leave_no_trace(device, batch, tokens, d, hidden,
                                         fc2_bias=to(b2), return_embedding=True)
     torch.testing.assert_close(emb.cpu().float(), want_emb, **TOL)
     torch.testing.assert_close(logits.cpu(), want_logits, **TOL)
+
+
+@pytest.mark.parametrize("tokens,d", [(2, 64), (17, 256), (23, 1000)])
+def test_pooling_alone_of_short_samples_does_not_depend_on_the_batch(device, tokens, d):
+    """Without the classifier a short sample's rows are added up in the same groups whatever the number of samples: the same bits."""
+    batch = 2 * torch.cuda.get_device_properties(device).multi_processor_count + 1
+    x, wt, wp, *_ = _draw(batch, tokens, d, 16, 1, seed=tokens)
+    kw = dict(cls_index=0, candidate_index=1, token_norm_weight=wt.to(device), pool_norm_weight=wp.to(device))
+    with torch.no_grad():
+        many = candidate_readout(x.to(device), **kw)
+        few = candidate_readout(x[:5].to(device), **kw)
+    assert torch.equal(few, many[:5])
