@@ -44,7 +44,7 @@ int backbone_setup(const taac_block_weights* blocks, int n, int32_t D, int32_t F
                    const int32_t* lengths, int32_t B, int32_t T, int32_t* rows, int32_t* n_rows, void* zero_rows,
                    uint32_t* counters, int32_t n_counters, hipStream_t s, const char* name);
 bool ffn_act_fold_supported(int32_t D, int32_t F);
-bool ffn_few_rows(int64_t M, int32_t D);
+bool ffn_few_rows(int64_t M, int32_t D, int32_t F);
 // Workgroups that share the hidden units of a token tile when the gated feed-forward over at most M rows runs as the few-token
 // kernel and is given the scratch memory for it (ffn_split_bytes; the counters behind the partials zeroed once): a power of
 // two as long as the tiles leave that many compute units idle. 1 otherwise.

@@ -1310,7 +1310,6 @@ int launch_ts(K kernel, const TsParams& p, int threads, int tokens_per_wg, size_
 
 bool ptr_ok(const void* p, uintptr_t mask) { return (reinterpret_cast<uintptr_t>(p) & mask) == 0; }
 
-constexpr int kMaxLdsBytes = 160 * 1024;
 
 }  // namespace
 }  // namespace taac
@@ -1564,7 +1563,7 @@ int ffn_entry(const char* name, const void* x, int64_t ldx, const void* out_bias
   if (p.units <= 0) return set_error(TAAC_ERR_LAUNCH, "%s: cannot query the device", name);
   if (const int limit = test_max_workgroups(); limit > 0 && limit < p.units) p.units = limit;  // taac_test_hooks
   hipStream_t s = as_stream(stream);
-  if (ffn_few_rows(M, D) && glu && update_gate == nullptr && packed_weights && (norm_weight == nullptr || norm_folded)) {
+  if (ffn_few_rows(M, D, F) && glu && update_gate == nullptr && packed_weights && (norm_weight == nullptr || norm_folded)) {
     if (split_scratch != nullptr && (p.splits = ffn_splits(M, D, F)) > 1) {
       p.split_partials = static_cast<float*>(split_scratch);
       p.split_counters = reinterpret_cast<uint32_t*>(p.split_partials + (M + 31) / 32 * p.splits * 32 * D);
@@ -1934,13 +1933,18 @@ int attn_out_ffn_count(const char* name, const void* attn, const void* out_bias,
 }
 
 // Whether the gated feed-forward over at most M rows of D features runs as the few-token kernel. M counts padded rows. With the out
-// projection in front, one launch, few-token / persistent kernel, us, all rows valid and 55 % of them: D = 256, F = 1024 - 512 rows
-// 17.6 / 50.9, 8103 23.0 / 56.2 and 19.6 / 52.4, 16384 32.4 / 57.6 and 26.1 / 52.2, 24576 54.1 / 59.0 and 29.2 / 55.8, 32768 60.9 /
-// 62.6 and 55.2 / 54.5, 49152 89.6 / 89.1 and 55.3 / 57.6, 65536 117 / 103 and 86.4 / 81.4; F = 512 - 24576 37.6 / 39.6 and 20.1 / 35.3,
-// 32768 40.8 / 41.0 and 36.3 / 36.1, 49152 58.9 / 56.1 and 37.0 / 37.8. D = 128, F = 512 - 512 8.2 / 20.2, 16384 14.4 / 22.2 and 12.7 /
-// 21.3, 49152 30.8 / 33.1 and 19.2 / 23.7, 65536 37.8 / 35.7 and 27.9 / 30.4; F = 256 - 49152 23.3 / 23.7 and 15.5 / 17.4, 65536 29.0 /
-// 25.8 and 21.6 / 21.4.
-bool ffn_few_rows(int64_t M, int32_t D) { return test_max_workgroups() == 0 && M <= (D == 256 ? 24576 : 49152); }
+// projection in front, one launch, few-token / persistent kernel, us, all rows valid and 55 % of them: D = 256 - F = 512, 24576 rows 37.6 /
+// 39.6 and 20.1 / 35.3, 32768 40.8 / 41.0 and 36.3 / 36.1, 49152 58.9 / 56.1 and 37.0 / 37.8; F = 1024, 512 rows 17.6 / 50.9, 8103 23.0 / 56.2
+// and 19.6 / 52.4, 16384 32.4 / 57.6 and 26.1 / 52.2, 24576 54.1 / 59.0 and 29.2 / 55.8, 32768 60.9 / 62.6 and 55.2 / 54.5, 49152 89.6 / 89.1 and
+// 55.3 / 57.6; F = 2048, 16384 61 / 97 and 42 / 91, 24576 98 / 106 and 51 / 93; F = 3072, 24576 141 / 144 and 70 / 132; without the projection, F =
+// 4096, 24576 180 / 186 and 89 / 174. D = 128 - F = 256, 49152 23.3 / 23.7 and 15.5 / 17.4, 65536 29.0 / 25.8 and 21.6 / 21.4; F = 512, 512 rows 8.2
+// / 20.2, 16384 14.4 / 22.2 and 12.7 / 21.3, 49152 30.8 / 33.1 and 19.2 / 23.7, 65536 37.8 / 35.7 and 27.9 / 30.4; 49152 rows, F = 640 36.1 / 37.9
+// and 22.0 / 26.0, F = 1024 49.8 / 52.9 and 29.4 / 35.2 (without the projection 53.4 / 50.7 and 30.6 / 34.5), F = 2048 86 / 94 and 51 / 62, F = 3072
+// 121 / 136 and 71 / 88. From F = 3936 on a compute unit has one place for two tiles of 128 features: F = 4096, 24576 rows 116 / 114 and 58 /
+// 110, 32768 124 / 121 and 112 / 112, 49152 182 / 173 and 114 / 115.
+bool ffn_few_rows(int64_t M, int32_t D, int32_t F) {
+  return test_max_workgroups() == 0 && M <= (D == 256 || F > 3904 ? 24576 : 49152);
+}
 
 // Whether a projection over at most M rows of D features runs as the few-token kernel (transform: with the query / key norm weight or
 // rotation in its epilogue). One launch, few-token / persistent kernel, us, all rows valid and 55 % of them, q | k | v: D = 256 - 512 rows

@@ -7,6 +7,8 @@
 // straight from L2 into MFMA operand registers - fragments are 1 KB of contiguous memory, no other wavefront of the workgroup
 // wants them, so a stop in LDS would only add a barrier. What bounds these kernels is latency: row count -> row index ->
 // token rows -> products -> store, with the weight fragments requested in front of that chain.
+#include <algorithm>
+
 #include "common.h"
 #include "ts_common.h"
 #include "ts_dense.h"
@@ -298,22 +300,18 @@ struct SharedPartials {
 // splits > 1 (see TsParams): for batches that leave most of the chip idle even so, the hidden units of a tile are also divided over
 // workgroups; the exchange costs 4 - 5 us, and the rule is at ffn_splits.
 // ------------------------------------------------------------------------------------------------------------------
-constexpr int kSlab = 64;  // 16-unit chunks whose hidden state lies in LDS at a time (F = 1024 in one piece)
+constexpr int kPiece = 64;  // 16-unit chunks whose hidden state lies in LDS in one piece at most (F = 1024)
 
-// LDS of the kernel for workgroups of TT token tiles and `chunks` chunks of hidden units: first the normalised rows of a tile that are
-// kept (one tile: read once, but the hidden state need not wait for it; two tiles, D = 256: the second one's fragments, for which there
-// are no registers), then the tokens as they come in (and the other normalised rows), whose place the hidden state takes. The
-// biases and sums come behind.
+// LDS of the kernel for workgroups of TT token tiles and `chunks` chunks of hidden units, at most `slab` at a time: first the normalised
+// rows of a tile that are kept (one tile: read once, but the hidden state need not wait for it; two tiles, D = 256: the second one's
+// fragments, for which there are no registers), then the tokens as they come in (and the other normalised rows), whose place the hidden
+// state takes. The biases and sums come behind.
 __host__ __device__ constexpr int small_kept_bytes(int D, int TT) { return TT == 1 || D == 256 ? 32 * (D * 2 + 16) : 0; }
-__host__ __device__ constexpr int small_tile_bytes(int D, int TT, int chunks) {
-  const int rows = 32 * (D * 2 + 16), hidden = TT * (chunks < kSlab ? chunks : kSlab) * kFrag;
+__host__ __device__ constexpr int small_tile_bytes(int D, int TT, int chunks, int slab) {
+  const int rows = 32 * (D * 2 + 16), hidden = TT * (chunks < slab ? chunks : slab) * kFrag;
   const int tokens = 2 * TT * rows - small_kept_bytes(D, TT);
   return small_kept_bytes(D, TT) + (hidden > tokens ? hidden : tokens);
 }
-
-// Workgroups that a compute unit holds: of the one-tile form, and of the form that takes one or two tiles.
-__host__ __device__ constexpr int small_one_residents(int D) { return D == 256 ? 1 : 3; }
-__host__ __device__ constexpr int small_pair_residents(int D) { return D == 256 ? 1 : 2; }
 
 // Groups of one chunk per wavefront that a workgroup of the kernel takes at most.
 __host__ __device__ constexpr int small_groups(int D, int F, int splits) {
@@ -334,7 +332,7 @@ struct SmallTokens {
   }
 };
 
-template <int D, int TT, bool OUTP, bool FOLD, bool SLABS>
+template <int D, int TT, bool OUTP, bool FOLD, int SLAB>
 __device__ __forceinline__ void ffn_small_tile(const TsParams& p, uint8_t* smem, int64_t count, int tile, int split,
                                                SmallTokens<D, TT>& tokens, bf16x8 (&ring)[D / 16]) {
   constexpr int KS = D / 16, MB = D / 32;
@@ -345,7 +343,7 @@ __device__ __forceinline__ void ffn_small_tile(const TsParams& p, uint8_t* smem,
   constexpr int XT = D == 256 ? 1 : TT;       // tiles whose normalised tokens stay in registers
   constexpr int kKept = small_kept_bytes(D, TT);
   static_assert(KS == 2 * NW, "a ring holds the down fragments of two groups of chunks");
-  static_assert(TT == 1 || !SLABS, "two tiles: one slab");
+  constexpr bool SLABS = SLAB > 0;
   const int F = p.F;
   const int nchunks = F / kHU;
   const int splits = TT == 1 && p.splits > 1 ? p.splits : 1;
@@ -359,7 +357,7 @@ __device__ __forceinline__ void ffn_small_tile(const TsParams& p, uint8_t* smem,
   };
   uint8_t* x_lds = smem + (TT == 1 ? kKept : kKept + (kKept > 0 ? 1 : 2) * 32 * kRow);
   uint8_t* hidden_lds = smem + kKept;
-  float* bias_lds = reinterpret_cast<float*>(smem + small_tile_bytes(D, TT, groups * NW));
+  float* bias_lds = reinterpret_cast<float*>(smem + small_tile_bytes(D, TT, groups * NW, SLABS ? SLAB : kPiece));
   bf16_t* end_lds = reinterpret_cast<bf16_t*>(bias_lds + 2 * F);  // down-projection bias, readout weight
   float* sums = reinterpret_cast<float*>(end_lds + 2 * D);  // [TT][NW][32]
 
@@ -449,7 +447,7 @@ __device__ __forceinline__ void ffn_small_tile(const TsParams& p, uint8_t* smem,
   // Groups in which the wavefront has a chunk: all but perhaps the last one of the workgroup. (A wavefront without a chunk in a slab
   // goes through the motions with the last chunk: what it leaves in its place of the hidden state is not used.)
   const int all_own = first_chunk(groups - 1) + wave < nchunks ? groups : groups - 1;
-  constexpr int kSlabGroups = kSlab / NW;
+  constexpr int kSlabGroups = (SLABS ? SLAB : kPiece) / NW;
   auto ring_up = [&](int group) {
     const int at = up_at(group);
     static_for<KS>([&](auto ic) { ring[decltype(ic)::value] = request_up(at, ic); });
@@ -592,6 +590,12 @@ __device__ __forceinline__ void ffn_small_tile(const TsParams& p, uint8_t* smem,
     if constexpr (TT == 1) __syncthreads();  // as below, and the biases
   }
   if constexpr (TT > 1) __syncthreads();  // the hidden state takes the place of the tokens
+  if constexpr (OUTP && SLABS) {  // x1 is kept as it is rounded (widened ahead of the loop it would be spilled)
+#pragma unroll
+    for (int t = 0; t < TT; ++t)
+#pragma unroll
+      for (int jq = 0; jq < 4; ++jq) asm volatile("" : "+v"(hv[t][jq]));
+  }
 
   f32x16 total[TT];
 #pragma unroll
@@ -760,14 +764,25 @@ __device__ __forceinline__ void ffn_small_tile(const TsParams& p, uint8_t* smem,
   }
 }
 
-// Forms of the kernel: one tile, one slab / one tile, several slabs (F > 1024) / one or two tiles, one slab. The last is for more
-// rows than the chip has places for one-tile workgroups: the number of tokens, known on the device only, decides whether its
-// workgroups take two tiles (D = 256, F = 1024: 12288 rows, all valid, 28.0 us, 39.3 with one tile in two rounds; 6758 valid 21.2, one tile
-// in one round).
-enum { kSmallOne, kSmallSlabs, kSmallPair };
+// Forms of the kernel. One tile per workgroup: its hidden state in one piece / in slabs of 1024 units / (D = 128) of 512, whose smaller
+// LDS leaves a compute unit three workgroups instead of two or one. For more rows than the chip has places for one-tile workgroups: the
+// number of tokens, known on the device only, decides whether workgroups take one tile or two (D = 256, F = 1024: 12288 rows, all valid,
+// 28.0 us, 39.3 with one tile in two rounds; 6758 valid 21.2, one tile in one round), in one piece / in slabs of 512 units (D = 128: 384 for
+// two tiles) where F is over 1024 or the pieces would leave a compute unit fewer workgroups. One launch behind the out projection, us, with
+// slabs for one tile only and places that do not depend on F / as it is: D = 256, F = 2048 - 9216 rows 66 / 45, 16384 78 / 61, 55 % valid 65 / 42,
+// 24576 117 / 98 and 68 / 51 (12288 rows, 55 % valid, 34 / 36: one tile in the larger kernel); D = 128 - F = 640, 40960 rows 40 / 34 and 27 / 21; F =
+// 1024, 16384 rows 24.4 / 21.9 and 23.0 / 18.9, 32768 38 / 34 and 36 / 27; F = 2048, 24576 rows 65 / 52 and 40 / 35, 49152 121 / 86 and 75 / 51.
+enum { kSmallOne, kSmallSlabs, kSmallHalfSlabs, kSmallPair, kSmallPairSlabs };
+__host__ __device__ constexpr bool small_pairs(int form) { return form == kSmallPair || form == kSmallPairSlabs; }
+// Chunks of hidden units in a slab of workgroups of TT tiles, 0 where they lie in one piece.
+__host__ __device__ constexpr int small_slab(int D, int TT, int form) {
+  if (form == kSmallOne || form == kSmallPair) return 0;
+  if (form == kSmallSlabs) return kPiece;
+  return TT == 2 ? (D == 256 ? 32 : 24) : (D == 256 ? kPiece : 32);
+}
 
 template <int D, bool OUTP, bool FOLD, int FORM>
-__global__ __launch_bounds__(D / 32 * kWave, D == 256 || FORM == kSmallPair ? 2 : 3) void swiglu_ffn_small_kernel(const TsParams p) {
+__global__ __launch_bounds__(D / 32 * kWave, D == 256 || small_pairs(FORM) ? 2 : 3) void swiglu_ffn_small_kernel(const TsParams p) {
   constexpr int KS = D / 16;
   extern __shared__ __attribute__((aligned(1024))) uint8_t smem[];
   const int tid = threadIdx.x;
@@ -794,14 +809,15 @@ __global__ __launch_bounds__(D / 32 * kWave, D == 256 || FORM == kSmallPair ? 2 
     });
     __builtin_amdgcn_sched_barrier(0);
   }
-  if constexpr (FORM == kSmallPair) {
-    if (count > static_cast<int64_t>(p.units) * (32 * small_pair_residents(D))) {
-      if (static_cast<int64_t>(tile) * 64 < count) ffn_small_tile<D, 2, OUTP, FOLD, false>(p, smem, count, tile, 0, two, ring);
+  if constexpr (small_pairs(FORM)) {
+    if (count > static_cast<int64_t>(p.units) * 32) {  // p.units: workgroups that run at once
+      if constexpr (FORM == kSmallPairSlabs) two.request(p, static_cast<int64_t>(tile) * 64, tid, lane % 32);
+      if (static_cast<int64_t>(tile) * 64 < count) ffn_small_tile<D, 2, OUTP, FOLD, small_slab(D, 2, FORM)>(p, smem, count, tile, 0, two, ring);
       return;
     }
   }
   if (static_cast<int64_t>(tile) * 32 < count)
-    ffn_small_tile<D, 1, OUTP, FOLD, FORM == kSmallSlabs>(p, smem, count, tile, split, one, ring);
+    ffn_small_tile<D, 1, OUTP, FOLD, small_slab(D, 1, FORM)>(p, smem, count, tile, split, one, ring);
 }
 
 }  // namespace
@@ -809,12 +825,13 @@ __global__ __launch_bounds__(D / 32 * kWave, D == 256 || FORM == kSmallPair ? 2 
 // Two or four workgroups per token tile as long as the tiles leave them a compute unit each, every wavefront keeps two chunks of
 // hidden units, and the weights are worth the exchange. Whole 4-block calls, 1 / 2 / 4 / 8 splits, us: D = 256, F = 1024 - 1 x 512
 // positions 146 / 125 / 116 / 119, 8 x 256 139 / 121 / 119; F = 512 (two chunks at two splits) - 1 x 512 115 / 112 / 108, 4 x 512
-// 116 / 115 / 116; D = 128, F = 512 - 1 x 512 86 / 84 / 82, 8 x 256 81 / 80 / 80; F = 256 - 78 / 79 / 79, 74 / 75 / 77.
+// 116 / 115 / 116; D = 128, F = 512 - 1 x 512 86 / 84 / 82, 8 x 256 81 / 80 / 80; F = 256 - 78 / 79 / 79, 74 / 75 / 77. (Those of a kernel whose
+// exchange was of all features, which gained from eight at F = 2048, 161 -> 156; four in this one: 130.)
 int ffn_splits(int64_t M, int32_t D, int32_t F) {
   const int64_t tiles = (M + 31) / 32;
   const int cus = compute_units();
   int splits = 1;
-  if (ffn_few_rows(M, D) && F >= 512)
+  if (ffn_few_rows(M, D, F) && F >= 512)
     while (splits < 4 && 2 * splits * tiles <= cus && 2 * splits * 2 * (D / 32) * kHU <= F) splits *= 2;
   return splits;
 }
@@ -849,18 +866,41 @@ int norm_linear_small(const TsParams& p, int32_t K, int qk_mode, hipStream_t s, 
 #undef TAAC_SMALL
 }
 
-int swiglu_ffn_small(const TsParams& p, int32_t D, bool with_proj, bool act_folded, hipStream_t s, const char* name) {
+// Bytes of LDS of a form (of the larger of the tiles its workgroups may take), and workgroups of it that a compute unit holds: by its
+// registers (launch bounds) and by its LDS, which is handed out in pieces of 1280 bytes.
+namespace {
+int small_lds(int D, int F, int chunks, int form) {
+  const int tt = small_pairs(form) ? 2 : 1;
+  auto tile = [&](int of) { return small_tile_bytes(D, of, chunks, small_slab(D, of, form) > 0 ? small_slab(D, of, form) : kPiece); };
+  const int tile_bytes = tt == 2 ? std::max(tile(1), tile(2)) : tile(1);
+  return tile_bytes + 2 * F * 4 + 4 * D + tt * (D / 32) * 32 * 4;
+}
+int small_places(int D, int F, int chunks, int form) {
+  const int by_registers = D == 256 ? 1 : (small_pairs(form) ? 2 : 3);
+  return std::min(by_registers, kMaxLdsBytes / ((small_lds(D, F, chunks, form) + 1279) / 1280 * 1280));
+}
+
+}  // namespace
+
+int swiglu_ffn_small(const TsParams& params, int32_t D, bool with_proj, bool act_folded, hipStream_t s, const char* name) {
+  TsParams p = params;
   const int splits = p.splits > 1 ? p.splits : 1;
   const int64_t tiles = (p.M + 31) / 32;
   const int chunks = small_groups(D, p.F, splits) * (D / 32);
-  const int form = chunks > kSlab ? kSmallSlabs : (tiles > small_one_residents(D) * p.units ? kSmallPair : kSmallOne);
-  const int tt = form == kSmallPair ? 2 : 1;
-  int tile_bytes = small_tile_bytes(D, 1, chunks);
-  if (tt == 2 && small_tile_bytes(D, 2, chunks) > tile_bytes) tile_bytes = small_tile_bytes(D, 2, chunks);
-  const size_t lds_bytes = tile_bytes + static_cast<size_t>(2) * p.F * 4 + 4 * D + static_cast<size_t>(tt) * (D / 32) * 32 * 4;
-  if (lds_bytes > 160 * 1024) return 1;
-  const int64_t pairs = (p.M + 63) / 64, residents = small_pair_residents(D) * p.units;  // (these take one tile while that suffices)
-  const dim3 grid(static_cast<uint32_t>(form == kSmallPair ? (pairs > residents ? pairs : residents) : tiles * splits));
+  auto places = [&](int form) { return small_places(D, p.F, chunks, form) * p.units; };
+  auto in_one_round = [&](int form) { return tiles * splits <= places(form); };
+  int form = chunks > kPiece ? kSmallSlabs : kSmallOne;
+  if (!in_one_round(form)) {
+    if (D == 128 && in_one_round(kSmallHalfSlabs))
+      form = kSmallHalfSlabs;
+    else
+      form = chunks > kPiece || places(kSmallPairSlabs) > places(kSmallPair) ? kSmallPairSlabs : kSmallPair;
+  }
+  const size_t lds_bytes = small_lds(D, p.F, chunks, form);
+  if (lds_bytes > kMaxLdsBytes) return 1;
+  p.units = places(form);
+  const int64_t pairs = (p.M + 63) / 64;  // (workgroups take one tile while one round of them suffices)
+  const dim3 grid(static_cast<uint32_t>(small_pairs(form) ? std::max<int64_t>(pairs, p.units) : tiles * splits));
 #define TAAC_SMALL_LAUNCH(DD, OO, FF, FORM)                                                                           \
   do {                                                                                                                \
     if (hipFuncSetAttribute(reinterpret_cast<const void*>(swiglu_ffn_small_kernel<DD, OO, FF, FORM>),                 \
@@ -872,7 +912,10 @@ int swiglu_ffn_small(const TsParams& p, int32_t D, bool with_proj, bool act_fold
 #define TAAC_SMALL(DD, OO, FF)                                        \
   do {                                                                \
     if (form == kSmallSlabs) TAAC_SMALL_LAUNCH(DD, OO, FF, kSmallSlabs); \
+    if constexpr (DD == 128)                                             \
+      if (form == kSmallHalfSlabs) TAAC_SMALL_LAUNCH(DD, OO, FF, kSmallHalfSlabs); \
     if (form == kSmallPair) TAAC_SMALL_LAUNCH(DD, OO, FF, kSmallPair);   \
+    if (form == kSmallPairSlabs) TAAC_SMALL_LAUNCH(DD, OO, FF, kSmallPairSlabs);   \
     TAAC_SMALL_LAUNCH(DD, OO, FF, kSmallOne);                         \
   } while (0)
 #define TAAC_SMALL_D(DD)                        \

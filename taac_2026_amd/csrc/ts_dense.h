@@ -17,6 +17,8 @@ constexpr int kStageWave = 32 * kStageRow;    // epilogue tile of one wavefront:
 
 }  // namespace
 
+constexpr int kMaxLdsBytes = 160 * 1024;  // of a compute unit
+
 struct TsParams {
   const bf16_t* x;          // [M, D] row stride ldx
   const bf16_t* norm_w;     // [D] or null (no normalisation)
@@ -37,7 +39,8 @@ struct TsParams {
                             // first *n_rows rows (a compact tensor whose length the host does not know)
   const int32_t* x_rows;    // optional, with rows: token i's row of x when it differs from rows[i] (x and residual / out
                             // laid out differently: samples with their valid tokens moved to the front on one side)
-  int32_t units;            // FFN: compute units the last, partial round of workgroups is spread over
+  int32_t units;            // FFN: compute units the last, partial round of workgroups is spread over; few-token kernel: its workgroups
+                            // that run at once
   // Query / key mode of the linear kernel (the packed q | k | v projection of an attention layer):
   const bf16_t* qk_w;       // [D] norm weight of the query features, or null (ones)
   const bf16_t* qk_wk;      // [D] norm weight of the key features, with qk_w

@@ -124,11 +124,13 @@ def test_feed_forward_matches_the_persistent_kernel(device, test_hooks, m, d, f,
 
 
 @pytest.mark.parametrize("d,f,rows_over,valid", [(256, 64, 1, 1.0), (256, 1024, 33, 1.0), (256, 96, 1, 0.5), (256, 64, 33, 0.99), (128, 32, 1, 1.0),
-                                                 (128, 512, 65, 0.8), (128, 32, 1, 0.4), (256, 1056, None, 1.0), (128, 2080, None, 0.7)])
+                                                 (128, 512, 65, 0.8), (128, 32, 1, 0.4), (256, 1056, None, 1.0), (128, 2080, None, 0.7),
+                                                 (128, 640, -40, 1.0), (128, 1024, 33, 1.0), (128, 1056, 1, 0.3), (128, 2080, 65, 0.6),
+                                                 (256, 1056, 33, 1.0), (256, 1056, 1, 0.4), (256, 2080, 65, 0.7)])
 def test_forms_of_the_few_token_feed_forward(device, test_hooks, d, f, rows_over, valid):
     """Rows just over the places that the chip has for one-tile workgroups (one per compute unit at D = 256, three at 128), with so many
-    valid that workgroups take two tiles, the last of them a remainder, or one; hidden sizes over one slab of 1024 units, with a
-    remainder (rows_over None: 70 rows). Bound: as in the test above. Rows that are not listed stay as they are."""
+    valid that workgroups take two tiles, the last of them a remainder, or one; hidden sizes over one slab of 1024 units (512 where two
+    tiles or several workgroups share the LDS), with a remainder (rows_over None: 70 rows). Bound: as in the test above. Rows that are not listed stay as they are."""
     places = torch.cuda.get_device_properties(device).multi_processor_count * (1 if d == 256 else 3)
     m = 70 if rows_over is None else 32 * places + rows_over
     g = torch.Generator().manual_seed(m + f)
