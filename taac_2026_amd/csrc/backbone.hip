@@ -629,7 +629,7 @@ extern "C" int taac_backbone_fwd(const void* emb, const int32_t* key_lengths, co
     if ((rc = backbone_setup(blocks, n_blocks, D, F, fp8 ? nullptr : pk.data(), pk.data() + n_blocks, pk.data() + 2 * n_blocks,
                              fold_act, qk_norms && rope_cos_sin == nullptr ? norm_product : nullptr, key_lengths, B, T, rows,
                              n_rows, sparse ? hidden_out : nullptr, ffn_split > 1 ? split_counters : qk_counters,
-                             ffn_split > 1 ? static_cast<int32_t>(tiles) : (dense_few_rows(M, D, true) ? 0 : kQkCounters),
+                             ffn_split > 1 ? static_cast<int32_t>(tiles) : (dense_few_rows(M, D, 3 * D, true, false) ? 0 : kQkCounters),
                              as_stream(stream), name)) != TAAC_OK)
       return rc;
   }

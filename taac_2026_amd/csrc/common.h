@@ -66,9 +66,9 @@ int norm_linear_qk_factors(const char* name, const void* x, int64_t ldx, const v
                            const void* packed_weights, void* out, int64_t ldo, int64_t M, int32_t d_model, int32_t num_heads,
                            int32_t tokens_per_sample, float qk_eps, float* qk_sumsq, float* qk_rstd, uint32_t* qk_counters,
                            const int32_t* rows, const int32_t* n_rows, const int32_t* x_rows, int norm_folded, void* stream);
-// Whether a projection over at most M rows of D features runs as the few-token kernel of ffn_small.hip; transform: its epilogue
-// applies the query / key norm weights or the rotation (the lower line).
-bool dense_few_rows(int64_t M, int32_t D, bool transform);
+// Whether a projection over at most M rows of D features to N runs as the few-token kernel of ffn_small.hip; transform: its epilogue
+// applies the query / key norm weights or the rotation; residual: it adds one.
+bool dense_few_rows(int64_t M, int32_t D, int32_t N, bool transform, bool residual);
 // Out projection + feed-forward half of a block (ffn.hip; attn_plane: 0 = rows of ld_attn elements, 32 / 64 = per-head
 // planes) that also writes the dot product of every stored output row with head_w to token_dots[row]; split_scratch:
 // ffn_split_bytes(M, D, F) bytes, or null.

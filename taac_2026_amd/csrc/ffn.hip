@@ -22,6 +22,8 @@
 // bf16, transposed through a wavefront-private LDS tile and written as 16-byte pieces, eight lanes per 128-byte row
 // segment; the residual is read the same way and added after the rounding of the layer output, which is the order
 // of roundings of the reference's bf16 evaluation (linear output rounded, then the residual add rounded).
+#include <algorithm>
+
 #include "common.h"
 #include "ts_common.h"
 #include "pack.h"
@@ -1778,7 +1780,7 @@ int norm_linear_launch(const char* name, const void* x, int64_t ldx, const void*
   p.tokens_per_sample = qk.tokens_per_sample;
   hipStream_t s = as_stream(stream);
   const bool qk_transform = qk.enabled && (qk.q_weight != nullptr || qk.cos_sin != nullptr);
-  if (dense_few_rows(M, K, qk_transform) && packed_weights && (norm_weight == nullptr || norm_folded))
+  if (dense_few_rows(M, K, N, qk_transform, residual != nullptr) && packed_weights && (norm_weight == nullptr || norm_folded))
     return norm_linear_small(p, K, qk_transform ? 2 : (qk.enabled ? 1 : 0), s, name);
   // Without a residual two token tiles per wavefront fit the register file: every weight fragment read from LDS then
   // feeds two MFMAs, which halves the LDS reads (and their share of the power budget) per token.
@@ -1946,15 +1948,23 @@ bool ffn_few_rows(int64_t M, int32_t D, int32_t F) {
   return test_max_workgroups() == 0 && M <= (D == 256 || F > 3904 ? 24576 : 49152);
 }
 
-// Whether a projection over at most M rows of D features runs as the few-token kernel (transform: with the query / key norm weight or
+// Whether a projection over at most M rows of D features to N runs as the few-token kernel (transform: with the query / key norm weight or
 // rotation in its epilogue). One launch, few-token / persistent kernel, us, all rows valid and 55 % of them, q | k | v: D = 256 - 512 rows
 // 5.1 / 14.6, 8103 10.6 / 16.2 and 7.6 / 15.4, 16384 17.2 / 22.0 and 11.3 / 16.4, 32768 25.4 / 25.9 and 16.4 / 20.6; with the factors of the query /
-// key norms 32768 27.2 / 29.5 and 18.1 / 23.5; rotated 8103 14.9 / 19.4, 24576 32.6 / 33.4 and 20.0 / 25.6, 32768 38.8 / 35.0 and 24.8 / 27.3;
-// a residual in N = 256 32768 14.9 / 15.8. D = 128 - 512 rows 4.0 / 9.4, 49152 14.4 / 16.0 and 10.8 / 13.4, with the factors 18.8 / 18.4 and
-// 13.1 / 14.9, rotated 22.8 / 23.9 and 16.0 / 18.6; 65536 17.4 / 18.2, 23.4 / 20.7, 28.1 / 25.7. Above the line every compute unit has its tiles
-// and the persistent kernel's weights, shared through LDS, cost it less.
-bool dense_few_rows(int64_t M, int32_t D, bool transform) {
-  return test_max_workgroups() == 0 && M <= (D != 256 ? 49152 : transform ? 24576 : 32768);  // (taac_test_hooks: a capped grid)
+// key norms 32768 27.2 / 29.5 and 18.1 / 23.5; rotated 8103 14.9 / 19.4, 24576 32.6 / 33.4 and 20.0 / 25.6, 32768 38.8 / 35.0 and 24.8 / 27.3.
+// D = 128 - 512 rows 4.0 / 9.4, 49152 14.4 / 16.0 and 10.8 / 13.4, with the factors 18.8 / 18.4 and 13.1 / 14.9, rotated 22.8 / 23.9 and 16.0 /
+// 18.6; 65536 17.4 / 18.2, 23.4 / 20.7, 28.1 / 25.7. Above the line every compute unit has its tiles and the persistent kernel's weights, shared
+// through LDS, cost it less.
+// More features (behind a norm): D = 256, N = 1024, 32768 rows 26.7 / 29.7 and 19.0 / 24.7; N = 1536, 20480 31.5 / 29.1,
+// 32768 45.6 / 41.1 and 27.8 / 29.0; N = 2048, 16384 27.4 / 29.5 and 19.2 / 23.1, 32768 52.3 / 45.8 and 29.4 / 31.8; D = 128, N = 1024, 49152 29.6 / 28.8
+// and 19.3 / 19.8; N = 2048, 32768 39.5 / 36.3, 49152 53.5 / 48.0. A residual, whose rows every workgroup waits for in each of its tiles: D = 256,
+// N = 256, 24576 14.0 / 13.6 and 10.1 / 11.3, 32768 17.2 / 15.2 and 12.2 / 13.4; N = 512, 20480 19.4 / 17.7; N = 768, 8192 15.3 / 14.8, 16384 24.2 / 19.0 and
+// 16.4 / 15.4, 24576 30.0 / 25.0 and 20.4 / 17.2; D = 128, N = 128, 49152 10.5 / 10.2 and 6.6 / 8.2; N = 384, 20480 11.2 / 10.8, 32768 16.1 / 14.5.
+bool dense_few_rows(int64_t M, int32_t D, int32_t N, bool transform, bool residual) {
+  int64_t line = D != 256 ? 49152 : transform ? 24576 : 32768;
+  if (N > 1024) line = D != 256 ? 24576 : 16384;
+  if (residual) line = std::min<int64_t>({line, D != 256 ? 49152 : 24576, (int64_t{1} << 23) / N});
+  return test_max_workgroups() == 0 && M <= line;  // (taac_test_hooks: a capped grid)
 }
 
 // Whether the kernels take the activation's constants from the packed weights at this shape: the gated form with the
