@@ -1199,20 +1199,21 @@ bool small_offsets(int64_t rows, int64_t stride) {
 
 // The fused kernel where a workgroup can hold a sample's keys (512 of 32 features, 256 of 64) and there are enough (sample, head)
 // pairs: it has one workgroup per pair where the two kernels have one per 128 rows. Two kernels / fused in us, lengths ~ U{16..rows}:
-//   up to 128 rows (as many workgroups either way):  48 x 32, 256 pairs 8.8 / 6.8, 8192 pairs 58 / 54;  128 x 64, 256 pairs 15.7 / 12.6,
-//   16384 pairs 453 / 330.
-//   256 x 32:  256 pairs 20.0 / 20.5, 512 pairs 27.7 / 24.9, 4096 pairs 165 / 122;  256 x 64:  256 pairs 27.1 / 28.7, 512 pairs 48 / 38,
-//   8192 pairs 523 / 387.
-//   More rows of 32 features, four key tiles per wavefront and half the wavefronts in flight. In three blocks of 128 the two kernels
-//   hold their own: 300 rows, 1024 pairs 55 / 54 and 50 / 53 (two draws of the lengths), 2048 pairs 85 / 92, 3584 pairs 169 / 164, 8192
-//   pairs 358 / 326. In four: 400 rows, 1024 pairs 85 / 70, 8192 pairs 687 / 462; 480 rows, 1024 pairs 102 / 103; 512 rows, 1024 pairs 108 /
-//   117 and 102 / 99, 1536 pairs 152 / 150 and 139 / 132, 8192 pairs 809 / 638. Causal, 300 rows, 512 pairs 31 / 28, 512 rows 65 / 54.
-// Mask bits: 64 features, 64 rows, 256 pairs 12.6 / 8.7, 8192 pairs 175 / 123, 256 rows, 512 pairs 59 / 45, 8192 pairs 674 / 534; 32 features,
-// 160 rows, 512 pairs 24.4 / 19.8, 256 rows, 512 pairs 34 / 31, 8192 pairs 370 / 290. Up to 128 rows of 32 features there is little to gain,
-// and the second dP loses it where the workgroups are several to a compute unit: 64 rows, 512 pairs 10.8 / 8.4, 1536 pairs 20.2 / 20.1, 3072
-// pairs 32.6 / 35.5; 96 rows, 2048 pairs 31.2 / 30.1, 4096 pairs 52 / 55; 128 rows, 2048 pairs 36.8 / 35.2. Over 256 rows of 32 features
-// they stay with the two kernels: the words' registers are the ones that the four key tiles of a wavefront need (already with one dP, 300
-// rows, 1024 pairs 67 / 74, 4096 pairs 239 / 274; 403 rows 117 / 116, 436 / 360).
+//   up to 128 rows (as many workgroups either way):  48 x 32, 256 pairs 9.9 / 9.0, 8192 pairs 65 / 58; 128 x 32, 8192 pairs 126 / 107;
+//   128 x 64, 256 pairs 16.9 / 12.8, 16384 pairs 456 / 328.
+//   256 x 32:  128 pairs 15.9 / 17.3, 256 pairs 20.1 / 19.1, 512 pairs 27.0 / 24.8, 4096 pairs 156 / 117;  256 x 64:  128 pairs 22.7 / 24.9, 256
+//   pairs 30.3 / 27.4, 512 pairs 48 / 39, 8192 pairs 538 / 376. (Between 256 and 512 pairs a few per cent lie on either side.)
+//   More rows of 32 features, four key tiles per wavefront and half the wavefronts in flight:  300 rows, 512 pairs 34.6 / 31.0, 1024 pairs
+//   55 / 48, 2048 pairs 93 / 82, 8192 pairs 361 / 283;  384 rows, 512 pairs 45.3 / 45.6, 1024 pairs 72 / 66, 2048 pairs 119 / 98;  400 rows, 1024
+//   pairs 92 / 71, 8192 pairs 654 / 411;  480 rows, 512 pairs 65 / 67, 1024 pairs 101 / 89;  512 rows, 512 pairs 62 / 61, 1024 pairs 109 / 89, 8192
+//   pairs 821 / 589. Causal, 300 rows, 512 pairs 29.8 / 23.4, 512 rows 60 / 45.
+// Mask bits: 64 features, 64 rows, 256 pairs 13.5 / 9.5, 8192 pairs 172 / 128, 256 rows, 256 pairs 37 / 36, 512 pairs 57 / 48, 8192 pairs 649 / 472;
+// 32 features, 160 rows, 512 pairs 24.0 / 20.0, 256 rows, 512 pairs 31.7 / 29.7, 8192 pairs 345 / 269. Up to 128 rows of 32 features there is
+// little to gain, and the second dP loses it where the workgroups are several to a compute unit: 64 rows, 512 pairs 12.2 / 9.9, 1536 pairs
+// 22.6 / 21.6, 2048 pairs 25.6 / 27.0, 8192 pairs 76 / 86; 96 rows, 2048 pairs 33.0 / 31.3, 4096 pairs 55.6 / 57.1; 128 rows, 2048 pairs 43.0 /
+// 38.5, 3072 pairs 52.6 / 50.7, 6144 pairs 97 / 103. Over 256 rows of 32 features they stay with the two kernels: the words' registers are the
+// ones that the four key tiles of a wavefront need (with one dP and before both forms' reads were requested ahead, 300 rows, 1024 pairs 67 / 74,
+// 4096 pairs 239 / 274; 403 rows 117 / 116, 436 / 360).
 template <typename T, int DP, int MODE, bool COMPACT>
 bool launch_bwd_fused(AttnBwdParams p, hipStream_t s) {
   constexpr int kSmall = 64 / DP, kLarge = 128 / DP;  // key tiles per wavefront
@@ -1220,7 +1221,7 @@ bool launch_bwd_fused(AttnBwdParams p, hipStream_t s) {
   const int64_t pairs = static_cast<int64_t>(p.B) * p.H;
   const int32_t rows = p.Tq > p.Tk ? p.Tq : p.Tk;
   int64_t enough = rows <= kOwn ? 1 : 512;
-  if (DP == 32 && rows > kRowsSmall && !p.causal) enough = rows <= 3 * kOwn ? 3584 : (rows <= 480 ? 1024 : 1536);
+  if (DP == 32 && rows > kRowsSmall && !p.causal) enough = 1024;
   if (rows > kRowsLarge || pairs < enough) return false;
   if (DP == 32 && MODE == kMaskBits && rows <= kOwn && pairs > (rows <= 64 ? 1536 : 2048)) return false;
   if (!small_offsets(p.Tq, p.qs[2]) || !small_offsets(p.Tq, p.dos[2]) || !small_offsets(p.Tk, p.ks[2])) return false;
