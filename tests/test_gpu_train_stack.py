@@ -86,6 +86,19 @@ def test_training_stack_at_the_edges_of_its_tiles(device, d_model, heads, d_ff, 
         _near(name, parameter.grad, reference[name].grad, n_blocks)
 
 
+@pytest.mark.parametrize("d_model,heads,d_ff,n_blocks,lengths,tokens,qk_norm,dtype", [
+    (256, 8, 1024, 1, [1], 1, False, torch.bfloat16),
+    (256, 4, 96, 2, [0, 65, 64, 1], 65, True, torch.float32),
+    (128, 4, 160, 2, [31, 33, 0], 33, True, torch.float32),
+    (256, 8, 512, 1, [(7 * i) % 33 for i in range(1100)], 32, False, torch.bfloat16),
+    (128, 4, 128, 1, [(5 * i) % 41 for i in range(900)], 40, False, torch.float32),
+])
+def test_training_stack_with_the_persistent_kernels(device, test_hooks, d_model, heads, d_ff, n_blocks, lengths, tokens, qk_norm, dtype):
+    """The same at sizes for which the few-token kernels are taken, through the kernels of large batches (a capped grid selects them)."""
+    test_hooks(max_workgroups=256)
+    test_training_stack_at_the_edges_of_its_tiles(device, d_model, heads, d_ff, n_blocks, lengths, tokens, qk_norm, dtype)
+
+
 def test_a_stack_is_its_blocks_one_after_the_other(device):
     """``run_interaction_blocks`` under autograd (17 blocks: more than one set-up launch) = the blocks called one by one, bit for
     bit: every kernel is the same, and gathering and scattering the valid rows in between changes no value."""
@@ -356,12 +369,18 @@ def test_training_stack_with_the_kernels_of_large_batches(device):
             _near(name, parameter.grad, reference[name].grad, 1)
 
 
-@pytest.mark.parametrize("d_model,heads,batch,tokens,full", [(256, 8, 140, 130, False), (256, 4, 600, 130, True), (128, 4, 300, 130, False)])
-def test_tokens_between_the_halves_of_a_large_batch(device, d_model, heads, batch, tokens, full):
-    """The persistent feed-forward kernel of the training forward stores the tokens between a block's halves while it projects: against
+@pytest.mark.parametrize("d_model,heads,batch,tokens,full,gate_first", [
+    (256, 8, 140, 130, False, True), (256, 4, 600, 130, True, True), (128, 4, 300, 130, False, True), (128, 2, 1100, 130, True, True),
+    (256, 4, 140, 130, False, False), (128, 4, 300, 130, False, False)])
+def test_tokens_between_the_halves_of_a_large_batch(device, test_hooks, d_model, heads, batch, tokens, full, gate_first):
+    """The persistent feed-forward kernel of the training forward (a capped grid selects it whatever the number of rows; with the
+    activation's constants in the weights, gate first, and without) stores the tokens between a block's halves while it projects: against
     the inference route, which writes them with a kernel of their own, over slices of a few wavefronts and, with enough tokens, over
     whole tiles and a remainder. Both round the projection and the sum once (2^-8 of values below 8: 2^-5 each); on the whole the
-    two differ by one rounding."""
+    two differ by one rounding. Gate last, the inference route's up weights hold the activation's constants and are rounded with them: a
+    gate and a value that are 2^-9 off each, 2^-8 of the update more."""
+    test_hooks(max_workgroups=256)
+    whole = 2.0 ** -8 if gate_first else 2.0 ** -7
     g = torch.Generator(device=device).manual_seed(batch)
     block = UnifiedInteractionBlock(d_model, heads, 2)
     with torch.no_grad():
@@ -369,6 +388,7 @@ def test_tokens_between_the_halves_of_a_large_batch(device, d_model, heads, batc
             p.copy_(torch.randn(p.shape, generator=torch.Generator().manual_seed(len(name))) * (p.shape[-1] ** -0.5 if p.ndim == 2 else 0.1)
                     + (1.0 if name.endswith("norm.weight") else 0.0))
     block = block.to(torch.bfloat16).to(device)
+    block.ffn.gate_first = gate_first
     x = torch.randn(batch, tokens, d_model, generator=g, device=device).to(torch.bfloat16)
     lengths = torch.randint(tokens - 1 if full else 0, tokens + 1, (batch,), generator=g, device=device, dtype=torch.int32)
     padding = torch.arange(tokens, device=device) >= lengths[:, None]
@@ -377,7 +397,7 @@ def test_tokens_between_the_halves_of_a_large_batch(device, d_model, heads, batc
     got_out, got_between = block.train()(x.clone().requires_grad_(True), padding, None, key_lengths=lengths)
     for got, want in ((got_between, between), (got_out, out)):
         a, b = got[~padding].float(), want[~padding].float()
-        assert b.abs().max() < 8 and (a - b).abs().max() <= 2.0 ** -4 and (a - b).norm() <= 2.0 ** -8 * b.norm()
+        assert b.abs().max() < 8 and (a - b).abs().max() <= 2.0 ** -4 and (a - b).norm() <= whole * b.norm()
         assert torch.equal(got[padding], x[padding])
 
 
